@@ -1,9 +1,12 @@
-// Plain tiled matrix product in float32 arithmetic for any storage types and any sizes:
+// Matrix product in float32 arithmetic for any storage types and any sizes:
 //   C[m, n] (+)= sum_k A[m, k] * W[n, k]      (weights are [out, in], k contiguous)
 // It is the whole matrix path of the float32 mode and the fallback of the bfloat16
-// mode for shapes its MFMA kernels refuse. Each output is summed over k ascending by
-// one thread with fused multiply-adds, so its value does not depend on M, on the tile
-// it falls in, or on what else is in the batch. (hb_gemm_plain_short_k is the entry for products with a
+// mode for shapes its own MFMA kernels refuse. Each output is summed over k ascending
+// with fused multiply-adds, so its value does not depend on M, on the tile or kernel
+// it falls in, or on what else is in the batch: the matrix cores' float32 products
+// (v_mfma_f32_16x16x4_f32) add their four k one after another with one rounding each,
+// bit for bit what fmaf gives in that order (checked on 16,384 sums of mixed magnitudes),
+// and every kernel here feeds them k in ascending order. (hb_gemm_plain_short_k is the entry for products with a
 // short k: it sends up to 32 float32 rows times bfloat16 rows to gemm_few_rows_kernel, whose four partial
 // sums a column differ from that order by float32 rounding, and everything else here.)
 // In xigh/herbert-rs: crates/backends/backend_bf16/src/kernels.rs:154-164 (float32 sums over k ascending of
@@ -12,9 +15,7 @@
 
 HB_MODULE_ERROR_SLOT()
 
-#define TILE_M 64
-#define TILE_N 64
-#define TILE_K 16
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // What a product may do to a sum before it stores it: nothing (rate null), or turn the pre-activation of a
 // decay into the decay itself, exp(-exp(rate[n / D]) * softplus(sum + bias[n])) for column n (float32; the
@@ -37,86 +38,269 @@ __device__ __forceinline__ float decay_of(const DecayEpilogue& ep, float sum, in
     return expf(-expf(ep.rate[n / ep.D]) * softplus);
 }
 
-template <class TA, class TW, class TC, bool ACCUM>
+// One 16 x 16 x 4 product: w is W[n = lane % 16, k], a is A[m = lane % 16, k], both for k = k0 + lane / 16; lane l's
+// four sums are those of n = 4 (l / 16) .. + 3 and m = l % 16.
+__device__ __forceinline__ f32x4 mfma_k4(float w, float a, f32x4 sums) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(w, a, sums, 0, 0, 0);
+}
+
+// Four neighbouring elements of a row as float32 (16 or 8 bytes, aligned), or what lies below `left` of them.
+template <bool VEC>
+__device__ __forceinline__ f32x4 load_quad(const float* p, int left) {
+    f32x4 r = {0.f, 0.f, 0.f, 0.f};
+    if (VEC) {
+        if (left > 0) r = *(const f32x4*)p;
+        return r;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (i < left) r[i] = p[i];
+    return r;
+}
+template <bool VEC>
+__device__ __forceinline__ f32x4 load_quad(const bf16* p, int left) {
+    f32x4 r = {0.f, 0.f, 0.f, 0.f};
+    if (VEC) {
+        if (left > 0) {
+            const uint2 u = *(const uint2*)p;
+            r[0] = __uint_as_float(u.x << 16), r[1] = __uint_as_float(u.x & 0xffff0000u);
+            r[2] = __uint_as_float(u.y << 16), r[3] = __uint_as_float(u.y & 0xffff0000u);
+        }
+        return r;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (i < left) r[i] = hb_to_float(p[i]);
+    return r;
+}
+
+// What a lane holds of one output column's four neighbouring rows n .. n + 3 into C[m, n ..].
+template <class TC, bool ACCUM, bool VEC>
+__device__ __forceinline__ void store_quad(TC* C, int ldc, int m, int n, int N, f32x4 sums, const DecayEpilogue& ep) {
+    TC* out = C + (size_t)m * ldc + n;
+    if (ep.rate) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (n + e < N) sums[e] = decay_of(ep, sums[e], n + e);
+    }
+    if (VEC && sizeof(TC) == 4) {
+        if (n >= N) return;
+        f32x4* o = (f32x4*)out;
+        if (ACCUM) sums += *o;
+        *o = sums;
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if (n + e >= N) return;
+        out[e] = hb_from_float<TC>(ACCUM ? hb_to_float(out[e]) + sums[e] : sums[e]);
+    }
+}
+
+// More than 16 rows: a workgroup of four waves (2 x 2) on a tile of BM rows of A by BN rows of W. Stages of BK elements
+// of k go through LDS in two buffers: a stage is asked for (16 bytes a lane) before the one at hand is multiplied and
+// written to the other buffer after it, so a stage costs one barrier and no wait for memory. A product of 16 x 16 x 4
+// wants k = k0 + lane / 16 from a lane, so within every 16 k LDS holds a row's elements transposed, element 4 s + q at
+// place 4 q + s: a lane's next four products are then one 16-byte read. Rows are BK + 4 floats apart: the reads of 16
+// rows meet no bank twice. Bound by the matrix cores (a library's large product reaches 154 TFLOP/s here):
+// 4096 x 4096 x 4096 in 1,082 us (127 TFLOP/s), 564 x 6144 x 2048 in 165, 564 x 2048 x 2048 in 67, 64 x 4096 x 4096 in
+// 55; the kernel of vector FMAs and 4-byte loads that this replaced took 2,465, 372, 323 and 632.
+template <class TA, class TW, class TC, bool ACCUM, int BM, int BN, int BK, bool VEC>
 __global__ void __launch_bounds__(256)
-gemm_plain_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* __restrict__ C, int M, int N,
-                  int K, int lda, int ldw, int ldc, size_t batch_a, size_t batch_w, size_t batch_c,
-                  DecayEpilogue ep) {
+gemm_plain_tile_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* __restrict__ C, int M, int N,
+                       int K, int lda, int ldw, int ldc, size_t batch_a, size_t batch_w, size_t batch_c,
+                       DecayEpilogue ep) {
     // (blockIdx.z: one of a batch of products whose operands lie batch_* elements apart)
     A += blockIdx.z * batch_a;
     W += blockIdx.z * batch_w;
     C += blockIdx.z * batch_c;
-    __shared__ float As[TILE_K][TILE_M + 1];
-    __shared__ float Ws[TILE_K][TILE_N + 1];
-    const int tid = threadIdx.x;
-    const int tx = tid % 16;   // column group
-    const int ty = tid / 16;   // row group
-    const int m0 = blockIdx.y * TILE_M;
-    const int n0 = blockIdx.x * TILE_N;
+    constexpr int LD = BK + 4, QUADS = BK / 4;
+    constexpr int QA = BM * QUADS / 256, QW = BN * QUADS / 256;      // quads a thread stages of either operand
+    constexpr int MB = BM / 32, NB = BN / 32;                        // blocks of 16 a wave
+    __shared__ __attribute__((aligned(16))) float As[2][BM * LD], Ws[2][BN * LD];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int r = lane & 15, q = lane >> 4;
+    const int across = (N + BN - 1) / BN;                            // tiles of a row of tiles
+    const int m0 = (int)(blockIdx.x / across) * BM, n0 = (int)(blockIdx.x % across) * BN;
+    const int wm = (wave & 1) * (BM / 2), wn = (wave >> 1) * (BN / 2);
 
-    float acc[4][4];
+    f32x4 a_next[QA], w_next[QW];
+    auto fetch = [&](int k0) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < QA; ++i) {
+            const int row = (tid + 256 * i) / QUADS, k = k0 + 4 * ((tid + 256 * i) % QUADS);
+            a_next[i] = load_quad<VEC>(A + (size_t)(m0 + row) * lda + k, m0 + row < M ? K - k : 0);
+        }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+        for (int i = 0; i < QW; ++i) {
+            const int row = (tid + 256 * i) / QUADS, k = k0 + 4 * ((tid + 256 * i) % QUADS);
+            w_next[i] = load_quad<VEC>(W + (size_t)(n0 + row) * ldw + k, n0 + row < N ? K - k : 0);
+        }
+    };
+    auto stash = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < QA; ++i) {
+            const int row = (tid + 256 * i) / QUADS, quad = (tid + 256 * i) % QUADS;
+            float* to = &As[buf][row * LD + (quad & ~3) * 4 + (quad & 3)];
+            to[0] = a_next[i][0], to[4] = a_next[i][1], to[8] = a_next[i][2], to[12] = a_next[i][3];
+        }
+#pragma unroll
+        for (int i = 0; i < QW; ++i) {
+            const int row = (tid + 256 * i) / QUADS, quad = (tid + 256 * i) % QUADS;
+            float* to = &Ws[buf][row * LD + (quad & ~3) * 4 + (quad & 3)];
+            to[0] = w_next[i][0], to[4] = w_next[i][1], to[8] = w_next[i][2], to[12] = w_next[i][3];
+        }
+    };
 
-    for (int k0 = 0; k0 < K; k0 += TILE_K) {
-        // 64 x 16 elements of each operand, 4 per thread; k runs fastest in memory.
+    f32x4 acc[NB][MB];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int e = tid + i * 256;
-            const int kk = e % TILE_K;
-            const int rr = e / TILE_K;
-            const int k = k0 + kk;
-            const int m = m0 + rr;
-            const int n = n0 + rr;
-            As[kk][rr] = (m < M && k < K) ? hb_to_float(A[(size_t)m * lda + k]) : 0.f;
-            Ws[kk][rr] = (n < N && k < K) ? hb_to_float(W[(size_t)n * ldw + k]) : 0.f;
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int i = 0; i < MB; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    fetch(0);
+    stash(0);
+    __syncthreads();
+    int buf = 0;
+    for (int k0 = 0; k0 < K; k0 += BK, buf ^= 1) {
+        const bool more = k0 + BK < K;
+        if (more) fetch(k0 + BK);
+#pragma unroll
+        for (int b = 0; b < BK / 16; ++b) {
+            f32x4 a[MB], w[NB];
+#pragma unroll
+            for (int i = 0; i < MB; ++i) a[i] = *(const f32x4*)&As[buf][(wm + 16 * i + r) * LD + 16 * b + 4 * q];
+#pragma unroll
+            for (int j = 0; j < NB; ++j) w[j] = *(const f32x4*)&Ws[buf][(wn + 16 * j + r) * LD + 16 * b + 4 * q];
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int j = 0; j < NB; ++j)
+#pragma unroll
+                    for (int i = 0; i < MB; ++i) acc[j][i] = mfma_k4(w[j][s], a[i][s], acc[j][i]);
         }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < TILE_K; ++kk) {
-            float a[4], w[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = As[kk][ty + 16 * i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) w[j] = Ws[kk][tx + 16 * j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], w[j], acc[i][j]);
-        }
+        if (more) stash(buf ^ 1);
         __syncthreads();
     }
 
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int m = m0 + ty + 16 * i;
+    for (int i = 0; i < MB; ++i) {
+        const int m = m0 + wm + 16 * i + r;
         if (m >= M) continue;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int n = n0 + tx + 16 * j;
-            if (n >= N) continue;
-            const size_t idx = (size_t)m * ldc + n;
-            if (ACCUM)
-                C[idx] = hb_from_float<TC>(hb_to_float(C[idx]) + acc[i][j]);
-            else
-                C[idx] = hb_from_float<TC>(ep.rate ? decay_of(ep, acc[i][j], n) : acc[i][j]);
+        for (int j = 0; j < NB; ++j)
+            store_quad<TC, ACCUM, VEC>(C, ldc, m, n0 + wn + 16 * j + 4 * q, N, acc[j][i], ep);
+    }
+}
+
+// Four quads, one a lane row of 16 (lane / 16), transposed in registers: x[i] of lane row q was element 4 q + i of 16
+// and becomes element 4 i + q, which is what the i-th of four products wants of that lane row.
+__device__ __forceinline__ void transpose_quads(f32x4& x) {
+    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+    auto halves = [](float& a, float& b) {
+        const u32x2 t = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+        a = __uint_as_float(t[0]), b = __uint_as_float(t[1]);
+    };
+    auto rows = [](float& a, float& b) {
+        const u32x2 t = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+        a = __uint_as_float(t[0]), b = __uint_as_float(t[1]);
+    };
+    float x0 = x[0], x1 = x[1], x2 = x[2], x3 = x[3];
+    halves(x0, x2);
+    halves(x1, x3);
+    rows(x0, x1);
+    rows(x2, x3);
+    x[0] = x0, x[1] = x1, x[2] = x2, x[3] = x3;
+}
+
+// Up to 16 rows (a decode step): a product bound by the weights' bytes. A wave alone on 16 rows of W: no LDS and no
+// barrier; every lane loads a quad of its row of W and of A for each of the next WAVE_DEPTH blocks of 16 k while the
+// WAVE_DEPTH before are multiplied, and the lanes' quads are transposed in registers. The sum over k is one chain as
+// everywhere here (no split of k: the order is the other kernel's), 8.5 us of products at K = 2048, which bounds narrow
+// weights; wide ones stream. 2 x 2048 x 2048 takes 19 us, 2 x 6144 x 2048 21, 2 x 32768 x 2048 52 (5.2 TB/s); tiles of
+// 32 x 32 take 21, 26 and 60, the kernel that these replaced took 253, 262 and 378. (8 blocks ahead; 16 take as long
+// at few rows and 10 % longer at many, 24 longer everywhere; two blocks of 16 rows of A a wave for 17 to 32 rows: 63 us
+// at 24 x 4096 x 4096 where tiles of 32 x 32 take 53.)
+#define WAVE_ROWS 16
+#define WAVE_DEPTH 8
+template <class TA, class TW, class TC, bool ACCUM>
+__global__ void __launch_bounds__(HB_WAVE)
+gemm_plain_wave_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* __restrict__ C, int M, int N,
+                       int K, int lda, int ldw, int ldc, size_t batch_a, size_t batch_w, size_t batch_c,
+                       DecayEpilogue ep) {
+    A += blockIdx.z * batch_a;
+    W += blockIdx.z * batch_w;
+    C += blockIdx.z * batch_c;
+    const int lane = threadIdx.x, r = lane & 15, q = lane >> 4;
+    const int n0 = blockIdx.x * 16;
+    // (rows beyond M or N are row 0 once more, whose sums go nowhere; blocks beyond K are zeros)
+    const TW* w_row = W + (size_t)(n0 + r < N ? n0 + r : 0) * ldw + 4 * q;
+    const TA* a_row = A + (size_t)(r < M ? r : 0) * lda + 4 * q;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f}, w_next[WAVE_DEPTH], a_next[WAVE_DEPTH];
+    auto fetch = [&](int k0) {
+#pragma unroll
+        for (int d = 0; d < WAVE_DEPTH; ++d) {
+            const int k = k0 + 16 * d;
+            w_next[d] = load_quad<true>(w_row + k, K - k);
+            a_next[d] = load_quad<true>(a_row + k, K - k);
+        }
+    };
+    fetch(0);
+    for (int k0 = 0; k0 < K; k0 += 16 * WAVE_DEPTH) {
+        f32x4 w[WAVE_DEPTH], a[WAVE_DEPTH];
+#pragma unroll
+        for (int d = 0; d < WAVE_DEPTH; ++d) w[d] = w_next[d], a[d] = a_next[d];
+        if (k0 + 16 * WAVE_DEPTH < K) fetch(k0 + 16 * WAVE_DEPTH);
+#pragma unroll
+        for (int d = 0; d < WAVE_DEPTH; ++d) {
+            transpose_quads(w[d]);
+            transpose_quads(a[d]);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) acc = mfma_k4(w[d][s], a[d][s], acc);
         }
     }
+    if (r < M) store_quad<TC, ACCUM, true>(C, ldc, r, n0 + 4 * q, N, acc, ep);
+}
+
+// The kernel of a product. 16-byte loads and stores where rows and strides allow them. Up to 16 rows of whole blocks of
+// 16 k take the wave kernel. Beyond, the largest tile that still fills the chip: 128 x 128 from two tiles for every CU on
+// (4096 x 4096 x 4096: 1,082 us; 64 x 64 1,281), 64 x 64 from two of those for every CU on (1200 x 4096 x 4096: 414;
+// 32 x 32 444, 128 x 128 539), else 32 x 32 (200 x 2048 x 2048: 30; 64 x 64 51; 564 x 2048 x 2048: 67; 64 x 64 84).
+template <class TA, class TW, class TC, bool ACCUM>
+static void launch_as(const TA* A, const TW* W, TC* C, int M, int N, int K, int lda, int ldw, int ldc,
+                      hipStream_t stream, int batch, size_t batch_a, size_t batch_w, size_t batch_c, DecayEpilogue ep) {
+    const bool vec = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && batch_a % 4 == 0 && batch_w % 4 == 0 &&
+                     (uintptr_t)A % (4 * sizeof(TA)) == 0 && (uintptr_t)W % (4 * sizeof(TW)) == 0 &&
+                     (sizeof(TC) != 4 || (N % 4 == 0 && ldc % 4 == 0 && batch_c % 4 == 0 && (uintptr_t)C % 16 == 0));
+    auto tiles = [&](int side) { return (long long)((N + side - 1) / side) * ((M + side - 1) / side) * batch; };
+#define HB_PLAIN_TILE(BM, BK, VEC)                                                                                    \
+    gemm_plain_tile_kernel<TA, TW, TC, ACCUM, BM, BM, BK, VEC>                                                        \
+        <<<dim3((unsigned)(tiles(BM) / batch), 1, batch), 256, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, batch_a, \
+                                                                            batch_w, batch_c, ep)
+    if (vec && M <= WAVE_ROWS && K % 16 == 0)
+        gemm_plain_wave_kernel<TA, TW, TC, ACCUM><<<dim3((N + 15) / 16, 1, batch), HB_WAVE, 0, stream>>>(
+            A, W, C, M, N, K, lda, ldw, ldc, batch_a, batch_w, batch_c, ep);
+    else if (!vec)
+        HB_PLAIN_TILE(32, 64, false);
+    else if (tiles(128) >= 512)
+        HB_PLAIN_TILE(128, 32, true);
+    else if (tiles(64) >= 512)
+        HB_PLAIN_TILE(64, 64, true);
+    else
+        HB_PLAIN_TILE(32, 64, true);
+#undef HB_PLAIN_TILE
 }
 
 template <class TA, class TW, class TC>
 static void launch(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc,
                    int accumulate, hipStream_t stream, int batch = 1, size_t batch_a = 0, size_t batch_w = 0,
                    size_t batch_c = 0, DecayEpilogue ep = DecayEpilogue{nullptr, nullptr, 1, 0.f}) {
-    dim3 grid((N + TILE_N - 1) / TILE_N, (M + TILE_M - 1) / TILE_M, batch);
     if (accumulate)
-        gemm_plain_kernel<TA, TW, TC, true><<<grid, 256, 0, stream>>>(
-            (const TA*)A, (const TW*)W, (TC*)C, M, N, K, lda, ldw, ldc, batch_a, batch_w, batch_c, ep);
+        launch_as<TA, TW, TC, true>((const TA*)A, (const TW*)W, (TC*)C, M, N, K, lda, ldw, ldc, stream, batch, batch_a,
+                                    batch_w, batch_c, ep);
     else
-        gemm_plain_kernel<TA, TW, TC, false><<<grid, 256, 0, stream>>>(
-            (const TA*)A, (const TW*)W, (TC*)C, M, N, K, lda, ldw, ldc, batch_a, batch_w, batch_c, ep);
+        launch_as<TA, TW, TC, false>((const TA*)A, (const TW*)W, (TC*)C, M, N, K, lda, ldw, ldc, stream, batch, batch_a,
+                                     batch_w, batch_c, ep);
 }
 
 
@@ -201,7 +385,7 @@ extern "C" int hb_gemm_plain(const void* A, int a_dtype, const void* W, int w_dt
                              hipStream_t stream) {
     HB_REQUIRE(M > 0 && N > 0 && K > 0, "gemm: empty problem (M=%d, N=%d, K=%d)", M, N, K);
     HB_REQUIRE(lda >= K && ldw >= K && ldc >= N, "gemm: a row stride is smaller than its row");
-    HB_REQUIRE((M + TILE_M - 1) / TILE_M <= 65535, "gemm: M=%d exceeds the grid", M);
+    HB_REQUIRE((M + 63) / 64 <= 65535, "gemm: M=%d exceeds the grid", M);
     const int key = a_dtype * 4 + w_dtype * 2 + c_dtype;
     switch (key) {
         case 0: launch<float, float, float>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, stream); break;
@@ -239,7 +423,7 @@ extern "C" int hb_gemm_plain_short_k(const void* A, int a_dtype, const void* W, 
         return 0;
     }
     if (!A_log) return hb_gemm_plain(A, a_dtype, W, w_dtype, C, c_dtype, M, N, K, lda, ldw, ldc, accumulate, stream);
-    HB_REQUIRE((M + TILE_M - 1) / TILE_M <= 65535, "gemm: M=%d exceeds the grid", M);
+    HB_REQUIRE((M + 63) / 64 <= 65535, "gemm: M=%d exceeds the grid", M);
     switch (a_dtype * 2 + w_dtype) {
         case 0: launch<float, float, float>(A, W, C, M, N, K, lda, ldw, ldc, 0, stream, 1, 0, 0, 0, ep); break;
         case 1: launch<float, bf16, float>(A, W, C, M, N, K, lda, ldw, ldc, 0, stream, 1, 0, 0, 0, ep); break;
@@ -259,7 +443,7 @@ extern "C" int hb_gemm_plain_batched(const void* A, int a_dtype, const void* W, 
                                      size_t batch_w, size_t batch_c, hipStream_t stream) {
     HB_REQUIRE(M > 0 && N > 0 && K > 0 && batch > 0, "gemm: empty problem (M=%d, N=%d, K=%d, batch=%d)", M, N, K, batch);
     HB_REQUIRE(lda >= K && ldw >= K && ldc >= N, "gemm: a row stride is smaller than its row");
-    HB_REQUIRE((M + TILE_M - 1) / TILE_M <= 65535 && batch <= 65535, "gemm: M=%d or batch=%d exceeds the grid", M, batch);
+    HB_REQUIRE((M + 63) / 64 <= 65535 && batch <= 65535, "gemm: M=%d or batch=%d exceeds the grid", M, batch);
     // few rows (one token a sequence) with a short k: the kernel made for them, a product of the batch a grid's layer
     if (few_rows_takes(A, a_dtype, W, w_dtype, c_dtype, M, K, lda, ldw, 0) && batch_a % 4 == 0 && batch_w % 8 == 0) {
         gemm_few_rows_kernel<<<dim3((N + 15) / 16, (M + FEW_ROWS_M - 1) / FEW_ROWS_M, batch), HB_WAVE, 0, stream>>>(

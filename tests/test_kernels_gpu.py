@@ -66,6 +66,31 @@ def test_gemm_plain(M, N, K, dts):
     assert torch.allclose(cb.float(), want, rtol=2 ** -8, atol=1e-3)
 
 
+@pytest.mark.parametrize("K", [16, 144, 2048, 100, 31])            # whole blocks of 16 k, part of one, no whole quad
+@pytest.mark.parametrize("wd", [torch.float32, torch.bfloat16])
+def test_gemm_plain_sums_do_not_depend_on_the_rows(K, wd):
+    """Every kernel and tile of the product sums k in one order: a row's results are the same bits whether it comes
+    alone, with 16 (the wave kernel), with some more (tiles of 32) or with a thousand (tiles of 64 and 128), also
+    where a row of N is cut by a tile's edge. Against float64: a chain of K fused steps is off by at most K / 2^24 of
+    the sum of the terms' sizes."""
+    from herbert_rs_amd.kernels import ops
+    for N in (2050, 4100):
+        a = rand(4200 if N == 4100 else 1030, K, seed=13)
+        w = rand(N, K, seed=14, dtype=wd)
+        whole = torch.empty(a.shape[0], N, device=dev())
+        ops.gemm_plain(a, w, whole)
+        want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+        assert bool(((whole.double() - want).abs() <= K * 2.0 ** -24 * size + 1e-30).all())
+        base = rand(a.shape[0], N, seed=15)
+        for rows in (1, 16, 17, 33, 130, 1025):
+            got = torch.empty(rows, N, device=dev())
+            ops.gemm_plain(a[:rows].contiguous(), w, got)
+            assert torch.equal(got, whole[:rows]), rows
+            added = base[:rows].clone()
+            ops.gemm_plain(a[:rows].contiguous(), w, added, accumulate=True)
+            assert torch.equal(added, base[:rows] + whole[:rows]), rows
+
+
 @pytest.mark.parametrize("I", [5, 128, 1000])
 def test_swiglu(I):
     from herbert_rs_amd.kernels import ops
