@@ -1,10 +1,21 @@
 // Plain attention over the paged cache, float32 arithmetic, any storage types,
 // any head size up to 512, any number of heads and groups.
-// One wave per (token, query head). The keys a query at position p sees are
+// The keys a query at position p sees are
 // [max(0, p + 1 - window), p] (window 0 = all keys from 0). They are walked in
 // chunks of 64 that start at multiples of 64 of the absolute position, with an
 // online softmax: the chunking, and so the rounding, depends on the positions only,
 // not on how the tokens were cut into steps or batches.
+// A workgroup of four waves takes 16 columns: the query heads of one key head for one token (a decode step), or for
+// the next few packed tokens (a prompt), each with its own mask. Both contractions run on the matrix cores in float32
+// (mfma_f32.h), whose sums are chains of fmaf over ascending k: a score over the head's entries, an output over a chunk's keys. A
+// wave scores 16 of a chunk's 64 keys, the scores meet in LDS, where every wave reads all 64 of its lanes' columns as the
+// second product wants them (the weights never leave the registers again), and each wave owns a quarter of the
+// head's entries of the output. A chunk's values are asked for before its scores are computed and the next chunk's keys after.
+// The sum of a chunk's weights is a fixed tree over the keys' numbers. A chunk that a column does not see leaves
+// it as it was, bit for bit, so a column's result is the same whatever tile it is in.
+// Bound by the chain of a chunk's steps in a workgroup (about 5 us a chunk of heads of 128, 4,096 keys 318); two prompts of 333 and
+// 230 tokens, 16 heads of 128 on 8, take 57 us and a decode step of them 36, where a wave a (token, head) with a
+// key a lane took 725 and 138 (1,683 at 4,096 keys).
 // In xigh/herbert-rs: scores q . k / sqrt(hd), query head h on kv head h / (nq / nkv)
 // (crates/backends/backend_common/src/generic_attention/decode.rs:126), causal by count
 // (crates/backends/backend_common/src/generic_attention/prefill/kernel_f32.rs:65-67), online softmax and
@@ -19,111 +30,252 @@
 // added (after the scale), n = min(i - j, bias_len - 1): a bias by distance, the last value from there on; and with
 // keep_first > 0 (and a window) the sequence's first so many keys are seen as well.
 #include "common.h"
+#include "mfma_f32.h"
 #include <math.h>
 
 HB_MODULE_ERROR_SLOT()
 
 #define HB_MAX_HEAD_DIM 512
-#define ACC_REGS (HB_MAX_HEAD_DIM / HB_WAVE)
+#define CHUNK 64
 
-template <class TQ, class TC, class TO>
-__global__ void __launch_bounds__(HB_WAVE)
-attention_plain_kernel(const TQ* __restrict__ q, const TC* __restrict__ k_cache,
-                       const TC* __restrict__ v_cache, TO* __restrict__ out,
+// What a query row sees: keys [lo, hi) and [0, kept).
+struct Seen {
+    int lo, hi, kept;
+};
+__device__ __forceinline__ Seen seen_by(int pos, int window, int chunk, int keep_first) {
+    Seen s;
+    s.hi = pos + 1;
+    s.lo = chunk > 0 ? pos / chunk * chunk : (window > 0 && s.hi > window) ? s.hi - window : 0;
+    s.kept = keep_first < s.lo ? keep_first : s.lo;
+    return s;
+}
+
+// NB: blocks of 16 of the head's entries that a wave owns of the output (the head has up to 64 NB entries). VEC: heads in
+// whole quads, rows aligned, and pages that hold whole chunks. AHEAD: the next chunk's keys and values are in flight
+// while a chunk is worked on (wide heads have no registers left for that).
+template <class T, class TO, int NB, bool VEC, bool AHEAD>
+__global__ void __launch_bounds__(256)
+attention_plain_kernel(const T* __restrict__ q, const T* __restrict__ k_cache,
+                       const T* __restrict__ v_cache, TO* __restrict__ out,
                        const int* __restrict__ positions, const int* __restrict__ seq_of,
                        const int* __restrict__ slots, const int* __restrict__ page_table, int max_pages,
-                       int page_size, int nq, int nkv, int hd, float scale, int window,
+                       int page_size, int n_tokens, int nq, int nkv, int hd, float scale, int window,
                        const float* __restrict__ sinks, int chunk, float softcap, const float* __restrict__ bias,
-                       int bias_ld, int bias_at, int bias_len, int keep_first) {
-    __shared__ float qs[HB_MAX_HEAD_DIM];
-    __shared__ float ps[HB_WAVE];
-    const int t = blockIdx.x;
-    const int h = blockIdx.y;
-    const int lane = threadIdx.x;
-    const int g = h / (nq / nkv);
-    const int pos = positions[t];
-    const int slot = slots[seq_of[t]];
-    const int* pt = page_table + (size_t)slot * max_pages;
+                       int bias_ld, int bias_at, int bias_len, int keep_first, int heads_a_tile, int tokens_a_tile) {
+    constexpr int DB = 4 * NB;                       // blocks of 16 entries of a head
+    constexpr int QLD = 16 * DB + 4, SLD = CHUNK + 4;
+    __shared__ __attribute__((aligned(16))) float qs[16 * QLD], ss[16 * SLD];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int r = lane & 15, g4 = lane >> 4;
+    const int group = nq / nkv, tiles_a_head = (group + heads_a_tile - 1) / heads_a_tile;
+    const int g = blockIdx.y / tiles_a_head, h_first = blockIdx.y % tiles_a_head * heads_a_tile;
+    const int t0 = blockIdx.x * tokens_a_tile;
+    const int n_here = n_tokens - t0 < tokens_a_tile ? n_tokens - t0 : tokens_a_tile;
 
-    const TQ* qrow = q + ((size_t)t * nq + h) * hd;
-    for (int d = lane; d < hd; d += HB_WAVE) qs[d] = hb_to_float(qrow[d]);
-    __syncthreads();
-
-    const int hi = pos + 1;
-    const int lo = chunk > 0 ? pos / chunk * chunk : (window > 0 && hi > window) ? hi - window : 0;
+    // the queries, zeros beyond the head's entries and in columns that are nobody's, every 16 entries transposed
+    for (int i = tid; i < 16 * 16 * DB; i += 256) {
+        const int c = i / (16 * DB), d = i % (16 * DB);
+        const int tok = c / heads_a_tile, head = h_first + c % heads_a_tile;
+        float v = 0.f;
+        if (tok < n_here && head < group && d < hd) v = hb_to_float(q[((size_t)(t0 + tok) * nq + g * group + head) * hd + d]);
+        qs[c * QLD + (d & ~15) + 4 * (d & 3) + ((d >> 2) & 3)] = v;
+    }
+    // this lane's column
+    const int my_tok = r / heads_a_tile, my_head = h_first + r % heads_a_tile;
+    const bool mine = my_tok < n_here && my_head < group;
+    const int h = g * group + (mine ? my_head : 0);
+    const int pos = positions[t0 + (mine ? my_tok : 0)];
+    const Seen see = seen_by(pos, window, chunk, keep_first);
     float m = -INFINITY, l = 0.f;
     if (sinks) m = sinks[h], l = 1.0f;
-    float acc[ACC_REGS];
+    f32x4 acc[NB];
 #pragma unroll
-    for (int i = 0; i < ACC_REGS; ++i) acc[i] = 0.f;
+    for (int i = 0; i < NB; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    __syncthreads();
 
-    // chunks: those that hold a kept first key, then those from the window's first key on
-    const int kept = keep_first < lo ? keep_first : lo;
-    int first = (lo / HB_WAVE) * HB_WAVE;
-    if (kept > 0) first = 0;
-    for (int c = first; c < hi; c += HB_WAVE) {
-        if (c >= kept && c + HB_WAVE <= lo) {
-            c = (lo / HB_WAVE) * HB_WAVE;
+    // runs of the tile's tokens that belong to one sequence (a prompt's tile has mostly one)
+    for (int first = 0; first < n_here;) {
+        const int seq = seq_of[t0 + first];
+        int last = first + 1;
+        while (last < n_here && seq_of[t0 + last] == seq) ++last;
+        const int* pt = page_table + (size_t)slots[seq] * max_pages;
+        const bool in_run = mine && my_tok >= first && my_tok < last;
+        // what the run's tokens see together
+        Seen all = seen_by(positions[t0 + first], window, chunk, keep_first);
+        for (int i = first + 1; i < last; ++i) {
+            const Seen s = seen_by(positions[t0 + i], window, chunk, keep_first);
+            all.lo = min(all.lo, s.lo), all.hi = max(all.hi, s.hi), all.kept = max(all.kept, s.kept);
         }
-        const int j = c + lane;
-        const bool valid = (j >= lo || j < kept) && j < hi;
-        float s = -INFINITY;
-        if (valid) {
-            const int page = pt[j / page_size];
-            const TC* kr = k_cache + (((size_t)page * nkv + g) * page_size + (j % page_size)) * hd;
-            float dot = 0.f;
-            for (int d = 0; d < hd; ++d) dot = fmaf(qs[d], hb_to_float(kr[d]), dot);
-            s = dot * scale;
-            if (softcap > 0.f) s = softcap * tanhf(s / softcap);
-            if (bias) {
-                const int n = pos - j < bias_len - 1 ? pos - j : bias_len - 1;
-                s += bias[(size_t)h * bias_ld + bias_at + bias_len - 1 - n];
-            }
-        }
-        const float m_new = fmaxf(m, hb_wave_max(s));
-        const float corr = expf(m - m_new);
-        const float p = valid ? expf(s - m_new) : 0.f;
-        l = l * corr + hb_wave_sum(p);
-        m = m_new;
-        __syncthreads();
-        ps[lane] = p;
-        __syncthreads();
-        const int jj0 = lo > c && c >= kept ? lo - c : 0;      // (a hidden key's weight is zero)
-        const int jj1 = hi - c < HB_WAVE ? hi - c : HB_WAVE;
+        first = last;
+        auto next_of = [&](int c) {        // the chunk after c - CHUNK that some token sees
+            return c >= all.kept && c + CHUNK <= all.lo ? all.lo / CHUNK * CHUNK : c;
+        };
+        // (keys from all.hi on are the last key once more; a table's entries are pages that exist)
+        f32x4 key[DB], val_next[AHEAD ? NB : 1][4];
+        auto fetch_keys = [&](int c, int page) {
+            const int j = min(c + 16 * wave + r, all.hi - 1);
+            const int in_page = VEC ? c % page_size + j - c : j % page_size;
+            const T* row = k_cache + (((size_t)(VEC ? page : pt[j / page_size]) * nkv + g) * page_size + in_page) * hd + 4 * g4;
 #pragma unroll
-        for (int i = 0; i < ACC_REGS; ++i) acc[i] *= corr;
-        for (int jj = jj0; jj < jj1; ++jj) {
-            const int jv = c + jj;
-            const int page = pt[jv / page_size];
-            // values are stored transposed: [page, kv head, hd, token]
-            const TC* vr = v_cache + ((size_t)page * nkv + g) * page_size * hd + (jv % page_size);
-            const float pj = ps[jj];
+            for (int b = 0; b < DB; ++b) key[b] = load_quad<VEC>(row + 16 * b, hd - 16 * b - 4 * g4);
+        };
+        auto fetch_values = [&](int c, int page, int i, f32x4 (&to)[4]) {       // of the wave's i-th block of entries
+            const T* at = v_cache + ((size_t)page * nkv + g) * hd * page_size + c % page_size + 4 * g4;
+            const int d = 16 * (wave + 4 * i) + r;
 #pragma unroll
-            for (int i = 0; i < ACC_REGS; ++i) {
-                const int d = lane + HB_WAVE * i;
-                if (d < hd) acc[i] = fmaf(pj, hb_to_float(vr[(size_t)d * page_size]), acc[i]);
+            for (int b = 0; b < 4; ++b) {
+                to[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+                const int j = c + 16 * b + 4 * g4;
+                if (VEC) {
+                    if (d < hd && j < all.hi) to[b] = load_quad<true>(at + (size_t)d * page_size + 16 * b, 4);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (d < hd && j + e < all.hi)
+                            to[b][e] = hb_to_float(v_cache[(((size_t)pt[(j + e) / page_size] * nkv + g) * hd + d) * page_size + (j + e) % page_size]);
+                }
             }
+        };
+        int c = next_of(all.kept > 0 ? 0 : all.lo / CHUNK * CHUNK);
+        int following = next_of(c + CHUNK);
+        // (the page after the next is looked up a chunk before its loads are asked for)
+        int page = pt[c / page_size], page_next = following < all.hi ? pt[following / page_size] : 0;
+        fetch_keys(c, page);
+        if (AHEAD) {
+#pragma unroll
+            for (int i = 0; i < NB; ++i) fetch_values(c, page, i, val_next[i]);
         }
+        while (c < all.hi) {
+            f32x4 val[AHEAD ? NB : 1][4];
+            if (AHEAD) {
+#pragma unroll
+                for (int i = 0; i < NB; ++i)
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) val[i][b] = val_next[i][b];
+            }
+            f32x4 dots = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int b = 0; b < DB; ++b) {
+                transpose_quads(key[b]);
+                const f32x4 qq = *(const f32x4*)&qs[r * QLD + 16 * b + 4 * g4];
+#pragma unroll
+                for (int s = 0; s < 4; ++s) dots = mfma_k4(key[b][s], qq[s], dots);
+            }
+            const int after = next_of(following + CHUNK);
+            const int page_after = after < all.hi ? pt[after / page_size] : 0;
+            if (AHEAD && following < all.hi) {
+                fetch_keys(following, page_next);
+#pragma unroll
+                for (int i = 0; i < NB; ++i) fetch_values(following, page_next, i, val_next[i]);
+            }
+            __syncthreads();                              // (the chunk before has been read)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int j = c + 16 * wave + 4 * g4 + e;
+                float s = dots[e] * scale;
+                if (softcap > 0.f) s = softcap * tanhf(s / softcap);
+                if (bias) {
+                    const int n = max(0, min(pos - j, bias_len - 1));
+                    s += bias[(size_t)h * bias_ld + bias_at + bias_len - 1 - n];
+                }
+                const bool valid = in_run && (j >= see.lo || j < see.kept) && j < see.hi;
+                ss[r * SLD + 16 * wave + 4 * e + g4] = valid ? s : -INFINITY;
+            }
+            __syncthreads();
+            // this lane's share of its column: keys 16 b + 4 s + g4
+            f32x4 p[4];
+            float top = -INFINITY;
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                p[b] = *(const f32x4*)&ss[r * SLD + 16 * b + 4 * g4];
+                top = fmaxf(top, fmaxf(fmaxf(p[b][0], p[b][1]), fmaxf(p[b][2], p[b][3])));
+            }
+            top = fmaxf(top, __shfl_xor(top, 16, HB_WAVE));
+            top = fmaxf(top, __shfl_xor(top, 32, HB_WAVE));
+            const bool sees = in_run && ((c < see.hi && c + CHUNK > see.lo) || c < see.kept);
+            float corr = 1.0f;
+            if (sees) {
+                const float m_new = fmaxf(m, top);
+                corr = expf(m - m_new);
+                m = m_new;
+            }
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+#pragma unroll
+                for (int s = 0; s < 4; ++s) p[b][s] = sees && p[b][s] != -INFINITY ? expf(p[b][s] - m) : 0.f;
+            // the tree: key j with j ^ 32, j ^ 16 (blocks), j ^ 8, j ^ 4 (quads), j ^ 2, j ^ 1 (lanes)
+            f32x4 t = (p[0] + p[2]) + (p[1] + p[3]);
+            float sum = (t[0] + t[2]) + (t[1] + t[3]);
+            sum += __shfl_xor(sum, 32, HB_WAVE);
+            sum += __shfl_xor(sum, 16, HB_WAVE);
+            l = l * corr + sum;
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                acc[i] *= corr;
+                f32x4 (&v)[4] = val[AHEAD ? i : 0];
+                if (!AHEAD) fetch_values(c, page, i, v);
+                // a value without a finite size, perhaps of a key that some column does not see: a weight of zero does
+                // not hide it
+                bool wild = false;
+#pragma unroll
+                for (int b = 0; b < 4; ++b)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        if (VEC && c + 16 * b + 4 * g4 + e >= all.hi) v[b][e] = 0.f;
+                        wild |= !(fabsf(v[b][e]) <= 3.4028235e38f);
+                    }
+                if (!__any(wild)) {
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) {
+                        transpose_quads(v[b]);
+#pragma unroll
+                        for (int s = 0; s < 4; ++s) acc[i] = mfma_k4(v[b][s], p[b][s], acc[i]);
+                    }
+                    continue;
+                }
+#pragma unroll
+                for (int b = 0; b < 4; ++b)
+                    for (int s = 0; s < 4; ++s)
+                        for (int k = 0; k < 4; ++k) {
+                            const int j = c + 16 * b + 4 * s + k;
+                            const float w = __shfl(s == 0 ? p[b][0] : s == 1 ? p[b][1] : s == 2 ? p[b][2] : p[b][3], 16 * k + r, HB_WAVE);
+                            if (j >= all.hi) continue;
+                            const T* v = v_cache + ((size_t)pt[j / page_size] * nkv + g) * hd * page_size + j % page_size;
+                            const bool valid = in_run && (j >= see.lo || j < see.kept) && j < see.hi;
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                const int d = 16 * (wave + 4 * i) + 4 * g4 + e;
+                                if (valid && d < hd) acc[i][e] = fmaf(w, hb_to_float(v[(size_t)d * page_size]), acc[i][e]);
+                            }
+                        }
+            }
+            if (!AHEAD && following < all.hi) fetch_keys(following, page_next);
+            c = following, following = after;
+            page = page_next, page_next = page_after;
+        }
+        __syncthreads();
     }
-
+    if (!mine) return;
     const float inv = l > 0.f ? 1.0f / l : 0.f;
-    TO* orow = out + ((size_t)t * nq + h) * hd;
+    TO* row = out + ((size_t)(t0 + my_tok) * nq + h) * hd;
 #pragma unroll
-    for (int i = 0; i < ACC_REGS; ++i) {
-        const int d = lane + HB_WAVE * i;
-        if (d < hd) orow[d] = hb_from_float<TO>(acc[i] * inv);
-    }
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int d = 16 * (wave + 4 * i) + 4 * g4 + e;
+            if (d < hd) row[d] = hb_from_float<TO>(acc[i][e] * inv);
+        }
 }
 
 // q, out: [T, nq * hd]; keys [pages, nkv, page_size, hd], values [pages, nkv, hd, page_size];
 // dtype covers q and cache, and out unless out_dtype says float32.
 extern "C" int hb_attention_plain(const void* q, const void* k_cache, const void* v_cache, void* out,
                                   int dtype, const int* positions, const int* seq_of, const int* slots,
-                                  const int* page_table, int max_pages, int page_size, int T, int nq,
+                                  const int* page_table, int max_pages, int page_size, int T, int n_seqs, int nq,
                                   int nkv, int hd, float scale, int window, const float* sinks,
                                   int chunk, float softcap, const float* bias, int bias_ld, int bias_at,
                                   int bias_len, int keep_first, int out_dtype, hipStream_t stream) {
-    HB_REQUIRE(T > 0 && nq > 0 && nkv > 0, "attention: empty input");
+    HB_REQUIRE(T > 0 && n_seqs > 0 && nq > 0 && nkv > 0, "attention: empty input");
     HB_REQUIRE(nq % nkv == 0, "attention: %d query heads not divisible by %d kv heads", nq, nkv);
     HB_REQUIRE(hd > 0 && hd <= HB_MAX_HEAD_DIM, "attention: head_dim %d not in 1..%d", hd,
                HB_MAX_HEAD_DIM);
@@ -133,24 +285,35 @@ extern "C" int hb_attention_plain(const void* q, const void* k_cache, const void
     HB_REQUIRE(!bias || (bias_len > 0 && bias_at >= 0 && bias_at + bias_len <= bias_ld), "attention: bad table of biases");
     HB_REQUIRE(nq <= 65535, "attention: too many heads for the grid");
     HB_REQUIRE(out_dtype == dtype || out_dtype == HB_F32, "attention: the output is stored as the cache is, or in float32");
-    dim3 grid(T, nq);
-    if (dtype == HB_BF16 && out_dtype == HB_F32)
-        attention_plain_kernel<bf16, bf16, float><<<grid, HB_WAVE, 0, stream>>>(
-            (const bf16*)q, (const bf16*)k_cache, (const bf16*)v_cache, (float*)out, positions, seq_of,
-            slots, page_table, max_pages, page_size, nq, nkv, hd, scale, window, sinks, chunk, softcap, bias,
-            bias_ld, bias_at, bias_len, keep_first);
-    else if (dtype == HB_F32)
-        attention_plain_kernel<float, float, float><<<grid, HB_WAVE, 0, stream>>>(
-            (const float*)q, (const float*)k_cache, (const float*)v_cache, (float*)out, positions, seq_of,
-            slots, page_table, max_pages, page_size, nq, nkv, hd, scale, window, sinks, chunk, softcap, bias,
-            bias_ld, bias_at, bias_len, keep_first);
-    else if (dtype == HB_BF16)
-        attention_plain_kernel<bf16, bf16, bf16><<<grid, HB_WAVE, 0, stream>>>(
-            (const bf16*)q, (const bf16*)k_cache, (const bf16*)v_cache, (bf16*)out, positions, seq_of,
-            slots, page_table, max_pages, page_size, nq, nkv, hd, scale, window, sinks, chunk, softcap, bias,
-            bias_ld, bias_at, bias_len, keep_first);
-    else
-        HB_REQUIRE(false, "attention: unknown dtype %d", dtype);
+    // a key head's query heads side by side; where there is room, and more tokens than sequences, several tokens
+    const int group = nq / nkv, heads_a_tile = group < 16 ? group : 16;
+    const int tokens_a_tile = T > n_seqs ? 16 / heads_a_tile : 1;
+    const int tiles_a_head = (group + heads_a_tile - 1) / heads_a_tile;
+    HB_REQUIRE((long long)nkv * tiles_a_head <= 65535, "attention: too many heads for the grid");
+    const dim3 grid((T + tokens_a_tile - 1) / tokens_a_tile, nkv * tiles_a_head);
+    const int size = dtype == HB_F32 ? 4 : 2;
+    const bool vec = hd % 4 == 0 && page_size % CHUNK == 0 && (uintptr_t)k_cache % (4 * size) == 0 && (uintptr_t)v_cache % (4 * size) == 0;
+#define HB_ATTENTION(TT, TO, NB, VEC)                                                                                 \
+    attention_plain_kernel<TT, TO, NB, VEC, (NB <= 2 && VEC)><<<grid, 256, 0, stream>>>(                                                \
+        (const TT*)q, (const TT*)k_cache, (const TT*)v_cache, (TO*)out, positions, seq_of, slots, page_table, max_pages, \
+        page_size, T, nq, nkv, hd, scale, window, sinks, chunk, softcap, bias, bias_ld, bias_at, bias_len, keep_first, \
+        heads_a_tile, tokens_a_tile)
+#define HB_ATTENTION_OF(TT, TO)                                                                                       \
+    do {                                                                                                              \
+        if (!vec && hd <= 64) HB_ATTENTION(TT, TO, 1, false);                                                         \
+        else if (!vec && hd <= 128) HB_ATTENTION(TT, TO, 2, false);                                                   \
+        else if (!vec) HB_ATTENTION(TT, TO, 8, false);                                                                \
+        else if (hd <= 64) HB_ATTENTION(TT, TO, 1, true);                                                             \
+        else if (hd <= 128) HB_ATTENTION(TT, TO, 2, true);                                                            \
+        else if (hd <= 256) HB_ATTENTION(TT, TO, 4, true);                                                            \
+        else HB_ATTENTION(TT, TO, 8, true);                                                                           \
+    } while (0)
+    if (dtype == HB_BF16 && out_dtype == HB_F32) HB_ATTENTION_OF(bf16, float);
+    else if (dtype == HB_F32) HB_ATTENTION_OF(float, float);
+    else if (dtype == HB_BF16) HB_ATTENTION_OF(bf16, bf16);
+    else HB_REQUIRE(false, "attention: unknown dtype %d", dtype);
+#undef HB_ATTENTION_OF
+#undef HB_ATTENTION
     HB_CHECK_LAUNCH("attention_plain");
     return 0;
 }

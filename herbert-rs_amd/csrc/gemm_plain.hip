@@ -12,10 +12,9 @@
 // In xigh/herbert-rs: crates/backends/backend_bf16/src/kernels.rs:154-164 (float32 sums over k ascending of
 // x[m, k] * float(w[n, k]), no bias); crates/backends/backend_vulkan/shaders/bf16_matmul.comp:31-60.
 #include "common.h"
+#include "mfma_f32.h"
 
 HB_MODULE_ERROR_SLOT()
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // What a product may do to a sum before it stores it: nothing (rate null), or turn the pre-activation of a
 // decay into the decay itself, exp(-exp(rate[n / D]) * softplus(sum + bias[n])) for column n (float32; the
@@ -36,42 +35,6 @@ __device__ __forceinline__ float decay_of(const DecayEpilogue& ep, float sum, in
     }
     const float softplus = a > 20.f ? a : log1pf(expf(a));
     return expf(-expf(ep.rate[n / ep.D]) * softplus);
-}
-
-// One 16 x 16 x 4 product: w is W[n = lane % 16, k], a is A[m = lane % 16, k], both for k = k0 + lane / 16; lane l's
-// four sums are those of n = 4 (l / 16) .. + 3 and m = l % 16.
-__device__ __forceinline__ f32x4 mfma_k4(float w, float a, f32x4 sums) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(w, a, sums, 0, 0, 0);
-}
-
-// Four neighbouring elements of a row as float32 (16 or 8 bytes, aligned), or what lies below `left` of them.
-template <bool VEC>
-__device__ __forceinline__ f32x4 load_quad(const float* p, int left) {
-    f32x4 r = {0.f, 0.f, 0.f, 0.f};
-    if (VEC) {
-        if (left > 0) r = *(const f32x4*)p;
-        return r;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        if (i < left) r[i] = p[i];
-    return r;
-}
-template <bool VEC>
-__device__ __forceinline__ f32x4 load_quad(const bf16* p, int left) {
-    f32x4 r = {0.f, 0.f, 0.f, 0.f};
-    if (VEC) {
-        if (left > 0) {
-            const uint2 u = *(const uint2*)p;
-            r[0] = __uint_as_float(u.x << 16), r[1] = __uint_as_float(u.x & 0xffff0000u);
-            r[2] = __uint_as_float(u.y << 16), r[3] = __uint_as_float(u.y & 0xffff0000u);
-        }
-        return r;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        if (i < left) r[i] = hb_to_float(p[i]);
-    return r;
 }
 
 // What a lane holds of one output column's four neighbouring rows n .. n + 3 into C[m, n ..].
@@ -191,26 +154,6 @@ gemm_plain_tile_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
         for (int j = 0; j < NB; ++j)
             store_quad<TC, ACCUM, VEC>(C, ldc, m, n0 + wn + 16 * j + 4 * q, N, acc[j][i], ep);
     }
-}
-
-// Four quads, one a lane row of 16 (lane / 16), transposed in registers: x[i] of lane row q was element 4 q + i of 16
-// and becomes element 4 i + q, which is what the i-th of four products wants of that lane row.
-__device__ __forceinline__ void transpose_quads(f32x4& x) {
-    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-    auto halves = [](float& a, float& b) {
-        const u32x2 t = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-        a = __uint_as_float(t[0]), b = __uint_as_float(t[1]);
-    };
-    auto rows = [](float& a, float& b) {
-        const u32x2 t = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-        a = __uint_as_float(t[0]), b = __uint_as_float(t[1]);
-    };
-    float x0 = x[0], x1 = x[1], x2 = x[2], x3 = x[3];
-    halves(x0, x2);
-    halves(x1, x3);
-    rows(x0, x1);
-    rows(x2, x3);
-    x[0] = x0, x[1] = x1, x[2] = x2, x[3] = x3;
 }
 
 // Up to 16 rows (a decode step): a product bound by the weights' bytes. A wave alone on 16 rows of W: no LDS and no

@@ -225,7 +225,7 @@ def attention_plain(q, meta, cache, out, nq, nkv, hd, scale, window, sinks=None,
     lib.call("attention_plain", "hb_attention_plain", q.data_ptr(), cache.k.data_ptr(),
              cache.v.data_ptr(), out.data_ptr(), dtype_code(q), meta.positions.data_ptr(),
              meta.seq_of.data_ptr(), meta.slots.data_ptr(), cache.page_table.data_ptr(),
-             cache.page_table.shape[1], cache.page_size, T, nq, nkv, hd, float(scale),
+             cache.page_table.shape[1], cache.page_size, T, meta.slots.shape[0], nq, nkv, hd, float(scale),
              int(window or 0), _ptr(sinks), int(chunk or 0), float(softcap or 0.0),
              None if bias is None else bias.rows.data_ptr(), 0 if bias is None else bias.rows.shape[1],
              0 if bias is None else bias.at, 0 if bias is None else bias.length, int(keep_first or 0), dtype_code(out), _stream())

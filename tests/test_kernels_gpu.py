@@ -319,6 +319,40 @@ def test_attention_plain(nq, nkv, hd, window, dtype):
     assert float((out.float().cpu() - want).abs().max()) <= tol * float(want.abs().max())
 
 
+@pytest.mark.parametrize("nq,nkv,hd", [(16, 8, 128), (4, 4, 64), (20, 1, 96), (2, 1, 300), (6, 2, 17)])
+def test_attention_plain_tiles_and_what_no_query_sees(nq, nkv, hd):
+    """The float32 attention's workgroups share chunks of keys between several tokens of a prompt, of one sequence or of
+    two that meet in a tile: a token's result is the same bits as alone (heads of one to 32 blocks of 16, of no whole
+    quad; groups of 1 to 20 query heads), and near a float32 reference. Keys and values that a query does not see
+    (those behind a sequence's end in its last page, and later tokens' own) may hold anything."""
+    from herbert_rs_amd.kernels import ops
+    lengths, new = [70, 3, 129, 200], [70, 3, 100, 1]
+    meta, kv, dense = paged_case(lengths, new, nkv, hd, torch.float32, seed=hd)
+    T, scale = sum(new), hd ** -0.5
+    q = rand(T, nq * hd, seed=21)
+    out = torch.empty_like(q)
+    ops.attention_plain(q, meta, kv, out, nq, nkv, hd, scale, 0)
+    want = attention_reference(q, meta, dense, nq, nkv, hd, scale, 0)
+    assert float((out.cpu() - want).abs().max()) <= 2e-5 * float(want.abs().max())
+    for t in (0, 5, 69, 70, 73, 74, 100, T - 1):            # alone: as many sequences as tokens
+        one = FakeMeta()
+        one.positions, one.seq_of = meta.positions[t:t + 1].clone(), torch.zeros(1, dtype=torch.int32, device=dev())
+        one.slots = meta.slots[int(meta.seq_of[t])][None].clone()
+        alone = torch.empty(1, nq * hd, device=dev())
+        ops.attention_plain(q[t:t + 1].contiguous(), one, kv, alone, nq, nkv, hd, scale, 0)
+        assert torch.equal(alone[0], out[t]), t
+    table = kv.page_table.cpu()
+    seen = out.clone()
+    for b, n in enumerate(lengths):                         # behind the ends of the sequences, and one later token's own
+        page = int(table[b + 1, (n - 1) // 64])
+        kv.k[page, :, (n - 1) % 64 + 1:] = float("nan")
+        kv.v[page, :, :, (n - 1) % 64 + 1:] = float("inf")
+    page = int(table[1, 0])
+    kv.k[page, :, 60], kv.v[page, :, :, 60] = float("nan"), float("nan")
+    ops.attention_plain(q, meta, kv, out, nq, nkv, hd, scale, 0)
+    assert torch.equal(out[:60], seen[:60]) and torch.equal(out[70:], seen[70:]) and bool(out[60:70].isnan().all())
+
+
 @pytest.mark.parametrize("tile_height", [32, 64])
 @pytest.mark.parametrize("nq,nkv,hd,window", [(4, 1, 128, 0), (8, 2, 64, 0), (6, 2, 32, 0), (5, 1, 64, 70),
                                               (3, 3, 128, 100), (16, 2, 128, 0), (2, 2, 32, 0)])
