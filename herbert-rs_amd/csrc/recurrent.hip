@@ -319,7 +319,7 @@ extern "C" int hb_lru_scan(const float* ug, float* gates, const float* rb, const
 //   S <- g S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q        (o sees the token's own write)
 // with g = exp(-exp(A_log[h]) * softplus(a + dt_bias[h])) and beta = sigmoid(b), a and b columns of
 // the projection's row. The columns of S never meet, and the tokens are a chain: the kernel is as
-// fast as one token's step is short. A column is held by LPC lanes (each 8 or 16 of its D numbers, in
+// fast as one token's step is short. (Portions of many tokens take recurrent_chunks.hip where it has their sizes.) A column is held by LPC lanes (each 8 or 16 of its D numbers, in
 // registers; LPC = 1 .. 16 for D up to 256), a wave holds 64 / LPC columns and walks the sequence's
 // tokens; a workgroup is one wave, so that a head's columns spread over many CUs. The two dot
 // products a token are summed over a column's lanes by exchanges within a row of 16 lanes (the first

@@ -1,0 +1,518 @@
+// The gated delta rule and the linear attention with a decay a key channel (recurrent.hip has the rules and the walk
+// token by token) for portions of many tokens: 64 tokens of a head at a time as float32 products on the matrix cores.
+// The walk is a chain of tokens, 0.38 us each whatever the GPU has free; here the chain is one of chunks.
+//
+// Within a chunk, with G_t the product of the decays up to token t (a vector over the key's entries), S_0 the state before it:
+//   u_t = beta_t (v_t - S_0^T (G_t k_t) - sum_(i<t) A_ti u_i),    A_ti = sum_d k_t k_i G_t / G_i
+//   o_t = S_0^T (G_t q_t) + sum_(i<=t) B_ti u_i,                  B_ti = sum_d q_t k_i G_t / G_i
+//   S   = G_64 S_0 + sum_i (G_64 / G_i k_i) u_i^T
+// so U = T (beta V) - T (beta G K) S_0 with T = (I + beta A)^-1, unit lower triangular. (The linear attention has u = v.)
+// No quotient of decays is ever formed: G_t / G_i is a product of the decays between, which can go to zero but not
+// beyond one. For pairs of tokens in different blocks of 16 it is split where the later block begins. Within a block
+// the pairs are taken in four levels, s = 1, 2, 4, 8: pairs whose halves of a run of 2 s tokens differ, split in the
+// middle of that run; the products over runs grow from level to level by one exchange between the lanes of 16 tokens.
+//
+// chunk_prepare_kernel: everything that does not need S_0, one workgroup a (chunk, head), all of them at once. It leaves
+// in scratch, as the operands that the second kernel's lanes load: G q, G_64 / G k, B, and -T beta G K and T beta V.
+// chunk_scan_kernel: the chain of chunks, one workgroup a (head, 16 columns of S): four waves, each 16 tokens of a
+// chunk (U and O) and a quarter of the state's rows (S).
+//
+// Sums over many k are taken as eight chains added in pairs, so that they round as the walk's sums over lanes do. Against 64
+// bits (random keys of unit length, three sequences of 65 to 200 tokens, the walk's error in brackets): 1.2e-7 (1.0e-7) with
+// decays spread over (0, 1), where most of an output is its own token's, 4.5e-7 (4.9e-7) with decays near one, a decay a
+// channel 1.1e-7 (1.0e-7) and 2.0e-7 (2.7e-7), the linear attention 1.0e-7 (0.8e-7) and 1.8e-7 (2.8e-7).
+//
+// 2,048 tokens of 16 heads of 128 x 128 take 190 us (the walk 793), with a decay a channel 198 (1,068), the linear attention
+// 139 (894); 8 sequences of 300 tokens 175 (450). Bound: the second kernel by its chain (112 products of 32 cycles a
+// chunk and wave and two exchanges through LDS), the first by its products, for which a (chunk, head) has one workgroup a CU.
+#include "common.h"
+#include "mfma_f32.h"
+#include <math.h>
+
+HB_MODULE_ERROR_SLOT()
+
+#define CHUNK 64
+
+// Where a (chunk, head)'s pieces lie in its part of the scratch, in floats.
+struct ChunkLayout {
+    int q, k, b, w, u, g, size;
+};
+__host__ __device__ inline ChunkLayout chunk_layout(int D, int V, bool delta) {
+    ChunkLayout l;
+    l.q = 0;                              // [4 blocks of tokens][D / 16][64 lanes][4]: G q, rows of tokens
+    l.k = l.q + CHUNK * D;                // [D / 16][4][64][4]: G_64 / G k, rows of key entries
+    l.b = l.k + CHUNK * D;                // [4][4][64][4]: B, rows of tokens
+    l.w = l.b + CHUNK * CHUNK;            // [4][D / 16][64][4]: -T beta G K, rows of tokens
+    l.u = l.w + (delta ? CHUNK * D : 0);  // [4][V / 16][64][4]: T beta V, as sums lie
+    l.g = l.u + (delta ? CHUNK * V : 0);  // [D]: G_64, then the first token that is not finite (64: none)
+    l.size = l.g + D + 4;
+    return l;
+}
+
+__device__ __forceinline__ int in_quads(int i) { return (i & ~15) + 4 * (i & 3) + ((i >> 2) & 3); }
+// A sum over many k as N chains that are added in pairs, so that it rounds as little as the walk's sums over lanes do.
+template <int N>
+struct Chains {
+    f32x4 part[N];
+    __device__ __forceinline__ Chains() {
+#pragma unroll
+        for (int i = 0; i < N; ++i) part[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    __device__ __forceinline__ void add(float w, float a, int i) { part[i % N] = mfma_k4(w, a, part[i % N]); }
+    __device__ __forceinline__ f32x4 sum() const {
+        f32x4 t[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) t[i] = part[i];
+#pragma unroll
+        for (int n = N / 2; n > 0; n /= 2)
+#pragma unroll
+            for (int i = 0; i < n; ++i) t[i] += t[i + n];
+        return t[0];
+    }
+};
+__device__ __forceinline__ bool not_finite(float v) { return !(fabsf(v) <= 3.4028235e38f); }
+
+template <int DB, bool CH, bool DELTA>
+__global__ void __launch_bounds__(256)
+chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restrict__ proj, int ld, int b_off, int a_off,
+                     const float* __restrict__ A_log, const float* __restrict__ dt_bias,
+                     const float* __restrict__ decay, const int* __restrict__ seq_starts, float* __restrict__ scratch,
+                     int kv_heads, int heads, int V, int c0, int span) {
+    constexpr int D = 16 * DB, KLD = D + 4, TLD = CHUNK + 4;
+    constexpr int NG = CH ? 4 * DB : 1;                       // decays a lane holds of its token
+    // columns' keys in the order their lanes read them, later G_64 / G k with a row a key entry
+    __shared__ __attribute__((aligned(16))) float cols[D * TLD];
+    __shared__ __attribute__((aligned(16))) float rows[CHUNK * (DELTA ? KLD : TLD)];     // B, later G k and -T beta G k
+    __shared__ __attribute__((aligned(16))) float lower[DELTA ? CHUNK * TLD : 4];        // beta A below the diagonal
+    __shared__ __attribute__((aligned(16))) float inverse[DELTA ? 4 * 16 * 20 : 4];      // of I + its diagonal blocks
+    __shared__ float total[4][CH ? D : 1];                    // a block's product of decays
+    __shared__ float betas[CHUNK];
+    __shared__ int wild_from;
+    const int h = blockIdx.y, seq = blockIdx.z;
+    const int first = seq_starts[seq] + (c0 + (int)blockIdx.x) * CHUNK;
+    const int n = min(CHUNK, seq_starts[seq + 1] - first);
+    if (n <= 0) return;
+    const ChunkLayout at = chunk_layout(D, V, DELTA);
+    float* out = scratch + (((size_t)seq * span + blockIdx.x) * heads + h) * at.size;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int r = lane & 15, q = lane >> 4;
+    const int kvh = h / (heads / kv_heads);
+    const int q_at = kvh * D, k_at = (kv_heads + kvh) * D, v_at = 2 * kv_heads * D + h * V;
+
+    // ---- this wave's 16 tokens: lane (r, q) holds entries 4 s + q of token r
+    const int token = 16 * wave + r;
+    bool real = token < n;
+    const float* row = qkv + (size_t)(first + (real ? token : 0)) * C;
+    f32x4 kq[DB], qq[DB];
+    float pre[NG], beta = 0.f;
+    bool wild = false;
+#pragma unroll
+    for (int b = 0; b < DB; ++b) {
+        kq[b] = load_quad<true>(row + k_at + 16 * b + 4 * q, 4);
+        qq[b] = load_quad<true>(row + q_at + 16 * b + 4 * q, 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) wild |= not_finite(kq[b][e]) | not_finite(qq[b][e]);
+    }
+    for (int v = 4 * q; v < V; v += 16) {
+        const f32x4 x = load_quad<true>(row + v_at + v, 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) wild |= not_finite(x[e]);
+    }
+    if (CH) {
+        const float* g = decay + ((size_t)(first + (real ? token : 0)) * heads + h) * D + 4 * q;
+#pragma unroll
+        for (int b = 0; b < DB; ++b) {
+            f32x4 x = load_quad<true>(g + 16 * b, 4);
+            transpose_quads(x);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) pre[4 * b + e] = x[e], wild |= not_finite(x[e]);
+        }
+    } else {
+        const float z = proj[(size_t)(first + (real ? token : 0)) * ld + a_off + h] + dt_bias[h];
+        pre[0] = expf(-expf(A_log[h]) * (z > 20.f ? z : log1pf(expf(z))));
+        wild |= not_finite(pre[0]);
+    }
+    if (DELTA) {
+        beta = 1.0f / (1.0f + expf(-proj[(size_t)(first + (real ? token : 0)) * ld + b_off + h]));
+        wild |= not_finite(beta);
+    }
+    if (tid == 0) wild_from = CHUNK;
+    __syncthreads();
+    if (real && wild) atomicMin(&wild_from, token);
+    __syncthreads();
+    // (tokens from one that is not finite on are left out here; the second kernel makes what comes of them not a number)
+    const int from = wild_from;
+    real = real && token < from;
+    float suf[NG];
+#pragma unroll
+    for (int i = 0; i < NG; ++i) pre[i] = real ? pre[i] : 1.0f, suf[i] = 1.0f;
+    if (!real) beta = 0.f;
+    if (q == 0) betas[token] = beta;
+    f32x4 part = {0.f, 0.f, 0.f, 0.f}, part2 = part;          // q . k of the token itself
+#pragma unroll
+    for (int b = 0; b < DB; ++b) {
+        if (!real) kq[b] = qq[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        transpose_quads(kq[b]);
+        transpose_quads(qq[b]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (b & 1) part2[e] = fmaf(qq[b][e], kq[b][e], part2[e]);
+            else part[e] = fmaf(qq[b][e], kq[b][e], part[e]);
+        }
+    }
+    part += part2;
+    float own = (part[0] + part[1]) + (part[2] + part[3]);
+    own += __shfl_xor(own, 16, HB_WAVE);
+    own += __shfl_xor(own, 32, HB_WAVE);
+
+    // ---- pairs within the block, level by level; sums lie as (later token 4 q + e, earlier token r)
+    f32x4 a_sum = {0.f, 0.f, 0.f, 0.f}, b_sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        if (4 * q + e == r) b_sum[e] = own;
+#pragma unroll
+    for (int level = 0; level < 4; ++level) {
+        const int s = 1 << level;
+        const bool late = (r / s) & 1;
+        Chains<8> ac, bc;
+#pragma unroll
+        for (int i = 0; i < 4 * DB; ++i) {
+            const float k = kq[i / 4][i % 4], p = pre[CH ? i : 0];
+            const float early_k = late ? 0.f : k * suf[CH ? i : 0];
+            if (DELTA) ac.add(late ? k * p : 0.f, early_k, i);
+            bc.add(late ? qq[i / 4][i % 4] * p : 0.f, early_k, i);
+        }
+        const f32x4 al = ac.sum(), bl = bc.sum();
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int t = 4 * q + e;
+            const bool pair = t / (2 * s) == r / (2 * s) && ((t / s) & 1) && !((r / s) & 1);
+            if (pair) a_sum[e] = al[e], b_sum[e] = bl[e];
+        }
+        // the products over runs of 2 s: up to a token from its run's start, and behind a token to its run's end
+        const int before = (lane & 48) + (r & ~(2 * s - 1)) + s - 1, after = before + s;
+#pragma unroll
+        for (int i = 0; i < NG; ++i) {
+            const float p = pre[i];
+            const float head = __shfl(p, before, HB_WAVE), tail = __shfl(p, after, HB_WAVE);
+            if (late) pre[i] = head * p;
+            else suf[i] *= tail;
+        }
+    }
+    if (CH) {
+        if (r == 15) {
+#pragma unroll
+            for (int i = 0; i < NG; ++i) total[wave][4 * i + q] = pre[i];
+        }
+    } else if (lane == 15) {
+        total[wave][0] = pre[0];
+    }
+#pragma unroll
+    for (int b = 0; b < DB; ++b) {
+        f32x4 k;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) k[e] = kq[b][e] * suf[CH ? 4 * b + e : 0];
+        *(f32x4*)&cols[((wave * DB + b) * 64 + lane) * 4] = k;
+    }
+    auto put = [&](f32x4 a, f32x4 b, int block) {             // sums of (16 wave + 4 q + e, 16 block + r)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int t = 16 * wave + 4 * q + e;
+            if (DELTA) lower[t * TLD + in_quads(16 * block + r)] = betas[t] * a[e];
+            rows[t * TLD + in_quads(16 * block + r)] = b[e];
+        }
+    };
+    put(a_sum, b_sum, wave);
+    __syncthreads();
+    if (DELTA) {
+        // the inverse of I + the diagonal block: column r of it, by substitution (the four lane rows do the same)
+        float x[16];
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            float v = t == r ? 1.0f : 0.0f;
+#pragma unroll
+            for (int i = 0; i < t; ++i) v = fmaf(-lower[(16 * wave + t) * TLD + in_quads(16 * wave + i)], x[i], v);
+            x[t] = v;
+        }
+#pragma unroll
+        for (int t = 0; t < 16; ++t)
+            if ((t & 3) == q) inverse[(16 * wave + t) * 20 + in_quads(r)] = x[t];
+    }
+    // ---- pairs with earlier blocks, from the nearest on: the rows' decays grow by a block's product at a time
+#pragma unroll
+    for (int b = 0; b < DB; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float p = pre[CH ? 4 * b + e : 0];
+            qq[b][e] *= p;
+        }
+    f32x4 gk[DELTA ? DB : 1];                                 // G k
+    if (DELTA) {
+#pragma unroll
+        for (int b = 0; b < DB; ++b)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) gk[b][e] = kq[b][e] * pre[CH ? 4 * b + e : 0];
+    }
+    for (int block = wave - 1; block >= 0; --block) {
+        Chains<8> ac, bc;
+#pragma unroll
+        for (int b = 0; b < DB; ++b) {
+            const f32x4 k = *(const f32x4*)&cols[((block * DB + b) * 64 + lane) * 4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (DELTA) ac.add(gk[b][e], k[e], 4 * b + e);
+                bc.add(qq[b][e], k[e], 4 * b + e);
+                const float p = CH ? total[block][16 * b + 4 * e + q] : total[block][0];
+                qq[b][e] *= p;
+                if (DELTA) gk[b][e] *= p;
+            }
+        }
+        put(ac.sum(), bc.sum(), block);
+    }
+#pragma unroll
+    for (int b = 0; b < DB; ++b) *(f32x4*)(out + at.q + ((wave * DB + b) * 64 + lane) * 4) = qq[b];
+    // behind a token to the chunk's end
+    for (int block = wave + 1; block < 4; ++block) {
+#pragma unroll
+        for (int i = 0; i < NG; ++i) suf[i] *= CH ? total[block][4 * i + q] : total[block][0];
+    }
+    // (blocks above the diagonal are never read: a token's row of B goes out up to its own block)
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+        if (b <= wave)
+            *(f32x4*)(out + at.b + ((wave * 4 + b) * 64 + lane) * 4) = *(const f32x4*)&rows[(16 * wave + r) * TLD + 16 * b + 4 * q];
+    if (CH) {
+        for (int d = tid; d < D; d += 256) out[at.g + d] = total[0][d] * total[1][d] * total[2][d] * total[3][d];
+    } else {
+        for (int d = tid; d < D; d += 256) out[at.g + d] = total[0][0] * total[1][0] * total[2][0] * total[3][0];
+    }
+    if (tid == 0) ((int*)out)[at.g + D] = from;
+    __syncthreads();                                          // cols and rows have been read
+#pragma unroll
+    for (int b = 0; b < DB; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int d = 16 * b + 4 * e + q;
+            cols[d * TLD + in_quads(token)] = kq[b][e] * suf[CH ? 4 * b + e : 0];
+            if (DELTA) rows[token * KLD + in_quads(d)] = gk[b][e];
+        }
+    __syncthreads();
+#pragma unroll
+    for (int b = wave; b < DB; b += 4)
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            *(f32x4*)(out + at.k + ((b * 4 + s) * 64 + lane) * 4) = *(const f32x4*)&cols[(16 * b + r) * TLD + 16 * s + 4 * q];
+    if (!DELTA) return;
+
+    // ---- T applied to [beta G K | beta V], 16 columns at a time, block by block of tokens
+    for (int cb = wave; cb < DB + V / 16; cb += 4) {
+        const bool of_k = cb < DB;
+        f32x4 x[4];                                           // solved blocks, as the products want them
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            f32x4 acc;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int t = 16 * i + 4 * q + e;
+                float v = 0.f;
+                if (of_k) v = rows[t * KLD + in_quads(16 * cb + r)];
+                else if (t < n && t < from) v = qkv[(size_t)(first + t) * C + v_at + 16 * (cb - DB) + r];
+                acc[e] = betas[t] * v;
+            }
+            if (i > 0) {
+                Chains<8> before;
+#pragma unroll
+                for (int j = 0; j < i; ++j) {
+                    const f32x4 l = *(const f32x4*)&lower[(16 * i + r) * TLD + 16 * j + 4 * q];
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) before.add(l[s], x[j][s], 4 * j + s);
+                }
+                acc -= before.sum();
+            }
+            transpose_quads(acc);
+            const f32x4 inv = *(const f32x4*)&inverse[(16 * i + r) * 20 + 4 * q];
+            Chains<4> with;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) with.add(inv[s], acc[s], s);
+            const f32x4 solved = with.sum();
+            if (of_k) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) rows[(16 * i + 4 * q + e) * KLD + in_quads(16 * cb + r)] = -solved[e];
+            } else {
+                *(f32x4*)(out + at.u + ((i * (V / 16) + cb - DB) * 64 + lane) * 4) = solved;
+            }
+            x[i] = solved;
+            transpose_quads(x[i]);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < DB; ++b)
+        *(f32x4*)(out + at.w + ((wave * DB + b) * 64 + lane) * 4) = *(const f32x4*)&rows[(16 * wave + r) * KLD + 16 * b + 4 * q];
+}
+
+template <int DB, bool DELTA>
+__global__ void __launch_bounds__(256)
+chunk_scan_kernel(const float* __restrict__ qkv, int C, const float* __restrict__ scratch, float* __restrict__ state,
+                  const int* __restrict__ seq_starts, const int* __restrict__ slots, float* __restrict__ out,
+                  int kv_heads, int heads, int V, int c0, int span, float out_scale) {
+    constexpr int D = 16 * DB, OWN = DB / 4;                  // blocks of 16 of the state's rows a wave owns
+    constexpr int SLD = D + 4, ULD = CHUNK + 4;
+    __shared__ __attribute__((aligned(16))) float s_lds[2][16 * SLD], u_lds[2][16 * ULD];
+    const int h = blockIdx.x, vb = blockIdx.y, seq = blockIdx.z;
+    const int begin = seq_starts[seq], n_all = seq_starts[seq + 1] - begin;
+    const int last = min(c0 + span, (n_all + CHUNK - 1) / CHUNK);
+    if (c0 >= last) return;
+    const ChunkLayout at = chunk_layout(D, V, DELTA);
+    const float* part = scratch + ((size_t)seq * span * heads + h) * at.size;
+    const size_t chunk_step = (size_t)heads * at.size;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int r = lane & 15, q = lane >> 4;
+    const int col = 16 * vb + r;
+    float* S_mem = state + ((size_t)slots[seq] * heads + h) * D * V + col;
+    f32x4 S[OWN];
+    auto share = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < OWN; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s_lds[buf][r * SLD + 16 * (wave + 4 * i) + 4 * e + q] = S[i][e];
+    };
+#pragma unroll
+    for (int i = 0; i < OWN; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[i][e] = S_mem[(size_t)(16 * (wave + 4 * i) + 4 * q + e) * V];
+    share(0);
+
+    struct Operands {
+        f32x4 w[DELTA ? DB : 1], qg[DB], b[4], k[OWN][4], u;
+        float g[OWN][4], v[DELTA ? 1 : 16];
+        int from;
+    };
+    auto fetch = [&](int c, Operands& o) {
+        const float* p = part + (size_t)(c - c0) * chunk_step;
+#pragma unroll
+        for (int b = 0; b < DB; ++b) {
+            if (DELTA) o.w[b] = *(const f32x4*)(p + at.w + ((wave * DB + b) * 64 + lane) * 4);
+            o.qg[b] = *(const f32x4*)(p + at.q + ((wave * DB + b) * 64 + lane) * 4);
+        }
+        if (DELTA) o.u = *(const f32x4*)(p + at.u + ((wave * (V / 16) + vb) * 64 + lane) * 4);
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+            if (b <= wave) o.b[b] = *(const f32x4*)(p + at.b + ((wave * 4 + b) * 64 + lane) * 4);
+#pragma unroll
+        for (int i = 0; i < OWN; ++i)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                o.k[i][s] = *(const f32x4*)(p + at.k + (((wave + 4 * i) * 4 + s) * 64 + lane) * 4);
+                o.g[i][s] = p[at.g + 16 * (wave + 4 * i) + 4 * q + s];
+            }
+        o.from = ((const int*)p)[at.g + D];
+        if (!DELTA) {
+            const int n = n_all - c * CHUNK;
+            const float* v = qkv + (size_t)(begin + c * CHUNK) * C + 2 * kv_heads * D + h * V + col;
+#pragma unroll
+            for (int s = 0; s < 16; ++s) o.v[s] = 4 * s + q < n ? v[(size_t)(4 * s + q) * C] : 0.f;
+        }
+    };
+    Operands next;
+    fetch(c0, next);
+    __syncthreads();
+    int buf = 0;
+    for (int c = c0; c < last; ++c, buf ^= 1) {
+        const Operands o = next;
+        if (c + 1 < last) fetch(c + 1, next);
+        Chains<8> uc, oc;
+#pragma unroll
+        for (int b = 0; b < DB; ++b) {
+            const f32x4 s = *(const f32x4*)&s_lds[buf][r * SLD + 16 * b + 4 * q];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (DELTA) uc.add(o.w[b][e], s[e], 4 * b + e);
+                oc.add(o.qg[b][e], s[e], 4 * b + e);
+            }
+        }
+        f32x4 us[4];
+        if (DELTA) {
+            const f32x4 u = o.u + uc.sum();
+#pragma unroll
+            for (int e = 0; e < 4; ++e) u_lds[buf][r * ULD + 16 * wave + 4 * e + q] = u[e];
+            __syncthreads();
+#pragma unroll
+            for (int b = 0; b < 4; ++b) us[b] = *(const f32x4*)&u_lds[buf][r * ULD + 16 * b + 4 * q];
+        } else {
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) us[b][e] = 16 * b + 4 * e + q < o.from ? o.v[4 * b + e] : 0.f;
+        }
+#pragma unroll
+        for (int i = 0; i < OWN; ++i) {
+            Chains<8> kc;
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) kc.add(o.k[i][b][e], us[b][e], 4 * b + e);
+            const f32x4 added = kc.sum();
+#pragma unroll
+            for (int e = 0; e < 4; ++e) S[i][e] = fmaf(S[i][e], o.g[i][e], added[e]);
+            if (o.from < CHUNK) S[i] = f32x4{NAN, NAN, NAN, NAN};
+        }
+        share(buf ^ 1);
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+            if (b <= wave) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) oc.add(o.b[b][e], us[b][e], 4 * b + e);
+            }
+        const f32x4 sums = oc.sum();
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int t = 16 * wave + 4 * q + e, at_token = c * CHUNK + t;
+            if (at_token < n_all)
+                out[(size_t)(begin + at_token) * heads * V + h * V + col] = t < o.from ? sums[e] * out_scale : NAN;
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < OWN; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S_mem[(size_t)(16 * (wave + 4 * i) + 4 * q + e) * V] = S[i][e];
+}
+
+// As hb_gated_delta of recurrent.hip, for keys of 64 or 128 and values in steps of 16, rows in whole quads. scratch holds
+// B x span x heads parts of chunk_floats (chunk_layout's size); longest: the most tokens that a sequence of the step brings. Sequences
+// longer than span chunks go through in several pairs of launches, their state carried in `state`.
+extern "C" int hb_chunked_delta(const float* qkv, int C, const float* proj, int ld, int b_off, int a_off, const float* A_log,
+                                const float* dt_bias, const float* decay, float* state, const int* seq_starts,
+                                const int* slots, float* out, float* scratch, int B, int kv_heads, int heads, int D,
+                                int V, int correction, float out_scale, int longest, int span, int chunk_floats,
+                                hipStream_t stream) {
+    HB_REQUIRE(correction || decay, "linear attention: a decay a key channel must be given");
+    HB_REQUIRE(B > 0 && longest > 0 && span > 0 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0, "delta rule: %d heads on %d key heads", heads, kv_heads);
+    HB_REQUIRE((D == 64 || D == 128) && V > 0 && V % 16 == 0, "delta rule in chunks: keys of %d, values of %d", D, V);
+    HB_REQUIRE(C >= 2 * kv_heads * D + heads * V && C % 4 == 0 && (uintptr_t)qkv % 16 == 0 && (uintptr_t)decay % 16 == 0 &&
+               (uintptr_t)scratch % 16 == 0, "delta rule in chunks: rows of %d are not in whole quads", C);
+    HB_REQUIRE(chunk_floats == chunk_layout(D, V, correction != 0).size,
+               "delta rule in chunks: a part of %d floats is not the kernel's layout", chunk_floats);
+    HB_REQUIRE(B <= 65535 && heads <= 65535 && V / 16 <= 65535, "delta rule: too many sequences or heads for the grid");
+    const int chunks = (longest + CHUNK - 1) / CHUNK;
+    for (int c0 = 0; c0 < chunks; c0 += span) {
+        const dim3 grid(span < chunks - c0 ? span : chunks - c0, heads, B), scan(heads, V / 16, B);
+#define HB_CHUNKS(DB, CH, DELTA)                                                                                      \
+    do {                                                                                                              \
+        chunk_prepare_kernel<DB, CH, DELTA><<<grid, 256, 0, stream>>>(qkv, C, proj, ld, b_off, a_off, A_log, dt_bias,  \
+            decay, seq_starts, scratch, kv_heads, heads, V, c0, span);                                                \
+        chunk_scan_kernel<DB, DELTA><<<scan, 256, 0, stream>>>(qkv, C, scratch, state, seq_starts, slots, out,        \
+            kv_heads, heads, V, c0, span, out_scale);                                                                 \
+    } while (0)
+        if (D == 128 && !correction) HB_CHUNKS(8, true, false);
+        else if (D == 128 && decay) HB_CHUNKS(8, true, true);
+        else if (D == 128) HB_CHUNKS(8, false, true);
+        else if (!correction) HB_CHUNKS(4, true, false);
+        else if (decay) HB_CHUNKS(4, true, true);
+        else HB_CHUNKS(4, false, true);
+#undef HB_CHUNKS
+        HB_CHECK_LAUNCH("chunked_delta");
+    }
+    return 0;
+}

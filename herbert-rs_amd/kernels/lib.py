@@ -63,6 +63,9 @@ SIGNATURES = {
         "hb_gated_head_norm": [_P, _P, _I, _I, _P, _P, _I, _I, _I, _I, _F, _I, _P],
         "hb_channel_decay": [_P, _I, _P, _P, _P, _I, _I, _I, _P],
     },
+    "recurrent_chunks": {
+        "hb_chunked_delta": [_P, _I, _P, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _I, _I, _P],
+    },
     "attention_latent": {
         "hb_latent_write": [_P, _I, _P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I, _P, _I,
                             _P, _P, _P],

@@ -87,15 +87,50 @@ def gated_group_norm(o, proj, z_off, weight, out, parts, eps):
              weight.data_ptr(), out.data_ptr(), dtype_code(out), T, width, int(parts), float(eps), _stream())
 
 
+# Portions of many tokens go through in chunks of CHUNK tokens (csrc/recurrent_chunks.hip), shorter ones token by token.
+CHUNK = 64
+# Scratch of one launch, in floats: longer prompts go through in several, their state carried from one to the next. (It
+# also stays below the 256 MB memory-side cache, from which the second kernel reads what the first has left.)
+CHUNK_SCRATCH = 48 << 20
+
+
+def chunk_floats(D, V, correction):
+    """Floats that a chunk of a head takes of the scratch (the kernel refuses another number)."""
+    return (3 if correction else 2) * CHUNK * D + CHUNK * CHUNK + (CHUNK * V if correction else 0) + D + 4
+
+
+def _takes_chunks(qkv, decay, meta, heads, D, V, correction):
+    """The walk takes 0.4 us a token of the longest portion while its waves fit the chip; the chunks 37 us (24 without the
+    correction) and 5 us a chunk. One sequence of 16 heads of 128: 96 tokens 43 us either way, 64 tokens 33 against 38
+    (without the correction 48 tokens: 28 against 25). With many sequences or heads the walk's waves wait for each other
+    and the chunks still fill the chip: 8 sequences of 64 tokens 108 against 57, of 32 tokens 60 against 55."""
+    least = 40 if meta.num_seqs * heads >= 128 else 96 if correction else 48
+    return (meta.max_new >= least and D in (64, 128) and V % 16 == 0 and qkv.shape[1] % 4 == 0
+            and qkv.data_ptr() % 16 == 0 and (decay is None or decay.data_ptr() % 16 == 0))
+
+
+def _chunked(rt, qkv, proj, b_off, a_off, a_log, dt_bias, decay, state, meta, out, kv_heads, heads, D, V, correction, out_scale):
+    size, chunks = chunk_floats(D, V, correction), -(-meta.max_new // CHUNK)
+    span = max(1, min(chunks, CHUNK_SCRATCH // (size * heads * meta.num_seqs)))
+    scratch = rt.buffer("delta_chunks", (meta.num_seqs * span * heads * size,), torch.float32)
+    lib.call("recurrent_chunks", "hb_chunked_delta", qkv.data_ptr(), qkv.shape[1], None if proj is None else proj.data_ptr(),
+             0 if proj is None else proj.shape[1], b_off, a_off, None if a_log is None else a_log.data_ptr(),
+             None if dt_bias is None else dt_bias.data_ptr(), None if decay is None else decay.data_ptr(), state.data_ptr(),
+             meta.seq_starts.data_ptr(), meta.slots.data_ptr(), out.data_ptr(), scratch.data_ptr(), meta.num_seqs, kv_heads,
+             heads, D, V, 1 if correction else 0, float(out_scale), int(meta.max_new), span, size, _stream())
+
+
 def gated_delta(qkv, proj, b_off, a_off, a_log, dt_bias, state, meta, out, kv_heads, heads, D, V, decay=None,
-                correction=True, out_scale=1.0):
+                correction=True, out_scale=1.0, rt=None):
     """The delta rule over every sequence of the step; qkv f32 [T, at least 2 kv_heads D + heads V] (queries,
     keys, values in a row's first columns), proj f32 [T, ld] with column b_off + h (beta's pre-activation) and a_off + h (the
     decay's), state f32 [slots, heads, D, V] advanced in place, out f32 [T, heads V].
     decay f32 [T, heads D]: a factor a key channel, as `channel_decay` leaves it; a_off, a_log and
     dt_bias are then not read (they may be None). correction False (a decay a key channel must be given):
     the linear attention S <- diag(decay) S + k v^T, o = S^T q; proj is then not read (it may be None).
-    out_scale: o is multiplied by it."""
+    out_scale: o is multiplied by it.
+    rt: a Runtime whose scratch buffers may be used: portions of many tokens then go through in chunks, which differs
+    from the walk token by token by float32 rounding."""
     T, C = qkv.shape
     if not correction:
         if decay is None:
@@ -108,6 +143,9 @@ def gated_delta(qkv, proj, b_off, a_off, a_log, dt_bias, state, meta, out, kv_he
         _check(meta.slots, "slots", torch.int32, (meta.num_seqs,))
         if heads % kv_heads or not 0 < D <= MAX_KEY_DIM or C < 2 * kv_heads * D + heads * V:
             raise BackendError(f"linear attention: {heads} heads on {kv_heads} key heads of {D} in rows of {C}")
+        if rt is not None and _takes_chunks(qkv, decay, meta, heads, D, V, False):
+            _chunked(rt, qkv, None, 0, 0, None, None, decay, state, meta, out, kv_heads, heads, D, V, False, out_scale)
+            return
         lib.call("recurrent", "hb_gated_delta", qkv.data_ptr(), C, None, 0, 0, 0, None, None, decay.data_ptr(),
                  state.data_ptr(), meta.seq_starts.data_ptr(), meta.slots.data_ptr(), out.data_ptr(), meta.num_seqs,
                  kv_heads, heads, D, V, 0, float(out_scale), _stream())
@@ -129,6 +167,10 @@ def gated_delta(qkv, proj, b_off, a_off, a_log, dt_bias, state, meta, out, kv_he
     _check(meta.slots, "slots", torch.int32, (meta.num_seqs,))
     if heads % kv_heads or not 0 < D <= MAX_KEY_DIM:
         raise BackendError(f"delta rule: {heads} heads on {kv_heads} key heads of {D}")
+    if rt is not None and _takes_chunks(qkv, decay, meta, heads, D, V, True):
+        _chunked(rt, qkv, proj, b_off, a_off, None if decay is not None else a_log, None if decay is not None else dt_bias,
+                 decay, state, meta, out, kv_heads, heads, D, V, True, out_scale)
+        return
     lib.call("recurrent", "hb_gated_delta", qkv.data_ptr(), C, proj.data_ptr(), ld, b_off, a_off,
              None if decay is not None else a_log.data_ptr(), None if decay is not None else dt_bias.data_ptr(),
              None if decay is None else decay.data_ptr(), state.data_ptr(), meta.seq_starts.data_ptr(),

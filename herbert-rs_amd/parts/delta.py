@@ -163,10 +163,10 @@ class GatedDelta(Part):
                 factors = rt.buffer("delta_decay", (T, self.decay_width), torch.float32)
                 recurrent.channel_decay(decay_rows, decay_off, self.a_log, self.dt_bias, factors, self.heads, self.dim)
             recurrent.gated_delta(qkv, proj, self.b_off, 0, None, None, state, ctx.meta, o,
-                                  self.kv_heads, self.heads, self.dim, self.vdim, decay=factors)
+                                  self.kv_heads, self.heads, self.dim, self.vdim, decay=factors, rt=rt)
         else:
             recurrent.gated_delta(qkv, decay_rows, self.b_off, decay_off, self.a_log, self.dt_bias, state, ctx.meta, o,
-                                  self.kv_heads, self.heads, self.dim, self.vdim)
+                                  self.kv_heads, self.heads, self.dim, self.vdim, rt=rt)
         gated = rt.buffer("delta_gated", (T, self.heads * self.vdim))
         recurrent.gated_head_norm(o, gate_rows, gate_off, self.norm_w, gated, self.heads, self.vdim, self.eps,
                                   gate=self.gate)

@@ -89,7 +89,7 @@ class DecayedLinearAttention(Part):
                                decay=("sigmoid_root", self.a2_bias, 1.0 / self.tau))
         o = rt.buffer("gla_o", (T, self.heads * self.vdim), torch.float32)
         recurrent.gated_delta(proj, None, 0, 0, None, None, state, ctx.meta, o, self.heads, self.heads, self.dim,
-                              self.vdim, decay=decay, correction=False, out_scale=self.dim ** -0.5)
+                              self.vdim, decay=decay, correction=False, out_scale=self.dim ** -0.5, rt=rt)
         gated = rt.buffer("gla_gated", (T, self.heads * self.vdim))
         recurrent.gated_head_norm(o, proj, self.g_off, self.norm_w, gated, self.heads, self.vdim, self.eps, gate="silu")
         self.o.forward(gated, x, accumulate=ctx.adds_to(x))

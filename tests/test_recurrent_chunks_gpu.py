@@ -1,0 +1,113 @@
+"""The delta rule and the linear attention in chunks of 64 tokens (csrc/recurrent_chunks.hip) against the rule token by token
+in float64: the edges of chunks and of their blocks of 16, several sequences, a head's keys shared, decays from one to zero, a
+state that is carried over several launches, and rows that are not finite."""
+import types
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def dev():
+    return torch.device("cuda", 0)
+
+
+def rule(q, k, v, beta, decay, S):
+    """q, k, decay [T, H, D], v [T, H, V], beta [T, H] or None, S [H, D, V]: (outputs, last state), token by token."""
+    out = []
+    for t in range(q.shape[0]):
+        S = S * decay[t][:, :, None]
+        u = v[t] if beta is None else beta[t][:, None] * (v[t] - (S * k[t][:, :, None]).sum(1))
+        S = S + k[t][:, :, None] * u[:, None, :]
+        out.append((S * q[t][:, :, None]).sum(1))
+    return torch.stack(out), S
+
+
+def step(lengths, kv_heads, heads, D, V, kind, rate, seed=0):
+    """A step of sequences of these lengths; kind "head" or "channel" (the delta rule's decay) or "linear"."""
+    g = torch.Generator().manual_seed(seed)
+    T, B, W = sum(lengths), len(lengths), 2 * kv_heads * D + heads * V + 4
+
+    def draw(*shape):
+        return torch.randn(*shape, generator=g)
+    qkv = draw(T, W if kind == "linear" else W - 4)        # (the linear attention reads the columns of a wider row)
+    for a in (0, kv_heads * D):
+        part = qkv[:, a:a + kv_heads * D].view(T, kv_heads, D)
+        part /= part.norm(dim=-1, keepdim=True)
+    proj, a_log, dt_bias = draw(T, 2 * heads + 3), 0.5 * draw(heads) + rate, 0.5 * draw(heads)
+    decay = torch.exp(-torch.exp(a_log)[:, None] * torch.nn.functional.softplus(draw(T, heads, D)))
+    if rate > 2:
+        decay[::5] = 0.0                                   # a memory that is dropped at once
+    starts = torch.tensor([0] + lengths).cumsum(0).to(torch.int32)
+    meta = types.SimpleNamespace(max_new=max(lengths), num_seqs=B, seq_starts=starts.to(dev()),
+                                 slots=torch.arange(B, 0, -1, dtype=torch.int32, device=dev()))
+    state = 0.3 * draw(B + 2, heads, D, V)
+    return qkv, proj, a_log, dt_bias, decay, state, meta
+
+
+def run(qkv, proj, a_log, dt_bias, decay, state, meta, kv_heads, heads, D, V, kind, out_scale=0.5):
+    from herbert_rs_amd.kernels import recurrent
+    from herbert_rs_amd.parts import Runtime
+    rt, T = Runtime(torch.float32, dev()), qkv.shape[0]
+    out, held = torch.full((T, heads * V), 7.0, device=dev()), state.to(dev())
+    d = None if kind == "head" else decay.reshape(T, heads * D).to(dev())
+    recurrent.gated_delta(qkv.to(dev()), None if kind == "linear" else proj.to(dev()), 0, heads, a_log.to(dev()),
+                          dt_bias.to(dev()), held, meta, out, kv_heads, heads, D, V, decay=d, correction=kind != "linear",
+                          out_scale=out_scale, rt=rt)
+    assert any(name == "delta_chunks" for name, _ in rt._buffers), "the step did not go through in chunks"
+    return out.cpu().view(T, heads, V), held.cpu()
+
+
+def expected(qkv, proj, a_log, dt_bias, decay, state, lengths, kv_heads, heads, D, V, kind, out_scale=0.5):
+    outs, states, at = [], state.double().clone(), 0
+    for b, n in enumerate(lengths):
+        rows = qkv[at:at + n].double()
+        rep = heads // kv_heads
+        q, k = (rows[:, a:a + kv_heads * D].view(n, kv_heads, D).repeat_interleave(rep, 1) for a in (0, kv_heads * D))
+        v = rows[:, 2 * kv_heads * D:2 * kv_heads * D + heads * V].view(n, heads, V)
+        p = proj[at:at + n].double()
+        beta = None if kind == "linear" else torch.sigmoid(p[:, :heads])
+        g = decay[at:at + n].double() if kind != "head" else torch.exp(
+            -torch.exp(a_log.double()) * torch.nn.functional.softplus(p[:, heads:2 * heads] + dt_bias.double()))[:, :, None].expand(n, heads, D)
+        slot = len(lengths) - b
+        o, states[slot] = rule(q, k, v, beta, g, states[slot])
+        outs.append(o * out_scale)
+        at += n
+    return torch.cat(outs), states
+
+
+@pytest.mark.parametrize("kind", ["head", "channel", "linear"])
+@pytest.mark.parametrize("rate", [-5.0, 0.0, 4.0])             # decays near one, spread over (0, 1), near zero and zero
+@pytest.mark.parametrize("lengths,kv_heads,heads,D,V", [([130], 2, 2, 128, 32), ([64, 1, 200, 16, 63], 2, 6, 64, 16), ([97, 129], 1, 4, 128, 48)])
+def test_chunks_follow_the_rule(lengths, kv_heads, heads, D, V, kind, rate, monkeypatch):
+    """Outputs and the state left, once in one pair of launches and once in several. float32 sums of up to 128 products of
+    numbers of unit size, a few of them in a row: 2e-6 of a sequence's norm (seen: 8e-7)."""
+    from herbert_rs_amd.kernels import recurrent
+    case = step(lengths, kv_heads, heads, D, V, kind, rate)
+    want, want_state = expected(*case[:6], lengths, kv_heads, heads, D, V, kind)
+    for scratch in (recurrent.CHUNK_SCRATCH, 1):               # (1: a chunk a launch)
+        monkeypatch.setattr(recurrent, "CHUNK_SCRATCH", scratch)
+        got, state = run(*case, kv_heads, heads, D, V, kind)
+        at = 0
+        for n in lengths:
+            assert float((got[at:at + n] - want[at:at + n]).norm() / want[at:at + n].norm()) <= 2e-6, (n, scratch)
+            at += n
+        assert float((state - want_state).norm() / want_state.norm()) <= 2e-6
+        assert torch.equal(state[0], case[5][0]) and torch.equal(state[-1], case[5][-1])      # nobody's slots
+
+
+@pytest.mark.parametrize("kind", ["head", "linear"])
+@pytest.mark.parametrize("place", [3, 64 + 17])
+def test_rows_that_are_not_finite_reach_no_earlier_token(kind, place):
+    """A value without a finite size: its head's outputs before it, other heads and other sequences are the same bits; its
+    head's own outputs from there on are not numbers."""
+    kv_heads, heads, D, V, lengths = 2, 2, 64, 32, [150, 100]
+    case = list(step(lengths, kv_heads, heads, D, V, kind, 0.0))
+    clean, state = run(*case, kv_heads, heads, D, V, kind)
+    case[0] = case[0].clone()
+    case[0][place, 2 * kv_heads * D + V + 5] = float("inf")     # a value of head 1
+    got, wild = run(*case, kv_heads, heads, D, V, kind)
+    assert torch.equal(got[150:], clean[150:]) and torch.equal(got[:, 0], clean[:, 0])
+    assert torch.allclose(got[:place, 1], clean[:place, 1], rtol=0, atol=0) and bool(got[place:150, 1].isnan().all())
+    assert torch.equal(wild[1], state[1]) and torch.equal(wild[2, 0], state[2, 0]) and bool(wild[2, 1].isnan().all())
