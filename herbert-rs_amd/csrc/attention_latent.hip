@@ -387,6 +387,216 @@ latent_attention_mfma_kernel(const float* __restrict__ q_full, const bf16* __res
     }
 }
 
+// ------------------------------------------------ the same for prompts: 64 rows share their keys
+// A workgroup takes 64 (token, head) rows of a sequence, head by head and token by token as they lie, and walks the keys that
+// any of them sees in chunks of 32. A chunk comes into LDS once for all of them (16 bytes a thread and load, asked for while the
+// chunk before is worked on), as operands of the scores and, transposed on the way (four keys of eight numbers a thread,
+// eight bytes a write), as operands of the weighted sums. Two waves on every 16 rows: each takes half of a row's numbers
+// in the scores (the halves meet in LDS, added in one order by both) and half of the rank in the sums, so that the
+// query's two bfloat16 halves (72 registers) and the sums (64) of a wave fit beside a second wave on its SIMD. Operands,
+// halves and order of keys are latent_attention_mfma_kernel's; the softmax runs in powers of two, and its reference moves
+// only where a weight would pass 2^LP_SLACK. A chunk that a row does not see leaves it as it was; keys behind the last
+// that a row sees are zeros.
+// 2,048 tokens of 16 heads, 512 + 64, take 282 us (a wave a token's 16 heads, keys from the L2s and V transposed by every
+// wave: 958), three prompts of 840 to 1,400 tokens 302 (1,086). Bound by the phases of a chunk (8,500 cycles), which the
+// barriers keep apart: LDS is busy for 3,700 of them (1,800 are writes that meet in a bank), the matrix cores for 2,200,
+// the vector units for 1,900.
+#define LP_ROWS 64
+#define LP_SLACK 8.0f
+#define LP_LOG2E 1.4426950408889634f
+template <int RBW, int KSW>
+__global__ void __launch_bounds__(512)
+latent_attention_prompt_kernel(const float* __restrict__ q_full, const bf16* __restrict__ pages, bf16* __restrict__ out,
+                               const float* __restrict__ gate, int gate_ld, const int* __restrict__ positions,
+                               const int* __restrict__ seq_starts, const int* __restrict__ slots,
+                               const int* __restrict__ page_table, int max_pages, int page_size, int H, int rank,
+                               int rot, float scale, const float* __restrict__ sinks) {
+    // operands of 64 lanes x 16 bytes, lane (n, g) at 16 g + (n + a rotation by the operand's number) % 16: reads meet no
+    // bank twice, and the writes of threads that hold a key's neighbouring numbers spread over the banks
+    __shared__ __attribute__((aligned(16))) uint4 keys[2][2][KSW][HB_WAVE];         // [block of 16 keys][half][32 numbers]
+    __shared__ __attribute__((aligned(16))) uint4 Vt[2][2][RBW][HB_WAVE];           // [buffer][half][16 numbers], 32 keys
+    __shared__ __attribute__((aligned(16))) la_f32x4 halves[8][2][HB_WAVE];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int n = lane & 15, g = lane >> 4, half = wave & 1;
+    const int kd = rank + rot, KS = kd / 32, vsteps = rank / 8;
+    const int ks_a = (KS + 1) / 2, db_a = (rank / 16 + 1) / 2;              // the first half's steps and blocks
+    const int seq = blockIdx.y, tile = gridDim.x - 1 - blockIdx.x;          // (the tiles with the most keys first)
+    const int begin = seq_starts[seq], rows = (seq_starts[seq + 1] - begin) * H;
+    if (tile * LP_ROWS >= rows) return;
+    const int in_seq = tile * LP_ROWS + 16 * (wave >> 1) + n;
+    const bool mine = in_seq < rows;
+    const int t = begin + (mine ? in_seq : rows - 1) / H, h = (mine ? in_seq : rows - 1) % H;
+    const int sees = mine ? positions[t] : -1;                              // the last key that this lane's row sees
+    const int pos_last = positions[begin + min(tile * LP_ROWS + LP_ROWS - 1, rows - 1) / H];
+    const int* pt = page_table + (size_t)slots[seq] * max_pages;
+    const int n_chunks = pos_last / LA_CHUNK + 1;
+    // this wave's share of the scores' steps and of the sums' blocks. (Steps beyond it are zeros in LDS against a query
+    // of zeros, blocks beyond it go into sums that go nowhere: there is no branch between the products.)
+    const int ks0 = half ? ks_a : 0, ks_n = half ? KS - ks_a : ks_a;
+    const int db0 = half ? db_a : 0, db_n = half ? rank / 16 - db_a : db_a;
+    for (int i = tid; i < 4 * KSW * HB_WAVE; i += 512) (&keys[0][0][0][0])[i] = uint4{0, 0, 0, 0};
+
+    la_bf16x8 qh[KSW], ql[KSW];
+    {
+        const float* qrow = q_full + ((size_t)t * H + h) * kd + 32 * ks0 + 8 * g;
+#pragma unroll
+        for (int ks = 0; ks < KSW; ++ks) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                __bf16 hi, lo;
+                la_split(ks < ks_n ? qrow[32 * ks + e] * (scale * LP_LOG2E) : 0.f, hi, lo);
+                qh[ks][e] = hi;
+                ql[ks][e] = lo;
+            }
+        }
+    }
+    float m = -INFINITY, l = 0.f;
+    la_f32x4 acc[RBW];
+#pragma unroll
+    for (int db = 0; db < RBW; ++db) acc[db] = la_f32x4{0.f, 0.f, 0.f, 0.f};
+
+    // a thread's share of a chunk: four keys of eight numbers of the latent, and eight of the rotated part of one
+    const int x = tid % vsteps, kg = tid / vsteps;
+    const int rx = rot ? tid % (rot / 8) : 0, rkey = rot ? tid / (rot / 8) : LA_CHUNK;
+    const int lat_at = 4 * kg * kd + 8 * x, turned_at = rkey * kd + rank + 8 * rx;
+    uint4 lat[4], turned;
+    auto fetch = [&](int c, int page) {
+        const int j0 = c * LA_CHUNK;
+        const bf16* chunk = pages + ((size_t)page * page_size + j0 % page_size) * kd;
+        if (kg < 8) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) lat[i] = *(const uint4*)(chunk + lat_at + i * kd);
+        }
+        if (rkey < LA_CHUNK) turned = *(const uint4*)(chunk + turned_at);
+        if (j0 + LA_CHUNK - 1 > pos_last) {                          // (a page's rows exist whether a token lies there or not)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (j0 + 4 * kg + i > pos_last) lat[i] = uint4{0, 0, 0, 0};
+            if (j0 + rkey > pos_last) turned = uint4{0, 0, 0, 0};
+        }
+    };
+    auto put_key = [&](int key, int segment, uint4 v) {
+        const int ks = segment / 4, of = ks >= ks_a, in = ks - (of ? ks_a : 0);
+        keys[key >> 4][of][in][16 * (segment & 3) + ((key + 4 * (in & 3)) & 15)] = v;
+    };
+    auto stash = [&](int buf) {
+        if (kg < 8) {
+            // eight numbers of a key: step x / 4 of the scores, lane row x % 4
+#pragma unroll
+            for (int i = 0; i < 4; ++i) put_key(4 * kg + i, x, lat[i]);
+            // keys 16 kb + 4 g' + i lie at g' 8 + kb 4 + i, the order in which a lane holds their weights
+            const unsigned *a = (const unsigned*)&lat[0], *b = (const unsigned*)&lat[1], *c = (const unsigned*)&lat[2], *d = (const unsigned*)&lat[3];
+            const int block = x / 2, of = block >= db_a, in = block - (of ? db_a : 0);
+            uint2* row = (uint2*)&Vt[buf][of][in][16 * (kg & 3)] + (kg >> 2);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const unsigned pick = e & 1 ? 0x07060302u : 0x05040100u;
+                row[2 * (((x & 1) * 8 + e + 2 * (in & 3)) & 15)] =
+                    uint2{__builtin_amdgcn_perm(b[e / 2], a[e / 2], pick), __builtin_amdgcn_perm(d[e / 2], c[e / 2], pick)};
+            }
+        }
+        if (rkey < LA_CHUNK) put_key(rkey, vsteps + rx, turned);
+    };
+    int page_next = pt[LA_CHUNK / page_size < max_pages ? LA_CHUNK / page_size : 0];
+    fetch(0, pt[0]);
+    __syncthreads();                                                 // (the zeros of the keys' unused steps are there)
+    stash(0);
+    __syncthreads();
+    for (int c = 0, buf = 0; c < n_chunks; ++c, buf ^= 1) {
+        if (c + 1 < n_chunks) {
+            fetch(c + 1, page_next);
+            if (c + 2 < n_chunks) page_next = pt[(c + 2) * LA_CHUNK / page_size];
+        }
+        la_f32x4 s[2], s_low[2];
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) s[kb] = s_low[kb] = la_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < KSW; ++ks) {
+            const int place = 16 * g + ((n + 4 * (ks & 3)) & 15);
+            const la_bf16x8 k0 = __builtin_bit_cast(la_bf16x8, keys[0][half][ks][place]);
+            const la_bf16x8 k1 = __builtin_bit_cast(la_bf16x8, keys[1][half][ks][place]);
+            s[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qh[ks], s[0], 0, 0, 0);
+            s[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, qh[ks], s[1], 0, 0, 0);
+            s_low[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, ql[ks], s_low[0], 0, 0, 0);
+            s_low[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, ql[ks], s_low[1], 0, 0, 0);
+        }
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+            s[kb] += s_low[kb];
+            halves[wave][kb][lane] = s[kb];
+        }
+        __syncthreads();                                             // (and nobody reads this chunk's keys any more)
+        // s[kb][i]: key 16 kb + 4 g + i of the chunk against row n, in powers of two
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) s[kb] += halves[wave ^ 1][kb][lane];
+        if (__any(c * LA_CHUNK + LA_CHUNK - 1 > sees)) {
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (c * LA_CHUNK + 16 * kb + 4 * g + i > sees) s[kb][i] = -INFINITY;
+        }
+        float cmax = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])),
+                           fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
+        cmax = fmaxf(cmax, __shfl_xor(cmax, 16, HB_WAVE));
+        cmax = fmaxf(cmax, __shfl_xor(cmax, 32, HB_WAVE));
+        // (the sums are brought to another reference only where a weight would pass 2^LP_SLACK)
+        if (__any(cmax > m + LP_SLACK)) {
+            const float m_new = fmaxf(m, cmax);
+            const float corr = m == m_new ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);
+            l *= corr;
+            m = m_new;
+#pragma unroll
+            for (int db = 0; db < RBW; ++db)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[db][i] *= corr;
+        }
+        const float base = m == -INFINITY ? 0.f : m;                 // (a row that has seen nothing yet)
+        la_bf16x8 ph, pl;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float p = __builtin_amdgcn_exp2f(s[kb][i] - base);
+                l += p;
+                __bf16 hi, lo;
+                la_split(p, hi, lo);
+                ph[4 * kb + i] = hi;
+                pl[4 * kb + i] = lo;
+            }
+#pragma unroll
+        for (int db = 0; db < RBW; db += 2) {
+            la_bf16x8 v[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                v[i] = __builtin_bit_cast(la_bf16x8, Vt[buf][half][db + i][16 * g + ((n + 2 * ((db + i) & 3)) & 15)]);
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i) acc[db + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[i], ph, acc[db + i], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) acc[db + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[i], pl, acc[db + i], 0, 0, 0);
+        }
+        if (c + 1 < n_chunks) stash(buf ^ 1);
+        __syncthreads();
+    }
+    l += __shfl_xor(l, 16, HB_WAVE);
+    l += __shfl_xor(l, 32, HB_WAVE);
+    if (!mine) return;
+    if (sinks) l += __builtin_amdgcn_exp2f(sinks[h] * LP_LOG2E - m);                 // (an infinite share, a sink far above every score, leaves 0)
+    float w = l > 0.f ? 1.0f / l : 0.f;
+    if (gate) w *= 1.0f / (1.0f + expf(-gate[(size_t)t * gate_ld + h]));
+#pragma unroll
+    for (int db = 0; db < RBW; ++db)
+        if (db < db_n) {
+            // acc[db][i]: number 16 (db0 + db) + 4 g + i of row n's sum
+            bf16 o[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[i] = hb_from_float<bf16>(acc[db][i] * w);
+            *(uint2*)(out + ((size_t)t * H + h) * rank + 16 * (db0 + db) + 4 * g) =
+                uint2{o[0].bits | ((unsigned)o[1].bits << 16), o[2].bits | ((unsigned)o[3].bits << 16)};
+        }
+}
+
 // out[row, :] = sum over the ranges (in order) of their sums, brought to one maximum, over the summed
 // denominators, times sigmoid(gate). One block a (token, head).
 __global__ void __launch_bounds__(256)
@@ -433,7 +643,8 @@ extern "C" int hb_latent_attention_mfma(const float* q_full, const void* pages, 
                                         float* part_ml, const float* gate, int gate_ld, const int* positions,
                                         const int* seq_of, const int* slots, const int* page_table, int max_pages,
                                         int page_size, int T, int H, int rank, int rot, float scale, int splits,
-                                        int chunks_per_split, const float* sinks, hipStream_t stream) {
+                                        int chunks_per_split, const float* sinks, const int* seq_starts, int n_seqs,
+                                        int longest, hipStream_t stream) {
     HB_REQUIRE(T > 0 && H > 0, "latent attention: empty input");
     HB_REQUIRE(rank > 0 && rank % 32 == 0 && rank <= 512 && rot % 32 == 0 && rank + rot <= 640,
                "latent attention: the matrix-core kernel takes a latent and a rotated part in steps of 32, up to 512 + 128, not %d + %d", rank, rot);
@@ -441,7 +652,23 @@ extern "C" int hb_latent_attention_mfma(const float* q_full, const void* pages, 
     HB_REQUIRE(splits >= 1 && splits <= HB_WAVE && chunks_per_split >= 1, "latent attention: %d ranges, the kernels take 1 to 64", splits);
     HB_REQUIRE(splits == 1 || (part_acc && part_ml), "latent attention: ranges need scratch");
     const long long blocks = (long long)T * ((H + 15) / 16);
-    HB_REQUIRE(blocks < (1ll << 31), "latent attention: too many tokens for the grid");
+    HB_REQUIRE(blocks < (1ll << 31) && (long long)T * H < (1ll << 31) - LP_ROWS, "latent attention: too many tokens for the grid");
+    if (seq_starts) {      // the prompts' kernel; longest: the most tokens that a sequence of the step brings
+        HB_REQUIRE(n_seqs > 0 && n_seqs <= 65535 && longest > 0 && longest <= T, "latent attention: %d sequences of up to %d tokens", n_seqs, longest);
+#define LP_LAUNCH(RBV, KSV)                                                                                           \
+    latent_attention_prompt_kernel<RBV, KSV>                                                                          \
+        <<<dim3((unsigned)(((long long)longest * H + LP_ROWS - 1) / LP_ROWS), n_seqs), 512, 0, stream>>>(             \
+            q_full, (const bf16*)pages, (bf16*)out, gate, gate_ld, positions, seq_starts, slots, page_table, max_pages, \
+            page_size, H, rank, rot, scale, sinks)
+        if (rank <= 128 && rank + rot <= 256) LP_LAUNCH(4, 4);
+        else if (rank <= 256 && rank + rot <= 384) LP_LAUNCH(8, 6);
+        else if (rank + rot <= 512) LP_LAUNCH(16, 8);
+        else if (rank + rot <= 576) LP_LAUNCH(16, 9);
+        else LP_LAUNCH(16, 10);
+#undef LP_LAUNCH
+        HB_CHECK_LAUNCH("latent_attention_prompt");
+        return 0;
+    }
     const dim3 grid((unsigned)blocks, splits);
 #define LA_LAUNCH(RBV, KSV)                                                                                      \
     latent_attention_mfma_kernel<RBV, KSV><<<grid, HB_WAVE, 0, stream>>>(                                          \

@@ -93,6 +93,12 @@ CHUNK = 32
 TARGET_WAVES = 1024        # a decode step's keys are cut into ranges until about this many waves run
 
 
+# Steps of several tokens a sequence take the kernel whose workgroups share their keys from contexts beyond this on: two
+# chunks of 32 keys leave it nothing to share (8 prompts of 64 tokens: 24 us, a wave a token's heads 23; of 20 tokens 32 and
+# 26), at 100 tokens it takes 40 us against 51.
+PROMPT_FROM = 64
+
+
 def mfma_takes(cache, rank, rot):
     """True if the matrix-core kernel takes this latent: bfloat16 rows, the latent and the rotated part in
     steps of 32, up to 512 + 128."""
@@ -101,8 +107,8 @@ def mfma_takes(cache, rank, rot):
 
 
 def latent_attention_mfma(q_full, meta, cache, out, gate, gate_off, H, rank, rot, scale, buffer, sinks=None):
-    """latent_attention_plain on the matrix cores (see mfma_takes). A step of one token a sequence cuts its
-    keys into ranges, whose partial results lie in scratch from `buffer(name, shape, dtype)`."""
+    """latent_attention_plain on the matrix cores (see mfma_takes). A prompt's tokens share their keys in LDS; a step of one
+    token a sequence cuts its keys into ranges, whose partial results lie in scratch from `buffer(name, shape, dtype)`."""
     if sinks is not None:
         _check(sinks, "sinks", torch.float32, (H,))
     T = q_full.shape[0]
@@ -129,7 +135,11 @@ def latent_attention_mfma(q_full, meta, cache, out, gate, gate_off, H, rank, rot
     if splits > 1:
         part_acc = buffer("latent_partial", (T * H * splits, rank), torch.float32)
         part_ml = buffer("latent_partial_ml", (T * H * splits, 2), torch.float32)
+    prompt = meta.max_new > 1 and meta.max_context > PROMPT_FROM
+    if prompt:
+        _check(meta.seq_starts, "seq_starts", torch.int32, (meta.num_seqs + 1,))
     lib.call("attention_latent", "hb_latent_attention_mfma", q_full.data_ptr(), cache.k.data_ptr(), out.data_ptr(),
              _ptr(part_acc), _ptr(part_ml), gate_ptr, gate_ld, meta.positions.data_ptr(), meta.seq_of.data_ptr(),
              meta.slots.data_ptr(), cache.page_table.data_ptr(), cache.page_table.shape[1], cache.page_size, T, H,
-             rank, rot, float(scale), splits, per, _ptr(sinks), _stream())
+             rank, rot, float(scale), splits, per, _ptr(sinks),
+             meta.seq_starts.data_ptr() if prompt else None, meta.num_seqs if prompt else 0, int(meta.max_new), _stream())

@@ -226,6 +226,42 @@ def test_a_single_far_key_holds_the_weight():
                 assert float(out[far - 1].abs().max()) < 0.5              # just before it: unseen
 
 
+@pytest.mark.parametrize("H,rank,rot", [(16, 512, 64), (5, 512, 128), (3, 480, 0), (20, 256, 96), (8, 32, 0), (64, 128, 32)])
+def test_prompt_tokens_share_their_keys(H, rank, rot):
+    """The prompt kernel of the latent attention, whose workgroups take 64 (token, head) rows of a sequence: heads that no tile
+    divides, latents of one step to sixteen (odd ones among them), sequences that go on in the
+    cache, a sink and a gate, against float64; rows behind the sequences' ends may hold anything. bfloat16 keys as
+    stored, queries and weights in 16 bits, an output of 8: 2^-8 of the largest entry."""
+    row, held, new = rank + rot, [150, 70, 1, 97], [150, 30, 1, 97]
+    cache = Cache({0: KVNeed(1, row, None, values=False)}, 64 * 16, 4096, torch.bfloat16, DEV, max_slots=len(held))
+    kv = cache.kv_view(0)
+    slots = [cache.alloc_slot() for _ in held]
+    for s, n, k in zip(slots, held, new):
+        if n > k:
+            step_meta(cache, [s], [n - k])
+    meta = step_meta(cache, slots, new)
+    kv.k.fill_(float("nan"))
+    rows = [rand(n, row, seed=i).to(torch.bfloat16) for i, n in enumerate(held)]
+    for s, r in zip(slots, rows):
+        table = kv.page_table[s].cpu().tolist()
+        for p in range(r.shape[0]):
+            kv.k[table[p // 64], 0, p % 64] = r[p].to(DEV)
+    T = sum(new)
+    q, gate, sinks = rand(T, H * row, seed=9), rand(T, H, seed=10), rand(H, seed=11)
+    out = torch.empty(T, H * rank, dtype=torch.bfloat16, device=DEV)
+    latent.latent_attention_mfma(q.to(DEV), meta, kv, out, gate.to(DEV), 0, H, rank, rot, row ** -0.5, None, sinks=sinks.to(DEV))
+    at = 0
+    for r, n, k in zip(rows, held, new):
+        for t in range(k):
+            keys = r[:n - k + t + 1].double()
+            score = q[at + t].view(H, row).double() @ keys.T * row ** -0.5
+            w = torch.softmax(torch.cat([score, sinks.double()[:, None]], 1), -1)[:, :-1]
+            want = (w @ keys[:, :rank]) * torch.sigmoid(gate[at + t].double())[:, None]
+            err = (out[at + t].cpu().double().view(H, rank) - want).abs().max()
+            assert float(err) <= 2.0 ** -8 * float(want.abs().max()) + 1e-3, (n, t)
+        at += k
+
+
 @pytest.mark.parametrize("T,E,top", [(1, 3, 3), (9, 5, 2), (300, 16, 4), (70, 130, 7)])
 def test_routing_groups_and_products(T, E, top):
     W, F = 64, 96                                          # (K in steps of 32: what the matrix-core product takes)
