@@ -370,34 +370,68 @@ extern "C" int hb_moe_activate(const float* gu, void* act, int act_dtype, int ro
 // shared [T, H] (or null): a part that every token takes, added times sigmoid(gate[t * gate_ld]).
 // input [T, H] (or null) with chosen [T, top] and real: a pair whose expert is `real` or beyond has no row in y;
 // its output is the token's own input row.
-template <class TIn>
+// A thread takes PER neighbouring columns of a token (four where rows lie in whole quads), so that a step of few tokens is
+// one round of loads: 4 tokens of 2,048 columns, four rows each 4 us, 2,048 tokens 18 (a column a thread and a row's
+// columns eight after another: 15 and 32).
+template <int PER>
+struct alignas(4 * PER) MoeColumns {
+    float v[PER];
+};
+template <int PER>
+__device__ __forceinline__ MoeColumns<PER> moe_columns(const float* p) {
+    return *(const MoeColumns<PER>*)p;
+}
+template <int PER>
+__device__ __forceinline__ MoeColumns<PER> moe_columns(const bf16* p) {
+    struct alignas(2 * PER) Stored {
+        bf16 v[PER];
+    };
+    const Stored s = *(const Stored*)p;
+    MoeColumns<PER> c;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) c.v[i] = hb_to_float(s.v[i]);
+    return c;
+}
+
+template <class TIn, int PER>
 __global__ void moe_combine_kernel(const float* __restrict__ y, const float* __restrict__ weight,
                                    const int* __restrict__ row_of, float* __restrict__ x, int top, int H,
                                    const float* __restrict__ shared, const float* __restrict__ gate, int gate_ld,
                                    const TIn* __restrict__ input, const int* __restrict__ chosen, int real) {
-    const int t = blockIdx.x;
+    const int t = blockIdx.x, at = (blockIdx.y * blockDim.x + threadIdx.x) * PER;
+    if (at >= H) return;
     const float open = shared ? 1.0f / (1.0f + expf(-gate[(size_t)t * gate_ld])) : 0.f;
-    // (a token's rows and weights once, eight at a time, then whole rows)
+    float* out = x + (size_t)t * H + at;
+    MoeColumns<PER> sum = moe_columns<PER>(out);
     for (int j0 = 0; j0 < top; j0 += 8) {
-        const float* rows[8];
+        MoeColumns<PER> rows[8];
         float w[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const bool in = j0 + j < top;
-            rows[j] = y + (size_t)row_of[(size_t)t * top + (in ? j0 + j : 0)] * H;
-            w[j] = in ? weight[(size_t)t * top + j0 + j] : 0.f;
-            if (input != nullptr && in && chosen[(size_t)t * top + j0 + j] >= real) rows[j] = nullptr;
-        }
-        for (int i = threadIdx.x; i < H; i += blockDim.x) {
-            float s = 0.f;
+        for (int j = 0; j < 8; ++j)
+            if (j0 + j < top) {
+                const size_t pair = (size_t)t * top + j0 + j;
+                w[j] = weight[pair];
+                if (input != nullptr && chosen[pair] >= real)
+                    rows[j] = moe_columns<PER>(input + (size_t)t * H + at);
+                else
+                    rows[j] = moe_columns<PER>(y + (size_t)row_of[pair] * H + at);
+            }
+        MoeColumns<PER> s = {};
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (j0 + j < top)
-                    s = fmaf(w[j], rows[j] != nullptr ? rows[j][i] : hb_to_float(input[(size_t)t * H + i]), s);
-            if (shared && j0 == 0) s = fmaf(open, shared[(size_t)t * H + i], s);
-            x[(size_t)t * H + i] += s;
+        for (int j = 0; j < 8; ++j)
+            if (j0 + j < top) {
+#pragma unroll
+                for (int i = 0; i < PER; ++i) s.v[i] = fmaf(w[j], rows[j].v[i], s.v[i]);
+            }
+        if (shared && j0 == 0) {
+            const MoeColumns<PER> part = moe_columns<PER>(shared + (size_t)t * H + at);
+#pragma unroll
+            for (int i = 0; i < PER; ++i) s.v[i] = fmaf(open, part.v[i], s.v[i]);
         }
+#pragma unroll
+        for (int i = 0; i < PER; ++i) sum.v[i] += s.v[i];
     }
+    *(MoeColumns<PER>*)out = sum;
 }
 
 extern "C" int hb_moe_combine(const float* y, const float* weight, const int* row_of, float* x, int T, int top, int H,
@@ -406,13 +440,20 @@ extern "C" int hb_moe_combine(const float* y, const float* weight, const int* ro
     HB_REQUIRE(shared == nullptr || (gate != nullptr && gate_ld > 0), "moe combine: a shared part needs its gate");
     HB_REQUIRE(T > 0 && top > 0 && H > 0, "moe combine: empty input");
     HB_REQUIRE(input == nullptr || chosen != nullptr, "moe combine: experts without matrices need the choices");
-    const int threads = H >= 1024 ? 256 : 64;
-    if (input != nullptr && input_dtype == HB_BF16)
-        moe_combine_kernel<bf16><<<T, threads, 0, stream>>>(y, weight, row_of, x, top, H, shared, gate, gate_ld,
-                                                            (const bf16*)input, chosen, real);
-    else
-        moe_combine_kernel<float><<<T, threads, 0, stream>>>(y, weight, row_of, x, top, H, shared, gate, gate_ld,
-                                                             (const float*)input, chosen, real);
+    const bool quads = H % 4 == 0 && (uintptr_t)y % 16 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)shared % 16 == 0 &&
+                       (uintptr_t)input % 16 == 0;
+    const int threads = H >= 1024 ? 256 : 64, per = quads ? 4 : 1;
+    const dim3 grid(T, (H + threads * per - 1) / (threads * per));
+    HB_REQUIRE(grid.y <= 65535, "moe combine: rows of %d columns exceed the grid", H);
+#define HB_COMBINE(TIn, PER)                                                                                          \
+    moe_combine_kernel<TIn, PER><<<grid, threads, 0, stream>>>(y, weight, row_of, x, top, H, shared, gate, gate_ld,   \
+                                                               (const TIn*)input, chosen, real)
+    const bool narrow = input != nullptr && input_dtype == HB_BF16;
+    if (quads && narrow) HB_COMBINE(bf16, 4);
+    else if (quads) HB_COMBINE(float, 4);
+    else if (narrow) HB_COMBINE(bf16, 1);
+    else HB_COMBINE(float, 1);
+#undef HB_COMBINE
     HB_CHECK_LAUNCH("moe_combine");
     return 0;
 }
