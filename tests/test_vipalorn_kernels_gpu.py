@@ -262,6 +262,33 @@ def test_prompt_tokens_share_their_keys(H, rank, rot):
         at += k
 
 
+@pytest.mark.parametrize("M", [1, 16, 17, 64, 65, 200, 700])
+@pytest.mark.parametrize("G,N,K,pad", [(1, 16, 32, 0), (5, 48, 160, 0), (3, 272, 64, 4), (4, 512, 96, 3)])
+def test_grouped_products_of_any_rows(M, G, N, K, pad):
+    """A product a group on the matrix cores, every epilogue: rows that fill no tile, more column blocks and tiles than a turn
+    over the XCDs and fewer, k that no workgroup's four waves divide, and output rows that start at no whole quad.
+    float32 sums of bfloat16 products: K / 2^24 of the terms' sizes."""
+    from herbert_rs_amd.kernels import moe
+    w, a = rand(G, N, K, seed=1).to(torch.bfloat16), rand(M, G * K, seed=2).to(torch.bfloat16)
+    for epi in (moe.EPI_F32, moe.EPI_BF16) + ((moe.EPI_GLU,) if N % 32 == 0 else ()):
+        cols = N // 2 if epi == moe.EPI_GLU else N
+        off = cols + pad
+        c = torch.full((M, G * off), 3.0, dtype=torch.float32 if epi == moe.EPI_F32 else torch.bfloat16, device=DEV)
+        moe.grouped_mfma(a.to(DEV), G * K, K, moe.pack_grouped(w.to(DEV)), c, G * off, off, epi, M=M, limit=2.0, alpha=1.702, shift=1.0)
+        got = c.cpu().double().view(M, G, off)
+        for g in range(G):
+            rows = a[:, g * K:(g + 1) * K].double()
+            want, size = rows @ w[g].double().T, rows.abs() @ w[g].double().abs().T
+            slack = K * 2.0 ** -24 * size + 1e-6
+            if epi == moe.EPI_GLU:
+                z, u = want[:, :cols].clamp(max=2.0), want[:, cols:].clamp(-2.0, 2.0)
+                want, slack = z * torch.sigmoid(1.702 * z) * (u + 1.0), 1e-4
+            if epi != moe.EPI_F32:
+                slack = slack + want.abs() * 2.0 ** -8
+            assert bool(((got[:, g, :cols] - want).abs() <= slack).all()), (epi, g)
+            assert bool((got[:, g, cols:] == 3.0).all())
+
+
 @pytest.mark.parametrize("T,E,top", [(1, 3, 3), (9, 5, 2), (300, 16, 4), (70, 130, 7)])
 def test_routing_groups_and_products(T, E, top):
     W, F = 64, 96                                          # (K in steps of 32: what the matrix-core product takes)
