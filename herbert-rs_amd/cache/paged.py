@@ -25,6 +25,7 @@ import numpy as np
 import torch
 
 from ..errors import CacheError
+from ..hosted import send
 from .needs import KVNeed, StateNeed
 from .slots import PAGE_TOKENS, FreeList, pages_for
 
@@ -76,21 +77,23 @@ class KVGroup:
         """How many pages `ensure(slot, new_length)` would take."""
         return max(0, pages_for(new_length) - max(self.held_end[slot], int(self.first_page[slot])))
 
-    def ensure(self, slot, new_length):
-        """Hold a page for every position below new_length that a query may still see."""
-        last = pages_for(new_length)
-        first_new = max(self.held_end[slot], int(self.first_page[slot]))
-        if first_new >= last:
-            return
-        row = self.table_host[slot]
-        for p in range(first_new, last):
-            row[p] = self.pages.take()
-        self.held_end[slot] = last
-        self._upload(slot, first_new, last)
-
-    def _upload(self, slot, a, b):
-        self.table[slot, a:b] = torch.from_numpy(np.maximum(self.table_host[slot, a:b], 0)).to(
-            self.table.device)
+    def ensure(self, targets):
+        """Hold a page for every position below new_length that a query may still see, for every (slot, new_length)."""
+        taken = []                    # places of the table, as if its rows lay end to end, and the pages that go there
+        for slot, new_length in targets:
+            last = pages_for(new_length)
+            first_new = max(self.held_end[slot], int(self.first_page[slot]))
+            if first_new >= last:
+                continue
+            row = self.table_host[slot]
+            for p in range(first_new, last):
+                row[p] = self.pages.take()
+                taken.append((slot * self.pages_per_slot + p, row[p]))
+            self.held_end[slot] = last
+        if taken:
+            # one copy and one kernel a step, behind what the stream holds
+            places, pages = send(np.array(taken, dtype=np.int64).T, self.table.device)
+            self.table.view(-1).index_copy_(0, places, pages.to(torch.int32))
 
     def release_unseen(self, slot, length):
         """With a window: give back pages wholly before the oldest key a later query sees (but the first pages,
@@ -168,6 +171,7 @@ class Cache:
         self.pad_slot = self.n_slots        # never handed out: where a step's padding rows write and read
         self.slots = FreeList(self.n_slots, "slot")
         self.lengths = np.zeros(self.n_slots, dtype=np.int64)
+        self._saved_slots = (None, None)    # the slots that save_state was last asked for, and their numbers on the GPU
         self.kv_groups = {}
         self.state_groups = {}
         self._kv_of = {}
@@ -242,7 +246,7 @@ class Cache:
             raise CacheError(f"slot {slot}: {new_length} positions exceed the model's "
                              f"{self.max_positions}")
         for g in self.kv_groups.values():
-            g.ensure(slot, new_length)
+            g.ensure([(slot, new_length)])
         return new_length
 
     def reserve_all(self, wanted):
@@ -261,21 +265,20 @@ class Cache:
             if need > g.pages.free_count:
                 raise CacheError(f"the step needs {need} more pages of {PAGE_TOKENS} tokens but only "
                                  f"{g.pages.free_count} of {g.pages.count} are free")
-        for slot, new_length in targets:
-            for g in self.kv_groups.values():
-                g.ensure(slot, new_length)
+        for g in self.kv_groups.values():
+            g.ensure(targets)
 
     def save_state(self, slots):
         """A copy of the fixed-size state of `slots` (None for a cache that has none): what
         `restore_state` puts back when the step that was to change it has failed."""
         if not self.state_groups:
             return None
-        index = torch.tensor(sorted(set(int(s) for s in slots)), dtype=torch.long)
-        saved = []
-        for g in self.state_groups.values():
-            at = index.to(g.data.device)
-            saved.append((g, at, g.data.index_select(1, at)))
-        return saved
+        key = tuple(sorted(set(int(s) for s in slots)))
+        if self._saved_slots[0] != key:           # (decode steps name the same slots again and again)
+            device = next(iter(self.state_groups.values())).data.device
+            self._saved_slots = (key, send(np.array(key, dtype=np.int64), device))
+        at = self._saved_slots[1]
+        return [(g, at, g.data.index_select(1, at)) for g in self.state_groups.values()]
 
     def restore_state(self, saved):
         for g, at, data in saved or ():

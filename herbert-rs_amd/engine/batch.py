@@ -11,6 +11,8 @@ from typing import List
 import numpy as np
 import torch
 
+from ..hosted import send
+
 
 @dataclass
 class StepEntry:
@@ -56,7 +58,7 @@ class BatchMeta:
                 if got is None:
                     return None
             else:
-                got = torch.from_numpy(range_list(self.host_context, items, unit)).to(self.token_ids.device)
+                got = send(range_list(self.host_context, items, unit), self.token_ids.device)
             self.derived[key] = got
         return got
 
@@ -149,7 +151,7 @@ def pack(entries, start_lengths, device, staging=None):
         for j in e.want:
             want[w] = a + j
             w += 1
-    dev = torch.from_numpy(host).to(device)
+    dev = send(host, device)
     o = 3 * T
     return BatchMeta(
         token_ids=dev[0:T], positions=dev[T:2 * T], seq_of=dev[2 * T:3 * T],

@@ -7,9 +7,11 @@ single-pass and a split decode attention by the context's length
 (crates/backends/backend_metal/src/kernels/attention.rs:73-91), as _decode_split does here."""
 import ctypes
 
+import numpy as np
 import torch
 
 from ..errors import BackendError
+from ..hosted import send
 from . import heads
 from . import lib
 from . import ops
@@ -511,7 +513,7 @@ def _prefill_tiles(meta, height=QUERY_TILE):
                 items.append((-last_position, i, r, n))
         items.sort()
         seq, row0, rows = [it[1] for it in items], [it[2] for it in items], [it[3] for it in items]
-        packed = torch.tensor([seq, row0, rows], dtype=torch.int32).to(meta.positions.device)
+        packed = send(np.array([seq, row0, rows], dtype=np.int32), meta.positions.device)
         tiles = (packed[0], packed[1], packed[2], len(seq))
         meta.derived[("prefill_tiles", height)] = tiles
     return tiles
