@@ -58,6 +58,70 @@ conv_silu_kernel(const float* __restrict__ proj, int ld, const float* __restrict
     for (int d = lane; d < len; d += HB_WAVE) row[c0 + d] *= inv;     // (each lane rescales what it wrote)
 }
 
+// The same four channels a thread, for filters of four taps over rows and sections in whole quads: the inputs of a channel's
+// last three tokens move through registers along CONV_ROWS tokens (a prompt), so a row is read once, 16 bytes a lane; a unit
+// section's sum of squares is taken by the lanes that hold it. One token a workgroup where the step has few (CONV_ROWS 1);
+// with one token a sequence (moves_state) the thread is its channels' only reader and moves the kept inputs on itself.
+// The sum over taps is the other kernel's, the sum of squares another order of it. Bound by memory: 2,048 tokens of 4,096
+// channels (67 MB) 21 us, 8 single tokens 2.9 with the state (a wave a token and section, every tap of every
+// channel a load of its own, and the state in a kernel of its own: 45 and 5.4 us).
+#define CONV_TAPS 4
+template <int CONV_ROWS>
+__global__ void __launch_bounds__(256)
+conv_silu_quads_kernel(const float* __restrict__ proj, int ld, const float* __restrict__ taps,
+                       float* __restrict__ conv_state, const int* __restrict__ seq_of,
+                       const int* __restrict__ seq_starts, const int* __restrict__ slots, float* __restrict__ out,
+                       int T, int C, int n_unit, int unit_dim, int n_scaled, float scale, float unit_eps,
+                       const float* __restrict__ bias, int moves_state) {
+    const int c = (blockIdx.y * 256 + threadIdx.x) * 4;
+    const bool live = c < C;
+    const int cc = live ? c : 0;
+    const int t0 = blockIdx.x * CONV_ROWS;
+    float4 w[4], x[CONV_ROWS], before[CONV_TAPS - 1];              // w[i]: the taps of channel c + i
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = *(const float4*)(taps + (size_t)(cc + i) * CONV_TAPS);
+#pragma unroll
+    for (int i = 0; i < CONV_ROWS; ++i) x[i] = *(const float4*)(proj + (size_t)min(t0 + i, T - 1) * ld + cc);
+    const float4 start = bias ? *(const float4*)(bias + cc) : make_float4(0.f, 0.f, 0.f, 0.f);
+    const bool unit = c < n_unit * unit_dim;
+    const float factor = unit && c / unit_dim < n_scaled ? scale : 1.0f;
+    int seq = -1;
+#pragma unroll
+    for (int i = 0; i < CONV_ROWS; ++i) {
+        const int t = t0 + i;
+        if (t >= T) break;
+        if (seq_of[t] != seq) {                                   // the inputs before this row: the step's, or the kept ones
+            seq = seq_of[t];
+            const int first = seq_starts[seq], at = t - first;
+            float* state = conv_state + (size_t)slots[seq] * (CONV_TAPS - 1) * C + cc;
+#pragma unroll
+            for (int j = 0; j < CONV_TAPS - 1; ++j) {
+                const int s = at - (CONV_TAPS - 1) + j;
+                before[j] = s >= 0 ? *(const float4*)(proj + (size_t)(first + s) * ld + cc)
+                                   : *(const float4*)(state + (size_t)(CONV_TAPS - 1 + s) * C);
+            }
+            if (moves_state && live) {
+                *(float4*)state = before[1];
+                *(float4*)(state + C) = before[2];
+                *(float4*)(state + 2 * (size_t)C) = x[i];
+            }
+        }
+        float4 y;
+        y.x = hb_silu(fmaf(w[0].w, x[i].x, fmaf(w[0].z, before[2].x, fmaf(w[0].y, before[1].x, fmaf(w[0].x, before[0].x, start.x)))));
+        y.y = hb_silu(fmaf(w[1].w, x[i].y, fmaf(w[1].z, before[2].y, fmaf(w[1].y, before[1].y, fmaf(w[1].x, before[0].y, start.y)))));
+        y.z = hb_silu(fmaf(w[2].w, x[i].z, fmaf(w[2].z, before[2].z, fmaf(w[2].y, before[1].z, fmaf(w[2].x, before[0].z, start.z)))));
+        y.w = hb_silu(fmaf(w[3].w, x[i].w, fmaf(w[3].z, before[2].w, fmaf(w[3].y, before[1].w, fmaf(w[3].x, before[0].w, start.w)))));
+        before[0] = before[1], before[1] = before[2], before[2] = x[i];
+        if (unit) {
+            float ss = fmaf(y.x, y.x, y.y * y.y) + fmaf(y.z, y.z, y.w * y.w);
+            for (int off = 1; off < unit_dim / 4; off <<= 1) ss += __shfl_xor(ss, off, HB_WAVE);
+            const float inv = factor / sqrtf(ss + unit_eps);
+            y.x *= inv, y.y *= inv, y.z *= inv, y.w *= inv;
+        }
+        if (live) *(float4*)(out + (size_t)t * C + c) = y;
+    }
+}
+
 // The state after the step: the last K - 1 inputs of each sequence, from the step's rows where it
 // brought that many, else the old state moved up. One thread a (sequence, channel).
 // (bias [C] or null: the inputs are the rows plus a bias a channel, and the state holds them with it)
@@ -81,13 +145,33 @@ __global__ void conv_state_kernel(const float* __restrict__ proj, int ld, float*
 extern "C" int hb_conv_silu(const float* proj, int ld, const float* taps, float* conv_state, const int* seq_of,
                             const int* seq_starts, const int* slots, float* out, int T, int B, int C, int K,
                             int n_unit, int unit_dim, int n_scaled, float scale, float unit_eps, int n_plain,
-                            int plain_dim, const float* bias, hipStream_t stream) {
+                            int plain_dim, const float* bias, int longest, hipStream_t stream) {
     HB_REQUIRE(T > 0 && B > 0 && C > 0, "conv: empty input");
     HB_REQUIRE(K >= 1 && K <= HB_MAX_TAPS, "conv: %d taps, the kernel takes 1 to %d", K, HB_MAX_TAPS);
     HB_REQUIRE(n_unit * unit_dim + n_plain * plain_dim >= C && (n_plain == 0 ? n_unit * unit_dim == C
                : n_unit * unit_dim + (n_plain - 1) * plain_dim < C) && ld >= C,
                "conv: the sections do not add up to %d channels", C);
     HB_REQUIRE(n_unit + n_plain <= 65535 && B <= 65535, "conv: too many sections or sequences for the grid");
+    // quads: four taps, everything in whole quads, unit sections that a power of two of at most 64 lanes holds
+    const bool quads = K == CONV_TAPS && C % 4 == 0 && ld % 4 == 0 && (uintptr_t)proj % 16 == 0 && (uintptr_t)taps % 16 == 0 &&
+                       (uintptr_t)conv_state % 16 == 0 && (uintptr_t)out % 16 == 0 && (uintptr_t)bias % 16 == 0 &&
+                       (n_unit == 0 || (n_unit * unit_dim <= C && unit_dim % 4 == 0 && unit_dim <= 256 && (unit_dim & (unit_dim - 1)) == 0));
+    if (quads && (C + 1023) / 1024 <= 65535) {
+        const int moves = longest == 1;
+        const unsigned across = (C + 1023) / 1024;
+#define HB_CONV(ROWS)                                                                                                 \
+    conv_silu_quads_kernel<ROWS><<<dim3((T + ROWS - 1) / ROWS, across), 256, 0, stream>>>(                            \
+        proj, ld, taps, conv_state, seq_of, seq_starts, slots, out, T, C, n_unit, unit_dim, n_scaled, scale, unit_eps, bias, moves)
+        if (T > 256) HB_CONV(8);
+        else HB_CONV(1);
+#undef HB_CONV
+        HB_CHECK_LAUNCH("conv_silu_quads");
+        if (!moves) {
+            conv_state_kernel<<<dim3(B, (C + 255) / 256), 256, 0, stream>>>(proj, ld, conv_state, seq_starts, slots, C, K, nullptr);
+            HB_CHECK_LAUNCH("conv_state");
+        }
+        return 0;
+    }
     conv_silu_kernel<<<dim3(T, n_unit + n_plain), HB_WAVE, 0, stream>>>(
         proj, ld, taps, conv_state, seq_of, seq_starts, slots, out, C, K, n_unit, unit_dim, n_scaled, scale,
         unit_eps, plain_dim, bias);

@@ -35,7 +35,7 @@ def conv_silu(proj, taps, conv_state, meta, out, n_unit, unit_dim, n_scaled, sca
     lib.call("recurrent", "hb_conv_silu", proj.data_ptr() + 4 * col0, ld, taps.data_ptr(), conv_state.data_ptr(),
              meta.seq_of.data_ptr(), meta.seq_starts.data_ptr(), meta.slots.data_ptr(), out.data_ptr(), T,
              meta.num_seqs, C, K, n_unit, unit_dim, n_scaled, float(scale), float(unit_eps), n_plain, plain_dim,
-             None if bias is None else bias.data_ptr(), _stream())
+             None if bias is None else bias.data_ptr(), int(meta.max_new), _stream())
 
 
 MAX_SSM_STATE = 256

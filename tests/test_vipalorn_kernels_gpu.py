@@ -109,6 +109,36 @@ def test_convolution_and_delta_rule_whole_in_portions_and_token_by_token(kv_head
             cache.free_slot(s)
 
 
+@pytest.mark.parametrize("D,units,C,biased", [(64, 3, 3 * 64 + 100, False), (128, 18, 18 * 128 + 4, True), (4, 5, 28, False),
+                                              (256, 4, 1024, False), (1, 0, 1540, True)])
+def test_convolution_of_quads_is_the_general_ones(D, units, C, biased):
+    """Rows of whole quads against rows of odd length (which take a wave a section): the sums and their activation are
+    the same operations, so plain sections are the same bits; unit ones differ by the order of their D squares, at most
+    (D + 3) roundings of half an ulp each in the sum and half of that in its root. Prompts and single tokens alike."""
+    section = min(256, C)
+    plain_n = -(-(C - units * D) // section) if C > units * D else 0
+    taps, bias = 0.25 + 0.3 * rand(C, 4, seed=5).to(DEV), 0.2 * rand(C, seed=6).to(DEV) if biased else None
+    got = []
+    for odd in (0, 3):
+        cache = Cache({0: (StateNeed((3, C)),)}, 64 * 16, 4096, torch.float32, DEV, max_slots=4)
+        conv_state, = cache.state_views(0)
+        slots = [cache.alloc_slot() for _ in range(3)]
+        outs = []
+        for step, counts in enumerate(([1, 1, 1], [300, 2, 11], [1, 1, 1], [1, 1, 1], [7, 1, 3], [1, 1, 1])):
+            meta = step_meta(cache, slots, counts)
+            T = sum(counts)
+            proj = torch.empty(T, C + 8 + odd, device=DEV)
+            proj[:, 4:4 + C] = rand(T, C, seed=20 + step, scale=1.5).to(DEV)
+            out = torch.empty(T, C, device=DEV)
+            recurrent.conv_silu(proj, taps, conv_state, meta, out, units, D, 1, 0.5, 1e-6, plain_n, section, col0=4, bias=bias)
+            outs += [out, conv_state[torch.tensor(slots, device=DEV)].clone()]
+        got.append(outs)
+    for a, b in zip(*got):
+        cut = units * D if a.dim() == 2 else 0
+        assert torch.equal(a[..., cut:], b[..., cut:])
+        assert torch.allclose(a[..., :cut], b[..., :cut], rtol=(D + 6) * 2.0 ** -24, atol=0)
+
+
 def test_gated_norm_a_head():
     T, heads, V = 5, 3, 70
     o, proj, w = rand(T, heads * V, seed=1), rand(T, heads * V + 9, seed=2), 1 + 0.1 * rand(V, seed=3)
