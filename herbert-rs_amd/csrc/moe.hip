@@ -21,147 +21,139 @@ HB_MODULE_ERROR_SLOT()
 #define MOE_MAX_E_PER_LANE 16
 
 // ------------------------------------------------------------------------ route
-// One wave a token; lane l holds the logits of experts l, l + 64, ...
-__global__ void __launch_bounds__(HB_WAVE)
-moe_route_kernel(const float* __restrict__ logits, int ld, const float* __restrict__ bias, int* __restrict__ chosen,
-                 float* __restrict__ weight, int E, int top) {
-    const int t = blockIdx.x, lane = threadIdx.x;
-    float z[MOE_MAX_E_PER_LANE];
-#pragma unroll
-    for (int i = 0; i < MOE_MAX_E_PER_LANE; ++i) {
-        const int e = lane + HB_WAVE * i;
-        z[i] = e < E ? logits[(size_t)t * ld + e] + (bias ? bias[e] : 0.f) : -INFINITY;
-    }
-    float first = 0.f, sum = 0.f;
-    for (int j = 0; j < top; ++j) {
-        float best = -INFINITY;
-        int at = 0x7fffffff;
-#pragma unroll
-        for (int i = 0; i < MOE_MAX_E_PER_LANE; ++i) {
-            const int e = lane + HB_WAVE * i;
-            if (e < E && (z[i] > best || (z[i] == best && e < at))) {
-                best = z[i];
-                at = e;
-            }
-        }
-#pragma unroll
-        for (int off = HB_WAVE / 2; off > 0; off >>= 1) {
-            const float ob = __shfl_xor(best, off, HB_WAVE);
-            const int oa = __shfl_xor(at, off, HB_WAVE);
-            if (ob > best || (ob == best && oa < at)) {
-                best = ob;
-                at = oa;
-            }
-        }
-        if (j == 0) first = best;                    // the first choice is the largest
-        const float p = expf(best - first);
-        sum += p;
-        if (lane == j % HB_WAVE) {                   // (the lane that divides it below)
-            chosen[(size_t)t * top + j] = at;
-            weight[(size_t)t * top + j] = p;
-        }
-#pragma unroll
-        for (int i = 0; i < MOE_MAX_E_PER_LANE; ++i)
-            if (lane + HB_WAVE * i == at) z[i] = -INFINITY;
-    }
-    for (int j = lane; j < top; j += HB_WAVE) weight[(size_t)t * top + j] /= sum;
-}
-
-// Routing by scores s = sigmoid(logit). The choice runs on s + correction, the weights on s itself:
+// Two ways to choose. By logits (by_scores 0): the largest logits (+ bias), weights a softmax over the chosen. By scores
+// s = sigmoid(logit): the choice runs on s + correction, the weights on s itself:
 // the experts form n_groups equal runs of adjacent experts, a group is worth the two highest of its
 // selection values, added; only the experts of the `keep` best groups can be chosen (the lower index of equals,
 // for groups as for experts), and the chosen experts' scores are divided by their sum + 1e-20.
 // Three parameters change the form: softmax_scores (s is the softmax of the logits over all E experts instead of
 // their sigmoids), worth_top (how many of a group's highest selection values make its worth: 2, or 1), renorm
 // (0: the weights are the chosen experts' scores as they are).
-// One wave a token; the scores lie in LDS.
-__global__ void __launch_bounds__(HB_WAVE)
-moe_route_scores_kernel(const float* __restrict__ logits, int ld, const float* __restrict__ correction,
-                        int* __restrict__ chosen, float* __restrict__ weight, int E, int top, int n_groups,
-                        int keep, int softmax_scores, int worth_top, int renorm) {
-    __shared__ float score[HB_WAVE * MOE_MAX_E_PER_LANE];
-    __shared__ float choice[HB_WAVE * MOE_MAX_E_PER_LANE];
-    __shared__ float worth[HB_WAVE * MOE_MAX_E_PER_LANE];
-    __shared__ int kept[HB_WAVE * MOE_MAX_E_PER_LANE];
-    const int t = blockIdx.x, lane = threadIdx.x;
-    const int size = E / n_groups;
-    float top_logit = -INFINITY, denom = 1.0f;
-    if (softmax_scores) {
-        for (int e = lane; e < E; e += HB_WAVE) top_logit = fmaxf(top_logit, logits[(size_t)t * ld + e]);
-        top_logit = hb_wave_max(top_logit);
-        float part = 0.f;
-        for (int e = lane; e < E; e += HB_WAVE) part += expf(logits[(size_t)t * ld + e] - top_logit);
-        denom = hb_wave_sum(part);
+struct RouteForm {
+    int by_scores, n_groups, keep, softmax_scores, worth_top, renorm;
+};
+
+// The largest of a wave's 64 numbers, in every lane.
+__device__ __forceinline__ unsigned wave_max_u32(unsigned v) {
+#define HB_STEP(CTRL, ROWS)                                                                      \
+    {                                                                                            \
+        const unsigned o = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false); \
+        v = v > o ? v : o;                                                                       \
     }
-    for (int e = lane; e < E; e += HB_WAVE) {
-        const float z = logits[(size_t)t * ld + e];
-        const float s = softmax_scores ? expf(z - top_logit) / denom : 1.0f / (1.0f + expf(-z));
-        score[e] = s;
-        choice[e] = s + (correction ? correction[e] : 0.f);
-    }
-    __syncthreads();
-    for (int g = lane; g < n_groups; g += HB_WAVE) {
-        float a = -INFINITY, b = -INFINITY;          // the largest and the second
-        for (int i = 0; i < size; ++i) {
-            const float c = choice[g * size + i];
-            if (c > a) {
-                b = a;
-                a = c;
-            } else if (c > b) {
-                b = c;
-            }
-        }
-        worth[g] = (size > 1 && worth_top > 1) ? a + b : a;
-    }
-    __syncthreads();
-    for (int g = lane; g < n_groups; g += HB_WAVE) {
-        int ahead = 0;
-        for (int o = 0; o < n_groups; ++o) ahead += (worth[o] > worth[g] || (worth[o] == worth[g] && o < g)) ? 1 : 0;
-        kept[g] = ahead < keep;
-    }
-    __syncthreads();
-    float z[MOE_MAX_E_PER_LANE];
+    HB_STEP(0x111, 0xf) HB_STEP(0x112, 0xf) HB_STEP(0x114, 0xf) HB_STEP(0x118, 0xf)   // along the rows of 16
+    HB_STEP(0x142, 0xa) HB_STEP(0x143, 0xc)                                           // a row's last lane to the next, two rows' to the others
+#undef HB_STEP
+    return (unsigned)__builtin_amdgcn_readlane((int)v, HB_WAVE - 1);
+}
+
+// The choice of one token by one wave: lane l holds experts l, l + 64, ... A selection value becomes a number that sorts
+// as it does (0: not to be chosen, 1: not a number), the largest of the wave's goes through the lanes' neighbours instead
+// of the LDS, and who holds it is a mask of lanes: some 150 clocks a chosen expert. Every wave of the workgroup calls it
+// together; a and b (E and n_groups floats) are the wave's own LDS, used only where there are groups.
+template <int PER>
+__device__ __forceinline__ void route_token(const float* __restrict__ logits, const float* __restrict__ bias, const RouteForm f,
+                                            int E, int top, float* a, float* b, int* chosen, int* chosen_too, float* weight,
+                                            bool stores) {
+    const int lane = threadIdx.x % HB_WAVE;
+    float c[PER], s[PER];                                // selection values and scores
+    unsigned key[PER];
 #pragma unroll
-    for (int i = 0; i < MOE_MAX_E_PER_LANE; ++i) {
+    for (int i = 0; i < PER; ++i) {
         const int e = lane + HB_WAVE * i;
-        z[i] = (e < E && kept[e / size]) ? choice[e] : -INFINITY;
+        s[i] = e < E ? logits[e] : -INFINITY;
+        c[i] = bias && e < E ? bias[e] : 0.f;
     }
-    float sum = 0.f;
+    if (f.by_scores) {
+        float top_logit = -INFINITY, denom = 1.0f;
+        if (f.softmax_scores) {
+#pragma unroll
+            for (int i = 0; i < PER; ++i) top_logit = fmaxf(top_logit, s[i]);
+            top_logit = hb_wave_max(top_logit);
+            float part = 0.f;
+#pragma unroll
+            for (int i = 0; i < PER; ++i)
+                if (lane + HB_WAVE * i < E) part += expf(s[i] - top_logit);
+            denom = hb_wave_sum(part);
+        }
+#pragma unroll
+        for (int i = 0; i < PER; ++i) s[i] = f.softmax_scores ? expf(s[i] - top_logit) / denom : 1.0f / (1.0f + expf(-s[i]));
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        c[i] += s[i];
+        const unsigned u = __float_as_uint(c[i] + 0.f);  // (-0 sorts as 0)
+        const bool live = lane + HB_WAVE * i < E && !(f.by_scores && c[i] == -INFINITY);
+        key[i] = !live ? 0u : c[i] != c[i] ? 1u : (u >> 31) ? ~u : u | 0x80000000u;
+    }
+    if (f.by_scores && f.n_groups > 1) {
+        const int size = E / f.n_groups;
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+            if (lane + HB_WAVE * i < E) a[lane + HB_WAVE * i] = c[i];
+        __syncthreads();
+        for (int g = lane; g < f.n_groups; g += HB_WAVE) {
+            float x = -INFINITY, y = -INFINITY;          // the largest and the second
+            for (int i = 0; i < size; ++i) {
+                const float v = a[g * size + i];
+                y = v > x ? x : v > y ? v : y;
+                x = v > x ? v : x;
+            }
+            b[g] = (size > 1 && f.worth_top > 1) ? x + y : x;
+        }
+        __syncthreads();
+        for (int g = lane; g < f.n_groups; g += HB_WAVE) {
+            int ahead = 0;
+            for (int o = 0; o < f.n_groups; ++o) ahead += (b[o] > b[g] || (b[o] == b[g] && o < g)) ? 1 : 0;
+            a[g] = ahead < f.keep ? 1.f : 0.f;           // (the values have been read: a group's worth needs no more of them)
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+            if (lane + HB_WAVE * i < E && a[(lane + HB_WAVE * i) / size] == 0.f) key[i] = 0u;
+    }
+    float first = 0.f, sum = 0.f;
     for (int j = 0; j < top; ++j) {
-        float best = -INFINITY;
-        int at = 0x7fffffff;
+        unsigned mine = key[0];
 #pragma unroll
-        for (int i = 0; i < MOE_MAX_E_PER_LANE; ++i) {
-            const int e = lane + HB_WAVE * i;
-            // (experts outside the kept groups and those already taken are never met: they are marked below)
-            if (e < E && z[i] != -INFINITY && (z[i] > best || at == 0x7fffffff || (z[i] == best && e < at))) {
-                best = z[i];
-                at = e;
+        for (int i = 1; i < PER; ++i) mine = mine > key[i] ? mine : key[i];
+        const unsigned best = wave_max_u32(mine);
+        int at = 0;                                      // (none left: only where the host's checks or infinite corrections allow it)
+        float value = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s[0]), 0));
+        bool found = best == 0u;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const unsigned long long who = __ballot(key[i] == best);
+            if (!found && who) {
+                const int l = __ffsll((long long)who) - 1;
+                found = true;
+                at = HB_WAVE * i + l;
+                value = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f.by_scores ? s[i] : c[i]), l));
+                if (lane == l) key[i] = 0u;
             }
         }
-#pragma unroll
-        for (int off = HB_WAVE / 2; off > 0; off >>= 1) {
-            const float ob = __shfl_xor(best, off, HB_WAVE);
-            const int oa = __shfl_xor(at, off, HB_WAVE);
-            if (oa != 0x7fffffff && (at == 0x7fffffff || ob > best || (ob == best && oa < at))) {
-                best = ob;
-                at = oa;
-            }
+        if (!f.by_scores) {
+            if (j == 0) first = value;                   // the first choice is the largest
+            value = expf(value - first);
         }
-        if (at == 0x7fffffff) at = 0;                // (fewer experts in the kept groups than `top`: the host refuses that)
-        const float s = score[at];
-        sum += s;
-        if (lane == j % HB_WAVE) {
-            chosen[(size_t)t * top + j] = at;
-            weight[(size_t)t * top + j] = s;
+        sum += value;
+        if (stores && lane == j % HB_WAVE) {             // (the lane that divides it below)
+            chosen[j] = at;
+            if (chosen_too) chosen_too[j] = at;
+            weight[j] = value;
         }
-#pragma unroll
-        for (int i = 0; i < MOE_MAX_E_PER_LANE; ++i)
-            if (lane + HB_WAVE * i == at) z[i] = -INFINITY;
     }
-    if (!renorm) return;
-    const float total = sum + 1e-20f;
-    for (int j = lane; j < top; j += HB_WAVE) weight[(size_t)t * top + j] /= total;
+    if (!stores || (f.by_scores && !f.renorm)) return;
+    const float total = f.by_scores ? sum + 1e-20f : sum;
+    for (int j = lane; j < top; j += HB_WAVE) weight[j] /= total;
+}
+
+template <int PER>
+__global__ void __launch_bounds__(HB_WAVE)
+moe_route_kernel(const float* __restrict__ logits, int ld, const float* __restrict__ bias, int* __restrict__ chosen,
+                 float* __restrict__ weight, int E, int top, RouteForm form) {
+    __shared__ float a[HB_WAVE * PER], b[HB_WAVE * PER];
+    const size_t t = blockIdx.x;
+    route_token<PER>(logits + t * ld, bias, form, E, top, a, b, chosen + t * top, nullptr, weight + t * top, true);
 }
 
 // ------------------------------------------------------------------------ group
@@ -170,54 +162,146 @@ moe_route_scores_kernel(const float* __restrict__ logits, int ld, const float* _
 // row_of[pair] = row. Every block counts all experts' pairs for itself (a histogram in LDS), so that
 // no kernel has to run before it. Experts from `real` on have no matrices (their output is their input): their
 // pairs get rows like any others, but their tiles are marked as holding nothing, so no product runs on them.
-__global__ void __launch_bounds__(256)
+// Each of the 16 waves goes over a run of the pairs of its own, twice: counting, then placing behind the waves before it
+// (two barriers in all). Choice and placing of 2,048 tokens, 8 of 64 experts: 64 us with a workgroup of four waves that met
+// at three barriers every 256 pairs, and a choice through the LDS; 12 now.
+__global__ void __launch_bounds__(1024)
 moe_place_kernel(const int* __restrict__ chosen, int* __restrict__ counts, int* __restrict__ order,
                  int* __restrict__ row_of, int* __restrict__ tile_expert, int* __restrict__ tile_row0,
                  int* __restrict__ tile_rows, int A, int E, int max_tiles, int real) {
     __shared__ int hist[HB_WAVE * MOE_MAX_E_PER_LANE];
-    __shared__ int wave_n[4];
-    __shared__ int base;
+    __shared__ int wave_n[16], firsts[16], tiles[16];
     const int e = blockIdx.x;
-    for (int i = threadIdx.x; i < E; i += blockDim.x) hist[i] = 0;
+    const int lane = threadIdx.x & (HB_WAVE - 1), wave = threadIdx.x / HB_WAVE;
+    const int run = ((A + 1023) / 1024) * HB_WAVE;       // pairs of a wave
+    const int a0 = min(A, wave * run), a1 = min(A, a0 + run);
+    for (int i = threadIdx.x; i < E; i += 1024) hist[i] = 0;
     __syncthreads();
-    for (int a = threadIdx.x; a < A; a += blockDim.x) atomicAdd(&hist[chosen[a]], 1);
+    int hits = 0;
+    for (int at = a0; at < a1; at += 4 * HB_WAVE) {
+        int x[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = at + i * HB_WAVE + lane < a1 ? chosen[at + i * HB_WAVE + lane] : -1;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (x[i] >= 0) atomicAdd(&hist[x[i]], 1);
+            hits += __popcll(__ballot(x[i] == e));
+        }
+    }
+    if (lane == 0) wave_n[wave] = hits;
     __syncthreads();
-    int first = 0, tile0 = 0;
-    for (int i = 0; i < (e < E ? e : E); ++i) {
-        first += hist[i];
-        tile0 += (hist[i] + MOE_TILE_M - 1) / MOE_TILE_M;
+    const int before = (int)threadIdx.x < min(e, E) ? hist[threadIdx.x] : 0;       // (E is at most the workgroup's threads)
+    int first = before, tile0 = (before + MOE_TILE_M - 1) / MOE_TILE_M;
+#pragma unroll
+    for (int off = HB_WAVE / 2; off > 0; off >>= 1) {
+        first += __shfl_xor(first, off, HB_WAVE);
+        tile0 += __shfl_xor(tile0, off, HB_WAVE);
+    }
+    if (lane == 0) {
+        firsts[wave] = first;
+        tiles[wave] = tile0;
+    }
+    __syncthreads();
+    first = tile0 = 0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+        first += firsts[w];
+        tile0 += tiles[w];
     }
     if (e == E) {
-        for (int i = tile0 + threadIdx.x; i < max_tiles; i += blockDim.x) tile_expert[i] = -1;
+        for (int i = tile0 + threadIdx.x; i < max_tiles; i += 1024) tile_expert[i] = -1;
         return;
     }
     const int count = hist[e];
     if (threadIdx.x == 0) counts[e] = count;
-    for (int i = threadIdx.x; i * MOE_TILE_M < count; i += blockDim.x) {
+    for (int i = threadIdx.x; i * MOE_TILE_M < count; i += 1024) {
         tile_expert[tile0 + i] = e < real ? e : -1;
         tile_row0[tile0 + i] = first + i * MOE_TILE_M;
         tile_rows[tile0 + i] = count - i * MOE_TILE_M < MOE_TILE_M ? count - i * MOE_TILE_M : MOE_TILE_M;
     }
-    if (count == 0) return;
-    if (threadIdx.x == 0) base = first;
-    __syncthreads();
-    const int lane = threadIdx.x & (HB_WAVE - 1), wave = threadIdx.x / HB_WAVE;
-    for (int a0 = 0; a0 < A; a0 += 256) {
-        const int a = a0 + threadIdx.x;
-        const bool hit = a < A && chosen[a] == e;
-        const unsigned long long mask = __ballot(hit);
-        if (lane == 0) wave_n[wave] = __popcll(mask);
-        __syncthreads();
-        int before = 0;
-        for (int w = 0; w < wave; ++w) before += wave_n[w];
-        if (hit) {
-            const int row = base + before + __popcll(mask & ((1ull << lane) - 1ull));
-            order[row] = a;
-            row_of[a] = row;
+    if (hits == 0) return;
+    int row = first;
+    for (int w = 0; w < wave; ++w) row += wave_n[w];
+    for (int at = a0; at < a1; at += 4 * HB_WAVE) {
+        int x[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = at + i * HB_WAVE + lane < a1 ? chosen[at + i * HB_WAVE + lane] : -1;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const unsigned long long mask = __ballot(x[i] == e);
+            if (x[i] == e) {
+                const int pair = at + i * HB_WAVE + lane, r = row + __popcll(mask & ((1ull << lane) - 1ull));
+                order[r] = pair;
+                row_of[pair] = r;
+            }
+            row += __popcll(mask);
         }
-        __syncthreads();
-        if (threadIdx.x == 0) base += wave_n[0] + wave_n[1] + wave_n[2] + wave_n[3];
-        __syncthreads();
+    }
+}
+
+// Both of a step of few tokens (decode) in one launch of one workgroup, a wave a token: the choices stay in LDS, a thread
+// a pair counts the pairs of its expert before it. Bound by its own chain of latencies: 8 of 64 experts for one token
+// 4.4 us, for 8 tokens 5.9 (16 and 17 by the two kernels before; 16 tokens 8.1, which the two kernels now do in 6.7: the
+// line lies at 8 tokens).
+#define FEW_TOKENS 8
+#define FEW_PAIRS 128
+template <int PER>
+__global__ void __launch_bounds__(HB_WAVE * FEW_TOKENS)
+moe_route_few_kernel(const float* __restrict__ logits, int ld, const float* __restrict__ bias, int* __restrict__ chosen,
+                     float* __restrict__ weight, int* __restrict__ counts, int* __restrict__ order, int* __restrict__ row_of,
+                     int* __restrict__ tile_expert, int* __restrict__ tile_row0, int* __restrict__ tile_rows, int T, int E,
+                     int top, int max_tiles, int real, RouteForm form) {
+    __shared__ float a[FEW_TOKENS][HB_WAVE * PER], b[FEW_TOKENS][HB_WAVE * PER];
+    __shared__ __attribute__((aligned(16))) int pair_expert[FEW_PAIRS + 4];
+    __shared__ int hist[HB_WAVE * PER];
+    __shared__ unsigned start[HB_WAVE * PER + 1];        // an expert's first tile (upper half) and row (lower half)
+    const int lane = threadIdx.x & (HB_WAVE - 1), wave = threadIdx.x / HB_WAVE;
+    const int A = T * top, threads = blockDim.x;
+    for (int i = threadIdx.x; i < HB_WAVE * PER; i += threads) hist[i] = 0;
+    const size_t t = min(wave, T - 1);
+    route_token<PER>(logits + t * ld, bias, form, E, top, a[wave], b[wave], chosen + t * top, pair_expert + t * top,
+                     weight + t * top, wave < T);
+    __syncthreads();
+    for (int p = threadIdx.x; p < A; p += threads) atomicAdd(&hist[pair_expert[p]], 1);
+    __syncthreads();
+    if (wave == 0) {                                     // PER experts a lane
+        unsigned own[PER], sum = 0;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int n = hist[lane * PER + i];
+            own[i] = sum;
+            sum += ((unsigned)((n + MOE_TILE_M - 1) / MOE_TILE_M) << 16) | (unsigned)n;
+        }
+        unsigned upto = sum;
+#pragma unroll
+        for (int off = 1; off < HB_WAVE; off <<= 1) {
+            const unsigned o = __shfl_up(upto, off, HB_WAVE);
+            if (lane >= off) upto += o;
+        }
+#pragma unroll
+        for (int i = 0; i < PER; ++i) start[lane * PER + i] = upto - sum + own[i];
+        if (lane == HB_WAVE - 1) start[HB_WAVE * PER] = upto;
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < E; e += threads) {
+        const int n = hist[e], tile0 = start[e] >> 16, row0 = start[e] & 0xffff;
+        counts[e] = n;
+        for (int i = 0; i * MOE_TILE_M < n; ++i) {
+            tile_expert[tile0 + i] = e < real ? e : -1;
+            tile_row0[tile0 + i] = row0 + i * MOE_TILE_M;
+            tile_rows[tile0 + i] = min(n - i * MOE_TILE_M, MOE_TILE_M);
+        }
+    }
+    for (int i = (int)(start[HB_WAVE * PER] >> 16) + threadIdx.x; i < max_tiles; i += threads) tile_expert[i] = -1;
+    for (int p = threadIdx.x; p < A; p += threads) {
+        const int e = pair_expert[p];
+        int r = start[e] & 0xffff;
+        for (int q = 0; q < p; q += 4) {
+            const int4 v = *(const int4*)(pair_expert + q);
+            r += (v.x == e) + (v.y == e && q + 1 < p) + (v.z == e && q + 2 < p) + (v.w == e && q + 3 < p);
+        }
+        order[r] = p;
+        row_of[p] = r;
     }
 }
 
@@ -238,13 +322,26 @@ extern "C" int hb_moe_route(const float* logits, const float* bias, int* chosen,
     const long long A = (long long)T * top;
     HB_REQUIRE(A < (1ll << 30), "moe: too many (token, expert) pairs");
     HB_REQUIRE(max_tiles >= (A + MOE_TILE_M - 1) / MOE_TILE_M + E, "moe: the tile list is too short");
-    if (by_scores)
-        moe_route_scores_kernel<<<T, HB_WAVE, 0, stream>>>(logits, ld, bias, chosen, weight, E, top, n_groups, keep,
-                                                           softmax_scores, worth_top, renorm);
-    else
-        moe_route_kernel<<<T, HB_WAVE, 0, stream>>>(logits, ld, bias, chosen, weight, E, top);
+    const RouteForm form = {by_scores, n_groups, keep, softmax_scores, worth_top, renorm};
+    if (T <= FEW_TOKENS && A <= FEW_PAIRS && E <= HB_WAVE * 4) {
+#define HB_FEW(PER)                                                                                                      \
+    moe_route_few_kernel<PER><<<1, HB_WAVE * (T < 4 ? 4 : T), 0, stream>>>(logits, ld, bias, chosen, weight, counts, order, \
+        row_of, tile_expert, tile_row0, tile_rows, T, E, top, max_tiles, real, form)
+        if (E <= HB_WAVE) HB_FEW(1);
+        else if (E <= HB_WAVE * 2) HB_FEW(2);
+        else HB_FEW(4);
+#undef HB_FEW
+        HB_CHECK_LAUNCH("moe_route_few");
+        return 0;
+    }
+#define HB_ROUTE(PER) moe_route_kernel<PER><<<T, HB_WAVE, 0, stream>>>(logits, ld, bias, chosen, weight, E, top, form)
+    if (E <= HB_WAVE) HB_ROUTE(1);
+    else if (E <= HB_WAVE * 2) HB_ROUTE(2);
+    else if (E <= HB_WAVE * 4) HB_ROUTE(4);
+    else HB_ROUTE(MOE_MAX_E_PER_LANE);
+#undef HB_ROUTE
     HB_CHECK_LAUNCH("moe_route");
-    moe_place_kernel<<<E + 1, 256, 0, stream>>>(chosen, counts, order, row_of, tile_expert, tile_row0, tile_rows, (int)A, E, max_tiles, real);
+    moe_place_kernel<<<E + 1, 1024, 0, stream>>>(chosen, counts, order, row_of, tile_expert, tile_row0, tile_rows, (int)A, E, max_tiles, real);
     HB_CHECK_LAUNCH("moe_place");
     return 0;
 }

@@ -319,6 +319,49 @@ def test_grouped_products_of_any_rows(M, G, N, K, pad):
             assert bool((got[:, g, cols:] == 3.0).all())
 
 
+@pytest.mark.parametrize("E,top,groups,keep,score,logit_form", [
+    (1, 1, 1, 1, "sigmoid", False), (64, 8, 8, 4, "sigmoid", False), (64, 16, 1, 1, "softmax", True), (65, 3, 5, 2, "softmax", False),
+    (128, 8, 1, 1, "sigmoid", False), (130, 65, 1, 1, "sigmoid", True), (200, 5, 200, 7, "sigmoid", False),
+    (256, 16, 16, 2, "softmax", False), (300, 6, 3, 1, "sigmoid", False), (1024, 9, 1, 1, "sigmoid", True)])
+def test_routing_of_few_tokens_is_the_many_tokens_one(E, top, groups, keep, score, logit_form):
+    """The choice is exact: equals by index, zeros of both signs are equals. Steps of 1, 8 and 9 tokens are rows of the
+    large step's, bit for bit, and rows, counts and tiles follow from the choice alone."""
+    T = 417
+    logits = rand(T, E + 1, seed=1, scale=1.5)
+    logits[::3] = (logits[::3] * 2).round() / 2             # many equals
+    logits[1::7] *= -0.0 if E < 65 else 1.0
+    bias = (0.25 * rand(E, seed=2)).round() if E % 2 else None
+
+    def go(rows):
+        n = rows.shape[0]
+        r = moe.Routing(torch.full((moe.Routing.ints_needed(n, E, top),), -7, dtype=torch.int32, device=DEV),
+                        torch.empty(n, top, device=DEV), n, E, top, real=max(1, E - 2))
+        moe.route(rows.to(DEV), None if bias is None else bias.to(DEV), r, scores=not logit_form, groups=groups, keep=keep, score=score)
+        chosen, pairs = r.chosen.view(n, top).cpu(), n * top
+        flat = chosen.flatten().long()
+        order = torch.sort(flat, stable=True).indices.int()
+        assert torch.equal(r.order.cpu(), order)
+        assert torch.equal(r.row_of.cpu()[order.long()], torch.arange(pairs, dtype=torch.int32))
+        counts = torch.bincount(flat, minlength=E)
+        assert torch.equal(r.counts.cpu().long(), counts)
+        tiles, row = [], 0
+        for e, c in enumerate(counts.tolist()):
+            tiles += [(e if e < r.real else -1, row + i, min(64, c - i)) for i in range(0, c, 64)]
+            row += c
+        got = list(zip(r.tile_expert.tolist(), r.tile_row0.tolist(), r.tile_rows.tolist()))
+        assert got[:len(tiles)] == tiles and all(t[0] == -1 for t in got[len(tiles):])
+        return chosen, r.weight.cpu()
+
+    chosen, weight = go(logits)
+    if logit_form:
+        values = logits[:, :E] + (0 if bias is None else bias)
+        assert torch.equal(chosen.long(), torch.sort(-values, dim=-1, stable=True).indices[:, :top])
+        assert torch.allclose(weight, torch.softmax(torch.gather(values, 1, chosen.long()), -1), rtol=1e-5, atol=1e-7)
+    for a, n in ((0, 1), (1, 8), (9, 9), (18, 3)):
+        c, w = go(logits[a:a + n])
+        assert torch.equal(c, chosen[a:a + n]) and torch.equal(w, weight[a:a + n])
+
+
 @pytest.mark.parametrize("T,E,top", [(1, 3, 3), (9, 5, 2), (300, 16, 4), (70, 130, 7)])
 def test_routing_groups_and_products(T, E, top):
     W, F = 64, 96                                          # (K in steps of 32: what the matrix-core product takes)
