@@ -148,7 +148,7 @@ def gated_delta(qkv, proj, b_off, a_off, a_log, dt_bias, state, meta, out, kv_he
             return
         lib.call("recurrent", "hb_gated_delta", qkv.data_ptr(), C, None, 0, 0, 0, None, None, decay.data_ptr(),
                  state.data_ptr(), meta.seq_starts.data_ptr(), meta.slots.data_ptr(), out.data_ptr(), meta.num_seqs,
-                 kv_heads, heads, D, V, 0, float(out_scale), _stream())
+                 kv_heads, heads, D, V, 0, float(out_scale), int(meta.max_new), _stream())
         return
     if decay is not None:
         _check(decay, "decay", torch.float32, (T, heads * D))
@@ -175,7 +175,7 @@ def gated_delta(qkv, proj, b_off, a_off, a_log, dt_bias, state, meta, out, kv_he
              None if decay is not None else a_log.data_ptr(), None if decay is not None else dt_bias.data_ptr(),
              None if decay is None else decay.data_ptr(), state.data_ptr(), meta.seq_starts.data_ptr(),
              meta.slots.data_ptr(),
-             out.data_ptr(), meta.num_seqs, kv_heads, heads, D, V, 1, float(out_scale), _stream())
+             out.data_ptr(), meta.num_seqs, kv_heads, heads, D, V, 1, float(out_scale), int(meta.max_new), _stream())
 
 
 def gated_head_norm(o, proj, g_off, weight, out, heads, V, eps, gate="silu"):

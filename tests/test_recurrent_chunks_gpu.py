@@ -21,7 +21,7 @@ def rule(q, k, v, beta, decay, S):
         u = v[t] if beta is None else beta[t][:, None] * (v[t] - (S * k[t][:, :, None]).sum(1))
         S = S + k[t][:, :, None] * u[:, None, :]
         out.append((S * q[t][:, :, None]).sum(1))
-    return torch.stack(out), S
+    return torch.stack(out) if out else v, S
 
 
 def step(lengths, kv_heads, heads, D, V, kind, rate, seed=0):
@@ -111,3 +111,26 @@ def test_rows_that_are_not_finite_reach_no_earlier_token(kind, place):
     assert torch.equal(got[150:], clean[150:]) and torch.equal(got[:, 0], clean[:, 0])
     assert torch.allclose(got[:place, 1], clean[:place, 1], rtol=0, atol=0) and bool(got[place:150, 1].isnan().all())
     assert torch.equal(wild[1], state[1]) and torch.equal(wild[2, 0], state[2, 0]) and bool(wild[2, 1].isnan().all())
+
+
+@pytest.mark.parametrize("kv_heads,heads,D,V", [(1, 1, 1, 4), (2, 4, 33, 36), (3, 3, 64, 100), (2, 4, 128, 128), (1, 2, 200, 8), (1, 1, 256, 64),
+                                                (2, 2, 48, 37)])
+@pytest.mark.parametrize("kind", ["head", "channel", "linear"])
+def test_one_token_a_sequence_is_a_step_of_the_walk(kv_heads, heads, D, V, kind):
+    """A step that brings at most one token a sequence (one brings none: its state stays) against float64, beside the walk
+    that takes longer portions: sums of D float32 products and what they are made of, (D + 16) roundings of the terms' sizes."""
+    from herbert_rs_amd.kernels import recurrent
+    lengths = [1, 0, 1, 1]
+    qkv, proj, a_log, dt_bias, decay, state, meta = step(lengths, kv_heads, heads, D, V, kind, 0.0, seed=D + V)
+    want, want_state = expected(qkv, proj, a_log, dt_bias, decay, state, lengths, kv_heads, heads, D, V, kind)
+    size = 4.0 + float(want.abs().max()) + float(want_state.abs().max())
+    for longest in (1, 2):
+        meta.max_new = longest
+        out, held = torch.full((3, heads * V), 7.0, device=dev()), state.to(dev())
+        recurrent.gated_delta(qkv.to(dev()), None if kind == "linear" else proj.to(dev()), 0, heads, a_log.to(dev()), dt_bias.to(dev()),
+                              held, meta, out, kv_heads, heads, D, V, decay=None if kind == "head" else decay.reshape(3, heads * D).to(dev()),
+                              correction=kind != "linear", out_scale=0.5)
+        slack = (D + 16) * 2.0 ** -24 * size * max(1.0, D ** 0.5)
+        assert float((out.cpu().view(3, heads, V).double() - want).abs().max()) <= slack, longest
+        assert float((held.cpu().double() - want_state).abs().max()) <= slack, longest
+        assert torch.equal(held.cpu()[meta.slots[1].item()], state[meta.slots[1].item()])
