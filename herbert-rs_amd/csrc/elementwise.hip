@@ -13,6 +13,7 @@
 //   the three fused  crates/backends/backend_metal/shaders/head_norm_rope_kv_append.metal:37-110 (norm, rotation, append)
 //   SwiGLU           crates/backends/backend_common/src/kernels.rs:676-687: g / (1 + exp(-g)) * u
 #include "common.h"
+#include "mfma_f32.h"
 
 HB_MODULE_ERROR_SLOT()
 
@@ -1304,14 +1305,15 @@ extern "C" int hb_gate_heads(const void* attn, int dtype, const float* gate_rows
 //     g = gelu_tanh(W_gate x) * e;   y = W_proj g;   x <- x + y / sqrt(mean(y^2) + eps) * w
 // x f32 [T, H] in place; W_gate [D, H], the table, and W_proj transposed [D, H] in one storage type; all arithmetic
 // float32. Three kernels, each of which fills the chip for a few tokens as for thousands:
-//   gate: a workgroup takes SIDE_TOKENS tokens and 4 x RW rows of W_gate (RW = 4; eight rows a wave were no faster); a wave takes RW of them, its lanes
-//     share a row's columns (whole lines of the matrix), every x is read once for the wave's RW rows; the sums
-//     over the lanes run in a fixed order; g f32 [T, D]; a step of few tokens gives a row to a whole workgroup;
+//   gate: tiles of tokens and gates on the matrix cores, in float32; a step of few tokens gives SIDE_TOKENS tokens and a row of
+//     W_gate to a workgroup, its lanes share the row's columns (whole lines of the matrix); all sums run in a fixed order;
+//     g f32 [T, D];
 //   proj: a workgroup takes SIDE_TOKENS tokens (their g in LDS) and 64 columns of y; a lane takes a column,
-//     its weights W_proj^T [j, c] lie side by side for neighbouring lanes, the four waves a quarter of the
+//     its weights W_proj^T [j, c] lie side by side for neighbouring lanes, the 16 waves a sixteenth of the
 //     gates each; y f32 [T, H];
 //   add: a workgroup a token: the row's mean of squares in a fixed order, then x += y / rms * w.
 #define SIDE_TOKENS 8
+// (many tokens: a wave takes RW rows of W_gate, its lanes share a row's columns, every x is read once for them)
 template <class TW, int RW>
 __global__ void __launch_bounds__(256)
 token_gate_kernel(const float* __restrict__ x, const int* __restrict__ tokens, const TW* __restrict__ table,
@@ -1353,6 +1355,103 @@ token_gate_kernel(const float* __restrict__ x, const int* __restrict__ tokens, c
         }
 }
 
+// (many tokens, rows of whole quads: 32 tokens x 32 gates a workgroup, a wave every eighth 16 columns of x with float32
+//  products on the matrix cores, 16 columns of a row in four lanes whose order of k both operands share. Sums start anew
+//  every 16 columns (one chain over all of a wave's would triple the error of a lane's own sums); the waves' meet in
+//  LDS. Tokens' tiles run along the grid's x, a multiple of the 8 XCDs: a tile's x is read into one L2.
+//  Bound by latency up to some 300 tokens, then by the float32 products: 256 gates of 2,048 columns, 300 tokens 26 -> 20 us,
+//  1,500 70 -> 35; 4,096 tokens of 2,560 columns and 128 gates 110 -> 44; the error against 64 bits is the same.)
+#define SIDE_TILE 32
+#define SIDE_SPLIT 8
+#define SIDE_AHEAD 4          // loads in flight, in steps of 16 columns
+template <class TW>
+struct alignas(4 * sizeof(TW)) SideQuad {
+    TW v[4];
+    __device__ __forceinline__ f32x4 values(bool in) const {
+        f32x4 r;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = in ? hb_to_float(v[i]) : 0.f;
+        return r;
+    }
+};
+template <class TW>
+__global__ void __launch_bounds__(64 * SIDE_SPLIT)
+token_gate_tile_kernel(const float* __restrict__ x, const int* __restrict__ tokens, const TW* __restrict__ table,
+                       int table_ld, int col0, const TW* __restrict__ w_gate, float* __restrict__ g, bf16* __restrict__ g16,
+                       int T, int H, int D) {
+    __shared__ f32x4 sums[SIDE_SPLIT][4][HB_WAVE];
+    constexpr int STRIDE = 16 * SIDE_SPLIT;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int t0 = blockIdx.x * SIDE_TILE, j0 = blockIdx.y * SIDE_TILE;
+    if (t0 >= T) return;
+    const int row = lane % 16, part = (lane / 16) * 4;
+    const float* xr[2];
+    const TW* wr[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {          // (rows past the end read the last one again: their sums are never stored)
+        xr[i] = x + (size_t)min(t0 + 16 * i + row, T - 1) * H;
+        wr[i] = w_gate + (size_t)min(j0 + 16 * i + row, D - 1) * H;
+    }
+    f32x4 total[2][2];
+    SideQuad<float> xq[SIDE_AHEAD][2];
+    SideQuad<TW> wq[SIDE_AHEAD][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int n = 0; n < 2; ++n) total[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto fetch = [&](int d, int c) {       // (past the row's end the last quad again, which counts as zeros: no load under a condition)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            xq[d][i] = *(const SideQuad<float>*)(xr[i] + min(c, H - 4));
+            wq[d][i] = *(const SideQuad<TW>*)(wr[i] + min(c, H - 4));
+        }
+    };
+#pragma unroll
+    for (int d = 0; d < SIDE_AHEAD; ++d) fetch(d, 16 * wave + part + STRIDE * d);
+    for (int c = 16 * wave + part; c - part < H; c += STRIDE * SIDE_AHEAD) {
+#pragma unroll
+        for (int d = 0; d < SIDE_AHEAD; ++d) {
+            const bool in = c + STRIDE * d < H;
+            const f32x4 xa[2] = {xq[d][0].values(in), xq[d][1].values(in)};
+            const f32x4 wa[2] = {wq[d][0].values(in), wq[d][1].values(in)};
+            fetch(d, c + STRIDE * (d + SIDE_AHEAD));
+            f32x4 acc[2][2];
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int n = 0; n < 2; ++n)
+                        acc[i][n] = mfma_k4(wa[n][k], xa[i][k], k ? acc[i][n] : f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int n = 0; n < 2; ++n) total[i][n] += acc[i][n];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int n = 0; n < 2; ++n) sums[wave][2 * i + n][lane] = total[i][n];
+    __syncthreads();
+    if (wave >= 4) return;
+    f32x4 z4 = sums[0][wave][lane] + sums[1][wave][lane];
+#pragma unroll
+    for (int o = 2; o < SIDE_SPLIT; o += 2) z4 += sums[o][wave][lane] + sums[o + 1][wave][lane];
+    const int t = t0 + 16 * (wave / 2) + row, j = j0 + 16 * (wave % 2) + part;
+    if (t >= T) return;
+    const TW* e = table + (size_t)tokens[t] * table_ld + col0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (j + i >= D) break;
+        const float z = z4[i];
+        const float gelu = 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
+        const float out = gelu * hb_to_float(e[j + i]);
+        if (g16) g16[(size_t)t * D + j + i] = hb_from_float<bf16>(out);       // (for a product on the matrix cores)
+        else g[(size_t)t * D + j + i] = out;
+    }
+}
+
 // (few tokens: all four waves of a workgroup share one row of W_gate, a quarter of its columns each)
 template <class TW>
 __global__ void __launch_bounds__(256)
@@ -1384,57 +1483,62 @@ token_gate_few_kernel(const float* __restrict__ x, const int* __restrict__ token
     }
 }
 
-// (64 columns of y a workgroup; wave q takes the q-th quarter of the D gates, and the four partial sums of a
-// column are added in their order)
+// (64 columns of y a workgroup; wave q takes the q-th sixteenth of the D gates, and the partial sums of a column are added
+//  in a fixed order. Bound by latency: 256 gates, 2,048 columns, 8 tokens 10.5 -> 4.6 us
+//  with 16 waves where there were four, a gate's tokens side by side in LDS)
+#define SIDE_WAVES 16
 template <class TW>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(64 * SIDE_WAVES)
 token_proj_kernel(const float* __restrict__ g, const TW* __restrict__ w_proj_t, float* __restrict__ y, int T, int H,
                   int D) {
-    extern __shared__ float side_g[];              // [SIDE_TOKENS][D], then the partial sums [3][SIDE_TOKENS][64]
-    float* const partial = side_g + SIDE_TOKENS * D;
+    extern __shared__ __attribute__((aligned(16))) float side_g[];      // [D][SIDE_TOKENS], then in its place the sums [SIDE_WAVES][SIDE_TOKENS][64]
     const int t0 = blockIdx.y * SIDE_TOKENS;
     const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
-    const int c = blockIdx.x * 64 + lane;
-    for (int i = threadIdx.x; i < SIDE_TOKENS * D; i += 256) {
-        const int k = i / D;
-        side_g[i] = t0 + k < T ? g[(size_t)(t0 + k) * D + (i - k * D)] : 0.f;
+    const int c = min((int)blockIdx.x * 64 + lane, H - 1);
+    for (int i = threadIdx.x; i < SIDE_TOKENS * D; i += 64 * SIDE_WAVES) {
+        const int k = i / D, j = i - k * D;
+        side_g[j * SIDE_TOKENS + k] = t0 + k < T ? g[(size_t)(t0 + k) * D + j] : 0.f;
     }
-    __syncthreads();
-    const int per = (D + 3) / 4;
+    const int per = (D + SIDE_WAVES - 1) / SIDE_WAVES;
     const int j0 = q * per, j1 = j0 + per < D ? j0 + per : D;
     float acc[SIDE_TOKENS];
 #pragma unroll
     for (int k = 0; k < SIDE_TOKENS; ++k) acc[k] = 0.f;
-    if (c < H) {
-        // sixteen weights asked for at once (one after the other, each would wait for memory), then their products
-        for (int j = j0; j < j1; j += 16) {
-            float w[16];
+    // sixteen weights asked for at once (one after the other, each would wait for memory), then their products
+    float w[16];
+    auto fetch = [&](int j) {
 #pragma unroll
-            // (no load stands under a condition, which would make it wait for the one before: past the end the last
-            //  weight is read again and counts as zero)
-            for (int o = 0; o < 16; ++o) w[o] = hb_to_float(w_proj_t[(size_t)(j + o < j1 ? j + o : j1 - 1) * H + c]);
-#pragma unroll
-            for (int o = 0; o < 16; ++o) {
-                const int at = j + o < j1 ? j + o : j1 - 1;
-                const float wo = j + o < j1 ? w[o] : 0.f;
-#pragma unroll
-                for (int k = 0; k < SIDE_TOKENS; ++k) acc[k] = fmaf(wo, side_g[k * D + at], acc[k]);
-            }
-        }
-    }
-    if (q > 0) {
-#pragma unroll
-        for (int k = 0; k < SIDE_TOKENS; ++k) partial[((q - 1) * SIDE_TOKENS + k) * 64 + lane] = acc[k];
-    }
+        // (no load stands under a condition, which would make it wait for the one before: past the end the last
+        //  weight is read again and is not used)
+        for (int o = 0; o < 16; ++o) w[o] = hb_to_float(w_proj_t[(size_t)min(j + o, D - 1) * H + c]);
+    };
+    fetch(j0);
     __syncthreads();
-    if (q > 0 || c >= H) return;
+    for (int j = j0; j < j1; j += 16) {
 #pragma unroll
-    for (int k = 0; k < SIDE_TOKENS; ++k) {
-        float sum = acc[k];
-#pragma unroll
-        for (int o = 0; o < 3; ++o) sum += partial[(o * SIDE_TOKENS + k) * 64 + lane];
-        if (t0 + k < T) y[(size_t)(t0 + k) * H + c] = sum;
+        for (int o = 0; o < 16; ++o) {
+            if (j + o >= j1) break;
+            const float4 a = *(const float4*)(side_g + (j + o) * SIDE_TOKENS), b = *(const float4*)(side_g + (j + o) * SIDE_TOKENS + 4);
+            acc[0] = fmaf(w[o], a.x, acc[0]), acc[1] = fmaf(w[o], a.y, acc[1]);
+            acc[2] = fmaf(w[o], a.z, acc[2]), acc[3] = fmaf(w[o], a.w, acc[3]);
+            acc[4] = fmaf(w[o], b.x, acc[4]), acc[5] = fmaf(w[o], b.y, acc[5]);
+            acc[6] = fmaf(w[o], b.z, acc[6]), acc[7] = fmaf(w[o], b.w, acc[7]);
+        }
+        if (j + 16 < j1) fetch(j + 16);
     }
+    __syncthreads();                                // (every wave has read its gates)
+#pragma unroll
+    for (int k = 0; k < SIDE_TOKENS; ++k) side_g[(q * SIDE_TOKENS + k) * 64 + lane] = acc[k];
+    __syncthreads();
+    if (q >= SIDE_TOKENS || t0 + q >= T || blockIdx.x * 64 + lane >= H) return;
+    float part[SIDE_WAVES];
+#pragma unroll
+    for (int o = 0; o < SIDE_WAVES; ++o) part[o] = side_g[(o * SIDE_TOKENS + q) * 64 + lane];
+#pragma unroll
+    for (int step = 1; step < SIDE_WAVES; step *= 2)
+#pragma unroll
+        for (int o = 0; o < SIDE_WAVES; o += 2 * step) part[o] += part[o + step];
+    y[(size_t)(t0 + q) * H + c] = part[0];
 }
 
 __global__ void __launch_bounds__(256)
@@ -1463,16 +1567,21 @@ extern "C" int hb_token_side(float* x, const int* tokens, const void* table, int
     }
     HB_REQUIRE(T > 0 && H > 0 && D > 0, "token input: empty input");
     HB_REQUIRE(col0 >= 0 && col0 + D <= table_ld, "token input: the layer's columns lie outside the table's rows");
-    const size_t lds = ((size_t)SIDE_TOKENS * D + 3 * SIDE_TOKENS * 64) * sizeof(float);
-    HB_REQUIRE(lds <= 60 * 1024, "token input: %d gates a token do not fit the kernel's LDS", D);
+    HB_REQUIRE(((size_t)SIDE_TOKENS * D + 3 * SIDE_TOKENS * 64) * sizeof(float) <= 60 * 1024, "token input: %d gates a token do not fit the kernel's LDS", D);
+    const size_t lds = SIDE_TOKENS * sizeof(float) * (D > SIDE_WAVES * 64 ? D : SIDE_WAVES * 64);
     const int tiles = (T + SIDE_TOKENS - 1) / SIDE_TOKENS;
     HB_REQUIRE(tiles <= 65535, "token input: too many tokens for the grid");
     const bool many = T > 64;          // (few tokens: a row a workgroup, so that the gate's rows are spread over more waves)
     HB_REQUIRE(g16 == nullptr || (many && stage == 0), "token input: bfloat16 gates are for many tokens and a product of the caller's");
     HB_REQUIRE(D <= 65535, "token input: too many gates for the grid");
+    const dim3 gate_grid((T + SIDE_TILE * 8 - 1) / (SIDE_TILE * 8) * 8, (D + SIDE_TILE - 1) / SIDE_TILE);
+    const bool vec = H % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w_gate % 16 == 0;     // (rows start at whole quads)
 #define HB_SIDE(TW)                                                                                                   \
     do {                                                                                                              \
-        if (many)                                                                                                     \
+        if (many && vec)                                                                                              \
+            token_gate_tile_kernel<TW><<<gate_grid, 64 * SIDE_SPLIT, 0, stream>>>(                                    \
+                x, tokens, (const TW*)table, table_ld, col0, (const TW*)w_gate, g, g16, T, H, D);                     \
+        else if (many)                                                                                                \
             token_gate_kernel<TW, 4><<<dim3((D + 15) / 16, tiles), 256, 0, stream>>>(                                  \
                 x, tokens, (const TW*)table, table_ld, col0, (const TW*)w_gate, g, g16, T, H, D);                     \
         else                                                                                                          \
@@ -1480,7 +1589,7 @@ extern "C" int hb_token_side(float* x, const int* tokens, const void* table, int
                 x, tokens, (const TW*)table, table_ld, col0, (const TW*)w_gate, g, T, H, D);                          \
         HB_CHECK_LAUNCH("token_gate");                                                                                \
         if (stage != 1) break;                                                                                        \
-        token_proj_kernel<TW><<<dim3((H + 63) / 64, tiles), 256, lds, stream>>>(g, (const TW*)w_proj_t, y, T, H, D);   \
+        token_proj_kernel<TW><<<dim3((H + 63) / 64, tiles), 64 * SIDE_WAVES, lds, stream>>>(g, (const TW*)w_proj_t, y, T, H, D); \
         HB_CHECK_LAUNCH("token_proj");                                                                                \
     } while (0)
     if (dtype == HB_F32) HB_SIDE(float);

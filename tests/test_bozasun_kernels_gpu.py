@@ -263,6 +263,35 @@ def test_routing_by_softmax_scores_with_identity_experts(E, identity, top, group
         assert torch.allclose(x.cpu(), want, atol=tol, rtol=tol)
 
 
+@pytest.mark.parametrize("T,H,D", [(65, 20, 1), (96, 72, 33), (97, 1030, 64), (289, 2052, 96), (9, 40, 1000), (70, 130, 1728)])
+def test_token_input_at_the_edges_of_its_tiles(T, H, D):
+    """Gates and products by themselves: float32 sums of H and of D products (each rounding at most half an ulp of the terms'
+    sizes), the gates' activation a few more; bfloat16 gates half an ulp of theirs."""
+    x, table, gate, proj = rand(T, H, seed=1), rand(50, D, seed=2), rand(D, H, seed=3, scale=H ** -0.5), rand(D, H, seed=4)
+    tokens = torch.randint(0, 50, (T,), generator=torch.Generator().manual_seed(6))
+    for dtype in (torch.float32, torch.bfloat16):
+        tb, gt, pj = (w.to(dtype) for w in (table, gate, proj))
+        z, size = x.double() @ gt.double().T, x.double().abs() @ gt.double().abs().T
+        rows = tb.double()[tokens]
+        want = torch.nn.functional.gelu(z, approximate="tanh") * rows
+        slack = ((H * 2.0 ** -24 * size + 4e-7 * (1 + z.abs())) * 1.2) * rows.abs() + 1e-30
+        got, y = torch.full((T, D), 7.0, device=DEV), torch.full((T, H), 7.0, device=DEV)
+        args = (g(x).clone(), tokens.to(torch.int32).to(DEV), g(tb), 0, g(gt), g(pj), torch.ones(H, device=DEV), 1e-5, got, y)
+        ops.token_side(*args, stage=1)
+        assert bool(((got.cpu().double() - want).abs() <= slack).all())
+        sums, terms = got.cpu().double() @ pj.double(), got.cpu().double().abs() @ pj.double().abs()
+        assert bool(((y.cpu().double() - sums).abs() <= D * 2.0 ** -24 * terms + 1e-30).all())
+        if T > ops.TOKEN_SIDE_FEW:
+            g16 = torch.full((T, D), 7.0, dtype=torch.bfloat16, device=DEV)
+            ops.token_side(*args, stage=0, g16=g16)
+            # (x has taken the layer's sum above: the gates of what it is now)
+            z = args[0].cpu().double() @ gt.double().T
+            size = args[0].cpu().double().abs() @ gt.double().abs().T
+            want = torch.nn.functional.gelu(z, approximate="tanh") * rows
+            slack = ((H * 2.0 ** -24 * size + 4e-7 * (1 + z.abs())) * 1.2) * rows.abs() + 1e-30
+            assert bool(((g16.cpu().double() - want).abs() <= slack + want.abs() * 2.0 ** -8).all())
+
+
 # ---------------------------------------------------------------- the per-layer token input
 @pytest.mark.parametrize("T,H,D,layers,layer", [(1, 72, 5, 4, 3), (7, 176, 12, 6, 0), (3, 64, 1, 2, 1), (130, 512, 64, 3, 2), (2, 2052, 48, 2, 1)])
 def test_token_input(T, H, D, layers, layer):
