@@ -300,10 +300,14 @@ __global__ void lru_scan_kernel(const float* __restrict__ ug, const float* __res
 // place takes a, i_pre's place b): the exponentials and the root are most of the arithmetic, and here they fill
 // the chip. The second walks S_t = a_t S_(t-1) + b_t, a chain, but one whose pieces compose: over a run of tokens
 // the state leaves as A S + B with A the product of the run's decays and B the run's walk from zero. A workgroup
-// is SEGS waves on 64 channels; a sequence's tokens are cut into SEGS runs. Every wave but the last first walks
-// its run from zero (A, B into LDS); then each wave takes the sequence's state through the runs before its own (at
-// most SEGS - 1 multiply-adds) and walks its run again from there, now storing the outputs. The chain is two runs
+// is 1,024 threads on WIDTH channels; a sequence's tokens are cut into 1024 / WIDTH runs. Every run but the last is first
+// walked from zero (A, B into LDS); then each takes the sequence's state through the runs before its own (a multiply-add
+// each) and is walked again from there, now storing the outputs. The chain is two runs
 // long instead of the whole portion. The result differs from the one-wave walk by float32 rounding (the runs' edges).
+// 64 channels a workgroup read whole lines, but leave most of the chip idle where there are few sequences: then 16 (64
+// bytes of a row, whose other half the next workgroup of the same XCD reads), 64 runs. Both
+// kernels, 2,560 channels: one sequence of 2,048 tokens (40 workgroups of 64 channels) 98 us with 64, 66 with 16; of 512
+// tokens 32 and 24; four sequences of 512 (160 workgroups) 58 and 61: the line lies at 96 workgroups.
 __global__ void lru_decay_input_kernel(const float* __restrict__ ug, float* __restrict__ gates,
                                        const float* __restrict__ rb, const float* __restrict__ ib,
                                        const float* __restrict__ lam, float rate, int W, int bw, size_t total) {
@@ -322,14 +326,16 @@ __global__ void lru_decay_input_kernel(const float* __restrict__ ug, float* __re
     row[gc + bw] = sqrtf(-expm1f(2.0f * log_a)) * i * ug[t * 2 * W + c];
 }
 
-template <class TOut, int SEGS>
-__global__ void __launch_bounds__(64 * SEGS)
+template <class TOut, int WIDTH>
+__global__ void __launch_bounds__(1024)
 lru_scan_runs_kernel(const float* __restrict__ ug, const float* __restrict__ ab, float* __restrict__ state,
                      const int* __restrict__ seq_starts, const int* __restrict__ slots, TOut* __restrict__ y, int W, int bw) {
-    __shared__ float sA[SEGS][64], sB[SEGS][64];
-    const int seq = blockIdx.x;
-    const int lane = threadIdx.x & 63, seg = threadIdx.x >> 6;
-    const int c = blockIdx.y * 64 + lane;
+    constexpr int SEGS = 1024 / WIDTH;
+    __shared__ float sA[SEGS][WIDTH], sB[SEGS][WIDTH];
+    const int seq = blockIdx.y;
+    const int lane = threadIdx.x % WIDTH, seg = threadIdx.x / WIDTH;
+    const int groups = gridDim.x;                      // (workgroups go to the 8 XCDs in turn: an XCD takes neighbouring channels)
+    const int c = (groups % 8 ? (int)blockIdx.x : (int)(blockIdx.x % 8) * (groups / 8) + (int)blockIdx.x / 8) * WIDTH + lane;
     const bool live = c < W;
     const int cc = live ? c : 0;
     const int gc = (cc / bw) * 2 * bw + cc % bw;
@@ -350,6 +356,7 @@ lru_scan_runs_kernel(const float* __restrict__ ug, const float* __restrict__ ab,
     __syncthreads();
     float* S_mem = state + (size_t)slots[seq] * W + cc;
     float S = live ? *S_mem : 0.f;
+#pragma unroll 8
     for (int k = 0; k < seg; ++k) S = fmaf(sA[k][lane], S, sB[k][lane]);
     if (!live) return;
 #pragma unroll 8
@@ -364,7 +371,6 @@ lru_scan_runs_kernel(const float* __restrict__ ug, const float* __restrict__ ab,
 // longest: the most tokens that one sequence of the step brings (the host knows it); portions of LRU_RUNS_FROM
 // tokens or more take the kernel that cuts them into runs.
 #define LRU_RUNS_FROM 128
-#define LRU_RUNS 16
 
 extern "C" int hb_lru_scan(const float* ug, float* gates, const float* rb, const float* ib, const float* lam,
                            float rate, float* state, const int* seq_starts, const int* slots, void* y, int y_dtype,
@@ -376,13 +382,17 @@ extern "C" int hb_lru_scan(const float* ug, float* gates, const float* rb, const
         HB_REQUIRE(T > 0 && (total + 255) / 256 <= 0x7fffffffu, "recurrent unit: %d tokens of %d channels exceed the grid", T, W);
         lru_decay_input_kernel<<<(unsigned)((total + 255) / 256), 256, 0, stream>>>(ug, gates, rb, ib, lam, rate, W, bw, total);
         HB_CHECK_LAUNCH("lru_decay_input");
-        const dim3 grid(B, (W + 63) / 64);
-        if (y_dtype == HB_F32)
-            lru_scan_runs_kernel<float, LRU_RUNS><<<grid, 64 * LRU_RUNS, 0, stream>>>(ug, gates, state, seq_starts, slots, (float*)y, W, bw);
-        else if (y_dtype == HB_BF16)
-            lru_scan_runs_kernel<bf16, LRU_RUNS><<<grid, 64 * LRU_RUNS, 0, stream>>>(ug, gates, state, seq_starts, slots, (bf16*)y, W, bw);
+        const bool narrow = (long long)B * ((W + 63) / 64) < 96;
+        const int width = narrow ? 16 : 64;
+        const dim3 grid((W + width - 1) / width, B);
+#define HB_RUNS(T, WIDTH) lru_scan_runs_kernel<T, WIDTH><<<grid, 1024, 0, stream>>>(ug, gates, state, seq_starts, slots, (T*)y, W, bw)
+        if (y_dtype == HB_F32 && narrow) HB_RUNS(float, 16);
+        else if (y_dtype == HB_F32) HB_RUNS(float, 64);
+        else if (y_dtype == HB_BF16 && narrow) HB_RUNS(bf16, 16);
+        else if (y_dtype == HB_BF16) HB_RUNS(bf16, 64);
         else
             HB_REQUIRE(false, "recurrent unit: unknown output dtype %d", y_dtype);
+#undef HB_RUNS
         HB_CHECK_LAUNCH("lru_scan_runs");
         return 0;
     }

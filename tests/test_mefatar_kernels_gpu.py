@@ -6,6 +6,7 @@ rotation of pairs with slowed wavelengths, the cache's rows) with the sink in th
 (prompts and single tokens across the pages' edges, one far key made to hold the weight, sinks large and
 small), and the linear attention (the decay through its narrow middle, the state a head, the norm a head)."""
 import math
+import types
 
 import pytest
 import torch
@@ -129,6 +130,30 @@ def test_recurrent_unit_whole_in_portions_and_token_by_token(W, blocks, K, lengt
             assert torch.allclose(torch.cat([p[1] for p in got[i]]), refs[i][2], atol=1e-5, rtol=1e-5), f"recurrence, cuts {cuts[:4]}"
         for s in slots:
             cache.free_slot(s)
+
+
+@pytest.mark.parametrize("W,copies", [(128, 1), (128, 130), (72, 1), (8, 256), (264, 52)])
+def test_recurrent_unit_in_runs_of_either_width(W, copies):
+    """Few sequences take 64 runs of 16 channels (grids that the XCDs divide and do not), many 16 runs of 64: both against
+    the recurrence in float64, at portions that leave runs empty, and a state that is carried from one to the next."""
+    b, tokens = 8, [131, 128, 200]
+    r_b, i_b, lam = 0.3 * rand(W, seed=7), 0.3 * rand(W, seed=8), torch.linspace(-8.0, 1.0, W)
+    ug, gates = rand(sum(tokens), 2 * W, seed=1), rand(sum(tokens), 2 * W, seed=2)
+    halves = gates.view(-1, W // b, 2, b).double()
+    r, i = (plain.sigmoid(halves[:, :, k].reshape(-1, W) + bias.double()) for k, bias in ((0, r_b), (1, i_b)))
+    want = plain.gated_recurrence(ug[:, :W].double(), r, i, lam.double()) * ug[:, W:].double()
+    state = torch.zeros(copies + 1, W, device=DEV)
+    at = 0
+    for n in tokens:
+        meta = types.SimpleNamespace(max_new=n, num_seqs=copies, slots=torch.arange(copies, 0, -1, dtype=torch.int32, device=DEV),
+                                     seq_starts=torch.arange(0, copies * n + 1, n, dtype=torch.int32, device=DEV))
+        out = torch.full((copies * n, W), 7.0, device=DEV)
+        rows = [t[at:at + n].repeat(copies, 1).to(DEV) for t in (ug, gates)]
+        recurrent.lru_scan(rows[0], rows[1], r_b.to(DEV), i_b.to(DEV), lam.to(DEV), 8.0, state, meta, out, b)
+        got = out.cpu().view(copies, n, W)
+        assert torch.allclose(got.double(), want[at:at + n].expand(copies, n, W), atol=1e-5, rtol=1e-5), n
+        assert bool((state[0] == 0).all())
+        at += n
 
 
 def test_recurrent_unit_remembers_its_first_token():
