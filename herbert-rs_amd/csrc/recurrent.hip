@@ -461,7 +461,7 @@ gated_delta_kernel(const float* __restrict__ qkv, int C, const float* __restrict
                    int a_off, const float* __restrict__ A_log, const float* __restrict__ dt_bias,
                    const float* __restrict__ decay, float* __restrict__ state,
                    const int* __restrict__ seq_starts, const int* __restrict__ slots,
-                   float* __restrict__ out, int kv_heads, int heads, int D, int V, float out_scale) {
+                   float* __restrict__ out, int kv_heads, int heads, int D, int V, float out_scale, const int* __restrict__ which) {
     constexpr int COLS = HB_WAVE / LPC;
     constexpr int DP = LPC * DELTA_PER;                 // D rounded up to what the lanes hold
     constexpr int DELTA_RING = DELTA_RING_OF(DP, CH);
@@ -475,7 +475,7 @@ gated_delta_kernel(const float* __restrict__ qkv, int C, const float* __restrict
     __shared__ __attribute__((aligned(16))) float kq_ring[SLOTS][NB * DP];
     __shared__ float v_ring[SLOTS][COLS];
     __shared__ float gb_ring[SLOTS][2];
-    const int seq = blockIdx.x, h = blockIdx.y;
+    const int seq = which ? which[blockIdx.x] : blockIdx.x, h = blockIdx.y;
     const int lane = threadIdx.x;
     const int part = lane % LPC;                       // which of the column's D numbers this lane holds
     const int lcol = lane / LPC;
@@ -641,9 +641,10 @@ gated_delta_step_kernel(const float* __restrict__ qkv, int C, const float* __res
                         int a_off, const float* __restrict__ A_log, const float* __restrict__ dt_bias,
                         const float* __restrict__ decay, float* __restrict__ state,
                         const int* __restrict__ seq_starts, const int* __restrict__ slots,
-                        float* __restrict__ out, int kv_heads, int heads, int D, int V, float out_scale) {
+                        float* __restrict__ out, int kv_heads, int heads, int D, int V, float out_scale,
+                        const int* __restrict__ which) {
     __shared__ __attribute__((aligned(16))) float4 parts[2][4][8];
-    const int seq = blockIdx.x, h = blockIdx.y;
+    const int seq = which ? which[blockIdx.x] : blockIdx.x, h = blockIdx.y;
     const int t = seq_starts[seq];
     if (seq_starts[seq + 1] == t) return;
     const int part = threadIdx.x % 8, row0 = threadIdx.x / 8, wave = threadIdx.x / HB_WAVE;
@@ -721,22 +722,24 @@ gated_delta_step_kernel(const float* __restrict__ qkv, int C, const float* __res
 // decay null: one factor a head, from the projection's column a_off + h, A_log and dt_bias.
 // decay [T, heads x D]: a factor a key channel, as given (a_off, A_log and dt_bias are not read).
 // correction 0 (a decay a key channel must be given): the linear attention, S <- diag(g) S + k v^T; proj is not read.
+// which [B]: the sequences of the step that take part (null: the step's B sequences); longest: the most tokens that one of them brings.
 extern "C" int hb_gated_delta(const float* qkv, int C, const float* proj, int ld, int b_off, int a_off,
                               const float* A_log, const float* dt_bias, const float* decay, float* state,
                               const int* seq_starts,
                               const int* slots, float* out, int B, int kv_heads, int heads, int D, int V,
-                              int correction, float out_scale, int longest, hipStream_t stream) {
+                              int correction, float out_scale, int longest, const int* which,
+                              hipStream_t stream) {
     HB_REQUIRE(correction || decay, "linear attention: the walk without a correction takes a decay a key channel");
     HB_REQUIRE(B > 0 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0, "delta rule: %d heads on %d key heads", heads, kv_heads);
     HB_REQUIRE(D > 0 && D <= 256, "delta rule: keys of %d, the kernel takes 1 to 256", D);
     HB_REQUIRE(V > 0 && C >= 2 * kv_heads * D + heads * V, "delta rule: rows of %d do not hold the heads' channels", C);
     HB_REQUIRE(B <= 65535 && heads <= 65535, "delta rule: too many sequences or heads for the grid");
-    // one token a sequence at most (longest: the most that a sequence of the step brings), columns in whole quads
+    // one token a sequence at most, columns in whole quads
     if (longest == 1 && V % 4 == 0 && (V + 31) / 32 <= 65535 && (uintptr_t)state % 16 == 0 && (uintptr_t)out % 16 == 0) {
         const dim3 step_grid(B, heads, (V + 31) / 32);
 #define HB_STEP_ONE(ROWS, CH, DELTA)                                                                                     \
     gated_delta_step_kernel<ROWS, CH, DELTA><<<step_grid, 256, 0, stream>>>(qkv, C, proj, ld, b_off, a_off, A_log, dt_bias, decay, \
-        state, seq_starts, slots, out, kv_heads, heads, D, V, out_scale)
+        state, seq_starts, slots, out, kv_heads, heads, D, V, out_scale, which)
 #define HB_STEP_OF(ROWS)                                                                                                 \
     do {                                                                                                                 \
         if (!decay) HB_STEP_ONE(ROWS, false, true);                                                                      \
@@ -766,13 +769,13 @@ extern "C" int hb_gated_delta(const float* qkv, int C, const float* proj, int ld
     do {                                                                                                          \
         if (decay && !correction)                                                                                 \
             gated_delta_kernel<L, P, true, false><<<grid, HB_WAVE, 0, stream>>>(qkv, C, proj, ld, b_off, a_off, A_log, \
-                dt_bias, decay, state, seq_starts, slots, out, kv_heads, heads, D, V, out_scale);                 \
+                dt_bias, decay, state, seq_starts, slots, out, kv_heads, heads, D, V, out_scale, which);          \
         else if (decay)                                                                                           \
             gated_delta_kernel<L, P, true, true><<<grid, HB_WAVE, 0, stream>>>(qkv, C, proj, ld, b_off, a_off, A_log, \
-                dt_bias, decay, state, seq_starts, slots, out, kv_heads, heads, D, V, out_scale);                 \
+                dt_bias, decay, state, seq_starts, slots, out, kv_heads, heads, D, V, out_scale, which);          \
         else                                                                                                      \
             gated_delta_kernel<L, P, false, true><<<grid, HB_WAVE, 0, stream>>>(qkv, C, proj, ld, b_off, a_off, A_log, \
-                dt_bias, decay, state, seq_starts, slots, out, kv_heads, heads, D, V, out_scale);                 \
+                dt_bias, decay, state, seq_starts, slots, out, kv_heads, heads, D, V, out_scale, which);          \
     } while (0)
     if (wide) {
         if (lpc == 1) HB_DELTA(1, 8);

@@ -76,8 +76,8 @@ template <int DB, bool CH, bool DELTA>
 __global__ void __launch_bounds__(256)
 chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restrict__ proj, int ld, int b_off, int a_off,
                      const float* __restrict__ A_log, const float* __restrict__ dt_bias,
-                     const float* __restrict__ decay, const int* __restrict__ seq_starts, float* __restrict__ scratch,
-                     int kv_heads, int heads, int V, int c0, int span) {
+                     const float* __restrict__ decay, const int2* __restrict__ chunks, float* __restrict__ scratch,
+                     int kv_heads, int heads, int V) {
     constexpr int D = 16 * DB, KLD = D + 4, TLD = CHUNK + 4;
     constexpr int NG = CH ? 4 * DB : 1;                       // decays a lane holds of its token
     // columns' keys in the order their lanes read them, later G_64 / G k with a row a key entry
@@ -88,12 +88,10 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
     __shared__ float total[4][CH ? D : 1];                    // a block's product of decays
     __shared__ float betas[CHUNK];
     __shared__ int wild_from;
-    const int h = blockIdx.y, seq = blockIdx.z;
-    const int first = seq_starts[seq] + (c0 + (int)blockIdx.x) * CHUNK;
-    const int n = min(CHUNK, seq_starts[seq + 1] - first);
-    if (n <= 0) return;
+    const int h = blockIdx.x, chunk = blockIdx.y;             // (heads first, as in the other kernel: what it reads lies in its XCD's L2)
+    const int first = chunks[chunk].x, n = chunks[chunk].y;
     const ChunkLayout at = chunk_layout(D, V, DELTA);
-    float* out = scratch + (((size_t)seq * span + blockIdx.x) * heads + h) * at.size;
+    float* out = scratch + ((size_t)chunk * heads + h) * at.size;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r = lane & 15, q = lane >> 4;
     const int kvh = h / (heads / kv_heads);
@@ -354,22 +352,21 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
 template <int DB, bool DELTA>
 __global__ void __launch_bounds__(256)
 chunk_scan_kernel(const float* __restrict__ qkv, int C, const float* __restrict__ scratch, float* __restrict__ state,
-                  const int* __restrict__ seq_starts, const int* __restrict__ slots, float* __restrict__ out,
-                  int kv_heads, int heads, int V, int c0, int span, float out_scale) {
+                  const int4* __restrict__ runs, const int* __restrict__ slots, float* __restrict__ out,
+                  int kv_heads, int heads, int V, float out_scale) {
     constexpr int D = 16 * DB, OWN = DB / 4;                  // blocks of 16 of the state's rows a wave owns
     constexpr int SLD = D + 4, ULD = CHUNK + 4;
     __shared__ __attribute__((aligned(16))) float s_lds[2][16 * SLD], u_lds[2][16 * ULD];
-    const int h = blockIdx.x, vb = blockIdx.y, seq = blockIdx.z;
-    const int begin = seq_starts[seq], n_all = seq_starts[seq + 1] - begin;
-    const int last = min(c0 + span, (n_all + CHUNK - 1) / CHUNK);
-    if (c0 >= last) return;
+    const int h = blockIdx.x, vb = blockIdx.y;
+    const int4 run = runs[blockIdx.z];
+    const int begin = run.z, n_all = run.w, last = (n_all + CHUNK - 1) / CHUNK;
     const ChunkLayout at = chunk_layout(D, V, DELTA);
-    const float* part = scratch + ((size_t)seq * span * heads + h) * at.size;
+    const float* part = scratch + ((size_t)run.y * heads + h) * at.size;
     const size_t chunk_step = (size_t)heads * at.size;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r = lane & 15, q = lane >> 4;
     const int col = 16 * vb + r;
-    float* S_mem = state + ((size_t)slots[seq] * heads + h) * D * V + col;
+    float* S_mem = state + ((size_t)slots[run.x] * heads + h) * D * V + col;
     f32x4 S[OWN];
     auto share = [&](int buf) {
 #pragma unroll
@@ -377,19 +374,13 @@ chunk_scan_kernel(const float* __restrict__ qkv, int C, const float* __restrict_
 #pragma unroll
             for (int e = 0; e < 4; ++e) s_lds[buf][r * SLD + 16 * (wave + 4 * i) + 4 * e + q] = S[i][e];
     };
-#pragma unroll
-    for (int i = 0; i < OWN; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) S[i][e] = S_mem[(size_t)(16 * (wave + 4 * i) + 4 * q + e) * V];
-    share(0);
-
     struct Operands {
         f32x4 w[DELTA ? DB : 1], qg[DB], b[4], k[OWN][4], u;
         float g[OWN][4], v[DELTA ? 1 : 16];
         int from;
     };
     auto fetch = [&](int c, Operands& o) {
-        const float* p = part + (size_t)(c - c0) * chunk_step;
+        const float* p = part + (size_t)c * chunk_step;
 #pragma unroll
         for (int b = 0; b < DB; ++b) {
             if (DELTA) o.w[b] = *(const f32x4*)(p + at.w + ((wave * DB + b) * 64 + lane) * 4);
@@ -415,10 +406,15 @@ chunk_scan_kernel(const float* __restrict__ qkv, int C, const float* __restrict_
         }
     };
     Operands next;
-    fetch(c0, next);
+    fetch(0, next);                                           // (asked for before the state, whose slot is a load away)
+#pragma unroll
+    for (int i = 0; i < OWN; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[i][e] = S_mem[(size_t)(16 * (wave + 4 * i) + 4 * q + e) * V];
+    share(0);
     __syncthreads();
     int buf = 0;
-    for (int c = c0; c < last; ++c, buf ^= 1) {
+    for (int c = 0; c < last; ++c, buf ^= 1) {
         const Operands o = next;
         if (c + 1 < last) fetch(c + 1, next);
         Chains<8> uc, oc;
@@ -479,40 +475,41 @@ chunk_scan_kernel(const float* __restrict__ qkv, int C, const float* __restrict_
         for (int e = 0; e < 4; ++e) S_mem[(size_t)(16 * (wave + 4 * i) + 4 * q + e) * V] = S[i][e];
 }
 
-// As hb_gated_delta of recurrent.hip, for keys of 64 or 128 and values in steps of 16, rows in whole quads. scratch holds
-// B x span x heads parts of chunk_floats (chunk_layout's size); longest: the most tokens that a sequence of the step brings. Sequences
-// longer than span chunks go through in several pairs of launches, their state carried in `state`.
+// As hb_gated_delta of recurrent.hip, for keys of 64 or 128 and values in steps of 16, rows in whole quads, and for those
+// sequences only that its lists name. chunks [n_chunks]: the row of the chunk's first token, and its tokens (1 to 64).
+// runs [n_runs]: the sequence, the place of its first chunk in `chunks` (the others follow), the row of its first token and
+// the tokens that its chunks hold (all but the last hold 64). scratch holds n_chunks x heads parts of chunk_floats
+// (chunk_layout's size). A sequence longer than the scratch goes through in several calls, its state carried in `state`.
 extern "C" int hb_chunked_delta(const float* qkv, int C, const float* proj, int ld, int b_off, int a_off, const float* A_log,
-                                const float* dt_bias, const float* decay, float* state, const int* seq_starts,
-                                const int* slots, float* out, float* scratch, int B, int kv_heads, int heads, int D,
-                                int V, int correction, float out_scale, int longest, int span, int chunk_floats,
+                                const float* dt_bias, const float* decay, float* state, const int* chunks, int n_chunks,
+                                const int* runs, int n_runs, const int* slots, float* out, float* scratch, int kv_heads,
+                                int heads, int D, int V, int correction, float out_scale, int chunk_floats,
                                 hipStream_t stream) {
     HB_REQUIRE(correction || decay, "linear attention: a decay a key channel must be given");
-    HB_REQUIRE(B > 0 && longest > 0 && span > 0 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0, "delta rule: %d heads on %d key heads", heads, kv_heads);
+    HB_REQUIRE(n_chunks > 0 && n_runs > 0 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0, "delta rule: %d heads on %d key heads", heads, kv_heads);
     HB_REQUIRE((D == 64 || D == 128) && V > 0 && V % 16 == 0, "delta rule in chunks: keys of %d, values of %d", D, V);
     HB_REQUIRE(C >= 2 * kv_heads * D + heads * V && C % 4 == 0 && (uintptr_t)qkv % 16 == 0 && (uintptr_t)decay % 16 == 0 &&
                (uintptr_t)scratch % 16 == 0, "delta rule in chunks: rows of %d are not in whole quads", C);
+    HB_REQUIRE((uintptr_t)chunks % 8 == 0 && (uintptr_t)runs % 16 == 0, "delta rule in chunks: the lists are not aligned");
     HB_REQUIRE(chunk_floats == chunk_layout(D, V, correction != 0).size,
                "delta rule in chunks: a part of %d floats is not the kernel's layout", chunk_floats);
-    HB_REQUIRE(B <= 65535 && heads <= 65535 && V / 16 <= 65535, "delta rule: too many sequences or heads for the grid");
-    const int chunks = (longest + CHUNK - 1) / CHUNK;
-    for (int c0 = 0; c0 < chunks; c0 += span) {
-        const dim3 grid(span < chunks - c0 ? span : chunks - c0, heads, B), scan(heads, V / 16, B);
+    HB_REQUIRE(n_runs <= 65535 && n_chunks <= 65535 && V / 16 <= 65535, "delta rule: too many sequences or heads for the grid");
+    const dim3 grid(heads, n_chunks), scan(heads, V / 16, n_runs);
 #define HB_CHUNKS(DB, CH, DELTA)                                                                                      \
     do {                                                                                                              \
         chunk_prepare_kernel<DB, CH, DELTA><<<grid, 256, 0, stream>>>(qkv, C, proj, ld, b_off, a_off, A_log, dt_bias,  \
-            decay, seq_starts, scratch, kv_heads, heads, V, c0, span);                                                \
-        chunk_scan_kernel<DB, DELTA><<<scan, 256, 0, stream>>>(qkv, C, scratch, state, seq_starts, slots, out,        \
-            kv_heads, heads, V, c0, span, out_scale);                                                                 \
+            decay, (const int2*)chunks, scratch, kv_heads, heads, V);                                                 \
+        HB_CHECK_LAUNCH("chunk_prepare");                                                                             \
+        chunk_scan_kernel<DB, DELTA><<<scan, 256, 0, stream>>>(qkv, C, scratch, state, (const int4*)runs, slots, out, \
+            kv_heads, heads, V, out_scale);                                                                           \
     } while (0)
-        if (D == 128 && !correction) HB_CHUNKS(8, true, false);
-        else if (D == 128 && decay) HB_CHUNKS(8, true, true);
-        else if (D == 128) HB_CHUNKS(8, false, true);
-        else if (!correction) HB_CHUNKS(4, true, false);
-        else if (decay) HB_CHUNKS(4, true, true);
-        else HB_CHUNKS(4, false, true);
+    if (D == 128 && !correction) HB_CHUNKS(8, true, false);
+    else if (D == 128 && decay) HB_CHUNKS(8, true, true);
+    else if (D == 128) HB_CHUNKS(8, false, true);
+    else if (!correction) HB_CHUNKS(4, true, false);
+    else if (decay) HB_CHUNKS(4, true, true);
+    else HB_CHUNKS(4, false, true);
 #undef HB_CHUNKS
-        HB_CHECK_LAUNCH("chunked_delta");
-    }
+    HB_CHECK_LAUNCH("chunk_scan");
     return 0;
 }

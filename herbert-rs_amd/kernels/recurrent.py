@@ -1,9 +1,11 @@
 """Host side of the kernels for mixers with state of fixed size (csrc/recurrent.hip): the short
 causal convolution with its activation and unit vectors, the gated delta rule, and the gated norm a
 head that follows it. Operand checks, then the launch."""
+import numpy as np
 import torch
 
 from ..errors import BackendError
+from ..hosted import send
 from . import lib
 from .ops import _check, _stream, dtype_code
 
@@ -89,8 +91,9 @@ def gated_group_norm(o, proj, z_off, weight, out, parts, eps):
 
 # Portions of many tokens go through in chunks of CHUNK tokens (csrc/recurrent_chunks.hip), shorter ones token by token.
 CHUNK = 64
-# Scratch of one launch, in floats: longer prompts go through in several, their state carried from one to the next. (It
-# also stays below the 256 MB memory-side cache, from which the second kernel reads what the first has left.)
+# Scratch of one call, in floats (or one chunk's, if that is more): a step with more chunks than fit goes through in
+# several calls, a sequence's state carried from one to the next. (It also stays below the 256 MB memory-side cache, from
+# which the second kernel reads what the first has left.)
 CHUNK_SCRATCH = 48 << 20
 
 
@@ -99,25 +102,108 @@ def chunk_floats(D, V, correction):
     return (3 if correction else 2) * CHUNK * D + CHUNK * CHUNK + (CHUNK * V if correction else 0) + D + 4
 
 
-def _takes_chunks(qkv, decay, meta, heads, D, V, correction):
-    """The walk takes 0.4 us a token of the longest portion while its waves fit the chip; the chunks 37 us (24 without the
+def chunks_from(portions, heads, correction):
+    """The fewest tokens with which one of a step's portions goes through in chunks.
+    The walk takes 0.4 us a token of the longest portion while its waves fit the chip; the chunks 37 us (24 without the
     correction) and 5 us a chunk. One sequence of 16 heads of 128: 96 tokens 43 us either way, 64 tokens 33 against 38
-    (without the correction 48 tokens: 28 against 25). With many sequences or heads the walk's waves wait for each other
-    and the chunks still fill the chip: 8 sequences of 64 tokens 108 against 57, of 32 tokens 60 against 55."""
-    least = 40 if meta.num_seqs * heads >= 128 else 96 if correction else 48
-    return (meta.max_new >= least and D in (64, 128) and V % 16 == 0 and qkv.shape[1] % 4 == 0
-            and qkv.data_ptr() % 16 == 0 and (decay is None or decay.data_ptr() % 16 == 0))
+    (without the correction 48 tokens: 28 against 25). With many such portions or heads the walk's waves wait for each other
+    and the chunks still fill the chip: 8 sequences of 64 tokens 108 against 57, of 32 tokens 60 against 57, 24 sequences of 18 to
+    90 tokens 366 against 170 (without the correction 16 sequences of 16 tokens: 71 against 57)."""
+    lines = [(24, 256), (32, 128), (96, 1)] if correction else [(16, 128), (48, 1)]      # tokens, (sequence, head) pairs from there on
+    for tokens, pairs in lines:
+        if int((portions >= tokens).sum()) * heads >= pairs:
+            return tokens
+    return int(portions.max(initial=0)) + 1
 
 
-def _chunked(rt, qkv, proj, b_off, a_off, a_log, dt_bias, decay, state, meta, out, kv_heads, heads, D, V, correction, out_scale):
-    size, chunks = chunk_floats(D, V, correction), -(-meta.max_new // CHUNK)
-    span = max(1, min(chunks, CHUNK_SCRATCH // (size * heads * meta.num_seqs)))
-    scratch = rt.buffer("delta_chunks", (meta.num_seqs * span * heads * size,), torch.float32)
-    lib.call("recurrent_chunks", "hb_chunked_delta", qkv.data_ptr(), qkv.shape[1], None if proj is None else proj.data_ptr(),
-             0 if proj is None else proj.shape[1], b_off, a_off, None if a_log is None else a_log.data_ptr(),
-             None if dt_bias is None else dt_bias.data_ptr(), None if decay is None else decay.data_ptr(), state.data_ptr(),
-             meta.seq_starts.data_ptr(), meta.slots.data_ptr(), out.data_ptr(), scratch.data_ptr(), meta.num_seqs, kv_heads,
-             heads, D, V, 1 if correction else 0, float(out_scale), int(meta.max_new), span, size, _stream())
+def walks_of(portions, least, heads):
+    """The launches of the portions of fewer than `least` tokens, which go token by token: lists of sequences. Single tokens get
+    one of their own (a kernel that streams the state, 47 of them 22 us) where they would hold up the walk of the longer
+    ones: one of 20 tokens beside 8 single ones takes 22 us so and 34 together, beside 2 of them 21 and 17."""
+    ones = [i for i, n in enumerate(portions) if n == 1 < least]
+    longer = [i for i, n in enumerate(portions) if 1 < n < least]
+    if longer and ones and len(ones) * heads < 64:
+        return [sorted(ones + longer)]
+    return [w for w in (ones, longer) if w]
+
+
+def chunk_calls(starts, least, room):
+    """Cut the portions of at least `least` tokens into chunks and these into calls of at most `room` chunks. starts: the
+    first packed row of each sequence and the last one's end. A call is (runs [n, 4], chunks [m, 2]) as hb_chunked_delta reads
+    them, the longest run first; a sequence's calls follow each other in the order of its tokens. Sequences share a call's
+    room evenly, what the short ones leave over goes to the long ones, and where there are more sequences than room
+    the longest come first."""
+    left = sorted((int(n), int(row), i) for i, (n, row) in enumerate(zip(np.diff(starts), starts)) if n >= least)
+    calls = []
+    while left:
+        free, taken, later = room, [], []
+        for k, (n, row, seq) in enumerate(left):                  # the shortest first
+            take = min(-(-n // CHUNK), free // (len(left) - k))
+            free -= take
+            tokens = min(n, take * CHUNK)
+            if tokens:
+                taken.append((tokens, row, seq))
+            if tokens < n:
+                later.append((n - tokens, row + tokens, seq))
+        runs, chunks = [], []
+        for tokens, row, seq in sorted(taken, reverse=True):
+            runs.append((seq, len(chunks), row, tokens))
+            chunks += [(row + a, min(CHUNK, tokens - a)) for a in range(0, tokens, CHUNK)]
+        calls.append((runs, chunks))
+        left = sorted(later)
+    return calls
+
+
+def _chunk_lists(meta, heads, correction, size):
+    """(calls, floats, walks) of the step, made once for all its layers: for each call in chunks the GPU's (runs, their number,
+    chunks, their number), the scratch they need, and for each launch of the other portions the GPU's list of sequences, their
+    number and the most tokens that one of them brings."""
+    key = ("delta_chunks", heads, correction, size, CHUNK_SCRATCH)
+    got = meta.derived.get(key)
+    if got is None:
+        portions = np.diff(meta.host_starts)
+        least = chunks_from(portions, heads, correction)
+        packed, calls, walks = [], [], []
+
+        def place(numbers):                                    # (16 bytes aligned)
+            at = len(packed)
+            packed.extend(numbers + [0] * (-len(numbers) % 4))
+            return at
+        for runs, chunks in chunk_calls(meta.host_starts, least, max(1, CHUNK_SCRATCH // (size * heads))):
+            calls.append((place([x for run in runs for x in run]), len(runs), place([x for chunk in chunks for x in chunk]), len(chunks)))
+        for which in walks_of(portions, least, heads):
+            walks.append((place(which), len(which), int(portions[which].max())))
+        on_gpu = send(np.array(packed, dtype=np.int32), meta.seq_starts.device)
+        calls = tuple((on_gpu[a:], n, on_gpu[b:], m) for a, n, b, m in calls)
+        walks = tuple((on_gpu[a:], n, longest) for a, n, longest in walks)
+        need = max((m for _, _, _, m in calls), default=0) * heads * size
+        # (the largest half, quarter, ... of the bound that will do: a buffer that is outgrown is replaced by one twice as large)
+        floats = CHUNK_SCRATCH
+        while floats // 2 >= need and floats > 1:
+            floats //= 2
+        got = meta.derived[key] = (calls, max(floats, need), walks)
+    return got
+
+
+def _rule(rt, qkv, proj, b_off, a_off, a_log, dt_bias, decay, state, meta, out, kv_heads, heads, D, V, correction, out_scale):
+    """The long portions in chunks (with a Runtime, for the sizes that those kernels take), the others token by token."""
+    operands = (qkv.data_ptr(), qkv.shape[1], None if proj is None else proj.data_ptr(), 0 if proj is None else proj.shape[1],
+                b_off, a_off, None if a_log is None else a_log.data_ptr(), None if dt_bias is None else dt_bias.data_ptr(),
+                None if decay is None else decay.data_ptr(), state.data_ptr())
+    walks = ((None, meta.num_seqs, int(meta.max_new)),)
+    if (rt is not None and meta.max_new > 1 and D in (64, 128) and V % 16 == 0 and qkv.shape[1] % 4 == 0
+            and qkv.data_ptr() % 16 == 0 and (decay is None or decay.data_ptr() % 16 == 0)):
+        size = chunk_floats(D, V, correction)
+        calls, floats, walks = _chunk_lists(meta, heads, correction, size)
+        scratch = rt.buffer("delta_chunks", (floats,), torch.float32) if calls else None
+        for runs, n_runs, chunks, n_chunks in calls:
+            lib.call("recurrent_chunks", "hb_chunked_delta", *operands, chunks.data_ptr(), n_chunks, runs.data_ptr(), n_runs,
+                     meta.slots.data_ptr(), out.data_ptr(), scratch.data_ptr(), kv_heads, heads, D, V, 1 if correction else 0,
+                     float(out_scale), size, _stream())
+    for which, n_seqs, longest in walks:
+        lib.call("recurrent", "hb_gated_delta", *operands, meta.seq_starts.data_ptr(), meta.slots.data_ptr(), out.data_ptr(),
+                 n_seqs, kv_heads, heads, D, V, 1 if correction else 0, float(out_scale), longest,
+                 None if which is None else which.data_ptr(), _stream())
 
 
 def gated_delta(qkv, proj, b_off, a_off, a_log, dt_bias, state, meta, out, kv_heads, heads, D, V, decay=None,
@@ -143,12 +229,7 @@ def gated_delta(qkv, proj, b_off, a_off, a_log, dt_bias, state, meta, out, kv_he
         _check(meta.slots, "slots", torch.int32, (meta.num_seqs,))
         if heads % kv_heads or not 0 < D <= MAX_KEY_DIM or C < 2 * kv_heads * D + heads * V:
             raise BackendError(f"linear attention: {heads} heads on {kv_heads} key heads of {D} in rows of {C}")
-        if rt is not None and _takes_chunks(qkv, decay, meta, heads, D, V, False):
-            _chunked(rt, qkv, None, 0, 0, None, None, decay, state, meta, out, kv_heads, heads, D, V, False, out_scale)
-            return
-        lib.call("recurrent", "hb_gated_delta", qkv.data_ptr(), C, None, 0, 0, 0, None, None, decay.data_ptr(),
-                 state.data_ptr(), meta.seq_starts.data_ptr(), meta.slots.data_ptr(), out.data_ptr(), meta.num_seqs,
-                 kv_heads, heads, D, V, 0, float(out_scale), int(meta.max_new), _stream())
+        _rule(rt, qkv, None, 0, 0, None, None, decay, state, meta, out, kv_heads, heads, D, V, False, out_scale)
         return
     if decay is not None:
         _check(decay, "decay", torch.float32, (T, heads * D))
@@ -167,15 +248,9 @@ def gated_delta(qkv, proj, b_off, a_off, a_log, dt_bias, state, meta, out, kv_he
     _check(meta.slots, "slots", torch.int32, (meta.num_seqs,))
     if heads % kv_heads or not 0 < D <= MAX_KEY_DIM:
         raise BackendError(f"delta rule: {heads} heads on {kv_heads} key heads of {D}")
-    if rt is not None and _takes_chunks(qkv, decay, meta, heads, D, V, True):
-        _chunked(rt, qkv, proj, b_off, a_off, None if decay is not None else a_log, None if decay is not None else dt_bias,
-                 decay, state, meta, out, kv_heads, heads, D, V, True, out_scale)
-        return
-    lib.call("recurrent", "hb_gated_delta", qkv.data_ptr(), C, proj.data_ptr(), ld, b_off, a_off,
-             None if decay is not None else a_log.data_ptr(), None if decay is not None else dt_bias.data_ptr(),
-             None if decay is None else decay.data_ptr(), state.data_ptr(), meta.seq_starts.data_ptr(),
-             meta.slots.data_ptr(),
-             out.data_ptr(), meta.num_seqs, kv_heads, heads, D, V, 1, float(out_scale), int(meta.max_new), _stream())
+    given = decay is not None
+    _rule(rt, qkv, proj, b_off, a_off, None if given else a_log, None if given else dt_bias, decay, state, meta, out, kv_heads,
+          heads, D, V, True, out_scale)
 
 
 def gated_head_norm(o, proj, g_off, weight, out, heads, V, eps, gate="silu"):

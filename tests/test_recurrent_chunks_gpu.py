@@ -40,7 +40,7 @@ def step(lengths, kv_heads, heads, D, V, kind, rate, seed=0):
     if rate > 2:
         decay[::5] = 0.0                                   # a memory that is dropped at once
     starts = torch.tensor([0] + lengths).cumsum(0).to(torch.int32)
-    meta = types.SimpleNamespace(max_new=max(lengths), num_seqs=B, seq_starts=starts.to(dev()),
+    meta = types.SimpleNamespace(max_new=max(lengths), num_seqs=B, seq_starts=starts.to(dev()), host_starts=starts.numpy(), derived={},
                                  slots=torch.arange(B, 0, -1, dtype=torch.int32, device=dev()))
     state = 0.3 * draw(B + 2, heads, D, V)
     return qkv, proj, a_log, dt_bias, decay, state, meta
@@ -86,6 +86,7 @@ def test_chunks_follow_the_rule(lengths, kv_heads, heads, D, V, kind, rate, monk
     from herbert_rs_amd.kernels import recurrent
     case = step(lengths, kv_heads, heads, D, V, kind, rate)
     want, want_state = expected(*case[:6], lengths, kv_heads, heads, D, V, kind)
+    monkeypatch.setattr(recurrent, "chunks_from", lambda *_: 1)        # (whatever is faster: every portion here)
     for scratch in (recurrent.CHUNK_SCRATCH, 1):               # (1: a chunk a launch)
         monkeypatch.setattr(recurrent, "CHUNK_SCRATCH", scratch)
         got, state = run(*case, kv_heads, heads, D, V, kind)
@@ -95,6 +96,32 @@ def test_chunks_follow_the_rule(lengths, kv_heads, heads, D, V, kind, rate, monk
             at += n
         assert float((state - want_state).norm() / want_state.norm()) <= 2e-6
         assert torch.equal(state[0], case[5][0]) and torch.equal(state[-1], case[5][-1])      # nobody's slots
+
+
+@pytest.mark.parametrize("kind", ["head", "channel", "linear"])
+@pytest.mark.parametrize("lengths", [[1, 200, 1, 0, 130, 1], [60, 20, 300, 96, 3, 47] + [64] * 30, [64] * 70 + [1]])
+def test_long_portions_take_chunks_beside_short_ones(kind, lengths, monkeypatch):
+    """Portions that go through in chunks, single tokens and a walk of what lies between in one step, with room for all chunks in
+    one call and for a few: the scratch stays within its bound and every sequence follows the rule."""
+    from herbert_rs_amd.kernels import recurrent
+    from herbert_rs_amd.parts import Runtime
+    kv_heads, heads, D, V = 2, 4, 64, 16
+    case = step(lengths, kv_heads, heads, D, V, kind, 0.0)
+    want, want_state = expected(*case[:6], lengths, kv_heads, heads, D, V, kind)
+    room = recurrent.chunk_floats(D, V, kind != "linear") * heads * 7
+    for scratch in (recurrent.CHUNK_SCRATCH, room):
+        monkeypatch.setattr(recurrent, "CHUNK_SCRATCH", scratch)
+        sizes = []
+        monkeypatch.setattr(Runtime, "buffer", lambda rt, name, shape, dtype=None, take=Runtime.buffer: sizes.append(shape) or take(rt, name, shape, dtype))
+        got, state = run(*case, kv_heads, heads, D, V, kind)
+        monkeypatch.undo()
+        assert sizes and max(n for n, in sizes) <= scratch
+        assert float((got - want).norm() / want.norm()) <= 2e-6 and float((state - want_state).norm() / want_state.norm()) <= 2e-6
+        at = 0
+        for n in lengths:
+            if n:
+                assert float((got[at:at + n] - want[at:at + n]).norm() / want[at:at + n].norm()) <= 2e-6, (n, scratch)
+            at += n
 
 
 @pytest.mark.parametrize("kind", ["head", "linear"])
