@@ -35,7 +35,7 @@ HB_MODULE_ERROR_SLOT()
 
 // Where a (chunk, head)'s pieces lie in its part of the scratch, in floats.
 struct ChunkLayout {
-    int q, k, b, w, u, g, size;
+    int q, k, b, w, u, g, from, lost, size;
 };
 __host__ __device__ inline ChunkLayout chunk_layout(int D, int V, bool delta) {
     ChunkLayout l;
@@ -44,8 +44,10 @@ __host__ __device__ inline ChunkLayout chunk_layout(int D, int V, bool delta) {
     l.b = l.k + CHUNK * D;                // [4][4][64][4]: B, rows of tokens
     l.w = l.b + CHUNK * CHUNK;            // [4][D / 16][64][4]: -T beta G K, rows of tokens
     l.u = l.w + (delta ? CHUNK * D : 0);  // [4][V / 16][64][4]: T beta V, as sums lie
-    l.g = l.u + (delta ? CHUNK * V : 0);  // [D]: G_64, then the first token that is not finite (64: none)
-    l.size = l.g + D + 4;
+    l.g = l.u + (delta ? CHUNK * V : 0);  // [D]: G_64
+    l.from = l.g + D;                     // [V] int: the token from which a column is not finite (64: none)
+    l.lost = l.from + V;                  // [4] int: a bit for each of a block's tokens whose query is not finite
+    l.size = l.lost + 4;
     return l;
 }
 
@@ -73,7 +75,7 @@ struct Chains {
 __device__ __forceinline__ bool not_finite(float v) { return !(fabsf(v) <= 3.4028235e38f); }
 
 template <int DB, bool CH, bool DELTA>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, DELTA ? 1 : 2)         // (without the correction two workgroups a CU fit the LDS)
 chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restrict__ proj, int ld, int b_off, int a_off,
                      const float* __restrict__ A_log, const float* __restrict__ dt_bias,
                      const float* __restrict__ decay, const int2* __restrict__ chunks, float* __restrict__ scratch,
@@ -87,7 +89,7 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
     __shared__ __attribute__((aligned(16))) float inverse[DELTA ? 4 * 16 * 20 : 4];      // of I + its diagonal blocks
     __shared__ float total[4][CH ? D : 1];                    // a block's product of decays
     __shared__ float betas[CHUNK];
-    __shared__ int wild_from;
+    __shared__ int wild_from, wild_values;
     const int h = blockIdx.x, chunk = blockIdx.y;             // (heads first, as in the other kernel: what it reads lies in its XCD's L2)
     const int first = chunks[chunk].x, n = chunks[chunk].y;
     const ChunkLayout at = chunk_layout(D, V, DELTA);
@@ -103,18 +105,18 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
     const float* row = qkv + (size_t)(first + (real ? token : 0)) * C;
     f32x4 kq[DB], qq[DB];
     float pre[NG], beta = 0.f;
-    bool wild = false;
+    bool wild = false, wild_query = false, wild_value = false;
 #pragma unroll
     for (int b = 0; b < DB; ++b) {
         kq[b] = load_quad<true>(row + k_at + 16 * b + 4 * q, 4);
         qq[b] = load_quad<true>(row + q_at + 16 * b + 4 * q, 4);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) wild |= not_finite(kq[b][e]) | not_finite(qq[b][e]);
+        for (int e = 0; e < 4; ++e) wild |= not_finite(kq[b][e]), wild_query |= not_finite(qq[b][e]);
     }
     for (int v = 4 * q; v < V; v += 16) {
         const f32x4 x = load_quad<true>(row + v_at + v, 4);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) wild |= not_finite(x[e]);
+        for (int e = 0; e < 4; ++e) wild_value |= not_finite(x[e]);
     }
     if (CH) {
         const float* g = decay + ((size_t)(first + (real ? token : 0)) * heads + h) * D + 4 * q;
@@ -134,12 +136,28 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
         beta = 1.0f / (1.0f + expf(-proj[(size_t)(first + (real ? token : 0)) * ld + b_off + h]));
         wild |= not_finite(beta);
     }
-    if (tid == 0) wild_from = CHUNK;
+    // What is not finite reaches what it reaches in the walk: a query its own token's output, a value its column from there on, a key,
+    // a decay or a beta all of the head from there on (the state too: with a row a key entry that would be lost alone, no
+    // later output is without it). It is left out here, and the second kernel makes what comes of it not a number.
+    if (tid == 0) wild_from = CHUNK, wild_values = 0;
     __syncthreads();
     if (real && wild) atomicMin(&wild_from, token);
+    if (real && wild_value) wild_values = 1;
+    unsigned long long lost = __ballot(real && wild_query);
+    lost |= lost >> 32;
+    lost = (lost | lost >> 16) & 0xffff;
+    const bool asks = !((lost >> r) & 1);
+    if (lane == 0) ((int*)out)[at.lost + wave] = (int)lost;
     __syncthreads();
-    // (tokens from one that is not finite on are left out here; the second kernel makes what comes of them not a number)
     const int from = wild_from;
+    const bool screen = wild_values;
+    for (int c = tid; c < V; c += 256) {
+        int f = from;
+        if (screen)
+            for (int t = min(n, from) - 1; t >= 0; --t)
+                if (not_finite(qkv[(size_t)(first + t) * C + v_at + c])) f = t;
+        ((int*)out)[at.from + c] = f;
+    }
     real = real && token < from;
     float suf[NG];
 #pragma unroll
@@ -149,7 +167,8 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
     f32x4 part = {0.f, 0.f, 0.f, 0.f}, part2 = part;          // q . k of the token itself
 #pragma unroll
     for (int b = 0; b < DB; ++b) {
-        if (!real) kq[b] = qq[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (!real) kq[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (!real || !asks) qq[b] = f32x4{0.f, 0.f, 0.f, 0.f};
         transpose_quads(kq[b]);
         transpose_quads(qq[b]);
 #pragma unroll
@@ -284,7 +303,6 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
     } else {
         for (int d = tid; d < D; d += 256) out[at.g + d] = total[0][0] * total[1][0] * total[2][0] * total[3][0];
     }
-    if (tid == 0) ((int*)out)[at.g + D] = from;
     __syncthreads();                                          // cols and rows have been read
 #pragma unroll
     for (int b = 0; b < DB; ++b)
@@ -315,6 +333,7 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
                 float v = 0.f;
                 if (of_k) v = rows[t * KLD + in_quads(16 * cb + r)];
                 else if (t < n && t < from) v = qkv[(size_t)(first + t) * C + v_at + 16 * (cb - DB) + r];
+                if (screen && not_finite(v)) v = 0.f;
                 acc[e] = betas[t] * v;
             }
             if (i > 0) {
@@ -377,7 +396,7 @@ chunk_scan_kernel(const float* __restrict__ qkv, int C, const float* __restrict_
     struct Operands {
         f32x4 w[DELTA ? DB : 1], qg[DB], b[4], k[OWN][4], u;
         float g[OWN][4], v[DELTA ? 1 : 16];
-        int from;
+        int from, lost;
     };
     auto fetch = [&](int c, Operands& o) {
         const float* p = part + (size_t)c * chunk_step;
@@ -397,7 +416,8 @@ chunk_scan_kernel(const float* __restrict__ qkv, int C, const float* __restrict_
                 o.k[i][s] = *(const f32x4*)(p + at.k + (((wave + 4 * i) * 4 + s) * 64 + lane) * 4);
                 o.g[i][s] = p[at.g + 16 * (wave + 4 * i) + 4 * q + s];
             }
-        o.from = ((const int*)p)[at.g + D];
+        o.from = ((const int*)p)[at.from + col];
+        o.lost = ((const int*)p)[at.lost + wave];
         if (!DELTA) {
             const int n = n_all - c * CHUNK;
             const float* v = qkv + (size_t)(begin + c * CHUNK) * C + 2 * kv_heads * D + h * V + col;
@@ -465,7 +485,7 @@ chunk_scan_kernel(const float* __restrict__ qkv, int C, const float* __restrict_
         for (int e = 0; e < 4; ++e) {
             const int t = 16 * wave + 4 * q + e, at_token = c * CHUNK + t;
             if (at_token < n_all)
-                out[(size_t)(begin + at_token) * heads * V + h * V + col] = t < o.from ? sums[e] * out_scale : NAN;
+                out[(size_t)(begin + at_token) * heads * V + h * V + col] = t < o.from && !(o.lost >> (4 * q + e) & 1) ? sums[e] * out_scale : NAN;
         }
         __syncthreads();
     }

@@ -99,7 +99,7 @@ CHUNK_SCRATCH = 48 << 20
 
 def chunk_floats(D, V, correction):
     """Floats that a chunk of a head takes of the scratch (the kernel refuses another number)."""
-    return (3 if correction else 2) * CHUNK * D + CHUNK * CHUNK + (CHUNK * V if correction else 0) + D + 4
+    return (3 if correction else 2) * CHUNK * D + CHUNK * CHUNK + (CHUNK * V if correction else 0) + D + V + 4
 
 
 def chunks_from(portions, heads, correction):

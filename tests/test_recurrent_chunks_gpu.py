@@ -124,20 +124,33 @@ def test_long_portions_take_chunks_beside_short_ones(kind, lengths, monkeypatch)
             at += n
 
 
-@pytest.mark.parametrize("kind", ["head", "linear"])
+@pytest.mark.parametrize("kind", ["head", "channel", "linear"])
 @pytest.mark.parametrize("place", [3, 64 + 17])
-def test_rows_that_are_not_finite_reach_no_earlier_token(kind, place):
-    """A value without a finite size: its head's outputs before it, other heads and other sequences are the same bits; its
-    head's own outputs from there on are not numbers."""
+@pytest.mark.parametrize("what", ["query", "key", "value"])
+def test_a_number_that_is_not_finite_reaches_what_it_reaches_in_the_walk(kind, place, what):
+    """A query spoils its own token's output, a value its column from there on, a key its head from there on: exactly what the
+    walk token by token loses is lost (of the linear attention's state, after a key, all rows for one that no later output
+    is without). All else is the same bits as without it."""
+    from herbert_rs_amd.kernels import recurrent
     kv_heads, heads, D, V, lengths = 2, 2, 64, 32, [150, 100]
     case = list(step(lengths, kv_heads, heads, D, V, kind, 0.0))
     clean, state = run(*case, kv_heads, heads, D, V, kind)
     case[0] = case[0].clone()
-    case[0][place, 2 * kv_heads * D + V + 5] = float("inf")     # a value of head 1
-    got, wild = run(*case, kv_heads, heads, D, V, kind)
-    assert torch.equal(got[150:], clean[150:]) and torch.equal(got[:, 0], clean[:, 0])
-    assert torch.allclose(got[:place, 1], clean[:place, 1], rtol=0, atol=0) and bool(got[place:150, 1].isnan().all())
-    assert torch.equal(wild[1], state[1]) and torch.equal(wild[2, 0], state[2, 0]) and bool(wild[2, 1].isnan().all())
+    at = {"query": D + 5, "key": (kv_heads + 1) * D + 5, "value": 2 * kv_heads * D + V + 5}[what]         # of head 1
+    case[0][place, at] = float("inf")
+    got, left = run(*case, kv_heads, heads, D, V, kind)
+
+    qkv, proj, a_log, dt_bias, decay, held, meta = case
+    out, held = torch.full((250, heads * V), 7.0, device=dev()), held.to(dev())
+    recurrent.gated_delta(qkv.to(dev()), None if kind == "linear" else proj.to(dev()), 0, heads, a_log.to(dev()), dt_bias.to(dev()), held,
+                          meta, out, kv_heads, heads, D, V, decay=None if kind == "head" else decay.reshape(250, heads * D).to(dev()),
+                          correction=kind != "linear", out_scale=0.5)
+    fine, fine_state = out.cpu().view(250, heads, V).isfinite(), held.cpu().isfinite()
+    assert torch.equal(got.isfinite(), fine) and torch.equal(got[fine], clean[fine])
+    if kind == "linear" and what == "key":
+        assert not fine_state[2, 1].all()
+        fine_state[2, 1] = False
+    assert torch.equal(left.isfinite(), fine_state) and torch.equal(left[fine_state], state[fine_state])
 
 
 @pytest.mark.parametrize("kv_heads,heads,D,V", [(1, 1, 1, 4), (2, 4, 33, 36), (3, 3, 64, 100), (2, 4, 128, 128), (1, 2, 200, 8), (1, 1, 256, 64),
