@@ -12,22 +12,30 @@
 // the pairs are taken in four levels, s = 1, 2, 4, 8: pairs whose halves of a run of 2 s tokens differ, split in the
 // middle of that run; the products over runs grow from level to level by one exchange between the lanes of 16 tokens.
 //
+// This is the chunked form of the delta rule with gates by Yang, Kautz and Hatamizadeh (Gated Delta Networks, 2024; without
+// gates Yang, Wang, Zhang, Shen and Kim, 2024) and of gated linear attention (Yang, Wang, Shen, Panda and Kim, 2023); T is
+// the triangular factor of a product of Householder-like matrices (Bischof and Van Loan, 1987). The levels are this file's.
+//
 // chunk_prepare_kernel: everything that does not need S_0, one workgroup a (chunk, head), all of them at once. It leaves
 // in scratch, as the operands that the second kernel's lanes load: G q, G_64 / G k, B, and -T beta G K and T beta V.
 // chunk_scan_kernel: the chain of chunks, one workgroup a (head, 16 columns of S): four waves, each 16 tokens of a
 // chunk (U and O) and a quarter of the state's rows (S).
 //
-// Sums over many k are taken as eight chains added in pairs, so that they round as the walk's sums over lanes do. Against 64
-// bits (random keys of unit length, three sequences of 65 to 200 tokens, the walk's error in brackets): 1.2e-7 (1.0e-7) with
-// decays spread over (0, 1), where most of an output is its own token's, 4.5e-7 (4.9e-7) with decays near one, a decay a
-// channel 1.1e-7 (1.0e-7) and 2.0e-7 (2.7e-7), the linear attention 1.0e-7 (0.8e-7) and 1.8e-7 (2.8e-7).
+// The walk rounds the state and what is subtracted from a value token by token; here a rounding of A, B or T reaches
+// many tokens. So A, B and T are sums in float64 (the decays of the delta rule too), rounded once; sums over tokens run in their order, the
+// latest and mostly largest last; sums over a key's entries are eight chains of float32 added in pairs. Against 64 bits, 333 tokens, 16
+// heads of 64 or 128, keys of unit length drawn at random or with cosines of 0.5 or 0.8, decays spread over (0, 1) or around 0.5 to
+// 0.999: the outputs' error is 0.67 to 0.97 of the walk's (0.8e-7 to 1e-6), 0.56 to 0.88 for the linear attention, and that of the
+// state left 0.76 to 1.06. (With A, B and T in float32 the outputs' was up to 1.3 of the walk's, the state's up to 2.)
 //
-// 2,048 tokens of 16 heads of 128 x 128 take 190 us (the walk 793), with a decay a channel 198 (1,068), the linear attention
-// 139 (894); 8 sequences of 300 tokens 175 (450). Bound: the second kernel by its chain (112 products of 32 cycles a
-// chunk and wave and two exchanges through LDS), the first by its products, for which a (chunk, head) has one workgroup a CU.
+// 2,048 tokens of 16 heads of 128 x 128 take 196 us (the walk 781), with a decay a channel 221 (1,084), the linear attention
+// 149 (909); 8 sequences of 300 tokens 192, 228 and 127 (446, 408 and 455). Bound: the second kernel by its chain (112
+// products of 32 cycles a chunk and wave and two exchanges through LDS, 118 us of the 196), the first by its products, in float64 of 64
+// cycles, for which a (chunk, head) has one workgroup a CU.
 #include "common.h"
 #include "mfma_f32.h"
 #include <math.h>
+#include <type_traits>
 
 HB_MODULE_ERROR_SLOT()
 
@@ -52,7 +60,7 @@ __host__ __device__ inline ChunkLayout chunk_layout(int D, int V, bool delta) {
 }
 
 __device__ __forceinline__ int in_quads(int i) { return (i & ~15) + 4 * (i & 3) + ((i >> 2) & 3); }
-// A sum over many k as N chains that are added in pairs, so that it rounds as little as the walk's sums over lanes do.
+// A sum over a key's entries as N chains that are added in pairs, as the walk adds its lanes' sums.
 template <int N>
 struct Chains {
     f32x4 part[N];
@@ -72,6 +80,12 @@ struct Chains {
         return t[0];
     }
 };
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+// mfma_k4 in float64; lane l's four sums are those of n = 4 e + l / 16 (not 4 (l / 16) + e) and m = l % 16, which is how the
+// products want the k of a next operand.
+__device__ __forceinline__ f64x4 mfma64_k4(double w, double a, f64x4 sums) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(w, a, sums, 0, 0, 0);
+}
 __device__ __forceinline__ bool not_finite(float v) { return !(fabsf(v) <= 3.4028235e38f); }
 
 template <int DB, bool CH, bool DELTA>
@@ -82,12 +96,15 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
                      int kv_heads, int heads, int V) {
     constexpr int D = 16 * DB, KLD = D + 4, TLD = CHUNK + 4;
     constexpr int NG = CH ? 4 * DB : 1;                       // decays a lane holds of its token
+    // (the linear attention's decays multiply single entries of a sum, whose roundings average out)
+    using Decay = typename std::conditional<DELTA, double, float>::type;
     // columns' keys in the order their lanes read them, later G_64 / G k with a row a key entry
     __shared__ __attribute__((aligned(16))) float cols[D * TLD];
     __shared__ __attribute__((aligned(16))) float rows[CHUNK * (DELTA ? KLD : TLD)];     // B, later G k and -T beta G k
     __shared__ __attribute__((aligned(16))) float lower[DELTA ? CHUNK * TLD : 4];        // beta A below the diagonal
     __shared__ __attribute__((aligned(16))) float inverse[DELTA ? 4 * 16 * 20 : 4];      // of I + its diagonal blocks
-    __shared__ float total[4][CH ? D : 1];                    // a block's product of decays
+    __shared__ __attribute__((aligned(16))) float solve[DELTA ? CHUNK * TLD : 4];        // T beta
+    __shared__ Decay total[4][CH ? D : 1];                    // a block's product of decays
     __shared__ float betas[CHUNK];
     __shared__ int wild_from, wild_values;
     const int h = blockIdx.x, chunk = blockIdx.y;             // (heads first, as in the other kernel: what it reads lies in its XCD's L2)
@@ -104,7 +121,8 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
     bool real = token < n;
     const float* row = qkv + (size_t)(first + (real ? token : 0)) * C;
     f32x4 kq[DB], qq[DB];
-    float pre[NG], beta = 0.f;
+    Decay pre[NG];
+    float beta = 0.f;
     bool wild = false, wild_query = false, wild_value = false;
 #pragma unroll
     for (int b = 0; b < DB; ++b) {
@@ -129,8 +147,9 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
         }
     } else {
         const float z = proj[(size_t)(first + (real ? token : 0)) * ld + a_off + h] + dt_bias[h];
-        pre[0] = expf(-expf(A_log[h]) * (z > 20.f ? z : log1pf(expf(z))));
-        wild |= not_finite(pre[0]);
+        const float factor = expf(-expf(A_log[h]) * (z > 20.f ? z : log1pf(expf(z))));
+        pre[0] = factor;
+        wild |= not_finite(factor);
     }
     if (DELTA) {
         beta = 1.0f / (1.0f + expf(-proj[(size_t)(first + (real ? token : 0)) * ld + b_off + h]));
@@ -159,12 +178,12 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
         ((int*)out)[at.from + c] = f;
     }
     real = real && token < from;
-    float suf[NG];
+    Decay suf[NG];
 #pragma unroll
-    for (int i = 0; i < NG; ++i) pre[i] = real ? pre[i] : 1.0f, suf[i] = 1.0f;
+    for (int i = 0; i < NG; ++i) pre[i] = real ? pre[i] : (Decay)1, suf[i] = 1;
     if (!real) beta = 0.f;
     if (q == 0) betas[token] = beta;
-    f32x4 part = {0.f, 0.f, 0.f, 0.f}, part2 = part;          // q . k of the token itself
+    double own = 0.0;                                         // q . k of the token itself
 #pragma unroll
     for (int b = 0; b < DB; ++b) {
         if (!real) kq[b] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -172,37 +191,35 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
         transpose_quads(kq[b]);
         transpose_quads(qq[b]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            if (b & 1) part2[e] = fmaf(qq[b][e], kq[b][e], part2[e]);
-            else part[e] = fmaf(qq[b][e], kq[b][e], part[e]);
-        }
+        for (int e = 0; e < 4; ++e) own = fma((double)qq[b][e], (double)kq[b][e], own);
     }
-    part += part2;
-    float own = (part[0] + part[1]) + (part[2] + part[3]);
     own += __shfl_xor(own, 16, HB_WAVE);
     own += __shfl_xor(own, 32, HB_WAVE);
 
-    // ---- pairs within the block, level by level; sums lie as (later token 4 q + e, earlier token r)
-    f32x4 a_sum = {0.f, 0.f, 0.f, 0.f}, b_sum = {0.f, 0.f, 0.f, 0.f};
+    // ---- pairs within the block, level by level; sums lie as (later token 4 e + q, earlier token r). (Sums of the pairs that
+    // are not a level's are not used: there is no need to make them zero.)
+    f64x4 a_sum = {0.0, 0.0, 0.0, 0.0}, b_sum = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-        if (4 * q + e == r) b_sum[e] = own;
+        if (4 * e + q == r) b_sum[e] = own;
 #pragma unroll
     for (int level = 0; level < 4; ++level) {
         const int s = 1 << level;
         const bool late = (r / s) & 1;
-        Chains<8> ac, bc;
+        // (the keys and queries are made float64 anew in every level: kept so they would take twice their registers)
+#pragma unroll
+        for (int b = 0; b < DB; ++b) asm volatile("" : "+v"(kq[b]), "+v"(qq[b]));
+        f64x4 al = {0.0, 0.0, 0.0, 0.0}, bl = al;
 #pragma unroll
         for (int i = 0; i < 4 * DB; ++i) {
-            const float k = kq[i / 4][i % 4], p = pre[CH ? i : 0];
-            const float early_k = late ? 0.f : k * suf[CH ? i : 0];
-            if (DELTA) ac.add(late ? k * p : 0.f, early_k, i);
-            bc.add(late ? qq[i / 4][i % 4] * p : 0.f, early_k, i);
+            const Decay f = late ? pre[CH ? i : 0] : suf[CH ? i : 0];
+            const double k = kq[i / 4][i % 4] * f;
+            if (DELTA) al = mfma64_k4(k, k, al);
+            bl = mfma64_k4(qq[i / 4][i % 4] * f, k, bl);
         }
-        const f32x4 al = ac.sum(), bl = bc.sum();
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int t = 4 * q + e;
+            const int t = 4 * e + q;
             const bool pair = t / (2 * s) == r / (2 * s) && ((t / s) & 1) && !((r / s) & 1);
             if (pair) a_sum[e] = al[e], b_sum[e] = bl[e];
         }
@@ -210,8 +227,8 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
         const int before = (lane & 48) + (r & ~(2 * s - 1)) + s - 1, after = before + s;
 #pragma unroll
         for (int i = 0; i < NG; ++i) {
-            const float p = pre[i];
-            const float head = __shfl(p, before, HB_WAVE), tail = __shfl(p, after, HB_WAVE);
+            const Decay p = pre[i];
+            const Decay head = __shfl(p, before, HB_WAVE), tail = __shfl(p, after, HB_WAVE);
             if (late) pre[i] = head * p;
             else suf[i] *= tail;
         }
@@ -228,66 +245,62 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
     for (int b = 0; b < DB; ++b) {
         f32x4 k;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) k[e] = kq[b][e] * suf[CH ? 4 * b + e : 0];
+        for (int e = 0; e < 4; ++e) k[e] = (float)(kq[b][e] * suf[CH ? 4 * b + e : 0]);
         *(f32x4*)&cols[((wave * DB + b) * 64 + lane) * 4] = k;
     }
-    auto put = [&](f32x4 a, f32x4 b, int block) {             // sums of (16 wave + 4 q + e, 16 block + r)
+    auto put = [&](f64x4 a, f64x4 b, int block) {             // sums of (16 wave + 4 e + q, 16 block + r)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int t = 16 * wave + 4 * q + e;
-            if (DELTA) lower[t * TLD + in_quads(16 * block + r)] = betas[t] * a[e];
-            rows[t * TLD + in_quads(16 * block + r)] = b[e];
+            const int t = 16 * wave + 4 * e + q;
+            if (DELTA) lower[t * TLD + in_quads(16 * block + r)] = (float)(betas[t] * a[e]);
+            rows[t * TLD + in_quads(16 * block + r)] = (float)b[e];
         }
     };
     put(a_sum, b_sum, wave);
     __syncthreads();
+    double x[DELTA ? 16 : 1];
     if (DELTA) {
         // the inverse of I + the diagonal block: column r of it, by substitution (the four lane rows do the same)
-        float x[16];
 #pragma unroll
         for (int t = 0; t < 16; ++t) {
-            float v = t == r ? 1.0f : 0.0f;
+            double v = t == r ? 1.0 : 0.0;
 #pragma unroll
-            for (int i = 0; i < t; ++i) v = fmaf(-lower[(16 * wave + t) * TLD + in_quads(16 * wave + i)], x[i], v);
+            for (int i = 0; i < t; ++i) v = fma(-(double)lower[(16 * wave + t) * TLD + in_quads(16 * wave + i)], x[i], v);
             x[t] = v;
         }
 #pragma unroll
         for (int t = 0; t < 16; ++t)
-            if ((t & 3) == q) inverse[(16 * wave + t) * 20 + in_quads(r)] = x[t];
+            if ((t & 3) == q) inverse[(16 * wave + t) * 20 + in_quads(r)] = (float)x[t];
     }
     // ---- pairs with earlier blocks, from the nearest on: the rows' decays grow by a block's product at a time
-#pragma unroll
-    for (int b = 0; b < DB; ++b)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float p = pre[CH ? 4 * b + e : 0];
-            qq[b][e] *= p;
-        }
-    f32x4 gk[DELTA ? DB : 1];                                 // G k
-    if (DELTA) {
-#pragma unroll
-        for (int b = 0; b < DB; ++b)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) gk[b][e] = kq[b][e] * pre[CH ? 4 * b + e : 0];
-    }
     for (int block = wave - 1; block >= 0; --block) {
-        Chains<8> ac, bc;
+        f64x4 al = {0.0, 0.0, 0.0, 0.0}, bl = al;
 #pragma unroll
         for (int b = 0; b < DB; ++b) {
             const f32x4 k = *(const f32x4*)&cols[((block * DB + b) * 64 + lane) * 4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                if (DELTA) ac.add(gk[b][e], k[e], 4 * b + e);
-                bc.add(qq[b][e], k[e], 4 * b + e);
-                const float p = CH ? total[block][16 * b + 4 * e + q] : total[block][0];
-                qq[b][e] *= p;
-                if (DELTA) gk[b][e] *= p;
+                const Decay p = pre[CH ? 4 * b + e : 0];
+                if (DELTA) al = mfma64_k4(kq[b][e] * p, k[e], al);
+                bl = mfma64_k4(qq[b][e] * p, k[e], bl);
+                if (CH) pre[4 * b + e] *= total[block][16 * b + 4 * e + q];
             }
         }
-        put(ac.sum(), bc.sum(), block);
+        if (!CH) pre[0] *= total[block][0];
+        put(al, bl, block);
     }
+    f32x4 gk[DELTA ? DB : 1];                                 // G k
 #pragma unroll
-    for (int b = 0; b < DB; ++b) *(f32x4*)(out + at.q + ((wave * DB + b) * 64 + lane) * 4) = qq[b];
+    for (int b = 0; b < DB; ++b) {
+        f32x4 gq;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const Decay p = pre[CH ? 4 * b + e : 0];
+            gq[e] = (float)(qq[b][e] * p);
+            if (DELTA) gk[b][e] = (float)(kq[b][e] * p);
+        }
+        *(f32x4*)(out + at.q + ((wave * DB + b) * 64 + lane) * 4) = gq;
+    }
     // behind a token to the chunk's end
     for (int block = wave + 1; block < 4; ++block) {
 #pragma unroll
@@ -301,7 +314,7 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
     if (CH) {
         for (int d = tid; d < D; d += 256) out[at.g + d] = total[0][d] * total[1][d] * total[2][d] * total[3][d];
     } else {
-        for (int d = tid; d < D; d += 256) out[at.g + d] = total[0][0] * total[1][0] * total[2][0] * total[3][0];
+        for (int d = tid; d < D; d += 256) out[at.g + d] = (float)(total[0][0] * total[1][0] * total[2][0] * total[3][0]);
     }
     __syncthreads();                                          // cols and rows have been read
 #pragma unroll
@@ -309,7 +322,7 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int d = 16 * b + 4 * e + q;
-            cols[d * TLD + in_quads(token)] = kq[b][e] * suf[CH ? 4 * b + e : 0];
+            cols[d * TLD + in_quads(token)] = (float)(kq[b][e] * suf[CH ? 4 * b + e : 0]);
             if (DELTA) rows[token * KLD + in_quads(d)] = gk[b][e];
         }
     __syncthreads();
@@ -320,46 +333,64 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
             *(f32x4*)(out + at.k + ((b * 4 + s) * 64 + lane) * 4) = *(const f32x4*)&cols[(16 * b + r) * TLD + 16 * s + 4 * q];
     if (!DELTA) return;
 
-    // ---- T applied to [beta G K | beta V], 16 columns at a time, block by block of tokens
+    // ---- T beta, a block of 16 columns a wave: its blocks of rows one after another, as the next product wants them
+    {
+        f64x4 t[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) t[0][e] = q == 0 ? x[4 * e] : q == 1 ? x[4 * e + 1] : q == 2 ? x[4 * e + 2] : x[4 * e + 3];
+#pragma unroll
+        for (int n_below = 0; n_below < 4; ++n_below) {       // (the block of rows wave + n_below)
+            const int i = wave + n_below;
+            if (i >= 4) break;
+            if (n_below > 0) {
+                f64x4 sum = {0.0, 0.0, 0.0, 0.0}, solved = sum;
+#pragma unroll
+                for (int j = 0; j < n_below; ++j) {
+                    const f32x4 l = *(const f32x4*)&lower[(16 * i + r) * TLD + 16 * (wave + j) + 4 * q];
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) sum = mfma64_k4(l[s], t[j][s], sum);
+                }
+                const f32x4 inv = *(const f32x4*)&inverse[(16 * i + r) * 20 + 4 * q];
+#pragma unroll
+                for (int s = 0; s < 4; ++s) solved = mfma64_k4(inv[s], -sum[s], solved);
+                t[n_below] = solved;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                solve[(16 * i + 4 * e + q) * TLD + in_quads(16 * wave + r)] = (float)(t[n_below][e] * betas[16 * wave + r]);
+        }
+    }
+    __syncthreads();
+    // ---- and applied to [G K | V], 16 columns at a time
     for (int cb = wave; cb < DB + V / 16; cb += 4) {
         const bool of_k = cb < DB;
-        f32x4 x[4];                                           // solved blocks, as the products want them
+        f32x4 y[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            f32x4 acc;
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int t = 16 * i + 4 * q + e;
+                const int t = 16 * j + 4 * e + q;
                 float v = 0.f;
                 if (of_k) v = rows[t * KLD + in_quads(16 * cb + r)];
                 else if (t < n && t < from) v = qkv[(size_t)(first + t) * C + v_at + 16 * (cb - DB) + r];
                 if (screen && not_finite(v)) v = 0.f;
-                acc[e] = betas[t] * v;
+                y[j][e] = v;
             }
-            if (i > 0) {
-                Chains<8> before;
 #pragma unroll
-                for (int j = 0; j < i; ++j) {
-                    const f32x4 l = *(const f32x4*)&lower[(16 * i + r) * TLD + 16 * j + 4 * q];
+        for (int i = 0; i < 4; ++i) {
+            f32x4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                    for (int s = 0; s < 4; ++s) before.add(l[s], x[j][s], 4 * j + s);
-                }
-                acc -= before.sum();
+            for (int j = 0; j <= i; ++j) {
+                const f32x4 w = *(const f32x4*)&solve[(16 * i + r) * TLD + 16 * j + 4 * q];
+#pragma unroll
+                for (int s = 0; s < 4; ++s) sum = mfma_k4(w[s], y[j][s], sum);
             }
-            transpose_quads(acc);
-            const f32x4 inv = *(const f32x4*)&inverse[(16 * i + r) * 20 + 4 * q];
-            Chains<4> with;
-#pragma unroll
-            for (int s = 0; s < 4; ++s) with.add(inv[s], acc[s], s);
-            const f32x4 solved = with.sum();
             if (of_k) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) rows[(16 * i + 4 * q + e) * KLD + in_quads(16 * cb + r)] = -solved[e];
+                for (int e = 0; e < 4; ++e) rows[(16 * i + 4 * q + e) * KLD + in_quads(16 * cb + r)] = -sum[e];
             } else {
-                *(f32x4*)(out + at.u + ((i * (V / 16) + cb - DB) * 64 + lane) * 4) = solved;
+                *(f32x4*)(out + at.u + ((i * (V / 16) + cb - DB) * 64 + lane) * 4) = sum;
             }
-            x[i] = solved;
-            transpose_quads(x[i]);
         }
     }
     __syncthreads();
@@ -461,26 +492,27 @@ chunk_scan_kernel(const float* __restrict__ qkv, int C, const float* __restrict_
 #pragma unroll
                 for (int e = 0; e < 4; ++e) us[b][e] = 16 * b + 4 * e + q < o.from ? o.v[4 * b + e] : 0.f;
         }
+        // The state and the outputs token by token in ascending order behind what the state before gives, so that the latest tokens,
+        // mostly the largest, are added last: as the walk rounds, without its decay of every token.
+        f32x4 sums = oc.sum();
 #pragma unroll
-        for (int i = 0; i < OWN; ++i) {
-            Chains<8> kc;
+        for (int i = 0; i < OWN; ++i)
 #pragma unroll
-            for (int b = 0; b < 4; ++b)
+            for (int e = 0; e < 4; ++e) S[i][e] *= o.g[i][e];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) kc.add(o.k[i][b][e], us[b][e], 4 * b + e);
-            const f32x4 added = kc.sum();
+        for (int b = 0; b < 4; ++b) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) S[i][e] = fmaf(S[i][e], o.g[i][e], added[e]);
-            if (o.from < CHUNK) S[i] = f32x4{NAN, NAN, NAN, NAN};
+            for (int e = 0; e < 4; ++e) {
+#pragma unroll
+                for (int i = 0; i < OWN; ++i) S[i] = mfma_k4(o.k[i][b][e], us[b][e], S[i]);
+                if (b <= wave) sums = mfma_k4(o.b[b][e], us[b][e], sums);
+            }
+        }
+        if (o.from < CHUNK) {
+#pragma unroll
+            for (int i = 0; i < OWN; ++i) S[i] = f32x4{NAN, NAN, NAN, NAN};
         }
         share(buf ^ 1);
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-            if (b <= wave) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) oc.add(o.b[b][e], us[b][e], 4 * b + e);
-            }
-        const f32x4 sums = oc.sum();
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int t = 16 * wave + 4 * q + e, at_token = c * CHUNK + t;

@@ -102,18 +102,18 @@ def chunk_floats(D, V, correction):
     return (3 if correction else 2) * CHUNK * D + CHUNK * CHUNK + (CHUNK * V if correction else 0) + D + V + 4
 
 
-def chunks_from(portions, heads, correction):
-    """The fewest tokens with which one of a step's portions goes through in chunks.
-    The walk takes 0.4 us a token of the longest portion while its waves fit the chip; the chunks 37 us (24 without the
-    correction) and 5 us a chunk. One sequence of 16 heads of 128: 96 tokens 43 us either way, 64 tokens 33 against 38
-    (without the correction 48 tokens: 28 against 25). With many such portions or heads the walk's waves wait for each other
-    and the chunks still fill the chip: 8 sequences of 64 tokens 108 against 57, of 32 tokens 60 against 57, 24 sequences of 18 to
-    90 tokens 366 against 170 (without the correction 16 sequences of 16 tokens: 71 against 57)."""
-    lines = [(24, 256), (32, 128), (96, 1)] if correction else [(16, 128), (48, 1)]      # tokens, (sequence, head) pairs from there on
-    for tokens, pairs in lines:
-        if int((portions >= tokens).sum()) * heads >= pairs:
-            return tokens
-    return int(portions.max(initial=0)) + 1
+def chunks_from(portions, heads, correction, channels):
+    """The fewest tokens with which one of a step's portions goes through in chunks (channels: a decay a key channel).
+    The walk takes 0.4 us a token of the longest portion (0.6 with a decay a channel) while its waves fit the chip; the chunks 42 us
+    (54, without the correction 27) and 4 us a chunk. One sequence of 16 heads of 128: 96 tokens 41 against 46 us, with a
+    decay a channel 57 either way, without the correction 48 tokens 27 either way. With many such portions or heads the
+    walk's waves wait for each other and the chunks still fill the chip: 8 sequences of 32 tokens 58 us either way, of 64 103 against
+    60, with a decay a channel 32 tokens 56 against 70 and 64 tokens 96 against 72, without the correction 12 of 20 tokens 64 against 51
+    and 8 of 16 37 against 40."""
+    few, many = (48, 20) if not correction else (96, 40) if channels else (112, 32)
+    if int((portions >= many).sum()) * heads >= 128:
+        return many
+    return few if portions.max(initial=0) >= few else int(portions.max(initial=0)) + 1
 
 
 def walks_of(portions, least, heads):
@@ -154,15 +154,15 @@ def chunk_calls(starts, least, room):
     return calls
 
 
-def _chunk_lists(meta, heads, correction, size):
+def _chunk_lists(meta, heads, correction, channels, size):
     """(calls, floats, walks) of the step, made once for all its layers: for each call in chunks the GPU's (runs, their number,
     chunks, their number), the scratch they need, and for each launch of the other portions the GPU's list of sequences, their
     number and the most tokens that one of them brings."""
-    key = ("delta_chunks", heads, correction, size, CHUNK_SCRATCH)
+    key = ("delta_chunks", heads, correction, channels, size, CHUNK_SCRATCH)
     got = meta.derived.get(key)
     if got is None:
         portions = np.diff(meta.host_starts)
-        least = chunks_from(portions, heads, correction)
+        least = chunks_from(portions, heads, correction, channels)
         packed, calls, walks = [], [], []
 
         def place(numbers):                                    # (16 bytes aligned)
@@ -194,7 +194,7 @@ def _rule(rt, qkv, proj, b_off, a_off, a_log, dt_bias, decay, state, meta, out, 
     if (rt is not None and meta.max_new > 1 and D in (64, 128) and V % 16 == 0 and qkv.shape[1] % 4 == 0
             and qkv.data_ptr() % 16 == 0 and (decay is None or decay.data_ptr() % 16 == 0)):
         size = chunk_floats(D, V, correction)
-        calls, floats, walks = _chunk_lists(meta, heads, correction, size)
+        calls, floats, walks = _chunk_lists(meta, heads, correction, decay is not None, size)
         scratch = rt.buffer("delta_chunks", (floats,), torch.float32) if calls else None
         for runs, n_runs, chunks, n_chunks in calls:
             lib.call("recurrent_chunks", "hb_chunked_delta", *operands, chunks.data_ptr(), n_chunks, runs.data_ptr(), n_runs,

@@ -58,13 +58,11 @@ def test_many_short_portions_keep_the_scratch_bounded():
 def test_the_portions_that_take_chunks_decide():
     """The lines for many portions count those that are long enough, not the single tokens beside them."""
     ones = [1] * 47
-    assert recurrent.chunks_from(np.array([95] + ones), 16, True) == 96                # none
-    assert recurrent.chunks_from(np.array([96] + ones), 16, True) == 96
-    assert recurrent.chunks_from(np.array([48] + ones), 16, False) == 48
-    assert recurrent.chunks_from(np.array([40] * 8 + ones), 16, True) == 32
-    assert recurrent.chunks_from(np.array([24] * 16 + ones), 16, True) == 24
-    assert recurrent.chunks_from(np.array([20] * 8 + ones), 16, False) == 16
-    assert recurrent.chunks_from(np.array([9] * 80 + ones), 16, True) == 10            # none
+    for few, many, form in ((112, 32, (True, False)), (96, 40, (True, True)), (48, 20, (False, True))):
+        assert recurrent.chunks_from(np.array([few - 1] + ones), 16, *form) == few                # none
+        assert recurrent.chunks_from(np.array([few] + ones), 16, *form) == few
+        assert recurrent.chunks_from(np.array([many] * 8 + ones), 16, *form) == many
+        assert recurrent.chunks_from(np.array([many - 1] * 80 + ones), 16, *form) == many         # none
 
 
 @pytest.mark.parametrize("portions,least,launches", [([1, 1], 96, 1), ([0, 0], 96, 0), ([3, 0, 1], 96, 1), ([5] + [1] * 8, 96, 2),

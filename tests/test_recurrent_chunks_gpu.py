@@ -125,6 +125,38 @@ def test_long_portions_take_chunks_beside_short_ones(kind, lengths, monkeypatch)
 
 
 @pytest.mark.parametrize("kind", ["head", "channel", "linear"])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("decay", [None, 0.5, 0.9, 0.99, 0.999])       # (None: spread over (0, 1))
+@pytest.mark.parametrize("cosine", [0.0, 0.8])
+def test_chunks_are_as_close_to_the_rule_as_the_walk(kind, D, decay, cosine):
+    """Keys drawn at random and keys that resemble each other, decays about a value: the outputs' error against 64 bits is no
+    larger than the walk's; the state's no larger by more than a tenth (seen: 1.06 of the walk's, both below 1.1e-7 there)."""
+    from herbert_rs_amd.kernels import recurrent
+    lengths, heads, V = [233], 8, 48
+    qkv, proj, a_log, dt_bias, decays, state, meta = step(lengths, heads, heads, D, V, kind, 0.0, seed=D)
+    g = torch.Generator().manual_seed(7)
+    if cosine:
+        keys = qkv[:, heads * D:2 * heads * D].view(233, heads, D)
+        base = torch.randn(heads, D, generator=g).abs()
+        keys.copy_((1 - cosine) ** 0.5 * keys + cosine ** 0.5 * base / base.norm(dim=-1, keepdim=True))
+        keys /= keys.norm(dim=-1, keepdim=True)
+    if decay is not None:
+        rate = -2.0 * torch.log(torch.tensor(decay))
+        decays = torch.exp(-rate * torch.rand(233, heads, D, generator=g))
+        a_log, dt_bias = torch.zeros(heads), torch.zeros(heads)
+        proj[:, heads:2 * heads] = torch.log(torch.expm1(rate * torch.rand(233, heads, generator=g).clamp(min=1e-4)))
+    case = (qkv, proj, a_log, dt_bias, decays, state)
+    want, want_state = expected(*case, lengths, heads, heads, D, V, kind)
+    got, left = run(*case, meta, heads, heads, D, V, kind)
+    out, held = torch.empty(233, heads * V, device=dev()), state.to(dev())
+    recurrent.gated_delta(qkv.to(dev()), None if kind == "linear" else proj.to(dev()), 0, heads, a_log.to(dev()), dt_bias.to(dev()), held,
+                          meta, out, heads, heads, D, V, decay=None if kind == "head" else decays.reshape(233, heads * D).to(dev()),
+                          correction=kind != "linear", out_scale=0.5)
+    assert float((got - want).norm()) <= float((out.cpu().view(233, heads, V) - want).norm())
+    assert float((left - want_state).norm()) <= 1.1 * float((held.cpu() - want_state).norm())
+
+
+@pytest.mark.parametrize("kind", ["head", "channel", "linear"])
 @pytest.mark.parametrize("place", [3, 64 + 17])
 @pytest.mark.parametrize("what", ["query", "key", "value"])
 def test_a_number_that_is_not_finite_reaches_what_it_reaches_in_the_walk(kind, place, what):
@@ -132,7 +164,7 @@ def test_a_number_that_is_not_finite_reaches_what_it_reaches_in_the_walk(kind, p
     walk token by token loses is lost (of the linear attention's state, after a key, all rows for one that no later output
     is without). All else is the same bits as without it."""
     from herbert_rs_amd.kernels import recurrent
-    kv_heads, heads, D, V, lengths = 2, 2, 64, 32, [150, 100]
+    kv_heads, heads, D, V, lengths = 2, 2, 64, 32, [150, 112]
     case = list(step(lengths, kv_heads, heads, D, V, kind, 0.0))
     clean, state = run(*case, kv_heads, heads, D, V, kind)
     case[0] = case[0].clone()
@@ -141,11 +173,11 @@ def test_a_number_that_is_not_finite_reaches_what_it_reaches_in_the_walk(kind, p
     got, left = run(*case, kv_heads, heads, D, V, kind)
 
     qkv, proj, a_log, dt_bias, decay, held, meta = case
-    out, held = torch.full((250, heads * V), 7.0, device=dev()), held.to(dev())
+    out, held = torch.full((262, heads * V), 7.0, device=dev()), held.to(dev())
     recurrent.gated_delta(qkv.to(dev()), None if kind == "linear" else proj.to(dev()), 0, heads, a_log.to(dev()), dt_bias.to(dev()), held,
-                          meta, out, kv_heads, heads, D, V, decay=None if kind == "head" else decay.reshape(250, heads * D).to(dev()),
+                          meta, out, kv_heads, heads, D, V, decay=None if kind == "head" else decay.reshape(262, heads * D).to(dev()),
                           correction=kind != "linear", out_scale=0.5)
-    fine, fine_state = out.cpu().view(250, heads, V).isfinite(), held.cpu().isfinite()
+    fine, fine_state = out.cpu().view(262, heads, V).isfinite(), held.cpu().isfinite()
     assert torch.equal(got.isfinite(), fine) and torch.equal(got[fine], clean[fine])
     if kind == "linear" and what == "key":
         assert not fine_state[2, 1].all()
