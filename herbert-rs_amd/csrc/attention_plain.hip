@@ -6,16 +6,17 @@
 // online softmax: the chunking, and so the rounding, depends on the positions only,
 // not on how the tokens were cut into steps or batches.
 // A workgroup of four waves takes 16 columns: the query heads of one key head for one token (a decode step), or for
-// the next few packed tokens (a prompt), each with its own mask. Both contractions run on the matrix cores in float32
+// the next few tokens of one sequence (a prompt), each with its own mask. Both contractions run on the matrix cores in float32
 // (mfma_f32.h), whose sums are chains of fmaf over ascending k: a score over the head's entries, an output over a chunk's keys. A
 // wave scores 16 of a chunk's 64 keys, the scores meet in LDS, where every wave reads all 64 of its lanes' columns as the
 // second product wants them (the weights never leave the registers again), and each wave owns a quarter of the
 // head's entries of the output. A chunk's values are asked for before its scores are computed and the next chunk's keys after.
 // The sum of a chunk's weights is a fixed tree over the keys' numbers. A chunk that a column does not see leaves
 // it as it was, bit for bit, so a column's result is the same whatever tile it is in.
-// Bound by the chain of a chunk's steps in a workgroup (about 5 us a chunk of heads of 128, 4,096 keys 318); two prompts of 333 and
-// 230 tokens, 16 heads of 128 on 8, take 57 us and a decode step of them 36, where a wave a (token, head) with a
-// key a lane took 725 and 138 (1,683 at 4,096 keys).
+// Bound by the chain of a chunk's steps in a workgroup (about 5 us a chunk of heads of 128, 4,096 keys 317); two prompts of 333 and
+// 230 tokens, 16 heads of 128 on 8, take 42 us and a decode step of them 33, where a wave a (token, head) with a
+// key a lane took 712 and 134 (1,681 at 4,096 keys). A tile holds tokens of one sequence: a prompt of 512 tokens beside 15 single
+// tokens at 4,096 keys takes 420 us, and took 2,670 where the next packed tokens were a tile whoever's they were.
 // In xigh/herbert-rs: scores q . k / sqrt(hd), query head h on kv head h / (nq / nkv)
 // (crates/backends/backend_common/src/generic_attention/decode.rs:126), causal by count
 // (crates/backends/backend_common/src/generic_attention/prefill/kernel_f32.rs:65-67), online softmax and
@@ -59,9 +60,10 @@ attention_plain_kernel(const T* __restrict__ q, const T* __restrict__ k_cache,
                        const T* __restrict__ v_cache, TO* __restrict__ out,
                        const int* __restrict__ positions, const int* __restrict__ seq_of,
                        const int* __restrict__ slots, const int* __restrict__ page_table, int max_pages,
-                       int page_size, int n_tokens, int nq, int nkv, int hd, float scale, int window,
+                       int page_size, int nq, int nkv, int hd, float scale, int window,
                        const float* __restrict__ sinks, int chunk, float softcap, const float* __restrict__ bias,
-                       int bias_ld, int bias_at, int bias_len, int keep_first, int heads_a_tile, int tokens_a_tile) {
+                       int bias_ld, int bias_at, int bias_len, int keep_first, int heads_a_tile,
+                       const int2* __restrict__ tiles) {
     constexpr int DB = 4 * NB;                       // blocks of 16 entries of a head
     constexpr int QLD = 16 * DB + 4, SLD = CHUNK + 4;
     __shared__ __attribute__((aligned(16))) float qs[16 * QLD], ss[16 * SLD];
@@ -69,8 +71,8 @@ attention_plain_kernel(const T* __restrict__ q, const T* __restrict__ k_cache,
     const int r = lane & 15, g4 = lane >> 4;
     const int group = nq / nkv, tiles_a_head = (group + heads_a_tile - 1) / heads_a_tile;
     const int g = blockIdx.y / tiles_a_head, h_first = blockIdx.y % tiles_a_head * heads_a_tile;
-    const int t0 = blockIdx.x * tokens_a_tile;
-    const int n_here = n_tokens - t0 < tokens_a_tile ? n_tokens - t0 : tokens_a_tile;
+    // (a list of the tiles' first tokens and how many they are, all of one sequence, or a token a tile)
+    const int t0 = tiles ? tiles[blockIdx.x].x : blockIdx.x, n_here = tiles ? tiles[blockIdx.x].y : 1;
 
     // the queries, zeros beyond the head's entries and in columns that are nobody's, every 16 entries transposed
     for (int i = tid; i < 16 * 16 * DB; i += 256) {
@@ -93,167 +95,158 @@ attention_plain_kernel(const T* __restrict__ q, const T* __restrict__ k_cache,
     for (int i = 0; i < NB; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     __syncthreads();
 
-    // runs of the tile's tokens that belong to one sequence (a prompt's tile has mostly one)
-    for (int first = 0; first < n_here;) {
-        const int seq = seq_of[t0 + first];
-        int last = first + 1;
-        while (last < n_here && seq_of[t0 + last] == seq) ++last;
-        const int* pt = page_table + (size_t)slots[seq] * max_pages;
-        const bool in_run = mine && my_tok >= first && my_tok < last;
-        // what the run's tokens see together
-        Seen all = seen_by(positions[t0 + first], window, chunk, keep_first);
-        for (int i = first + 1; i < last; ++i) {
-            const Seen s = seen_by(positions[t0 + i], window, chunk, keep_first);
-            all.lo = min(all.lo, s.lo), all.hi = max(all.hi, s.hi), all.kept = max(all.kept, s.kept);
-        }
-        first = last;
-        auto next_of = [&](int c) {        // the chunk after c - CHUNK that some token sees
-            return c >= all.kept && c + CHUNK <= all.lo ? all.lo / CHUNK * CHUNK : c;
-        };
-        // (keys from all.hi on are the last key once more; a table's entries are pages that exist)
-        f32x4 key[DB], val_next[AHEAD ? NB : 1][4];
-        auto fetch_keys = [&](int c, int page) {
-            const int j = min(c + 16 * wave + r, all.hi - 1);
-            const int in_page = VEC ? c % page_size + j - c : j % page_size;
-            const T* row = k_cache + (((size_t)(VEC ? page : pt[j / page_size]) * nkv + g) * page_size + in_page) * hd + 4 * g4;
+    const int* pt = page_table + (size_t)slots[seq_of[t0]] * max_pages;
+    // what the tile's tokens see together
+    Seen all = seen_by(positions[t0], window, chunk, keep_first);
+    for (int i = 1; i < n_here; ++i) {
+        const Seen s = seen_by(positions[t0 + i], window, chunk, keep_first);
+        all.lo = min(all.lo, s.lo), all.hi = max(all.hi, s.hi), all.kept = max(all.kept, s.kept);
+    }
+    auto next_of = [&](int c) {        // the chunk after c - CHUNK that some token sees
+        return c >= all.kept && c + CHUNK <= all.lo ? all.lo / CHUNK * CHUNK : c;
+    };
+    // (keys from all.hi on are the last key once more; a table's entries are pages that exist)
+    f32x4 key[DB], val_next[AHEAD ? NB : 1][4];
+    auto fetch_keys = [&](int c, int page) {
+        const int j = min(c + 16 * wave + r, all.hi - 1);
+        const int in_page = VEC ? c % page_size + j - c : j % page_size;
+        const T* row = k_cache + (((size_t)(VEC ? page : pt[j / page_size]) * nkv + g) * page_size + in_page) * hd + 4 * g4;
 #pragma unroll
-            for (int b = 0; b < DB; ++b) key[b] = load_quad<VEC>(row + 16 * b, hd - 16 * b - 4 * g4);
-        };
-        auto fetch_values = [&](int c, int page, int i, f32x4 (&to)[4]) {       // of the wave's i-th block of entries
-            const T* at = v_cache + ((size_t)page * nkv + g) * hd * page_size + c % page_size + 4 * g4;
-            const int d = 16 * (wave + 4 * i) + r;
+        for (int b = 0; b < DB; ++b) key[b] = load_quad<VEC>(row + 16 * b, hd - 16 * b - 4 * g4);
+    };
+    auto fetch_values = [&](int c, int page, int i, f32x4 (&to)[4]) {       // of the wave's i-th block of entries
+        const T* at = v_cache + ((size_t)page * nkv + g) * hd * page_size + c % page_size + 4 * g4;
+        const int d = 16 * (wave + 4 * i) + r;
 #pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                to[b] = f32x4{0.f, 0.f, 0.f, 0.f};
-                const int j = c + 16 * b + 4 * g4;
-                if (VEC) {
-                    if (d < hd && j < all.hi) to[b] = load_quad<true>(at + (size_t)d * page_size + 16 * b, 4);
-                } else {
+        for (int b = 0; b < 4; ++b) {
+            to[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+            const int j = c + 16 * b + 4 * g4;
+            if (VEC) {
+                if (d < hd && j < all.hi) to[b] = load_quad<true>(at + (size_t)d * page_size + 16 * b, 4);
+            } else {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (d < hd && j + e < all.hi)
-                            to[b][e] = hb_to_float(v_cache[(((size_t)pt[(j + e) / page_size] * nkv + g) * hd + d) * page_size + (j + e) % page_size]);
-                }
+                for (int e = 0; e < 4; ++e)
+                    if (d < hd && j + e < all.hi)
+                        to[b][e] = hb_to_float(v_cache[(((size_t)pt[(j + e) / page_size] * nkv + g) * hd + d) * page_size + (j + e) % page_size]);
             }
-        };
-        int c = next_of(all.kept > 0 ? 0 : all.lo / CHUNK * CHUNK);
-        int following = next_of(c + CHUNK);
-        // (the page after the next is looked up a chunk before its loads are asked for)
-        int page = pt[c / page_size], page_next = following < all.hi ? pt[following / page_size] : 0;
-        fetch_keys(c, page);
+        }
+    };
+    int c = next_of(all.kept > 0 ? 0 : all.lo / CHUNK * CHUNK);
+    int following = next_of(c + CHUNK);
+    // (the page after the next is looked up a chunk before its loads are asked for)
+    int page = pt[c / page_size], page_next = following < all.hi ? pt[following / page_size] : 0;
+    fetch_keys(c, page);
+    if (AHEAD) {
+#pragma unroll
+        for (int i = 0; i < NB; ++i) fetch_values(c, page, i, val_next[i]);
+    }
+    while (c < all.hi) {
+        f32x4 val[AHEAD ? NB : 1][4];
         if (AHEAD) {
 #pragma unroll
-            for (int i = 0; i < NB; ++i) fetch_values(c, page, i, val_next[i]);
+            for (int i = 0; i < NB; ++i)
+#pragma unroll
+                for (int b = 0; b < 4; ++b) val[i][b] = val_next[i][b];
         }
-        while (c < all.hi) {
-            f32x4 val[AHEAD ? NB : 1][4];
-            if (AHEAD) {
+        f32x4 dots = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int i = 0; i < NB; ++i)
+        for (int b = 0; b < DB; ++b) {
+            transpose_quads(key[b]);
+            const f32x4 qq = *(const f32x4*)&qs[r * QLD + 16 * b + 4 * g4];
 #pragma unroll
-                    for (int b = 0; b < 4; ++b) val[i][b] = val_next[i][b];
+            for (int s = 0; s < 4; ++s) dots = mfma_k4(key[b][s], qq[s], dots);
+        }
+        const int after = next_of(following + CHUNK);
+        const int page_after = after < all.hi ? pt[after / page_size] : 0;
+        if (AHEAD && following < all.hi) {
+            fetch_keys(following, page_next);
+#pragma unroll
+            for (int i = 0; i < NB; ++i) fetch_values(following, page_next, i, val_next[i]);
+        }
+        __syncthreads();                              // (the chunk before has been read)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int j = c + 16 * wave + 4 * g4 + e;
+            float s = dots[e] * scale;
+            if (softcap > 0.f) s = softcap * tanhf(s / softcap);
+            if (bias) {
+                const int n = max(0, min(pos - j, bias_len - 1));
+                s += bias[(size_t)h * bias_ld + bias_at + bias_len - 1 - n];
             }
-            f32x4 dots = {0.f, 0.f, 0.f, 0.f};
+            const bool valid = mine && (j >= see.lo || j < see.kept) && j < see.hi;
+            ss[r * SLD + 16 * wave + 4 * e + g4] = valid ? s : -INFINITY;
+        }
+        __syncthreads();
+        // this lane's share of its column: keys 16 b + 4 s + g4
+        f32x4 p[4];
+        float top = -INFINITY;
 #pragma unroll
-            for (int b = 0; b < DB; ++b) {
-                transpose_quads(key[b]);
-                const f32x4 qq = *(const f32x4*)&qs[r * QLD + 16 * b + 4 * g4];
+        for (int b = 0; b < 4; ++b) {
+            p[b] = *(const f32x4*)&ss[r * SLD + 16 * b + 4 * g4];
+            top = fmaxf(top, fmaxf(fmaxf(p[b][0], p[b][1]), fmaxf(p[b][2], p[b][3])));
+        }
+        top = fmaxf(top, __shfl_xor(top, 16, HB_WAVE));
+        top = fmaxf(top, __shfl_xor(top, 32, HB_WAVE));
+        const bool sees = mine && ((c < see.hi && c + CHUNK > see.lo) || c < see.kept);
+        float corr = 1.0f;
+        if (sees) {
+            const float m_new = fmaxf(m, top);
+            corr = expf(m - m_new);
+            m = m_new;
+        }
 #pragma unroll
-                for (int s = 0; s < 4; ++s) dots = mfma_k4(key[b][s], qq[s], dots);
-            }
-            const int after = next_of(following + CHUNK);
-            const int page_after = after < all.hi ? pt[after / page_size] : 0;
-            if (AHEAD && following < all.hi) {
-                fetch_keys(following, page_next);
+        for (int b = 0; b < 4; ++b)
 #pragma unroll
-                for (int i = 0; i < NB; ++i) fetch_values(following, page_next, i, val_next[i]);
-            }
-            __syncthreads();                              // (the chunk before has been read)
+            for (int s = 0; s < 4; ++s) p[b][s] = sees && p[b][s] != -INFINITY ? expf(p[b][s] - m) : 0.f;
+        // the tree: key j with j ^ 32, j ^ 16 (blocks), j ^ 8, j ^ 4 (quads), j ^ 2, j ^ 1 (lanes)
+        f32x4 t = (p[0] + p[2]) + (p[1] + p[3]);
+        float sum = (t[0] + t[2]) + (t[1] + t[3]);
+        sum += __shfl_xor(sum, 32, HB_WAVE);
+        sum += __shfl_xor(sum, 16, HB_WAVE);
+        l = l * corr + sum;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int j = c + 16 * wave + 4 * g4 + e;
-                float s = dots[e] * scale;
-                if (softcap > 0.f) s = softcap * tanhf(s / softcap);
-                if (bias) {
-                    const int n = max(0, min(pos - j, bias_len - 1));
-                    s += bias[(size_t)h * bias_ld + bias_at + bias_len - 1 - n];
-                }
-                const bool valid = in_run && (j >= see.lo || j < see.kept) && j < see.hi;
-                ss[r * SLD + 16 * wave + 4 * e + g4] = valid ? s : -INFINITY;
-            }
-            __syncthreads();
-            // this lane's share of its column: keys 16 b + 4 s + g4
-            f32x4 p[4];
-            float top = -INFINITY;
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                p[b] = *(const f32x4*)&ss[r * SLD + 16 * b + 4 * g4];
-                top = fmaxf(top, fmaxf(fmaxf(p[b][0], p[b][1]), fmaxf(p[b][2], p[b][3])));
-            }
-            top = fmaxf(top, __shfl_xor(top, 16, HB_WAVE));
-            top = fmaxf(top, __shfl_xor(top, 32, HB_WAVE));
-            const bool sees = in_run && ((c < see.hi && c + CHUNK > see.lo) || c < see.kept);
-            float corr = 1.0f;
-            if (sees) {
-                const float m_new = fmaxf(m, top);
-                corr = expf(m - m_new);
-                m = m_new;
-            }
+        for (int i = 0; i < NB; ++i) {
+            acc[i] *= corr;
+            f32x4 (&v)[4] = val[AHEAD ? i : 0];
+            if (!AHEAD) fetch_values(c, page, i, v);
+            // a value without a finite size, perhaps of a key that some column does not see: a weight of zero does
+            // not hide it
+            bool wild = false;
 #pragma unroll
             for (int b = 0; b < 4; ++b)
 #pragma unroll
-                for (int s = 0; s < 4; ++s) p[b][s] = sees && p[b][s] != -INFINITY ? expf(p[b][s] - m) : 0.f;
-            // the tree: key j with j ^ 32, j ^ 16 (blocks), j ^ 8, j ^ 4 (quads), j ^ 2, j ^ 1 (lanes)
-            f32x4 t = (p[0] + p[2]) + (p[1] + p[3]);
-            float sum = (t[0] + t[2]) + (t[1] + t[3]);
-            sum += __shfl_xor(sum, 32, HB_WAVE);
-            sum += __shfl_xor(sum, 16, HB_WAVE);
-            l = l * corr + sum;
-#pragma unroll
-            for (int i = 0; i < NB; ++i) {
-                acc[i] *= corr;
-                f32x4 (&v)[4] = val[AHEAD ? i : 0];
-                if (!AHEAD) fetch_values(c, page, i, v);
-                // a value without a finite size, perhaps of a key that some column does not see: a weight of zero does
-                // not hide it
-                bool wild = false;
-#pragma unroll
-                for (int b = 0; b < 4; ++b)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        if (VEC && c + 16 * b + 4 * g4 + e >= all.hi) v[b][e] = 0.f;
-                        wild |= !(fabsf(v[b][e]) <= 3.4028235e38f);
-                    }
-                if (!__any(wild)) {
-#pragma unroll
-                    for (int b = 0; b < 4; ++b) {
-                        transpose_quads(v[b]);
-#pragma unroll
-                        for (int s = 0; s < 4; ++s) acc[i] = mfma_k4(v[b][s], p[b][s], acc[i]);
-                    }
-                    continue;
+                for (int e = 0; e < 4; ++e) {
+                    if (VEC && c + 16 * b + 4 * g4 + e >= all.hi) v[b][e] = 0.f;
+                    wild |= !(fabsf(v[b][e]) <= 3.4028235e38f);
                 }
+            if (!__any(wild)) {
 #pragma unroll
-                for (int b = 0; b < 4; ++b)
-                    for (int s = 0; s < 4; ++s)
-                        for (int k = 0; k < 4; ++k) {
-                            const int j = c + 16 * b + 4 * s + k;
-                            const float w = __shfl(s == 0 ? p[b][0] : s == 1 ? p[b][1] : s == 2 ? p[b][2] : p[b][3], 16 * k + r, HB_WAVE);
-                            if (j >= all.hi) continue;
-                            const T* v = v_cache + ((size_t)pt[j / page_size] * nkv + g) * hd * page_size + j % page_size;
-                            const bool valid = in_run && (j >= see.lo || j < see.kept) && j < see.hi;
+                for (int b = 0; b < 4; ++b) {
+                    transpose_quads(v[b]);
 #pragma unroll
-                            for (int e = 0; e < 4; ++e) {
-                                const int d = 16 * (wave + 4 * i) + 4 * g4 + e;
-                                if (valid && d < hd) acc[i][e] = fmaf(w, hb_to_float(v[(size_t)d * page_size]), acc[i][e]);
-                            }
-                        }
+                    for (int s = 0; s < 4; ++s) acc[i] = mfma_k4(v[b][s], p[b][s], acc[i]);
+                }
+                continue;
             }
-            if (!AHEAD && following < all.hi) fetch_keys(following, page_next);
-            c = following, following = after;
-            page = page_next, page_next = page_after;
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+                for (int s = 0; s < 4; ++s)
+                    for (int k = 0; k < 4; ++k) {
+                        const int j = c + 16 * b + 4 * s + k;
+                        const float w = __shfl(s == 0 ? p[b][0] : s == 1 ? p[b][1] : s == 2 ? p[b][2] : p[b][3], 16 * k + r, HB_WAVE);
+                        if (j >= all.hi) continue;
+                        const T* v = v_cache + ((size_t)pt[j / page_size] * nkv + g) * hd * page_size + j % page_size;
+                        const bool valid = mine && (j >= see.lo || j < see.kept) && j < see.hi;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const int d = 16 * (wave + 4 * i) + 4 * g4 + e;
+                            if (valid && d < hd) acc[i][e] = fmaf(w, hb_to_float(v[(size_t)d * page_size]), acc[i][e]);
+                        }
+                    }
         }
-        __syncthreads();
+        if (!AHEAD && following < all.hi) fetch_keys(following, page_next);
+        c = following, following = after;
+        page = page_next, page_next = page_after;
     }
     if (!mine) return;
     const float inv = l > 0.f ? 1.0f / l : 0.f;
@@ -269,13 +262,16 @@ attention_plain_kernel(const T* __restrict__ q, const T* __restrict__ k_cache,
 
 // q, out: [T, nq * hd]; keys [pages, nkv, page_size, hd], values [pages, nkv, hd, page_size];
 // dtype covers q and cache, and out unless out_dtype says float32.
+// tiles [n_tiles, 2] or null: the tiles that the packed tokens are cut into, as the first token and how many, up to tokens_a_tile
+// (as many as fit 16 columns beside a key head's query heads) of one sequence; null: every token is a tile.
 extern "C" int hb_attention_plain(const void* q, const void* k_cache, const void* v_cache, void* out,
                                   int dtype, const int* positions, const int* seq_of, const int* slots,
-                                  const int* page_table, int max_pages, int page_size, int T, int n_seqs, int nq,
+                                  const int* page_table, int max_pages, int page_size, int T, const int* tiles,
+                                  int n_tiles, int tokens_a_tile, int nq,
                                   int nkv, int hd, float scale, int window, const float* sinks,
                                   int chunk, float softcap, const float* bias, int bias_ld, int bias_at,
                                   int bias_len, int keep_first, int out_dtype, hipStream_t stream) {
-    HB_REQUIRE(T > 0 && n_seqs > 0 && nq > 0 && nkv > 0, "attention: empty input");
+    HB_REQUIRE(T > 0 && nq > 0 && nkv > 0, "attention: empty input");
     HB_REQUIRE(nq % nkv == 0, "attention: %d query heads not divisible by %d kv heads", nq, nkv);
     HB_REQUIRE(hd > 0 && hd <= HB_MAX_HEAD_DIM, "attention: head_dim %d not in 1..%d", hd,
                HB_MAX_HEAD_DIM);
@@ -285,19 +281,20 @@ extern "C" int hb_attention_plain(const void* q, const void* k_cache, const void
     HB_REQUIRE(!bias || (bias_len > 0 && bias_at >= 0 && bias_at + bias_len <= bias_ld), "attention: bad table of biases");
     HB_REQUIRE(nq <= 65535, "attention: too many heads for the grid");
     HB_REQUIRE(out_dtype == dtype || out_dtype == HB_F32, "attention: the output is stored as the cache is, or in float32");
-    // a key head's query heads side by side; where there is room, and more tokens than sequences, several tokens
+    // a key head's query heads side by side; where there is room, and a list of tiles, several tokens of a sequence
     const int group = nq / nkv, heads_a_tile = group < 16 ? group : 16;
-    const int tokens_a_tile = T > n_seqs ? 16 / heads_a_tile : 1;
+    HB_REQUIRE(!tiles || (n_tiles > 0 && n_tiles <= T && tokens_a_tile == 16 / heads_a_tile && (uintptr_t)tiles % 8 == 0),
+               "attention: a list of %d tiles of %d tokens for %d tokens and groups of %d heads", n_tiles, tokens_a_tile, T, group);
     const int tiles_a_head = (group + heads_a_tile - 1) / heads_a_tile;
     HB_REQUIRE((long long)nkv * tiles_a_head <= 65535, "attention: too many heads for the grid");
-    const dim3 grid((T + tokens_a_tile - 1) / tokens_a_tile, nkv * tiles_a_head);
+    const dim3 grid(tiles ? n_tiles : T, nkv * tiles_a_head);
     const int size = dtype == HB_F32 ? 4 : 2;
     const bool vec = hd % 4 == 0 && page_size % CHUNK == 0 && (uintptr_t)k_cache % (4 * size) == 0 && (uintptr_t)v_cache % (4 * size) == 0;
 #define HB_ATTENTION(TT, TO, NB, VEC)                                                                                 \
     attention_plain_kernel<TT, TO, NB, VEC, (NB <= 2 && VEC)><<<grid, 256, 0, stream>>>(                                                \
         (const TT*)q, (const TT*)k_cache, (const TT*)v_cache, (TO*)out, positions, seq_of, slots, page_table, max_pages, \
-        page_size, T, nq, nkv, hd, scale, window, sinks, chunk, softcap, bias, bias_ld, bias_at, bias_len, keep_first, \
-        heads_a_tile, tokens_a_tile)
+        page_size, nq, nkv, hd, scale, window, sinks, chunk, softcap, bias, bias_ld, bias_at, bias_len, keep_first,    \
+        heads_a_tile, (const int2*)tiles)
 #define HB_ATTENTION_OF(TT, TO)                                                                                       \
     do {                                                                                                              \
         if (!vec && hd <= 64) HB_ATTENTION(TT, TO, 1, false);                                                         \

@@ -80,7 +80,7 @@ SIGNATURES = {
         "hb_grouped_mfma": [_P, _I, _SZ, _P, _I, _I, _P, _I, _SZ, _I, _P, _I, _P, _P, _P, _I, _I, _I, _F, _F, _F, _I, _P],
     },
     "attention_plain": {
-        "hb_attention_plain": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I, _P, _I, _F, _P, _I, _I, _I, _I,
+        "hb_attention_plain": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _P, _I, _I, _I, _I, _I, _F, _I, _P, _I, _F, _P, _I, _I, _I, _I,
                                _I, _P],
     },
     "sampling": {

@@ -11,9 +11,11 @@ append, attention, residual sums), several of them to a kernel here.
 """
 import threading
 
+import numpy as np
 import torch
 
 from ..errors import BackendError
+from ..hosted import send
 from . import lib
 
 F32 = 0
@@ -205,6 +207,25 @@ class DistanceBias:
         _check(self.rows, "distance bias", torch.float32, (heads, self.FRONT + self.length + self.BACK))
 
 
+def token_tiles(starts, context, most):
+    """Cut each sequence's tokens of a step into tiles of at most `most`: (first packed token, tokens), those with the
+    longest contexts first. starts: the first packed row of each sequence and the last one's end; context: the positions it
+    holds after the step."""
+    tiles = []
+    for a, end, held in zip(starts[:-1], starts[1:], context):
+        tiles += [(int(held) - int(end) + i, int(i), min(most, int(end) - i)) for i in range(int(a), int(end), most)]
+    return [(first, n) for _, first, n in sorted(tiles, reverse=True)]
+
+
+def _token_tiles(meta, most):
+    key = ("token_tiles", most)
+    tiles = meta.derived.get(key)
+    if tiles is None:
+        packed = np.array(token_tiles(meta.host_starts, meta.host_context, most), dtype=np.int32)
+        tiles = meta.derived[key] = send(packed, meta.positions.device)
+    return tiles
+
+
 def attention_plain(q, meta, cache, out, nq, nkv, hd, scale, window, sinks=None, chunk=None, softcap=None, bias=None,
                     keep_first=0):
     """Causal (and windowed) attention of every token over its slot's pages. sinks f32 [nq]: the softmax's
@@ -222,10 +243,13 @@ def attention_plain(q, meta, cache, out, nq, nkv, hd, scale, window, sinks=None,
     _check_paged(meta, cache, T)
     if tuple(cache.k.shape[1:]) != (nkv, cache.page_size, hd):
         raise BackendError(f"cache pages {list(cache.k.shape)} do not fit {nkv} kv heads of {hd}")
+    # (several tokens of a sequence share a workgroup; of several sequences they would walk their contexts one after another)
+    most = 16 // min(16, nq // nkv) if nkv > 0 and nq % nkv == 0 else 1
+    tiles = _token_tiles(meta, most) if most > 1 and T > meta.slots.shape[0] else None
     lib.call("attention_plain", "hb_attention_plain", q.data_ptr(), cache.k.data_ptr(),
              cache.v.data_ptr(), out.data_ptr(), dtype_code(q), meta.positions.data_ptr(),
              meta.seq_of.data_ptr(), meta.slots.data_ptr(), cache.page_table.data_ptr(),
-             cache.page_table.shape[1], cache.page_size, T, meta.slots.shape[0], nq, nkv, hd, float(scale),
+             cache.page_table.shape[1], cache.page_size, T, _ptr(tiles), 0 if tiles is None else len(tiles), most, nq, nkv, hd, float(scale),
              int(window or 0), _ptr(sinks), int(chunk or 0), float(softcap or 0.0),
              None if bias is None else bias.rows.data_ptr(), 0 if bias is None else bias.rows.shape[1],
              0 if bias is None else bias.at, 0 if bias is None else bias.length, int(keep_first or 0), dtype_code(out), _stream())
