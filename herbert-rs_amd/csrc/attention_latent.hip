@@ -395,10 +395,10 @@ latent_attention_mfma_kernel(const float* __restrict__ q_full, const bf16* __res
 // in the scores (the halves meet in LDS, added in one order by both) and half of the rank in the sums, so that the
 // query's two bfloat16 halves (72 registers) and the sums (64) of a wave fit beside a second wave on its SIMD. Operands,
 // halves and order of keys are latent_attention_mfma_kernel's; the softmax runs in powers of two, and its reference moves
-// only where a weight would pass 2^LP_SLACK. A chunk that a row does not see leaves it as it was; keys behind the last
-// that a row sees are zeros.
-// 2,048 tokens of 16 heads, 512 + 64, take 282 us (a wave a token's 16 heads, keys from the L2s and V transposed by every
-// wave: 958), three prompts of 840 to 1,400 tokens 302 (1,086). Bound by the phases of a chunk (8,500 cycles), which the
+// only where a weight would pass 2^LP_SLACK. A chunk that a row does not see leaves it as it was, also where its numbers are
+// not finite; keys behind the last that a row sees are zeros.
+// 2,048 tokens of 16 heads, 512 + 64, take 286 us (a wave a token's 16 heads, keys from the L2s and V transposed by every
+// wave: 974), three prompts of 840 to 1,400 tokens 324 (829). Bound by the phases of a chunk (8,500 cycles), which the
 // barriers keep apart: LDS is busy for 3,700 of them (1,800 are writes that meet in a bank), the matrix cores for 2,200,
 // the vector units for 1,900.
 #define LP_ROWS 64
@@ -416,6 +416,7 @@ latent_attention_prompt_kernel(const float* __restrict__ q_full, const bf16* __r
     __shared__ __attribute__((aligned(16))) uint4 keys[2][2][KSW][HB_WAVE];         // [block of 16 keys][half][32 numbers]
     __shared__ __attribute__((aligned(16))) uint4 Vt[2][2][RBW][HB_WAVE];           // [buffer][half][16 numbers], 32 keys
     __shared__ __attribute__((aligned(16))) la_f32x4 halves[8][2][HB_WAVE];
+    __shared__ __attribute__((aligned(16))) int lost_from[32 * RBW];                // [number]: the key from which on it is not finite
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int n = lane & 15, g = lane >> 4, half = wave & 1;
     const int kd = rank + rot, KS = kd / 32, vsteps = rank / 8;
@@ -427,6 +428,7 @@ latent_attention_prompt_kernel(const float* __restrict__ q_full, const bf16* __r
     const bool mine = in_seq < rows;
     const int t = begin + (mine ? in_seq : rows - 1) / H, h = (mine ? in_seq : rows - 1) % H;
     const int sees = mine ? positions[t] : -1;                              // the last key that this lane's row sees
+    const int pos_first = positions[begin + tile * LP_ROWS / H];
     const int pos_last = positions[begin + min(tile * LP_ROWS + LP_ROWS - 1, rows - 1) / H];
     const int* pt = page_table + (size_t)slots[seq] * max_pages;
     const int n_chunks = pos_last / LA_CHUNK + 1;
@@ -435,6 +437,7 @@ latent_attention_prompt_kernel(const float* __restrict__ q_full, const bf16* __r
     const int ks0 = half ? ks_a : 0, ks_n = half ? KS - ks_a : ks_a;
     const int db0 = half ? db_a : 0, db_n = half ? rank / 16 - db_a : db_a;
     for (int i = tid; i < 4 * KSW * HB_WAVE; i += 512) (&keys[0][0][0][0])[i] = uint4{0, 0, 0, 0};
+    for (int i = tid; i < 32 * RBW; i += 512) lost_from[i] = 0x7fffffff;
 
     la_bf16x8 qh[KSW], ql[KSW];
     {
@@ -479,11 +482,34 @@ latent_attention_prompt_kernel(const float* __restrict__ q_full, const bf16* __r
         const int ks = segment / 4, of = ks >= ks_a, in = ks - (of ? ks_a : 0);
         keys[key >> 4][of][in][16 * (segment & 3) + ((key + 4 * (in & 3)) & 15)] = v;
     };
-    auto stash = [&](int buf) {
+    auto stash = [&](int c, int buf) {
         if (kg < 8) {
             // eight numbers of a key: step x / 4 of the scores, lane row x % 4
 #pragma unroll
             for (int i = 0; i < 4; ++i) put_key(4 * kg + i, x, lat[i]);
+            // a number without a finite size of a key that not every row sees: a weight of zero does not hide it from those that do
+            // not, so it stays out of the sums, and the rows that see it lose this number at the end
+            if (c * LA_CHUNK + LA_CHUNK - 1 > pos_first) {
+                unsigned wild = 0;                                    // (an exponent of all ones carries into the sign's place)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const unsigned any = ((lat[i].x & 0x7f807f80u) + 0x00800080u) | ((lat[i].y & 0x7f807f80u) + 0x00800080u) |
+                                         ((lat[i].z & 0x7f807f80u) + 0x00800080u) | ((lat[i].w & 0x7f807f80u) + 0x00800080u);
+                    if (c * LA_CHUNK + 4 * kg + i > pos_first) wild |= any & 0x80008000u;
+                }
+                if (wild)
+                    for (int i = 0; i < 4; ++i) {
+                        const int key = c * LA_CHUNK + 4 * kg + i;
+                        unsigned* pair = i == 0 ? (unsigned*)&lat[0] : i == 1 ? (unsigned*)&lat[1] : i == 2 ? (unsigned*)&lat[2] : (unsigned*)&lat[3];
+                        for (int e = 0; e < 8 && key > pos_first; ++e) {
+                            const unsigned half_of = e & 1 ? 0xffff0000u : 0xffffu;
+                            if ((~pair[e / 2] & 0x7f807f80u & half_of) == 0) {
+                                atomicMin(&lost_from[8 * x + e], key);
+                                pair[e / 2] &= ~half_of;
+                            }
+                        }
+                    }
+            }
             // keys 16 kb + 4 g' + i lie at g' 8 + kb 4 + i, the order in which a lane holds their weights
             const unsigned *a = (const unsigned*)&lat[0], *b = (const unsigned*)&lat[1], *c = (const unsigned*)&lat[2], *d = (const unsigned*)&lat[3];
             const int block = x / 2, of = block >= db_a, in = block - (of ? db_a : 0);
@@ -500,7 +526,7 @@ latent_attention_prompt_kernel(const float* __restrict__ q_full, const bf16* __r
     int page_next = pt[LA_CHUNK / page_size < max_pages ? LA_CHUNK / page_size : 0];
     fetch(0, pt[0]);
     __syncthreads();                                                 // (the zeros of the keys' unused steps are there)
-    stash(0);
+    stash(0, 0);
     __syncthreads();
     for (int c = 0, buf = 0; c < n_chunks; ++c, buf ^= 1) {
         if (c + 1 < n_chunks) {
@@ -540,9 +566,10 @@ latent_attention_prompt_kernel(const float* __restrict__ q_full, const bf16* __r
                            fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
         cmax = fmaxf(cmax, __shfl_xor(cmax, 16, HB_WAVE));
         cmax = fmaxf(cmax, __shfl_xor(cmax, 32, HB_WAVE));
-        // (the sums are brought to another reference only where a weight would pass 2^LP_SLACK)
+        // (a row's sums are brought to another reference only where a weight would pass 2^LP_SLACK: by its own weights, so
+        //  that nothing of it depends on the rows beside it)
         if (__any(cmax > m + LP_SLACK)) {
-            const float m_new = fmaxf(m, cmax);
+            const float m_new = cmax > m + LP_SLACK ? cmax : m;
             const float corr = m == m_new ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);
             l *= corr;
             m = m_new;
@@ -576,7 +603,7 @@ latent_attention_prompt_kernel(const float* __restrict__ q_full, const bf16* __r
 #pragma unroll
             for (int i = 0; i < 2; ++i) acc[db + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[i], pl, acc[db + i], 0, 0, 0);
         }
-        if (c + 1 < n_chunks) stash(buf ^ 1);
+        if (c + 1 < n_chunks) stash(c + 1, buf ^ 1);
         __syncthreads();
     }
     l += __shfl_xor(l, 16, HB_WAVE);
@@ -591,7 +618,8 @@ latent_attention_prompt_kernel(const float* __restrict__ q_full, const bf16* __r
             // acc[db][i]: number 16 (db0 + db) + 4 g + i of row n's sum
             bf16 o[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) o[i] = hb_from_float<bf16>(acc[db][i] * w);
+            for (int i = 0; i < 4; ++i)
+                o[i] = hb_from_float<bf16>(lost_from[16 * (db0 + db) + 4 * g + i] > sees ? acc[db][i] * w : NAN);
             *(uint2*)(out + ((size_t)t * H + h) * rank + 16 * (db0 + db) + 4 * g) =
                 uint2{o[0].bits | ((unsigned)o[1].bits << 16), o[2].bits | ((unsigned)o[3].bits << 16)};
         }

@@ -290,6 +290,16 @@ def test_prompt_tokens_share_their_keys(H, rank, rot):
             err = (out[at + t].cpu().double().view(H, rank) - want).abs().max()
             assert float(err) <= 2.0 ** -8 * float(want.abs().max()) + 1e-3, (n, t)
         at += k
+    # a later token's key without finite numbers, and one that is only larger: the tokens before it are the same bits; those
+    # that see it lose at least the numbers that are not finite
+    late, table = 140, kv.page_table[slots[0]].cpu().tolist()
+    for what in (float("inf"), float("nan"), 40.0):
+        kv.k[table[late // 64], 0, late % 64, 7:9] = what
+        again = torch.empty_like(out)
+        latent.latent_attention_mfma(q.to(DEV), meta, kv, again, gate.to(DEV), 0, H, rank, rot, row ** -0.5, None, sinks=sinks.to(DEV))
+        assert torch.equal(again[:late], out[:late]) and torch.equal(again[150:], out[150:])
+        if what != 40.0:
+            assert not again[late:150].view(10, H, rank)[:, :, 7:9].isfinite().any()
 
 
 @pytest.mark.parametrize("M", [1, 16, 17, 64, 65, 200, 700])
