@@ -894,10 +894,11 @@ extern "C" int hb_grouped_mfma(const void* A, int lda, size_t a_group_off, const
 #undef HB_GROUPED_STREAM
     const int quads = ldc % 4 == 0 && c_group_off % 4 == 0 && (uintptr_t)C % 16 == 0;
     const long long runs = (long long)((tiles + TILE_RUN - 1) / TILE_RUN) * grid.x;
-    HB_REQUIRE(runs < (1ll << 26), "grouped product: %lld runs of tiles exceed the grid", runs);
-    const unsigned blocks = (unsigned)((runs + XCDS - 1) / XCDS * XCDS * TILE_RUN);
+    const long long blocks = (runs + XCDS - 1) / XCDS * XCDS * TILE_RUN;
+    // (a grid's x holds fewer than 2^32 threads: 65,535 tiles of 255 blocks of columns, whose sums no card holds)
+    HB_REQUIRE(blocks < (1ll << 24), "grouped product: %d tiles of %d columns exceed the grid", tiles, out_cols);
 #define HB_GROUPED(E)                                                                                               \
-    grouped_mfma_kernel<E><<<blocks, 256, 0, stream>>>((const bf16*)A, lda, a_group_off, (const bf16*)W, N, K, C, ldc, \
+    grouped_mfma_kernel<E><<<(unsigned)blocks, 256, 0, stream>>>((const bf16*)A, lda, a_group_off, (const bf16*)W, N, K, C, ldc, \
                                                        c_group_off, order, top, tile_group, tile_row0, tile_rows, M, \
                                                        m_tiles, limit, alpha, shift, tiles, (int)grid.x, quads)
     if (epi == 0) HB_GROUPED(0);
