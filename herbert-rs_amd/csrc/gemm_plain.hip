@@ -83,8 +83,9 @@ gemm_plain_tile_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
     __shared__ __attribute__((aligned(16))) float As[2][BM * LD], Ws[2][BN * LD];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r = lane & 15, q = lane >> 4;
-    const int across = (N + BN - 1) / BN;                            // tiles of a row of tiles
-    const int m0 = (int)(blockIdx.x / across) * BM, n0 = (int)(blockIdx.x % across) * BN;
+    const unsigned across = (N + BN - 1) / BN, tile = blockIdx.y * gridDim.x + blockIdx.x;   // (tiles of a row of tiles)
+    if (tile / across >= (unsigned)(M + BM - 1) / BM) return;
+    const int m0 = (int)(tile / across) * BM, n0 = (int)(tile % across) * BN;
     const int wm = (wave & 1) * (BM / 2), wn = (wave >> 1) * (BN / 2);
 
     f32x4 a_next[QA], w_next[QW];
@@ -209,6 +210,13 @@ gemm_plain_wave_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
 // 16 k take the wave kernel. Beyond, the largest tile that still fills the chip: 128 x 128 from two tiles for every CU on
 // (4096 x 4096 x 4096: 1,082 us; 64 x 64 1,281), 64 x 64 from two of those for every CU on (1200 x 4096 x 4096: 414;
 // 32 x 32 444, 128 x 128 539), else 32 x 32 (200 x 2048 x 2048: 30; 64 x 64 51; 564 x 2048 x 2048: 67; 64 x 64 84).
+#define GRID_X (1 << 23)
+// What the entries take: rows as ever, and tiles of 32 x 32 that GRID_X times 256 hold (2 T sums a product).
+#define HB_REQUIRE_TILES(M, N)                                                                                        \
+    do {                                                                                                              \
+        HB_REQUIRE((M) <= 65535 * 64, "gemm: M=%d, at most 4194240 rows are taken", M);                               \
+        HB_REQUIRE((((M) + 31) / 32) * (((N) + 31ll) / 32) < (1ll << 31), "gemm: %d x %d sums exceed the grid", M, N); \
+    } while (0)
 template <class TA, class TW, class TC, bool ACCUM>
 static void launch_as(const TA* A, const TW* W, TC* C, int M, int N, int K, int lda, int ldw, int ldc,
                       hipStream_t stream, int batch, size_t batch_a, size_t batch_w, size_t batch_c, DecayEpilogue ep) {
@@ -216,10 +224,14 @@ static void launch_as(const TA* A, const TW* W, TC* C, int M, int N, int K, int 
                      (uintptr_t)A % (4 * sizeof(TA)) == 0 && (uintptr_t)W % (4 * sizeof(TW)) == 0 &&
                      (sizeof(TC) != 4 || (N % 4 == 0 && ldc % 4 == 0 && batch_c % 4 == 0 && (uintptr_t)C % 16 == 0));
     auto tiles = [&](int side) { return (long long)((N + side - 1) / side) * ((M + side - 1) / side) * batch; };
+    // (a grid's x holds fewer than 2^32 threads: beyond GRID_X tiles the rest lie along its y)
+    auto grid = [&](int side) {
+        const long long n = tiles(side) / batch, x = n < GRID_X ? n : GRID_X;
+        return dim3((unsigned)x, (unsigned)((n + x - 1) / x), batch);
+    };
 #define HB_PLAIN_TILE(BM, BK, VEC)                                                                                    \
     gemm_plain_tile_kernel<TA, TW, TC, ACCUM, BM, BM, BK, VEC>                                                        \
-        <<<dim3((unsigned)(tiles(BM) / batch), 1, batch), 256, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, batch_a, \
-                                                                            batch_w, batch_c, ep)
+        <<<grid(BM), 256, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, batch_a, batch_w, batch_c, ep)
     if (vec && M <= WAVE_ROWS && K % 16 == 0)
         gemm_plain_wave_kernel<TA, TW, TC, ACCUM><<<dim3((N + 15) / 16, 1, batch), HB_WAVE, 0, stream>>>(
             A, W, C, M, N, K, lda, ldw, ldc, batch_a, batch_w, batch_c, ep);
@@ -328,7 +340,7 @@ extern "C" int hb_gemm_plain(const void* A, int a_dtype, const void* W, int w_dt
                              hipStream_t stream) {
     HB_REQUIRE(M > 0 && N > 0 && K > 0, "gemm: empty problem (M=%d, N=%d, K=%d)", M, N, K);
     HB_REQUIRE(lda >= K && ldw >= K && ldc >= N, "gemm: a row stride is smaller than its row");
-    HB_REQUIRE((M + 63) / 64 <= 65535, "gemm: M=%d exceeds the grid", M);
+    HB_REQUIRE_TILES(M, N);
     const int key = a_dtype * 4 + w_dtype * 2 + c_dtype;
     switch (key) {
         case 0: launch<float, float, float>(A, W, C, M, N, K, lda, ldw, ldc, accumulate, stream); break;
@@ -366,7 +378,7 @@ extern "C" int hb_gemm_plain_short_k(const void* A, int a_dtype, const void* W, 
         return 0;
     }
     if (!A_log) return hb_gemm_plain(A, a_dtype, W, w_dtype, C, c_dtype, M, N, K, lda, ldw, ldc, accumulate, stream);
-    HB_REQUIRE((M + 63) / 64 <= 65535, "gemm: M=%d exceeds the grid", M);
+    HB_REQUIRE_TILES(M, N);
     switch (a_dtype * 2 + w_dtype) {
         case 0: launch<float, float, float>(A, W, C, M, N, K, lda, ldw, ldc, 0, stream, 1, 0, 0, 0, ep); break;
         case 1: launch<float, bf16, float>(A, W, C, M, N, K, lda, ldw, ldc, 0, stream, 1, 0, 0, 0, ep); break;
@@ -386,7 +398,8 @@ extern "C" int hb_gemm_plain_batched(const void* A, int a_dtype, const void* W, 
                                      size_t batch_w, size_t batch_c, hipStream_t stream) {
     HB_REQUIRE(M > 0 && N > 0 && K > 0 && batch > 0, "gemm: empty problem (M=%d, N=%d, K=%d, batch=%d)", M, N, K, batch);
     HB_REQUIRE(lda >= K && ldw >= K && ldc >= N, "gemm: a row stride is smaller than its row");
-    HB_REQUIRE((M + 63) / 64 <= 65535 && batch <= 65535, "gemm: M=%d or batch=%d exceeds the grid", M, batch);
+    HB_REQUIRE(batch <= 65535, "gemm: batch=%d exceeds the grid", batch);
+    HB_REQUIRE_TILES(M, N);
     // few rows (one token a sequence) with a short k: the kernel made for them, a product of the batch a grid's layer
     if (few_rows_takes(A, a_dtype, W, w_dtype, c_dtype, M, K, lda, ldw, 0) && batch_a % 4 == 0 && batch_w % 8 == 0) {
         gemm_few_rows_kernel<<<dim3((N + 15) / 16, (M + FEW_ROWS_M - 1) / FEW_ROWS_M, batch), HB_WAVE, 0, stream>>>(

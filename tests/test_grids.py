@@ -15,3 +15,9 @@ def grouped(M, groups, N):
 def test_a_grouped_product_whose_tiles_exceed_the_grid_is_refused(M, groups, N):
     with pytest.raises(BackendError, match="exceed the grid"):
         grouped(M, groups, N)
+
+
+@pytest.mark.parametrize("M, N, text", [(4194241, 16, "at most 4194240 rows"), (4194240, 1 << 20, "exceed the grid")])
+def test_a_product_beyond_the_rows_or_the_grid_is_refused(M, N, text):
+    with pytest.raises(BackendError, match=text):
+        lib.call("gemm_plain", "hb_gemm_plain", None, 0, None, 0, None, 0, M, N, 1, 1, 1, N, 0, None)

@@ -66,6 +66,20 @@ def test_gemm_plain(M, N, K, dts):
     assert torch.allclose(cb.float(), want, rtol=2 ** -8, atol=1e-3)
 
 
+def test_gemm_plain_of_more_tiles_than_a_grids_x_holds():
+    """The most rows that are taken, of a width whose tiles of 32 x 32 times 256 threads pass 2^32: whole numbers, so every
+    sum is exact in bfloat16."""
+    from herbert_rs_amd.kernels import ops
+    M, N, K = 65535 * 64, 4097, 3
+    g = torch.Generator(device=dev()).manual_seed(3)
+    a = torch.randint(-3, 4, (M, K), generator=g, device=dev()).float()
+    w = torch.randint(-3, 4, (N, K), generator=g, device=dev()).float()
+    c = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=dev())
+    ops.gemm_plain(a, w, c)
+    for at in range(0, M, 65535):
+        assert torch.equal(c[at:at + 65535], (a[at:at + 65535] @ w.t()).bfloat16()), at
+
+
 @pytest.mark.parametrize("K", [16, 144, 2048, 100, 31])            # whole blocks of 16 k, part of one, no whole quad
 @pytest.mark.parametrize("wd", [torch.float32, torch.bfloat16])
 def test_gemm_plain_sums_do_not_depend_on_the_rows(K, wd):
