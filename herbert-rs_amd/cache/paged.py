@@ -91,7 +91,7 @@ class KVGroup:
                 taken.append((slot * self.pages_per_slot + p, row[p]))
             self.held_end[slot] = last
         if taken:
-            # one copy and one kernel a step, behind what the stream holds
+            # one copy and two kernels a step (the pages' numbers to int32, and to their places), behind what the stream holds
             places, pages = send(np.array(taken, dtype=np.int64).T, self.table.device)
             self.table.view(-1).index_copy_(0, places, pages.to(torch.int32))
 
@@ -171,7 +171,7 @@ class Cache:
         self.pad_slot = self.n_slots        # never handed out: where a step's padding rows write and read
         self.slots = FreeList(self.n_slots, "slot")
         self.lengths = np.zeros(self.n_slots, dtype=np.int64)
-        self._saved_slots = (None, None)    # the slots that save_state was last asked for, and their numbers on the GPU
+        self._saved_slots = (None, None)    # the slots that save_state was last asked for and the stream, and their numbers on the GPU
         self.kv_groups = {}
         self.state_groups = {}
         self._kv_of = {}
@@ -273,10 +273,13 @@ class Cache:
         `restore_state` puts back when the step that was to change it has failed."""
         if not self.state_groups:
             return None
-        key = tuple(sorted(set(int(s) for s in slots)))
-        if self._saved_slots[0] != key:           # (decode steps name the same slots again and again)
-            device = next(iter(self.state_groups.values())).data.device
-            self._saved_slots = (key, send(np.array(key, dtype=np.int64), device))
+        index = sorted(set(int(s) for s in slots))
+        device = next(iter(self.state_groups.values())).data.device
+        # (decode steps name the same slots again and again. Their numbers serve the stream that they were sent on: another one
+        #  neither waits for the copy, nor does their memory, once replaced, wait for what another one still reads)
+        key = (index, torch.cuda.current_stream(device).cuda_stream if device.type == "cuda" else None)
+        if self._saved_slots[0] != key:
+            self._saved_slots = (key, send(np.array(index, dtype=np.int64), device))
         at = self._saved_slots[1]
         return [(g, at, g.data.index_select(1, at)) for g in self.state_groups.values()]
 

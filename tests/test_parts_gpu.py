@@ -884,3 +884,22 @@ def plain_layer_of(w, p, x, positions, inter):
     x = x + plain_mixer(w, p, pops.rms_norm(x, w[p + "n1"], 1e-6), positions)
     y = pops.rms_norm(x, w[p + "n2"], 1e-6)
     return x + pops.swiglu_mlp(y, w[p + "g"], w[p + "u"], w[p + "d"]), None
+
+
+def test_state_set_aside_on_another_stream_has_its_own_list_of_slots():
+    """The slots' numbers are sent on the current stream, which alone is known to be behind the copy."""
+    cache = Cache({0: StateNeed((8,), torch.float32)}, 64 * 4, 256, torch.float32, DEV, max_slots=4)
+    group = next(iter(cache.state_groups.values()))
+    group.data.normal_()
+    kept = group.data.clone()
+    here = cache.save_state([2, 1])
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.Stream()):
+        there = cache.save_state([1, 2])
+        assert there[0][1] is not here[0][1] and cache.save_state([1, 2])[0][1] is there[0][1]
+        group.data.zero_()
+        cache.restore_state(there)
+    torch.cuda.synchronize()
+    for saved in (here, there):
+        assert saved[0][1].tolist() == [1, 2] and torch.equal(saved[0][2], kept[:, 1:3])
+    assert torch.equal(group.data[:, 1:3], kept[:, 1:3]) and not group.data[:, 3].any()
