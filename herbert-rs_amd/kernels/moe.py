@@ -127,7 +127,11 @@ def combine(y, routing, x, shared=None, gate=None, identity=None):
 
 
 EPI_F32, EPI_BF16, EPI_GLU = 0, 1, 2
-FEW_ROWS = 16      # up to so many rows a group the kernel without a stage in LDS runs (decoding)
+# Up to so many rows a group the kernel without a stage in LDS runs (decoding). Microseconds of an expert layer's two products
+# by it / by the tiles: 32 experts of 768 on 2,048: 8 rows an expert 62 / 76, 16 rows 75 / 78, 20 rows 80 / 79, 32 rows 94 / 80,
+# where the line lies; 64 of 1,536 on 4,096: 8 rows 404 / 415, 12 rows 429 / 418, 16 rows 465 / 421; 16 of 512 on 1,024: 16 rows
+# 19 / 32, 64 rows 32 / 37. A head's product of rows that all heads share, 16 of 512 x 128: 16 rows 4.4 / 5.4, 64 rows 5.4 / 8.0.
+FEW_ROWS = 16
 
 
 def mfma_takes(K, lda, a_group_off=0, N=16):
