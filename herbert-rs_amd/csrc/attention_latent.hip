@@ -9,6 +9,7 @@
 // Pages: row of position p of a slot at page_table[slot * max_pages + p / page_size], pages
 // [page, page_size, rank + rot].
 #include "common.h"
+#include "lds_read.h"
 #include <math.h>
 
 HB_MODULE_ERROR_SLOT()
@@ -30,8 +31,8 @@ __device__ __forceinline__ void rotate_pair(float a, float b, float angle, float
 // [T, rank + rot] float32: the first `rank` RMS-normed with norm_w -> the row's c; the last `rot`
 // rotated (the first rot_dims of them: entry i with i + rot_dims / 2, angle pos * inv_freq[i]; the rest
 // unchanged) -> the row's r. q [T, H, qd + rot] float32: every head's last `rot` rotated the same way
-// into q_full[t, h, rank ...] (q_full [T, H, rank + rot] float32; its first `rank` are written by the
-// product with W_uk^T). One block a token.
+// into q_full[t, h, q_at ...] (q_full [T, H, q_row] float32: rows of rank + rot, whose first `rank` are written by the
+// product with W_uk^T, or of `rot` alone). One block a token.
 // Queries that come from a latent of their own are not there yet when the cache's row is written: the kernel then
 // runs twice, first with H = 0 and down's neighbour columns q_down [T, q_rank] (rows down_ld apart), which are
 // RMS-normed with q_norm_w into c_q [T, q_rank] (the product that makes the queries reads it), then for the queries alone.
@@ -43,7 +44,7 @@ __global__ void latent_write_kernel(const float* __restrict__ down, int down_ld,
                                     const int* __restrict__ page_table, int max_pages, int page_size,
                                     TC* __restrict__ pages, int H, int qd, int rank, int rot, int rot_dims,
                                     float eps, int write_cache, const float* __restrict__ q_down, int q_rank,
-                                    const float* __restrict__ q_norm_w, TC* __restrict__ c_q) {
+                                    const float* __restrict__ q_norm_w, TC* __restrict__ c_q, int q_row, int q_at) {
     __shared__ float red[16];
     const int t = blockIdx.x;
     const int pos = positions[t];
@@ -89,7 +90,7 @@ __global__ void latent_write_kernel(const float* __restrict__ down, int down_ld,
             rotate_pair(in[j], in[j + half], p * inv_freq[j], ra, rb);
             v = i < half ? ra : rb;
         }
-        q_full[((size_t)t * H + h) * (rank + rot) + rank + i] = v;
+        q_full[((size_t)t * H + h) * q_row + q_at + i] = v;
     }
     // the unrotated parts once more as bfloat16 [T, H, qd], for a matrix-core product with W_uk^T
     if (q_plain)
@@ -103,7 +104,9 @@ extern "C" int hb_latent_write(const float* down, int down_ld, const float* norm
                                void* q_plain, const float* inv_freq, const int* positions, const int* seq_of, const int* slots,
                                const int* page_table, int max_pages, int page_size, void* pages, int dtype, int T,
                                int H, int qd, int rank, int rot, int rot_dims, float eps, int write_cache,
-                               const float* q_down, int q_rank, const float* q_norm_w, void* c_q, hipStream_t stream) {
+                               const float* q_down, int q_rank, const float* q_norm_w, void* c_q, int q_row, int q_at,
+                               hipStream_t stream) {
+    HB_REQUIRE(H == 0 || (q_at >= 0 && q_row >= q_at + rot), "latent write: %d turned entries at %d of rows of %d", rot, q_at, q_row);
     HB_REQUIRE(!q_down || (q_rank > 0 && q_norm_w && c_q), "latent write: a query latent needs its norm and a place");
     HB_REQUIRE(T > 0 && (H > 0 || (H == 0 && (q_down || write_cache))) && rank > 0 && rot >= 0 && qd >= 0, "latent write: empty input");
     HB_REQUIRE(rot_dims >= 0 && rot_dims <= rot && rot_dims % 2 == 0, "latent write: %d rotated of %d", rot_dims, rot);
@@ -111,12 +114,12 @@ extern "C" int hb_latent_write(const float* down, int down_ld, const float* norm
         latent_write_kernel<float><<<T, 256, 0, stream>>>(down, down_ld, norm_w, q, q_ld, q_full, (bf16*)q_plain, inv_freq, positions, seq_of, slots,
                                                           page_table, max_pages, page_size, (float*)pages, H, qd,
                                                           rank, rot, rot_dims, eps, write_cache, q_down, q_rank, q_norm_w,
-                                                          (float*)c_q);
+                                                          (float*)c_q, q_row, q_at);
     else if (dtype == HB_BF16)
         latent_write_kernel<bf16><<<T, 256, 0, stream>>>(down, down_ld, norm_w, q, q_ld, q_full, (bf16*)q_plain, inv_freq, positions, seq_of, slots,
                                                          page_table, max_pages, page_size, (bf16*)pages, H, qd,
                                                          rank, rot, rot_dims, eps, write_cache, q_down, q_rank, q_norm_w,
-                                                          (bf16*)c_q);
+                                                          (bf16*)c_q, q_row, q_at);
     else
         HB_REQUIRE(false, "latent write: unknown dtype %d", dtype);
     HB_CHECK_LAUNCH("latent_write");
@@ -623,6 +626,418 @@ latent_attention_prompt_kernel(const float* __restrict__ q_full, const bf16* __r
             *(uint2*)(out + ((size_t)t * H + h) * rank + 16 * (db0 + db) + 4 * g) =
                 uint2{o[0].bits | ((unsigned)o[1].bits << 16), o[2].bits | ((unsigned)o[3].bits << 16)};
         }
+}
+
+// ------------------------------------------------ prompts with the heads' keys and values built
+// Where a sequence brings many tokens, building every head's keys and values once costs less than scoring on the
+// latents: a pair of query and key takes dim + rot + vdim products a head (320) in place of 2 rank + rot (1,088), and the
+// two products that take queries and sums through the heads' matrices go. Two kernels: the first leaves keys and values of all
+// positions that the step's sequences hold in scratch, in the order in which the second one's matrix products read them;
+// so these come into LDS by plain copies and go on to the products without a bank met twice. 2,048 tokens of 16 heads, 128 + 64 and 128
+// on 512: 67 us and 21 to build the heads (scoring on the latents 286, and 81 for the two products); three prompts of 1,054 to 1,400 tokens
+// 87 and 38 (396 and 79).
+// Scratch, in blocks of 32 keys (a sequence's tiles of 64 keys follow each other, the sequences too):
+//   keys [H][block][dim / 16][64 lanes][8]: lane = key + 32 * (d / 8 % 2), the shared rotated parts [block][rot / 16][64][8] alike;
+//   values [H][block][vdim / 32][2][64 lanes][8]: lane = v % 32 + 32 g, entry e of step s = key 16 s + 8 (e / 4) + 4 g + e % 4, the
+//   order in which a lane of the scores' product holds its weights. Keys behind a sequence's last are zeros.
+typedef float la_f32x16 __attribute__((ext_vector_type(16)));
+#define LH_TILE 64
+#define LH_RANK 512
+
+// The sequence of the step whose tiles hold tile `tile`, and how many tiles lie before that sequence's.
+__device__ __forceinline__ int lh_sequence_of(int tile, const int* context_lens, int n_seqs, int& before) {
+    const int lane = threadIdx.x & (HB_WAVE - 1);
+    before = 0;
+    for (int first = 0; first < n_seqs; first += HB_WAVE) {
+        int upto = first + lane < n_seqs ? (context_lens[first + lane] + LH_TILE - 1) / LH_TILE : 0;
+#pragma unroll
+        for (int off = 1; off < HB_WAVE; off <<= 1) {
+            const int v = __shfl_up(upto, off, HB_WAVE);
+            if (lane >= off) upto += v;
+        }
+        const unsigned long long beyond = __ballot(before + upto > tile);
+        if (beyond) {
+            const int at = __ffsll(beyond) - 1;
+            if (at) before += __shfl(upto, at - 1, HB_WAVE);
+            return first + at;
+        }
+        before += __shfl(upto, HB_WAVE - 1, HB_WAVE);
+    }
+    return -1;
+}
+
+// A workgroup: 64 keys of one head (dim = vdim); each of its four waves takes blocks of 32 of a key's and a value's numbers, one
+// of either at a time. The latents come into LDS (rows 16 bytes apart beyond their length, so that 16 rows' reads spread over the banks),
+// the matrices' operands straight from the L2s, a step ahead. K^T = W_uk c^T and V = c W_uv^T: what leaves is
+// what a lane holds.
+__global__ void __launch_bounds__(256)
+latent_heads_kernel(const bf16* __restrict__ pages, const bf16* __restrict__ w_uk, const bf16* __restrict__ w_uv,
+                    bf16* __restrict__ keys, bf16* __restrict__ turned, bf16* __restrict__ values,
+                    const int* __restrict__ context_lens, int n_seqs, const int* __restrict__ slots,
+                    const int* __restrict__ page_table, int max_pages, int page_size, int tiles, int dim, int rank,
+                    int rot) {
+    __shared__ __attribute__((aligned(16))) char lh_lds[LH_TILE * (LH_RANK * 2 + 16)];
+    const int tile = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int before;
+    const int seq = lh_sequence_of(tile, context_lens, n_seqs, before);
+    if (seq < 0) return;
+    const int key0 = (tile - before) * LH_TILE, held = context_lens[seq];
+    const int kd = rank + rot, octets = rank / 8, pitch = rank * 2 + 16;
+    // (a tile lies in one page)
+    const bf16* row0 = pages + ((size_t)page_table[(size_t)slots[seq] * max_pages + key0 / page_size] * page_size + key0 % page_size) * kd;
+    for (int i0 = tid; i0 < LH_TILE * octets; i0 += 8 * 256) {
+        uint4 v[8];                                            // (eight loads on their way at a time)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int i = i0 + 256 * u, key = i / octets;
+            v[u] = uint4{0, 0, 0, 0};
+            if (i < LH_TILE * octets && key0 + key < held) v[u] = *(const uint4*)(row0 + key * kd + 8 * (i % octets));
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int i = i0 + 256 * u;
+            if (i < LH_TILE * octets) *(uint4*)(lh_lds + i / octets * pitch + 16 * (i % octets)) = v[u];
+        }
+    }
+    if (h == 0)
+        for (int i = tid; i < LH_TILE * (rot / 8); i += 256) {
+            const int key = i / (rot / 8), o = i % (rot / 8);
+            uint4 v = uint4{0, 0, 0, 0};
+            if (key0 + key < held) v = *(const uint4*)(row0 + key * kd + rank + 8 * o);
+            ((uint4*)turned)[(((size_t)2 * tile + key / 32) * (rot / 16) + o / 2) * HB_WAVE + key % 32 + 32 * (o & 1)] = v;
+        }
+    __syncthreads();
+    const int n = lane & 31, g = lane >> 5, KT = rank / 32;
+    const char* c_at = lh_lds + n * pitch + 16 * g;
+    // operand of 32 rows x 16 k from packed blocks [k / 32][rows / 16][lane = 16 (k / 8 % 4) + row % 16][8]
+    const size_t w_step = (size_t)dim / 16 * HB_WAVE * 8;
+    for (int b = wave; b < dim / 32; b += 4) {
+        const size_t at = (size_t)h * dim * rank + ((size_t)(2 * b + (n >> 4)) * HB_WAVE + 16 * g + (n & 15)) * 8;
+        la_f32x16 kt[2], v[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) kt[j][e] = v[j][e] = 0.f;
+        // four steps of 32 k in flight (beyond the last: the last once more, which goes nowhere)
+        la_bf16x8 wk[4][2], wv[4][2];
+        auto load = [&](int to, int k) {
+            const size_t kk = at + min(k, KT - 1) * w_step;
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                wk[to][s] = *(const la_bf16x8*)(w_uk + kk + s * 32 * 8);
+                wv[to][s] = *(const la_bf16x8*)(w_uv + kk + s * 32 * 8);
+            }
+        };
+        auto use = [&](int from, int k) {
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const la_bf16x8 c = *(const la_bf16x8*)(c_at + 32 * j * pitch + 64 * k + 32 * s);
+                    kt[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wk[from][s], c, kt[j], 0, 0, 0);
+                    v[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c, wv[from][s], v[j], 0, 0, 0);
+                }
+        };
+#pragma unroll
+        for (int u = 0; u < 4; ++u) load(u, u);
+        int k = 0;
+        for (; k + 4 <= KT; k += 4) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                __builtin_amdgcn_sched_barrier(0);
+                use(u, k + u);
+                load(u, k + 4 + u);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 3; ++u)
+            if (k + u < KT) use(u, k + u);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const size_t block = ((size_t)h * tiles + tile) * 2 + j;
+            // kt[j][4 a + c]: number 32 b + 8 a + 4 g + c of key 32 j + n
+            bf16* to = keys + (block * (dim / 16) + 2 * b) * HB_WAVE * 8;
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                bf16 o[4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) o[c] = hb_from_float<bf16>(kt[j][4 * a + c]);
+                *(uint2*)(to + ((a >> 1) * HB_WAVE + n + 32 * (a & 1)) * 8 + 4 * g) =
+                    uint2{o[0].bits | ((unsigned)o[1].bits << 16), o[2].bits | ((unsigned)o[3].bits << 16)};
+            }
+            // v[j][e]: key 32 j + 8 (e / 4) + 4 g + e % 4, number 32 b + n
+            to = values + (block * (dim / 32) + b) * 2 * HB_WAVE * 8;
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                bf16 o[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) o[e] = hb_from_float<bf16>(v[j][8 * s + e]);
+                *(uint4*)(to + (s * HB_WAVE + lane) * 8) =
+                    uint4{o[0].bits | ((unsigned)o[1].bits << 16), o[2].bits | ((unsigned)o[3].bits << 16),
+                          o[4].bits | ((unsigned)o[5].bits << 16), o[6].bits | ((unsigned)o[7].bits << 16)};
+            }
+        }
+    }
+}
+
+// A workgroup: 64 queries of one head and sequence, four waves: two groups of 32 queries (a lane's column) x the two blocks of a
+// tile of 64 keys, so that the longest row's chain is half its keys; the two blocks' sums meet at the end. The query (times the
+// scale) is two bfloat16 halves and so are the weights, as in the kernels above; the reference of the
+// exponents moves as in latent_attention_prompt_kernel. A tile's keys come in while the tile before is worked on, its values while its scores
+// are: two barriers a tile, 64 KB of LDS, two workgroups a CU. Bound by a tile's chain in a wave (scores, exponentials, sums: 1.7 us,
+// 0.55 of it the matrix cores'), which two waves a SIMD only partly cover. The tiles with the most keys start first, those with the fewest
+// follow, so that a CU that takes two of them gets one of either kind.
+template <int DS, int RS, int VB>
+__global__ void __launch_bounds__(256, 2)
+latent_attention_heads_kernel(const float* __restrict__ q, size_t q_ld, const float* __restrict__ q_turned,
+                              const bf16* __restrict__ keys, const bf16* __restrict__ turned,
+                              const bf16* __restrict__ values, bf16* __restrict__ out, const float* __restrict__ gate,
+                              int gate_ld, const int* __restrict__ positions, const int* __restrict__ seq_starts,
+                              const int* __restrict__ context_lens, int n_seqs, int tiles, int H, float scale,
+                              const float* __restrict__ sinks) {
+    constexpr int KS = DS + RS, DIM = 16 * DS, ROT = 16 * RS, VD = 32 * VB;
+    constexpr int AHEAD = 3;                                               // reads of LDS ahead of their products
+    constexpr int K_LOADS = 2 * KS / 4, V_LOADS = VB;                      // a wave's share of a tile, in kilobytes
+    static_assert(2 * KS % 4 == 0, "a tile's keys are dealt out to four waves");
+    __shared__ __attribute__((aligned(16))) uint4 K[2][2][KS][HB_WAVE];
+    __shared__ __attribute__((aligned(16))) uint4 V[2][VB][2][HB_WAVE];
+    __shared__ float met[2][2][32];                                        // the other block's reference and sum of a row
+    __shared__ int lost_from[VD];                                          // [number]: the key from which on it is not finite
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 31, g = lane >> 5, group = wave & 1, block = wave >> 1;
+    const int seq = blockIdx.y, h = blockIdx.x % H, nth = blockIdx.x / H, most = gridDim.x / H;
+    const int tile = nth < (most + 1) / 2 ? most - 1 - nth : nth - (most + 1) / 2;
+    const int begin = seq_starts[seq], rows = seq_starts[seq + 1] - begin;
+    if (tile * 64 >= rows) return;
+    int before = 0;
+    for (int s = lane; s < seq; s += HB_WAVE) before += (context_lens[s] + LH_TILE - 1) / LH_TILE;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) before += __shfl_xor(before, off, HB_WAVE);
+    before = __builtin_amdgcn_readfirstlane(before);
+    const int pos0 = __builtin_amdgcn_readfirstlane(positions[begin]);     // (a sequence's tokens follow each other)
+    const int in_seq = tile * 64 + 32 * group + n;
+    const bool mine = in_seq < rows;
+    const int t = begin + (mine ? in_seq : rows - 1);
+    const int sees = mine ? pos0 + in_seq : -1;
+    const int first = pos0 + tile * 64;                                    // what the workgroup's first row sees
+    const int last = pos0 + min(tile * 64 + 63, rows - 1);
+    const int wave_last = pos0 + min(tile * 64 + 32 * group + 31, rows - 1);
+    const int n_tiles = last / LH_TILE + 1;
+    for (int i = tid; i < VD; i += 256) lost_from[i] = 0x7fffffff;
+
+    const char* k_src = (const char*)(keys + ((size_t)h * tiles + before) * 2 * DS * HB_WAVE * 8) + 16 * lane;
+    const char* r_src = (const char*)(turned + (size_t)before * 2 * RS * HB_WAVE * 8) + 16 * lane;
+    const char* v_src = (const char*)(values + ((size_t)h * tiles + before) * 2 * VB * 2 * HB_WAVE * 8) + 16 * lane;
+    auto ask_keys = [&](int c, int buf) {
+#pragma unroll
+        for (int i = 0; i < K_LOADS; ++i) {
+            const int piece = wave * K_LOADS + i, b = piece / KS, ks = piece % KS;
+            const char* src = ks < DS ? k_src + ((size_t)(2 * c + b) * DS + ks) * 1024 : r_src + ((size_t)(2 * c + b) * RS + ks - DS) * 1024;
+            hb_load_to_lds(src, &K[buf][0][0][0] + piece * HB_WAVE);
+        }
+    };
+    auto ask_values = [&](int c) {
+#pragma unroll
+        for (int i = 0; i < V_LOADS; ++i) {
+            const int piece = wave * V_LOADS + i;
+            hb_load_to_lds(v_src + ((size_t)c * 4 * VB + piece) * 1024, &V[0][0][0][0] + piece * HB_WAVE);
+        }
+    };
+    la_bf16x8 qh[KS], ql[KS];
+    {
+        const float* row = q + (size_t)t * q_ld + (size_t)h * (DIM + ROT) + 8 * g;
+        const float* trow = q_turned + ((size_t)t * H + h) * ROT + 8 * g;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                __bf16 hi, lo;
+                la_split((ks < DS ? row[16 * ks + e] : trow[16 * (ks - DS) + e]) * (scale * LP_LOG2E), hi, lo);
+                qh[ks][e] = hi;
+                ql[ks][e] = lo;
+            }
+    }
+    ask_keys(0, 0);
+    float m = -INFINITY, l = 0.f;
+    la_f32x16 acc[VB];
+#pragma unroll
+    for (int b = 0; b < VB; ++b)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[b][e] = 0.f;
+
+    for (int c = 0, buf = 0; c < n_tiles; ++c, buf ^= 1) {
+        const int key0 = c * LH_TILE + 32 * block;
+        const bool works = key0 <= wave_last;
+        hb_wait_vmcnt<0>();
+        hb_workgroup_barrier();                      // the tile's keys are there; nobody reads the tile before any more
+        ask_values(c);
+        if (c + 1 < n_tiles) ask_keys(c + 1, buf ^ 1);
+        la_bf16x8 ph[2], pl[2];
+        if (works) {
+            la_f32x16 s, s_low;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) s[e] = s_low[e] = 0.f;
+            const uint4* const at = &K[buf][block][0][lane];
+            la_bf16x8 k[KS];
+            static_for<0, AHEAD>([&](auto t) { k[t()] = lds_read_ahead<1024 * t()>(at); });
+            static_for<0, KS>([&](auto t) {
+                constexpr int ks = t();
+                if constexpr (ks + AHEAD < KS) k[ks + AHEAD] = lds_read_ahead<1024 * (ks + AHEAD)>(at);
+                lds_wait<(ks + AHEAD < KS ? AHEAD : KS - 1 - ks)>(k[ks]);
+                s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k[ks], qh[ks], s, 0, 0, 0);
+                s_low = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k[ks], ql[ks], s_low, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            s += s_low;
+            // s[e]: key key0 + 8 (e / 4) + 4 g + e % 4 against query n, in powers of two
+            if (__any(key0 + 31 > sees)) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    if (key0 + 8 * (e >> 2) + 4 * g + (e & 3) > sees) s[e] = -INFINITY;
+            }
+            float cmax = s[0];
+#pragma unroll
+            for (int e = 1; e < 16; ++e) cmax = fmaxf(cmax, s[e]);
+            cmax = fmaxf(cmax, __shfl_xor(cmax, 32, HB_WAVE));
+            if (__any(cmax > m + LP_SLACK)) {
+                const float m_new = cmax > m + LP_SLACK ? cmax : m;
+                const float corr = m == m_new ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);
+                l *= corr;
+                m = m_new;
+#pragma unroll
+                for (int b = 0; b < VB; ++b)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) acc[b][e] *= corr;
+            }
+            const float base = m == -INFINITY ? 0.f : m;             // (a row that has seen nothing yet)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const float p = __builtin_amdgcn_exp2f(s[e] - base);
+                l += p;
+                __bf16 hi, lo;
+                la_split(p, hi, lo);
+                ph[e >> 3][e & 7] = hi;
+                pl[e >> 3][e & 7] = lo;
+            }
+        }
+        if (c + 1 < n_tiles) hb_wait_vmcnt<K_LOADS>();               // (the values were asked for before the next keys)
+        else hb_wait_vmcnt<0>();
+        hb_workgroup_barrier();
+        if (c * LH_TILE + LH_TILE - 1 > first) {
+            // Keys that not every row sees: a weight of zero does not hide a number without a finite size from the rows that
+            // do not see it, so such a number stays out of the sums, and the rows that see its key lose it at the end.
+            for (int i = tid; i < 2 * VB * 2 * HB_WAVE; i += 256) {
+                uint4* at = &V[0][0][0][0] + i;
+                const uint4 v = *at;
+                const unsigned any = (((v.x & 0x7f807f80u) + 0x00800080u) | ((v.y & 0x7f807f80u) + 0x00800080u) |
+                                      ((v.z & 0x7f807f80u) + 0x00800080u) | ((v.w & 0x7f807f80u) + 0x00800080u)) & 0x80008000u;
+                if (any) {
+                    const int b = i / (VB * 2 * HB_WAVE), step = i / HB_WAVE % 2, of = i % HB_WAVE;
+                    const int number = 32 * (i / (2 * HB_WAVE) % VB) + of % 32;
+                    unsigned short* entry = (unsigned short*)at;
+                    for (int e = 0; e < 8; ++e) {
+                        const int key = c * LH_TILE + 32 * b + 16 * step + 8 * (e >> 2) + 4 * (of >> 5) + (e & 3);
+                        if (key > first && (entry[e] & 0x7f80) == 0x7f80) {
+                            atomicMin(&lost_from[number], key);
+                            entry[e] = 0;
+                        }
+                    }
+                }
+            }
+            hb_workgroup_barrier();
+        }
+        if (works) {
+            const uint4* const at = &V[block][0][0][lane];
+            la_bf16x8 v[2 * VB];
+            static_for<0, AHEAD>([&](auto t) { v[t()] = lds_read_ahead<1024 * t()>(at); });
+            static_for<0, 2 * VB>([&](auto t) {
+                constexpr int i = t(), b = i / 2, s = i % 2;
+                if constexpr (i + AHEAD < 2 * VB) v[i + AHEAD] = lds_read_ahead<1024 * (i + AHEAD)>(at);
+                lds_wait<(i + AHEAD < 2 * VB ? AHEAD : 2 * VB - 1 - i)>(v[i]);
+                acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v[i], ph[s], acc[b], 0, 0, 0);
+                acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v[i], pl[s], acc[b], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        }
+    }
+    l += __shfl_xor(l, 32, HB_WAVE);
+    __syncthreads();
+    // the second block's sums go through the keys' place
+    static_assert(sizeof(K) >= 2 * VB * 16 * HB_WAVE * sizeof(float), "the sums of two waves fit where the keys lay");
+    float* there = (float*)&K[0][0][0][0] + group * VB * 16 * HB_WAVE + lane;
+    if (block == 1) {
+#pragma unroll
+        for (int b = 0; b < VB; ++b)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) there[(b * 16 + e) * HB_WAVE] = acc[b][e];
+        if (g == 0) met[group][0][n] = m, met[group][1][n] = l;
+    }
+    __syncthreads();
+    if (block == 1 || !mine) return;
+    const float m1 = met[group][0][n], top = fmaxf(m, m1);
+    const float base = top == -INFINITY ? 0.f : top;
+    const float f0 = __builtin_amdgcn_exp2f(m - base), f1 = __builtin_amdgcn_exp2f(m1 - base);
+    l = l * f0 + met[group][1][n] * f1;
+    if (sinks) l += __builtin_amdgcn_exp2f(sinks[h] * LP_LOG2E - base);    // (an infinite share, a sink far above every score, leaves 0)
+    float w = l > 0.f ? 1.0f / l : 0.f;
+    if (gate) w *= 1.0f / (1.0f + expf(-gate[(size_t)t * gate_ld + h]));
+    const float w0 = f0 * w, w1 = f1 * w;
+    bf16* to = out + ((size_t)t * H + h) * VD + 4 * g;
+#pragma unroll
+    for (int b = 0; b < VB; ++b)
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            // acc[b][4 a + e]: number 32 b + 8 a + 4 g + e of query n
+            bf16 o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float v = acc[b][4 * a + e] * w0 + there[(b * 16 + 4 * a + e) * HB_WAVE] * w1;
+                o[e] = hb_from_float<bf16>(lost_from[32 * b + 8 * a + 4 * g + e] > sees ? v : NAN);
+            }
+            *(uint2*)(to + 32 * b + 8 * a) = uint2{o[0].bits | ((unsigned)o[1].bits << 16), o[2].bits | ((unsigned)o[3].bits << 16)};
+        }
+}
+
+// tiles: the step's sequences' tiles of 64 keys together; scratch: keys [H][2 tiles][dim / 16][64][8], turned [2 tiles][rot / 16][64][8],
+// values [H][2 tiles][vdim / 32][2][64][8]. w_uk / w_uv: [H] matrices of dim / vdim rows of rank, packed.
+extern "C" int hb_latent_attention_heads(const float* q, int q_ld, const float* q_turned, const void* pages, const void* w_uk,
+                                         const void* w_uv, void* keys, void* turned, void* values, void* out,
+                                         const float* gate, int gate_ld, const int* positions, const int* seq_starts,
+                                         const int* context_lens, int n_seqs, const int* slots, const int* page_table,
+                                         int max_pages, int page_size, int tiles, int longest, int T, int H, int dim,
+                                         int vdim, int rank, int rot, float scale, const float* sinks, hipStream_t stream) {
+    HB_REQUIRE(T > 0 && H > 0 && H <= 65535 && n_seqs > 0 && n_seqs <= 65535 && longest > 0 && longest <= T,
+               "latent attention: %d sequences of up to %d of %d tokens, %d heads", n_seqs, longest, T, H);
+    HB_REQUIRE(rank > 0 && rank % 32 == 0 && rank <= LH_RANK, "latent attention: built heads take a latent in steps of 32 up to 512, not %d", rank);
+    HB_REQUIRE((dim == 64 || dim == 128) && vdim == dim && (rot == 0 || rot == 32 || rot == 64),
+               "latent attention: heads of %d + %d and %d are not built", dim, rot, vdim);
+    HB_REQUIRE(page_size > 0 && page_size % LH_TILE == 0, "latent attention: pages of %d positions", page_size);
+    HB_REQUIRE(tiles > 0 && q_ld >= H * (dim + rot), "latent attention: empty input");
+    const long long blocks = ((long long)longest + 63) / 64 * H;
+    HB_REQUIRE(blocks < (1ll << 23) && tiles < (1 << 23), "latent attention: too many tokens for the grid");
+    latent_heads_kernel<<<dim3(tiles, H), 256, 0, stream>>>((const bf16*)pages, (const bf16*)w_uk, (const bf16*)w_uv, (bf16*)keys, (bf16*)turned,
+                                                            (bf16*)values, context_lens, n_seqs, slots, page_table, max_pages, page_size,
+                                                            tiles, dim, rank, rot);
+    HB_CHECK_LAUNCH("latent_heads");
+    const dim3 grid((unsigned)blocks, n_seqs);
+#define LH_LAUNCH(DSV, RSV, VBV)                                                                                    \
+    latent_attention_heads_kernel<DSV, RSV, VBV><<<grid, 256, 0, stream>>>(                                         \
+        q, (size_t)q_ld, q_turned, (const bf16*)keys, (const bf16*)turned, (const bf16*)values, (bf16*)out, gate, gate_ld, \
+        positions, seq_starts, context_lens, n_seqs, tiles, H, scale, sinks)
+    if (dim == 128) {
+        if (rot == 64) LH_LAUNCH(8, 4, 4);
+        else if (rot == 32) LH_LAUNCH(8, 2, 4);
+        else LH_LAUNCH(8, 0, 4);
+    } else {
+        if (rot == 64) LH_LAUNCH(4, 4, 2);
+        else if (rot == 32) LH_LAUNCH(4, 2, 2);
+        else LH_LAUNCH(4, 0, 2);
+    }
+#undef LH_LAUNCH
+    HB_CHECK_LAUNCH("latent_attention_heads");
+    return 0;
 }
 
 // out[row, :] = sum over the ranges (in order) of their sums, brought to one maximum, over the summed

@@ -27,8 +27,8 @@
 // crates/backends/backend_common/src/avx512_attn_dot8_bf16.S. The new key's norm, rotation and cache write inside the
 // decode kernel: crates/backends/backend_metal/shaders/head_norm_rope_kv_append.metal:37-110.
 #include "common.h"
+#include "lds_read.h"
 #include <math.h>
-#include <type_traits>
 
 HB_MODULE_ERROR_SLOT()
 
@@ -196,35 +196,6 @@ __device__ __forceinline__ float softmax_reference(f32x16 st[2], int g2, int pag
 }
 
 // ----------------------------------------------------------------- prefill
-// A read of 16 bytes from LDS that the compiler does not follow: it neither waits for it nor
-// knows that it is in flight, so the caller waits by count (lds_wait<N>: at most N reads, in the
-// order in which they were issued, may still be on their way) before the value is used. The
-// compiler's own waits drain every read in flight (lgkmcnt(0)) each time a value is needed, the
-// one issued a moment ago included; with three reads ahead of their products a wave of the
-// prompt kernels then stood still for a read's whole way through LDS eleven times a page.
-template <int BYTES_ON>
-__device__ __forceinline__ bf16x8 lds_read_ahead(const bf16* p) {
-    bf16x8 v;
-    const uint32_t at = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) bf16*)p;
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(BYTES_ON));
-    return v;
-}
-// (the value that is about to be used goes through the wait, so that its use cannot be moved before it)
-template <int N>
-__device__ __forceinline__ void lds_wait(bf16x8& arrived) {
-    asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(arrived) : "n"(N));
-}
-
-// f(integral_constant<int, B>), ..., f(integral_constant<int, E - 1>): a loop whose index is a
-// constant inside the body
-template <int B, int E, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (B < E) {
-        f(std::integral_constant<int, B>{});
-        static_for<B + 1, E>(f);
-    }
-}
-
 // What a lane needs to find its operands in the LDS stages of a page's keys and values.
 struct PrefillLane {
     int c32, g2, krow, k_read[2], v_swz;

@@ -7,9 +7,10 @@ score is the dot product of query and key times `scale`, causal, plain softmax; 
 multiplied by sigmoid(W_g h)_n and the heads go through W_o.
 
 What a token leaves in the cache is c and the rotated part, one row of kv_rank + rot_dim numbers, and
-no values beside them. The kernels never build a head's keys or values: the query's unrotated part is taken through
+no values beside them. Steps of few tokens never build a head's keys or values: the query's unrotated part is taken through
 W_uk,n^T first (kv_rank numbers), scores and weighted sums then run on the cached rows themselves,
-one shared "key head" for all query heads, and the summed latents go through W_uv,n afterwards.
+one shared "key head" for all query heads, and the summed latents go through W_uv,n afterwards. Prompts in bfloat16 build
+them for the step, from the cached rows (kernels.latent.heads_pay says when).
 Scores, softmax and the weighted sums are float32 in either mode.
 
 Two parameters change the form. `gate="elementwise"`: W_g has a row for every entry of the joined heads, and
@@ -118,6 +119,7 @@ class LatentAttention(Part):
         self.norm_w = rt.weight(tensors[n["dkv_norm"]], matrix=False)
         # W_uk a head, transposed: [H, rank, dim], so that q' = W_uk,n^T q_n is a product with rows of k = dim
         uk = rt.weight(tensors[n["uk"]]).view(H, self.dim, self.rank)
+        self.uk = None
         self.uk_t = uk.transpose(1, 2).contiguous()
         self.uv = rt.weight(tensors[n["uv"]]).view(H, self.vdim, self.rank).contiguous()
         self.o = Linear(rt.weight(tensors[n["o"]]), scratch=rt.scratch)
@@ -125,6 +127,9 @@ class LatentAttention(Part):
         self.cores = (rt.dtype == torch.bfloat16 and moe.mfma_takes(self.dim, H * self.dim, self.dim, self.rank)
                       and moe.mfma_takes(self.rank, H * self.rank, self.rank, self.vdim))
         if self.cores:
+            # (as they are stored too, for prompts whose heads' keys are built)
+            if self.dim in (64, 128) and self.vdim == self.dim and self.rank <= 512:
+                self.uk = moe.pack_grouped(uk.contiguous())
             self.uk_t, self.uv = moe.pack_grouped(self.uk_t), moe.pack_grouped(self.uv)
 
     def forward(self, ctx, y, x):
@@ -133,12 +138,18 @@ class LatentAttention(Part):
         kv = ctx.cache.kv_view(ctx.cache_entry)
         proj = rt.buffer("latent_proj", (T, self.width), torch.float32)
         self.proj.forward(y, proj)
-        q_full = rt.buffer("latent_q_full", (T, H * self.row), torch.float32)
         cores = self.cores
-        q_plain = rt.buffer("latent_q_plain", (T, H * self.dim), torch.bfloat16) if cores else None
+        built = self.uk is not None and latent.heads_pay(ctx.meta, kv, H, self.dim, self.vdim, self.rank, self.rot_dim)
+        q_full = turned = q_plain = None
+        if built:
+            turned = rt.buffer("latent_turned", (T, H * self.rot_dim), torch.float32)
+        else:
+            q_full = rt.buffer("latent_q_full", (T, H * self.row), torch.float32)
+            q_plain = rt.buffer("latent_q_plain", (T, H * self.dim), torch.bfloat16) if cores else None
+
         def write(**args):
             latent.latent_write(proj, 0, self.q_width, self.norm_w, q_full, self.inv_freq, ctx.meta, kv, H, self.dim,
-                                self.rank, self.rot_dim, self.rot_dims, self.eps, **args)
+                                self.rank, self.rot_dim, self.rot_dims, self.eps, turned=turned, **args)
         q_rows, q_ld = proj, self.width
         if self.uq is not None:
             # the cache's row and the queries' normed latent, then the queries themselves
@@ -147,31 +158,35 @@ class LatentAttention(Part):
             q_ld = H * (self.dim + self.rot_dim)
             q_rows = rt.buffer("latent_queries", (T, q_ld), torch.float32)
             self.uq.forward(c_q, q_rows)
-            if cores or self.rot_dim:
+            if q_plain is not None or self.rot_dim:
                 write(write_cache=False, q_plain=q_plain, queries=q_rows)
         else:
             write(write_cache=ctx.owns_cache, q_plain=q_plain)
-        # q'[t, n, :] = W_uk,n^T q[t, n, :dim]: a product a head, all heads in one launch
-        if cores:
-            moe.grouped_mfma(q_plain, H * self.dim, self.dim, self.uk_t, q_full, H * self.row, self.row, moe.EPI_F32, M=T)
-        else:
-            ops.gemm_plain_batched(q_rows, self.uk_t, q_full, T, self.rank, self.dim, q_ld, self.dim,
-                                   H * self.row, H, self.dim + self.rot_dim, self.rank * self.dim, self.row)
-        mixed = rt.buffer("latent_mixed", (T, H * self.rank))
         gate = proj if self.gated and self.gate_kind == "head" else None
-        if latent.mfma_takes(kv, self.rank, self.rot_dim):
-            latent.latent_attention_mfma(q_full, ctx.meta, kv, mixed, gate, self.q_width + self.row, H, self.rank,
-                                         self.rot_dim, self.scale, rt.buffer, sinks=self.sink_w)
-        else:
-            latent.latent_attention_plain(q_full, ctx.meta, kv, mixed, gate, self.q_width + self.row, H, self.rank,
-                                          self.rot_dim, self.scale, sinks=self.sink_w)
-        # a head's summed latents through its W_uv
         attn = rt.buffer("latent_attn", (T, H * self.vdim))
-        if cores:
-            moe.grouped_mfma(mixed, H * self.rank, self.rank, self.uv, attn, H * self.vdim, self.vdim, moe.EPI_BF16, M=T)
+        if built:
+            latent.latent_attention_heads(q_rows, 0, turned, ctx.meta, kv, self.uk, self.uv, attn, gate, self.q_width + self.row,
+                                          self.dim, self.vdim, self.rank, self.rot_dim, self.scale, rt.buffer, sinks=self.sink_w)
         else:
-            ops.gemm_plain_batched(mixed, self.uv, attn, T, self.vdim, self.rank, H * self.rank, self.rank,
-                                   H * self.vdim, H, self.rank, self.vdim * self.rank, self.vdim)
+            # q'[t, n, :] = W_uk,n^T q[t, n, :dim]: a product a head, all heads in one launch
+            if cores:
+                moe.grouped_mfma(q_plain, H * self.dim, self.dim, self.uk_t, q_full, H * self.row, self.row, moe.EPI_F32, M=T)
+            else:
+                ops.gemm_plain_batched(q_rows, self.uk_t, q_full, T, self.rank, self.dim, q_ld, self.dim,
+                                       H * self.row, H, self.dim + self.rot_dim, self.rank * self.dim, self.row)
+            mixed = rt.buffer("latent_mixed", (T, H * self.rank))
+            if latent.mfma_takes(kv, self.rank, self.rot_dim):
+                latent.latent_attention_mfma(q_full, ctx.meta, kv, mixed, gate, self.q_width + self.row, H, self.rank,
+                                             self.rot_dim, self.scale, rt.buffer, sinks=self.sink_w)
+            else:
+                latent.latent_attention_plain(q_full, ctx.meta, kv, mixed, gate, self.q_width + self.row, H, self.rank,
+                                              self.rot_dim, self.scale, sinks=self.sink_w)
+            # a head's summed latents through its W_uv
+            if cores:
+                moe.grouped_mfma(mixed, H * self.rank, self.rank, self.uv, attn, H * self.vdim, self.vdim, moe.EPI_BF16, M=T)
+            else:
+                ops.gemm_plain_batched(mixed, self.uv, attn, T, self.vdim, self.rank, H * self.rank, self.rank,
+                                       H * self.vdim, H, self.rank, self.vdim * self.rank, self.vdim)
         if self.gated and self.gate_kind == "elementwise":
             gated = rt.buffer("latent_gated", (T, H * self.vdim))
             ops.gate_heads(attn, proj, self.q_width + self.row, gated, H, self.vdim, self.vdim)
