@@ -1,13 +1,16 @@
 // Matrix product in float32 arithmetic for any storage types and any sizes:
 //   C[m, n] (+)= sum_k A[m, k] * W[n, k]      (weights are [out, in], k contiguous)
 // It is the whole matrix path of the float32 mode and the fallback of the bfloat16
-// mode for shapes its own MFMA kernels refuse. Each output is summed over k ascending
-// with fused multiply-adds, so its value does not depend on M, on the tile or kernel
-// it falls in, or on what else is in the batch: the matrix cores' float32 products
-// (v_mfma_f32_16x16x4_f32) add their four k one after another with one rounding each,
+// mode for shapes its own MFMA kernels refuse. Each output is summed in stretches of K_BLOCK
+// elements of k: a stretch from zero over k ascending with fused multiply-adds, then the
+// stretches' sums one after another. Stretches lie at fixed places, so an output's value does
+// not depend on M, on the tile or kernel it falls in, or on what else is in the batch, and yet
+// a product of few rows can give every stretch a wave of its own. The matrix cores' float32
+// products (v_mfma_f32_16x16x4_f32) add their four k one after another with one rounding each,
 // bit for bit what fmaf gives in that order (checked on 16,384 sums of mixed magnitudes),
-// and every kernel here feeds them k in ascending order. (hb_gemm_plain_short_k is the entry for products with a
-// short k: it sends up to 32 float32 rows times bfloat16 rows to gemm_few_rows_kernel, whose four partial
+// and every kernel here feeds them k in ascending order. (One chain over all of k, which this
+// replaced, was further from 64 bits: at K = 2048 8.1e-7 of the sums' root mean square, now 4.1e-7; at K = 12288 20e-7
+// and 4.2e-7.) (hb_gemm_plain_short_k is the entry for products with a short k: it sends up to 32 float32 rows times bfloat16 rows to gemm_few_rows_kernel, whose four partial
 // sums a column differ from that order by float32 rounding, and everything else here.)
 // In xigh/herbert-rs: crates/backends/backend_bf16/src/kernels.rs:154-164 (float32 sums over k ascending of
 // x[m, k] * float(w[n, k]), no bias); crates/backends/backend_vulkan/shaders/bf16_matmul.comp:31-60.
@@ -15,6 +18,9 @@
 #include "mfma_f32.h"
 
 HB_MODULE_ERROR_SLOT()
+
+// Elements of k that are summed as one chain; a multiple of every kernel's stage.
+#define K_BLOCK 512
 
 // What a product may do to a sum before it stores it: nothing (rate null), or turn the pre-activation of a
 // decay into the decay itself, exp(-exp(rate[n / D]) * softplus(sum + bias[n])) for column n (float32; the
@@ -69,7 +75,7 @@ __device__ __forceinline__ void store_quad(TC* C, int ldc, int m, int n, int N, 
 // 4096 x 4096 x 4096 in 1,082 us (127 TFLOP/s), 564 x 6144 x 2048 in 165, 564 x 2048 x 2048 in 67, 64 x 4096 x 4096 in
 // 55; the kernel of vector FMAs and 4-byte loads that this replaced took 2,465, 372, 323 and 632.
 template <class TA, class TW, class TC, bool ACCUM, int BM, int BN, int BK, bool VEC>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, 2)
 gemm_plain_tile_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* __restrict__ C, int M, int N,
                        int K, int lda, int ldw, int ldc, size_t batch_a, size_t batch_w, size_t batch_c,
                        DecayEpilogue ep) {
@@ -116,11 +122,12 @@ gemm_plain_tile_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
         }
     };
 
-    f32x4 acc[NB][MB];
+    static_assert(K_BLOCK % BK == 0, "a stretch of k is whole stages");
+    f32x4 acc[NB][MB], total[NB][MB];
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll
-        for (int i = 0; i < MB; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < MB; ++i) total[j][i] = acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     fetch(0);
     stash(0);
@@ -144,6 +151,12 @@ gemm_plain_tile_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
                     for (int i = 0; i < MB; ++i) acc[j][i] = mfma_k4(w[j][s], a[i][s], acc[j][i]);
         }
         if (more) stash(buf ^ 1);
+        if (!more || (k0 + BK) % K_BLOCK == 0) {
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+#pragma unroll
+                for (int i = 0; i < MB; ++i) total[j][i] += acc[j][i], acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
         __syncthreads();
     }
 
@@ -153,57 +166,79 @@ gemm_plain_tile_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
         if (m >= M) continue;
 #pragma unroll
         for (int j = 0; j < NB; ++j)
-            store_quad<TC, ACCUM, VEC>(C, ldc, m, n0 + wn + 16 * j + 4 * q, N, acc[j][i], ep);
+            store_quad<TC, ACCUM, VEC>(C, ldc, m, n0 + wn + 16 * j + 4 * q, N, total[j][i], ep);
     }
 }
 
-// Up to 16 rows (a decode step): a product bound by the weights' bytes. A wave alone on 16 rows of W: no LDS and no
-// barrier; every lane loads a quad of its row of W and of A for each of the next WAVE_DEPTH blocks of 16 k while the
-// WAVE_DEPTH before are multiplied, and the lanes' quads are transposed in registers. The sum over k is one chain as
-// everywhere here (no split of k: the order is the other kernel's), 8.5 us of products at K = 2048, which bounds narrow
-// weights; wide ones stream. 2 x 2048 x 2048 takes 19 us, 2 x 6144 x 2048 21, 2 x 32768 x 2048 52 (5.2 TB/s); tiles of
-// 32 x 32 take 21, 26 and 60, the kernel that these replaced took 253, 262 and 378. (8 blocks ahead; 16 take as long
-// at few rows and 10 % longer at many, 24 longer everywhere; two blocks of 16 rows of A a wave for 17 to 32 rows: 63 us
-// at 24 x 4096 x 4096 where tiles of 32 x 32 take 53.)
+// Up to 16 rows (a decode step): a product bound by the weights' bytes and, narrow ones, by the chain of k. A workgroup
+// on 16 rows of W, a wave on every stretch of K_BLOCK (up to WAVE_WAVES of them at a time): no load waits for another
+// wave, and a wave asks for all of its stretch of W at once (32 quads a lane), for A eight blocks of 16 k ahead; the
+// lanes' quads are transposed in registers. The stretches' sums meet in LDS, where a thread an output adds them in
+// their order. 2 x 2048 x 2048 takes 10.7 us (one wave for all of k, a chain of 512 products with eight blocks in
+// flight: 19.4), 2 x 2048 x 3072 12.8 (27.9), 2 x 4096 x 2048 13.3 (20.0), 8 x 4096 x 12288 62 (106); with bfloat16
+// weights 10.5 (36), 12.9 (53), 11 (38) and 43 (233). Wide weights stream: 2 x 6144 x 2048 19.9 (21.3), 2 x 32768 x
+// 2048 64 (60; a wave after the other's stretches there, so that no workgroup waits for another's: 83).
 #define WAVE_ROWS 16
+#define WAVE_WAVES 8
 #define WAVE_DEPTH 8
 template <class TA, class TW, class TC, bool ACCUM>
-__global__ void __launch_bounds__(HB_WAVE)
+__global__ void __launch_bounds__(WAVE_WAVES * HB_WAVE)
 gemm_plain_wave_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* __restrict__ C, int M, int N,
                        int K, int lda, int ldw, int ldc, size_t batch_a, size_t batch_w, size_t batch_c,
                        DecayEpilogue ep) {
     A += blockIdx.z * batch_a;
     W += blockIdx.z * batch_w;
     C += blockIdx.z * batch_c;
-    const int lane = threadIdx.x, r = lane & 15, q = lane >> 4;
+    constexpr int GROUPS = K_BLOCK / 16 / WAVE_DEPTH;
+    __shared__ __attribute__((aligned(16))) f32x4 sums[WAVE_WAVES][HB_WAVE];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    const int r = lane & 15, q = lane >> 4;
     const int n0 = blockIdx.x * 16;
     // (rows beyond M or N are row 0 once more, whose sums go nowhere; blocks beyond K are zeros)
     const TW* w_row = W + (size_t)(n0 + r < N ? n0 + r : 0) * ldw + 4 * q;
     const TA* a_row = A + (size_t)(r < M ? r : 0) * lda + 4 * q;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f}, w_next[WAVE_DEPTH], a_next[WAVE_DEPTH];
-    auto fetch = [&](int k0) {
+    f32x4 total = {0.f, 0.f, 0.f, 0.f};
+    for (int first = 0; first < K; first += waves * K_BLOCK) {
+        const int k0 = first + wave * K_BLOCK;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        if (k0 + K_BLOCK <= K) {
+            f32x4 w[GROUPS][WAVE_DEPTH], a[2][WAVE_DEPTH];
+            auto fetch_a = [&](int g) {
 #pragma unroll
-        for (int d = 0; d < WAVE_DEPTH; ++d) {
-            const int k = k0 + 16 * d;
-            w_next[d] = load_quad<true>(w_row + k, K - k);
-            a_next[d] = load_quad<true>(a_row + k, K - k);
+                for (int d = 0; d < WAVE_DEPTH; ++d) a[g & 1][d] = load_quad<true>(a_row + k0 + 16 * (g * WAVE_DEPTH + d), 4);
+            };
+            fetch_a(0);
+#pragma unroll
+            for (int g = 0; g < GROUPS; ++g)
+#pragma unroll
+                for (int d = 0; d < WAVE_DEPTH; ++d) w[g][d] = load_quad<true>(w_row + k0 + 16 * (g * WAVE_DEPTH + d), 4);
+#pragma unroll
+            for (int g = 0; g < GROUPS; ++g) {
+                if (g + 1 < GROUPS) fetch_a(g + 1);
+#pragma unroll
+                for (int d = 0; d < WAVE_DEPTH; ++d) {
+                    transpose_quads(w[g][d]);
+                    transpose_quads(a[g & 1][d]);
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) acc = mfma_k4(w[g][d][s], a[g & 1][d][s], acc);
+                }
+            }
+        } else {
+            for (int k = k0; k < K; k += 16) {       // (what is left of k, blocks of 16)
+                f32x4 w = load_quad<true>(w_row + k, 4), a = load_quad<true>(a_row + k, 4);
+                transpose_quads(w);
+                transpose_quads(a);
+#pragma unroll
+                for (int s = 0; s < 4; ++s) acc = mfma_k4(w[s], a[s], acc);
+            }
         }
-    };
-    fetch(0);
-    for (int k0 = 0; k0 < K; k0 += 16 * WAVE_DEPTH) {
-        f32x4 w[WAVE_DEPTH], a[WAVE_DEPTH];
-#pragma unroll
-        for (int d = 0; d < WAVE_DEPTH; ++d) w[d] = w_next[d], a[d] = a_next[d];
-        if (k0 + 16 * WAVE_DEPTH < K) fetch(k0 + 16 * WAVE_DEPTH);
-#pragma unroll
-        for (int d = 0; d < WAVE_DEPTH; ++d) {
-            transpose_quads(w[d]);
-            transpose_quads(a[d]);
-#pragma unroll
-            for (int s = 0; s < 4; ++s) acc = mfma_k4(w[d][s], a[d][s], acc);
-        }
+        if (first) __syncthreads();                  // (the round before has been read)
+        sums[wave][lane] = acc;
+        __syncthreads();
+        if (wave == 0)
+            for (int b = 0; b < waves && first + b * K_BLOCK < K; ++b) total += sums[b][lane];
     }
-    if (r < M) store_quad<TC, ACCUM, true>(C, ldc, r, n0 + 4 * q, N, acc, ep);
+    if (wave == 0 && r < M) store_quad<TC, ACCUM, true>(C, ldc, r, n0 + 4 * q, N, total, ep);
 }
 
 // The kernel of a product. 16-byte loads and stores where rows and strides allow them. Up to 16 rows of whole blocks of
@@ -229,11 +264,12 @@ static void launch_as(const TA* A, const TW* W, TC* C, int M, int N, int K, int 
         const long long n = tiles(side) / batch, x = n < GRID_X ? n : GRID_X;
         return dim3((unsigned)x, (unsigned)((n + x - 1) / x), batch);
     };
+    const int stretches = (K + K_BLOCK - 1) / K_BLOCK, wave_threads = HB_WAVE * (stretches < WAVE_WAVES ? stretches : WAVE_WAVES);
 #define HB_PLAIN_TILE(BM, BK, VEC)                                                                                    \
     gemm_plain_tile_kernel<TA, TW, TC, ACCUM, BM, BM, BK, VEC>                                                        \
         <<<grid(BM), 256, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, batch_a, batch_w, batch_c, ep)
     if (vec && M <= WAVE_ROWS && K % 16 == 0)
-        gemm_plain_wave_kernel<TA, TW, TC, ACCUM><<<dim3((N + 15) / 16, 1, batch), HB_WAVE, 0, stream>>>(
+        gemm_plain_wave_kernel<TA, TW, TC, ACCUM><<<dim3((N + 15) / 16, 1, batch), wave_threads, 0, stream>>>(
             A, W, C, M, N, K, lda, ldw, ldc, batch_a, batch_w, batch_c, ep);
     else if (!vec)
         HB_PLAIN_TILE(32, 64, false);

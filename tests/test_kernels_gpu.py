@@ -66,6 +66,25 @@ def test_gemm_plain(M, N, K, dts):
     assert torch.allclose(cb.float(), want, rtol=2 ** -8, atol=1e-3)
 
 
+@pytest.mark.parametrize("K", [512, 528, 1024, 1504, 4096, 4656, 8704])
+@pytest.mark.parametrize("wd", [torch.float32, torch.bfloat16])
+def test_gemm_plain_stretches_of_k_are_the_same_in_every_kernel(K, wd):
+    """k is summed in stretches of 512 wherever a row falls: one stretch, a stretch and part of the next, as many as a
+    workgroup of the few-row kernel has waves, and more. The first row alone, with 16 and among 40 is the same bits, and
+    off from float64 by at most 512 roundings of a chain and one for each stretch's addition."""
+    from herbert_rs_amd.kernels import ops
+    N = 100
+    a, w = rand(40, K, seed=23), rand(N, K, seed=24, dtype=wd)
+    got = {}
+    for rows in (1, 16, 40):
+        got[rows] = torch.empty(rows, N, device=dev())
+        ops.gemm_plain(a[:rows].contiguous(), w, got[rows])
+    assert torch.equal(got[1], got[16][:1]) and torch.equal(got[16], got[40][:16])
+    want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    steps = min(K, 512) + (K + 511) // 512
+    assert bool(((got[40].double() - want).abs() <= steps * 2.0 ** -24 * size + 1e-30).all())
+
+
 def test_gemm_plain_of_more_tiles_than_a_grids_x_holds():
     """The most rows that are taken, of a width whose tiles of 32 x 32 times 256 threads pass 2^32: whole numbers, so every
     sum is exact in bfloat16."""
