@@ -168,7 +168,7 @@ moe_route_kernel(const float* __restrict__ logits, int ld, const float* __restri
 __global__ void __launch_bounds__(1024)
 moe_place_kernel(const int* __restrict__ chosen, int* __restrict__ counts, int* __restrict__ order,
                  int* __restrict__ row_of, int* __restrict__ tile_expert, int* __restrict__ tile_row0,
-                 int* __restrict__ tile_rows, int A, int E, int max_tiles, int real) {
+                 int* __restrict__ tile_rows, int A, int E, int max_tiles, int real, int tile_m) {
     __shared__ int hist[HB_WAVE * MOE_MAX_E_PER_LANE];
     __shared__ int wave_n[16], firsts[16], tiles[16];
     const int e = blockIdx.x;
@@ -191,7 +191,7 @@ moe_place_kernel(const int* __restrict__ chosen, int* __restrict__ counts, int* 
     if (lane == 0) wave_n[wave] = hits;
     __syncthreads();
     const int before = (int)threadIdx.x < min(e, E) ? hist[threadIdx.x] : 0;       // (E is at most the workgroup's threads)
-    int first = before, tile0 = (before + MOE_TILE_M - 1) / MOE_TILE_M;
+    int first = before, tile0 = (before + tile_m - 1) / tile_m;
 #pragma unroll
     for (int off = HB_WAVE / 2; off > 0; off >>= 1) {
         first += __shfl_xor(first, off, HB_WAVE);
@@ -214,10 +214,10 @@ moe_place_kernel(const int* __restrict__ chosen, int* __restrict__ counts, int* 
     }
     const int count = hist[e];
     if (threadIdx.x == 0) counts[e] = count;
-    for (int i = threadIdx.x; i * MOE_TILE_M < count; i += 1024) {
+    for (int i = threadIdx.x; i * tile_m < count; i += 1024) {
         tile_expert[tile0 + i] = e < real ? e : -1;
-        tile_row0[tile0 + i] = first + i * MOE_TILE_M;
-        tile_rows[tile0 + i] = count - i * MOE_TILE_M < MOE_TILE_M ? count - i * MOE_TILE_M : MOE_TILE_M;
+        tile_row0[tile0 + i] = first + i * tile_m;
+        tile_rows[tile0 + i] = count - i * tile_m < tile_m ? count - i * tile_m : tile_m;
     }
     if (hits == 0) return;
     int row = first;
@@ -311,7 +311,8 @@ moe_route_few_kernel(const float* __restrict__ logits, int ld, const float* __re
 extern "C" int hb_moe_route(const float* logits, const float* bias, int* chosen, float* weight, int* counts,
                             int* order, int* row_of, int* tile_expert, int* tile_row0, int* tile_rows, int T, int E,
                             int top, int max_tiles, int ld, int by_scores, int n_groups, int keep, int real,
-                            int softmax_scores, int worth_top, int renorm, hipStream_t stream) {
+                            int softmax_scores, int worth_top, int renorm, int tile_m, hipStream_t stream) {
+    HB_REQUIRE(tile_m == MOE_TILE_M || tile_m == 128 || tile_m == 192 || tile_m == 256, "moe: row tiles of %d", tile_m);
     HB_REQUIRE(ld >= E, "moe: logits rows %d apart for %d experts", ld, E);
     HB_REQUIRE(!by_scores || (n_groups > 0 && E % n_groups == 0 && keep > 0 && keep <= n_groups &&
                               top <= keep * (E / n_groups)),
@@ -321,9 +322,9 @@ extern "C" int hb_moe_route(const float* logits, const float* bias, int* chosen,
     HB_REQUIRE(E <= HB_WAVE * MOE_MAX_E_PER_LANE, "moe: %d experts, the router takes up to %d", E, HB_WAVE * MOE_MAX_E_PER_LANE);
     const long long A = (long long)T * top;
     HB_REQUIRE(A < (1ll << 30), "moe: too many (token, expert) pairs");
-    HB_REQUIRE(max_tiles >= (A + MOE_TILE_M - 1) / MOE_TILE_M + E, "moe: the tile list is too short");
+    HB_REQUIRE(max_tiles >= (A + tile_m - 1) / tile_m + E, "moe: the tile list is too short");
     const RouteForm form = {by_scores, n_groups, keep, softmax_scores, worth_top, renorm};
-    if (T <= FEW_TOKENS && A <= FEW_PAIRS && E <= HB_WAVE * 4) {
+    if (T <= FEW_TOKENS && A <= FEW_PAIRS && E <= HB_WAVE * 4 && tile_m == MOE_TILE_M) {
 #define HB_FEW(PER)                                                                                                      \
     moe_route_few_kernel<PER><<<1, HB_WAVE * (T < 4 ? 4 : T), 0, stream>>>(logits, ld, bias, chosen, weight, counts, order, \
         row_of, tile_expert, tile_row0, tile_rows, T, E, top, max_tiles, real, form)
@@ -341,7 +342,7 @@ extern "C" int hb_moe_route(const float* logits, const float* bias, int* chosen,
     else HB_ROUTE(MOE_MAX_E_PER_LANE);
 #undef HB_ROUTE
     HB_CHECK_LAUNCH("moe_route");
-    moe_place_kernel<<<E + 1, 1024, 0, stream>>>(chosen, counts, order, row_of, tile_expert, tile_row0, tile_rows, (int)A, E, max_tiles, real);
+    moe_place_kernel<<<E + 1, 1024, 0, stream>>>(chosen, counts, order, row_of, tile_expert, tile_row0, tile_rows, (int)A, E, max_tiles, real, tile_m);
     HB_CHECK_LAUNCH("moe_place");
     return 0;
 }
@@ -724,6 +725,238 @@ grouped_mfma_kernel(const bf16* __restrict__ A, int lda, size_t a_group_off, con
             }
         }
     }
+}
+
+// The same for groups of many rows: a workgroup on 64 TM rows (128, 192 or 256) and 256 weight rows (EPI 2: 128 gate rows and the
+// 128 up rows that go with them, in turns of 16), each of four waves on 128 weight rows x 32 TM rows by 32x32x16 products. What bounds
+// it are the bytes that a CU takes out of the caches, about 45 a nanosecond whatever the kernel: 48 to 64 KB a step of 64 k here, which last
+// longer than the step's products, so the tile is as high as a group's rows fill it (rows beyond a tile's own read its last row
+// again, which costs no such bytes). The kernel above reads the weights for every 64 rows. Weights and activations go straight into rings in LDS (hb_load_to_lds),
+// waited for by count before a bare barrier. There is no branch in the main loop (the last step is peeled off); reads and loads are dealt
+// out between the products, the reads of a k-step during the products of the one before. An activation row is 128 bytes, its 16-byte
+// chunk c at chunk c ^ ((row >> 1) & 7); a block of 16 weight rows and 32 k is 1 KB as packed. K in steps of 64.
+// Both products of a layer, 32 experts of 768 on 2,048, weights from memory (40 and 20 us at the rate of a large copy), by tiles of 64 and
+// by the tile that tile_rows of moe.py takes: 2,048 tokens, four experts each 197 us, 158 (128 rows); 1,712 154, 124 (256); 1,282 149, 105
+// (192); 512 93, 86 (128). 64 experts of 1,536 on 4,096, 2,500 tokens: 781, 571 (192).
+typedef float hb_f32x16 __attribute__((ext_vector_type(16)));
+#define TALL_BN 256
+#define TALL_W_STAGE (TALL_BN * 64)          // elements
+// (a third stage of the weights for tiles of 128 and 192; with one 256 takes as long or 3 % longer)
+constexpr int tall_wst(int TM) { return TM <= 3 ? 3 : 2; }
+constexpr int tall_lds_of(int TM) { return (tall_wst(TM) * TALL_W_STAGE + 2 * 64 * TM * 64) * 2; }
+template <int EPI, int TM>
+__global__ void __launch_bounds__(256)
+grouped_tile_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W, int N, int K, void* __restrict__ Cv, int ldc,
+                    const int* __restrict__ order, int top, const int* __restrict__ tile_group,
+                    const int* __restrict__ tile_row0, const int* __restrict__ tile_rows, float limit, float alpha, float shift,
+                    int tiles, int columns) {
+    extern __shared__ __attribute__((aligned(1024))) bf16 tall_lds[];       // [WST][W_STAGE], then [XST][X_STAGE]
+    constexpr int WST = tall_wst(TM), XST = 2, X_STAGE = 64 * TM * 64;
+    bf16* const xlds = tall_lds + WST * TALL_W_STAGE;
+    // (which tile and block of columns: as in the kernel above)
+    const int turn = blockIdx.x / XCDS, run = turn / TILE_RUN * XCDS + blockIdx.x % XCDS;
+    const int tile = run / columns * TILE_RUN + turn % TILE_RUN, column = run % columns;
+    if (tile >= tiles) return;
+    const int group = tile_group[tile];
+    if (group < 0) return;
+    const int row0 = tile_row0[tile], rows = tile_rows[tile];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c32 = lane & 31, g2 = lane >> 5;
+    const int wn = wave >> 1, wm = wave & 1;
+    const int F = N / 2, out_cols = EPI == 2 ? F : N;
+    const int nsteps = K / 64;
+    const size_t wstep = (size_t)(N / 16) * 512;
+    constexpr int WL = 4, XR = 2 * TM, NLW = 2 * WL, NLX = XR, TN = 4;
+    constexpr int LATER = WST == 3 ? NLW : 0;              // loads that may be in flight at the barrier: a later step's weights
+    const bf16* wsrc[WL];
+#pragma unroll
+    for (int i = 0; i < WL; ++i) {
+        const int blk = wave * WL + i;
+        int nb = column * (TALL_BN / 16) + blk, last = N / 16 - 1;
+        if (EPI == 2) nb = column * (TALL_BN / 32) + blk / 2, last = F / 16 - 1;
+        if (nb > last) nb = last;                          // (a block that exists; its sums are not stored)
+        if (EPI == 2 && (blk & 1)) nb += F / 16;
+        wsrc[i] = W + (size_t)group * N * K + ((size_t)nb * 64 + lane) * 8;
+    }
+    const bf16* xsrc[XR];
+#pragma unroll
+    for (int i = 0; i < XR; ++i) {
+        const int r = (wave * XR + i) * 8 + (lane >> 3), m = r < rows ? r : rows - 1;
+        const int src = top > 0 ? order[row0 + m] / top : row0 + m;
+        xsrc[i] = A + (size_t)src * lda + ((lane & 7) ^ ((r >> 1) & 7)) * 8;
+    }
+    // the idx-th load of a step: first the activations of step xstep, then the weights of step w_step
+    auto load_one = [&](int xstep, int xstage, int w_step, int wstage, int idx) {
+        if (idx < NLX) {
+            hb_load_to_lds(xsrc[idx] + (size_t)xstep * 64, xlds + xstage * X_STAGE + (wave * XR + idx) * 512);
+        } else {
+            const int ks = (idx - NLX) / WL, w = (idx - NLX) % WL;
+            hb_load_to_lds(wsrc[w] + ((size_t)w_step * 2 + ks) * wstep,
+                           tall_lds + wstage * TALL_W_STAGE + ks * (TALL_BN / 16) * 512 + (wave * WL + w) * 512);
+        }
+    };
+    hb_f32x16 acc[TN][TM];
+#pragma unroll
+    for (int a = 0; a < TN; ++a)
+#pragma unroll
+        for (int b = 0; b < TM; ++b)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.f;
+    constexpr int NM = 2 * TN * TM, NR = 2 * (TN + TM), SLOTS = NM - 4;
+    const int w_lane = (c32 >> 4) * 512 + (16 * g2 + (lane & 15)) * 8 + wn * 8 * 512;
+    const int x_lane = (wm * TM * 32 + c32) * 64, x_swizzle = (c32 >> 1) & 7;
+    hb_bf16x8 wv[2][2][TN], xv[2][2][TM];                  // [set][k-half][piece]
+    auto mfma_one = [&](int set, int j) {
+        const int h = j / (TN * TM), a = j / TM % TN, b = j % TM;
+        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv[set][h][a], xv[set][h][b], acc[a][b], 0, 0, 0);
+    };
+    auto read_one = [&](int set, int step, int ks, int idx) {
+        const int h = idx / (TN + TM), r = idx % (TN + TM);
+        if (r < TN)
+            wv[set][h][r] = *(const hb_bf16x8*)(tall_lds + (step % WST) * TALL_W_STAGE + ks * (TALL_BN / 16) * 512 + w_lane +
+                                                r * 1024 + h * 256);
+        else
+            xv[set][h][r - TN] = *(const hb_bf16x8*)(xlds + (step % XST) * X_STAGE + x_lane + (r - TN) * 32 * 64 +
+                                                     (((4 * ks + 2 * h + g2) ^ x_swizzle) * 8));
+    };
+    // between the products j and j + 1 of a k-step: nl loads and NR reads, dealt out over the first SLOTS products
+    auto between = [&](int j, int nl, auto&& load, auto&& read) {
+        const int no = nl + NR;
+        const int from = (j < SLOTS ? j : SLOTS) * no / SLOTS, to = (j + 1 < SLOTS ? j + 1 : SLOTS) * no / SLOTS;
+#pragma unroll
+        for (int o = from; o < to; ++o) {
+            const int loads_before = o * nl / no, loads_after = (o + 1) * nl / no;
+            if (loads_after > loads_before) load(loads_before);
+            else read(o - loads_before);
+        }
+    };
+    auto clamp = [&](int step) { return step < nsteps ? step : nsteps - 1; };   // past the end: the last step again
+    // in flight before the loop: steps 0 and 1, and with a third stage step 2 of the weights
+#pragma unroll
+    for (int i = 0; i < NLX + NLW; ++i) load_one(0, 0, 0, 0, i);
+#pragma unroll
+    for (int i = 0; i < NLX + NLW; ++i) load_one(clamp(1), 1, clamp(1), 1, i);
+    if (WST == 3) {
+#pragma unroll
+        for (int i = NLX; i < NLX + NLW; ++i) load_one(0, 0, clamp(2), 2, i);
+    }
+    hb_wait_vmcnt<NLX + NLW + LATER>();
+    hb_workgroup_barrier();
+#pragma unroll
+    for (int i = 0; i < NR; ++i) read_one(0, 0, 0, i);
+    for (int t = 0; t + 1 < nsteps; ++t) {
+#pragma unroll
+        for (int j = 0; j < NM; ++j) {
+            mfma_one(0, j);
+            between(j, 0, [&](int) {}, [&](int i) { read_one(1, t, 1, i); });
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // step t + 1 has landed (in flight at most the weights of a later step) and, after the barrier, nobody reads step t any more
+        hb_wait_vmcnt<LATER>();
+        hb_workgroup_barrier();
+        const int xstep = clamp(t + XST), w_step = clamp(t + WST);
+#pragma unroll
+        for (int j = 0; j < NM; ++j) {
+            mfma_one(1, j);
+            between(j, NLX + NLW, [&](int i) { load_one(xstep, t % XST, w_step, t % WST, i); },
+                    [&](int i) { read_one(0, t + 1, 0, i); });
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    {
+        const int t = nsteps - 1;
+#pragma unroll
+        for (int j = 0; j < NM; ++j) {
+            mfma_one(0, j);
+            between(j, 0, [&](int) {}, [&](int i) { read_one(1, t, 1, i); });
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int j = 0; j < NM; ++j) mfma_one(1, j);
+    }
+    hb_wait_vmcnt<0>();      // the loads past the end (repeats of the last step) have landed too
+    hb_workgroup_barrier();
+    // A lane holds runs of four columns of rows 32 b + c32: through LDS of the wave's own, so that whole rows leave. Rows of CH
+    // 16-byte chunks, chunk c of row r at c ^ (r mod CH).
+    constexpr int COLS = EPI == 2 ? 64 : 128;              // the wave's output columns
+    constexpr int PER = EPI == 0 ? 4 : 8;                  // columns a chunk
+    constexpr int CH = COLS / PER, RPI = 64 / CH;          // chunks of a row, rows an instruction
+    char* const stage = (char*)tall_lds + wave * (32 * CH * 16);       // 32 rows at a time
+    static_assert(4 * 32 * CH * 16 <= tall_lds_of(TM), "the waves' rows fit the LDS");
+    const int rrow = lane / CH, rchunk = lane % CH;
+    const int n = column * (EPI == 2 ? TALL_BN / 2 : TALL_BN) + wn * COLS + rchunk * PER;
+#pragma unroll
+    for (int b = 0; b < TM; ++b) {
+#pragma unroll
+        for (int a = 0; a < TN; ++a)
+#pragma unroll
+            for (int q = 0; q < (EPI == 2 ? 2 : 4); ++q) {
+                hb_f32x4 v;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    v[i] = acc[a][b][4 * q + i];
+                    if (EPI == 2) {                        // rows 0 .. 15 of a piece are gate rows, 16 .. 31 their up rows
+                        const float g = fminf(v[i], limit), u = fminf(fmaxf(acc[a][b][4 * q + 8 + i], -limit), limit);
+                        v[i] = g / (1.0f + expf(-alpha * g)) * (u + shift);
+                    }
+                }
+                const int col = (EPI == 2 ? 16 : 32) * a + 8 * q + 4 * g2;
+                char* const at = stage + (c32 * CH + ((col / PER) ^ (c32 & (CH - 1)))) * 16;
+                if (EPI == 0) {
+                    *(hb_f32x4*)at = v;
+                } else {
+                    bf16 o[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) o[i] = hb_from_float<bf16>(v[i]);
+                    *(uint2*)(at + (col % PER) * 2) = uint2{o[0].bits | ((unsigned)o[1].bits << 16), o[2].bits | ((unsigned)o[3].bits << 16)};
+                }
+            }
+#pragma unroll
+        for (int i = 0; i < 32 / RPI; ++i) {
+            const int row = i * RPI + rrow, m = (wm * TM + b) * 32 + row;
+            const uint4 v = *(const uint4*)(stage + (row * CH + (rchunk ^ (row & (CH - 1)))) * 16);
+            if (m < rows && n < out_cols)                  // (columns come in whole blocks of 16)
+                *(uint4*)((char*)Cv + ((size_t)(row0 + m) * ldc + n) * (EPI == 0 ? 4 : 2)) = v;
+        }
+    }
+}
+
+// hb_grouped_mfma for a list of tiles of up to tile_m rows (128, 192 or 256), K in steps of 64, C in rows of whole 16 bytes.
+extern "C" int hb_grouped_tall(const void* A, int lda, const void* W, int N, int K, void* C, int ldc, int epi, const int* order,
+                               int top, const int* tile_group, const int* tile_row0, const int* tile_rows, int tiles,
+                               int tile_m, float limit, float alpha, float shift, hipStream_t stream) {
+    HB_REQUIRE(N > 0 && K > 0 && K % 64 == 0, "grouped product: K = %d must be a positive multiple of 64", K);
+    HB_REQUIRE(N % 16 == 0 && (epi != 2 || N % 32 == 0), "grouped product: %d weight rows are no whole blocks of 16", N);
+    HB_REQUIRE(epi >= 0 && epi <= 2, "grouped product: unknown epilogue %d", epi);
+    HB_REQUIRE(lda % 8 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0 && ldc % (epi == 0 ? 4 : 8) == 0 && (uintptr_t)C % 16 == 0,
+               "grouped product: operands must lie at multiples of 16 bytes");
+    HB_REQUIRE(tile_m == 128 || tile_m == 192 || tile_m == 256, "grouped product: row tiles of %d", tile_m);
+    HB_REQUIRE(tile_group && tiles > 0 && tiles <= 65535, "grouped product: %d row tiles exceed the grid", tiles);
+    const int out_cols = epi == 2 ? N / 2 : N, per = epi == 2 ? TALL_BN / 2 : TALL_BN, columns = (out_cols + per - 1) / per;
+    const long long runs = (long long)((tiles + TILE_RUN - 1) / TILE_RUN) * columns;
+    const long long blocks = (runs + XCDS - 1) / XCDS * XCDS * TILE_RUN;
+    HB_REQUIRE(blocks < (1ll << 24), "grouped product: %d tiles of %d columns exceed the grid", tiles, out_cols);
+#define HB_TALL(E, TM)                                                                                                      \
+    do {                                                                                                                    \
+        constexpr int lds = tall_lds_of(TM);                                                                                \
+        const hipError_t e_ = hipFuncSetAttribute((const void*)grouped_tile_kernel<E, TM>, hipFuncAttributeMaxDynamicSharedMemorySize, lds); \
+        HB_REQUIRE(e_ == hipSuccess, "grouped product: cannot have %d bytes of LDS: %s", lds, hipGetErrorString(e_));        \
+        grouped_tile_kernel<E, TM><<<(unsigned)blocks, 256, lds, stream>>>((const bf16*)A, lda, (const bf16*)W, N, K, C, ldc, order, top, \
+            tile_group, tile_row0, tile_rows, limit, alpha, shift, tiles, columns);                                          \
+    } while (0)
+#define HB_TALL_OF(E)                       \
+    do {                                    \
+        if (tile_m == 128) HB_TALL(E, 2);   \
+        else if (tile_m == 192) HB_TALL(E, 3); \
+        else HB_TALL(E, 4);                 \
+    } while (0)
+    if (epi == 0) HB_TALL_OF(0);
+    else if (epi == 1) HB_TALL_OF(1);
+    else HB_TALL_OF(2);
+#undef HB_TALL_OF
+#undef HB_TALL
+    HB_CHECK_LAUNCH("grouped_tall");
+    return 0;
 }
 
 // The same for tiles of few rows (decoding), a product bound by the weights' bytes: the four waves of a workgroup take a

@@ -1,5 +1,8 @@
 """Host side of the routed feed-forward's kernels (csrc/moe.hip): routing and grouping, the products
 of an expert's rows with its matrices, the activation, and the weighted sum."""
+import functools
+import math
+
 import torch
 
 from ..errors import BackendError
@@ -7,22 +10,25 @@ from . import lib
 from .ops import _check, _ptr, _stream, dtype_code
 
 TILE_M = 64
+TALL_TILES = (128, 192, 256)           # of the matrix-core product of many rows an expert
 MAX_EXPERTS = 1024
 
 
-def max_tiles(pairs, experts):
+def max_tiles(pairs, experts, tile_m=TILE_M):
     """The length of the list of row tiles for that many (token, expert) pairs."""
-    return (pairs + TILE_M - 1) // TILE_M + experts
+    return (pairs + tile_m - 1) // tile_m + experts
 
 
 class Routing:
     """The buffers that routing fills for a step of T tokens: chosen int32 [T, top], weight f32 [T, top],
     order / row_of int32 [T top], the tiles' lists."""
 
-    def __init__(self, ints, weight, T, E, top, real=None):
-        """real: the first `real` of the E experts have matrices (None: all); the others' output is their input."""
+    def __init__(self, ints, weight, T, E, top, real=None, tile_m=TILE_M):
+        """real: the first `real` of the E experts have matrices (None: all); the others' output is their input.
+        tile_m: the rows of a tile, TILE_M or one of TALL_TILES."""
         self.real = E if real is None else int(real)
-        A, tiles = T * top, max_tiles(T * top, E)
+        self.tile_m = int(tile_m)
+        A, tiles = T * top, max_tiles(T * top, E, self.tile_m)
         need = 3 * A + E + 3 * tiles
         if ints.numel() < need or ints.dtype != torch.int32:
             raise BackendError("routing: the int32 buffer is too small")
@@ -70,13 +76,16 @@ def route(logits, bias, routing, scores=False, groups=1, keep=1, score="sigmoid"
     lib.call("moe", "hb_moe_route", logits.data_ptr(), _ptr(bias), r.chosen.data_ptr(), r.weight.data_ptr(),
              r.counts.data_ptr(), r.order.data_ptr(), r.row_of.data_ptr(), r.tile_expert.data_ptr(),
              r.tile_row0.data_ptr(), r.tile_rows.data_ptr(), r.T, r.E, r.top, r.tiles, ld, 1 if scores else 0,
-             int(groups), int(keep), r.real, 1 if score == "softmax" else 0, int(worth_top), 1 if renorm else 0, _stream())
+             int(groups), int(keep), r.real, 1 if score == "softmax" else 0, int(worth_top), 1 if renorm else 0,
+             r.tile_m, _stream())
 
 
 def gemm_plain(a, w, c, routing, gather):
     """c[row] = a[src(row)] @ w[expert of row]^T for every pair's row; w [E, N, K]; a [T, K] with
     gather (src = the pair's token) or [pairs, K]; c f32 [pairs, N]."""
     r = routing
+    if r.tile_m != TILE_M:
+        raise BackendError(f"moe product: tiles of {r.tile_m} rows")
     E, N, K = w.shape
     _check(w, "w", None, (r.real, N, K))
     _check(a, "a", None, (r.T if gather else r.T * r.top, K))
@@ -132,12 +141,38 @@ EPI_F32, EPI_BF16, EPI_GLU = 0, 1, 2
 # where the line lies; 64 of 1,536 on 4,096: 8 rows 404 / 415, 12 rows 429 / 418, 16 rows 465 / 421; 16 of 512 on 1,024: 16 rows
 # 19 / 32, 64 rows 32 / 37. A head's product of rows that all heads share, 16 of 512 x 128: 16 rows 4.4 / 5.4, 64 rows 5.4 / 8.0.
 FEW_ROWS = 16
+# From so many rows an expert on the kernel of tall tiles runs. Microseconds of a layer's two products by tiles of 64 / of 128 (weights from
+# memory): 32 experts of 768 on 2,048: 32 rows an expert 85 / 81, 50 rows 88 / 83, 64 rows 93 / 86, 96 rows 95 / 87 (gate/up gains, down
+# loses a fifth: its few steps of k do not pay for a tile's start and end); 64 of 1,536 on 4,096: 62 rows 532 / 492; where fewer than
+# half the CUs get a tile (16 of 512 on 1,024: 64 rows 37 / 38) nothing is gained.
+TALL_ROWS = 48
 
 
 def mfma_takes(K, lda, a_group_off=0, N=16):
     """True if the matrix-core kernel takes products of this inner size, layout and N weight rows
     (bfloat16 operands)."""
     return K % 32 == 0 and lda % 8 == 0 and a_group_off % 8 == 0 and N % 16 == 0
+
+
+@functools.lru_cache(maxsize=1024)
+def tile_rows(T, top, routed, experts, hidden, inter):
+    """The rows of a tile for a step of T tokens, each on `top` of `routed` outputs of the router, the first `experts` of which have
+    bfloat16 matrices in the cores' order. Tall tiles from TALL_ROWS rows an expert on, for sizes that they take; of those the one
+    that brings the fewest bytes into a CU: rounds of tiles over the CUs times weight and activation rows of a step (an
+    expert's rows are taken to be spread around their mean as a random choice spreads them)."""
+    rows = T * top / routed
+    if rows < TALL_ROWS or hidden % 64 or inter % 64:
+        return TILE_M
+    columns = -(-2 * inter // 256)
+
+    def workgroups(height):
+        tiles, k = 1.0, 1
+        while k * height < rows + 4.0 * rows ** 0.5:       # more than k tiles: the chance that an expert has more than k height rows
+            tiles += 0.5 * math.erfc((k * height - rows) / (2.0 * rows) ** 0.5)
+            k += 1
+        return experts * tiles * columns
+    fits = [h for h in TALL_TILES if workgroups(h) >= 128]
+    return min(fits, key=lambda h: math.ceil(workgroups(h) / 256 - 0.05) * (256 + h), default=TILE_M)
 
 
 def pack_grouped(w):
@@ -175,8 +210,14 @@ def grouped_mfma(a, lda, a_group_off, w, c, ldc, c_group_off, epi, routing=None,
         rows_a = rows_c = M
         lists = (None, 0, None, None, None, 0, M, G)
         few = M <= FEW_ROWS
+    if routing is not None and routing.tile_m != TILE_M and (K % 64 or a_group_off or c_group_off or ldc % 8):
+        raise BackendError(f"grouped product: tall tiles refuse K = {K} and rows {ldc} apart")
     if (rows_a - 1) * lda + (G - 1) * a_group_off + K > a.numel() or \
             (rows_c - 1) * ldc + (G - 1) * c_group_off + out_cols > c.numel():
         raise BackendError("grouped product: an operand does not hold every row that is addressed")
+    if routing is not None and routing.tile_m != TILE_M:
+        lib.call("moe", "hb_grouped_tall", a.data_ptr(), lda, w.data_ptr(), N, K, c.data_ptr(), ldc, epi, *lists[:6], routing.tile_m, float(limit),
+                 float(alpha), float(shift), _stream())
+        return
     lib.call("moe", "hb_grouped_mfma", a.data_ptr(), lda, a_group_off, w.data_ptr(), N, K, c.data_ptr(), ldc,
              c_group_off, epi, *lists, float(limit), float(alpha), float(shift), 1 if few else 0, _stream())

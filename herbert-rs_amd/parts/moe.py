@@ -137,7 +137,8 @@ class RoutedExperts(Part):
         logits = rt.buffer("moe_logits", (T, self.router_width), torch.float32)
         self.router.forward(y, logits)          # float32 sums of the rows' products with the router's matrix
         routing = moe.Routing(rt.buffer("moe_ints", (moe.Routing.ints_needed(T, E, top),), torch.int32),
-                              rt.buffer("moe_weight", (T, top), torch.float32), T, E, top, real=self.experts)
+                              rt.buffer("moe_weight", (T, top), torch.float32), T, E, top, real=self.experts,
+                              tile_m=moe.tile_rows(T, top, E, self.experts, self.hidden_size, F) if self.cores else moe.TILE_M)
         if self.routing == "scores":
             moe.route(logits, self.router_bias, routing, scores=True, groups=self.groups, keep=self.keep,
                       score=self.scoring, worth_top=self.group_worth, renorm=self.renormalize)

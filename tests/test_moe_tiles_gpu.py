@@ -1,0 +1,57 @@
+"""The experts' products by tall row tiles (csrc/moe.hip, grouped_tile_kernel): every height against float64."""
+import pytest
+import torch
+
+from herbert_rs_amd.kernels import moe
+
+DEV = "cuda"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile_m", moe.TALL_TILES)
+@pytest.mark.parametrize("T,E,real,top,W,F", [(1, 2, 2, 1, 64, 64), (129, 1, 1, 1, 128, 64), (700, 3, 3, 2, 192, 128),
+                                              (900, 5, 4, 2, 320, 448), (513, 2, 2, 1, 1024, 192)])
+def test_tall_tiles(T, E, real, top, W, F, tile_m):
+    """One row, rows that just pass a tile, experts with none, experts without matrices; one step of k and several; columns that
+    fill no block of 256. The sums are float32 over bfloat16 operands: off by at most K roundings of the terms' sizes; the
+    gated unit is rounded to bfloat16 (2^-9, and as much for what its inputs are off)."""
+    g = torch.Generator().manual_seed(T + F)
+    logits = torch.randn(T, E, generator=g)
+    logits[:, 0] += 1.0                                     # (unequal experts)
+    y = torch.randn(T, W, generator=g).bfloat16()
+    gate_up = (torch.randn(real, 2 * F, W, generator=g) * W ** -0.5).bfloat16()
+    down = (torch.randn(real, W, F, generator=g) * F ** -0.5).bfloat16()
+    r = moe.Routing(torch.empty(moe.Routing.ints_needed(T, E, top), dtype=torch.int32, device=DEV),
+                    torch.empty(T, top, device=DEV), T, E, top, real=real, tile_m=tile_m)
+    moe.route(logits.to(DEV), None, r)
+    act = torch.full((T * top, F), 7.0, dtype=torch.bfloat16, device=DEV)
+    out = torch.full((T * top, W), 7.0, device=DEV)
+    moe.grouped_mfma(y.to(DEV), W, 0, moe.pack_grouped(gate_up).to(DEV), act, F, 0, moe.EPI_GLU, r, gather=True, limit=2.0, alpha=1.702)
+    moe.grouped_mfma(act, F, 0, moe.pack_grouped(down).to(DEV), out, W, 0, moe.EPI_F32, r)
+    order, chosen = r.order.cpu().long(), r.chosen.cpu().long()
+    expert = chosen[order]
+    for e in range(E):
+        rows = (expert == e).nonzero().flatten()
+        if not rows.numel():
+            continue
+        if e >= real:                                       # no matrices: nothing is written
+            assert bool((act[rows] == 7.0).all()) and bool((out[rows] == 7.0).all())
+            continue
+        x = y[order[rows] // top].double() @ gate_up[e].double().T
+        gate, up = x[:, :F].clamp(max=2.0), x[:, F:].clamp(-2.0, 2.0)
+        want = gate * torch.sigmoid(1.702 * gate) * (up + 1.0)
+        got = act[rows].cpu().double()
+        assert bool(((got - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all()), e
+        terms = got @ down[e].double().T
+        size = got.abs() @ down[e].double().abs().T
+        assert bool(((out[rows].cpu().double() - terms).abs() <= F * 2.0 ** -24 * size + 1e-30).all()), e
+
+
+def test_tile_heights_by_the_rows_an_expert_has():
+    """Few rows keep the low tiles, as do sizes that the tall ones refuse and steps that would leave most CUs without one."""
+    assert moe.tile_rows(256, 4, 32, 32, 2048, 768) == moe.TILE_M
+    assert moe.tile_rows(2048, 4, 32, 32, 2048, 800) == moe.TILE_M
+    assert moe.tile_rows(1600, 2, 64, 64, 64, 64) == moe.TILE_M
+    assert moe.tile_rows(768, 4, 32, 32, 2048, 768) == 128
+    assert moe.tile_rows(1602, 4, 40, 32, 2048, 768) == 192
+    assert moe.tile_rows(1712, 4, 32, 32, 2048, 768) == 256
