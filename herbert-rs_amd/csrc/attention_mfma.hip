@@ -889,8 +889,28 @@ struct HeadsFusion {
     float eps;
 };
 
+// The LDS of a wave of the decode kernel, bytes: its queries and, FORM_HEADS, a row of the projection and the angles. A wave
+// that is not its workgroup's first later hands it outputs, references and sums in the same place.
+template <int HD, int FUSED>
+__host__ __device__ constexpr int decode_own_lds() {
+    return FUSED == FORM_PLAIN ? 0 : 32 * HD * 2 + (FUSED == FORM_HEADS ? 5 * HD * 4 + HD / 2 * 8 : 0);
+}
+template <int HD, int FUSED>
+__host__ __device__ constexpr int decode_handed_lds() {
+    const int own = decode_own_lds<HD, FUSED>(), handed = HD / 32 * 4 * 64 * 16 + 64 * 8;
+    return own > handed ? own : handed;
+}
+template <int HD, int FUSED>
+constexpr int decode_lds_of(int waves) {      // (four waves of heads of 128: 62 KB)
+    return decode_own_lds<HD, FUSED>() + (waves - 1) * decode_handed_lds<HD, FUSED>();
+}
+
+// A workgroup is a wave, whose partial results a second kernel merges, or the two to four waves that share a sequence
+// and key head: they cut its own pages into equal ranges and the first of them adds up the others' results, in the order of the
+// ranges, out of LDS and stores the output (one sequence of 100 tokens, heads of 128: 10.4 us, 7.5 and 4.0 with the merge and 1.2
+// between the two; 8 of 121 to 309 tokens: 13.0, 9.6 + 4.7 + 1.2).
 template <int HD, int FUSED, bool EXT, int QS = 1>
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(256)
 attn_decode_kernel(const bf16* __restrict__ q, bf16* __restrict__ k_cache, bf16* __restrict__ v_cache,
                    float* __restrict__ partial_o, float* __restrict__ partial_ml,
                    const int* __restrict__ context_lens, const int* __restrict__ slots,
@@ -906,8 +926,9 @@ attn_decode_kernel(const bf16* __restrict__ q, bf16* __restrict__ k_cache, bf16*
     // into, and items from ranges[n_seqs] on are nothing. The partial results are then laid out
     // [head, item]: those of one sequence and head lie side by side.
     const int kvh = blockIdx.y, splits = gridDim.z;
-    const int lane = threadIdx.x, c32 = lane & 31, g2 = lane >> 5;
-    int b = blockIdx.x, split = blockIdx.z;
+    const int lane = threadIdx.x & 63, c32 = lane & 31, g2 = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+    int b = blockIdx.x, split = blockIdx.z + wave;       // (of several waves gridDim.z is 1)
     if (ranges) {
         const int item = blockIdx.z;
         b = 0;                                              // sequences wholly before the item
@@ -928,6 +949,7 @@ attn_decode_kernel(const bf16* __restrict__ q, bf16* __restrict__ k_cache, bf16*
     const PageWalk walk(lo, keep);                   // (EXT: pages are counted along the walk)
     auto page_at = [&](int v) { return EXT ? walk.page(v) : v; };
     const int hp = EXT ? walk.upto(hi / PAGE) : hi / PAGE;       // the page of the new position
+    if (waves > 1) pages_per_split = (hp - (EXT ? 0 : lo / PAGE) + waves) / waves;
     const int first_page = (EXT ? 0 : lo / PAGE) + split * pages_per_split;
     int last_page = first_page + pages_per_split - 1;
     if (last_page > hp) last_page = hp;
@@ -1087,10 +1109,18 @@ attn_decode_kernel(const bf16* __restrict__ q, bf16* __restrict__ k_cache, bf16*
                 _Pragma("unroll") for (int h2 = 0; h2 < 2; ++h2)                             \
                     va[d][kb][h2] = *(const bf16x8*)(vp + (size_t)(d * 32 + c32) * PAGE + kb * 32 + h2 * 16); \
     }
-    __shared__ __attribute__((aligned(16))) bf16 qs[FUSED != FORM_PLAIN ? 32 * HD : 8];
+    extern __shared__ __attribute__((aligned(16))) char decode_lds[];
+    constexpr int HANDED = decode_handed_lds<HD, FUSED>();
+    char* const wave_lds = decode_lds + (wave == 0 ? 0 : decode_own_lds<HD, FUSED>() + (wave - 1) * HANDED);
+    bf16* const qs = (bf16*)wave_lds;
     // (FORM_HEADS: a row of the projection normed, and the angles)
-    __shared__ float hraw[FUSED == FORM_HEADS ? (PRE + 1) * HD : 1];
-    __shared__ float2 hturn[FUSED == FORM_HEADS ? HD / 2 : 1];
+    float* const hraw = (float*)(wave_lds + 32 * HD * 2);
+    float2* const hturn = (float2*)(hraw + (PRE + 1) * HD);
+    // (a wave's own LDS: its accesses happen in their order, only the compiler has to keep it)
+    auto wave_sync = []() __attribute__((always_inline)) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
     auto heads_prologue = [&]() __attribute__((always_inline)) {
         if (lane < HD / 2) hturn[lane] = turn;
         const bool normed = hf.q_norm_w != nullptr;
@@ -1161,7 +1191,7 @@ attn_decode_kernel(const bf16* __restrict__ q, bf16* __restrict__ k_cache, bf16*
         if (writer) lay_key(x[PRE], hraw + PRE * HD);
 #pragma unroll
         for (int it = 0; it < PRE; ++it) lay(x[it], hraw + it * HD);
-        __syncthreads();
+        wave_sync();
         if (writer) {
             const int in_page = hi % PAGE;
             bf16* const kdst = k_cache + (((size_t)new_page * nkv + kvh) * PAGE + in_page) * HD;
@@ -1178,7 +1208,7 @@ attn_decode_kernel(const bf16* __restrict__ q, bf16* __restrict__ k_cache, bf16*
         }
         for (int it0 = 0; it0 < G; it0 += PRE) {
             if (it0 > 0) {
-                __syncthreads();
+                wave_sync();
 #pragma unroll
                 for (int e = 0; e < E; ++e)
 #pragma unroll
@@ -1190,7 +1220,7 @@ attn_decode_kernel(const bf16* __restrict__ q, bf16* __restrict__ k_cache, bf16*
                     for (int e = 0; e < E; ++e) x[it][e] = channel(lane + 64 * e, hf.dim, hq[it][e], hqb[it][e]);
                     lay(x[it], hraw + it * HD);
                 }
-                __syncthreads();
+                wave_sync();
             }
 #pragma unroll
             for (int it = 0; it < PRE; ++it) {
@@ -1285,7 +1315,7 @@ attn_decode_kernel(const bf16* __restrict__ q, bf16* __restrict__ k_cache, bf16*
         }
     }
     if (FUSED != FORM_PLAIN) {
-        __syncthreads();
+        wave_sync();
         const bf16* qrow = qs + (c32 < G ? c32 : G - 1) * HD + g2 * HALF;
 #pragma unroll
         for (int s2 = 0; s2 < HD / 16; ++s2) qreg[s2] = *(const bf16x8*)(qrow + s2 * 8);
@@ -1325,6 +1355,45 @@ attn_decode_kernel(const bf16* __restrict__ q, bf16* __restrict__ k_cache, bf16*
 #undef LOAD_K
 #undef LOAD_V
     l += __shfl_xor(l, 32, 64);
+    if (waves > 1) {
+        constexpr int ML = HD / 32 * 4 * 64 * 16;
+        if (wave > 0) {
+            f32x4* const o = (f32x4*)wave_lds;
+#pragma unroll
+            for (int d = 0; d < HD / 32; ++d)
+#pragma unroll
+                for (int qd = 0; qd < 4; ++qd)
+                    o[(d * 4 + qd) * 64 + lane] = f32x4{oacc[d][4 * qd], oacc[d][4 * qd + 1], oacc[d][4 * qd + 2], oacc[d][4 * qd + 3]};
+            ((float2*)(wave_lds + ML))[lane] = make_float2(m, l);
+        }
+        __syncthreads();
+        if (wave > 0) return;
+        const char* const handed = decode_lds + decode_own_lds<HD, FUSED>();
+        float top = m;
+        for (int w = 0; w < waves - 1; ++w) top = fmaxf(top, ((const float2*)(handed + w * HANDED + ML))[lane].x);
+        // (a range that holds no visible key has a reference of -inf)
+        const float own = m == -INFINITY ? 0.f : fast_exp2((m - top) * c);
+        l *= own;
+#pragma unroll
+        for (int d = 0; d < HD / 32; ++d)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) oacc[d][i] *= own;
+        for (int w = 0; w < waves - 1; ++w) {
+            const f32x4* const o = (const f32x4*)(handed + w * HANDED);
+            const float2 ml = ((const float2*)(handed + w * HANDED + ML))[lane];
+            const float share = ml.x == -INFINITY ? 0.f : fast_exp2((ml.x - top) * c);
+            l = fmaf(share, ml.y, l);
+#pragma unroll
+            for (int d = 0; d < HD / 32; ++d)
+#pragma unroll
+                for (int qd = 0; qd < 4; ++qd) {
+                    const f32x4 v = o[(d * 4 + qd) * 64 + lane];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) oacc[d][4 * qd + e] = fmaf(share, v[e], oacc[d][4 * qd + e]);
+                }
+        }
+        m = top;
+    }
     if (FUSED == FORM_HEADS && out && ho.own) {
         // one range a sequence, the heads leave at their own size (see HeadsOut): maps are neighbouring lanes
         if (sinks) l += sink_share(sinks[head], m, c);
@@ -1555,6 +1624,15 @@ attn_decode_merge_own_kernel(const float* __restrict__ partial_o, const float* _
 // ---------------------------------------------------------------- launchers
 #define LOG2E 1.4426950408889634f
 
+// The waves of a workgroup of the decode kernel that take a sequence's ranges (1: a range is a workgroup, and a second kernel
+// merges them). Where every workgroup has a CU to itself, and four waves make a range longer by a page or two at most: a
+// merge costs a launch and 4 us. More workgroups than CUs leave some CUs with twice the waves of others (384 pairs of two ranges: 58 -> 62 us).
+static int waves_of_ranges(int pairs, int splits, int pages_per_split) {
+    if (pairs > 256) return 1;
+    if (splits <= 4) return splits;
+    return (splits * pages_per_split + 3) / 4 <= pages_per_split + 2 ? 4 : 1;
+}
+
 static int check_extras(const float* rel, int rel_len, int rel_ld, int keep_first, int window, int chunk, float softcap) {
     if (!rel && keep_first == 0) return 0;
     HB_REQUIRE(!rel || (rel_len > 0 && rel_ld >= REL_FRONT + rel_len + REL_BACK), "attention: a table of %d biases in rows of %d", rel_len, rel_ld);
@@ -1686,25 +1764,27 @@ extern "C" int hb_attn_decode_mfma(const void* q, void* k_cache, void* v_cache, 
     HB_REQUIRE(qkv_slices == 1 || (qkv && hd == 128 && (qkv_slices == 2 || qkv_slices == 4 || qkv_slices == 8) &&
                                    slice_stride >= (size_t)B * (nq + 2 * nkv) * hd),
                "attn_decode: %d slices of the projection are not taken here", qkv_slices);
-    dim3 grid(ranges ? 1 : B, nkv, splits);
+    const int waves = ranges ? 1 : waves_of_ranges(B * nkv, splits, pages_per_split);
+    dim3 grid(ranges ? 1 : B, nkv, waves > 1 ? 1 : splits);
     const float c = scale * LOG2E;
     const DecodeFusion fu = {qkv, q_norm_w, k_norm_w, cos_t, sin_t, eps, write_kv, slice_stride, q_temp_coef, q_temp_every};
-    bf16* const direct = splits == 1 ? (bf16*)out : nullptr;      // one range: the kernel writes the output itself
+    bf16* const direct = splits == 1 || waves > 1 ? (bf16*)out : nullptr;      // the kernel writes the output itself
     HB_REQUIRE(qkv || q, "attn_decode: neither q nor the projection rows are given");
     HB_REQUIRE((cos_t == nullptr) == (sin_t == nullptr), "attn_decode: cos and sin tables come together");
 #define DECODE_ARGS(QPTR) QPTR, (bf16*)k_cache, (bf16*)v_cache, partial_o, partial_ml, context_lens, slots, \
                           page_table, max_pages, nq, nkv, c, window, pages_per_split, fu, direct, ranges, B, \
                           direct ? sinks : nullptr, chunk, softcap / scale, ext, HeadsFusion{}, HeadsOut{}
+#define DECODE_LDS(HDV, FORM) decode_lds_of<HDV, FORM>(waves)
 #define LAUNCH_DECODE_FORM(HDV, FORM) do {                                                               \
     if (qkv)                                                                                             \
-        attn_decode_kernel<HDV, FORM_FUSED, FORM><<<grid, 64, 0, stream>>>(DECODE_ARGS(nullptr));              \
+        attn_decode_kernel<HDV, FORM_FUSED, FORM><<<grid, 64 * waves, DECODE_LDS(HDV, FORM_FUSED), stream>>>(DECODE_ARGS(nullptr));              \
     else                                                                                                 \
-        attn_decode_kernel<HDV, FORM_PLAIN, FORM><<<grid, 64, 0, stream>>>(DECODE_ARGS((const bf16*)q));      \
+        attn_decode_kernel<HDV, FORM_PLAIN, FORM><<<grid, 64 * waves, DECODE_LDS(HDV, FORM_PLAIN), stream>>>(DECODE_ARGS((const bf16*)q));      \
     } while (0)
 #define LAUNCH_DECODE(HDV) do { if (extended) LAUNCH_DECODE_FORM(HDV, true); else LAUNCH_DECODE_FORM(HDV, false); } while (0)
 #define LAUNCH_SLICES(QSV) do {                                                                          \
-    if (extended) attn_decode_kernel<128, FORM_FUSED, true, QSV><<<grid, 64, 0, stream>>>(DECODE_ARGS(nullptr)); \
-    else attn_decode_kernel<128, FORM_FUSED, false, QSV><<<grid, 64, 0, stream>>>(DECODE_ARGS(nullptr));       \
+    if (extended) attn_decode_kernel<128, FORM_FUSED, true, QSV><<<grid, 64 * waves, DECODE_LDS(128, FORM_FUSED), stream>>>(DECODE_ARGS(nullptr)); \
+    else attn_decode_kernel<128, FORM_FUSED, false, QSV><<<grid, 64 * waves, DECODE_LDS(128, FORM_FUSED), stream>>>(DECODE_ARGS(nullptr));       \
     } while (0)
     if (qkv_slices == 2) LAUNCH_SLICES(2);
     else if (qkv_slices == 4) LAUNCH_SLICES(4);
@@ -1717,6 +1797,7 @@ extern "C" int hb_attn_decode_mfma(const void* q, void* k_cache, void* v_cache, 
 #undef LAUNCH_DECODE
 #undef LAUNCH_DECODE_FORM
 #undef LAUNCH_SLICES
+#undef DECODE_LDS
 #undef DECODE_ARGS
     HB_CHECK_LAUNCH("attn_decode");
     if (!direct) {
@@ -1765,7 +1846,9 @@ extern "C" int hb_attn_decode_heads_mfma(const float* proj, int ld, int slices, 
                             maps, dim, vdim, map_stride, k_off, v_off, eps};
     const HeadsOut ho = {1, maps, vdim, gate_off < 0 ? nullptr : proj + gate_off, ld, slices, slice_stride, lambda, factor, eps};
     bf16* const direct = splits == 1 ? (bf16*)out : nullptr;
-#define HEADS_GO(HDV, QSV)                                                                                                  attn_decode_kernel<HDV, FORM_HEADS, false, QSV><<<grid, 64, 0, stream>>>(                                                   nullptr, (bf16*)k_cache, (bf16*)v_cache, partial_o, partial_ml, context_lens, slots, page_table, max_pages, nq, nkv, c,         window, pages_per_split, DecodeFusion{}, direct, ranges, B, direct ? sinks : nullptr, chunk, softcap / scale,           AttnExtras{}, hf, ho)
+#define HEADS_GO(HDV, QSV)                                                                                              \
+    attn_decode_kernel<HDV, FORM_HEADS, false, QSV><<<grid, 64, decode_lds_of<HDV, FORM_HEADS>(1), stream>>>( \
+        nullptr, (bf16*)k_cache, (bf16*)v_cache, partial_o, partial_ml, context_lens, slots, page_table, max_pages, nq, nkv, c,         window, pages_per_split, DecodeFusion{}, direct, ranges, B, direct ? sinks : nullptr, chunk, softcap / scale,           AttnExtras{}, hf, ho)
     if (slices == 2) HEADS_GO(128, 2);
     else if (slices == 4) HEADS_GO(128, 4);
     else if (slices == 8) HEADS_GO(128, 8);
