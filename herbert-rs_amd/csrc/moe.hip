@@ -168,9 +168,10 @@ moe_route_kernel(const float* __restrict__ logits, int ld, const float* __restri
 __global__ void __launch_bounds__(1024)
 moe_place_kernel(const int* __restrict__ chosen, int* __restrict__ counts, int* __restrict__ order,
                  int* __restrict__ row_of, int* __restrict__ tile_expert, int* __restrict__ tile_row0,
-                 int* __restrict__ tile_rows, int A, int E, int max_tiles, int real, int tile_m) {
+                 int* __restrict__ tile_rows, int A, int E, int max_tiles, int real, int* __restrict__ tall,
+                 int tall_m, int max_tall) {
     __shared__ int hist[HB_WAVE * MOE_MAX_E_PER_LANE];
-    __shared__ int wave_n[16], firsts[16], tiles[16];
+    __shared__ int wave_n[16], firsts[16], tiles[16], talls[16];
     const int e = blockIdx.x;
     const int lane = threadIdx.x & (HB_WAVE - 1), wave = threadIdx.x / HB_WAVE;
     const int run = ((A + 1023) / 1024) * HB_WAVE;       // pairs of a wave
@@ -191,33 +192,42 @@ moe_place_kernel(const int* __restrict__ chosen, int* __restrict__ counts, int* 
     if (lane == 0) wave_n[wave] = hits;
     __syncthreads();
     const int before = (int)threadIdx.x < min(e, E) ? hist[threadIdx.x] : 0;       // (E is at most the workgroup's threads)
-    int first = before, tile0 = (before + tile_m - 1) / tile_m;
+    int first = before, tile0 = (before + MOE_TILE_M - 1) / MOE_TILE_M, tall0 = tall_m ? (before + tall_m - 1) / tall_m : 0;
 #pragma unroll
     for (int off = HB_WAVE / 2; off > 0; off >>= 1) {
         first += __shfl_xor(first, off, HB_WAVE);
         tile0 += __shfl_xor(tile0, off, HB_WAVE);
+        tall0 += __shfl_xor(tall0, off, HB_WAVE);
     }
     if (lane == 0) {
         firsts[wave] = first;
         tiles[wave] = tile0;
+        talls[wave] = tall0;
     }
     __syncthreads();
-    first = tile0 = 0;
+    first = tile0 = tall0 = 0;
 #pragma unroll
     for (int w = 0; w < 16; ++w) {
         first += firsts[w];
         tile0 += tiles[w];
+        tall0 += talls[w];
     }
     if (e == E) {
         for (int i = tile0 + threadIdx.x; i < max_tiles; i += 1024) tile_expert[i] = -1;
+        for (int i = tall0 + threadIdx.x; tall_m && i < max_tall; i += 1024) tall[i] = -1;
         return;
     }
     const int count = hist[e];
     if (threadIdx.x == 0) counts[e] = count;
-    for (int i = threadIdx.x; i * tile_m < count; i += 1024) {
+    for (int i = threadIdx.x; i * MOE_TILE_M < count; i += 1024) {
         tile_expert[tile0 + i] = e < real ? e : -1;
-        tile_row0[tile0 + i] = first + i * tile_m;
-        tile_rows[tile0 + i] = count - i * tile_m < tile_m ? count - i * tile_m : tile_m;
+        tile_row0[tile0 + i] = first + i * MOE_TILE_M;
+        tile_rows[tile0 + i] = count - i * MOE_TILE_M < MOE_TILE_M ? count - i * MOE_TILE_M : MOE_TILE_M;
+    }
+    for (int i = threadIdx.x; tall_m && i * tall_m < count; i += 1024) {
+        tall[tall0 + i] = e < real ? e : -1;
+        tall[max_tall + tall0 + i] = first + i * tall_m;
+        tall[2 * max_tall + tall0 + i] = count - i * tall_m < tall_m ? count - i * tall_m : tall_m;
     }
     if (hits == 0) return;
     int row = first;
@@ -305,14 +315,16 @@ moe_route_few_kernel(const float* __restrict__ logits, int ld, const float* __re
     }
 }
 
+// tall [3, max_tall] (or null): the same list for tiles of tall_m rows, an expert, a first row and the rows of each.
 // logits' rows are ld floats apart (their first E count).
 // by_scores 0: the largest logits (+ bias), weights a softmax over the chosen.
 // by_scores 1: sigmoid scores, `bias` is the correction of the choice, n_groups groups of which `keep` count.
 extern "C" int hb_moe_route(const float* logits, const float* bias, int* chosen, float* weight, int* counts,
                             int* order, int* row_of, int* tile_expert, int* tile_row0, int* tile_rows, int T, int E,
                             int top, int max_tiles, int ld, int by_scores, int n_groups, int keep, int real,
-                            int softmax_scores, int worth_top, int renorm, int tile_m, hipStream_t stream) {
-    HB_REQUIRE(tile_m == MOE_TILE_M || tile_m == 128 || tile_m == 192 || tile_m == 256, "moe: row tiles of %d", tile_m);
+                            int softmax_scores, int worth_top, int renorm, int* tall, int tall_m, int max_tall,
+                            hipStream_t stream) {
+    HB_REQUIRE(tall_m == 0 || ((tall_m == 128 || tall_m == 192 || tall_m == 256) && tall), "moe: row tiles of %d", tall_m);
     HB_REQUIRE(ld >= E, "moe: logits rows %d apart for %d experts", ld, E);
     HB_REQUIRE(!by_scores || (n_groups > 0 && E % n_groups == 0 && keep > 0 && keep <= n_groups &&
                               top <= keep * (E / n_groups)),
@@ -322,9 +334,10 @@ extern "C" int hb_moe_route(const float* logits, const float* bias, int* chosen,
     HB_REQUIRE(E <= HB_WAVE * MOE_MAX_E_PER_LANE, "moe: %d experts, the router takes up to %d", E, HB_WAVE * MOE_MAX_E_PER_LANE);
     const long long A = (long long)T * top;
     HB_REQUIRE(A < (1ll << 30), "moe: too many (token, expert) pairs");
-    HB_REQUIRE(max_tiles >= (A + tile_m - 1) / tile_m + E, "moe: the tile list is too short");
+    HB_REQUIRE(max_tiles >= (A + MOE_TILE_M - 1) / MOE_TILE_M + E && (tall_m == 0 || max_tall >= (A + tall_m - 1) / tall_m + E),
+               "moe: the tile list is too short");
     const RouteForm form = {by_scores, n_groups, keep, softmax_scores, worth_top, renorm};
-    if (T <= FEW_TOKENS && A <= FEW_PAIRS && E <= HB_WAVE * 4 && tile_m == MOE_TILE_M) {
+    if (T <= FEW_TOKENS && A <= FEW_PAIRS && E <= HB_WAVE * 4 && tall_m == 0) {
 #define HB_FEW(PER)                                                                                                      \
     moe_route_few_kernel<PER><<<1, HB_WAVE * (T < 4 ? 4 : T), 0, stream>>>(logits, ld, bias, chosen, weight, counts, order, \
         row_of, tile_expert, tile_row0, tile_rows, T, E, top, max_tiles, real, form)
@@ -342,7 +355,7 @@ extern "C" int hb_moe_route(const float* logits, const float* bias, int* chosen,
     else HB_ROUTE(MOE_MAX_E_PER_LANE);
 #undef HB_ROUTE
     HB_CHECK_LAUNCH("moe_route");
-    moe_place_kernel<<<E + 1, 1024, 0, stream>>>(chosen, counts, order, row_of, tile_expert, tile_row0, tile_rows, (int)A, E, max_tiles, real, tile_m);
+    moe_place_kernel<<<E + 1, 1024, 0, stream>>>(chosen, counts, order, row_of, tile_expert, tile_row0, tile_rows, (int)A, E, max_tiles, real, tall, tall_m, max_tall);
     HB_CHECK_LAUNCH("moe_place");
     return 0;
 }
@@ -735,9 +748,9 @@ grouped_mfma_kernel(const bf16* __restrict__ A, int lda, size_t a_group_off, con
 // waited for by count before a bare barrier. There is no branch in the main loop (the last step is peeled off); reads and loads are dealt
 // out between the products, the reads of a k-step during the products of the one before. An activation row is 128 bytes, its 16-byte
 // chunk c at chunk c ^ ((row >> 1) & 7); a block of 16 weight rows and 32 k is 1 KB as packed. K in steps of 64.
-// Both products of a layer, 32 experts of 768 on 2,048, weights from memory (40 and 20 us at the rate of a large copy), by tiles of 64 and
-// by the tile that tile_rows of moe.py takes: 2,048 tokens, four experts each 197 us, 158 (128 rows); 1,712 154, 124 (256); 1,282 149, 105
-// (192); 512 93, 86 (128). 64 experts of 1,536 on 4,096, 2,500 tokens: 781, 571 (192).
+// Gate/up of 32 experts of 768 on 2,048, weights from memory (40 us at the rate of a large copy), by tiles of 64 and by the tile that
+// tall_rows of moe.py takes: 2,048 tokens, four experts each, 127 us, 90 (128 rows); 1,712 103, 76 (256); 1,282 101, 60 (192); 512 63, 49
+// (128). 64 experts of 1,536 on 4,096, 2,500 tokens: 522, 353 (192).
 typedef float hb_f32x16 __attribute__((ext_vector_type(16)));
 #define TALL_BN 256
 #define TALL_W_STAGE (TALL_BN * 64)          // elements

@@ -14,22 +14,23 @@ TALL_TILES = (128, 192, 256)           # of the matrix-core product of many rows
 MAX_EXPERTS = 1024
 
 
-def max_tiles(pairs, experts, tile_m=TILE_M):
+def max_tiles(pairs, experts, rows=TILE_M):
     """The length of the list of row tiles for that many (token, expert) pairs."""
-    return (pairs + tile_m - 1) // tile_m + experts
+    return (pairs + rows - 1) // rows + experts
 
 
 class Routing:
     """The buffers that routing fills for a step of T tokens: chosen int32 [T, top], weight f32 [T, top],
     order / row_of int32 [T top], the tiles' lists."""
 
-    def __init__(self, ints, weight, T, E, top, real=None, tile_m=TILE_M):
+    def __init__(self, ints, weight, T, E, top, real=None, tall=0):
         """real: the first `real` of the E experts have matrices (None: all); the others' output is their input.
-        tile_m: the rows of a tile, TILE_M or one of TALL_TILES."""
+        tall: 0, or one of TALL_TILES: a second list, of tiles of that many rows."""
         self.real = E if real is None else int(real)
-        self.tile_m = int(tile_m)
-        A, tiles = T * top, max_tiles(T * top, E, self.tile_m)
-        need = 3 * A + E + 3 * tiles
+        self.tall = int(tall)
+        A, tiles = T * top, max_tiles(T * top, E)
+        self.tall_tiles = max_tiles(A, E, self.tall) if self.tall else 0
+        need = 3 * A + E + 3 * tiles + 3 * self.tall_tiles
         if ints.numel() < need or ints.dtype != torch.int32:
             raise BackendError("routing: the int32 buffer is too small")
         self.T, self.E, self.top, self.tiles = T, E, top, tiles
@@ -41,11 +42,12 @@ class Routing:
         self.tile_expert, o = ints[o:o + tiles], o + tiles
         self.tile_row0, o = ints[o:o + tiles], o + tiles
         self.tile_rows, o = ints[o:o + tiles], o + tiles
+        self.tall_list = ints[o:o + 3 * self.tall_tiles].view(3, -1) if self.tall else None
         self.weight = weight
 
     @staticmethod
-    def ints_needed(T, E, top):
-        return 3 * T * top + E + 3 * max_tiles(T * top, E)
+    def ints_needed(T, E, top, tall=0):
+        return 3 * T * top + E + 3 * max_tiles(T * top, E) + (3 * max_tiles(T * top, E, tall) if tall else 0)
 
 
 def route(logits, bias, routing, scores=False, groups=1, keep=1, score="sigmoid", worth_top=2, renorm=True):
@@ -77,15 +79,13 @@ def route(logits, bias, routing, scores=False, groups=1, keep=1, score="sigmoid"
              r.counts.data_ptr(), r.order.data_ptr(), r.row_of.data_ptr(), r.tile_expert.data_ptr(),
              r.tile_row0.data_ptr(), r.tile_rows.data_ptr(), r.T, r.E, r.top, r.tiles, ld, 1 if scores else 0,
              int(groups), int(keep), r.real, 1 if score == "softmax" else 0, int(worth_top), 1 if renorm else 0,
-             r.tile_m, _stream())
+             _ptr(r.tall_list), r.tall, r.tall_tiles, _stream())
 
 
 def gemm_plain(a, w, c, routing, gather):
     """c[row] = a[src(row)] @ w[expert of row]^T for every pair's row; w [E, N, K]; a [T, K] with
     gather (src = the pair's token) or [pairs, K]; c f32 [pairs, N]."""
     r = routing
-    if r.tile_m != TILE_M:
-        raise BackendError(f"moe product: tiles of {r.tile_m} rows")
     E, N, K = w.shape
     _check(w, "w", None, (r.real, N, K))
     _check(a, "a", None, (r.T if gather else r.T * r.top, K))
@@ -141,10 +141,13 @@ EPI_F32, EPI_BF16, EPI_GLU = 0, 1, 2
 # where the line lies; 64 of 1,536 on 4,096: 8 rows 404 / 415, 12 rows 429 / 418, 16 rows 465 / 421; 16 of 512 on 1,024: 16 rows
 # 19 / 32, 64 rows 32 / 37. A head's product of rows that all heads share, 16 of 512 x 128: 16 rows 4.4 / 5.4, 64 rows 5.4 / 8.0.
 FEW_ROWS = 16
-# From so many rows an expert on the kernel of tall tiles runs. Microseconds of a layer's two products by tiles of 64 / of 128 (weights from
-# memory): 32 experts of 768 on 2,048: 32 rows an expert 85 / 81, 50 rows 88 / 83, 64 rows 93 / 86, 96 rows 95 / 87 (gate/up gains, down
-# loses a fifth: its few steps of k do not pay for a tile's start and end); 64 of 1,536 on 4,096: 62 rows 532 / 492; where fewer than
-# half the CUs get a tile (16 of 512 on 1,024: 64 rows 37 / 38) nothing is gained.
+# From so many rows an expert on the kernel of tall tiles takes gate/up. Microseconds by tiles of 64 / of 128 (weights from memory): 32
+# experts of 768 on 2,048: 32 rows an expert 58 / 48, 50 rows 59 / 48, 64 rows 63 / 49, 96 rows 63 / 50; 64 of 1,536 on 4,096: 62 rows
+# 363 / 310; where fewer than half the CUs get a tile (16 of 512 on 1,024: 64 rows 24 / 23) nothing is gained. A tile's start and
+# end weigh as much as eight of its steps of 64 k, so down, whose k is short, takes tall tiles from DOWN_STEPS steps and DOWN_ROWS rows on:
+# 12 steps 52 / 67 in a model whose experts are unequally busy (214 rows on average), 68 / 67 (256 rows); 24 steps, 156 rows 259 / 218, 62
+# rows 169 / 182.
+DOWN_STEPS, DOWN_ROWS = 16, 128
 TALL_ROWS = 48
 
 
@@ -155,14 +158,14 @@ def mfma_takes(K, lda, a_group_off=0, N=16):
 
 
 @functools.lru_cache(maxsize=1024)
-def tile_rows(T, top, routed, experts, hidden, inter):
-    """The rows of a tile for a step of T tokens, each on `top` of `routed` outputs of the router, the first `experts` of which have
+def tall_rows(T, top, routed, experts, hidden, inter):
+    """The rows of a tall tile (0: none) for a step of T tokens, each on `top` of `routed` outputs of the router, the first `experts` of which have
     bfloat16 matrices in the cores' order. Tall tiles from TALL_ROWS rows an expert on, for sizes that they take; of those the one
     that brings the fewest bytes into a CU: rounds of tiles over the CUs times weight and activation rows of a step (an
     expert's rows are taken to be spread around their mean as a random choice spreads them)."""
     rows = T * top / routed
     if rows < TALL_ROWS or hidden % 64 or inter % 64:
-        return TILE_M
+        return 0
     columns = -(-2 * inter // 256)
 
     def workgroups(height):
@@ -172,7 +175,7 @@ def tile_rows(T, top, routed, experts, hidden, inter):
             k += 1
         return experts * tiles * columns
     fits = [h for h in TALL_TILES if workgroups(h) >= 128]
-    return min(fits, key=lambda h: math.ceil(workgroups(h) / 256 - 0.05) * (256 + h), default=TILE_M)
+    return min(fits, key=lambda h: math.ceil(workgroups(h) / 256 - 0.05) * (256 + h), default=0)
 
 
 def pack_grouped(w):
@@ -185,12 +188,12 @@ def pack_grouped(w):
 
 
 def grouped_mfma(a, lda, a_group_off, w, c, ldc, c_group_off, epi, routing=None, gather=False, M=0, limit=0.0,
-                 alpha=0.0, shift=1.0):
+                 alpha=0.0, shift=1.0, tall=False):
     """Group g: C[rows, g * c_group_off + n] = sum_k A[src(row), g * a_group_off + k] * w[g][n, k], bfloat16
     operands, float32 sums; w as pack_grouped gives it. With `routing` the rows are the (token, expert) pairs in their experts' order
     (gather: A's rows are the tokens'); without, every group takes the same M rows. epi: EPI_F32 / EPI_BF16
     store C in that type; EPI_GLU: w[g] is [2 F, K] (gate rows, then up rows) and C bfloat16 [*, F] receives
-    the experts' activation with `limit`, `alpha` and `shift` (see activate)."""
+    the experts' activation with `limit`, `alpha` and `shift` (see activate). tall: by the routing's list of tall tiles."""
     G, N, K = w.shape
     _check(a, "a", torch.bfloat16)
     _check(w, "w", torch.bfloat16, (G, N, K))
@@ -210,13 +213,14 @@ def grouped_mfma(a, lda, a_group_off, w, c, ldc, c_group_off, epi, routing=None,
         rows_a = rows_c = M
         lists = (None, 0, None, None, None, 0, M, G)
         few = M <= FEW_ROWS
-    if routing is not None and routing.tile_m != TILE_M and (K % 64 or a_group_off or c_group_off or ldc % 8):
-        raise BackendError(f"grouped product: tall tiles refuse K = {K} and rows {ldc} apart")
+    if tall and (routing is None or not routing.tall or K % 64 or a_group_off or c_group_off or ldc % 8):
+        raise BackendError(f"grouped product: tall tiles refuse K = {K}, rows {ldc} apart or a routing without a list of them")
     if (rows_a - 1) * lda + (G - 1) * a_group_off + K > a.numel() or \
             (rows_c - 1) * ldc + (G - 1) * c_group_off + out_cols > c.numel():
         raise BackendError("grouped product: an operand does not hold every row that is addressed")
-    if routing is not None and routing.tile_m != TILE_M:
-        lib.call("moe", "hb_grouped_tall", a.data_ptr(), lda, w.data_ptr(), N, K, c.data_ptr(), ldc, epi, *lists[:6], routing.tile_m, float(limit),
+    if tall:
+        lib.call("moe", "hb_grouped_tall", a.data_ptr(), lda, w.data_ptr(), N, K, c.data_ptr(), ldc, epi, r.order.data_ptr(),
+                 r.top if gather else 0, *(part.data_ptr() for part in r.tall_list), r.tall_tiles, r.tall, float(limit),
                  float(alpha), float(shift), _stream())
         return
     lib.call("moe", "hb_grouped_mfma", a.data_ptr(), lda, a_group_off, w.data_ptr(), N, K, c.data_ptr(), ldc,

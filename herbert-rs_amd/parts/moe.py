@@ -136,9 +136,9 @@ class RoutedExperts(Part):
         T, E, top, F = y.shape[0], self.routed, self.top, self.inter
         logits = rt.buffer("moe_logits", (T, self.router_width), torch.float32)
         self.router.forward(y, logits)          # float32 sums of the rows' products with the router's matrix
-        routing = moe.Routing(rt.buffer("moe_ints", (moe.Routing.ints_needed(T, E, top),), torch.int32),
-                              rt.buffer("moe_weight", (T, top), torch.float32), T, E, top, real=self.experts,
-                              tile_m=moe.tile_rows(T, top, E, self.experts, self.hidden_size, F) if self.cores else moe.TILE_M)
+        tall = moe.tall_rows(T, top, E, self.experts, self.hidden_size, F) if self.cores else 0
+        routing = moe.Routing(rt.buffer("moe_ints", (moe.Routing.ints_needed(T, E, top, tall),), torch.int32),
+                              rt.buffer("moe_weight", (T, top), torch.float32), T, E, top, real=self.experts, tall=tall)
         if self.routing == "scores":
             moe.route(logits, self.router_bias, routing, scores=True, groups=self.groups, keep=self.keep,
                       score=self.scoring, worth_top=self.group_worth, renorm=self.renormalize)
@@ -161,8 +161,9 @@ class RoutedExperts(Part):
         if self.cores:
             # matrix cores; the activation is the first product's epilogue
             moe.grouped_mfma(y, self.hidden_size, 0, self.gate_up, act, F, 0, moe.EPI_GLU, routing, gather=True,
-                             limit=self.limit, alpha=self.alpha, shift=self.shift)
-            moe.grouped_mfma(act, F, 0, self.down, out, self.hidden_size, 0, moe.EPI_F32, routing)
+                             limit=self.limit, alpha=self.alpha, shift=self.shift, tall=tall > 0)
+            moe.grouped_mfma(act, F, 0, self.down, out, self.hidden_size, 0, moe.EPI_F32, routing,
+                             tall=tall > 0 and F >= 64 * moe.DOWN_STEPS and T * top >= moe.DOWN_ROWS * E)
         else:
             gu = rt.buffer("moe_gate_up", (T * top, 2 * F), torch.float32)
             moe.gemm_plain(y, self.gate_up, gu, routing, gather=True)

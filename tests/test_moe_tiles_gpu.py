@@ -21,13 +21,20 @@ def test_tall_tiles(T, E, real, top, W, F, tile_m):
     y = torch.randn(T, W, generator=g).bfloat16()
     gate_up = (torch.randn(real, 2 * F, W, generator=g) * W ** -0.5).bfloat16()
     down = (torch.randn(real, W, F, generator=g) * F ** -0.5).bfloat16()
-    r = moe.Routing(torch.empty(moe.Routing.ints_needed(T, E, top), dtype=torch.int32, device=DEV),
-                    torch.empty(T, top, device=DEV), T, E, top, real=real, tile_m=tile_m)
+    r = moe.Routing(torch.empty(moe.Routing.ints_needed(T, E, top, tile_m), dtype=torch.int32, device=DEV),
+                    torch.empty(T, top, device=DEV), T, E, top, real=real, tall=tile_m)
     moe.route(logits.to(DEV), None, r)
     act = torch.full((T * top, F), 7.0, dtype=torch.bfloat16, device=DEV)
     out = torch.full((T * top, W), 7.0, device=DEV)
-    moe.grouped_mfma(y.to(DEV), W, 0, moe.pack_grouped(gate_up).to(DEV), act, F, 0, moe.EPI_GLU, r, gather=True, limit=2.0, alpha=1.702)
-    moe.grouped_mfma(act, F, 0, moe.pack_grouped(down).to(DEV), out, W, 0, moe.EPI_F32, r)
+    moe.grouped_mfma(y.to(DEV), W, 0, moe.pack_grouped(gate_up).to(DEV), act, F, 0, moe.EPI_GLU, r, gather=True, limit=2.0, alpha=1.702,
+                     tall=True)
+    moe.grouped_mfma(act, F, 0, moe.pack_grouped(down).to(DEV), out, W, 0, moe.EPI_F32, r, tall=True)
+    counts, tiles, row = r.counts.tolist(), [], 0
+    for e, c in enumerate(counts):
+        tiles += [(e if e < real else -1, row + i, min(tile_m, c - i)) for i in range(0, c, tile_m)]
+        row += c
+    got = list(zip(*r.tall_list.tolist()))
+    assert got[:len(tiles)] == tiles and all(t[0] == -1 for t in got[len(tiles):])
     order, chosen = r.order.cpu().long(), r.chosen.cpu().long()
     expert = chosen[order]
     for e in range(E):
@@ -49,9 +56,9 @@ def test_tall_tiles(T, E, real, top, W, F, tile_m):
 
 def test_tile_heights_by_the_rows_an_expert_has():
     """Few rows keep the low tiles, as do sizes that the tall ones refuse and steps that would leave most CUs without one."""
-    assert moe.tile_rows(256, 4, 32, 32, 2048, 768) == moe.TILE_M
-    assert moe.tile_rows(2048, 4, 32, 32, 2048, 800) == moe.TILE_M
-    assert moe.tile_rows(1600, 2, 64, 64, 64, 64) == moe.TILE_M
-    assert moe.tile_rows(768, 4, 32, 32, 2048, 768) == 128
-    assert moe.tile_rows(1602, 4, 40, 32, 2048, 768) == 192
-    assert moe.tile_rows(1712, 4, 32, 32, 2048, 768) == 256
+    assert moe.tall_rows(256, 4, 32, 32, 2048, 768) == 0
+    assert moe.tall_rows(2048, 4, 32, 32, 2048, 800) == 0
+    assert moe.tall_rows(1600, 2, 64, 64, 64, 64) == 0
+    assert moe.tall_rows(768, 4, 32, 32, 2048, 768) == 128
+    assert moe.tall_rows(1602, 4, 40, 32, 2048, 768) == 192
+    assert moe.tall_rows(1712, 4, 32, 32, 2048, 768) == 256
