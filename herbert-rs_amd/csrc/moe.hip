@@ -169,7 +169,7 @@ __global__ void __launch_bounds__(1024)
 moe_place_kernel(const int* __restrict__ chosen, int* __restrict__ counts, int* __restrict__ order,
                  int* __restrict__ row_of, int* __restrict__ tile_expert, int* __restrict__ tile_row0,
                  int* __restrict__ tile_rows, int A, int E, int max_tiles, int real, int* __restrict__ tall,
-                 int tall_m, int max_tall) {
+                 int tall_m, int max_tall, int top, int shared_rows) {
     __shared__ int hist[HB_WAVE * MOE_MAX_E_PER_LANE];
     __shared__ int wave_n[16], firsts[16], tiles[16], talls[16];
     const int e = blockIdx.x;
@@ -213,8 +213,18 @@ moe_place_kernel(const int* __restrict__ chosen, int* __restrict__ counts, int* 
         tall0 += talls[w];
     }
     if (e == E) {
-        for (int i = tile0 + threadIdx.x; i < max_tiles; i += 1024) tile_expert[i] = -1;
-        for (int i = tall0 + threadIdx.x; tall_m && i < max_tall; i += 1024) tall[i] = -1;
+        // (behind all pairs a row a token for the expert that every token takes, the matrices after the others')
+        for (int t = threadIdx.x; t < shared_rows; t += 1024) order[A + t] = t * top;
+        for (int i = threadIdx.x; tile0 + i < max_tiles; i += 1024) {
+            const int left = shared_rows - i * MOE_TILE_M;
+            tile_expert[tile0 + i] = left > 0 ? real : -1;
+            if (left > 0) tile_row0[tile0 + i] = A + i * MOE_TILE_M, tile_rows[tile0 + i] = min(left, MOE_TILE_M);
+        }
+        for (int i = threadIdx.x; tall_m && tall0 + i < max_tall; i += 1024) {
+            const int left = shared_rows - i * tall_m;
+            tall[tall0 + i] = left > 0 ? real : -1;
+            if (left > 0) tall[max_tall + tall0 + i] = A + i * tall_m, tall[2 * max_tall + tall0 + i] = min(left, tall_m);
+        }
         return;
     }
     const int count = hist[e];
@@ -260,7 +270,7 @@ __global__ void __launch_bounds__(HB_WAVE * FEW_TOKENS)
 moe_route_few_kernel(const float* __restrict__ logits, int ld, const float* __restrict__ bias, int* __restrict__ chosen,
                      float* __restrict__ weight, int* __restrict__ counts, int* __restrict__ order, int* __restrict__ row_of,
                      int* __restrict__ tile_expert, int* __restrict__ tile_row0, int* __restrict__ tile_rows, int T, int E,
-                     int top, int max_tiles, int real, RouteForm form) {
+                     int top, int max_tiles, int real, int shared_rows, RouteForm form) {
     __shared__ float a[FEW_TOKENS][HB_WAVE * PER], b[FEW_TOKENS][HB_WAVE * PER];
     __shared__ __attribute__((aligned(16))) int pair_expert[FEW_PAIRS + 4];
     __shared__ int hist[HB_WAVE * PER];
@@ -302,7 +312,13 @@ moe_route_few_kernel(const float* __restrict__ logits, int ld, const float* __re
             tile_rows[tile0 + i] = min(n - i * MOE_TILE_M, MOE_TILE_M);
         }
     }
-    for (int i = (int)(start[HB_WAVE * PER] >> 16) + threadIdx.x; i < max_tiles; i += threads) tile_expert[i] = -1;
+    const int used = start[HB_WAVE * PER] >> 16;
+    for (int i = used + threadIdx.x; i < max_tiles; i += threads) {
+        const bool own = i == used && shared_rows > 0;     // (the expert that every token takes: up to FEW_TOKENS rows)
+        tile_expert[i] = own ? real : -1;
+        if (own) tile_row0[i] = A, tile_rows[i] = shared_rows;
+    }
+    if ((int)threadIdx.x < shared_rows) order[A + threadIdx.x] = threadIdx.x * top;
     for (int p = threadIdx.x; p < A; p += threads) {
         const int e = pair_expert[p];
         int r = start[e] & 0xffff;
@@ -316,6 +332,8 @@ moe_route_few_kernel(const float* __restrict__ logits, int ld, const float* __re
 }
 
 // tall [3, max_tall] (or null): the same list for tiles of tall_m rows, an expert, a first row and the rows of each.
+// shared_rows T (or 0): after the pairs' rows, and after their tiles in either list, come a row a token of one more expert, number
+// `real`, that every token takes: order there is token times top.
 // logits' rows are ld floats apart (their first E count).
 // by_scores 0: the largest logits (+ bias), weights a softmax over the chosen.
 // by_scores 1: sigmoid scores, `bias` is the correction of the choice, n_groups groups of which `keep` count.
@@ -323,7 +341,7 @@ extern "C" int hb_moe_route(const float* logits, const float* bias, int* chosen,
                             int* order, int* row_of, int* tile_expert, int* tile_row0, int* tile_rows, int T, int E,
                             int top, int max_tiles, int ld, int by_scores, int n_groups, int keep, int real,
                             int softmax_scores, int worth_top, int renorm, int* tall, int tall_m, int max_tall,
-                            hipStream_t stream) {
+                            int shared_rows, hipStream_t stream) {
     HB_REQUIRE(tall_m == 0 || ((tall_m == 128 || tall_m == 192 || tall_m == 256) && tall), "moe: row tiles of %d", tall_m);
     HB_REQUIRE(ld >= E, "moe: logits rows %d apart for %d experts", ld, E);
     HB_REQUIRE(!by_scores || (n_groups > 0 && E % n_groups == 0 && keep > 0 && keep <= n_groups &&
@@ -334,13 +352,16 @@ extern "C" int hb_moe_route(const float* logits, const float* bias, int* chosen,
     HB_REQUIRE(E <= HB_WAVE * MOE_MAX_E_PER_LANE, "moe: %d experts, the router takes up to %d", E, HB_WAVE * MOE_MAX_E_PER_LANE);
     const long long A = (long long)T * top;
     HB_REQUIRE(A < (1ll << 30), "moe: too many (token, expert) pairs");
-    HB_REQUIRE(max_tiles >= (A + MOE_TILE_M - 1) / MOE_TILE_M + E && (tall_m == 0 || max_tall >= (A + tall_m - 1) / tall_m + E),
+    HB_REQUIRE(shared_rows == 0 || (shared_rows == T && real == E), "moe: %d rows of a shared expert for %d tokens, %d of %d experts with matrices",
+               shared_rows, T, real, E);
+    HB_REQUIRE(max_tiles >= (A + MOE_TILE_M - 1) / MOE_TILE_M + E + (shared_rows + MOE_TILE_M - 1) / MOE_TILE_M &&
+                   (tall_m == 0 || max_tall >= (A + tall_m - 1) / tall_m + E + (shared_rows + tall_m - 1) / tall_m),
                "moe: the tile list is too short");
     const RouteForm form = {by_scores, n_groups, keep, softmax_scores, worth_top, renorm};
     if (T <= FEW_TOKENS && A <= FEW_PAIRS && E <= HB_WAVE * 4 && tall_m == 0) {
 #define HB_FEW(PER)                                                                                                      \
     moe_route_few_kernel<PER><<<1, HB_WAVE * (T < 4 ? 4 : T), 0, stream>>>(logits, ld, bias, chosen, weight, counts, order, \
-        row_of, tile_expert, tile_row0, tile_rows, T, E, top, max_tiles, real, form)
+        row_of, tile_expert, tile_row0, tile_rows, T, E, top, max_tiles, real, shared_rows, form)
         if (E <= HB_WAVE) HB_FEW(1);
         else if (E <= HB_WAVE * 2) HB_FEW(2);
         else HB_FEW(4);
@@ -355,7 +376,8 @@ extern "C" int hb_moe_route(const float* logits, const float* bias, int* chosen,
     else HB_ROUTE(MOE_MAX_E_PER_LANE);
 #undef HB_ROUTE
     HB_CHECK_LAUNCH("moe_route");
-    moe_place_kernel<<<E + 1, 1024, 0, stream>>>(chosen, counts, order, row_of, tile_expert, tile_row0, tile_rows, (int)A, E, max_tiles, real, tall, tall_m, max_tall);
+    moe_place_kernel<<<E + 1, 1024, 0, stream>>>(chosen, counts, order, row_of, tile_expert, tile_row0, tile_rows, (int)A, E, max_tiles, real, tall, tall_m, max_tall,
+                                              top, shared_rows);
     HB_CHECK_LAUNCH("moe_place");
     return 0;
 }

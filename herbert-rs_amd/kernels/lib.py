@@ -74,7 +74,7 @@ SIGNATURES = {
         "hb_latent_attention_plain": [_P, _P, _P, _I, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P, _P],
     },
     "moe": {
-        "hb_moe_route": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _I, _I, _P],
+        "hb_moe_route": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _I, _I, _I, _P],
         "hb_moe_gemm_plain": [_P, _I, _P, _I, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _P],
         "hb_moe_activate": [_P, _P, _I, _I, _I, _F, _F, _F, _P],
         "hb_moe_combine": [_P, _P, _P, _P, _I, _I, _I, _P, _P, _I, _P, _I, _P, _I, _P],

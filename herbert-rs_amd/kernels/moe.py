@@ -14,29 +14,32 @@ TALL_TILES = (128, 192, 256)           # of the matrix-core product of many rows
 MAX_EXPERTS = 1024
 
 
-def max_tiles(pairs, experts, rows=TILE_M):
-    """The length of the list of row tiles for that many (token, expert) pairs."""
-    return (pairs + rows - 1) // rows + experts
+def max_tiles(pairs, experts, rows=TILE_M, shared=0):
+    """The length of the list of row tiles for that many (token, expert) pairs and rows of a shared expert."""
+    return -(-pairs // rows) + experts + -(-shared // rows)
 
 
 class Routing:
     """The buffers that routing fills for a step of T tokens: chosen int32 [T, top], weight f32 [T, top],
     order / row_of int32 [T top], the tiles' lists."""
 
-    def __init__(self, ints, weight, T, E, top, real=None, tall=0):
+    def __init__(self, ints, weight, T, E, top, real=None, tall=0, shared=False):
         """real: the first `real` of the E experts have matrices (None: all); the others' output is their input.
-        tall: 0, or one of TALL_TILES: a second list, of tiles of that many rows."""
+        tall: 0, or one of TALL_TILES: a second list, of tiles of that many rows.
+        shared: every token takes one more expert, the matrices behind the others'; its rows, a token each, follow the pairs'."""
         self.real = E if real is None else int(real)
         self.tall = int(tall)
-        A, tiles = T * top, max_tiles(T * top, E)
-        self.tall_tiles = max_tiles(A, E, self.tall) if self.tall else 0
-        need = 3 * A + E + 3 * tiles + 3 * self.tall_tiles
+        self.shared_rows = T if shared else 0
+        A, tiles = T * top, max_tiles(T * top, E, shared=self.shared_rows)
+        self.rows = A + self.shared_rows
+        self.tall_tiles = max_tiles(A, E, self.tall, self.shared_rows) if self.tall else 0
+        need = self.ints_needed(T, E, top, tall, shared)
         if ints.numel() < need or ints.dtype != torch.int32:
             raise BackendError("routing: the int32 buffer is too small")
         self.T, self.E, self.top, self.tiles = T, E, top, tiles
         o = 0
         self.chosen, o = ints[o:o + A], o + A
-        self.order, o = ints[o:o + A], o + A
+        self.order, o = ints[o:o + self.rows], o + self.rows
         self.row_of, o = ints[o:o + A], o + A
         self.counts, o = ints[o:o + E], o + E
         self.tile_expert, o = ints[o:o + tiles], o + tiles
@@ -46,8 +49,9 @@ class Routing:
         self.weight = weight
 
     @staticmethod
-    def ints_needed(T, E, top, tall=0):
-        return 3 * T * top + E + 3 * max_tiles(T * top, E) + (3 * max_tiles(T * top, E, tall) if tall else 0)
+    def ints_needed(T, E, top, tall=0, shared=False):
+        rows = T if shared else 0
+        return 3 * T * top + rows + E + 3 * max_tiles(T * top, E, shared=rows) + (3 * max_tiles(T * top, E, tall, rows) if tall else 0)
 
 
 def route(logits, bias, routing, scores=False, groups=1, keep=1, score="sigmoid", worth_top=2, renorm=True):
@@ -79,7 +83,7 @@ def route(logits, bias, routing, scores=False, groups=1, keep=1, score="sigmoid"
              r.counts.data_ptr(), r.order.data_ptr(), r.row_of.data_ptr(), r.tile_expert.data_ptr(),
              r.tile_row0.data_ptr(), r.tile_rows.data_ptr(), r.T, r.E, r.top, r.tiles, ld, 1 if scores else 0,
              int(groups), int(keep), r.real, 1 if score == "softmax" else 0, int(worth_top), 1 if renorm else 0,
-             _ptr(r.tall_list), r.tall, r.tall_tiles, _stream())
+             _ptr(r.tall_list), r.tall, r.tall_tiles, r.shared_rows, _stream())
 
 
 def gemm_plain(a, w, c, routing, gather):
@@ -203,12 +207,12 @@ def grouped_mfma(a, lda, a_group_off, w, c, ldc, c_group_off, epi, routing=None,
     out_cols = N // 2 if epi == EPI_GLU else N
     if routing is not None:
         r = routing
-        rows_a, rows_c = (r.T if gather else r.T * r.top), r.T * r.top
-        if G != r.real:
+        rows_a, rows_c = (r.T if gather else r.rows), r.rows
+        if G != r.real + (1 if r.shared_rows else 0):
             raise BackendError("grouped product: one matrix an expert")
         lists = (r.order.data_ptr(), r.top if gather else 0, r.tile_expert.data_ptr(), r.tile_row0.data_ptr(),
                  r.tile_rows.data_ptr(), r.tiles, 0, 0)
-        few = r.T * r.top <= FEW_ROWS * G          # (on average; the kernels take any tile either way)
+        few = r.T * r.top <= FEW_ROWS * r.real          # (on average; the kernels take any tile either way)
     else:
         rows_a = rows_c = M
         lists = (None, 0, None, None, None, 0, M, G)

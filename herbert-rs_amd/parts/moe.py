@@ -99,6 +99,16 @@ class RoutedExperts(Part):
         n = self.names
         router = rt.weight(tensors[n["router"]])
         self.shared_up = self.shared_down = None
+        W, F = self.hidden_size, self.inter
+        # bfloat16 with sizes the matrix cores take: the matrices are kept in their operands' order
+        self.cores = (rt.dtype == torch.bfloat16 and moe.mfma_takes(W, W, 0, 2 * F) and moe.mfma_takes(F, F, 0, W)
+                      and F % 16 == 0)
+        # a shared expert of the others' size and activation is one more of them, with a row for every token: its two products
+        # and the kernel between them (18 us a layer for eight tokens, 32 experts of 768 on 2,048) go, and the experts' products grow
+        # by one expert's tiles (2 us)
+        self.folded = (self.cores and self.shared_expert is not None and self.shared_expert[0] == F
+                       and (self.limit, self.alpha, self.shift) == (math.inf, 1.0, 0.0))
+        matrices = [n] * self.experts
         if self.shared_expert is not None:
             # the shared expert's gate is one more row of the router's product (rows up to a multiple of
             # 16, zeros, so that the matrix cores take the product)
@@ -108,6 +118,9 @@ class RoutedExperts(Part):
             wide[:self.experts] = router
             wide[self.experts] = rt.weight(tensors[sn["sg"]])[0]
             router = wide
+        if self.folded:
+            matrices.append(sn)
+        elif self.shared_expert is not None:
             gate, up = rt.weight(tensors[sn["gate"]]), rt.weight(tensors[sn["up"]])
             self.shared_fused = (rt.dtype == torch.bfloat16 and Fs % 16 == 0 and self.hidden_size % 32 == 0
                                  and mfma.gemm_supported(gate[:1], gate, swiglu=True))
@@ -120,14 +133,9 @@ class RoutedExperts(Part):
         self.router_width = router.shape[0]
         self.router_bias = rt.weight(tensors[n["router_bias"]], matrix=False) if n.get("router_bias") else None
         # [E, 2 F, W]: an expert's gate rows, then its up rows; [E, W, F]
-        self.gate_up = torch.stack([torch.cat([rt.weight(tensors[n["gate"].format(e=e)]),
-                                               rt.weight(tensors[n["up"].format(e=e)])], 0)
-                                    for e in range(self.experts)]).contiguous()
-        self.down = torch.stack([rt.weight(tensors[n["down"].format(e=e)]) for e in range(self.experts)]).contiguous()
-        # bfloat16 with sizes the matrix cores take: the matrices are kept in their operands' order
-        W, F = self.hidden_size, self.inter
-        self.cores = (rt.dtype == torch.bfloat16 and moe.mfma_takes(W, W, 0, 2 * F) and moe.mfma_takes(F, F, 0, W)
-                      and F % 16 == 0)
+        self.gate_up = torch.stack([torch.cat([rt.weight(tensors[m["gate"].format(e=e)]), rt.weight(tensors[m["up"].format(e=e)])], 0)
+                                    for e, m in enumerate(matrices)]).contiguous()
+        self.down = torch.stack([rt.weight(tensors[m["down"].format(e=e)]) for e, m in enumerate(matrices)]).contiguous()
         if self.cores:
             self.gate_up, self.down = moe.pack_grouped(self.gate_up), moe.pack_grouped(self.down)
 
@@ -137,15 +145,16 @@ class RoutedExperts(Part):
         logits = rt.buffer("moe_logits", (T, self.router_width), torch.float32)
         self.router.forward(y, logits)          # float32 sums of the rows' products with the router's matrix
         tall = moe.tall_rows(T, top, E, self.experts, self.hidden_size, F) if self.cores else 0
-        routing = moe.Routing(rt.buffer("moe_ints", (moe.Routing.ints_needed(T, E, top, tall),), torch.int32),
-                              rt.buffer("moe_weight", (T, top), torch.float32), T, E, top, real=self.experts, tall=tall)
+        routing = moe.Routing(rt.buffer("moe_ints", (moe.Routing.ints_needed(T, E, top, tall, self.folded),), torch.int32),
+                              rt.buffer("moe_weight", (T, top), torch.float32), T, E, top, real=self.experts, tall=tall,
+                              shared=self.folded)
         if self.routing == "scores":
             moe.route(logits, self.router_bias, routing, scores=True, groups=self.groups, keep=self.keep,
                       score=self.scoring, worth_top=self.group_worth, renorm=self.renormalize)
         else:
             moe.route(logits, self.router_bias, routing)
         shared = None
-        if self.shared_expert is not None:
+        if self.shared_expert is not None and not self.folded:
             Fs = self.shared_expert[0]
             s_act = rt.buffer("moe_shared_act", (T, Fs))
             if self.shared_fused:
@@ -156,8 +165,8 @@ class RoutedExperts(Part):
                 ops.swiglu(s_gu, s_act)
             shared = rt.buffer("moe_shared_out", (T, self.hidden_size), torch.float32)
             self.shared_down.forward(s_act, shared)
-        act = rt.buffer("moe_act", (T * top, F))
-        out = rt.buffer("moe_out", (T * top, self.hidden_size), torch.float32)
+        act = rt.buffer("moe_act", (routing.rows, F))
+        out = rt.buffer("moe_out", (routing.rows, self.hidden_size), torch.float32)
         if self.cores:
             # matrix cores; the activation is the first product's epilogue
             moe.grouped_mfma(y, self.hidden_size, 0, self.gate_up, act, F, 0, moe.EPI_GLU, routing, gather=True,
@@ -169,5 +178,7 @@ class RoutedExperts(Part):
             moe.gemm_plain(y, self.gate_up, gu, routing, gather=True)
             moe.activate(gu, act, self.limit, self.alpha, self.shift)
             moe.gemm_plain(act, self.down, out, routing, gather=False)
+        if self.folded:
+            shared, out = out[T * top:], out[:T * top]
         moe.combine(out, routing, x, shared=shared, gate=None if shared is None else (logits, E),
                     identity=y if self.identity else None)

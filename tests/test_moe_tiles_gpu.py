@@ -54,6 +54,57 @@ def test_tall_tiles(T, E, real, top, W, F, tile_m):
         assert bool(((out[rows].cpu().double() - terms).abs() <= F * 2.0 ** -24 * size + 1e-30).all()), e
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,E,top,tall", [(1, 3, 2, 0), (8, 5, 3, 0), (8, 5, 3, 128), (9, 4, 1, 0), (70, 3, 2, 0), (300, 3, 2, 192), (257, 2, 1, 256)])
+def test_rows_of_a_shared_expert(T, E, top, tall):
+    """An expert that every token takes, its matrices behind the others': a row a token behind the pairs', its tiles behind
+    theirs in either list; the pairs' own parts are what they are without it. Products and sum against float64 (bounds as above;
+    the sum of top + 1 terms adds as many roundings)."""
+    W, F = 128, 64
+    g = torch.Generator().manual_seed(T)
+    logits, y = torch.randn(T, E, generator=g).to(DEV), torch.randn(T, W, generator=g).bfloat16()
+    gate = torch.randn(T, 3, generator=g).to(DEV)
+    gate_up = (torch.randn(E + 1, 2 * F, W, generator=g) * W ** -0.5).bfloat16()
+    down = (torch.randn(E + 1, W, F, generator=g) * F ** -0.5).bfloat16()
+    made = {}
+    for shared in (False, True):
+        r = moe.Routing(torch.full((moe.Routing.ints_needed(T, E, top, tall, shared),), -7, dtype=torch.int32, device=DEV),
+                        torch.empty(T, top, device=DEV), T, E, top, tall=tall, shared=shared)
+        moe.route(logits, None, r)
+        made[shared] = r
+    r, A = made[True], T * top
+    for name in ("chosen", "row_of", "counts", "weight"):
+        assert torch.equal(getattr(r, name), getattr(made[False], name))
+    assert torch.equal(r.order[:A], made[False].order) and torch.equal(r.order[A:].cpu(), torch.arange(T, dtype=torch.int32) * top)
+    lists = [(64, torch.stack([r.tile_expert, r.tile_row0, r.tile_rows]))] + ([(tall, r.tall_list)] if tall else [])
+    for rows, got in lists:
+        want, at = [], 0
+        for e, c in enumerate(r.counts.tolist() + [T]):
+            want += [(e, at + i, min(rows, c - i)) for i in range(0, c, rows)]
+            at += c
+        got = list(zip(*got.tolist()))
+        assert got[:len(want)] == want and all(t[0] == -1 for t in got[len(want):])
+    act = torch.empty(r.rows, F, dtype=torch.bfloat16, device=DEV)
+    out = torch.empty(r.rows, W, device=DEV)
+    moe.grouped_mfma(y.to(DEV), W, 0, moe.pack_grouped(gate_up).to(DEV), act, F, 0, moe.EPI_GLU, r, gather=True, limit=float("inf"),
+                     alpha=1.0, shift=0.0, tall=tall > 0)
+    moe.grouped_mfma(act, F, 0, moe.pack_grouped(down).to(DEV), out, W, 0, moe.EPI_F32, r, tall=tall > 0)
+    expert = torch.cat([r.chosen.cpu()[r.order.cpu().long()[:A]].long(), torch.full((T,), E)])
+    got = act.cpu().double()
+    for e in range(E + 1):
+        rows = (expert == e).nonzero().flatten()
+        x = y[r.order.cpu().long()[rows] // top].double() @ gate_up[e].double().T
+        want = torch.nn.functional.silu(x[:, :F]) * x[:, F:]
+        assert bool(((got[rows] - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all()), e
+        size = got[rows].abs() @ down[e].double().abs().T
+        assert bool(((out[rows].cpu().double() - got[rows] @ down[e].double().T).abs() <= F * 2.0 ** -24 * size + 1e-30).all()), e
+    x = torch.zeros(T, W, device=DEV)
+    moe.combine(out[:A], r, x, shared=out[A:], gate=(gate, 1))
+    terms = out.cpu().double()[r.row_of.cpu().long()].view(T, top, W) * r.weight.cpu().double()[:, :, None]
+    terms = torch.cat([terms, (torch.sigmoid(gate[:, 1:2].cpu().double()) * out[A:].cpu().double())[:, None]], 1)
+    assert bool(((x.cpu().double() - terms.sum(1)).abs() <= (top + 4) * 2.0 ** -23 * terms.abs().sum(1) + 1e-30).all())
+
+
 def test_tile_heights_by_the_rows_an_expert_has():
     """Few rows keep the low tiles, as do sizes that the tall ones refuse and steps that would leave most CUs without one."""
     assert moe.tall_rows(256, 4, 32, 32, 2048, 768) == 0
