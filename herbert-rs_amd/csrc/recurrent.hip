@@ -878,14 +878,14 @@ __global__ void __launch_bounds__(256)
 ssm_scan_kernel(const float* __restrict__ u, int ldu, const float* __restrict__ proj, int ld, int dt_off,
                 const float* __restrict__ dt_bias, const float* __restrict__ A_log, const float* __restrict__ Dskip,
                 float* __restrict__ state, const int* __restrict__ seq_starts, const int* __restrict__ slots,
-                float* __restrict__ y, int heads, int groups, int N, int P) {
+                float* __restrict__ y, int heads, int groups, int N, int P, const int* __restrict__ which) {
     constexpr int CPW = 256 / LPC;                      // columns a workgroup
     constexpr int MAXN = LPC * NR;                      // rows that the lanes' registers hold (those from N on stay zero)
     constexpr int ROW = 2 * MAXN + CPW;                 // a token's inputs: B | C | x
     constexpr int STRIDE = ROW + 4;                     // then dt, the decay, and two unused
     constexpr int PER = (SSM_TOKENS * ROW + 255) / 256;
     __shared__ __attribute__((aligned(16))) float in_lds[SSM_TOKENS * STRIDE];
-    const int tile = blockIdx.x, h = blockIdx.y, seq = blockIdx.z;
+    const int tile = blockIdx.x, h = blockIdx.y, seq = which ? which[blockIdx.z] : blockIdx.z;
     const int tid = threadIdx.x, col = tid / LPC, part = tid % LPC;
     const int p = tile * CPW + col;
     const bool live = p < P;
@@ -984,10 +984,11 @@ extern "C" int hb_ssm_state_floats(int N, int P) {
     return (P + cpw - 1) / cpw * 256 * nr;
 }
 
+// which (or null: all B sequences of the step): the B sequences that are walked.
 extern "C" int hb_ssm_scan(const float* u, int ldu, const float* proj, int ld, int dt_off, const float* dt_bias,
                            const float* A_log, const float* Dskip, float* state, const int* seq_starts,
                            const int* slots, float* y, int B, int heads, int groups, int N, int P,
-                           int state_floats, hipStream_t stream) {
+                           int state_floats, const int* which, hipStream_t stream) {
     HB_REQUIRE(B > 0 && heads > 0 && groups > 0 && N > 0 && P > 0, "state-space walk: empty input");
     HB_REQUIRE(N <= 256 && state_floats == hb_ssm_state_floats(N, P),
                "state-space walk: a head's state of %d floats is not the kernel's layout for %d x %d", state_floats, N, P);
@@ -998,7 +999,7 @@ extern "C" int hb_ssm_scan(const float* u, int ldu, const float* proj, int ld, i
     HB_REQUIRE(heads <= 65535 && B <= 65535, "state-space walk: too many heads or sequences for the grid");
 #define HB_SSM(NRV, LPCV)                                                                                              \
     ssm_scan_kernel<NRV, LPCV><<<dim3((P + 256 / LPCV - 1) / (256 / LPCV), heads, B), 256, 0, stream>>>(               \
-        u, ldu, proj, ld, dt_off, dt_bias, A_log, Dskip, state, seq_starts, slots, y, heads, groups, N, P)
+        u, ldu, proj, ld, dt_off, dt_bias, A_log, Dskip, state, seq_starts, slots, y, heads, groups, N, P, which)
     int nr, lpc;
     ssm_layout(N, &nr, &lpc);
     if (nr == 4 && lpc == 4) HB_SSM(4, 4);

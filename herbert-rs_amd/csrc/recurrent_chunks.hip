@@ -565,3 +565,301 @@ extern "C" int hb_chunked_delta(const float* qkv, int C, const float* proj, int 
     HB_CHECK_LAUNCH("chunk_scan");
     return 0;
 }
+
+// ---------------------------------------------------------------- state-space layer with one decay a head, in chunks
+// recurrent.hip has the rule: S <- a S + dt B x^T, y = S^T C + D x, with a = exp(-rate dt), one number a head and token, and B and C
+// shared by the heads of a group. With c_t the sum of rate dt up to token t of a chunk,
+//   y_t = exp(-c_t) S_0^T C_t + sum_(i<=t) (C_t . B_i) exp(c_i - c_t) dt_i x_i + D x_t
+//   S   = exp(-c_64) S_0 + sum_i B_i exp(c_i - c_64) dt_i x_i
+// (Dao and Gu, 2024: state-space duality; the sums c and their differences in float64, so that a pair's decay is exact to its
+// own size, and no quotient of decays is formed.) Products on the matrix cores, in float32, those of pairs in float64 and rounded once.
+// ssm_pairs_kernel: C_t . B_i of a (chunk, group) once for all its heads, as the second kernel's lanes load them.
+// ssm_chunks_kernel: the chain of chunks, a workgroup a (head, 32 columns of S, sequence): four waves, each 16 tokens of a chunk for the outputs and a
+// quarter of the state's rows. A chunk that holds something not finite is walked token by token instead (ssm_slowly), so that it
+// spoils what it spoils in the walk.
+// 64 heads of 128 x 64 on 8 groups, one sequence of 2,048 tokens 318 us (the walk 802), of 512 91 (209), four of 512 133 (313), 16 of 128 140
+// (310). Bound by a chunk's chain in a workgroup, 9.5 us: 160 products of 40 cycles a wave, and as long again for the decays and for
+// laying out the state and the columns. Errors against 64 bits are 0.2 to 1.02 of the walk's.
+template <int DB>
+__global__ void __launch_bounds__(256)
+ssm_pairs_kernel(const float* __restrict__ u, int ldu, int b_at, int c_at, const int2* __restrict__ chunks,
+                 float* __restrict__ pairs, int groups) {
+    constexpr int N = 16 * DB;
+    const int g = blockIdx.x, chunk = blockIdx.y;
+    const int first = chunks[chunk].x, n = chunks[chunk].y;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
+    auto row_of = [&](int t) { return u + (size_t)(first + min(t, n - 1)) * ldu; };    // (tokens past the end: the last one again, unused)
+    f32x4 c[DB];
+    const float* c_row = row_of(16 * wave + r) + c_at + g * N + 4 * q;
+#pragma unroll
+    for (int b = 0; b < DB; ++b) c[b] = load_quad<true>(c_row + 16 * b, 4);
+#pragma unroll
+    for (int b = 0; b < DB; ++b) transpose_quads(c[b]);
+    float* out = pairs + ((size_t)chunk * groups + g) * CHUNK * CHUNK;
+    for (int block = 0; block <= wave; ++block) {
+        const float* b_row = row_of(16 * block + r) + b_at + g * N + 4 * q;
+        f32x4 k[DB];
+#pragma unroll
+        for (int b = 0; b < DB; ++b) k[b] = load_quad<true>(b_row + 16 * b, 4);
+        f64x4 sum = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int b = 0; b < DB; ++b) {
+            transpose_quads(k[b]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum = mfma64_k4(k[b][e], c[b][e], sum);
+        }
+        // (earlier token 16 block + 4 e + q, later token 16 wave + r)
+        const f32x4 s = {(float)sum[0], (float)sum[1], (float)sum[2], (float)sum[3]};
+        *(f32x4*)(out + ((wave * 4 + block) * 64 + lane) * 4) = s;
+    }
+}
+
+// One chunk of 32 columns token by token; the state lies in LDS, a column's entry n at in_quads(n). Eight lanes a column.
+template <int N, int SLD>
+__device__ __forceinline__ void ssm_slowly(float* s_lds, const float* u, int ldu, const float* proj, int ld, int n, int x_at, int b_at, int c_at,
+                                           float bias, float rate, float skip, float* y, int ldy, int cols) {
+    const int col = threadIdx.x / 8, part = threadIdx.x % 8;
+    for (int t = 0; t < n; ++t) {
+        const float* row = u + (size_t)t * ldu;
+        const float z = proj[(size_t)t * ld] + bias, dt = z > 20.f ? z : log1pf(expf(z)), a = expf(-rate * dt);
+        const float x = row[x_at + col], dx = dt * x;
+        float acc = 0.f;
+        for (int i = part * (N / 8); i < (part + 1) * (N / 8); ++i) {
+            float& s = s_lds[col * SLD + in_quads(i)];
+            s = fmaf(a, s, dx * row[b_at + i]);
+            acc = fmaf(s, row[c_at + i], acc);
+        }
+#pragma unroll
+        for (int off = 1; off < 8; off <<= 1) acc += __shfl_xor(acc, off, HB_WAVE);
+        if (part == 0 && col < cols) y[(size_t)t * ldy + col] = fmaf(skip, x, acc);
+    }
+}
+
+#define SSM_COLS 32
+template <int DB>
+__global__ void __launch_bounds__(256, 2)
+ssm_chunks_kernel(const float* __restrict__ u, int ldu, const float* __restrict__ proj, int ld, int dt_off,
+                  const float* __restrict__ dt_bias, const float* __restrict__ A_log, const float* __restrict__ Dskip,
+                  const float* __restrict__ pairs, float* __restrict__ state, const int4* __restrict__ runs,
+                  const int* __restrict__ slots, float* __restrict__ y, int heads, int groups, int P) {
+    constexpr int N = 16 * DB, OWN = DB / 4, CB = SSM_COLS / 16;
+    constexpr int SLD = N + 4, XLD = CHUNK + 4;
+    __shared__ __attribute__((aligned(16))) float s_lds[2][SSM_COLS * SLD], x_lds[2][SSM_COLS * XLD];
+    __shared__ double c_lds[4][CHUNK];
+    __shared__ float dt_lds[4][CHUNK];
+    __shared__ int spoilt[2];
+    const int h = blockIdx.x, col0 = blockIdx.y * SSM_COLS, cols = min(SSM_COLS, P - col0);
+    const int4 run = runs[blockIdx.z];
+    const int begin = run.z, n_all = run.w, last = (n_all + CHUNK - 1) / CHUNK;
+    const int g = h / (heads / groups), inner = heads * P;
+    const int x_at = h * P + col0, b_at = inner + g * N, c_at = inner + (groups + g) * N;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, q = lane >> 4;
+    const float rate = expf(A_log[h]), bias = dt_bias[h], skip = Dskip[h];
+    // the walk keeps a column's N entries side by side
+    float* S_mem = state + ((size_t)slots[run.x] * heads + h) * P * N + (size_t)col0 * N;
+    f32x4 S[OWN][CB];
+#pragma unroll
+    for (int i = 0; i < OWN; ++i)
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb)
+            S[i][cb] = 16 * cb < cols ? *(const f32x4*)(S_mem + (size_t)(16 * cb + r) * N + 16 * (wave + 4 * i) + 4 * q) : f32x4{0.f, 0.f, 0.f, 0.f};
+    auto share = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < OWN; ++i)
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s_lds[buf][(16 * cb + r) * SLD + 16 * (wave + 4 * i) + 4 * e + q] = S[i][cb][e];
+    };
+    // a chunk's inputs that all waves share: thread tid brings eight columns of token tid / 4 (columns past the head's are zeros)
+    const int my_token = tid / 4, my_col = tid % 4 * 8;
+    f32x4 x_next[2];
+    float z_next;
+    auto fetch = [&](int c) {
+        const int n = min(CHUNK, n_all - c * CHUNK);
+        const float* row = u + (size_t)(begin + c * CHUNK + my_token) * ldu + x_at + my_col;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            x_next[i] = my_token < n && my_col + 4 * i < cols ? *(const f32x4*)(row + 4 * i) : f32x4{0.f, 0.f, 0.f, 0.f};
+        z_next = lane < n ? proj[(size_t)(begin + c * CHUNK + lane) * ld + dt_off + h] : 0.f;
+    };
+    // ... into LDS: the columns as a product wants a column's tokens, and every wave its own copy of the step sizes and their sums
+    auto place = [&](int c, int buf) {
+        const int n = min(CHUNK, n_all - c * CHUNK);
+        const float z = z_next + bias;
+        const float dt = lane < n ? (z > 20.f ? z : log1pf(expf(z))) : 0.f;
+        double sum = lane < n ? (double)(rate * dt) : 0.0;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const double o = __shfl_up(sum, off, HB_WAVE);
+            if (lane >= off) sum += o;
+        }
+        c_lds[wave][lane] = sum;
+        dt_lds[wave][lane] = dt;
+        const float my_dt = __shfl(dt, my_token & 63, HB_WAVE);
+        bool bad = not_finite(dt) || not_finite((float)sum);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                bad |= not_finite(x_next[i][e]) || not_finite(x_next[i][e] * my_dt);
+                x_lds[buf][(my_col + 4 * i + e) * XLD + in_quads(my_token)] = x_next[i][e];
+            }
+        if (bad) spoilt[buf] = 1;
+    };
+    // what a wave reads of a chunk for itself: its 16 tokens of C and their pairs, all tokens' B for its rows of the state
+    f32x4 cq[DB], pr[4];
+    float k[OWN][16];
+    auto ask = [&](int c) {
+        const int n = min(CHUNK, n_all - c * CHUNK), t0 = begin + c * CHUNK;
+        const float* c_row = u + (size_t)(t0 + min(16 * wave + r, n - 1)) * ldu + c_at + 4 * q;
+#pragma unroll
+        for (int b = 0; b < DB; ++b) cq[b] = load_quad<true>(c_row + 16 * b, 4);
+        const float* p = pairs + ((size_t)(run.y + c) * groups + g) * CHUNK * CHUNK;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) pr[b] = b <= wave ? *(const f32x4*)(p + ((wave * 4 + b) * 64 + lane) * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < 16; ++s) {
+            const float* b_row = u + (size_t)(t0 + min(4 * s + q, n - 1)) * ldu + b_at + r;
+#pragma unroll
+            for (int i = 0; i < OWN; ++i) k[i][s] = b_row[16 * (wave + 4 * i)];
+        }
+    };
+    if (tid < 2) spoilt[tid] = 0;
+    fetch(0);
+    ask(0);
+    share(0);
+    __syncthreads();
+    place(0, 0);
+    __syncthreads();
+    for (int c = 0; c < last; ++c) {
+        const int buf = c & 1, n = min(CHUNK, n_all - c * CHUNK), t0 = begin + c * CHUNK;
+        const bool more = c + 1 < last;
+        if (more) fetch(c + 1);
+        bool bad = false;
+#pragma unroll
+        for (int b = 0; b < DB; ++b)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) bad |= not_finite(cq[b][e]);
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) bad |= not_finite(pr[b][e]);
+#pragma unroll
+        for (int s = 0; s < 16; ++s)
+#pragma unroll
+            for (int i = 0; i < OWN; ++i) bad |= not_finite(k[i][s]);
+        // (an entry so large that a product before its decay may pass float32's range is the walk's too)
+#pragma unroll
+        for (int i = 0; i < OWN; ++i)
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) bad |= !(fabsf(S[i][cb][e]) <= 1e30f);
+        if (__any(bad) && lane == 0) spoilt[buf] = 1;
+        // the decays: of a token from the chunk's start, of a pair, and to the chunk's end
+        const double own = c_lds[wave][16 * wave + r], end = c_lds[wave][CHUNK - 1];
+        float from_start[4], to_end[16], dt[16];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) from_start[e] = expf((float)-c_lds[wave][16 * wave + 4 * q + e]);
+        const float all = expf((float)-end);
+#pragma unroll
+        for (int s = 0; s < 16; ++s) {
+            const int i = 4 * s + q;
+            const double at = c_lds[wave][i];
+            dt[s] = dt_lds[wave][i];
+            to_end[s] = expf((float)(at - end));
+            pr[s / 4][s % 4] *= i <= 16 * wave + r ? expf((float)(at - own)) : 0.f;
+        }
+        __syncthreads();                                      // (everyone has looked for what is not finite)
+        if (spoilt[buf]) {
+            ssm_slowly<N, SLD>(s_lds[buf], u + (size_t)t0 * ldu, ldu, proj + (size_t)t0 * ld + dt_off + h, ld, n, x_at, b_at, c_at, bias, rate, skip,
+                               y + (size_t)t0 * inner + x_at, inner, cols);
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < OWN; ++i)
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) S[i][cb][e] = s_lds[buf][(16 * cb + r) * SLD + 16 * (wave + 4 * i) + 4 * e + q];
+        } else {
+#pragma unroll
+            for (int b = 0; b < DB; ++b) transpose_quads(cq[b]);
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) {
+                Chains<8> part;
+#pragma unroll
+                for (int b = 0; b < DB; ++b) {
+                    const f32x4 s = *(const f32x4*)&s_lds[buf][(16 * cb + r) * SLD + 16 * b + 4 * q];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) part.add(cq[b][e], s[e], 4 * b + e);
+                }
+                f32x4 sums = part.sum();
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sums[e] *= from_start[e];
+#pragma unroll
+                for (int i = 0; i < OWN; ++i) S[i][cb] *= all;
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    f32x4 x = *(const f32x4*)&x_lds[buf][(16 * cb + r) * XLD + 16 * b + 4 * q];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        x[e] *= dt[4 * b + e];
+                        const float late = x[e] * to_end[4 * b + e];
+#pragma unroll
+                        for (int i = 0; i < OWN; ++i) S[i][cb] = mfma_k4(k[i][4 * b + e], late, S[i][cb]);
+                        if (b <= wave) sums = mfma_k4(pr[b][e], x[e], sums);
+                    }
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int t = 16 * wave + 4 * q + e;
+                    if (t < n && 16 * cb < cols)
+                        y[(size_t)(t0 + t) * inner + x_at + 16 * cb + r] =
+                            fmaf(skip, x_lds[buf][(16 * cb + r) * XLD + in_quads(t)], sums[e]);
+                }
+            }
+        }
+        if (more) {
+            ask(c + 1);                                       // (on their way while the state and the columns are laid out)
+            share(buf ^ 1);
+            place(c + 1, buf ^ 1);
+        }
+        __syncthreads();
+        if (tid == 0) spoilt[buf] = 0;                        // (read again two chunks on, behind a barrier)
+    }
+#pragma unroll
+    for (int i = 0; i < OWN; ++i)
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb)
+            if (16 * cb < cols) *(f32x4*)(S_mem + (size_t)(16 * cb + r) * N + 16 * (wave + 4 * i) + 4 * q) = S[i][cb];
+}
+
+// As hb_ssm_scan of recurrent.hip, for states of 64 or 128 rows and columns in steps of 16, and for those sequences only that its
+// lists name (see hb_chunked_delta). pairs holds n_chunks x groups x 64 x 64 floats.
+extern "C" int hb_chunked_ssm(const float* u, int ldu, const float* proj, int ld, int dt_off, const float* dt_bias,
+                              const float* A_log, const float* Dskip, float* state, const int* chunks, int n_chunks,
+                              const int* runs, int n_runs, const int* slots, float* y, float* pairs, int heads, int groups, int N,
+                              int P, int state_floats, hipStream_t stream) {
+    HB_REQUIRE(n_chunks > 0 && n_runs > 0 && heads > 0 && groups > 0 && heads % groups == 0, "state-space chunks: %d heads in %d groups", heads, groups);
+    HB_REQUIRE((N == 64 || N == 128) && P > 0 && P % 16 == 0 && state_floats == N * P, "state-space chunks: a state of %d x %d in %d floats", N, P, state_floats);
+    HB_REQUIRE(ldu >= heads * P + 2 * groups * N && ldu % 4 == 0 && (uintptr_t)u % 16 == 0 && (uintptr_t)state % 16 == 0 && (uintptr_t)pairs % 16 == 0,
+               "state-space chunks: rows of %d are not in whole quads", ldu);
+    HB_REQUIRE(dt_off >= 0 && dt_off + heads <= ld, "state-space chunks: the columns lie outside their rows");
+    HB_REQUIRE((uintptr_t)chunks % 8 == 0 && (uintptr_t)runs % 16 == 0, "state-space chunks: the lists are not aligned");
+    const int tiles = (P + SSM_COLS - 1) / SSM_COLS;
+    HB_REQUIRE(n_runs <= 65535 && n_chunks <= 65535 && tiles <= 65535, "state-space chunks: too many sequences or columns for the grid");
+#define HB_SSM_CHUNKS(DB)                                                                                                    \
+    do {                                                                                                                     \
+        ssm_pairs_kernel<DB><<<dim3(groups, n_chunks), 256, 0, stream>>>(u, ldu, heads * P, heads * P + groups * N,          \
+                                                                         (const int2*)chunks, pairs, groups);                \
+        HB_CHECK_LAUNCH("ssm_pairs");                                                                                        \
+        ssm_chunks_kernel<DB><<<dim3(heads, tiles, n_runs), 256, 0, stream>>>(u, ldu, proj, ld, dt_off, dt_bias, A_log, Dskip, \
+            pairs, state, (const int4*)runs, slots, y, heads, groups, P);                                                    \
+    } while (0)
+    if (N == 128) HB_SSM_CHUNKS(8);
+    else HB_SSM_CHUNKS(4);
+#undef HB_SSM_CHUNKS
+    HB_CHECK_LAUNCH("ssm_chunks");
+    return 0;
+}

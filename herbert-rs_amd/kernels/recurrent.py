@@ -54,11 +54,12 @@ def ssm_state_floats(N, P):
     return -(-P // cols) * 256 * nr
 
 
-def ssm_scan(u, proj, dt_off, dt_bias, a_log, d_skip, state, meta, out, heads, groups, N, P):
+def ssm_scan(u, proj, dt_off, dt_bias, a_log, d_skip, state, meta, out, heads, groups, N, P, rt=None):
     """The state-space walk of every sequence of the step: u f32 [T, heads P + 2 groups N] (x, B, C as the
     convolution left them), the step sizes' pre-activations in columns [dt_off, + heads) of proj (f32 [T, ld]);
     dt = softplus(. + dt_bias), S <- exp(-exp(a_log) dt) S + dt B x^T, out = S^T C + d_skip x; state f32
-    [slots, heads, ssm_state_floats(N, P)] advanced in place (zeros: an empty state), out f32 [T, heads P]."""
+    [slots, heads, ssm_state_floats(N, P)] advanced in place (zeros: an empty state), out f32 [T, heads P]. With a Runtime the
+    long portions go through in chunks, for the sizes that those kernels take."""
     T = u.shape[0]
     _check(u, "u", torch.float32, (T, heads * P + 2 * groups * N))
     _check(proj, "proj", torch.float32, (T, None))
@@ -70,9 +71,19 @@ def ssm_scan(u, proj, dt_off, dt_bias, a_log, d_skip, state, meta, out, heads, g
     _check(meta.slots, "slots", torch.int32, (meta.num_seqs,))
     if heads % groups or not 0 < N <= MAX_SSM_STATE or dt_off < 0 or dt_off + heads > proj.shape[1]:
         raise BackendError(f"state-space walk: {heads} heads in {groups} groups, a state of {N} rows")
-    lib.call("recurrent", "hb_ssm_scan", u.data_ptr(), u.shape[1], proj.data_ptr(), proj.shape[1], int(dt_off),
-             dt_bias.data_ptr(), a_log.data_ptr(), d_skip.data_ptr(), state.data_ptr(), meta.seq_starts.data_ptr(),
-             meta.slots.data_ptr(), out.data_ptr(), meta.num_seqs, heads, groups, N, P, state.shape[2], _stream())
+    operands = (u.data_ptr(), u.shape[1], proj.data_ptr(), proj.shape[1], int(dt_off), dt_bias.data_ptr(), a_log.data_ptr(),
+                d_skip.data_ptr(), state.data_ptr())
+    walks = ((None, meta.num_seqs),)
+    if (rt is not None and meta.max_new >= SSM_CHUNKS_FROM and N in (64, 128) and P % 16 == 0 and u.shape[1] % 4 == 0
+            and u.data_ptr() % 16 == 0 and state.data_ptr() % 16 == 0):
+        calls, floats, walks = _ssm_lists(meta, groups)
+        pairs = rt.buffer("ssm_pairs", (floats,), torch.float32)
+        for runs, n_runs, chunks, n_chunks in calls:
+            lib.call("recurrent_chunks", "hb_chunked_ssm", *operands, chunks.data_ptr(), n_chunks, runs.data_ptr(), n_runs,
+                     meta.slots.data_ptr(), out.data_ptr(), pairs.data_ptr(), heads, groups, N, P, state.shape[2], _stream())
+    for which, n_seqs in walks:
+        lib.call("recurrent", "hb_ssm_scan", *operands, meta.seq_starts.data_ptr(), meta.slots.data_ptr(), out.data_ptr(), n_seqs,
+                 heads, groups, N, P, state.shape[2], None if which is None else which.data_ptr(), _stream())
 
 
 def gated_group_norm(o, proj, z_off, weight, out, parts, eps):
@@ -182,6 +193,36 @@ def _chunk_lists(meta, heads, correction, channels, size):
         while floats // 2 >= need and floats > 1:
             floats //= 2
         got = meta.derived[key] = (calls, max(floats, need), walks)
+    return got
+
+
+# Portions of so many tokens of a state-space layer go through in chunks. Microseconds by the walk / in chunks, 64 heads of 128 x 64: one
+# sequence of 32 tokens 17 / 22, 48 23 / 22, 64 30 / 22; four of 32 25 / 29, 48 34 / 30; 16 of 32 81 / 78, 48 116 / 82.
+SSM_CHUNKS_FROM = 48
+
+
+def _ssm_lists(meta, groups):
+    """As _chunk_lists, for state-space layers of that many groups: (calls, floats, walks)."""
+    key = ("ssm_chunks", groups, CHUNK_SCRATCH, SSM_CHUNKS_FROM)
+    got = meta.derived.get(key)
+    if got is None:
+        size, packed = groups * CHUNK * CHUNK, []
+
+        def place(numbers):                                    # (16 bytes aligned)
+            at = len(packed)
+            packed.extend(numbers + [0] * (-len(numbers) % 4))
+            return at
+        calls = [(place([x for run in runs for x in run]), len(runs), place([x for chunk in chunks for x in chunk]), len(chunks))
+                 for runs, chunks in chunk_calls(meta.host_starts, SSM_CHUNKS_FROM, max(1, CHUNK_SCRATCH // size))]
+        short = [i for i, n in enumerate(np.diff(meta.host_starts)) if n < SSM_CHUNKS_FROM]
+        walks = [(place(short), len(short))] if short else []
+        on_gpu = send(np.array(packed, dtype=np.int32), meta.seq_starts.device)
+        need = max(m for _, _, _, m in calls) * size
+        floats = CHUNK_SCRATCH
+        while floats // 2 >= need:
+            floats //= 2
+        got = meta.derived[key] = (tuple((on_gpu[a:], n, on_gpu[b:], m) for a, n, b, m in calls), max(floats, need),
+                                   tuple((on_gpu[a:], n) for a, n in walks))
     return got
 
 

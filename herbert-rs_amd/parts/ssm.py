@@ -109,7 +109,7 @@ class StateSpace(Part):
                             col0=self.inner, bias=self.conv_b)
         walked = rt.buffer("ssm_y", (T, self.inner), torch.float32)
         recurrent.ssm_scan(u, proj, self.inner + C, self.dt_bias, self.a_log, self.d_skip, views[0], ctx.meta, walked,
-                           self.heads, self.groups, self.N, self.P)
+                           self.heads, self.groups, self.N, self.P, rt=rt)
         gated = rt.buffer("ssm_gated", (T, self.inner))
         recurrent.gated_group_norm(walked, proj, 0, self.norm_w, gated, self.norm_groups, self.eps)
         adds = ctx.adds_to(x)
