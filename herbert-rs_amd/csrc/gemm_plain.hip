@@ -242,9 +242,10 @@ gemm_plain_wave_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
 }
 
 // The kernel of a product. 16-byte loads and stores where rows and strides allow them. Up to 16 rows of whole blocks of
-// 16 k take the wave kernel. Beyond, the largest tile that still fills the chip: 128 x 128 from two tiles for every CU on
-// (4096 x 4096 x 4096: 1,082 us; 64 x 64 1,281), 64 x 64 from two of those for every CU on (1200 x 4096 x 4096: 414;
-// 32 x 32 444, 128 x 128 539), else 32 x 32 (200 x 2048 x 2048: 30; 64 x 64 51; 564 x 2048 x 2048: 67; 64 x 64 84).
+// 16 k take the wave kernel. Beyond, the tile with the least estimated time: what a CU spends on one (microseconds at K = 2048 on all
+// CUs: 128 x 128 137, alone on a CU 152; 64 x 64 43.5 and 52; 32 x 32 12.8, of which four or more share a CU and few are left over) times
+// the most that a CU gets. Measured by 128 / 64 / 32: 564 x 6144 x 2048 156 / 168 / 173 us, 564 x 4096 x 2048 155 / 132 / 116, 564 x 2048 x
+// 2048 152 / 87 / 68, 1200 x 4096 x 4096 546 / 419 / 456, 4096 x 4096 x 4096 1,098 / 1,307 / 1,489. (Tiles of 64 x 32: 162, 115, 72.)
 #define GRID_X (1 << 23)
 // What the entries take: rows as ever, and tiles of 32 x 32 that GRID_X times 256 hold (2 T sums a product).
 #define HB_REQUIRE_TILES(M, N)                                                                                        \
@@ -265,6 +266,10 @@ static void launch_as(const TA* A, const TW* W, TC* C, int M, int N, int K, int 
         return dim3((unsigned)x, (unsigned)((n + x - 1) / x), batch);
     };
     const int stretches = (K + K_BLOCK - 1) / K_BLOCK, wave_threads = HB_WAVE * (stretches < WAVE_WAVES ? stretches : WAVE_WAVES);
+    auto most = [&](int side) { return (double)((tiles(side) + 255) / 256); };
+    // (a decay's exponentials and logarithms are a tile's own tail: not 64 of them a lane)
+    const double large = ep.rate ? 1e30 : tiles(128) <= 256 ? 152.0 : 137.0 * most(128), medium = tiles(64) <= 256 ? 52.0 : 43.5 * most(64),
+                 small = 12.8 * (tiles(32) <= 460 ? 1.8 : tiles(32) / 256.0);
 #define HB_PLAIN_TILE(BM, BK, VEC)                                                                                    \
     gemm_plain_tile_kernel<TA, TW, TC, ACCUM, BM, BM, BK, VEC>                                                        \
         <<<grid(BM), 256, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, batch_a, batch_w, batch_c, ep)
@@ -273,9 +278,9 @@ static void launch_as(const TA* A, const TW* W, TC* C, int M, int N, int K, int 
             A, W, C, M, N, K, lda, ldw, ldc, batch_a, batch_w, batch_c, ep);
     else if (!vec)
         HB_PLAIN_TILE(32, 64, false);
-    else if (tiles(128) >= 512)
+    else if (large <= medium && large <= small)
         HB_PLAIN_TILE(128, 32, true);
-    else if (tiles(64) >= 512)
+    else if (medium <= small)
         HB_PLAIN_TILE(64, 64, true);
     else
         HB_PLAIN_TILE(32, 64, true);
