@@ -239,6 +239,57 @@ __global__ void lru_inputs_kernel(const float* __restrict__ proj, int ld, const 
     out[(size_t)t * 2 * W + W + c] = lru_gelu_tanh(proj[(size_t)t * ld + W + c] + by[c]);
 }
 
+// The same, bit for bit, for filters of four taps over rows in whole quads: four channels a thread along LRU_ROWS tokens, whose last three
+// inputs move through registers, so that a row is read once, 16 bytes a lane. Bound by memory: 1,777 tokens of 2 x 2,048 channels (58 MB)
+// 15.2 us; a channel a thread and every tap a load of its own 31.
+#define LRU_ROWS 8
+__global__ void __launch_bounds__(256)
+lru_inputs_quads_kernel(const float* __restrict__ proj, int ld, const float* __restrict__ bx, const float* __restrict__ by,
+                        const float* __restrict__ taps, const float* __restrict__ fb, const float* __restrict__ conv_state,
+                        const int* __restrict__ seq_of, const int* __restrict__ seq_starts, const int* __restrict__ slots,
+                        float* __restrict__ out, int T, int W) {
+    typedef float quad __attribute__((ext_vector_type(4)));
+    const int c = (blockIdx.y * 256 + threadIdx.x) * 4, t0 = blockIdx.x * LRU_ROWS;
+    if (c >= W) return;
+    quad w[4], x[LRU_ROWS], z[LRU_ROWS], before[CONV_TAPS - 1];       // w[i]: the taps of channel c + i
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = *(const quad*)(taps + (size_t)(c + i) * CONV_TAPS);
+#pragma unroll
+    for (int i = 0; i < LRU_ROWS; ++i) {
+        const float* row = proj + (size_t)min(t0 + i, T - 1) * ld + c;
+        x[i] = *(const quad*)row;
+        z[i] = *(const quad*)(row + W);
+    }
+    const quad b = *(const quad*)(bx + c), start = fb ? *(const quad*)(fb + c) : quad{0.f, 0.f, 0.f, 0.f}, bz = *(const quad*)(by + c);
+    int seq = -1;
+#pragma unroll
+    for (int i = 0; i < LRU_ROWS; ++i) {
+        const int t = t0 + i;
+        if (t >= T) break;
+        if (seq_of[t] != seq) {                                   // the inputs before this row: the step's, or the kept ones
+            seq = seq_of[t];
+            const int first = seq_starts[seq], at = t - first;
+            const float* state = conv_state + (size_t)slots[seq] * (CONV_TAPS - 1) * W + c;
+#pragma unroll
+            for (int j = 0; j < CONV_TAPS - 1; ++j) {
+                const int s = at - (CONV_TAPS - 1) + j;
+                before[j] = s >= 0 ? *(const quad*)(proj + (size_t)(first + s) * ld + c) + b : *(const quad*)(state + (size_t)(CONV_TAPS - 1 + s) * W);
+            }
+        }
+        const quad v = x[i] + b;
+        quad u, g;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            u[e] = fmaf(w[e][3], v[e], fmaf(w[e][2], before[2][e], fmaf(w[e][1], before[1][e], fmaf(w[e][0], before[0][e], start[e]))));
+            g[e] = lru_gelu_tanh(z[i][e] + bz[e]);
+        }
+        before[0] = before[1], before[1] = before[2], before[2] = v;
+        float* to = out + (size_t)t * 2 * W + c;
+        *(quad*)to = u;
+        *(quad*)(to + W) = g;
+    }
+}
+
 extern "C" int hb_lru_inputs(const float* proj, int ld, const float* bx, const float* by, const float* taps,
                              const float* fb, float* conv_state, const int* seq_of, const int* seq_starts,
                              const int* slots, float* out, int T, int B, int W, int K, int longest, hipStream_t stream) {
@@ -247,7 +298,13 @@ extern "C" int hb_lru_inputs(const float* proj, int ld, const float* bx, const f
     HB_REQUIRE((W + 255) / 256 <= 65535 && B <= 65535, "recurrent unit: too many channels or sequences for the grid");
     // one token a sequence at most (longest: the most that a sequence of the step brings): the kernel moves the state on itself
     const int moves_state = longest == 1 && K > 1;
-    lru_inputs_kernel<<<dim3(T, (W + 255) / 256), 256, 0, stream>>>(proj, ld, bx, by, taps, fb, conv_state, seq_of,
+    const uintptr_t places = (uintptr_t)proj | (uintptr_t)bx | (uintptr_t)by | (uintptr_t)taps | (uintptr_t)fb | (uintptr_t)conv_state | (uintptr_t)out;
+    // (few tokens: a thread a token and channel fills more of the chip)
+    if (K == CONV_TAPS && T > 256 && !moves_state && W % 4 == 0 && ld % 4 == 0 && places % 16 == 0)
+        lru_inputs_quads_kernel<<<dim3((T + LRU_ROWS - 1) / LRU_ROWS, (W + 1023) / 1024), 256, 0, stream>>>(
+            proj, ld, bx, by, taps, fb, conv_state, seq_of, seq_starts, slots, out, T, W);
+    else
+        lru_inputs_kernel<<<dim3(T, (W + 255) / 256), 256, 0, stream>>>(proj, ld, bx, by, taps, fb, conv_state, seq_of,
                                                                     seq_starts, slots, out, W, K, moves_state);
     HB_CHECK_LAUNCH("lru_inputs");
     if (K > 1 && !moves_state) {
@@ -325,6 +382,43 @@ __global__ void lru_decay_input_kernel(const float* __restrict__ ug, float* __re
     row[gc] = expf(log_a);
     row[gc + bw] = sqrtf(-expm1f(2.0f * log_a)) * i * ug[t * 2 * W + c];
 }
+// The same, bit for bit, where blocks come in whole quads: four channels a thread along LRU_TOKENS tokens, which share the
+// channels' exponentials of lam; 1,777 tokens of 2,048 channels (73 MB) 20.9 us, a (token, channel) a thread 26.
+#define LRU_TOKENS 4
+__global__ void __launch_bounds__(256)
+lru_decay_input_quads_kernel(const float* __restrict__ ug, float* __restrict__ gates, const float* __restrict__ rb, const float* __restrict__ ib,
+                             const float* __restrict__ lam, float rate, int W, int bw, int T) {
+    typedef float quad __attribute__((ext_vector_type(4)));
+    const int c = (blockIdx.y * 256 + threadIdx.x) * 4, t0 = blockIdx.x * LRU_TOKENS;
+    if (c >= W) return;
+    const int gc = (c / bw) * 2 * bw + c % bw;
+    quad r[LRU_TOKENS], i[LRU_TOKENS], u[LRU_TOKENS], step;
+#pragma unroll
+    for (int k = 0; k < LRU_TOKENS; ++k) {
+        const size_t t = min(t0 + k, T - 1);
+        r[k] = *(const quad*)(gates + t * 2 * W + gc);
+        i[k] = *(const quad*)(gates + t * 2 * W + gc + bw);
+        u[k] = *(const quad*)(ug + t * 2 * W + c);
+    }
+    const quad z = *(const quad*)(lam + c), br = *(const quad*)(rb + c), bi = *(const quad*)(ib + c);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) step[e] = -rate * (z[e] > 20.f ? z[e] : log1pf(expf(z[e])));
+#pragma unroll
+    for (int k = 0; k < LRU_TOKENS; ++k) {
+        if (t0 + k >= T) break;
+        quad a, b;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float opened = 1.0f / (1.0f + expf(-(r[k][e] + br[e]))), taken = 1.0f / (1.0f + expf(-(i[k][e] + bi[e])));
+            const float log_a = step[e] * opened;
+            a[e] = expf(log_a);
+            b[e] = sqrtf(-expm1f(2.0f * log_a)) * taken * u[k][e];
+        }
+        float* row = gates + (size_t)(t0 + k) * 2 * W + gc;
+        *(quad*)row = a;
+        *(quad*)(row + bw) = b;
+    }
+}
 
 template <class TOut, int WIDTH>
 __global__ void __launch_bounds__(1024)
@@ -380,7 +474,11 @@ extern "C" int hb_lru_scan(const float* ug, float* gates, const float* rb, const
     if (longest >= LRU_RUNS_FROM) {
         const size_t total = (size_t)T * W;
         HB_REQUIRE(T > 0 && (total + 255) / 256 <= 0x7fffffffu, "recurrent unit: %d tokens of %d channels exceed the grid", T, W);
-        lru_decay_input_kernel<<<(unsigned)((total + 255) / 256), 256, 0, stream>>>(ug, gates, rb, ib, lam, rate, W, bw, total);
+        const uintptr_t places = (uintptr_t)ug | (uintptr_t)gates | (uintptr_t)rb | (uintptr_t)ib | (uintptr_t)lam;
+        if (bw % 4 == 0 && places % 16 == 0 && W <= 65535 * 1024)
+            lru_decay_input_quads_kernel<<<dim3((T + LRU_TOKENS - 1) / LRU_TOKENS, (W + 1023) / 1024), 256, 0, stream>>>(ug, gates, rb, ib, lam, rate, W, bw, T);
+        else
+            lru_decay_input_kernel<<<(unsigned)((total + 255) / 256), 256, 0, stream>>>(ug, gates, rb, ib, lam, rate, W, bw, total);
         HB_CHECK_LAUNCH("lru_decay_input");
         const bool narrow = (long long)B * ((W + 63) / 64) < 96;
         const int width = narrow ? 16 : 64;
