@@ -47,12 +47,19 @@ __device__ __forceinline__ float silu_mul(float g, float u) {
     return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * u;
 }
 
-// the gated unit of epilogue 2: silu(g) u or max(g, 0) u
+// gelu(g) u with gelu in its tanh form: z (1 + tanh a) / 2 = z / (1 + exp(-2 a)), a = sqrt(2 / pi) (z + 0.044715 z^3), which loses
+// no digits where the tanh is near -1; the reciprocal as above.
+__device__ __forceinline__ float gelu_tanh_mul(float g, float u) {
+    return g * __builtin_amdgcn_rcpf(1.0f + __expf(-1.5957691216f * fmaf(0.044715f * g * g, g, g))) * u;
+}
+
+// the gated unit of epilogue 2: silu(g) u, max(g, 0) u or gelu(g) u
 #define GLU_SILU 0
 #define GLU_RELU 1
+#define GLU_GELU_TANH 2
 template <int GLU>
 __device__ __forceinline__ float glu_mul(float g, float u) {
-    return GLU == GLU_RELU ? fmaxf(g, 0.f) * u : silu_mul(g, u);
+    return GLU == GLU_RELU ? fmaxf(g, 0.f) * u : GLU == GLU_GELU_TANH ? gelu_tanh_mul(g, u) : silu_mul(g, u);
 }
 
 // the activation of epilogue 5: max(z, 0)^2, or the exact gelu z (1 + erf(z / sqrt 2)) / 2. With q = erfc(|z| / sqrt 2) it
@@ -422,8 +429,9 @@ gemm_skinny_kernel(const void* __restrict__ Xv, const bf16* __restrict__ W, void
                     const int n = out_n0 + (a / 2) * 16 + g4 * 4 + i;
                     if (n < N / 2)
                         C[(size_t)m * ldc + n] = hb_from_float<bf16>(
-                            hand.glu == GLU_RELU ? glu_mul<GLU_RELU>(acc[a][b][i], acc[a + 1][b][i])
-                                                 : glu_mul<GLU_SILU>(acc[a][b][i], acc[a + 1][b][i]));
+                            hand.glu == GLU_RELU        ? glu_mul<GLU_RELU>(acc[a][b][i], acc[a + 1][b][i])
+                            : hand.glu == GLU_GELU_TANH ? glu_mul<GLU_GELU_TANH>(acc[a][b][i], acc[a + 1][b][i])
+                                                        : glu_mul<GLU_SILU>(acc[a][b][i], acc[a + 1][b][i]));
                 }
             }
     } else if (EPI == EPI_ACT) {
@@ -1242,6 +1250,9 @@ gemm_tile_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, void* _
             if (scale.glu == GLU_RELU)
                 store_wave_tile_swiglu_lds<TN32, TM32, GLU_RELU>(acc, (bf16*)Cv, M, N, ldc, m0 + wm * TMB * 16,
                                                                  n0 + wn * TNB * 16, lane, stage);
+            else if (scale.glu == GLU_GELU_TANH)
+                store_wave_tile_swiglu_lds<TN32, TM32, GLU_GELU_TANH>(acc, (bf16*)Cv, M, N, ldc, m0 + wm * TMB * 16,
+                                                                 n0 + wn * TNB * 16, lane, stage);
             else
                 store_wave_tile_swiglu_lds<TN32, TM32, GLU_SILU>(acc, (bf16*)Cv, M, N, ldc, m0 + wm * TMB * 16,
                                                                  n0 + wn * TNB * 16, lane, stage);
@@ -1274,6 +1285,8 @@ gemm_tile_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, void* _
             store_wave_tile<EPI_STORE, TN32, TM32>(acc, dst, M, N, N, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
         } else if (EPI == EPI_SWIGLU && scale.glu == GLU_RELU) {
             store_wave_tile<EPI, TN32, TM32, GLU_RELU>(acc, Cv, M, N, ldc, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
+        } else if (EPI == EPI_SWIGLU && scale.glu == GLU_GELU_TANH) {
+            store_wave_tile<EPI, TN32, TM32, GLU_GELU_TANH>(acc, Cv, M, N, ldc, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
         } else {
             store_wave_tile<EPI, TN32, TM32>(acc, Cv, M, N, ldc, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
         }
@@ -1397,6 +1410,8 @@ gemm_tile32_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, void*
     static_assert((int)GLU_RELU == (int)UNARY_GELU, "the second of either kind");
     if ((EPI == EPI_SWIGLU || EPI == EPI_ACT) && glu == GLU_RELU)
         store_wave_tile<EPI, TN32, TM32, GLU_RELU>(acc, Cv, M, N, ldc, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
+    else if (EPI == EPI_SWIGLU && glu == GLU_GELU_TANH)
+        store_wave_tile<EPI, TN32, TM32, GLU_GELU_TANH>(acc, Cv, M, N, ldc, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
     else
         store_wave_tile<EPI, TN32, TM32>(acc, Cv, M, N, ldc, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
 }
@@ -1743,7 +1758,7 @@ extern "C" int hb_gemm_mfma(const void* X, const void* W, void* C, int M, int N,
                             const float* scale_partial, int scale_parts, float scale_eps, float emit_eps,
                             int* deferred_slices, int glu, hipStream_t stream) {
     const NormHandoff hand = {emit_g, (bf16*)emit_xg, emit_partial, scale_partial, scale_parts, scale_eps, emit_eps, glu};
-    HB_REQUIRE(glu == 0 || (glu == 1 && (epi == EPI_SWIGLU || epi == EPI_ACT)), "gemm_mfma: unknown gated unit or activation %d", glu);
+    HB_REQUIRE(glu == 0 || (glu == 1 && (epi == EPI_SWIGLU || epi == EPI_ACT)) || (glu == GLU_GELU_TANH && epi == EPI_SWIGLU), "gemm_mfma: unknown gated unit or activation %d", glu);
     const bool emit_whole = emit_g && !emit_partial;      // the second kernel of a product cut into slices norms
     HB_REQUIRE(!scale_partial || (M <= 16 && !norm_w), "gemm_mfma: a norm is handed on for at most 16 rows");
     HB_REQUIRE(!emit_g || (epi == EPI_ADD && emit_xg && !norm_w), "gemm_mfma: only the adding product leaves a norm behind");
@@ -1828,6 +1843,9 @@ extern "C" int hb_gemm_mfma(const void* X, const void* W, void* C, int M, int N,
                                                                            emit_eps, (bf16*)emit_xg, emit_partial);
         else if (epi == EPI_SWIGLU && glu == GLU_RELU)
             gemm_slices_swiglu_kernel<GLU_RELU><<<(unsigned)((total / 2 + 255) / 256), 256, 0, stream>>>(
+                workspace, (bf16*)C, M, N, ldc, slices);
+        else if (epi == EPI_SWIGLU && glu == GLU_GELU_TANH)
+            gemm_slices_swiglu_kernel<GLU_GELU_TANH><<<(unsigned)((total / 2 + 255) / 256), 256, 0, stream>>>(
                 workspace, (bf16*)C, M, N, ldc, slices);
         else if (epi == EPI_SWIGLU)
             gemm_slices_swiglu_kernel<GLU_SILU><<<(unsigned)((total / 2 + 255) / 256), 256, 0, stream>>>(

@@ -414,7 +414,7 @@ def interleave_gate_up(gate, up):
     return torch.stack([gate.view(I // 16, 16, K), up.view(I // 16, 16, K)], 1).reshape(2 * I, K).contiguous()
 
 
-GATED_UNITS = {"silu": 0, "relu": 1}      # what the epilogue of a gate/up product applies to the gate
+GATED_UNITS = {"silu": 0, "relu": 1, "gelu_tanh": 2}      # what the epilogue of a gate/up product applies to the gate
 
 
 def gemm_swiglu(a, w_interleaved, out, packed=False, norm=None, tile=0, row_scale=None, scratch=None, activation="silu"):
