@@ -14,6 +14,7 @@ TALL_TILES = (128, 192, 256)           # of the matrix-core product of many rows
 MAX_EXPERTS = 1024
 
 
+@functools.lru_cache(maxsize=1024)
 def max_tiles(pairs, experts, rows=TILE_M, shared=0):
     """The length of the list of row tiles for that many (token, expert) pairs and rows of a shared expert."""
     return -(-pairs // rows) + experts + -(-shared // rows)
@@ -49,6 +50,7 @@ class Routing:
         self.weight = weight
 
     @staticmethod
+    @functools.lru_cache(maxsize=1024)
     def ints_needed(T, E, top, tall=0, shared=False):
         rows = T if shared else 0
         return 3 * T * top + rows + E + 3 * max_tiles(T * top, E, shared=rows) + (3 * max_tiles(T * top, E, tall, rows) if tall else 0)
