@@ -144,7 +144,7 @@ class RoutedExperts(Part):
         T, E, top, F = y.shape[0], self.routed, self.top, self.inter
         logits = rt.buffer("moe_logits", (T, self.router_width), torch.float32)
         self.router.forward(y, logits)          # float32 sums of the rows' products with the router's matrix
-        tall = moe.tall_rows(T, top, E, self.experts, self.hidden_size, F) if self.cores else 0
+        tall = moe.tall_rows(T, top, E, self.experts, self.hidden_size, F, self.folded) if self.cores else 0
         routing = moe.Routing(rt.buffer("moe_ints", (moe.Routing.ints_needed(T, E, top, tall, self.folded),), torch.int32),
                               rt.buffer("moe_weight", (T, top), torch.float32), T, E, top, real=self.experts, tall=tall,
                               shared=self.folded)

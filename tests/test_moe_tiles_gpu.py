@@ -113,3 +113,4 @@ def test_tile_heights_by_the_rows_an_expert_has():
     assert moe.tall_rows(768, 4, 32, 32, 2048, 768) == 128
     assert moe.tall_rows(1602, 4, 40, 32, 2048, 768) == 192
     assert moe.tall_rows(1712, 4, 32, 32, 2048, 768) == 256
+    assert moe.tall_rows(1712, 4, 32, 32, 2048, 768, True) == 128
