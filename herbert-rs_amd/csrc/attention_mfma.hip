@@ -905,12 +905,12 @@ constexpr int decode_lds_of(int waves) {      // (four waves of heads of 128: 62
     return decode_own_lds<HD, FUSED>() + (waves - 1) * decode_handed_lds<HD, FUSED>();
 }
 
-// A workgroup is a wave, whose partial results a second kernel merges, or the two to four waves that share a sequence
+// A workgroup is a wave, whose partial results a second kernel merges, or (MERGES) the two to four waves that share a sequence
 // and key head: they cut its own pages into equal ranges and the first of them adds up the others' results, in the order of the
-// ranges, out of LDS and stores the output (one sequence of 100 tokens, heads of 128: 10.4 us, 7.5 and 4.0 with the merge and 1.2
-// between the two; 8 of 121 to 309 tokens: 13.0, 9.6 + 4.7 + 1.2).
-template <int HD, int FUSED, bool EXT, int QS = 1>
-__global__ void __launch_bounds__(256)
+// ranges, out of LDS and stores the output (waves_of_ranges below says where). Two kernels: one for
+// either number of waves cost the single waves 0.2 % of a step (8B shape, 511 tokens: one sequence 3,308 -> 3,314 us, eight 3,585 -> 3,592).
+template <int HD, int FUSED, bool EXT, int QS = 1, bool MERGES = false>
+__global__ void __launch_bounds__(MERGES ? 256 : 64)
 attn_decode_kernel(const bf16* __restrict__ q, bf16* __restrict__ k_cache, bf16* __restrict__ v_cache,
                    float* __restrict__ partial_o, float* __restrict__ partial_ml,
                    const int* __restrict__ context_lens, const int* __restrict__ slots,
@@ -926,10 +926,10 @@ attn_decode_kernel(const bf16* __restrict__ q, bf16* __restrict__ k_cache, bf16*
     // into, and items from ranges[n_seqs] on are nothing. The partial results are then laid out
     // [head, item]: those of one sequence and head lie side by side.
     const int kvh = blockIdx.y, splits = gridDim.z;
-    const int lane = threadIdx.x & 63, c32 = lane & 31, g2 = lane >> 5;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
-    int b = blockIdx.x, split = blockIdx.z + wave;       // (of several waves gridDim.z is 1)
-    if (ranges) {
+    const int lane = MERGES ? threadIdx.x & 63 : threadIdx.x, c32 = lane & 31, g2 = lane >> 5;
+    const int wave = MERGES ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0, waves = MERGES ? blockDim.x >> 6 : 1;
+    int b = blockIdx.x, split = MERGES ? wave : blockIdx.z;
+    if (!MERGES && ranges) {
         const int item = blockIdx.z;
         b = 0;                                              // sequences wholly before the item
         for (int first = 0; first < n_seqs; first += 64) {
@@ -949,7 +949,7 @@ attn_decode_kernel(const bf16* __restrict__ q, bf16* __restrict__ k_cache, bf16*
     const PageWalk walk(lo, keep);                   // (EXT: pages are counted along the walk)
     auto page_at = [&](int v) { return EXT ? walk.page(v) : v; };
     const int hp = EXT ? walk.upto(hi / PAGE) : hi / PAGE;       // the page of the new position
-    if (waves > 1) pages_per_split = (hp - (EXT ? 0 : lo / PAGE) + waves) / waves;
+    if (MERGES) pages_per_split = (hp - (EXT ? 0 : lo / PAGE) + waves) / waves;
     const int first_page = (EXT ? 0 : lo / PAGE) + split * pages_per_split;
     int last_page = first_page + pages_per_split - 1;
     if (last_page > hp) last_page = hp;
@@ -1109,17 +1109,22 @@ attn_decode_kernel(const bf16* __restrict__ q, bf16* __restrict__ k_cache, bf16*
                 _Pragma("unroll") for (int h2 = 0; h2 < 2; ++h2)                             \
                     va[d][kb][h2] = *(const bf16x8*)(vp + (size_t)(d * 32 + c32) * PAGE + kb * 32 + h2 * 16); \
     }
-    extern __shared__ __attribute__((aligned(16))) char decode_lds[];
-    constexpr int HANDED = decode_handed_lds<HD, FUSED>();
-    char* const wave_lds = decode_lds + (wave == 0 ? 0 : decode_own_lds<HD, FUSED>() + (wave - 1) * HANDED);
+    extern __shared__ __attribute__((aligned(16))) char decode_lds[];                         // (MERGES: of the launch)
+    constexpr int OWN = decode_own_lds<HD, FUSED>(), HANDED = decode_handed_lds<HD, FUSED>();
+    __shared__ __attribute__((aligned(16))) char own_lds[MERGES || OWN == 0 ? 16 : OWN];
+    char* const wave_lds = !MERGES ? own_lds : decode_lds + (wave == 0 ? 0 : OWN + (wave - 1) * HANDED);
     bf16* const qs = (bf16*)wave_lds;
     // (FORM_HEADS: a row of the projection normed, and the angles)
     float* const hraw = (float*)(wave_lds + 32 * HD * 2);
     float2* const hturn = (float2*)(hraw + (PRE + 1) * HD);
     // (a wave's own LDS: its accesses happen in their order, only the compiler has to keep it)
     auto wave_sync = []() __attribute__((always_inline)) {
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+        if (MERGES) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        } else {
+            __syncthreads();
+        }
     };
     auto heads_prologue = [&]() __attribute__((always_inline)) {
         if (lane < HD / 2) hturn[lane] = turn;
@@ -1355,7 +1360,7 @@ attn_decode_kernel(const bf16* __restrict__ q, bf16* __restrict__ k_cache, bf16*
 #undef LOAD_K
 #undef LOAD_V
     l += __shfl_xor(l, 32, 64);
-    if (waves > 1) {
+    if constexpr (MERGES) {
         constexpr int ML = HD / 32 * 4 * 64 * 16;
         if (wave > 0) {
             f32x4* const o = (f32x4*)wave_lds;
@@ -1368,7 +1373,7 @@ attn_decode_kernel(const bf16* __restrict__ q, bf16* __restrict__ k_cache, bf16*
         }
         __syncthreads();
         if (wave > 0) return;
-        const char* const handed = decode_lds + decode_own_lds<HD, FUSED>();
+        const char* const handed = decode_lds + OWN;
         float top = m;
         for (int w = 0; w < waves - 1; ++w) top = fmaxf(top, ((const float2*)(handed + w * HANDED + ML))[lane].x);
         // (a range that holds no visible key has a reference of -inf)
@@ -1774,17 +1779,21 @@ extern "C" int hb_attn_decode_mfma(const void* q, void* k_cache, void* v_cache, 
 #define DECODE_ARGS(QPTR) QPTR, (bf16*)k_cache, (bf16*)v_cache, partial_o, partial_ml, context_lens, slots, \
                           page_table, max_pages, nq, nkv, c, window, pages_per_split, fu, direct, ranges, B, \
                           direct ? sinks : nullptr, chunk, softcap / scale, ext, HeadsFusion{}, HeadsOut{}
-#define DECODE_LDS(HDV, FORM) decode_lds_of<HDV, FORM>(waves)
-#define LAUNCH_DECODE_FORM(HDV, FORM) do {                                                               \
-    if (qkv)                                                                                             \
-        attn_decode_kernel<HDV, FORM_FUSED, FORM><<<grid, 64 * waves, DECODE_LDS(HDV, FORM_FUSED), stream>>>(DECODE_ARGS(nullptr));              \
+#define DECODE_GO(HDV, FORM, EXTV, QSV, QPTR) do {                                                       \
+    if (waves > 1)                                                                                       \
+        attn_decode_kernel<HDV, FORM, EXTV, QSV, true>                                                   \
+            <<<grid, 64 * waves, decode_lds_of<HDV, FORM>(waves), stream>>>(DECODE_ARGS(QPTR));          \
     else                                                                                                 \
-        attn_decode_kernel<HDV, FORM_PLAIN, FORM><<<grid, 64 * waves, DECODE_LDS(HDV, FORM_PLAIN), stream>>>(DECODE_ARGS((const bf16*)q));      \
+        attn_decode_kernel<HDV, FORM, EXTV, QSV><<<grid, 64, 0, stream>>>(DECODE_ARGS(QPTR));            \
+    } while (0)
+#define LAUNCH_DECODE_FORM(HDV, EXTV) do {                                                               \
+    if (qkv) DECODE_GO(HDV, FORM_FUSED, EXTV, 1, nullptr);                                               \
+    else DECODE_GO(HDV, FORM_PLAIN, EXTV, 1, (const bf16*)q);                                            \
     } while (0)
 #define LAUNCH_DECODE(HDV) do { if (extended) LAUNCH_DECODE_FORM(HDV, true); else LAUNCH_DECODE_FORM(HDV, false); } while (0)
 #define LAUNCH_SLICES(QSV) do {                                                                          \
-    if (extended) attn_decode_kernel<128, FORM_FUSED, true, QSV><<<grid, 64 * waves, DECODE_LDS(128, FORM_FUSED), stream>>>(DECODE_ARGS(nullptr)); \
-    else attn_decode_kernel<128, FORM_FUSED, false, QSV><<<grid, 64 * waves, DECODE_LDS(128, FORM_FUSED), stream>>>(DECODE_ARGS(nullptr));       \
+    if (extended) DECODE_GO(128, FORM_FUSED, true, QSV, nullptr);                                        \
+    else DECODE_GO(128, FORM_FUSED, false, QSV, nullptr);                                                \
     } while (0)
     if (qkv_slices == 2) LAUNCH_SLICES(2);
     else if (qkv_slices == 4) LAUNCH_SLICES(4);
@@ -1797,7 +1806,7 @@ extern "C" int hb_attn_decode_mfma(const void* q, void* k_cache, void* v_cache, 
 #undef LAUNCH_DECODE
 #undef LAUNCH_DECODE_FORM
 #undef LAUNCH_SLICES
-#undef DECODE_LDS
+#undef DECODE_GO
 #undef DECODE_ARGS
     HB_CHECK_LAUNCH("attn_decode");
     if (!direct) {
@@ -1847,7 +1856,7 @@ extern "C" int hb_attn_decode_heads_mfma(const float* proj, int ld, int slices, 
     const HeadsOut ho = {1, maps, vdim, gate_off < 0 ? nullptr : proj + gate_off, ld, slices, slice_stride, lambda, factor, eps};
     bf16* const direct = splits == 1 ? (bf16*)out : nullptr;
 #define HEADS_GO(HDV, QSV)                                                                                              \
-    attn_decode_kernel<HDV, FORM_HEADS, false, QSV><<<grid, 64, decode_lds_of<HDV, FORM_HEADS>(1), stream>>>( \
+    attn_decode_kernel<HDV, FORM_HEADS, false, QSV><<<grid, 64, 0, stream>>>(                                      \
         nullptr, (bf16*)k_cache, (bf16*)v_cache, partial_o, partial_ml, context_lens, slots, page_table, max_pages, nq, nkv, c,         window, pages_per_split, DecodeFusion{}, direct, ranges, B, direct ? sinks : nullptr, chunk, softcap / scale,           AttnExtras{}, hf, ho)
     if (slices == 2) HEADS_GO(128, 2);
     else if (slices == 4) HEADS_GO(128, 4);
