@@ -907,7 +907,7 @@ constexpr int decode_lds_of(int waves) {      // (four waves of heads of 128: 62
 
 // A workgroup is a wave, whose partial results a second kernel merges, or (MERGES) the two to four waves that share a sequence
 // and key head: they cut its own pages into equal ranges and the first of them adds up the others' results, in the order of the
-// ranges, out of LDS and stores the output (waves_of_ranges below says where). Two kernels: one for
+// ranges, out of LDS and stores the output (_range_waves of mfma.py says where, with both forms' times). Two kernels: one for
 // either number of waves cost the single waves 0.2 % of a step (8B shape, 511 tokens: one sequence 3,308 -> 3,314 us, eight 3,585 -> 3,592).
 template <int HD, int FUSED, bool EXT, int QS = 1, bool MERGES = false>
 __global__ void __launch_bounds__(MERGES ? 256 : 64)
@@ -1629,15 +1629,6 @@ attn_decode_merge_own_kernel(const float* __restrict__ partial_o, const float* _
 // ---------------------------------------------------------------- launchers
 #define LOG2E 1.4426950408889634f
 
-// The waves of a workgroup of the decode kernel that take a sequence's ranges (1: a range is a workgroup, and a second kernel
-// merges them). Where every workgroup has a CU to itself, and four waves make a range longer by a page or two at most: a
-// merge costs a launch and 4 us. More workgroups than CUs leave some CUs with twice the waves of others (384 pairs of two ranges: 58 -> 62 us).
-static int waves_of_ranges(int pairs, int splits, int pages_per_split) {
-    if (pairs > 256) return 1;
-    if (splits <= 4) return splits;
-    return (splits * pages_per_split + 3) / 4 <= pages_per_split + 2 ? 4 : 1;
-}
-
 static int check_extras(const float* rel, int rel_len, int rel_ld, int keep_first, int window, int chunk, float softcap) {
     if (!rel && keep_first == 0) return 0;
     HB_REQUIRE(!rel || (rel_len > 0 && rel_ld >= REL_FRONT + rel_len + REL_BACK), "attention: a table of %d biases in rows of %d", rel_len, rel_ld);
@@ -1742,6 +1733,8 @@ extern "C" int hb_attn_prefill_heads_mfma(const void* q, const void* k_cache, co
 
 // qkv != null: the fused form (see DecodeFusion); q is then not read. qkv_slices > 1 (2, 4 or 8, heads
 // of 128 only): qkv is the first of that many slices of the projection's sums, slice_stride floats apart.
+// waves > 1: a sequence's keys are cut into that many ranges by the kernel, which merges them itself (splits and
+// pages_per_split, which then say no more than that the sequence is not empty, and the partial buffers are not used).
 extern "C" int hb_attn_decode_mfma(const void* q, void* k_cache, void* v_cache, void* out,
                                    float* partial_o, float* partial_ml, const int* context_lens,
                                    const int* slots, const int* page_table, int max_pages, int page_size,
@@ -1750,7 +1743,7 @@ extern "C" int hb_attn_decode_mfma(const void* q, void* k_cache, void* v_cache, 
                                    const float* k_norm_w, const float* cos_t, const float* sin_t, float eps,
                                    int write_kv, int qkv_slices, size_t slice_stride, const int* ranges,
                                    float q_temp_coef, int q_temp_every, const float* sinks, int chunk,
-                                   float softcap, const float* rel, int rel_len, int rel_ld, int keep_first,
+                                   float softcap, const float* rel, int rel_len, int rel_ld, int keep_first, int waves,
                                    hipStream_t stream) {
     const bool extended = rel || keep_first > 0;
     if (check_extras(rel, rel_len, rel_ld, keep_first, window, chunk, softcap)) return 1;
@@ -1769,7 +1762,7 @@ extern "C" int hb_attn_decode_mfma(const void* q, void* k_cache, void* v_cache, 
     HB_REQUIRE(qkv_slices == 1 || (qkv && hd == 128 && (qkv_slices == 2 || qkv_slices == 4 || qkv_slices == 8) &&
                                    slice_stride >= (size_t)B * (nq + 2 * nkv) * hd),
                "attn_decode: %d slices of the projection are not taken here", qkv_slices);
-    const int waves = ranges ? 1 : waves_of_ranges(B * nkv, splits, pages_per_split);
+    HB_REQUIRE(waves == 1 || (waves > 1 && waves <= 4 && !ranges), "attn_decode: %d waves a sequence and kv head", waves);
     dim3 grid(ranges ? 1 : B, nkv, waves > 1 ? 1 : splits);
     const float c = scale * LOG2E;
     const DecodeFusion fu = {qkv, q_norm_w, k_norm_w, cos_t, sin_t, eps, write_kv, slice_stride, q_temp_coef, q_temp_every};

@@ -457,7 +457,7 @@ lib.register_signatures("attention_mfma", {
                                   _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _I, _I, _P, _P, _I, _F, _P],
     "hb_attn_prefill_mfma": [_P, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I, _I, _P, _I, _F, _P, _I, _I, _I, _P],
     "hb_attn_decode_mfma": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _I, _I,
-                            _P, _P, _P, _P, _P, _F, _I, _I, ctypes.c_size_t, _P, _F, _I, _P, _I, _F, _P, _I, _I, _I, _P],
+                            _P, _P, _P, _P, _P, _F, _I, _I, ctypes.c_size_t, _P, _F, _I, _P, _I, _F, _P, _I, _I, _I, _I, _P],
 })
 
 ATTENTION_HEAD_DIMS = (32, 64, 128)
@@ -569,6 +569,31 @@ def _decode_split(meta, nkv, window, chunk=0, keep_first=0):
     return best
 
 
+def _range_waves(pairs, splits, per):
+    """The waves of a workgroup of the decode kernel that share a (sequence, kv head) and merge their ranges in LDS (a wave then takes
+    an equal share of the sequence's own pages); 1: the ranges of _decode_split, a workgroup each, and a second kernel that merges
+    them. That kernel and its launch cost 4 to 6 us a layer, a page more in a wave's chain 2 to 3, and more workgroups than CUs
+    leave some CUs with twice the waves of others. Microseconds of a decode step by the second kernel / 2 / 3 / 4 waves, 28 layers of
+    2,048 on 8 kv heads of 128 (pairs = 8 x sequences):
+       64 pairs  100 tokens 1,443 / 1,401 / 1,408 / 1,414, 220 1,444 / 1,437 / 1,443 / 1,450, 500 1,479 / 1,555 / 1,514 / 1,539
+       96 pairs  220 1,558 / 1,516 / 1,523 / 1,530, 300 1,561 / 1,520 / 1,530 / 1,537, 500 1,591 / 1,641 / 1,597 / 1,625
+      128 pairs  300 1,667 / 1,600 / 1,610 / 1,618, 500 1,709 / 1,733 / 1,686 / 1,711
+      160 pairs  500 1,935 / 1,916 / 1,889 / 1,900, 1,000 2,116 / 2,131 / 2,133 / 2,159, 2,000 2,582 / 2,628 / 2,620 / 2,621
+      192 pairs  700 2,066 / 2,003 / 2,032 / 2,037, 1,530 2,472 / 2,410 / 2,436 / 2,442, 3,000 3,155 / 3,029 / 3,049 / 3,103,
+                 4,090 3,661 / 3,690 / 3,672 / 3,660
+      256 pairs  450 2,111 / 2,058 / 2,039 / 2,052, 1,000 2,418 / 2,342 / 2,336 / 2,362, 4,090 4,333 / 4,329 / 4,211 / 4,268
+    (one sequence of 450 tokens, 4 layers of 1,024: 144 / 157 / 152 / 156, of 100 143.4 / 138.6 / 139.7 / 140.7). So two waves up to
+    four pages, three up to eight from 96 pairs on, and three where the pairs leave room for four or five ranges at most."""
+    pages = splits * per
+    if pairs > 256 or splits == 1:
+        return 1
+    if pages <= 4:
+        return 2
+    if pages <= 8:
+        return 3 if pairs >= 96 else 1
+    return 3 if splits <= 4 or (splits == 5 and pages < 64) else 1
+
+
 def _decode_ranges(meta, nkv, window, chunk=0):
     """(items of the grid, list of ranges on the GPU) for a step whose contexts are of very unequal
     lengths, else None. Equal shares would leave the waves of the short sequences with nothing and
@@ -665,7 +690,7 @@ def attention_decode_fused(qkv, q_norm_w, k_norm_w, cos, sin, meta, kv, out, nq,
              None if k_norm_w is None else k_norm_w.data_ptr(), None if cos is None else cos.data_ptr(),
              None if sin is None else sin.data_ptr(), float(eps), 1, n_slices, stride,
              None if ranges is None else ranges.data_ptr(), coef, every, None if sinks is None else sinks.data_ptr(), 0, 0.0,
-             *extras, _stream())
+             *extras, 1 if ranges is not None else _range_waves(B * nkv, splits, per), _stream())
 
 
 def heads_supported(kv, layout, dtype):
@@ -805,7 +830,8 @@ def attention(q, meta, kv, out, nq, nkv, hd, scale, window, tile_height=None, sc
                  out.data_ptr(), po.data_ptr(), pml.data_ptr(), meta.context_lens.data_ptr(),
                  meta.slots.data_ptr(), kv.page_table.data_ptr(), kv.page_table.shape[1], kv.page_size,
                  T, nq, nkv, hd, float(scale), window, splits, per, None, None, None, None, None, 0.0, 0, 1, 0,
-                 None if ranges is None else ranges.data_ptr(), 0.0, 0, sinks_ptr, chunk, softcap, *extras, _stream())
+                 None if ranges is None else ranges.data_ptr(), 0.0, 0, sinks_ptr, chunk, softcap, *extras,
+                 1 if ranges is not None else _range_waves(T * nkv, splits, per), _stream())
         return
     _check(meta.positions, "positions", torch.int32, (T,))
     height = tile_height or _prefill_tile_height(meta, nkv, nq // nkv)

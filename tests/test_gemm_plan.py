@@ -139,6 +139,32 @@ def test_decode_attention_ranges_by_how_evenly_the_waves_sit():
             assert ranges >= 1 and per >= 1 and ranges * per >= span > (ranges - 1) * per, (b, t)
 
 
+def test_decode_attention_merges_in_a_workgroup_only_where_ranges_stay_short():
+    """The waves of a workgroup that share a (sequence, kv head), by pairs of those and bucket of the context: none where they would
+    make a range several times longer, but for contexts of up to 256 tokens and, where single pages would sit two and more to a
+    CU, of up to 512."""
+    from herbert_rs_amd.kernels import mfma
+
+    class Meta:
+        def __init__(self, seqs, tokens):
+            self.num_seqs, self.context_bucket = seqs, tokens
+    waves = lambda pairs, tokens, window=0: mfma._range_waves(pairs, *mfma._decode_split(Meta(pairs, tokens), 1, window))
+    for pairs in (1, 8, 64, 95):
+        assert waves(pairs, 256) == 2, pairs
+        for tokens in (512, 768, 1024, 1536, 2048, 4096, 32768):
+            assert waves(pairs, tokens) == 1, (pairs, tokens)
+    for pairs in (96, 128, 160):
+        assert [waves(pairs, t) for t in (256, 512, 768, 1024, 2048, 4096)] == [2, 3, 1, 1, 1, 1], pairs
+    assert [waves(192, t) for t in (256, 512, 768, 1024, 3072, 4096)] == [2, 3, 3, 3, 3, 1]
+    assert [waves(256, t) for t in (256, 512, 768, 1024, 2048, 4096)] == [2, 3, 3, 3, 3, 3]
+    assert [waves(257, t) for t in (256, 512, 1024, 4096)] == [1, 1, 1, 1] and waves(600, 256) == 1
+    assert waves(8, 4096, window=64) == 2 and waves(8, 4096, window=400) == 1
+    for pairs, tokens in itertools.product(range(1, 300, 9), (256, 512, 768, 1280, 2048, 8192)):
+        splits, per = mfma._decode_split(Meta(pairs, tokens), 1, 0)
+        n = waves(pairs, tokens)
+        assert n == 1 or splits * per <= 8 or -(-splits * per // n) <= 2 * per, (pairs, tokens)
+
+
 def test_decode_attention_takes_a_list_of_ranges_only_where_it_fits():
     """The list that deals the decode grid out over sequences of unequal lengths: for two sequences
     or more without a window, a round of waves or two items a sequence, up to the kernel's 1,024

@@ -481,6 +481,23 @@ def test_attention_mfma_decode_of_many_sequences_in_shorter_ranges():
     assert mfma._decode_split(meta64, nkv, 0)[0] == 1
 
 
+@pytest.mark.parametrize("waves", [1, 2, 3, 4])
+@pytest.mark.parametrize("nq,nkv,hd", [(8, 2, 128), (3, 1, 64), (4, 4, 32)])
+def test_attention_mfma_decode_by_the_waves_of_a_workgroup(nq, nkv, hd, waves, monkeypatch):
+    """Every number of waves that share a sequence and kv head: fewer pages than waves, equal shares, a last share that is
+    short, and a window that leaves a wave nothing; the bound of the other decode tests."""
+    from herbert_rs_amd.kernels import mfma
+    monkeypatch.setattr(mfma, "_range_waves", lambda *a: waves)
+    lengths = [1, 64, 65, 128, 130, 192, 193, 257, 320, 385, 513, 700]
+    meta, kv, dense = paged_case(lengths, [1] * len(lengths), nkv, hd, torch.bfloat16, seed=6)
+    q = rand(len(lengths), nq * hd, seed=27, dtype=torch.bfloat16)
+    for window in (0, 70, 200):
+        out = torch.full_like(q, 9.0)
+        mfma.attention(q, meta, kv, out, nq, nkv, hd, hd ** -0.5, window)
+        want = attention_reference(q, meta, dense, nq, nkv, hd, hd ** -0.5, window)
+        assert float((out.float().cpu() - want).abs().max()) <= 2 ** -7 * float(want.abs().max()), window
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("nq,nkv,hd,rot,norm", [(4, 2, 128, 128, True), (3, 1, 64, 64, False), (2, 2, 96, 0, True),
                                                 (5, 1, 32, 32, True), (2, 1, 80, 40, True), (1, 1, 256, 256, True),
