@@ -40,6 +40,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 #define EPI_QKV 3
 #define EPI_JOIN 4
 #define EPI_ACT 5
+#define EPI_GEGLU 6          // (epilogue 2 with the gated unit GLU_GELU_TANH, inside this file)
 
 // silu(g) u with the hardware's reciprocal (1 ulp; the result is rounded to bfloat16): a full division
 // is a dozen instructions, and the epilogue of a 256 x 256 tile does 128 of these a lane
@@ -415,7 +416,7 @@ gemm_skinny_kernel(const void* __restrict__ Xv, const bf16* __restrict__ W, void
         }
         return;
     }
-    if (EPI == EPI_SWIGLU) {
+    if (EPI == EPI_SWIGLU || EPI == EPI_GEGLU) {
         bf16* C = (bf16*)Cv;
         const int out_n0 = n0 / 2;
 #pragma unroll
@@ -429,9 +430,9 @@ gemm_skinny_kernel(const void* __restrict__ Xv, const bf16* __restrict__ W, void
                     const int n = out_n0 + (a / 2) * 16 + g4 * 4 + i;
                     if (n < N / 2)
                         C[(size_t)m * ldc + n] = hb_from_float<bf16>(
-                            hand.glu == GLU_RELU        ? glu_mul<GLU_RELU>(acc[a][b][i], acc[a + 1][b][i])
-                            : hand.glu == GLU_GELU_TANH ? glu_mul<GLU_GELU_TANH>(acc[a][b][i], acc[a + 1][b][i])
-                                                        : glu_mul<GLU_SILU>(acc[a][b][i], acc[a + 1][b][i]));
+                            EPI == EPI_GEGLU       ? glu_mul<GLU_GELU_TANH>(acc[a][b][i], acc[a + 1][b][i])
+                            : hand.glu == GLU_RELU ? glu_mul<GLU_RELU>(acc[a][b][i], acc[a + 1][b][i])
+                                                   : glu_mul<GLU_SILU>(acc[a][b][i], acc[a + 1][b][i]));
                 }
             }
     } else if (EPI == EPI_ACT) {
@@ -627,9 +628,11 @@ static void launch_skinny(const void* X, const void* W, void* C, int M, int N, i
         if constexpr (MB == 1 && WAVES == 4) {
             if (packed) {
                 if (epi == EPI_STORE) SKINNY_GO(EPI_STORE, true, true);
+                else if (hand.glu == GLU_GELU_TANH) SKINNY_GO(EPI_GEGLU, true, true);
                 else SKINNY_GO(EPI_SWIGLU, true, true);
             } else {
                 if (epi == EPI_STORE) SKINNY_GO(EPI_STORE, false, true);
+                else if (hand.glu == GLU_GELU_TANH) SKINNY_GO(EPI_GEGLU, false, true);
                 else SKINNY_GO(EPI_SWIGLU, false, true);
             }
         }
@@ -637,11 +640,13 @@ static void launch_skinny(const void* X, const void* W, void* C, int M, int N, i
         if (epi == EPI_STORE) SKINNY_GO(EPI_STORE, true, false);
         else if (epi == EPI_ADD) SKINNY_GO(EPI_ADD, true, false);
         else if (epi == EPI_ACT) SKINNY_GO(EPI_ACT, true, false);
+        else if (hand.glu == GLU_GELU_TANH) SKINNY_GO(EPI_GEGLU, true, false);
         else SKINNY_GO(EPI_SWIGLU, true, false);
     } else {
         if (epi == EPI_STORE) SKINNY_GO(EPI_STORE, false, false);
         else if (epi == EPI_ADD) SKINNY_GO(EPI_ADD, false, false);
         else if (epi == EPI_ACT) SKINNY_GO(EPI_ACT, false, false);
+        else if (hand.glu == GLU_GELU_TANH) SKINNY_GO(EPI_GEGLU, false, false);
         else SKINNY_GO(EPI_SWIGLU, false, false);
     }
 #undef SKINNY_GO
@@ -1243,15 +1248,15 @@ gemm_tile_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, void* _
         const bool sliced = gridDim.y > 1;
         float* const dst = sliced ? partial + (size_t)blockIdx.y * M * N : (float*)Cv;
         const int ld = sliced ? N : ldc;
-        constexpr bool SWIGLU_VIA_LDS = EPI == EPI_SWIGLU && BM >= 128 && REGION >= 32 * TM32 * TN32 * 32;
+        constexpr bool SWIGLU_VIA_LDS = (EPI == EPI_SWIGLU || EPI == EPI_GEGLU) && BM >= 128 && REGION >= 32 * TM32 * TN32 * 32;
         if (SWIGLU_VIA_LDS && !sliced && (ldc & 7) == 0 && ((size_t)Cv & 15) == 0) {
             hb_workgroup_barrier();
             bf16* const stage = (bf16*)((char*)lds + wave * REGION);
-            if (scale.glu == GLU_RELU)
-                store_wave_tile_swiglu_lds<TN32, TM32, GLU_RELU>(acc, (bf16*)Cv, M, N, ldc, m0 + wm * TMB * 16,
-                                                                 n0 + wn * TNB * 16, lane, stage);
-            else if (scale.glu == GLU_GELU_TANH)
+            if constexpr (EPI == EPI_GEGLU)
                 store_wave_tile_swiglu_lds<TN32, TM32, GLU_GELU_TANH>(acc, (bf16*)Cv, M, N, ldc, m0 + wm * TMB * 16,
+                                                                      n0 + wn * TNB * 16, lane, stage);
+            else if (scale.glu == GLU_RELU)
+                store_wave_tile_swiglu_lds<TN32, TM32, GLU_RELU>(acc, (bf16*)Cv, M, N, ldc, m0 + wm * TMB * 16,
                                                                  n0 + wn * TNB * 16, lane, stage);
             else
                 store_wave_tile_swiglu_lds<TN32, TM32, GLU_SILU>(acc, (bf16*)Cv, M, N, ldc, m0 + wm * TMB * 16,
@@ -1285,8 +1290,8 @@ gemm_tile_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, void* _
             store_wave_tile<EPI_STORE, TN32, TM32>(acc, dst, M, N, N, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
         } else if (EPI == EPI_SWIGLU && scale.glu == GLU_RELU) {
             store_wave_tile<EPI, TN32, TM32, GLU_RELU>(acc, Cv, M, N, ldc, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
-        } else if (EPI == EPI_SWIGLU && scale.glu == GLU_GELU_TANH) {
-            store_wave_tile<EPI, TN32, TM32, GLU_GELU_TANH>(acc, Cv, M, N, ldc, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
+        } else if constexpr (EPI == EPI_GEGLU) {
+            store_wave_tile<EPI_SWIGLU, TN32, TM32, GLU_GELU_TANH>(acc, Cv, M, N, ldc, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
         } else {
             store_wave_tile<EPI, TN32, TM32>(acc, Cv, M, N, ldc, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
         }
@@ -1410,8 +1415,8 @@ gemm_tile32_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, void*
     static_assert((int)GLU_RELU == (int)UNARY_GELU, "the second of either kind");
     if ((EPI == EPI_SWIGLU || EPI == EPI_ACT) && glu == GLU_RELU)
         store_wave_tile<EPI, TN32, TM32, GLU_RELU>(acc, Cv, M, N, ldc, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
-    else if (EPI == EPI_SWIGLU && glu == GLU_GELU_TANH)
-        store_wave_tile<EPI, TN32, TM32, GLU_GELU_TANH>(acc, Cv, M, N, ldc, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
+    else if constexpr (EPI == EPI_GEGLU)
+        store_wave_tile<EPI_SWIGLU, TN32, TM32, GLU_GELU_TANH>(acc, Cv, M, N, ldc, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
     else
         store_wave_tile<EPI, TN32, TM32>(acc, Cv, M, N, ldc, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
 }
@@ -1447,11 +1452,13 @@ static int launch_tiles(Kernel kern, size_t lds, int threads, long total, int sl
             if (epi == EPI_STORE) return launch_tiles(KERNEL<EPI_STORE, true, __VA_ARGS__>, lds, threads, total, slices, x, w, C, M, N, K, ldc, m_tiles, n_tiles, stream EXTRA); \
             if (epi == EPI_ADD) return launch_tiles(KERNEL<EPI_ADD, true, __VA_ARGS__>, lds, threads, total, slices, x, w, C, M, N, K, ldc, m_tiles, n_tiles, stream EXTRA); \
             if (epi == EPI_ACT) return launch_tiles(KERNEL<EPI_ACT, true, __VA_ARGS__>, lds, threads, total, slices, x, w, C, M, N, K, ldc, m_tiles, n_tiles, stream EXTRA); \
+            if (glu == GLU_GELU_TANH) return launch_tiles(KERNEL<EPI_GEGLU, true, __VA_ARGS__>, lds, threads, total, slices, x, w, C, M, N, K, ldc, m_tiles, n_tiles, stream EXTRA); \
             return launch_tiles(KERNEL<EPI_SWIGLU, true, __VA_ARGS__>, lds, threads, total, slices, x, w, C, M, N, K, ldc, m_tiles, n_tiles, stream EXTRA); \
         }                                                                                            \
         if (epi == EPI_STORE) return launch_tiles(KERNEL<EPI_STORE, false, __VA_ARGS__>, lds, threads, total, slices, x, w, C, M, N, K, ldc, m_tiles, n_tiles, stream EXTRA); \
         if (epi == EPI_ADD) return launch_tiles(KERNEL<EPI_ADD, false, __VA_ARGS__>, lds, threads, total, slices, x, w, C, M, N, K, ldc, m_tiles, n_tiles, stream EXTRA); \
         if (epi == EPI_ACT) return launch_tiles(KERNEL<EPI_ACT, false, __VA_ARGS__>, lds, threads, total, slices, x, w, C, M, N, K, ldc, m_tiles, n_tiles, stream EXTRA); \
+        if (glu == GLU_GELU_TANH) return launch_tiles(KERNEL<EPI_GEGLU, false, __VA_ARGS__>, lds, threads, total, slices, x, w, C, M, N, K, ldc, m_tiles, n_tiles, stream EXTRA); \
         return launch_tiles(KERNEL<EPI_SWIGLU, false, __VA_ARGS__>, lds, threads, total, slices, x, w, C, M, N, K, ldc, m_tiles, n_tiles, stream EXTRA); \
     } while (0)
 
@@ -1471,6 +1478,7 @@ static int launch_tile64(const void* X, const void* W, void* C, int M, int N, in
     // (a handed-on norm and K slices go together: every slice's sums are scaled, and so is their sum)
     HB_REQUIRE(!scale.partial || (M <= 16 && epi != EPI_ADD), "gemm_mfma: this product takes no handed-on norm");
     HB_REQUIRE((K / 64 + slices - 1) / slices * (slices - 1) < K / 64, "gemm_mfma: a slice of K would be empty");
+    const int glu = scale.glu;
 #define EXTRA , partial, QkvEpilogue{}, scale
     TILE_DISPATCH(gemm_tile_kernel, TNB, TMB, WNW, WMW, WST, XST);
 #undef EXTRA
@@ -1490,11 +1498,16 @@ static int launch_tile64_swiglu(const void* X, const void* W, void* C, int M, in
     const size_t lds = (size_t)(WST * BN + XST * BM) * 64 * sizeof(bf16) + WNW * WMW * 16 * sizeof(float);
     const bf16* x = (const bf16*)X;
     const bf16* w = (const bf16*)W;
-    if (packed)
-        return launch_tiles(gemm_tile_kernel<EPI_SWIGLU, true, TNB, TMB, WNW, WMW, WST, XST>, lds, 64 * WNW * WMW, total, 1,
-                            x, w, C, M, N, K, ldc, m_tiles, n_tiles, stream, (float*)nullptr, QkvEpilogue{}, scale);
-    return launch_tiles(gemm_tile_kernel<EPI_SWIGLU, false, TNB, TMB, WNW, WMW, WST, XST>, lds, 64 * WNW * WMW, total, 1,
-                        x, w, C, M, N, K, ldc, m_tiles, n_tiles, stream, (float*)nullptr, QkvEpilogue{}, scale);
+#define SWIGLU_GO(EPIV, PK)                                                                                                    \
+    return launch_tiles(gemm_tile_kernel<EPIV, PK, TNB, TMB, WNW, WMW, WST, XST>, lds, 64 * WNW * WMW, total, 1, x, w, C, M, N, K, \
+                        ldc, m_tiles, n_tiles, stream, (float*)nullptr, QkvEpilogue{}, scale)
+    if (scale.glu == GLU_GELU_TANH) {
+        if (packed) SWIGLU_GO(EPI_GEGLU, true);
+        SWIGLU_GO(EPI_GEGLU, false);
+    }
+    if (packed) SWIGLU_GO(EPI_SWIGLU, true);
+    SWIGLU_GO(EPI_SWIGLU, false);
+#undef SWIGLU_GO
 }
 
 template <int TNB, int TMB, int WNW, int WMW, int STAGES>
@@ -1743,8 +1756,8 @@ extern "C" double hb_gemm_mfma_plan_cost(int M, int N, int K, int epi, int norme
 }
 
 // C (+)= X @ W^T. X [M, K] bf16, W [N, K] bf16. epi 0: C f32 [M, N] stored; 1: added to;
-// 2: W's rows are gate/up interleaved in blocks of 16 and C is bf16 [M, N / 2] = silu(gate) * up (glu 0), or
-// max(gate, 0) * up (glu 1); 5: C is bf16 [M, N], every sum through the activation that glu names (unary).
+// 2: W's rows are gate/up interleaved in blocks of 16 and C is bf16 [M, N / 2] = silu(gate) * up (glu 0),
+// max(gate, 0) * up (glu 1) or gelu(gate) * up with gelu in its tanh form (glu 2); 5: C is bf16 [M, N], every sum through the activation that glu names (unary).
 // packed != 0: W is stored as [K / 32][N / 16][64 lanes][8]: lane = 16 * (k / 8 % 4) + n % 16.
 // All blocks of one k-step lie together: workgroups that advance through K side by side read one
 // contiguous stretch of memory at a time, as a streaming copy would.
