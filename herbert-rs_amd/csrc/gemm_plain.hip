@@ -72,7 +72,7 @@ __device__ __forceinline__ void store_quad(TC* C, int ldc, int m, int n, int N, 
 // wants k = k0 + lane / 16 from a lane, so within every 16 k LDS holds a row's elements transposed, element 4 s + q at
 // place 4 q + s: a lane's next four products are then one 16-byte read. Rows are BK + 4 floats apart: the reads of 16
 // rows meet no bank twice. Bound by the matrix cores (a library's large product reaches 154 TFLOP/s here):
-// 4096 x 4096 x 4096 in 1,082 us (127 TFLOP/s), 564 x 6144 x 2048 in 165, 564 x 2048 x 2048 in 67, 64 x 4096 x 4096 in
+// 4096 x 4096 x 4096 in 1,098 us (125 TFLOP/s), 564 x 6144 x 2048 in 156, 564 x 2048 x 2048 in 68, 64 x 4096 x 4096 in
 // 55; the kernel of vector FMAs and 4-byte loads that this replaced took 2,465, 372, 323 and 632.
 template <class TA, class TW, class TC, bool ACCUM, int BM, int BN, int BK, bool VEC>
 __global__ void __launch_bounds__(256, 2)
@@ -176,8 +176,7 @@ gemm_plain_tile_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
 // lanes' quads are transposed in registers. The stretches' sums meet in LDS, where a thread an output adds them in
 // their order. 2 x 2048 x 2048 takes 10.7 us (one wave for all of k, a chain of 512 products with eight blocks in
 // flight: 19.4), 2 x 2048 x 3072 12.8 (27.9), 2 x 4096 x 2048 13.3 (20.0), 8 x 4096 x 12288 62 (106); with bfloat16
-// weights 10.5 (36), 12.9 (53), 11 (38) and 43 (233). Wide weights stream: 2 x 6144 x 2048 19.9 (21.3), 2 x 32768 x
-// 2048 64 (60; a wave after the other's stretches there, so that no workgroup waits for another's: 83).
+// weights 10.5 (36), 12.9 (53), 11 (38) and 43 (233).
 #define WAVE_ROWS 16
 #define WAVE_WAVES 8
 #define WAVE_DEPTH 8
@@ -241,8 +240,56 @@ gemm_plain_wave_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
     if (wave == 0 && r < M) store_quad<TC, ACCUM, true>(C, ldc, r, n0 + 4 * q, N, total, ep);
 }
 
+// The same rows for float32 weights that fill the chip with a wave for every 16 of their rows, or whose k is so short that there
+// is nothing to share: no LDS and no barrier; a wave goes through the stretches one after another, the next WAVE_DEPTH blocks of 16 k of
+// W and A on their way while the WAVE_DEPTH before are multiplied. Microseconds by the kernel above / this one, two rows: 4096 x 480 10.8 /
+// 6.8, 2048 x 896 10.8 / 10.0, 4096 x 1024 9.4 / 11.3, 8192 x 1024 13.8 / 12.5, 8192 x 1504 20.7 / 17.3, 8192 x 2048 20.1 / 21.7, 12288 x 2048 24.1 /
+// 23.6, 12288 x 4096 46.7 / 42.2, 32768 x 2048 61.6 / 54.6, 4096 x 64 2.9 / 3.0, 4096 x 16 2.4 / 3.1. With bfloat16 weights it is the slower one
+// everywhere (32768 x 2048 46.9 / 79.4).
+template <class TA, class TW, class TC, bool ACCUM>
+__global__ void __launch_bounds__(HB_WAVE)
+gemm_plain_stream_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* __restrict__ C, int M, int N,
+                         int K, int lda, int ldw, int ldc, size_t batch_a, size_t batch_w, size_t batch_c,
+                         DecayEpilogue ep) {
+    A += blockIdx.z * batch_a;
+    W += blockIdx.z * batch_w;
+    C += blockIdx.z * batch_c;
+    static_assert(K_BLOCK % (16 * WAVE_DEPTH) == 0, "a stretch of k is whole rounds of loads");
+    const int lane = threadIdx.x, r = lane & 15, q = lane >> 4;
+    const int n0 = blockIdx.x * 16;
+    // (rows beyond M or N are row 0 once more, whose sums go nowhere; blocks beyond K are zeros)
+    const TW* w_row = W + (size_t)(n0 + r < N ? n0 + r : 0) * ldw + 4 * q;
+    const TA* a_row = A + (size_t)(r < M ? r : 0) * lda + 4 * q;
+    f32x4 total = {0.f, 0.f, 0.f, 0.f}, acc = total, w_next[WAVE_DEPTH], a_next[WAVE_DEPTH];
+    auto fetch = [&](int k0) {
+#pragma unroll
+        for (int d = 0; d < WAVE_DEPTH; ++d) {
+            const int k = k0 + 16 * d;
+            w_next[d] = load_quad<true>(w_row + k, K - k);
+            a_next[d] = load_quad<true>(a_row + k, K - k);
+        }
+    };
+    fetch(0);
+    for (int k0 = 0; k0 < K; k0 += 16 * WAVE_DEPTH) {
+        f32x4 w[WAVE_DEPTH], a[WAVE_DEPTH];
+#pragma unroll
+        for (int d = 0; d < WAVE_DEPTH; ++d) w[d] = w_next[d], a[d] = a_next[d];
+        const bool more = k0 + 16 * WAVE_DEPTH < K;
+        if (more) fetch(k0 + 16 * WAVE_DEPTH);
+#pragma unroll
+        for (int d = 0; d < WAVE_DEPTH; ++d) {
+            transpose_quads(w[d]);
+            transpose_quads(a[d]);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) acc = mfma_k4(w[d][s], a[d][s], acc);
+        }
+        if (!more || (k0 + 16 * WAVE_DEPTH) % K_BLOCK == 0) total += acc, acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    if (r < M) store_quad<TC, ACCUM, true>(C, ldc, r, n0 + 4 * q, N, total, ep);
+}
+
 // The kernel of a product. 16-byte loads and stores where rows and strides allow them. Up to 16 rows of whole blocks of
-// 16 k take the wave kernel. Beyond, the tile with the least estimated time: what a CU spends on one (microseconds at K = 2048 on all
+// 16 k take one of the two kernels above. Beyond, the tile with the least estimated time: what a CU spends on one (microseconds at K = 2048 on all
 // CUs: 128 x 128 137, alone on a CU 152; 64 x 64 43.5 and 52; 32 x 32 12.8, of which four or more share a CU and few are left over) times
 // the most that a CU gets. Measured by 128 / 64 / 32: 564 x 6144 x 2048 156 / 168 / 173 us, 564 x 4096 x 2048 155 / 132 / 116, 564 x 2048 x
 // 2048 152 / 87 / 68, 1200 x 4096 x 4096 546 / 419 / 456, 4096 x 4096 x 4096 1,098 / 1,307 / 1,489. (Tiles of 64 x 32: 162, 115, 72.)
@@ -273,7 +320,13 @@ static void launch_as(const TA* A, const TW* W, TC* C, int M, int N, int K, int 
 #define HB_PLAIN_TILE(BM, BK, VEC)                                                                                    \
     gemm_plain_tile_kernel<TA, TW, TC, ACCUM, BM, BM, BK, VEC>                                                        \
         <<<grid(BM), 256, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, batch_a, batch_w, batch_c, ep)
-    if (vec && M <= WAVE_ROWS && K % 16 == 0)
+    // (both sides of these lines stand at gemm_plain_stream_kernel)
+    const long long strips = (N + 15ll) / 16 * batch;
+    const bool streams = sizeof(TW) == 4 && K > 64 && (K < 1024 || strips >= 768 || (K < 2048 && strips >= 512));
+    if (vec && M <= WAVE_ROWS && K % 16 == 0 && streams)
+        gemm_plain_stream_kernel<TA, TW, TC, ACCUM><<<dim3((N + 15) / 16, 1, batch), HB_WAVE, 0, stream>>>(
+            A, W, C, M, N, K, lda, ldw, ldc, batch_a, batch_w, batch_c, ep);
+    else if (vec && M <= WAVE_ROWS && K % 16 == 0)
         gemm_plain_wave_kernel<TA, TW, TC, ACCUM><<<dim3((N + 15) / 16, 1, batch), wave_threads, 0, stream>>>(
             A, W, C, M, N, K, lda, ldw, ldc, batch_a, batch_w, batch_c, ep);
     else if (!vec)

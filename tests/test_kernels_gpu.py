@@ -85,6 +85,24 @@ def test_gemm_plain_stretches_of_k_are_the_same_in_every_kernel(K, wd):
     assert bool(((got[40].double() - want).abs() <= steps * 2.0 ** -24 * size + 1e-30).all())
 
 
+@pytest.mark.parametrize("N,K", [(100, 80), (100, 480), (4, 512), (60, 528), (100, 1008), (8196, 1504), (12292, 1024), (12276, 2064), (12272, 2064)])
+@pytest.mark.parametrize("ad", [torch.float32, torch.bfloat16])
+def test_gemm_plain_rows_that_stream_are_the_same_bits(N, K, ad):
+    """Up to 16 rows on float32 weights of short k or of many rows: a wave goes through the stretches by itself. The same
+    bits as among 40 rows (tiles), with and without adding to what is there; the last widths lie on either side of the line."""
+    from herbert_rs_amd.kernels import ops
+    a, w, start = rand(40, K, seed=25, dtype=ad), rand(N, K, seed=26), rand(40, N, seed=27)
+    for accumulate in (False, True):
+        got = {}
+        for rows in (1, 16, 40):
+            got[rows] = start[:rows].clone()
+            ops.gemm_plain(a[:rows].contiguous(), w, got[rows], accumulate=accumulate)
+        assert torch.equal(got[1], got[16][:1]) and torch.equal(got[16], got[40][:16])
+    want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T + start.double().abs()
+    steps = min(K, 512) + (K + 511) // 512 + 1
+    assert bool(((got[40].double() - start.double() - want).abs() <= steps * 2.0 ** -24 * size + 1e-30).all())
+
+
 def test_gemm_plain_of_more_tiles_than_a_grids_x_holds():
     """The most rows that are taken, of a width whose tiles of 32 x 32 times 256 threads pass 2^32: whole numbers, so every
     sum is exact in bfloat16."""
