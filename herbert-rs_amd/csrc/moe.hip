@@ -771,7 +771,7 @@ grouped_mfma_kernel(const bf16* __restrict__ A, int lda, size_t a_group_off, con
 // out between the products, the reads of a k-step during the products of the one before. An activation row is 128 bytes, its 16-byte
 // chunk c at chunk c ^ ((row >> 1) & 7); a block of 16 weight rows and 32 k is 1 KB as packed. K in steps of 64.
 // Gate/up of 32 experts of 768 on 2,048, weights from memory (40 us at the rate of a large copy), by tiles of 64 and by the tile that
-// tall_rows of moe.py takes: 2,048 tokens, four experts each, 127 us, 90 (128 rows); 1,712 103, 76 (256); 1,282 101, 60 (192); 512 63, 49
+// tall_rows of moe.py takes: 2,048 tokens, four experts each, 127 us, 90 (128 rows); 1,712 (without a shared expert) 103, 76 (256); 1,282 101, 60 (192); 512 63, 49
 // (128). 64 experts of 1,536 on 4,096, 2,500 tokens: 522, 353 (192).
 typedef float hb_f32x16 __attribute__((ext_vector_type(16)));
 #define TALL_BN 256

@@ -167,10 +167,13 @@ def mfma_takes(K, lda, a_group_off=0, N=16):
 def tall_rows(T, top, routed, experts, hidden, inter, shared=False):
     """The rows of a tall tile (0: none) for a step of T tokens, each on `top` of `routed` outputs of the router, the first `experts` of which have
     bfloat16 matrices in the cores' order. Tall tiles from TALL_ROWS rows an expert on, for sizes that they take; of those the one
-    that brings the fewest bytes into a CU: rounds of tiles over the CUs times weight and activation rows of a step (an
-    expert's rows are taken to be spread around their mean as a random choice spreads them, and a round to be full at nine tenths, since
-    some experts of a model are busier than that: 234 expected tiles of 256 rows took 126 us, two rounds; tiles of 128 take a layer's
-    step 33 us less). shared: every token takes one more expert."""
+    that brings the fewest bytes into a CU: rounds of tiles over the CUs times weight and activation rows of a step. An expert's rows are
+    taken to be spread around their mean as a random choice spreads them, and a round to be full at nine tenths, since some experts of a
+    model are busier than that. Over 132 layers (16 to 256 experts, 400 to 4,096 tokens) the height that this gives is 2.3 % slower than
+    the best one where experts are chosen at random (2.1 with rounds full to the last tile, 7.8 full at eight tenths) and 10.3 % where
+    they are very unequally busy, deviations of 0.5 to 1.2 of the mean (11.2, 9.3): there one height for all experts costs a round that
+    is nearly empty more often than not. An estimate that averaged the rounds over both kinds of routing was better by a tenth of
+    a layer's time at some token counts and worse by as much at others. shared: every token takes one more expert."""
     rows = T * top / routed
     if rows < TALL_ROWS or hidden % 64 or inter % 64:
         return 0
@@ -184,6 +187,21 @@ def tall_rows(T, top, routed, experts, hidden, inter, shared=False):
         return (experts * tiles + (-(-T // height) if shared else 0)) * columns
     fits = [h for h in TALL_TILES if workgroups(h) >= 128]
     return min(fits, key=lambda h: math.ceil(workgroups(h) / 256 + 0.1) * (256 + h), default=0)
+
+
+def fold_pays(T, top, experts, hidden, inter):
+    """True if a step of T tokens takes a shared expert of the others' size as one more of them: its two products and the kernel between
+    them go, and its rows follow the pairs' in the experts' products. Microseconds of a layer with the shared expert's own products /
+    folded: 32 experts of 768 on 2,048, four each: 8 tokens 66 / 56, 128 124 / 111, 512 134 / 110, 2,048 249 / 227; 64 of 1,408, six
+    each: 128 tokens 253 / 245, 512 307 / 296. In steps of few rows an expert (the form that streams the matrices) a tile of 64 of the
+    shared expert's rows reads its matrices again, which a dense product does not: 128 of 768, one each: 512 tokens 156 / 152, 1,024
+    200 / 216, 2,048 273 / 315; 256 of 512, eight each: 512 tokens 319 / 312; 64 of 1,536 on 4,096, four each: 32 tokens 304 / 299,
+    64 343 / 349, 128 398 / 408, 256 520 / 526, and beyond those steps 512 505 / 461, 1,024 629 / 565."""
+    if T * top > FEW_ROWS * experts:
+        return True
+    if hidden * inter >= 4 << 20:
+        return T <= 32
+    return -(-T // TILE_M) * hidden * inter <= 13 << 20
 
 
 def pack_grouped(w):

@@ -103,11 +103,10 @@ class RoutedExperts(Part):
         # bfloat16 with sizes the matrix cores take: the matrices are kept in their operands' order
         self.cores = (rt.dtype == torch.bfloat16 and moe.mfma_takes(W, W, 0, 2 * F) and moe.mfma_takes(F, F, 0, W)
                       and F % 16 == 0)
-        # a shared expert of the others' size and activation is one more of them, with a row for every token: its two products
-        # and the kernel between them (18 us a layer for eight tokens, 32 experts of 768 on 2,048) go, and the experts' products grow
-        # by one expert's tiles (2 us)
-        self.folded = (self.cores and self.shared_expert is not None and self.shared_expert[0] == F
-                       and (self.limit, self.alpha, self.shift) == (math.inf, 1.0, 0.0))
+        # a shared expert of the others' size and activation can be one more of them, with a row for every token, in the steps where
+        # that pays (moe.fold_pays); its matrices are kept in either form
+        self.foldable = (self.cores and self.shared_expert is not None and self.shared_expert[0] == F
+                         and (self.limit, self.alpha, self.shift) == (math.inf, 1.0, 0.0))
         matrices = [n] * self.experts
         if self.shared_expert is not None:
             # the shared expert's gate is one more row of the router's product (rows up to a multiple of
@@ -118,9 +117,8 @@ class RoutedExperts(Part):
             wide[:self.experts] = router
             wide[self.experts] = rt.weight(tensors[sn["sg"]])[0]
             router = wide
-        if self.folded:
-            matrices.append(sn)
-        elif self.shared_expert is not None:
+            if self.foldable:
+                matrices.append(sn)
             gate, up = rt.weight(tensors[sn["gate"]]), rt.weight(tensors[sn["up"]])
             self.shared_fused = (rt.dtype == torch.bfloat16 and Fs % 16 == 0 and self.hidden_size % 32 == 0
                                  and mfma.gemm_supported(gate[:1], gate, swiglu=True))
@@ -138,23 +136,24 @@ class RoutedExperts(Part):
         self.down = torch.stack([rt.weight(tensors[m["down"].format(e=e)]) for e, m in enumerate(matrices)]).contiguous()
         if self.cores:
             self.gate_up, self.down = moe.pack_grouped(self.gate_up), moe.pack_grouped(self.down)
+            self.routed_alone = self.gate_up[:self.experts], self.down[:self.experts]
 
     def forward(self, ctx, y, x):
         rt = ctx.rt
         T, E, top, F = y.shape[0], self.routed, self.top, self.inter
         logits = rt.buffer("moe_logits", (T, self.router_width), torch.float32)
         self.router.forward(y, logits)          # float32 sums of the rows' products with the router's matrix
-        tall = moe.tall_rows(T, top, E, self.experts, self.hidden_size, F, self.folded) if self.cores else 0
-        routing = moe.Routing(rt.buffer("moe_ints", (moe.Routing.ints_needed(T, E, top, tall, self.folded),), torch.int32),
-                              rt.buffer("moe_weight", (T, top), torch.float32), T, E, top, real=self.experts, tall=tall,
-                              shared=self.folded)
+        folded = self.foldable and moe.fold_pays(T, top, E, self.hidden_size, F)
+        tall = moe.tall_rows(T, top, E, self.experts, self.hidden_size, F, folded) if self.cores else 0
+        routing = moe.Routing(rt.buffer("moe_ints", (moe.Routing.ints_needed(T, E, top, tall, folded),), torch.int32),
+                              rt.buffer("moe_weight", (T, top), torch.float32), T, E, top, real=self.experts, tall=tall, shared=folded)
         if self.routing == "scores":
             moe.route(logits, self.router_bias, routing, scores=True, groups=self.groups, keep=self.keep,
                       score=self.scoring, worth_top=self.group_worth, renorm=self.renormalize)
         else:
             moe.route(logits, self.router_bias, routing)
         shared = None
-        if self.shared_expert is not None and not self.folded:
+        if self.shared_expert is not None and not folded:
             Fs = self.shared_expert[0]
             s_act = rt.buffer("moe_shared_act", (T, Fs))
             if self.shared_fused:
@@ -169,16 +168,17 @@ class RoutedExperts(Part):
         out = rt.buffer("moe_out", (routing.rows, self.hidden_size), torch.float32)
         if self.cores:
             # matrix cores; the activation is the first product's epilogue
-            moe.grouped_mfma(y, self.hidden_size, 0, self.gate_up, act, F, 0, moe.EPI_GLU, routing, gather=True,
+            gate_up, down = (self.gate_up, self.down) if folded else self.routed_alone
+            moe.grouped_mfma(y, self.hidden_size, 0, gate_up, act, F, 0, moe.EPI_GLU, routing, gather=True,
                              limit=self.limit, alpha=self.alpha, shift=self.shift, tall=tall > 0)
-            moe.grouped_mfma(act, F, 0, self.down, out, self.hidden_size, 0, moe.EPI_F32, routing,
+            moe.grouped_mfma(act, F, 0, down, out, self.hidden_size, 0, moe.EPI_F32, routing,
                              tall=tall > 0 and F >= 64 * moe.DOWN_STEPS and T * top >= moe.DOWN_ROWS * E)
         else:
             gu = rt.buffer("moe_gate_up", (T * top, 2 * F), torch.float32)
             moe.gemm_plain(y, self.gate_up, gu, routing, gather=True)
             moe.activate(gu, act, self.limit, self.alpha, self.shift)
             moe.gemm_plain(act, self.down, out, routing, gather=False)
-        if self.folded:
+        if folded:
             shared, out = out[T * top:], out[:T * top]
         moe.combine(out, routing, x, shared=shared, gate=None if shared is None else (logits, E),
                     identity=y if self.identity else None)

@@ -114,3 +114,67 @@ def test_tile_heights_by_the_rows_an_expert_has():
     assert moe.tall_rows(1602, 4, 40, 32, 2048, 768) == 192
     assert moe.tall_rows(1712, 4, 32, 32, 2048, 768) == 256
     assert moe.tall_rows(1712, 4, 32, 32, 2048, 768, True) == 128
+
+
+def test_a_shared_expert_is_folded_only_where_that_pays():
+    """Both sides of the lines: always beyond the steps of few rows an expert, in them while its rows are few tiles of matrices
+    that are small enough to be read again."""
+    assert all(moe.fold_pays(T, 4, 32, 2048, 768) for T in (1, 8, 128, 129, 512, 2048, 8192))
+    assert all(moe.fold_pays(T, 8, 256, 2048, 512) for T in (1, 64, 512, 513, 2048))
+    assert moe.fold_pays(512, 1, 128, 2048, 768) and not moe.fold_pays(1024, 1, 128, 2048, 768)
+    assert not moe.fold_pays(2048, 1, 128, 2048, 768) and moe.fold_pays(2049, 1, 128, 2048, 768)
+    assert moe.fold_pays(32, 4, 64, 4096, 1536) and not moe.fold_pays(33, 4, 64, 4096, 1536)
+    assert not moe.fold_pays(256, 4, 64, 4096, 1536) and moe.fold_pays(257, 4, 64, 4096, 1536)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 7, 70, 300])
+def test_a_shared_expert_folded_and_by_its_own_products(T, monkeypatch):
+    """The same layer either way. The shared expert's activations are rounded to bfloat16 from float32 sums in another order, so one may
+    fall to the neighbouring value (2^-7 of it); its product passes that on, the sums themselves are off by K roundings."""
+    from herbert_rs_amd.parts import PartSpec, Runtime, StepContext, build
+    E, top, W, F = 6, 2, 128, 64
+    part = build("feed_forward", PartSpec("routed_experts", {
+        "hidden_size": W, "intermediate_size": F, "experts": E, "top": top, "activation": "silu", "routing": "scores",
+        "names": {"router": "r", "router_bias": "b", "gate": "g{e}", "up": "u{e}", "down": "d{e}"},
+        "shared_expert": {"intermediate_size": F, "names": {"gate": "sg", "up": "su", "down": "sd", "sg": "s"}}}))
+    g = torch.Generator().manual_seed(T)
+    tensors = {name: torch.randn(*need.shape, generator=g) * need.shape[-1] ** -0.5 for name, need in part.tensor_needs().items()}
+    rt = Runtime(torch.bfloat16, DEV)
+    part.load({name: t if name == "b" else t.bfloat16() for name, t in tensors.items()}, rt)
+    assert part.foldable
+    y, got = torch.randn(T, W, generator=g).bfloat16(), {}
+    for fold in (False, True):
+        monkeypatch.setattr(moe, "fold_pays", lambda *a: fold)
+        got[fold] = torch.zeros(T, W, device=DEV)
+        part.forward(StepContext(rt=rt, meta=None, cache=None), y.to(DEV), got[fold])
+    x = y.double()
+    gate, up, down, sg = (tensors[n].bfloat16().double() for n in ("sg", "su", "sd", "s"))
+    act = torch.nn.functional.silu(x @ gate.T) * (x @ up.T)
+    size = torch.sigmoid(x @ sg.T) * (act.abs() @ down.abs().T)
+    off = (got[True] - got[False]).cpu().double().abs()
+    assert bool((off <= 2.0 ** -7 * size + 2.0 ** -20 * (got[False].cpu().double().abs() + size)).all())
+    assert float(size.min()) > 0 and bool((got[True].cpu().double().abs().sum(1) > 0).all())
+
+
+@pytest.mark.gpu
+def test_rows_by_tall_tiles_and_by_low_ones():
+    """The same rows by tiles of 64 and by every tall height: k is added in another order, so the float32 sums differ by
+    at most K roundings of the terms' sizes either way; the heights agree bit for bit."""
+    T, E, top, W, F = 700, 3, 2, 256, 128
+    g = torch.Generator().manual_seed(3)
+    logits, y = torch.randn(T, E, generator=g).to(DEV), torch.randn(T, W, generator=g).bfloat16()
+    w = (torch.randn(E, F, W, generator=g) * W ** -0.5).bfloat16()
+    got = {}
+    for height in (0,) + moe.TALL_TILES:
+        r = moe.Routing(torch.empty(moe.Routing.ints_needed(T, E, top, height), dtype=torch.int32, device=DEV),
+                        torch.empty(T, top, device=DEV), T, E, top, tall=height)
+        moe.route(logits, None, r)
+        got[height] = torch.empty(T * top, F, device=DEV)
+        moe.grouped_mfma(y.to(DEV), W, 0, moe.pack_grouped(w).to(DEV), got[height], F, 0, moe.EPI_F32, r, gather=True, tall=height > 0)
+    order, chosen = r.order.cpu().long(), r.chosen.cpu().long()
+    rows, expert = y[order // top].double(), chosen[order]
+    size = torch.stack([rows[i].abs() @ w[expert[i]].double().abs().T for i in range(T * top)])
+    assert torch.equal(got[128], got[192]) and torch.equal(got[128], got[256])
+    off = (got[128].cpu().double() - got[0].cpu().double()).abs()
+    assert bool((off <= 2 * W * 2.0 ** -24 * size).all())
