@@ -413,7 +413,7 @@ latent_attention_prompt_kernel(const float* __restrict__ q_full, const bf16* __r
                                const float* __restrict__ gate, int gate_ld, const int* __restrict__ positions,
                                const int* __restrict__ seq_starts, const int* __restrict__ slots,
                                const int* __restrict__ page_table, int max_pages, int page_size, int H, int rank,
-                               int rot, float scale, const float* __restrict__ sinks) {
+                               int rot, float scale, const float* __restrict__ sinks, const int* __restrict__ which) {
     // operands of 64 lanes x 16 bytes, lane (n, g) at 16 g + (n + a rotation by the operand's number) % 16: reads meet no
     // bank twice, and the writes of threads that hold a key's neighbouring numbers spread over the banks
     __shared__ __attribute__((aligned(16))) uint4 keys[2][2][KSW][HB_WAVE];         // [block of 16 keys][half][32 numbers]
@@ -424,7 +424,7 @@ latent_attention_prompt_kernel(const float* __restrict__ q_full, const bf16* __r
     const int n = lane & 15, g = lane >> 4, half = wave & 1;
     const int kd = rank + rot, KS = kd / 32, vsteps = rank / 8;
     const int ks_a = (KS + 1) / 2, db_a = (rank / 16 + 1) / 2;              // the first half's steps and blocks
-    const int seq = blockIdx.y, tile = gridDim.x - 1 - blockIdx.x;          // (the tiles with the most keys first)
+    const int seq = which ? which[blockIdx.y] : blockIdx.y, tile = gridDim.x - 1 - blockIdx.x;      // (the tiles with the most keys first)
     const int begin = seq_starts[seq], rows = (seq_starts[seq + 1] - begin) * H;
     if (tile * LP_ROWS >= rows) return;
     const int in_seq = tile * LP_ROWS + 16 * (wave >> 1) + n;
@@ -644,12 +644,14 @@ typedef float la_f32x16 __attribute__((ext_vector_type(16)));
 #define LH_TILE 64
 #define LH_RANK 512
 
-// The sequence of the step whose tiles hold tile `tile`, and how many tiles lie before that sequence's.
-__device__ __forceinline__ int lh_sequence_of(int tile, const int* context_lens, int n_seqs, int& before) {
+// The n_seqs sequences that take this form are those that `which` names (null: all of the step, in their order). The one of them
+// whose tiles hold tile `tile`, and how many tiles lie before its own.
+__device__ __forceinline__ int lh_sequence_of(int tile, const int* context_lens, const int* which, int n_seqs, int& before) {
     const int lane = threadIdx.x & (HB_WAVE - 1);
     before = 0;
     for (int first = 0; first < n_seqs; first += HB_WAVE) {
-        int upto = first + lane < n_seqs ? (context_lens[first + lane] + LH_TILE - 1) / LH_TILE : 0;
+        int upto = 0;
+        if (first + lane < n_seqs) upto = (context_lens[which ? which[first + lane] : first + lane] + LH_TILE - 1) / LH_TILE;
 #pragma unroll
         for (int off = 1; off < HB_WAVE; off <<= 1) {
             const int v = __shfl_up(upto, off, HB_WAVE);
@@ -659,7 +661,7 @@ __device__ __forceinline__ int lh_sequence_of(int tile, const int* context_lens,
         if (beyond) {
             const int at = __ffsll(beyond) - 1;
             if (at) before += __shfl(upto, at - 1, HB_WAVE);
-            return first + at;
+            return which ? which[first + at] : first + at;
         }
         before += __shfl(upto, HB_WAVE - 1, HB_WAVE);
     }
@@ -675,12 +677,12 @@ latent_heads_kernel(const bf16* __restrict__ pages, const bf16* __restrict__ w_u
                     bf16* __restrict__ keys, bf16* __restrict__ turned, bf16* __restrict__ values,
                     const int* __restrict__ context_lens, int n_seqs, const int* __restrict__ slots,
                     const int* __restrict__ page_table, int max_pages, int page_size, int tiles, int dim, int rank,
-                    int rot) {
+                    int rot, const int* __restrict__ which) {
     __shared__ __attribute__((aligned(16))) char lh_lds[LH_TILE * (LH_RANK * 2 + 16)];
     const int tile = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int before;
-    const int seq = lh_sequence_of(tile, context_lens, n_seqs, before);
+    const int seq = lh_sequence_of(tile, context_lens, which, n_seqs, before);
     if (seq < 0) return;
     const int key0 = (tile - before) * LH_TILE, held = context_lens[seq];
     const int kd = rank + rot, octets = rank / 8, pitch = rank * 2 + 16;
@@ -790,12 +792,12 @@ latent_heads_kernel(const bf16* __restrict__ pages, const bf16* __restrict__ w_u
 // follow, so that a CU that takes two of them gets one of either kind.
 template <int DS, int RS, int VB>
 __global__ void __launch_bounds__(256, 2)
-latent_attention_heads_kernel(const float* __restrict__ q, size_t q_ld, const float* __restrict__ q_turned,
+latent_attention_heads_kernel(const float* __restrict__ q, size_t q_ld, const float* __restrict__ q_turned, int turned_ld,
                               const bf16* __restrict__ keys, const bf16* __restrict__ turned,
                               const bf16* __restrict__ values, bf16* __restrict__ out, const float* __restrict__ gate,
                               int gate_ld, const int* __restrict__ positions, const int* __restrict__ seq_starts,
-                              const int* __restrict__ context_lens, int n_seqs, int tiles, int H, float scale,
-                              const float* __restrict__ sinks) {
+                              const int* __restrict__ context_lens, int tiles, int H, float scale,
+                              const float* __restrict__ sinks, const int* __restrict__ which) {
     constexpr int KS = DS + RS, DIM = 16 * DS, ROT = 16 * RS, VD = 32 * VB;
     constexpr int AHEAD = 3;                                               // reads of LDS ahead of their products
     constexpr int K_LOADS = 2 * KS / 4, V_LOADS = VB;                      // a wave's share of a tile, in kilobytes
@@ -807,12 +809,12 @@ latent_attention_heads_kernel(const float* __restrict__ q, size_t q_ld, const fl
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 31, g = lane >> 5, group = wave & 1, block = wave >> 1;
-    const int seq = blockIdx.y, h = blockIdx.x % H, nth = blockIdx.x / H, most = gridDim.x / H;
+    const int listed = blockIdx.y, seq = which ? which[listed] : listed, h = blockIdx.x % H, nth = blockIdx.x / H, most = gridDim.x / H;
     const int tile = nth < (most + 1) / 2 ? most - 1 - nth : nth - (most + 1) / 2;
     const int begin = seq_starts[seq], rows = seq_starts[seq + 1] - begin;
     if (tile * 64 >= rows) return;
     int before = 0;
-    for (int s = lane; s < seq; s += HB_WAVE) before += (context_lens[s] + LH_TILE - 1) / LH_TILE;
+    for (int s = lane; s < listed; s += HB_WAVE) before += (context_lens[which ? which[s] : s] + LH_TILE - 1) / LH_TILE;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) before += __shfl_xor(before, off, HB_WAVE);
     before = __builtin_amdgcn_readfirstlane(before);
@@ -848,7 +850,7 @@ latent_attention_heads_kernel(const float* __restrict__ q, size_t q_ld, const fl
     la_bf16x8 qh[KS], ql[KS];
     {
         const float* row = q + (size_t)t * q_ld + (size_t)h * (DIM + ROT) + 8 * g;
-        const float* trow = q_turned + ((size_t)t * H + h) * ROT + 8 * g;
+        const float* trow = q_turned + ((size_t)t * H + h) * turned_ld + 8 * g;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
@@ -1000,16 +1002,20 @@ latent_attention_heads_kernel(const float* __restrict__ q, size_t q_ld, const fl
         }
 }
 
-// tiles: the step's sequences' tiles of 64 keys together; scratch: keys [H][2 tiles][dim / 16][64][8], turned [2 tiles][rot / 16][64][8],
-// values [H][2 tiles][vdim / 32][2][64][8]. w_uk / w_uv: [H] matrices of dim / vdim rows of rank, packed.
-extern "C" int hb_latent_attention_heads(const float* q, int q_ld, const float* q_turned, const void* pages, const void* w_uk,
+// tiles: the tiles of 64 keys of the sequences together that `which` names (n_seqs of the step's; null: its first n_seqs), longest: the most
+// tokens that one of them brings; scratch: keys [H][2 tiles][dim / 16][64][8], turned [2 tiles][rot / 16][64][8], values [H][2 tiles][vdim / 32]
+// [2][64][8]. q_turned: the queries' rotated parts, turned_ld floats from a head's to the next. w_uk / w_uv: [H] matrices of dim / vdim rows of
+// rank, packed. Other sequences' rows of out are left as they are.
+extern "C" int hb_latent_attention_heads(const float* q, int q_ld, const float* q_turned, int turned_ld, const void* pages, const void* w_uk,
                                          const void* w_uv, void* keys, void* turned, void* values, void* out,
                                          const float* gate, int gate_ld, const int* positions, const int* seq_starts,
                                          const int* context_lens, int n_seqs, const int* slots, const int* page_table,
                                          int max_pages, int page_size, int tiles, int longest, int T, int H, int dim,
-                                         int vdim, int rank, int rot, float scale, const float* sinks, hipStream_t stream) {
+                                         int vdim, int rank, int rot, float scale, const float* sinks, const int* which,
+                                         hipStream_t stream) {
     HB_REQUIRE(T > 0 && H > 0 && H <= 65535 && n_seqs > 0 && n_seqs <= 65535 && longest > 0 && longest <= T,
                "latent attention: %d sequences of up to %d of %d tokens, %d heads", n_seqs, longest, T, H);
+    HB_REQUIRE(turned_ld >= rot, "latent attention: rotated parts of %d in rows of %d", rot, turned_ld);
     HB_REQUIRE(rank > 0 && rank % 32 == 0 && rank <= LH_RANK, "latent attention: built heads take a latent in steps of 32 up to 512, not %d", rank);
     HB_REQUIRE((dim == 64 || dim == 128) && vdim == dim && (rot == 0 || rot == 32 || rot == 64),
                "latent attention: heads of %d + %d and %d are not built", dim, rot, vdim);
@@ -1019,13 +1025,13 @@ extern "C" int hb_latent_attention_heads(const float* q, int q_ld, const float* 
     HB_REQUIRE(blocks < (1ll << 23) && tiles < (1 << 23), "latent attention: too many tokens for the grid");
     latent_heads_kernel<<<dim3(tiles, H), 256, 0, stream>>>((const bf16*)pages, (const bf16*)w_uk, (const bf16*)w_uv, (bf16*)keys, (bf16*)turned,
                                                             (bf16*)values, context_lens, n_seqs, slots, page_table, max_pages, page_size,
-                                                            tiles, dim, rank, rot);
+                                                            tiles, dim, rank, rot, which);
     HB_CHECK_LAUNCH("latent_heads");
     const dim3 grid((unsigned)blocks, n_seqs);
 #define LH_LAUNCH(DSV, RSV, VBV)                                                                                    \
     latent_attention_heads_kernel<DSV, RSV, VBV><<<grid, 256, 0, stream>>>(                                         \
-        q, (size_t)q_ld, q_turned, (const bf16*)keys, (const bf16*)turned, (const bf16*)values, (bf16*)out, gate, gate_ld, \
-        positions, seq_starts, context_lens, n_seqs, tiles, H, scale, sinks)
+        q, (size_t)q_ld, q_turned, turned_ld, (const bf16*)keys, (const bf16*)turned, (const bf16*)values, (bf16*)out, gate, gate_ld, \
+        positions, seq_starts, context_lens, tiles, H, scale, sinks, which)
     if (dim == 128) {
         if (rot == 64) LH_LAUNCH(8, 4, 4);
         else if (rot == 32) LH_LAUNCH(8, 2, 4);
@@ -1087,7 +1093,7 @@ extern "C" int hb_latent_attention_mfma(const float* q_full, const void* pages, 
                                         const int* seq_of, const int* slots, const int* page_table, int max_pages,
                                         int page_size, int T, int H, int rank, int rot, float scale, int splits,
                                         int chunks_per_split, const float* sinks, const int* seq_starts, int n_seqs,
-                                        int longest, hipStream_t stream) {
+                                        int longest, const int* which, hipStream_t stream) {
     HB_REQUIRE(T > 0 && H > 0, "latent attention: empty input");
     HB_REQUIRE(rank > 0 && rank % 32 == 0 && rank <= 512 && rot % 32 == 0 && rank + rot <= 640,
                "latent attention: the matrix-core kernel takes a latent and a rotated part in steps of 32, up to 512 + 128, not %d + %d", rank, rot);
@@ -1096,13 +1102,14 @@ extern "C" int hb_latent_attention_mfma(const float* q_full, const void* pages, 
     HB_REQUIRE(splits == 1 || (part_acc && part_ml), "latent attention: ranges need scratch");
     const long long blocks = (long long)T * ((H + 15) / 16);
     HB_REQUIRE(blocks < (1ll << 31) && (long long)T * H < (1ll << 31) - LP_ROWS, "latent attention: too many tokens for the grid");
-    if (seq_starts) {      // the prompts' kernel; longest: the most tokens that a sequence of the step brings
+    // the prompts' kernel, for the n_seqs sequences that `which` names (null: all of the step); longest: the most tokens that one brings
+    if (seq_starts) {
         HB_REQUIRE(n_seqs > 0 && n_seqs <= 65535 && longest > 0 && longest <= T, "latent attention: %d sequences of up to %d tokens", n_seqs, longest);
 #define LP_LAUNCH(RBV, KSV)                                                                                           \
     latent_attention_prompt_kernel<RBV, KSV>                                                                          \
         <<<dim3((unsigned)(((long long)longest * H + LP_ROWS - 1) / LP_ROWS), n_seqs), 512, 0, stream>>>(             \
             q_full, (const bf16*)pages, (bf16*)out, gate, gate_ld, positions, seq_starts, slots, page_table, max_pages, \
-            page_size, H, rank, rot, scale, sinks)
+            page_size, H, rank, rot, scale, sinks, which)
         if (rank <= 128 && rank + rot <= 256) LP_LAUNCH(4, 4);
         else if (rank <= 256 && rank + rot <= 384) LP_LAUNCH(8, 6);
         else if (rank + rot <= 512) LP_LAUNCH(16, 8);

@@ -1,9 +1,12 @@
 """Host side of the attention over latent rows (csrc/attention_latent.hip): what a token writes
 (its cache row [latent | rotated part] and its rotated query parts) and the attention itself."""
+import functools
+
 import numpy as np
 import torch
 
 from ..errors import BackendError
+from ..hosted import send
 from . import lib
 from .ops import _check, _ptr, _stream, dtype_code
 
@@ -111,47 +114,130 @@ def mfma_takes(cache, rank, rot):
             and cache.page_size % CHUNK == 0)
 
 
-# What the built keys and values of a step's sequences may take beyond what the other form of the same step takes.
+# What the built keys and values that one call leaves in scratch may take beyond what the other form takes for the same
+# sequences. (They lie in buffers of their own names, which a process that uses both forms keeps beside the other's; a buffer that has
+# become too small is replaced by one at least twice as large, and kept.)
 HEADS_BYTES = 256 << 20
 HEADS_TILE = 64
+HEADS_MOST = 4          # times the other form's work on the chip
+RUNS = 3                # of neighbouring sequences that score on the latents beside others: that many calls of their own
 
 
-def _tiles(meta):
-    return sum(-(-int(n) // HEADS_TILE) for n in meta.host_context)
+def _heads_take(kv, dim, vdim, rank, rot):
+    return (mfma_takes(kv, rank, rot) and dim in (64, 128) and vdim == dim and rot in (0, 32, 64)
+            and kv.page_size % HEADS_TILE == 0)
+
+
+@functools.lru_cache(maxsize=4096)
+def _sequence_form(new, context, H, dim, rank, rot, most_bytes):
+    """For a sequence that brings `new` tokens and holds `context` with them: whether its attention builds every head's keys and values
+    (latent_attention_heads) instead of scoring on the latents, and the bytes that either form takes in scratch for it. The two round
+    differently (keys and values to bfloat16 here, mapped queries and summed latents there), so the choice is by what the sequence brings
+    and holds alone, and a row's result does not depend on what else the step holds.
+    It is built where the estimate of its time alone is the smaller and the work that it puts on the chip no more than HEADS_MOST times
+    the other's, so that a step of many sequences with a few tokens each behind long contexts does not pay for every one's contexts.
+    The estimates: products of the heads' matrices with latents (keys here, tokens there) at 400 TFLOP/s, the attentions' own at 600 and
+    500, and alone no less than the context's chain of tiles, 1.7 us for 64 keys here and 3.2 us for 32 there. Microseconds of a layer's
+    kernels on the latents / built, 16 heads of 128 + 64 and 128 on 512: prompts of 2 tokens 31 / 22, of 64 53 / 23, 8 of 8 45 / 24, 32 of
+    64 137 / 38; 16 tokens behind 1,000 124 / 48 (4.7 times the work: on the latents), 30 behind 1,000 134 / 47, 20 behind 8,192 818 / 239,
+    50 behind 4,096: one 433 / 131, 4 435 / 200, 10 438 / 442, 32 867 / 1,292; 8 heads of 128 + 64 on 256: 2 tokens 20 / 19, 32 of 64 66 / 27,
+    50 behind 4,096: one 275 / 118, 32 317 / 590."""
+    pairs = new * (context - new) + new * (new + 1) // 2
+    matrices = 4 * H * rank * dim / 400e6                   # (microseconds a row)
+    here, there = 4 * pairs * H * (2 * dim + rot) / 600e6, 4 * pairs * H * (2 * rank + rot) / 500e6
+    build, take = context * matrices, new * matrices
+    bytes_here = 2 * _tiles(context) * HEADS_TILE * (2 * H * dim + rot) + 4 * new * H * rot
+    bytes_there = new * H * (4 * (rank + rot) + 2 * (rank + dim))
+    built = (new > 1 and build + here <= HEADS_MOST * (take + there)
+             and build + max(here, context / 64 * 1.7) < take + max(there, context / 32 * 3.2)
+             and bytes_here <= max(bytes_there, most_bytes))
+    return built, bytes_here, bytes_there
+
+
+def _tiles(context):
+    return -(-context // HEADS_TILE)
+
+
+class Forms:
+    """How a step's sequences go through a layer's latent attention. calls: for each call of latent_attention_heads (which, sequences,
+    tiles, longest); rest: of those that score on the latents (which, sequences, first row, rows, longest, longest context, apart) for every
+    run of neighbours, or of all of them where there are more than RUNS runs (apart: others' rows lie between theirs). `which` is the list of
+    the sequences on the GPU, None where it is all of the step's."""
+
+    def __init__(self, calls=(), rest=()):
+        self.calls, self.rest = calls, rest
+
+
+def forms(meta, kv, H, dim, vdim, rank, rot):
+    """The step's Forms, worked out once for all layers of these sizes."""
+    if meta.max_new == 1 or not _heads_take(kv, dim, vdim, rank, rot):
+        return LATENTS
+    key = ("latent_forms", H, dim, rank, rot)
+    got = meta.derived.get(key)
+    if got is None:
+        got = meta.derived[key] = _forms(meta, H, dim, rank, rot)
+    return got
+
+
+def _forms(meta, H, dim, rank, rot):
+    starts, context = meta.host_starts.tolist(), meta.host_context.tolist()
+    new = [b - a for a, b in zip(starts, starts[1:])]
+    groups, runs, rest, held, other = [], [], [], 0, 0
+    for i, (n, c) in enumerate(zip(new, context)):
+        built, here, there = _sequence_form(n, c, H, dim, rank, rot, HEADS_BYTES)
+        if built:
+            if not groups or held + here > max(HEADS_BYTES, other + there):
+                groups.append([])
+                held = other = 0
+            groups[-1].append(i)
+            held, other = held + here, other + there
+        elif n:
+            if not rest or any(new[rest[-1] + 1:i]):
+                runs.append([])
+            runs[-1].append(i)
+            rest.append(i)
+    if not groups:
+        return LATENTS
+    apart = len(runs) > RUNS
+    if apart:
+        runs = [rest]
+    whole = len(groups) == 1 and len(groups[0]) == len(new)
+    packed, places = [], []
+    for one in groups + runs:
+        places.append(len(packed))
+        packed += one
+    on_gpu = None if whole else send(np.array(packed, dtype=np.int32), meta.seq_starts.device)
+    at = lambda place: None if on_gpu is None else on_gpu[place:]
+    calls = tuple((at(place), len(one), sum(_tiles(context[i]) for i in one), max(new[i] for i in one)) for place, one in zip(places, groups))
+    left = tuple((at(place), len(one), starts[one[0]], starts[one[-1] + 1] - starts[one[0]], max(new[i] for i in one),
+                  max(context[i] for i in one), apart) for place, one in zip(places[len(groups):], runs))
+    return Forms(calls, left)
+
+
+LATENTS = Forms()       # all of the step scores on the latents
 
 
 def heads_pay(meta, kv, H, dim, vdim, rank, rot):
-    """True if a step's latent attention builds every head's keys and values (latent_attention_heads) instead of scoring on the
-    latents: for the sizes that its kernels take, where the estimate of its time is the smaller, in scratch that stays within its
-    bound. The estimates: products of the heads' matrices with latents (keys here, tokens there) at 400 TFLOP/s, the
-    attentions' own at 600 and 500, and no less than the longest context's chain of tiles, 1.7 us for 64 keys here and 3.2 us
-    for 32 there. Microseconds of a whole layer, latents / built, 16 heads of 128 + 64 and 128 on 512: 65 tokens 79 / 47, 300 tokens
-    108 / 56, 16 tokens behind 1,000 144 / 64, behind 8,000 805 / 267; 4 heads of 64 + 32 and 64 on 256: 51 / 32, 65 / 35, 93 / 41
-    and 528 / 158."""
-    if (meta.max_new == 1 or meta.max_context <= PROMPT_FROM or not mfma_takes(kv, rank, rot) or dim not in (64, 128)
-            or vdim != dim or rot not in (0, 32, 64) or kv.page_size % HEADS_TILE):
-        return False
-    new = np.diff(meta.host_starts).astype(np.int64)
-    context = meta.host_context.astype(np.int64)
-    pairs, T, tiles = int((new * (context - new) + new * (new + 1) // 2).sum()), int(new.sum()), _tiles(meta)
-    matrices = 2 * H * rank * (dim + vdim) / 400e6          # (microseconds a row)
-    built = tiles * HEADS_TILE * matrices + max(4 * pairs * H * (dim + rot + vdim) / 600e6, meta.max_context / 64 * 1.7)
-    latent = T * matrices + max(4 * pairs * H * (2 * rank + rot) / 500e6, meta.max_context / 32 * 3.2)
-    scratch = 2 * tiles * HEADS_TILE * (H * (dim + vdim) + rot) + 4 * T * H * rot
-    other = T * H * (4 * (rank + rot) + 2 * (rank + dim))
-    return built < latent and scratch <= max(other, HEADS_BYTES)
+    """True if a sequence of the step builds its heads' keys and values (see _sequence_form)."""
+    return (meta.max_new > 1 and _heads_take(kv, dim, vdim, rank, rot)
+            and any(_sequence_form(int(n), int(c), H, dim, rank, rot, HEADS_BYTES)[0]
+                    for n, c in zip(np.diff(meta.host_starts), meta.host_context)))
 
 
 def latent_attention_heads(q, q_off, turned, meta, kv, w_uk, w_uv, out, gate, gate_off, dim, vdim, rank, rot, scale, buffer,
-                           sinks=None):
+                           sinks=None, call=None, turned_at=None):
     """out[t, h, :] = softmax over the slot's rows j <= position of (query . [W_uk,h c_j | r_j] * scale) times W_uv,h c_j, times
     sigmoid(gate[t, gate_off + h]) if a gate is given; bfloat16 [T, H vdim]. q f32 [T, ld]: columns [q_off, + H (dim + rot)) are the
-    queries, whose rotated parts are read from turned f32 [T, H rot] instead. w_uk [H, dim, rank], w_uv [H, vdim, rank] as
-    moe.pack_grouped gives them. Only where heads_pay says so; scratch from `buffer(name, shape, dtype)`."""
+    queries, whose rotated parts are read from turned f32 [T, H rot] instead, or with turned_at = (floats a head, the first one) from
+    there in turned f32 [T, H x floats]. w_uk [H, dim, rank], w_uv [H, vdim, rank] as moe.pack_grouped gives them. call: one of Forms'
+    calls (None: all sequences); other sequences' rows of out stay as they are. Scratch from `buffer(name, shape, dtype)`."""
     H = w_uk.shape[0]
     T, ld = q.shape
     _check(q, "q", torch.float32, (T, ld))
-    _check(turned, "turned", torch.float32, (T, H * rot))
+    turned_row, turned_first = (rot, 0) if turned_at is None else turned_at
+    if turned_first < 0 or turned_first + rot > turned_row:
+        raise BackendError("latent attention: the rotated parts lie outside their rows")
+    _check(turned, "turned", torch.float32, (T, H * turned_row))
     _check(w_uk, "w_uk", torch.bfloat16, (H, dim, rank))
     _check(w_uv, "w_uv", torch.bfloat16, (H, vdim, rank))
     _check(out, "out", torch.bfloat16, (T, H * vdim))
@@ -170,20 +256,25 @@ def latent_attention_heads(q, q_off, turned, meta, kv, w_uk, w_uv, out, gate, ga
         if gate_off < 0 or gate_off + H > gate_ld:
             raise BackendError("latent attention: the gate's columns lie outside its rows")
         gate_ptr = gate.data_ptr() + 4 * gate_off
-    tiles = _tiles(meta)
+    if call is None:
+        call = None, meta.num_seqs, sum(_tiles(int(n)) for n in meta.host_context), int(meta.max_new)
+    which, n_seqs, tiles, longest = call
+    if which is not None and (which.dtype != torch.int32 or which.numel() < n_seqs):
+        raise BackendError("latent attention: the list of sequences is too short")
     keys = buffer("latent_heads_keys", (H, tiles * HEADS_TILE, dim), torch.bfloat16)
     shared = buffer("latent_heads_turned", (tiles * HEADS_TILE, max(rot, 1)), torch.bfloat16)
     values = buffer("latent_heads_values", (H, tiles * HEADS_TILE, vdim), torch.bfloat16)
-    lib.call("attention_latent", "hb_latent_attention_heads", q.data_ptr() + 4 * q_off, ld, turned.data_ptr(), kv.k.data_ptr(),
-             w_uk.data_ptr(), w_uv.data_ptr(), keys.data_ptr(), shared.data_ptr(), values.data_ptr(), out.data_ptr(), gate_ptr,
-             gate_ld, meta.positions.data_ptr(), meta.seq_starts.data_ptr(), meta.context_lens.data_ptr(), meta.num_seqs,
-             meta.slots.data_ptr(), kv.page_table.data_ptr(), kv.page_table.shape[1], kv.page_size, tiles, int(meta.max_new), T,
-             H, dim, vdim, rank, rot, float(scale), _ptr(sinks), _stream())
+    lib.call("attention_latent", "hb_latent_attention_heads", q.data_ptr() + 4 * q_off, ld, turned.data_ptr() + 4 * turned_first,
+             turned_row, kv.k.data_ptr(), w_uk.data_ptr(), w_uv.data_ptr(), keys.data_ptr(), shared.data_ptr(), values.data_ptr(), out.data_ptr(), gate_ptr,
+             gate_ld, meta.positions.data_ptr(), meta.seq_starts.data_ptr(), meta.context_lens.data_ptr(), n_seqs,
+             meta.slots.data_ptr(), kv.page_table.data_ptr(), kv.page_table.shape[1], kv.page_size, tiles, longest, T,
+             H, dim, vdim, rank, rot, float(scale), _ptr(sinks), _ptr(which), _stream())
 
 
-def latent_attention_mfma(q_full, meta, cache, out, gate, gate_off, H, rank, rot, scale, buffer, sinks=None):
+def latent_attention_mfma(q_full, meta, cache, out, gate, gate_off, H, rank, rot, scale, buffer, sinks=None, part=None):
     """latent_attention_plain on the matrix cores (see mfma_takes). A prompt's tokens share their keys in LDS; a step of one
-    token a sequence cuts its keys into ranges, whose partial results lie in scratch from `buffer(name, shape, dtype)`."""
+    token a sequence cuts its keys into ranges, whose partial results lie in scratch from `buffer(name, shape, dtype)`.
+    part: one of Forms' `rest`, for those sequences alone (of the rows between its first and last any may be written)."""
     if sinks is not None:
         _check(sinks, "sinks", torch.float32, (H,))
     T = q_full.shape[0]
@@ -199,22 +290,28 @@ def latent_attention_mfma(q_full, meta, cache, out, gate, gate_off, H, rank, rot
         if gate_off < 0 or gate_off + H > gate_ld:
             raise BackendError("latent attention: the gate's columns lie outside its rows")
         gate_ptr = gate.data_ptr() + 4 * gate_off
+    which, n_seqs, first, rows, longest, context, apart = part or (None, meta.num_seqs, 0, T, int(meta.max_new), meta.max_context, False)
+    prompt = apart or (longest > 1 and context > PROMPT_FROM)
     splits, per = 1, 1 << 30
-    if meta.max_new == 1:
+    if longest == 1 and not prompt:
         # the grid must not depend on the contexts themselves (a recorded step is replayed at others of its bucket)
-        chunks = -(-max(meta.context_bucket, meta.max_context) // CHUNK)
-        blocks = T * ((H + 15) // 16)
+        chunks = -(-max(meta.context_bucket if part is None else 0, context) // CHUNK)
+        blocks = rows * ((H + 15) // 16)
         splits = max(1, min(TARGET_WAVES // blocks, chunks, 64))
         per = -(-chunks // splits)
     part_acc = part_ml = None
     if splits > 1:
-        part_acc = buffer("latent_partial", (T * H * splits, rank), torch.float32)
-        part_ml = buffer("latent_partial_ml", (T * H * splits, 2), torch.float32)
-    prompt = meta.max_new > 1 and meta.max_context > PROMPT_FROM
+        part_acc = buffer("latent_partial", (rows * H * splits, rank), torch.float32)
+        part_ml = buffer("latent_partial_ml", (rows * H * splits, 2), torch.float32)
     if prompt:
+        # (rows as the sequences' starts count them)
         _check(meta.seq_starts, "seq_starts", torch.int32, (meta.num_seqs + 1,))
-    lib.call("attention_latent", "hb_latent_attention_mfma", q_full.data_ptr(), cache.k.data_ptr(), out.data_ptr(),
-             _ptr(part_acc), _ptr(part_ml), gate_ptr, gate_ld, meta.positions.data_ptr(), meta.seq_of.data_ptr(),
-             meta.slots.data_ptr(), cache.page_table.data_ptr(), cache.page_table.shape[1], cache.page_size, T, H,
-             rank, rot, float(scale), splits, per, _ptr(sinks),
-             meta.seq_starts.data_ptr() if prompt else None, meta.num_seqs if prompt else 0, int(meta.max_new), _stream())
+        first, rows = 0, T
+    if which is not None and (which.dtype != torch.int32 or which.numel() < n_seqs):
+        raise BackendError("latent attention: the list of sequences is too short")
+    lib.call("attention_latent", "hb_latent_attention_mfma", q_full.data_ptr() + 4 * first * H * (rank + rot), cache.k.data_ptr(),
+             out.data_ptr() + 2 * first * H * rank, _ptr(part_acc), _ptr(part_ml),
+             None if gate_ptr is None else gate_ptr + 4 * first * gate_ld, gate_ld, meta.positions.data_ptr() + 4 * first,
+             meta.seq_of.data_ptr() + 4 * first, meta.slots.data_ptr(), cache.page_table.data_ptr(), cache.page_table.shape[1],
+             cache.page_size, rows, H, rank, rot, float(scale), splits, per, _ptr(sinks),
+             meta.seq_starts.data_ptr() if prompt else None, n_seqs if prompt else 0, longest, _ptr(which) if prompt else None, _stream())

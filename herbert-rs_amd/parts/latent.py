@@ -10,7 +10,7 @@ What a token leaves in the cache is c and the rotated part, one row of kv_rank +
 no values beside them. Steps of few tokens never build a head's keys or values: the query's unrotated part is taken through
 W_uk,n^T first (kv_rank numbers), scores and weighted sums then run on the cached rows themselves,
 one shared "key head" for all query heads, and the summed latents go through W_uv,n afterwards. Prompts in bfloat16 build
-them for the step, from the cached rows (kernels.latent.heads_pay says when).
+them for the step, from the cached rows, a sequence by what it brings and holds itself (kernels.latent.forms).
 Scores, softmax and the weighted sums are float32 in either mode.
 
 Two parameters change the form. `gate="elementwise"`: W_g has a row for every entry of the joined heads, and
@@ -139,9 +139,12 @@ class LatentAttention(Part):
         proj = rt.buffer("latent_proj", (T, self.width), torch.float32)
         self.proj.forward(y, proj)
         cores = self.cores
-        built = self.uk is not None and latent.heads_pay(ctx.meta, kv, H, self.dim, self.vdim, self.rank, self.rot_dim)
+        forms = latent.LATENTS
+        if self.uk is not None:
+            forms = latent.forms(ctx.meta, kv, H, self.dim, self.vdim, self.rank, self.rot_dim)
+        alone = bool(forms.calls) and not forms.rest        # every sequence's heads are built
         q_full = turned = q_plain = None
-        if built:
+        if alone:
             turned = rt.buffer("latent_turned", (T, H * self.rot_dim), torch.float32)
         else:
             q_full = rt.buffer("latent_q_full", (T, H * self.row), torch.float32)
@@ -164,29 +167,33 @@ class LatentAttention(Part):
             write(write_cache=ctx.owns_cache, q_plain=q_plain)
         gate = proj if self.gated and self.gate_kind == "head" else None
         attn = rt.buffer("latent_attn", (T, H * self.vdim))
-        if built:
-            latent.latent_attention_heads(q_rows, 0, turned, ctx.meta, kv, self.uk, self.uv, attn, gate, self.q_width + self.row,
-                                          self.dim, self.vdim, self.rank, self.rot_dim, self.scale, rt.buffer, sinks=self.sink_w)
-        else:
+        for part in () if alone else forms.rest or (None,):
             # q'[t, n, :] = W_uk,n^T q[t, n, :dim]: a product a head, all heads in one launch
+            first, rows = part[2:4] if part else (0, T)
+            of = slice(first, first + rows)
             if cores:
-                moe.grouped_mfma(q_plain, H * self.dim, self.dim, self.uk_t, q_full, H * self.row, self.row, moe.EPI_F32, M=T)
+                moe.grouped_mfma(q_plain[of], H * self.dim, self.dim, self.uk_t, q_full[of], H * self.row, self.row, moe.EPI_F32, M=rows)
             else:
                 ops.gemm_plain_batched(q_rows, self.uk_t, q_full, T, self.rank, self.dim, q_ld, self.dim,
                                        H * self.row, H, self.dim + self.rot_dim, self.rank * self.dim, self.row)
             mixed = rt.buffer("latent_mixed", (T, H * self.rank))
             if latent.mfma_takes(kv, self.rank, self.rot_dim):
                 latent.latent_attention_mfma(q_full, ctx.meta, kv, mixed, gate, self.q_width + self.row, H, self.rank,
-                                             self.rot_dim, self.scale, rt.buffer, sinks=self.sink_w)
+                                             self.rot_dim, self.scale, rt.buffer, sinks=self.sink_w, part=part)
             else:
                 latent.latent_attention_plain(q_full, ctx.meta, kv, mixed, gate, self.q_width + self.row, H, self.rank,
                                               self.rot_dim, self.scale, sinks=self.sink_w)
             # a head's summed latents through its W_uv
             if cores:
-                moe.grouped_mfma(mixed, H * self.rank, self.rank, self.uv, attn, H * self.vdim, self.vdim, moe.EPI_BF16, M=T)
+                moe.grouped_mfma(mixed[of], H * self.rank, self.rank, self.uv, attn[of], H * self.vdim, self.vdim, moe.EPI_BF16, M=rows)
             else:
                 ops.gemm_plain_batched(mixed, self.uv, attn, T, self.vdim, self.rank, H * self.rank, self.rank,
                                        H * self.vdim, H, self.rank, self.vdim * self.rank, self.vdim)
+        # (after the others: rows between those of the sequences that score on the latents hold what is not theirs)
+        for call in forms.calls:
+            latent.latent_attention_heads(q_rows, 0, turned if alone else q_full, ctx.meta, kv, self.uk, self.uv, attn, gate,
+                                          self.q_width + self.row, self.dim, self.vdim, self.rank, self.rot_dim, self.scale, rt.buffer,
+                                          sinks=self.sink_w, call=call, turned_at=None if alone else (self.row, self.rank))
         if self.gated and self.gate_kind == "elementwise":
             gated = rt.buffer("latent_gated", (T, H * self.vdim))
             ops.gate_heads(attn, proj, self.q_width + self.row, gated, H, self.vdim, self.vdim)
