@@ -574,12 +574,17 @@ extern "C" int hb_chunked_delta(const float* qkv, int C, const float* proj, int 
 // (Dao and Gu, 2024: state-space duality; the sums c and their differences in float64, so that a pair's decay is exact to its
 // own size, and no quotient of decays is formed.) Products on the matrix cores, in float32, those of pairs in float64 and rounded once.
 // ssm_pairs_kernel: C_t . B_i of a (chunk, group) once for all its heads, as the second kernel's lanes load them.
+// A factor beyond TOO_LARGE (inputs, B, C, the state) counts as not finite here: below it no product before its decay passes float32's
+// range (sums of 128 products of two are 1.3e38 at most), beyond it one may where the walk, whose state decays first, stays within.
 // ssm_chunks_kernel: the chain of chunks, a workgroup a (head, 32 columns of S, sequence): four waves, each 16 tokens of a chunk for the outputs and a
 // quarter of the state's rows. A chunk that holds something not finite is walked token by token instead (ssm_slowly), so that it
 // spoils what it spoils in the walk.
 // 64 heads of 128 x 64 on 8 groups, one sequence of 2,048 tokens 318 us (the walk 802), of 512 91 (209), four of 512 133 (313), 16 of 128 140
 // (310). Bound by a chunk's chain in a workgroup, 9.5 us: 160 products of 40 cycles a wave, and as long again for the decays and for
 // laying out the state and the columns. Errors against 64 bits are 0.2 to 1.02 of the walk's.
+#define TOO_LARGE 1e18f
+__device__ __forceinline__ bool too_large(float v) { return !(fabsf(v) <= TOO_LARGE); }
+
 template <int DB>
 __global__ void __launch_bounds__(256)
 ssm_pairs_kernel(const float* __restrict__ u, int ldu, int b_at, int c_at, const int2* __restrict__ chunks,
@@ -702,7 +707,7 @@ ssm_chunks_kernel(const float* __restrict__ u, int ldu, const float* __restrict_
         for (int i = 0; i < 2; ++i)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                bad |= not_finite(x_next[i][e]) || not_finite(x_next[i][e] * my_dt);
+                bad |= too_large(x_next[i][e]) || too_large(x_next[i][e] * my_dt);
                 x_lds[buf][(my_col + 4 * i + e) * XLD + in_quads(my_token)] = x_next[i][e];
             }
         if (bad) spoilt[buf] = 1;
@@ -740,22 +745,17 @@ ssm_chunks_kernel(const float* __restrict__ u, int ldu, const float* __restrict_
 #pragma unroll
         for (int b = 0; b < DB; ++b)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) bad |= not_finite(cq[b][e]);
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) bad |= not_finite(pr[b][e]);
+            for (int e = 0; e < 4; ++e) bad |= too_large(cq[b][e]);
 #pragma unroll
         for (int s = 0; s < 16; ++s)
 #pragma unroll
-            for (int i = 0; i < OWN; ++i) bad |= not_finite(k[i][s]);
-        // (an entry so large that a product before its decay may pass float32's range is the walk's too)
+            for (int i = 0; i < OWN; ++i) bad |= too_large(k[i][s]);
 #pragma unroll
         for (int i = 0; i < OWN; ++i)
 #pragma unroll
             for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) bad |= !(fabsf(S[i][cb][e]) <= 1e30f);
+                for (int e = 0; e < 4; ++e) bad |= too_large(S[i][cb][e]);
         if (__any(bad) && lane == 0) spoilt[buf] = 1;
         // the decays: of a token from the chunk's start, of a pair, and to the chunk's end
         const double own = c_lds[wave][16 * wave + r], end = c_lds[wave][CHUNK - 1];

@@ -99,3 +99,28 @@ def test_what_is_not_finite_reaches_what_it_reaches_in_the_walk(place, what):
         assert torch.equal(a.isfinite(), b.isfinite())
         fine = b.isfinite()
         assert float((a - b)[fine].abs().max()) <= 1e-4 * float(b[fine].abs().max())
+
+
+@pytest.mark.parametrize("place", ["x", "B", "C", "state"])
+@pytest.mark.parametrize("rate", [0.0, 1.0])
+@pytest.mark.parametrize("what", [1e16, 1e22, 1e30])
+def test_large_numbers_pass_no_range_that_they_do_not_pass_in_the_walk(place, what, rate):
+    """A state of 1e20 and an input whose product with it, with another input or with a later one passes float32's range before the
+    decays bring it back, or only after they have: finite where the walk is, and there near it."""
+    heads, groups, N, P, lengths = 4, 2, 64, 48, [200, 100]
+    u, proj, a_log, dt_bias, d_skip, state, meta = step(lengths, heads, groups, N, P, rate)
+    state[2, 1] *= 1e20
+    for t in (50, 64 + 21):
+        at = {"x": P + 5, "B": heads * P + 3, "C": heads * P + groups * N + 7, "state": None}[place]
+        if at is not None:
+            u[t, at] = what
+    if place == "state":
+        state[2, 1, 3, 9] = what
+        u[40, heads * P + groups * N:] *= 1e20               # (C of a token whose decays bring the state far down)
+    case = (u, proj, a_log, dt_bias, d_skip, state, meta)
+    got, after = run(*case, heads, groups, N, P)
+    walk, walk_after = run(*case, heads, groups, N, P, chunks=False)
+    for a, b in ((got, walk), (after, walk_after)):
+        assert torch.equal(a.isfinite(), b.isfinite())
+        fine = b.isfinite()
+        assert float((a - b)[fine].abs().max()) <= 1e-4 * float(b[fine].abs().max())
