@@ -323,9 +323,11 @@ static void launch_as(const TA* A, const TW* W, TC* C, int M, int N, int K, int 
     // (both sides of these lines stand at gemm_plain_stream_kernel)
     const long long strips = (N + 15ll) / 16 * batch;
     const bool streams = sizeof(TW) == 4 && K > 64 && (K < 1024 || strips >= 768 || (K < 2048 && strips >= 512));
-    if (vec && M <= WAVE_ROWS && K % 16 == 0 && streams)
-        gemm_plain_stream_kernel<TA, TW, TC, ACCUM><<<dim3((N + 15) / 16, 1, batch), HB_WAVE, 0, stream>>>(
-            A, W, C, M, N, K, lda, ldw, ldc, batch_a, batch_w, batch_c, ep);
+    if (vec && M <= WAVE_ROWS && K % 16 == 0 && streams) {
+        if constexpr (sizeof(TW) == 4)
+            gemm_plain_stream_kernel<TA, TW, TC, ACCUM><<<dim3((N + 15) / 16, 1, batch), HB_WAVE, 0, stream>>>(
+                A, W, C, M, N, K, lda, ldw, ldc, batch_a, batch_w, batch_c, ep);
+    }
     else if (vec && M <= WAVE_ROWS && K % 16 == 0)
         gemm_plain_wave_kernel<TA, TW, TC, ACCUM><<<dim3((N + 15) / 16, 1, batch), wave_threads, 0, stream>>>(
             A, W, C, M, N, K, lda, ldw, ldc, batch_a, batch_w, batch_c, ep);
