@@ -167,13 +167,16 @@ def mfma_takes(K, lda, a_group_off=0, N=16):
 def tall_rows(T, top, routed, experts, hidden, inter, shared=False):
     """The rows of a tall tile (0: none) for a step of T tokens, each on `top` of `routed` outputs of the router, the first `experts` of which have
     bfloat16 matrices in the cores' order. Tall tiles from TALL_ROWS rows an expert on, for sizes that they take; of those the one
-    that brings the fewest bytes into a CU: rounds of tiles over the CUs times weight and activation rows of a step. An expert's rows are
-    taken to be spread around their mean as a random choice spreads them, and a round to be full at nine tenths, since some experts of a
-    model are busier than that. Over 132 layers (16 to 256 experts, 400 to 4,096 tokens) the height that this gives is 2.3 % slower than
-    the best one where experts are chosen at random (2.1 with rounds full to the last tile, 7.8 full at eight tenths) and 10.3 % where
-    they are very unequally busy, deviations of 0.5 to 1.2 of the mean (11.2, 9.3): there one height for all experts costs a round that
-    is nearly empty more often than not. An estimate that averaged the rounds over both kinds of routing was better by a tenth of
-    a layer's time at some token counts and worse by as much at others. shared: every token takes one more expert."""
+    that brings the fewest bytes into a CU: rounds of tiles over the CUs times weight and activation rows of a step; and none where the low
+    tiles of 64, two to a CU, are expected to be done sooner (a round of theirs as long as one of 284 rows: 64 experts of 1,536 on 4,096,
+    four each and a shared one, 800 tokens: 307 us, 353 by tiles of 128; 64 of 1,408 on 2,048, six each and a shared one, 512 tokens 160 and
+    157 to 174). An expert's rows are taken to be spread around their mean as a random choice spreads them, and a round to be full at
+    nine tenths, since some experts of a model are busier than that. Over 132 layers (16 to 256 experts, 400 to 4,096 tokens) the height
+    that this gives is 2.0 % slower than the best one where experts are chosen at random (without the low tiles 2.3; 2.1 with rounds full
+    to the last tile, 7.8 full at eight tenths) and 9.7 % where they are very unequally busy, deviations of 0.5 to 1.2 of the mean (10.3;
+    11.2, 9.3): there one height for all experts costs a round that is nearly empty more often than not. An estimate that averaged the
+    rounds over both kinds of routing was better by a tenth of a layer's time at some token counts and worse by as much at others.
+    shared: every token takes one more expert."""
     rows = T * top / routed
     if rows < TALL_ROWS or hidden % 64 or inter % 64:
         return 0
@@ -185,8 +188,9 @@ def tall_rows(T, top, routed, experts, hidden, inter, shared=False):
             tiles += 0.5 * math.erfc((k * height - rows) / (2.0 * rows) ** 0.5)
             k += 1
         return (experts * tiles + (-(-T // height) if shared else 0)) * columns
-    fits = [h for h in TALL_TILES if workgroups(h) >= 128]
-    return min(fits, key=lambda h: math.ceil(workgroups(h) / 256 + 0.1) * (256 + h), default=0)
+    cost = {h: math.ceil(workgroups(h) / 256 + 0.1) * (256 + h) for h in TALL_TILES if workgroups(h) >= 128}
+    cost[0] = math.ceil(workgroups(TILE_M) / 512 + 0.1) * 540 if cost else 0
+    return min(cost, key=cost.get)
 
 
 def fold_pays(T, top, experts, hidden, inter):

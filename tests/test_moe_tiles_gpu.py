@@ -114,6 +114,9 @@ def test_tile_heights_by_the_rows_an_expert_has():
     assert moe.tall_rows(1602, 4, 40, 32, 2048, 768) == 192
     assert moe.tall_rows(1712, 4, 32, 32, 2048, 768) == 256
     assert moe.tall_rows(1712, 4, 32, 32, 2048, 768, True) == 128
+    # (the low ones where the tall ones would take a round more than they save)
+    assert moe.tall_rows(800, 4, 64, 64, 4096, 1536, True) == 0 and moe.tall_rows(1500, 4, 64, 64, 4096, 1536, True) == 128
+    assert moe.tall_rows(512, 6, 64, 64, 2048, 1408, True) == 0 and moe.tall_rows(1600, 8, 256, 256, 2048, 512) == 0
 
 
 def test_a_shared_expert_is_folded_only_where_that_pays():
