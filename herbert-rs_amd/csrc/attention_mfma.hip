@@ -909,8 +909,10 @@ constexpr int decode_lds_of(int waves) {      // (four waves of heads of 128: 62
 // and key head: they cut its own pages into equal ranges and the first of them adds up the others' results, in the order of the
 // ranges, out of LDS and stores the output (_range_waves of mfma.py says where, with both forms' times). Two kernels: one for
 // either number of waves cost the single waves 0.2 % of a step (8B shape, 511 tokens: one sequence 3,308 -> 3,314 us, eight 3,585 -> 3,592).
+// (FORM_HEADS is bounded as if it had four waves, which the compiler schedules better: 24 sequences of up to 98 tokens 13.5 us for 14.2 in
+// two slices and 15.4 for 16.1 in four.)
 template <int HD, int FUSED, bool EXT, int QS = 1, bool MERGES = false>
-__global__ void __launch_bounds__(MERGES ? 256 : 64)
+__global__ void __launch_bounds__(MERGES || FUSED == FORM_HEADS ? 256 : 64)
 attn_decode_kernel(const bf16* __restrict__ q, bf16* __restrict__ k_cache, bf16* __restrict__ v_cache,
                    float* __restrict__ partial_o, float* __restrict__ partial_ml,
                    const int* __restrict__ context_lens, const int* __restrict__ slots,
@@ -926,7 +928,7 @@ attn_decode_kernel(const bf16* __restrict__ q, bf16* __restrict__ k_cache, bf16*
     // into, and items from ranges[n_seqs] on are nothing. The partial results are then laid out
     // [head, item]: those of one sequence and head lie side by side.
     const int kvh = blockIdx.y, splits = gridDim.z;
-    const int lane = MERGES ? threadIdx.x & 63 : threadIdx.x, c32 = lane & 31, g2 = lane >> 5;
+    const int lane = threadIdx.x & 63, c32 = lane & 31, g2 = lane >> 5;
     const int wave = MERGES ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0, waves = MERGES ? blockDim.x >> 6 : 1;
     int b = blockIdx.x, split = MERGES ? wave : blockIdx.z;
     if (!MERGES && ranges) {
