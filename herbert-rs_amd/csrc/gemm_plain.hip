@@ -2,20 +2,18 @@
 //   C[m, n] (+)= sum_k A[m, k] * W[n, k]      (weights are [out, in], k contiguous)
 // It is the whole matrix path of the float32 mode and the fallback of the bfloat16
 // mode for shapes its own MFMA kernels refuse. Each output is summed in stretches of K_BLOCK
-// elements of k: a stretch from zero over k ascending with fused multiply-adds, then the
-// stretches' sums one after another. Stretches lie at fixed places, so an output's value does
+// elements of k: a stretch from zero over k ascending in blocks of 32 by the split products of mfma_split.h, then the
+// stretches' sums one after another. Stretches and blocks lie at fixed places and a block's products come in one order, so an output's value does
 // not depend on M, on the tile or kernel it falls in, or on what else is in the batch, and yet
-// a product of few rows can give every stretch a wave of its own. The matrix cores' float32
-// products (v_mfma_f32_16x16x4_f32) add their four k one after another with one rounding each,
-// bit for bit what fmaf gives in that order (checked on 16,384 sums of mixed magnitudes),
-// and every kernel here feeds them k in ascending order. (One chain over all of k, which this
-// replaced, was further from 64 bits: at K = 2048 8.1e-7 of the sums' root mean square, now 4.1e-7; at K = 12288 20e-7
-// and 4.2e-7.) (hb_gemm_plain_short_k is the entry for products with a short k: it sends up to 32 float32 rows times bfloat16 rows to gemm_few_rows_kernel, whose four partial
+// a product of few rows can give every stretch a wave of its own. (The float32 matrix instructions in the
+// same stretches, which this replaced, were further from 64 bits: at K = 2048 4.1e-7 of the sums' root mean square, now 1.3e-7; at
+// K = 8704 4.1e-7 and 1.5e-7.) (hb_gemm_plain_short_k is the entry for products with a short k: it sends up to 32 float32 rows times bfloat16 rows to gemm_few_rows_kernel, whose four partial
 // sums a column differ from that order by float32 rounding, and everything else here.)
 // In xigh/herbert-rs: crates/backends/backend_bf16/src/kernels.rs:154-164 (float32 sums over k ascending of
 // x[m, k] * float(w[n, k]), no bias); crates/backends/backend_vulkan/shaders/bf16_matmul.comp:31-60.
 #include "common.h"
-#include "mfma_f32.h"
+#include "mfma_split.h"
+#include <type_traits>
 
 HB_MODULE_ERROR_SLOT()
 
@@ -66,16 +64,32 @@ __device__ __forceinline__ void store_quad(TC* C, int ldc, int m, int n, int N, 
     }
 }
 
-// More than 16 rows: a workgroup of four waves (2 x 2) on a tile of BM rows of A by BN rows of W. Stages of BK elements
-// of k go through LDS in two buffers: a stage is asked for (16 bytes a lane) before the one at hand is multiplied and
-// written to the other buffer after it, so a stage costs one barrier and no wait for memory. A product of 16 x 16 x 4
-// wants k = k0 + lane / 16 from a lane, so within every 16 k LDS holds a row's elements transposed, element 4 s + q at
-// place 4 q + s: a lane's next four products are then one 16-byte read. Rows are BK + 4 floats apart: the reads of 16
-// rows meet no bank twice. Bound by the matrix cores (a library's large product reaches 154 TFLOP/s here):
-// 4096 x 4096 x 4096 in 1,098 us (125 TFLOP/s), 564 x 6144 x 2048 in 156, 564 x 2048 x 2048 in 68, 64 x 4096 x 4096 in
-// 55; the kernel of vector FMAs and 4-byte loads that this replaced took 2,465, 372, 323 and 632.
-template <class TA, class TW, class TC, bool ACCUM, int BM, int BN, int BK, bool VEC>
-__global__ void __launch_bounds__(256, 2)
+// A sum that is not finite is summed again in plain float32 (an infinity among the operands, or one that rounds to it): what
+// it then is, a chain of fmaf says. Elements n .. n + 3 of row m.
+template <class TA, class TW>
+__device__ __forceinline__ void mend_quad(const TA* A, const TW* W, int lda, int ldw, int m, int n, int N, int K, f32x4& sums) {
+    bool fine = true;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) fine = fine && fabsf(sums[e]) < INFINITY;
+    if (fine) return;
+#pragma unroll 1
+    for (int e = 0; e < 4 && n + e < N; ++e) {
+        const float sum = hb_sum_in_order(A + (size_t)m * lda, W + (size_t)(n + e) * ldw, K, K_BLOCK);
+        sums[0] = e == 0 ? sum : sums[0], sums[1] = e == 1 ? sum : sums[1];
+        sums[2] = e == 2 ? sum : sums[2], sums[3] = e == 3 ? sum : sums[3];
+    }
+}
+
+// How a tile's operands are loaded: element by element; 16 bytes at a time; the same, K being whole stages (then a row is a 32-bit
+// offset from the tile's first and no lane looks where K ends).
+enum { SINGLE, QUADS, WHOLE };
+
+// More than 16 rows: a workgroup on a tile of BM rows of A by BN rows of W, a wave on WM x WN of it, in stages of 32 k. A stage
+// is asked for two stages ahead (a lane's eight elements, 32 bytes), split into its parts by the wave that asked and
+// written to one of two LDS buffers, where an operand of a 16 x 16 x 32 product lies as its lanes read it: no read and no write meets a
+// bank twice, and a stage costs one barrier that waits for no load.
+template <class TA, class TW, class TC, bool ACCUM, int BM, int BN, int WM, int WN, int LOADS>
+__global__ void __launch_bounds__(64 * (BM / WM) * (BN / WN), 2)
 gemm_plain_tile_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* __restrict__ C, int M, int N,
                        int K, int lda, int ldw, int ldc, size_t batch_a, size_t batch_w, size_t batch_c,
                        DecayEpilogue ep) {
@@ -83,169 +97,273 @@ gemm_plain_tile_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
     A += blockIdx.z * batch_a;
     W += blockIdx.z * batch_w;
     C += blockIdx.z * batch_c;
-    constexpr int LD = BK + 4, QUADS = BK / 4;
-    constexpr int QA = BM * QUADS / 256, QW = BN * QUADS / 256;      // quads a thread stages of either operand
-    constexpr int MB = BM / 32, NB = BN / 32;                        // blocks of 16 a wave
-    __shared__ __attribute__((aligned(16))) float As[2][BM * LD], Ws[2][BN * LD];
+    constexpr int WAVES = (BM / WM) * (BN / WN), STAGE = 32, STAGES = K_BLOCK / STAGE, AHEAD = (BM + BN) / 16 / WAVES > 2 ? 2 : 4;
+    constexpr int AB = BM / 16, WB = BN / 16;                            // blocks of 16 rows of a tile's operands
+    constexpr bool EITHER = AB % WAVES != 0;                             // of which a wave stages one, of either operand, or so many of both
+    constexpr int AU = EITHER ? 1 : AB / WAVES, WU = EITHER ? 1 : WB / WAVES;
+    constexpr int MB = WM / 16, NB = WN / 16;                            // and multiplies so many
+    constexpr int AP = Parts<TA>::COUNT, WP = Parts<TW>::COUNT;
+    static_assert(EITHER ? AB == WB && AB + WB == WAVES && std::is_same<TA, TW>::value && LOADS == WHOLE : WB % WAVES == 0, "every wave stages whole blocks");
+    typedef SplitOrder<WP, AP> order;
+    __shared__ __attribute__((aligned(16))) bf16x8 a_lds[2 * AB * AP * HB_WAVE], w_lds[2 * WB * WP * HB_WAVE];   // [buffer][block][part][lane]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r = lane & 15, q = lane >> 4;
     const unsigned across = (N + BN - 1) / BN, tile = blockIdx.y * gridDim.x + blockIdx.x;   // (tiles of a row of tiles)
     if (tile / across >= (unsigned)(M + BM - 1) / BM) return;
     const int m0 = (int)(tile / across) * BM, n0 = (int)(tile % across) * BN;
-    const int wm = (wave & 1) * (BM / 2), wn = (wave >> 1) * (BN / 2);
-
-    f32x4 a_next[QA], w_next[QW];
-    auto fetch = [&](int k0) {
+    const int wm = wave % (BM / WM) * MB, wn = wave / (BM / WM) * NB;    // (in blocks)
+    // rows beyond M or N are the tile's first once more, whose sums go nowhere
+    const TA* const a_tile = A + (size_t)m0 * lda;
+    const TW* const w_tile = W + (size_t)n0 * ldw;
+    unsigned a_row[AU], w_row[WU];
 #pragma unroll
-        for (int i = 0; i < QA; ++i) {
-            const int row = (tid + 256 * i) / QUADS, k = k0 + 4 * ((tid + 256 * i) % QUADS);
-            a_next[i] = load_quad<VEC>(A + (size_t)(m0 + row) * lda + k, m0 + row < M ? K - k : 0);
+    for (int i = 0; i < AU; ++i) {
+        const int row = 16 * ((EITHER ? wave % AB : wave * AU) + i) + r;
+        a_row[i] = (m0 + row < M ? row : 0) * (unsigned)lda + (LOADS == WHOLE ? 8 * q : 0);
+    }
+#pragma unroll
+    for (int i = 0; i < WU; ++i) {
+        const int row = 16 * ((EITHER ? wave % WB : wave * WU) + i) + r;
+        w_row[i] = (n0 + row < N ? row : 0) * (unsigned)ldw + (LOADS == WHOLE ? 8 * q : 0);
+    }
+    const bool stages_w = EITHER && wave >= AB;
+    Oct<TA> a_next[AHEAD][AU];
+    Oct<TW> w_next[AHEAD][WU];
+    auto fetch = [&](int s, Oct<TA>* a, Oct<TW>* w) {
+        const int k = s * STAGE, from = LOADS == WHOLE && k > K - STAGE ? K - STAGE : k;      // (a stage beyond K is the last once more)
+        if constexpr (EITHER) {
+            a[0] = load_oct((stages_w ? w_tile : a_tile) + from, stages_w ? w_row[0] : a_row[0]);
+            return;
         }
 #pragma unroll
-        for (int i = 0; i < QW; ++i) {
-            const int row = (tid + 256 * i) / QUADS, k = k0 + 4 * ((tid + 256 * i) % QUADS);
-            w_next[i] = load_quad<VEC>(W + (size_t)(n0 + row) * ldw + k, n0 + row < N ? K - k : 0);
+        for (int i = 0; i < AU; ++i)
+            a[i] = LOADS == WHOLE ? load_oct(a_tile + from, a_row[i]) : load_oct<LOADS == QUADS>(a_tile + a_row[i], k + 8 * q, K);
+#pragma unroll
+        for (int i = 0; i < WU; ++i)
+            w[i] = LOADS == WHOLE ? load_oct(w_tile + from, w_row[i]) : load_oct<LOADS == QUADS>(w_tile + w_row[i], k + 8 * q, K);
+    };
+    auto cut = [&](int s, Oct<TA>* a, Oct<TW>* w) {          // what lies beyond K
+        const int left = K - s * STAGE;
+        if (LOADS == SINGLE || left >= STAGE) return;
+#pragma unroll
+        for (int i = 0; i < AU; ++i) ends(a[i], left - 8 * q);
+#pragma unroll
+        for (int i = 0; i < (EITHER ? 0 : WU); ++i) ends(w[i], left - 8 * q);
+    };
+    auto stash = [&](int buf, const Oct<TA>* a, const Oct<TW>* w) {
+#pragma unroll
+        for (int i = 0; i < AU; ++i) {
+            const Parts<TA> parts = split(a[i]);
+#pragma unroll
+            for (int p = 0; p < AP; ++p)
+                (stages_w ? w_lds : a_lds)[((buf * AB + (EITHER ? wave % AB : wave * AU) + i) * AP + p) * HB_WAVE + lane] = parts.part[p];
+        }
+#pragma unroll
+        for (int i = 0; i < (EITHER ? 0 : WU); ++i) {
+            const Parts<TW> parts = split(w[i]);
+#pragma unroll
+            for (int p = 0; p < WP; ++p) w_lds[((buf * WB + wave * WU + i) * WP + p) * HB_WAVE + lane] = parts.part[p];
         }
     };
-    auto stash = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < QA; ++i) {
-            const int row = (tid + 256 * i) / QUADS, quad = (tid + 256 * i) % QUADS;
-            float* to = &As[buf][row * LD + (quad & ~3) * 4 + (quad & 3)];
-            to[0] = a_next[i][0], to[4] = a_next[i][1], to[8] = a_next[i][2], to[12] = a_next[i][3];
-        }
-#pragma unroll
-        for (int i = 0; i < QW; ++i) {
-            const int row = (tid + 256 * i) / QUADS, quad = (tid + 256 * i) % QUADS;
-            float* to = &Ws[buf][row * LD + (quad & ~3) * 4 + (quad & 3)];
-            to[0] = w_next[i][0], to[4] = w_next[i][1], to[8] = w_next[i][2], to[12] = w_next[i][3];
-        }
-    };
 
-    static_assert(K_BLOCK % BK == 0, "a stretch of k is whole stages");
-    f32x4 acc[NB][MB], total[NB][MB];
+    f32x4 top[NB][MB], low[NB][MB], total[NB][MB];
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll
-        for (int i = 0; i < MB; ++i) total[j][i] = acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < MB; ++i) total[j][i] = top[j][i] = low[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    fetch(0);
-    stash(0);
-    __syncthreads();
-    int buf = 0;
-    for (int k0 = 0; k0 < K; k0 += BK, buf ^= 1) {
-        const bool more = k0 + BK < K;
-        if (more) fetch(k0 + BK);
+    // stage s, in LDS; the one AHEAD from here is asked for, the next one written to the other buffer.
+    auto step = [&](int s, int at) {
+        const int buf = at & 1;
+        Oct<TA>* a_near = a_next[(at + 1) % AHEAD];
+        Oct<TW>* w_near = w_next[(at + 1) % AHEAD];
+        cut(s + 1, a_near, w_near);
+        fetch(s + AHEAD, a_next[at], w_next[at]);
+        bf16x8 a[MB][AP], w[NB][WP];
 #pragma unroll
-        for (int b = 0; b < BK / 16; ++b) {
-            f32x4 a[MB], w[NB];
+        for (int i = 0; i < MB; ++i)
 #pragma unroll
-            for (int i = 0; i < MB; ++i) a[i] = *(const f32x4*)&As[buf][(wm + 16 * i + r) * LD + 16 * b + 4 * q];
+            for (int p = 0; p < AP; ++p) a[i][p] = a_lds[((buf * AB + wm + i) * AP + p) * HB_WAVE + lane];
 #pragma unroll
-            for (int j = 0; j < NB; ++j) w[j] = *(const f32x4*)&Ws[buf][(wn + 16 * j + r) * LD + 16 * b + 4 * q];
+        for (int j = 0; j < NB; ++j)
 #pragma unroll
-            for (int s = 0; s < 4; ++s)
+            for (int p = 0; p < WP; ++p) w[j][p] = w_lds[((buf * WB + wn + j) * WP + p) * HB_WAVE + lane];
+#pragma unroll
+        for (int p = 0; p < SPLIT_PRODUCTS; ++p)
+            if (order::there(p)) {
 #pragma unroll
                 for (int j = 0; j < NB; ++j)
 #pragma unroll
-                    for (int i = 0; i < MB; ++i) acc[j][i] = mfma_k4(w[j][s], a[i][s], acc[j][i]);
-        }
-        if (more) stash(buf ^ 1);
-        if (!more || (k0 + BK) % K_BLOCK == 0) {
+                    for (int i = 0; i < MB; ++i) {
+                        f32x4& sums = p == SPLIT_PRODUCTS - 1 ? top[j][i] : low[j][i];
+                        sums = mfma_k32(w[j][order::w[p] % WP], a[i][order::a[p] % AP], sums);
+                    }
+            }
+        stash(buf ^ 1, a_near, w_near);
+        hb_workgroup_barrier();
+    };
 #pragma unroll
-            for (int j = 0; j < NB; ++j)
+    for (int i = 0; i < AHEAD; ++i) fetch(i, a_next[i], w_next[i]);
+    cut(0, a_next[0], w_next[0]);
+    stash(0, a_next[0], w_next[0]);
+    hb_workgroup_barrier();
+    for (int s = 0; s * STAGE < K;) {
+        // (AHEAD stages at a time: what lies beyond K are zeros)
+        const int left = K - s * STAGE, stop = s + (left >= K_BLOCK ? STAGES : (left + AHEAD * STAGE - 1) / (AHEAD * STAGE) * AHEAD);
+        for (; s < stop; s += AHEAD)
 #pragma unroll
-                for (int i = 0; i < MB; ++i) total[j][i] += acc[j][i], acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
-        __syncthreads();
+            for (int at = 0; at < AHEAD; ++at) step(s + at, at);
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int i = 0; i < MB; ++i) {
+                total[j][i] += top[j][i] + low[j][i];
+                top[j][i] = low[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
     }
 
 #pragma unroll
     for (int i = 0; i < MB; ++i) {
-        const int m = m0 + wm + 16 * i + r;
+        const int m = m0 + 16 * (wm + i) + r;
         if (m >= M) continue;
 #pragma unroll
-        for (int j = 0; j < NB; ++j)
-            store_quad<TC, ACCUM, VEC>(C, ldc, m, n0 + wn + 16 * j + 4 * q, N, total[j][i], ep);
+        for (int j = 0; j < NB; ++j) {
+            const int n = n0 + 16 * (wn + j) + 4 * q;
+            mend_quad(A, W, lda, ldw, m, n, N, K, total[j][i]);
+            store_quad<TC, ACCUM, LOADS != SINGLE>(C, ldc, m, n, N, total[j][i], ep);
+        }
     }
 }
 
-// Up to 16 rows (a decode step): a product bound by the weights' bytes and, narrow ones, by the chain of k. A workgroup
-// on 16 rows of W, a wave on every stretch of K_BLOCK (up to WAVE_WAVES of them at a time): no load waits for another
-// wave, and a wave asks for all of its stretch of W at once (32 quads a lane), for A eight blocks of 16 k ahead; the
-// lanes' quads are transposed in registers. The stretches' sums meet in LDS, where a thread an output adds them in
-// their order. 2 x 2048 x 2048 takes 10.7 us (one wave for all of k, a chain of 512 products with eight blocks in
-// flight: 19.4), 2 x 2048 x 3072 12.8 (27.9), 2 x 4096 x 2048 13.3 (20.0), 8 x 4096 x 12288 62 (106); with bfloat16
-// weights 10.5 (36), 12.9 (53), 11 (38) and 43 (233).
-#define WAVE_ROWS 16
+// Few rows of A (a decode step, a short prompt): a product bound by the weights' bytes and, narrow ones, by the chain of k. A
+// workgroup on 16 rows of W and MB blocks of 16 rows of A, a wave on every stretch of K_BLOCK (up to MOST of them at a
+// time): no load waits for another wave, and a wave asks for all of its stretch of W at once (16 pieces of 8 elements a lane), for A
+// some pieces ahead, and splits both in registers. The stretches' sums meet in LDS, where a thread an output adds them in
+// their order.
 #define WAVE_WAVES 8
-#define WAVE_DEPTH 8
-template <class TA, class TW, class TC, bool ACCUM>
-__global__ void __launch_bounds__(WAVE_WAVES * HB_WAVE)
+#define WAVE_DEPTH 4
+template <class TA, class TW, class TC, bool ACCUM, int MB, int NB, int AHEAD>
+__global__ void __launch_bounds__(WAVE_WAVES * HB_WAVE, AHEAD == 8 ? 4 : 2)
 gemm_plain_wave_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* __restrict__ C, int M, int N,
                        int K, int lda, int ldw, int ldc, size_t batch_a, size_t batch_w, size_t batch_c,
                        DecayEpilogue ep) {
     A += blockIdx.z * batch_a;
     W += blockIdx.z * batch_w;
     C += blockIdx.z * batch_c;
-    constexpr int GROUPS = K_BLOCK / 16 / WAVE_DEPTH;
-    __shared__ __attribute__((aligned(16))) f32x4 sums[WAVE_WAVES][HB_WAVE];
+    constexpr int UNITS = K_BLOCK / 32, A_AHEAD = NB > 1 ? 4 : AHEAD == UNITS ? 8 : 2;
+    __shared__ __attribute__((aligned(16))) f32x4 sums[WAVE_WAVES][NB][MB][HB_WAVE];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
     const int r = lane & 15, q = lane >> 4;
-    const int n0 = blockIdx.x * 16;
-    // (rows beyond M or N are row 0 once more, whose sums go nowhere; blocks beyond K are zeros)
-    const TW* w_row = W + (size_t)(n0 + r < N ? n0 + r : 0) * ldw + 4 * q;
-    const TA* a_row = A + (size_t)(r < M ? r : 0) * lda + 4 * q;
-    f32x4 total = {0.f, 0.f, 0.f, 0.f};
+    const int n0 = blockIdx.x * 16 * NB, m0 = blockIdx.y * 16 * MB;
+    // (rows beyond M or N are rows at hand once more, whose sums go nowhere; pieces beyond K are zeros)
+    const TW* w_row[NB];
+    const TA* a_row[MB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) w_row[j] = W + (size_t)(n0 + 16 * j + r < N ? n0 + 16 * j + r : n0) * ldw;
+#pragma unroll
+    for (int i = 0; i < MB; ++i) a_row[i] = A + (size_t)(m0 + 16 * i + r < M ? m0 + 16 * i + r : m0) * lda;
+    f32x4 total[NB][MB], top[NB][MB], low[NB][MB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int i = 0; i < MB; ++i) total[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int first = 0; first < K; first += waves * K_BLOCK) {
         const int k0 = first + wave * K_BLOCK;
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int i = 0; i < MB; ++i) top[j][i] = low[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (k0 + K_BLOCK <= K) {
-            f32x4 w[GROUPS][WAVE_DEPTH], a[2][WAVE_DEPTH];
-            auto fetch_a = [&](int g) {
+            Oct<TW> w[AHEAD][NB];
+            Oct<TA> a[A_AHEAD][MB];
+            auto fetch_w = [&](int u) {
 #pragma unroll
-                for (int d = 0; d < WAVE_DEPTH; ++d) a[g & 1][d] = load_quad<true>(a_row + k0 + 16 * (g * WAVE_DEPTH + d), 4);
+                for (int j = 0; j < NB; ++j) w[u % AHEAD][j] = load_oct(w_row[j] + k0 + 32 * u, 8u * q);
             };
-            fetch_a(0);
+            auto fetch_a = [&](int u) {
 #pragma unroll
-            for (int g = 0; g < GROUPS; ++g)
+                for (int i = 0; i < MB; ++i) a[u % A_AHEAD][i] = load_oct(a_row[i] + k0 + 32 * u, 8u * q);
+            };
 #pragma unroll
-                for (int d = 0; d < WAVE_DEPTH; ++d) w[g][d] = load_quad<true>(w_row + k0 + 16 * (g * WAVE_DEPTH + d), 4);
+            for (int u = 0; u < A_AHEAD; ++u) fetch_a(u);
 #pragma unroll
-            for (int g = 0; g < GROUPS; ++g) {
-                if (g + 1 < GROUPS) fetch_a(g + 1);
+            for (int u = 0; u < AHEAD; ++u) fetch_w(u);
+            __builtin_amdgcn_sched_barrier(0);       // (no load waits for the sums before it)
 #pragma unroll
-                for (int d = 0; d < WAVE_DEPTH; ++d) {
-                    transpose_quads(w[g][d]);
-                    transpose_quads(a[g & 1][d]);
+            for (int u = 0; u < UNITS; ++u) {
+                Parts<TW> w_parts[NB];
 #pragma unroll
-                    for (int s = 0; s < 4; ++s) acc = mfma_k4(w[g][d][s], a[g & 1][d][s], acc);
+                for (int j = 0; j < NB; ++j) w_parts[j] = split(w[u % AHEAD][j]);
+                if (u + AHEAD < UNITS) fetch_w(u + AHEAD);
+#pragma unroll
+                for (int i = 0; i < MB; ++i) {
+                    const Parts<TA> a_parts = split(a[u % A_AHEAD][i]);
+#pragma unroll
+                    for (int j = 0; j < NB; ++j) mfma_split<TW, TA>(w_parts[j], a_parts, top[j][i], low[j][i]);
                 }
+                if (u + A_AHEAD < UNITS) fetch_a(u + A_AHEAD);
             }
         } else {
-            for (int k = k0; k < K; k += 16) {       // (what is left of k, blocks of 16)
-                f32x4 w = load_quad<true>(w_row + k, 4), a = load_quad<true>(a_row + k, 4);
-                transpose_quads(w);
-                transpose_quads(a);
+            for (int k = k0; k < K; k += 32 * WAVE_DEPTH) {      // (what is left of k)
+                Oct<TW> w[WAVE_DEPTH][NB];
+                Oct<TA> a[WAVE_DEPTH][MB];
 #pragma unroll
-                for (int s = 0; s < 4; ++s) acc = mfma_k4(w[s], a[s], acc);
+                for (int d = 0; d < WAVE_DEPTH; ++d) {
+#pragma unroll
+                    for (int j = 0; j < NB; ++j) w[d][j] = load_oct<true>(w_row[j], k + 32 * d + 8 * q, K);
+#pragma unroll
+                    for (int i = 0; i < MB; ++i) a[d][i] = load_oct<true>(a_row[i], k + 32 * d + 8 * q, K);
+                }
+#pragma unroll
+                for (int d = 0; d < WAVE_DEPTH; ++d) {
+                    const int left = K - k - 32 * d;
+                    if (left <= 0) break;
+                    Parts<TW> w_parts[NB];
+#pragma unroll
+                    for (int j = 0; j < NB; ++j) {
+                        if (left < 32) ends(w[d][j], left - 8 * q);
+                        w_parts[j] = split(w[d][j]);
+                    }
+#pragma unroll
+                    for (int i = 0; i < MB; ++i) {
+                        if (left < 32) ends(a[d][i], left - 8 * q);
+                        const Parts<TA> a_parts = split(a[d][i]);
+#pragma unroll
+                        for (int j = 0; j < NB; ++j) mfma_split<TW, TA>(w_parts[j], a_parts, top[j][i], low[j][i]);
+                    }
+                }
             }
         }
         if (first) __syncthreads();                  // (the round before has been read)
-        sums[wave][lane] = acc;
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int i = 0; i < MB; ++i) sums[wave][j][i][lane] = top[j][i] + low[j][i];
         __syncthreads();
         if (wave == 0)
-            for (int b = 0; b < waves && first + b * K_BLOCK < K; ++b) total += sums[b][lane];
+            for (int b = 0; b < waves && first + b * K_BLOCK < K; ++b)
+#pragma unroll
+                for (int j = 0; j < NB; ++j)
+#pragma unroll
+                    for (int i = 0; i < MB; ++i) total[j][i] += sums[b][j][i][lane];
     }
-    if (wave == 0 && r < M) store_quad<TC, ACCUM, true>(C, ldc, r, n0 + 4 * q, N, total, ep);
+    if (wave) return;
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+        const int m = m0 + 16 * i + r;
+        if (m >= M) continue;
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+            const int n = n0 + 16 * j + 4 * q;
+            mend_quad(A, W, lda, ldw, m, n, N, K, total[j][i]);
+            store_quad<TC, ACCUM, true>(C, ldc, m, n, N, total[j][i], ep);
+        }
+    }
 }
 
-// The same rows for float32 weights that fill the chip with a wave for every 16 of their rows, or whose k is so short that there
-// is nothing to share: no LDS and no barrier; a wave goes through the stretches one after another, the next WAVE_DEPTH blocks of 16 k of
-// W and A on their way while the WAVE_DEPTH before are multiplied. Microseconds by the kernel above / this one, two rows: 4096 x 480 10.8 /
-// 6.8, 2048 x 896 10.8 / 10.0, 4096 x 1024 9.4 / 11.3, 8192 x 1024 13.8 / 12.5, 8192 x 1504 20.7 / 17.3, 8192 x 2048 20.1 / 21.7, 12288 x 2048 24.1 /
-// 23.6, 12288 x 4096 46.7 / 42.2, 32768 x 2048 61.6 / 54.6, 4096 x 64 2.9 / 3.0, 4096 x 16 2.4 / 3.1. With bfloat16 weights it is the slower one
-// everywhere (32768 x 2048 46.9 / 79.4).
+// Up to 16 rows on float32 weights whose k is so short that there
+// is nothing to share: no LDS and no barrier; a wave goes through the stretches one after another, the next WAVE_DEPTH pieces of 32 k of
+// W and A on their way while the WAVE_DEPTH before are multiplied.
 template <class TA, class TW, class TC, bool ACCUM>
 __global__ void __launch_bounds__(HB_WAVE)
 gemm_plain_stream_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* __restrict__ C, int M, int N,
@@ -254,45 +372,80 @@ gemm_plain_stream_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC*
     A += blockIdx.z * batch_a;
     W += blockIdx.z * batch_w;
     C += blockIdx.z * batch_c;
-    static_assert(K_BLOCK % (16 * WAVE_DEPTH) == 0, "a stretch of k is whole rounds of loads");
+    constexpr int ROUND = 32 * WAVE_DEPTH;
+    static_assert(K_BLOCK % ROUND == 0, "a stretch of k is whole rounds of loads");
     const int lane = threadIdx.x, r = lane & 15, q = lane >> 4;
     const int n0 = blockIdx.x * 16;
-    // (rows beyond M or N are row 0 once more, whose sums go nowhere; blocks beyond K are zeros)
-    const TW* w_row = W + (size_t)(n0 + r < N ? n0 + r : 0) * ldw + 4 * q;
-    const TA* a_row = A + (size_t)(r < M ? r : 0) * lda + 4 * q;
-    f32x4 total = {0.f, 0.f, 0.f, 0.f}, acc = total, w_next[WAVE_DEPTH], a_next[WAVE_DEPTH];
+    // (rows beyond M or N are row 0 once more, whose sums go nowhere; pieces beyond K are zeros)
+    const TW* w_row = W + (size_t)(n0 + r < N ? n0 + r : 0) * ldw;
+    const TA* a_row = A + (size_t)(r < M ? r : 0) * lda;
+    f32x4 total = {0.f, 0.f, 0.f, 0.f}, top = total, low = total;
+    Oct<TW> w_next[WAVE_DEPTH];
+    Oct<TA> a_next[WAVE_DEPTH];
     auto fetch = [&](int k0) {
 #pragma unroll
         for (int d = 0; d < WAVE_DEPTH; ++d) {
-            const int k = k0 + 16 * d;
-            w_next[d] = load_quad<true>(w_row + k, K - k);
-            a_next[d] = load_quad<true>(a_row + k, K - k);
+            w_next[d] = load_oct<true>(w_row, k0 + 32 * d + 8 * q, K);
+            a_next[d] = load_oct<true>(a_row, k0 + 32 * d + 8 * q, K);
         }
     };
     fetch(0);
-    for (int k0 = 0; k0 < K; k0 += 16 * WAVE_DEPTH) {
-        f32x4 w[WAVE_DEPTH], a[WAVE_DEPTH];
+    for (int k0 = 0; k0 < K; k0 += ROUND) {
+        Oct<TW> w[WAVE_DEPTH];
+        Oct<TA> a[WAVE_DEPTH];
 #pragma unroll
         for (int d = 0; d < WAVE_DEPTH; ++d) w[d] = w_next[d], a[d] = a_next[d];
-        const bool more = k0 + 16 * WAVE_DEPTH < K;
-        if (more) fetch(k0 + 16 * WAVE_DEPTH);
+        const bool more = k0 + ROUND < K;
+        fetch(k0 + ROUND);
+        if (!more)
 #pragma unroll
-        for (int d = 0; d < WAVE_DEPTH; ++d) {
-            transpose_quads(w[d]);
-            transpose_quads(a[d]);
+            for (int d = 0; d < WAVE_DEPTH; ++d) {
+                ends(w[d], K - k0 - 32 * d - 8 * q);
+                ends(a[d], K - k0 - 32 * d - 8 * q);
+            }
 #pragma unroll
-            for (int s = 0; s < 4; ++s) acc = mfma_k4(w[d][s], a[d][s], acc);
+        for (int d = 0; d < WAVE_DEPTH; ++d) mfma_split<TW, TA>(split(w[d]), split(a[d]), top, low);
+        if (!more || (k0 + ROUND) % K_BLOCK == 0) {
+            total += top + low;
+            top = low = f32x4{0.f, 0.f, 0.f, 0.f};
         }
-        if (!more || (k0 + 16 * WAVE_DEPTH) % K_BLOCK == 0) total += acc, acc = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    if (r < M) store_quad<TC, ACCUM, true>(C, ldc, r, n0 + 4 * q, N, total, ep);
+    if (r < M) {
+        mend_quad(A, W, lda, ldw, r, n0 + 4 * q, N, K, total);
+        store_quad<TC, ACCUM, true>(C, ldc, r, n0 + 4 * q, N, total, ep);
+    }
 }
 
-// The kernel of a product. 16-byte loads and stores where rows and strides allow them. Up to 16 rows of whole blocks of
-// 16 k take one of the two kernels above. Beyond, the tile with the least estimated time: what a CU spends on one (microseconds at K = 2048 on all
-// CUs: 128 x 128 137, alone on a CU 152; 64 x 64 43.5 and 52; 32 x 32 12.8, of which four or more share a CU and few are left over) times
-// the most that a CU gets. Measured by 128 / 64 / 32: 564 x 6144 x 2048 156 / 168 / 173 us, 564 x 4096 x 2048 155 / 132 / 116, 564 x 2048 x
-// 2048 152 / 87 / 68, 1200 x 4096 x 4096 546 / 419 / 456, 4096 x 4096 x 4096 1,098 / 1,307 / 1,489. (Tiles of 64 x 32: 162, 115, 72.)
+// The kernel of a product of more than 16 rows: the one with the least estimated time, in microseconds. A wave of 16 x 16 or 32 x 32
+// (x 512 of k) costs what a SIMD takes for it times the waves a SIMD gets; a tile's stage of 32 k what a CU takes for it times the
+// tiles a CU gets, and no less than the chain from its reads of LDS over its products and the next stage's splitting to the barrier. Both sides float32 | one of
+// them bfloat16: 16 x 16 8.0 | 5.3, 32 x 32 by a wave 16.2 | 11.5, tiles of 32 x 32 0.23 | 0.18 a stage (at least 0.295 | 0.27), 64 x 64 0.48 | 0.35,
+// 128 x 128 1.35 | 0.80. Measured, microseconds by 16 x 16 / 32 x 32 / tiles of 32 / 64 / 128 [the float32 matrix instructions before], float32 weights: 17 x
+// 2048 x 2048 11 / 21 / 21 / 32 / 76 [22], 17 x 4096 x 2048 17 / 28 / 21 / 32 / 77 [29], 128 x 2048 x 2048 33 / 21 / 21 / 33 / 78 [23], 200 x 4096 x 2048 97 / 60 / 60 /
+// 37 / 78 [54], 563 x 4096 x 2048 262 / 139 / 137 / 94 / 80 [114], 563 x 6144 x 2048 388 / 207 / 210 / 126 / 93 [155], 563 x 2048 x 3072 232 / 133 / 113 / 89 / 116 [98];
+// bfloat16 weights: 64 x 2048 x 2048 13 / 16 / 19 / 25 / 49 [39], 563 x 4096 x 2048 191 / 105 / 110 / 69 / 52 [163].
+// whole: K is whole stages, the larger tiles take nothing else; a decay's exponentials and logarithms are a tile's own tail: not 64 of them a lane.
+enum { STREAM, WAVE, WAVE_RING, WAVE_SQUARE, TILE_SINGLE, TILE_QUADS, TILE_32, TILE_64, TILE_128 };
+static int gemm_plain_choice(int M, int N, int K, int batch, bool both, bool whole, bool decay) {
+    auto tiles = [&](int side) { return (double)((N + side - 1ll) / side * ((M + side - 1) / side) * batch); };
+    auto most = [&](int side) { return (double)(((long long)tiles(side) + 255) / 256); };
+    auto larger = [](double a, double b) { return a > b ? a : b; };
+    const double never = 1e30, stages = (K + 127) / 128 * 4, part = K < K_BLOCK ? (double)K / K_BLOCK : 1.0;
+    const double per_simd = part * ((K + K_BLOCK - 1) / K_BLOCK) / 1024.0, least = K < K_BLOCK ? 0.2 * part : 0.5;
+    const struct {
+        int kernel;
+        double cost;
+    } all[5] = {
+        {WAVE, M > 4096 ? never : 2.6 + (both ? 8.0 : 5.3) * larger(per_simd * tiles(16), least)},
+        {WAVE_SQUARE, M > 4096 ? never : both ? 5.0 + larger(16.2 * per_simd * tiles(32), 12.0 * part) : 3.5 + larger(11.5 * per_simd * tiles(32), 10.0 * part)},
+        {whole ? TILE_32 : TILE_QUADS, 2.4 + stages * (both ? larger(0.295, 0.03 + 0.23 * most(32)) : larger(0.27, 0.03 + 0.18 * most(32)))},
+        {TILE_64, !whole ? never : 2.4 + stages * (both ? 0.48 : 0.35) * most(64)},
+        {TILE_128, !whole || decay ? never : 3.0 + stages * (both ? 1.35 : 0.80) * most(128)}};
+    int best = 0;
+    for (int i = 1; i < 5; ++i) best = all[i].cost < all[best].cost ? i : best;
+    return all[best].kernel;
+}
+
 #define GRID_X (1 << 23)
 // What the entries take: rows as ever, and tiles of 32 x 32 that GRID_X times 256 hold (2 T sums a product).
 #define HB_REQUIRE_TILES(M, N)                                                                                        \
@@ -303,42 +456,56 @@ gemm_plain_stream_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC*
 template <class TA, class TW, class TC, bool ACCUM>
 static void launch_as(const TA* A, const TW* W, TC* C, int M, int N, int K, int lda, int ldw, int ldc,
                       hipStream_t stream, int batch, size_t batch_a, size_t batch_w, size_t batch_c, DecayEpilogue ep) {
-    const bool vec = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && batch_a % 4 == 0 && batch_w % 4 == 0 &&
-                     (uintptr_t)A % (4 * sizeof(TA)) == 0 && (uintptr_t)W % (4 * sizeof(TW)) == 0 &&
+    // (16-byte loads and stores where rows and strides allow them)
+    constexpr int EA = 16 / sizeof(TA), EW = 16 / sizeof(TW);
+    const bool vec = K % EA == 0 && K % EW == 0 && lda % EA == 0 && ldw % EW == 0 && batch_a % EA == 0 && batch_w % EW == 0 &&
+                     (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0 &&
                      (sizeof(TC) != 4 || (N % 4 == 0 && ldc % 4 == 0 && batch_c % 4 == 0 && (uintptr_t)C % 16 == 0));
-    auto tiles = [&](int side) { return (long long)((N + side - 1) / side) * ((M + side - 1) / side) * batch; };
+    auto tiles = [&](int high, int wide) { return (long long)((N + wide - 1) / wide) * ((M + high - 1) / high) * batch; };
     // (a grid's x holds fewer than 2^32 threads: beyond GRID_X tiles the rest lie along its y)
-    auto grid = [&](int side) {
-        const long long n = tiles(side) / batch, x = n < GRID_X ? n : GRID_X;
+    auto grid = [&](int high, int wide) {
+        const long long n = tiles(high, wide) / batch, x = n < GRID_X ? n : GRID_X;
         return dim3((unsigned)x, (unsigned)((n + x - 1) / x), batch);
     };
-    const int stretches = (K + K_BLOCK - 1) / K_BLOCK, wave_threads = HB_WAVE * (stretches < WAVE_WAVES ? stretches : WAVE_WAVES);
-    auto most = [&](int side) { return (double)((tiles(side) + 255) / 256); };
-    // (a decay's exponentials and logarithms are a tile's own tail: not 64 of them a lane)
-    const double large = ep.rate ? 1e30 : tiles(128) <= 256 ? 152.0 : 137.0 * most(128), medium = tiles(64) <= 256 ? 52.0 : 43.5 * most(64),
-                 small = 12.8 * (tiles(32) <= 460 ? 1.8 : tiles(32) / 256.0);
-#define HB_PLAIN_TILE(BM, BK, VEC)                                                                                    \
-    gemm_plain_tile_kernel<TA, TW, TC, ACCUM, BM, BM, BK, VEC>                                                        \
-        <<<grid(BM), 256, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, batch_a, batch_w, batch_c, ep)
-    // (both sides of these lines stand at gemm_plain_stream_kernel)
+    const int stretches = (K + K_BLOCK - 1) / K_BLOCK;
+#define HB_PLAIN_TILE(BM, BN, WM, WN, LOADS)                                                                          \
+    gemm_plain_tile_kernel<TA, TW, TC, ACCUM, BM, BN, WM, WN, LOADS>                                                  \
+        <<<grid(BM, BN), 64 * (BM / WM) * (BN / WN), 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, batch_a, batch_w,  \
+                                                                 batch_c, ep)
+#define HB_PLAIN_WAVE(MB, NB, AHEAD)                                                                                  \
+    gemm_plain_wave_kernel<TA, TW, TC, ACCUM, MB, NB, AHEAD>                                                          \
+        <<<dim3((N + 16 * NB - 1) / (16 * NB), (M + 16 * MB - 1) / (16 * MB), batch), HB_WAVE * at_once, 0, stream>>>( \
+            A, W, C, M, N, K, lda, ldw, ldc, batch_a, batch_w, batch_c, ep)
+    // (both sides of the first two lines stand at the kernels)
     const long long strips = (N + 15ll) / 16 * batch;
-    const bool streams = sizeof(TW) == 4 && K > 64 && (K < 1024 || strips >= 768 || (K < 2048 && strips >= 512));
-    if (vec && M <= WAVE_ROWS && K % 16 == 0 && streams) {
-        if constexpr (sizeof(TW) == 4)
-            gemm_plain_stream_kernel<TA, TW, TC, ACCUM><<<dim3((N + 15) / 16, 1, batch), HB_WAVE, 0, stream>>>(
-                A, W, C, M, N, K, lda, ldw, ldc, batch_a, batch_w, batch_c, ep);
+    const int at_once = stretches < WAVE_WAVES ? stretches : WAVE_WAVES;
+    const int which = !vec                                                      ? TILE_SINGLE
+                      : M <= 16 && sizeof(TW) == 4 && K < 1024 && K > 64 && K % K_BLOCK ? STREAM
+                      : M <= 16                                                 ? strips * at_once > 2048 ? WAVE_RING : WAVE
+                                                                                : gemm_plain_choice(M, N, K, batch, Parts<TA>::COUNT + Parts<TW>::COUNT == 6,
+                                                                                                    K % 32 == 0 && lda < 1 << 23 && ldw < 1 << 23, ep.rate != nullptr);
+    switch (which) {
+        case STREAM:
+            if constexpr (sizeof(TW) == 4)
+                gemm_plain_stream_kernel<TA, TW, TC, ACCUM><<<dim3((N + 15) / 16, 1, batch), HB_WAVE, 0, stream>>>(
+                    A, W, C, M, N, K, lda, ldw, ldc, batch_a, batch_w, batch_c, ep);
+            break;
+        case WAVE: HB_PLAIN_WAVE(1, 1, 16); break;
+        case WAVE_RING: HB_PLAIN_WAVE(1, 1, 8); break;
+        case WAVE_SQUARE: HB_PLAIN_WAVE(2, 2, 4); break;
+        case TILE_SINGLE: HB_PLAIN_TILE(32, 32, 16, 32, SINGLE); break;
+        case TILE_QUADS: HB_PLAIN_TILE(32, 32, 16, 32, QUADS); break;
+        case TILE_32:            // (a wave stages a block of either operand, where both are of a kind: half the splitting in a stage's chain)
+            if constexpr (std::is_same<TA, TW>::value) HB_PLAIN_TILE(32, 32, 16, 16, WHOLE);
+            else HB_PLAIN_TILE(32, 32, 16, 32, WHOLE);
+            break;
+        case TILE_64:
+            if constexpr (std::is_same<TA, TW>::value) HB_PLAIN_TILE(64, 64, 16, 32, WHOLE);
+            else HB_PLAIN_TILE(64, 64, 32, 32, WHOLE);
+            break;
+        case TILE_128: HB_PLAIN_TILE(128, 128, 64, 32, WHOLE); break;
     }
-    else if (vec && M <= WAVE_ROWS && K % 16 == 0)
-        gemm_plain_wave_kernel<TA, TW, TC, ACCUM><<<dim3((N + 15) / 16, 1, batch), wave_threads, 0, stream>>>(
-            A, W, C, M, N, K, lda, ldw, ldc, batch_a, batch_w, batch_c, ep);
-    else if (!vec)
-        HB_PLAIN_TILE(32, 64, false);
-    else if (large <= medium && large <= small)
-        HB_PLAIN_TILE(128, 32, true);
-    else if (medium <= small)
-        HB_PLAIN_TILE(64, 64, true);
-    else
-        HB_PLAIN_TILE(32, 64, true);
+#undef HB_PLAIN_WAVE
 #undef HB_PLAIN_TILE
 }
 

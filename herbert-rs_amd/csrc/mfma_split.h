@@ -1,0 +1,124 @@
+// Float32 products on the bfloat16 matrix cores. A float32 number is the sum of three bfloat16 ones, exactly: v rounded to
+// bfloat16, the rest rounded, and what then is left, which has at most eight bits. Of the nine products of two such
+// numbers' parts six are summed (the other three are below 2^-25 of the whole product), each exact: a product of
+// 16 x 16 x 32 costs six instructions of 16 cycles where the float32 matrix instructions need eight of 32, three
+// where one side is stored in bfloat16. The leading parts' products and the five smaller ones have a sum each: the matrix cores round a
+// sum once in 32 k, and the smaller sums' roundings weigh next to nothing. Over normal, positive and very uneven operands and K from
+// 32 to 12288 the error against 64 bits is 0.32 to 0.94 of that of a chain of fmaf in the same stretches (all six in one sum: 0.36 to 0.92, with a drift
+// towards -infinity that the matrix cores' own adding brings and the short sums here do not show).
+// What is not finite spoils its parts (infinity minus infinity), as does what rounds to infinity: callers take a sum that is
+// not finite from `hb_sum_in_order` instead. Numbers below 2^-110 lose the bits that bfloat16 cannot hold (below 2^-133).
+#pragma once
+#include "mfma_f32.h"
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+// Eight neighbouring elements of a row as they are stored, and their parts. A lane's eight are those of row lane % 16 at
+// k0 + 8 (lane / 16): what a product of 16 x 16 x 32 wants of either operand.
+template <class T> struct Oct;
+template <> struct Oct<float> {
+    f32x4 quad[2];
+};
+template <> struct Oct<bf16> {
+    bf16x8 all;
+};
+template <class T> struct Parts {
+    static constexpr int COUNT = sizeof(T) == 4 ? 3 : 1;
+    bf16x8 part[COUNT];
+};
+
+// The eight of `row` from k on. VEC: 16-byte loads (the row aligned to 16 bytes, K a multiple of what one holds); what lies at
+// or beyond K is something of the row's: `ends` makes zeros of it. No branch hangs on k, so that no load is waited for where
+// the paths of one would meet. Otherwise: element by element, zeros from K on.
+template <bool VEC>
+__device__ __forceinline__ Oct<float> load_oct(const float* row, int k, int K) {
+    if (VEC) return Oct<float>{{*(const f32x4*)(row + (k < K ? k : 0)), *(const f32x4*)(row + (k + 4 < K ? k + 4 : 0))}};
+    return Oct<float>{{load_quad<false>(row + k, K - k), load_quad<false>(row + k + 4, K - k - 4)}};
+}
+template <bool VEC>
+__device__ __forceinline__ Oct<bf16> load_oct(const bf16* row, int k, int K) {
+    if (VEC) return Oct<bf16>{*(const bf16x8*)(row + (k < K ? k : 0))};
+    Oct<bf16> r;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r.all[i] = k + i < K ? __builtin_bit_cast(__bf16, row[k + i].bits) : (__bf16)0.f;
+    return r;
+}
+// The eight at `offset` elements from a place that is the same for all lanes.
+__device__ __forceinline__ Oct<float> load_oct(const float* place, unsigned offset) {
+    const char* at = (const char*)place + offset * 4u;
+    return Oct<float>{{*(const f32x4*)at, *(const f32x4*)(at + 16)}};
+}
+__device__ __forceinline__ Oct<bf16> load_oct(const bf16* place, unsigned offset) {
+    return Oct<bf16>{*(const bf16x8*)((const char*)place + offset * 2u)};
+}
+__device__ __forceinline__ void ends(Oct<float>& o, int left) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o.quad[i / 4][i % 4] = i < left ? o.quad[i / 4][i % 4] : 0.f;
+}
+__device__ __forceinline__ void ends(Oct<bf16>& o, int left) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o.all[i] = i < left ? o.all[i] : (__bf16)0.f;
+}
+
+// Each rest, v - (float)part, is exact and one instruction: a product of two pairs and a sum, with -1 and 0. (The pair -1, 0 is hidden
+// from the compiler, which would write the float -1, whose halves are 0, -1, in its place.)
+__device__ __forceinline__ void split_pair(float v0, float v1, bf16x2& top, bf16x2& mid, bf16x2& low) {
+    unsigned first_bits = 0x0000bf80u, second_bits = 0xbf800000u;
+    asm("" : "+s"(first_bits), "+s"(second_bits));
+    const bf16x2 first = __builtin_bit_cast(bf16x2, first_bits), second = __builtin_bit_cast(bf16x2, second_bits);
+    top = bf16x2{(__bf16)v0, (__bf16)v1};
+    v0 = __builtin_amdgcn_fdot2_f32_bf16(top, first, v0, false), v1 = __builtin_amdgcn_fdot2_f32_bf16(top, second, v1, false);
+    mid = bf16x2{(__bf16)v0, (__bf16)v1};
+    v0 = __builtin_amdgcn_fdot2_f32_bf16(mid, first, v0, false), v1 = __builtin_amdgcn_fdot2_f32_bf16(mid, second, v1, false);
+    low = bf16x2{(__bf16)v0, (__bf16)v1};
+}
+__device__ __forceinline__ Parts<float> split(const Oct<float>& o) {
+    Parts<float> r;
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) {
+        bf16x2 top, mid, low;
+        split_pair(o.quad[i / 4][i % 4], o.quad[i / 4][i % 4 + 1], top, mid, low);
+        r.part[0][i] = top[0], r.part[0][i + 1] = top[1];
+        r.part[1][i] = mid[0], r.part[1][i + 1] = mid[1];
+        r.part[2][i] = low[0], r.part[2][i + 1] = low[1];
+    }
+    return r;
+}
+__device__ __forceinline__ Parts<bf16> split(const Oct<bf16>& o) { return Parts<bf16>{{o.all}}; }
+
+// Which parts meet, the smallest products first; the last one has the sum `top`, the others `low`.
+#define SPLIT_PRODUCTS 6
+template <int W_PARTS, int A_PARTS>
+struct SplitOrder {
+    static constexpr int w[SPLIT_PRODUCTS] = {0, 2, 1, 0, 1, 0}, a[SPLIT_PRODUCTS] = {2, 0, 1, 1, 0, 0};
+    static constexpr bool there(int p) { return w[p] < W_PARTS && a[p] < A_PARTS; }
+};
+__device__ __forceinline__ f32x4 mfma_k32(bf16x8 w, bf16x8 a, f32x4 sums) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, a, sums, 0, 0, 0);
+}
+// One 16 x 16 x 32 product; a lane's four sums are those of mfma_k4.
+template <class TW, class TA>
+__device__ __forceinline__ void mfma_split(const Parts<TW>& w, const Parts<TA>& a, f32x4& top, f32x4& low) {
+    typedef SplitOrder<Parts<TW>::COUNT, Parts<TA>::COUNT> order;
+#pragma unroll
+    for (int p = 0; p < SPLIT_PRODUCTS; ++p)
+        if (order::there(p)) {
+            f32x4& sums = p == SPLIT_PRODUCTS - 1 ? top : low;
+            sums = mfma_k32(w.part[order::w[p] % Parts<TW>::COUNT], a.part[order::a[p] % Parts<TA>::COUNT], sums);
+        }
+}
+
+// The sum of one output in plain float32: a chain of fmaf over each stretch of `block` elements of k, the stretches' sums
+// one after another.
+template <class TA, class TW>
+__device__ __forceinline__ float hb_sum_in_order(const TA* a, const TW* w, int K, int block) {
+    float total = 0.f;
+    for (int k0 = 0; k0 < K; k0 += block) {
+        float sum = 0.f;
+#pragma unroll 1
+        for (int k = k0; k < K && k < k0 + block; ++k) sum = fmaf(hb_to_float(w[k]), hb_to_float(a[k]), sum);
+        total += sum;
+    }
+    return total;
+}

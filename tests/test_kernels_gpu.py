@@ -142,6 +142,34 @@ def test_gemm_plain_sums_do_not_depend_on_the_rows(K, wd):
             assert torch.equal(added, base[:rows] + whole[:rows]), rows
 
 
+@pytest.mark.parametrize("M,N,K", [(4, 100, 512), (16, 1000, 1504), (17, 36, 1024), (33, 100, 544), (64, 2050, 2048), (130, 4100, 512), (290, 516, 4656), (700, 2052, 1056)])
+@pytest.mark.parametrize("ad,wd", [(torch.float32, torch.float32), (torch.float32, torch.bfloat16), (torch.bfloat16, torch.float32)])
+def test_gemm_plain_splits_float32_without_loss(M, N, K, ad, wd):
+    """Float32 operands go to the bfloat16 matrix cores in three parts: over magnitudes that differ by e^10 a sum is off
+    from float64 by at most two units in the last place (2^-24 each) for every 32 of a stretch's k, one for every stretch and four for the
+    parts that are left out and the smaller sum. Sums of what is not finite, or rounds to infinity in bfloat16, are plain chains
+    of at most 512 steps."""
+    from herbert_rs_amd.kernels import ops
+    a, w = rand(M, K, seed=31) * torch.exp(2.5 * rand(M, K, seed=32)), rand(N, K, seed=33) * torch.exp(2.5 * rand(N, K, seed=34))
+    a, w = a.to(ad), w.to(wd)
+    c = torch.empty(M, N, device=dev())
+    ops.gemm_plain(a, w, c)
+    want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    units = 2 * min((K + 31) // 32, 16) + (K + 511) // 512 + 4
+    assert bool(((c.double() - want).abs() <= units * 2.0 ** -24 * size).all())
+    # infinities, NaN, a weight that bfloat16 rounds to infinity (halved it is within range, times eight it is not)
+    a[:, 3], a[1, 5], a[2, 7], w[9, 3], w[11, K - 1] = 0.5, math.inf, math.nan, 3.4e38, -math.inf
+    a[0], a[M - 1, 3], w[20] = 0, -8, 1e-30
+    ops.gemm_plain(a, w, c)
+    want = a.double() @ w.double().T
+    as_stored = want.float()
+    assert torch.equal(c.isnan(), as_stored.isnan()) and torch.equal(c.isinf(), as_stored.isinf())
+    assert torch.equal(c[c.isinf()], as_stored[c.isinf()])
+    size = a.double().abs() @ w.double().abs().T
+    fine = as_stored.isfinite()
+    assert bool(((c.double() - want).abs()[fine] <= (units + 512) * 2.0 ** -24 * size[fine]).all())
+
+
 @pytest.mark.parametrize("I", [5, 128, 1000])
 def test_swiglu(I):
     from herbert_rs_amd.kernels import ops
