@@ -13,9 +13,11 @@
 // head's entries of the output. A chunk's values are asked for before its scores are computed and the next chunk's keys after.
 // The sum of a chunk's weights is a fixed tree over the keys' numbers. A chunk that a column does not see leaves
 // it as it was, bit for bit, so a column's result is the same whatever tile it is in.
-// Bound by the chain of a chunk's steps in a workgroup (about 5 us a chunk of heads of 128, 4,096 keys 317); two prompts of 333 and
-// 230 tokens, 16 heads of 128 on 8, take 42 us and a decode step of them 33, where a wave a (token, head) with a
-// key a lane took 712 and 134 (1,681 at 4,096 keys). A tile holds tokens of one sequence: a prompt of 512 tokens beside 15 single
+// Bound by a wave's instructions on a chunk (alone on its SIMD it issues one in four or five cycles): about 2.8 us a chunk of heads of 128, of which the
+// products are one; 4,000 keys take 175 us, two prompts of 333 and 230 tokens, 16 heads of 128 on 8, 34 and a decode step of them 22. A
+// branch an element (a weight only where there is a score, a load only within the head), every wave taking all 64 keys' exponentials, and masks and
+// searches for infinities where nothing is masked cost 307, 41 and 33; two or three groups of four waves that take chunks in turn gained
+// a tenth at 4,000 keys and lost up to a third of a prompt. A tile holds tokens of one sequence: a prompt of 512 tokens beside 15 single
 // tokens at 4,096 keys takes 420 us, and took 2,670 where the next packed tokens were a tile whoever's they were.
 // In xigh/herbert-rs: scores q . k / sqrt(hd), query head h on kv head h / (nq / nkv)
 // (crates/backends/backend_common/src/generic_attention/decode.rs:126), causal by count
@@ -52,7 +54,7 @@ __device__ __forceinline__ Seen seen_by(int pos, int window, int chunk, int keep
 }
 
 // NB: blocks of 16 of the head's entries that a wave owns of the output (the head has up to 64 NB entries). VEC: heads in
-// whole quads, rows aligned, and pages that hold whole chunks. AHEAD: the next chunk's keys and values are in flight
+// whole quads, rows aligned, and pages that hold whole chunks. AHEAD: the next chunk's values are in flight
 // while a chunk is worked on (wide heads have no registers left for that).
 template <class T, class TO, int NB, bool VEC, bool AHEAD>
 __global__ void __launch_bounds__(256)
@@ -67,6 +69,7 @@ attention_plain_kernel(const T* __restrict__ q, const T* __restrict__ k_cache,
     constexpr int DB = 4 * NB;                       // blocks of 16 entries of a head
     constexpr int QLD = 16 * DB + 4, SLD = CHUNK + 4;
     __shared__ __attribute__((aligned(16))) float qs[16 * QLD], ss[16 * SLD];
+    __shared__ float tops[4][16];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r = lane & 15, g4 = lane >> 4;
     const int group = nq / nkv, tiles_a_head = (group + heads_a_tile - 1) / heads_a_tile;
@@ -93,7 +96,6 @@ attention_plain_kernel(const T* __restrict__ q, const T* __restrict__ k_cache,
     f32x4 acc[NB];
 #pragma unroll
     for (int i = 0; i < NB; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    __syncthreads();
 
     const int* pt = page_table + (size_t)slots[seq_of[t0]] * max_pages;
     // what the tile's tokens see together
@@ -102,52 +104,51 @@ attention_plain_kernel(const T* __restrict__ q, const T* __restrict__ k_cache,
         const Seen s = seen_by(positions[t0 + i], window, chunk, keep_first);
         all.lo = min(all.lo, s.lo), all.hi = max(all.hi, s.hi), all.kept = max(all.kept, s.kept);
     }
-    auto next_of = [&](int c) {        // the chunk after c - CHUNK that some token sees
-        return c >= all.kept && c + CHUNK <= all.lo ? all.lo / CHUNK * CHUNK : c;
-    };
+    // the chunks that some token sees: those of the kept keys, then those from the window's (or the sequence's) first key on
+    const int from = all.lo / CHUNK, kept_chunks = min((all.kept + CHUNK - 1) / CHUNK, from);
+    const int count = kept_chunks + (all.hi + CHUNK - 1) / CHUNK - from;
+    auto chunk_at = [&](int i) { return CHUNK * (i < kept_chunks ? i : from + i - kept_chunks); };
     // (keys from all.hi on are the last key once more; a table's entries are pages that exist)
-    f32x4 key[DB], val_next[AHEAD ? NB : 1][4];
+    f32x4 key[DB], val[AHEAD ? NB : 1][4];
     auto fetch_keys = [&](int c, int page) {
         const int j = min(c + 16 * wave + r, all.hi - 1);
         const int in_page = VEC ? c % page_size + j - c : j % page_size;
-        const T* row = k_cache + (((size_t)(VEC ? page : pt[j / page_size]) * nkv + g) * page_size + in_page) * hd + 4 * g4;
+        const T* row = k_cache + (((size_t)(VEC ? page : pt[j / page_size]) * nkv + g) * page_size + in_page) * hd;
 #pragma unroll
-        for (int b = 0; b < DB; ++b) key[b] = load_quad<VEC>(row + 16 * b, hd - 16 * b - 4 * g4);
+        for (int b = 0; b < DB; ++b)
+            key[b] = VEC ? load_quad<true>(row + (16 * b + 4 * g4 < hd ? 16 * b + 4 * g4 : 0), 4) : load_quad<false>(row + 16 * b + 4 * g4, hd - 16 * b - 4 * g4);
     };
     auto fetch_values = [&](int c, int page, int i, f32x4 (&to)[4]) {       // of the wave's i-th block of entries
         const T* at = v_cache + ((size_t)page * nkv + g) * hd * page_size + c % page_size + 4 * g4;
         const int d = 16 * (wave + 4 * i) + r;
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
+            if (VEC) {      // (a page holds a whole chunk; what lies beyond all.hi is made zeros below)
+                to[b] = load_quad<true>(at + (size_t)(d < hd ? d : 0) * page_size + 16 * b, 4);
+                continue;
+            }
             to[b] = f32x4{0.f, 0.f, 0.f, 0.f};
             const int j = c + 16 * b + 4 * g4;
-            if (VEC) {
-                if (d < hd && j < all.hi) to[b] = load_quad<true>(at + (size_t)d * page_size + 16 * b, 4);
-            } else {
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (d < hd && j + e < all.hi)
-                        to[b][e] = hb_to_float(v_cache[(((size_t)pt[(j + e) / page_size] * nkv + g) * hd + d) * page_size + (j + e) % page_size]);
-            }
+            for (int e = 0; e < 4; ++e)
+                if (d < hd && j + e < all.hi)
+                    to[b][e] = hb_to_float(v_cache[(((size_t)pt[(j + e) / page_size] * nkv + g) * hd + d) * page_size + (j + e) % page_size]);
         }
     };
-    int c = next_of(all.kept > 0 ? 0 : all.lo / CHUNK * CHUNK);
-    int following = next_of(c + CHUNK);
-    // (the page after the next is looked up a chunk before its loads are asked for)
-    int page = pt[c / page_size], page_next = following < all.hi ? pt[following / page_size] : 0;
-    fetch_keys(c, page);
+    // (the page after the next is looked up a chunk before its loads are asked for; beyond the last chunk the last once more)
+    auto page_at = [&](int i) { return pt[chunk_at(min(i, count - 1)) / page_size]; };
+    int page = page_at(0), page_next = page_at(1);
+    fetch_keys(chunk_at(0), page);
     if (AHEAD) {
 #pragma unroll
-        for (int i = 0; i < NB; ++i) fetch_values(c, page, i, val_next[i]);
+        for (int i = 0; i < NB; ++i) fetch_values(chunk_at(0), page, i, val[i]);
     }
-    while (c < all.hi) {
-        f32x4 val[AHEAD ? NB : 1][4];
-        if (AHEAD) {
+    __syncthreads();
+    for (int at = 0; at < count; ++at) {
+        const int c = chunk_at(at), following = chunk_at(min(at + 1, count - 1));
+        if (VEC && hd < 16 * DB)
 #pragma unroll
-            for (int i = 0; i < NB; ++i)
-#pragma unroll
-                for (int b = 0; b < 4; ++b) val[i][b] = val_next[i][b];
-        }
+            for (int b = 0; b < DB; ++b) key[b] = 16 * b + 4 * g4 < hd ? key[b] : f32x4{0.f, 0.f, 0.f, 0.f};
         f32x4 dots = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int b = 0; b < DB; ++b) {
@@ -156,48 +157,44 @@ attention_plain_kernel(const T* __restrict__ q, const T* __restrict__ k_cache,
 #pragma unroll
             for (int s = 0; s < 4; ++s) dots = mfma_k4(key[b][s], qq[s], dots);
         }
-        const int after = next_of(following + CHUNK);
-        const int page_after = after < all.hi ? pt[after / page_size] : 0;
-        if (AHEAD && following < all.hi) {
-            fetch_keys(following, page_next);
+        const int page_after = page_at(at + 2);
+        if (AHEAD) fetch_keys(following, page_next);
+        dots *= scale;
+        if (softcap > 0.f)
 #pragma unroll
-            for (int i = 0; i < NB; ++i) fetch_values(following, page_next, i, val_next[i]);
-        }
-        __syncthreads();                              // (the chunk before has been read)
+            for (int e = 0; e < 4; ++e) dots[e] = softcap * tanhf(dots[e] / softcap);
+        if (bias)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int n = max(0, min(pos - (c + 16 * wave + 4 * g4 + e), bias_len - 1));
+                dots[e] += bias[(size_t)h * bias_ld + bias_at + bias_len - 1 - n];
+            }
+        const bool sees = mine && ((c < see.hi && c + CHUNK > see.lo) || c < see.kept);
+        float top = -INFINITY;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int j = c + 16 * wave + 4 * g4 + e;
-            float s = dots[e] * scale;
-            if (softcap > 0.f) s = softcap * tanhf(s / softcap);
-            if (bias) {
-                const int n = max(0, min(pos - j, bias_len - 1));
-                s += bias[(size_t)h * bias_ld + bias_at + bias_len - 1 - n];
-            }
-            const bool valid = mine && (j >= see.lo || j < see.kept) && j < see.hi;
-            ss[r * SLD + 16 * wave + 4 * e + g4] = valid ? s : -INFINITY;
-        }
-        __syncthreads();
-        // this lane's share of its column: keys 16 b + 4 s + g4
-        f32x4 p[4];
-        float top = -INFINITY;
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            p[b] = *(const f32x4*)&ss[r * SLD + 16 * b + 4 * g4];
-            top = fmaxf(top, fmaxf(fmaxf(p[b][0], p[b][1]), fmaxf(p[b][2], p[b][3])));
+            dots[e] = sees && (j >= see.lo || j < see.kept) && j < see.hi ? dots[e] : -INFINITY;
+            top = fmaxf(top, dots[e]);
         }
         top = fmaxf(top, __shfl_xor(top, 16, HB_WAVE));
         top = fmaxf(top, __shfl_xor(top, 32, HB_WAVE));
-        const bool sees = mine && ((c < see.hi && c + CHUNK > see.lo) || c < see.kept);
-        float corr = 1.0f;
-        if (sees) {
-            const float m_new = fmaxf(m, top);
-            corr = expf(m - m_new);
-            m = m_new;
+        if (g4 == 0) tops[wave][r] = top;
+        hb_workgroup_barrier();                       // (and the weights of the chunk before have been read)
+        const float m_new = fmaxf(m, fmaxf(fmaxf(tops[0][r], tops[1][r]), fmaxf(tops[2][r], tops[3][r])));
+        const float corr = expf(sees ? m - m_new : 0.f);
+        m = m_new;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {                 // (the exponential in any case: no branch an element)
+            const bool there = dots[e] != -INFINITY;
+            const float weight = expf(there ? dots[e] - m_new : 0.f);
+            ss[r * SLD + 16 * wave + 4 * e + g4] = there ? weight : 0.f;
         }
+        hb_workgroup_barrier();
+        // this lane's share of its column: keys 16 b + 4 s + g4
+        f32x4 p[4];
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
-#pragma unroll
-            for (int s = 0; s < 4; ++s) p[b][s] = sees && p[b][s] != -INFINITY ? expf(p[b][s] - m) : 0.f;
+        for (int b = 0; b < 4; ++b) p[b] = *(const f32x4*)&ss[r * SLD + 16 * b + 4 * g4];
         // the tree: key j with j ^ 32, j ^ 16 (blocks), j ^ 8, j ^ 4 (quads), j ^ 2, j ^ 1 (lanes)
         f32x4 t = (p[0] + p[2]) + (p[1] + p[3]);
         float sum = (t[0] + t[2]) + (t[1] + t[3]);
@@ -211,41 +208,43 @@ attention_plain_kernel(const T* __restrict__ q, const T* __restrict__ k_cache,
             if (!AHEAD) fetch_values(c, page, i, v);
             // a value without a finite size, perhaps of a key that some column does not see: a weight of zero does
             // not hide it
-            bool wild = false;
+            if (VEC && (c + CHUNK > all.hi || hd < 16 * DB))
+#pragma unroll
+                for (int b = 0; b < 4; ++b)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[b][e] = 16 * (wave + 4 * i) + r < hd && c + 16 * b + 4 * g4 + e < all.hi ? v[b][e] : 0.f;
+            f32x4 nothing = {0.f, 0.f, 0.f, 0.f};     // (or NaN)
 #pragma unroll
             for (int b = 0; b < 4; ++b)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    if (VEC && c + 16 * b + 4 * g4 + e >= all.hi) v[b][e] = 0.f;
-                    wild |= !(fabsf(v[b][e]) <= 3.4028235e38f);
-                }
-            if (!__any(wild)) {
+                for (int e = 0; e < 4; ++e) nothing[b] = fmaf(v[b][e], 0.f, nothing[b]);
+            if (!__any(!((nothing[0] + nothing[1]) + (nothing[2] + nothing[3]) == 0.f))) {
 #pragma unroll
                 for (int b = 0; b < 4; ++b) {
                     transpose_quads(v[b]);
 #pragma unroll
                     for (int s = 0; s < 4; ++s) acc[i] = mfma_k4(v[b][s], p[b][s], acc[i]);
                 }
-                continue;
-            }
+            } else {
 #pragma unroll
-            for (int b = 0; b < 4; ++b)
-                for (int s = 0; s < 4; ++s)
-                    for (int k = 0; k < 4; ++k) {
-                        const int j = c + 16 * b + 4 * s + k;
-                        const float w = __shfl(s == 0 ? p[b][0] : s == 1 ? p[b][1] : s == 2 ? p[b][2] : p[b][3], 16 * k + r, HB_WAVE);
-                        if (j >= all.hi) continue;
-                        const T* v = v_cache + ((size_t)pt[j / page_size] * nkv + g) * hd * page_size + j % page_size;
-                        const bool valid = mine && (j >= see.lo || j < see.kept) && j < see.hi;
+                for (int b = 0; b < 4; ++b)
+                    for (int s = 0; s < 4; ++s)
+                        for (int k = 0; k < 4; ++k) {
+                            const int j = c + 16 * b + 4 * s + k;
+                            const float w = __shfl(s == 0 ? p[b][0] : s == 1 ? p[b][1] : s == 2 ? p[b][2] : p[b][3], 16 * k + r, HB_WAVE);
+                            if (j >= all.hi) continue;
+                            const T* v = v_cache + ((size_t)pt[j / page_size] * nkv + g) * hd * page_size + j % page_size;
+                            const bool valid = mine && (j >= see.lo || j < see.kept) && j < see.hi;
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            const int d = 16 * (wave + 4 * i) + 4 * g4 + e;
-                            if (valid && d < hd) acc[i][e] = fmaf(w, hb_to_float(v[(size_t)d * page_size]), acc[i][e]);
+                            for (int e = 0; e < 4; ++e) {
+                                const int d = 16 * (wave + 4 * i) + 4 * g4 + e;
+                                if (valid && d < hd) acc[i][e] = fmaf(w, hb_to_float(v[(size_t)d * page_size]), acc[i][e]);
+                            }
                         }
-                    }
+            }
+            if (AHEAD) fetch_values(following, page_next, i, v);
         }
-        if (!AHEAD && following < all.hi) fetch_keys(following, page_next);
-        c = following, following = after;
+        if (!AHEAD && at + 1 < count) fetch_keys(following, page_next);
         page = page_next, page_next = page_after;
     }
     if (!mine) return;
@@ -291,7 +290,7 @@ extern "C" int hb_attention_plain(const void* q, const void* k_cache, const void
     const int size = dtype == HB_F32 ? 4 : 2;
     const bool vec = hd % 4 == 0 && page_size % CHUNK == 0 && (uintptr_t)k_cache % (4 * size) == 0 && (uintptr_t)v_cache % (4 * size) == 0;
 #define HB_ATTENTION(TT, TO, NB, VEC)                                                                                 \
-    attention_plain_kernel<TT, TO, NB, VEC, (NB <= 2 && VEC)><<<grid, 256, 0, stream>>>(                                                \
+    attention_plain_kernel<TT, TO, NB, VEC, (NB <= 2 && VEC)><<<grid, 256, 0, stream>>>(                              \
         (const TT*)q, (const TT*)k_cache, (const TT*)v_cache, (TO*)out, positions, seq_of, slots, page_table, max_pages, \
         page_size, nq, nkv, hd, scale, window, sinks, chunk, softcap, bias, bias_ld, bias_at, bias_len, keep_first,    \
         heads_a_tile, (const int2*)tiles)
