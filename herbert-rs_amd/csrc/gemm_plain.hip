@@ -17,8 +17,7 @@
 
 HB_MODULE_ERROR_SLOT()
 
-// Elements of k that are summed as one chain; a multiple of every kernel's stage.
-#define K_BLOCK 512
+#define K_BLOCK SPLIT_STRETCH
 
 // What a product may do to a sum before it stores it: nothing (rate null), or turn the pre-activation of a
 // decay into the decay itself, exp(-exp(rate[n / D]) * softplus(sum + bias[n])) for column n (float32; the
@@ -241,7 +240,6 @@ gemm_plain_tile_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
 // some pieces ahead, and splits both in registers. The stretches' sums meet in LDS, where a thread an output adds them in
 // their order.
 #define WAVE_WAVES 8
-#define WAVE_DEPTH 4
 template <class TA, class TW, class TC, bool ACCUM, int MB, int NB, int AHEAD>
 __global__ void __launch_bounds__(WAVE_WAVES * HB_WAVE, AHEAD == 8 ? 4 : 2)
 gemm_plain_wave_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* __restrict__ C, int M, int N,
@@ -250,7 +248,7 @@ gemm_plain_wave_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
     A += blockIdx.z * batch_a;
     W += blockIdx.z * batch_w;
     C += blockIdx.z * batch_c;
-    constexpr int UNITS = K_BLOCK / 32, A_AHEAD = NB > 1 ? 4 : AHEAD == UNITS ? 8 : 2;
+    constexpr int A_AHEAD = NB > 1 ? 4 : AHEAD == 16 ? 8 : 2;
     __shared__ __attribute__((aligned(16))) f32x4 sums[WAVE_WAVES][NB][MB][HB_WAVE];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
     const int r = lane & 15, q = lane >> 4;
@@ -273,67 +271,7 @@ gemm_plain_wave_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
         for (int j = 0; j < NB; ++j)
 #pragma unroll
             for (int i = 0; i < MB; ++i) top[j][i] = low[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (k0 + K_BLOCK <= K) {
-            Oct<TW> w[AHEAD][NB];
-            Oct<TA> a[A_AHEAD][MB];
-            auto fetch_w = [&](int u) {
-#pragma unroll
-                for (int j = 0; j < NB; ++j) w[u % AHEAD][j] = load_oct(w_row[j] + k0 + 32 * u, 8u * q);
-            };
-            auto fetch_a = [&](int u) {
-#pragma unroll
-                for (int i = 0; i < MB; ++i) a[u % A_AHEAD][i] = load_oct(a_row[i] + k0 + 32 * u, 8u * q);
-            };
-#pragma unroll
-            for (int u = 0; u < A_AHEAD; ++u) fetch_a(u);
-#pragma unroll
-            for (int u = 0; u < AHEAD; ++u) fetch_w(u);
-            __builtin_amdgcn_sched_barrier(0);       // (no load waits for the sums before it)
-#pragma unroll
-            for (int u = 0; u < UNITS; ++u) {
-                Parts<TW> w_parts[NB];
-#pragma unroll
-                for (int j = 0; j < NB; ++j) w_parts[j] = split(w[u % AHEAD][j]);
-                if (u + AHEAD < UNITS) fetch_w(u + AHEAD);
-#pragma unroll
-                for (int i = 0; i < MB; ++i) {
-                    const Parts<TA> a_parts = split(a[u % A_AHEAD][i]);
-#pragma unroll
-                    for (int j = 0; j < NB; ++j) mfma_split<TW, TA>(w_parts[j], a_parts, top[j][i], low[j][i]);
-                }
-                if (u + A_AHEAD < UNITS) fetch_a(u + A_AHEAD);
-            }
-        } else {
-            for (int k = k0; k < K; k += 32 * WAVE_DEPTH) {      // (what is left of k)
-                Oct<TW> w[WAVE_DEPTH][NB];
-                Oct<TA> a[WAVE_DEPTH][MB];
-#pragma unroll
-                for (int d = 0; d < WAVE_DEPTH; ++d) {
-#pragma unroll
-                    for (int j = 0; j < NB; ++j) w[d][j] = load_oct<true>(w_row[j], k + 32 * d + 8 * q, K);
-#pragma unroll
-                    for (int i = 0; i < MB; ++i) a[d][i] = load_oct<true>(a_row[i], k + 32 * d + 8 * q, K);
-                }
-#pragma unroll
-                for (int d = 0; d < WAVE_DEPTH; ++d) {
-                    const int left = K - k - 32 * d;
-                    if (left <= 0) break;
-                    Parts<TW> w_parts[NB];
-#pragma unroll
-                    for (int j = 0; j < NB; ++j) {
-                        if (left < 32) ends(w[d][j], left - 8 * q);
-                        w_parts[j] = split(w[d][j]);
-                    }
-#pragma unroll
-                    for (int i = 0; i < MB; ++i) {
-                        if (left < 32) ends(a[d][i], left - 8 * q);
-                        const Parts<TA> a_parts = split(a[d][i]);
-#pragma unroll
-                        for (int j = 0; j < NB; ++j) mfma_split<TW, TA>(w_parts[j], a_parts, top[j][i], low[j][i]);
-                    }
-                }
-            }
-        }
+        sum_stretch<AHEAD, A_AHEAD>(w_row, a_row, k0, K, q, top, low);
         if (first) __syncthreads();                  // (the round before has been read)
 #pragma unroll
         for (int j = 0; j < NB; ++j)

@@ -122,3 +122,77 @@ __device__ __forceinline__ float hb_sum_in_order(const TA* a, const TW* w, int K
     }
     return total;
 }
+
+// Elements of k that are summed from zero; a multiple of every kernel's stage.
+#define SPLIT_STRETCH 512
+// Pieces of 32 k that are asked for at once where a stretch is not whole.
+#define WAVE_DEPTH 4
+
+// A wave's sums over the stretch of k that starts at k0, for NB blocks of 16 rows of W and MB of A (w_row, a_row: the lane's own rows,
+// 16 bytes at a time; q = lane / 16). AHEAD pieces of 32 k of W and A_AHEAD of A are in flight.
+template <int AHEAD, int A_AHEAD, class TW, class TA, int NB, int MB>
+__device__ __forceinline__ void sum_stretch(const TW* const (&w_row)[NB], const TA* const (&a_row)[MB], int k0, int K, int q,
+                                            f32x4 (&top)[NB][MB], f32x4 (&low)[NB][MB]) {
+    constexpr int UNITS = SPLIT_STRETCH / 32;
+    if (k0 + SPLIT_STRETCH <= K) {
+        Oct<TW> w[AHEAD][NB];
+        Oct<TA> a[A_AHEAD][MB];
+        auto fetch_w = [&](int u) {
+#pragma unroll
+            for (int j = 0; j < NB; ++j) w[u % AHEAD][j] = load_oct(w_row[j] + k0 + 32 * u, 8u * q);
+        };
+        auto fetch_a = [&](int u) {
+#pragma unroll
+            for (int i = 0; i < MB; ++i) a[u % A_AHEAD][i] = load_oct(a_row[i] + k0 + 32 * u, 8u * q);
+        };
+#pragma unroll
+        for (int u = 0; u < A_AHEAD; ++u) fetch_a(u);
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) fetch_w(u);
+        __builtin_amdgcn_sched_barrier(0);           // (no load waits for the sums before it)
+#pragma unroll
+        for (int u = 0; u < UNITS; ++u) {
+            Parts<TW> w_parts[NB];
+#pragma unroll
+            for (int j = 0; j < NB; ++j) w_parts[j] = split(w[u % AHEAD][j]);
+            if (u + AHEAD < UNITS) fetch_w(u + AHEAD);
+#pragma unroll
+            for (int i = 0; i < MB; ++i) {
+                const Parts<TA> a_parts = split(a[u % A_AHEAD][i]);
+#pragma unroll
+                for (int j = 0; j < NB; ++j) mfma_split<TW, TA>(w_parts[j], a_parts, top[j][i], low[j][i]);
+            }
+            if (u + A_AHEAD < UNITS) fetch_a(u + A_AHEAD);
+        }
+        return;
+    }
+    for (int k = k0; k < K; k += 32 * WAVE_DEPTH) {          // (what is left of k)
+        Oct<TW> w[WAVE_DEPTH][NB];
+        Oct<TA> a[WAVE_DEPTH][MB];
+#pragma unroll
+        for (int d = 0; d < WAVE_DEPTH; ++d) {
+#pragma unroll
+            for (int j = 0; j < NB; ++j) w[d][j] = load_oct<true>(w_row[j], k + 32 * d + 8 * q, K);
+#pragma unroll
+            for (int i = 0; i < MB; ++i) a[d][i] = load_oct<true>(a_row[i], k + 32 * d + 8 * q, K);
+        }
+#pragma unroll
+        for (int d = 0; d < WAVE_DEPTH; ++d) {
+            const int left = K - k - 32 * d;
+            if (left <= 0) break;
+            Parts<TW> w_parts[NB];
+#pragma unroll
+            for (int j = 0; j < NB; ++j) {
+                if (left < 32) ends(w[d][j], left - 8 * q);
+                w_parts[j] = split(w[d][j]);
+            }
+#pragma unroll
+            for (int i = 0; i < MB; ++i) {
+                if (left < 32) ends(a[d][i], left - 8 * q);
+                const Parts<TA> a_parts = split(a[d][i]);
+#pragma unroll
+                for (int j = 0; j < NB; ++j) mfma_split<TW, TA>(w_parts[j], a_parts, top[j][i], low[j][i]);
+            }
+        }
+    }
+}

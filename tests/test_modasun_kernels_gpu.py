@@ -364,6 +364,35 @@ def test_experts_products_and_the_shared_experts_gated_sum():
         assert torch.allclose(x.cpu(), want, atol=tol, rtol=tol), f"{dtype}"
 
 
+@pytest.mark.parametrize("T,E,top,N,K", [(1, 8, 2, 33, 512), (5, 4, 3, 96, 1536), (17, 1, 1, 70, 2048), (40, 3, 1, 64, 100), (150, 2, 2, 36, 5004), (9, 4, 2, 40, 30)])
+@pytest.mark.parametrize("wd", [torch.float32, torch.bfloat16])
+def test_products_of_experts_in_float32(T, E, top, N, K, wd):
+    """Tiles of one to 64 rows of an expert, gathered or not, whole stretches of k, parts of them, and rows off 16-byte borders (the
+    kernel of vector products): off from float64 by at most a rounding of every step of a chain (a stretch's 512 where split
+    products are summed: fewer), and a token's row the same bits whoever else is in the step."""
+    rows, bias = rand(T, E, seed=41), rand(E, seed=42)
+    a, w = rand(T, K, seed=43).to(DEV), rand(E, N, K, seed=44).to(wd).to(DEV)
+
+    def both(n):
+        routing = moe.Routing(torch.empty(moe.Routing.ints_needed(n, E, top), dtype=torch.int32, device=DEV),
+                              torch.empty(n, top, device=DEV), n, E, top)
+        moe.route(rows[:n].contiguous().to(DEV), bias.to(DEV), routing)
+        order, chosen = routing.order.cpu().tolist(), routing.chosen.cpu().tolist()
+        c, d = (torch.full((n * top, N), math.nan, device=DEV) for _ in range(2))
+        moe.gemm_plain(a[:n].contiguous(), w, c, routing, gather=True)
+        moe.gemm_plain(a[[p // top for p in order]].contiguous(), w, d, routing, gather=False)
+        assert torch.equal(c, d)
+        return c, order, chosen
+    c, order, chosen = both(T)
+    steps = min(K, 512) + (K + 511) // 512 if K % 4 == 0 else K
+    for i, p in enumerate(order):
+        x, m = a[p // top].double(), w[chosen[p]].double()
+        assert bool(((c[i].double() - m @ x).abs() <= steps * 2.0 ** -24 * (m.abs() @ x.abs())).all()), i
+    alone, order1, _ = both(1)
+    for i, p in enumerate(order1):
+        assert torch.equal(alone[i], c[order.index(p)])
+
+
 # ---------------------------------------------------------------- the second product of a pair through a narrow middle
 @pytest.mark.parametrize("M,N,K,col0,ld", [(1, 128, 32, 0, 32), (8, 2048, 128, 260, 400), (32, 48, 64, 4, 72), (7, 50, 96, 8, 104),
                                            (33, 64, 32, 0, 32), (5, 40, 24, 0, 24), (6, 32, 32, 3, 40)])
