@@ -171,6 +171,7 @@ class Cache:
         self.pad_slot = self.n_slots        # never handed out: where a step's padding rows write and read
         self.slots = FreeList(self.n_slots, "slot")
         self.lengths = np.zeros(self.n_slots, dtype=np.int64)
+        self._taken = set()      # slots taken whose state is still to be cleared
         self._saved_slots = (None, None)    # the slots that save_state was last asked for and the stream, and their numbers on the GPU
         self.kv_groups = {}
         self.state_groups = {}
@@ -221,11 +222,34 @@ class Cache:
 
     # ---- slots
     def alloc_slot(self):
+        """A free slot, of length 0 and with fixed-size state of zeros. (The state is cleared before anything reads it, with
+        that of all other slots taken meanwhile: see `clear_taken`.)"""
         slot = self.slots.take()
         self.lengths[slot] = 0
-        for g in self.state_groups.values():
-            g.clear_slot(slot)
+        if self.state_groups:
+            self._taken.add(slot)
         return slot
+
+    def clear_taken(self):
+        """Clear the state of the slots that were taken since the last call. Whoever is to read or write state calls it."""
+        if self._taken:
+            taken, self._taken = self._taken, set()
+            self.clear_slots(taken)
+
+    def clear_slots(self, slots):
+        """Fixed-size state of `slots` made zeros, a kernel a group however many they are."""
+        if not self.state_groups or not slots:
+            return
+        slots = sorted(int(s) for s in slots)
+        first, behind = slots[0], slots[-1] + 1
+        groups = list(self.state_groups.values())
+        if behind - first == len(slots):
+            for g in groups:
+                g.data[:, first:behind].zero_()
+            return
+        at = send(np.array(slots, dtype=np.int64), groups[0].data.device)
+        for g in groups:
+            g.data.index_fill_(1, at, 0)
 
     def free_slot(self, slot):
         self.slots.give_back(slot)
@@ -273,6 +297,7 @@ class Cache:
         `restore_state` puts back when the step that was to change it has failed."""
         if not self.state_groups:
             return None
+        self.clear_taken()
         index = sorted(set(int(s) for s in slots))
         device = next(iter(self.state_groups.values())).data.device
         # (decode steps name the same slots again and again. Their numbers serve the stream that they were sent on: another one
@@ -326,6 +351,7 @@ class Cache:
         return self._kv_of[entry].view(entry)
 
     def state_views(self, entry):
+        self.clear_taken()
         return [g.view(entry) for g in self._state_of.get(entry, [])]
 
     def check(self):

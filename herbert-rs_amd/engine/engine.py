@@ -218,15 +218,23 @@ class Engine:
             starts.append(start)
         # all pages of the step or none: a step that does not fit leaves the cache as it was
         self.cache.reserve_all([(e.slot, len(e.tokens)) for e in entries])
-        # fixed-size state is changed in place by the parts: what the step's slots hold is set aside
-        # first, so that a step that fails leaves them as they were (nothing for a cache without state)
-        state_before = self.cache.save_state([e.slot for e in entries])
+        # fixed-size state is changed in place by the parts: what the step's slots hold is set aside before parts run one after
+        # another, so that a step that fails leaves them as they were (a graph's replay begins as a whole or not at all; a sequence's
+        # first step found zeros; nothing for a cache without state)
+        self.cache.clear_taken()
+        state_before = []
+
+        def set_aside():
+            held = [e.slot for e, start in zip(entries, starts) if start]
+            if held and not state_before:
+                state_before.extend(self.cache.save_state(held) or ())
         try:
             if self.static_decode and all(len(e.tokens) == 1 and list(e.want) == [0] for e in entries):
-                logits = self._decode_step(entries, starts, tokens_on_device)
+                logits = self._decode_step(entries, starts, tokens_on_device, set_aside)
                 if keep_logits:
                     logits = logits.clone()
             else:
+                set_aside()
                 meta = batching.pack(entries, starts, self.device)
                 if tokens_on_device is not None:
                     meta.token_ids.copy_(tokens_on_device)
@@ -235,13 +243,14 @@ class Engine:
             for e in entries:       # nothing was committed: give back what was taken for the step
                 self.cache.unreserve(e.slot)
             self.cache.restore_state(state_before)
+            self.cache.clear_slots([e.slot for e, start in zip(entries, starts) if start == 0])
             raise
         for e in entries:
             self.cache.commit(e.slot, len(e.tokens))
         self.steps_run += 1
         return logits
 
-    def _decode_step(self, entries, starts, tokens_on_device=None):
+    def _decode_step(self, entries, starts, tokens_on_device, set_aside):
         """One token for each sequence, every logit wanted: the launch-bound case. The step's
         metadata lives in fixed buffers, and the forward pass of a shape is recorded into a HIP graph
         that is replayed from then on, so that the host launches one graph and not hundreds of
@@ -253,7 +262,8 @@ class Engine:
         deals its grid out by a list). All graphs write their logits into the first rows of the
         engine's one buffer; what is returned here is a view of those rows, which the next decode
         step writes again (`step` copies it for callers that keep it). At most MAX_GRAPHS graphs and
-        MAX_DECODE_BATCH_SIZES batch sizes are kept, the least recently used go first."""
+        MAX_DECODE_BATCH_SIZES batch sizes are kept, the least recently used go first. `set_aside` is called before
+        anything runs outside a graph that exists already."""
         n = len(entries)
         B = decode_batch_bucket(n)          # the step runs at this size, the rows beyond n are padding
         state = self._decode.get(B)
@@ -279,6 +289,7 @@ class Engine:
         if tokens_on_device is not None:
             meta.token_ids[:n].copy_(tokens_on_device)      # behind the copy from the host, before the graph
         if not self.use_graphs:
+            set_aside()
             return self.model.forward(self.rt, meta, self.cache, logits_out=state.logits)[:n]
         key = (B, meta.context_bucket, meta.unequal)
         graph = self._graphs.get(key)
@@ -286,6 +297,7 @@ class Engine:
             self._graphs.move_to_end(key)
             graph.replay()
             return state.logits[:n]
+        set_aside()
         if B > self._sized_rows:
             # no step this large has run yet: it runs as it is, which also sizes every scratch buffer
             self._sized_rows = B

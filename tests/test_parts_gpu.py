@@ -501,6 +501,42 @@ def test_a_step_that_fails_leaves_the_state_as_it_was():
     assert torch.equal(run(True), run(False))
 
 
+def test_slots_that_come_back_start_from_zeros_whichever_they_are():
+    """Slots are cleared together, before their state is first read: neighbours, slots with others between them and one alone
+    give what a fresh cache gives, also after a first step that failed."""
+    from herbert_rs_amd.weights import random_tensors
+    from herbert_rs_amd.engine.model import Model
+    spec = toy_spec()
+    w = random_tensors(Model(spec).tensor_needs(), 3, "float32", std=0.15, norm_std=0.1)
+    seqs = [[5, 9, 33, 2, 41], [7, 3, 50, 1], [11, 12], [4]]
+
+    def step(engine, slots, seqs):
+        return engine.step([StepEntry(s, t, [len(t) - 1]) for s, t in zip(slots, seqs)]).cpu()
+    fresh = Engine(None, spec, w, dtype="float32", max_tokens=512)
+    want = step(fresh, [fresh.alloc_slot() for _ in seqs], seqs)
+    engine = Engine(None, spec, w, dtype="float32", max_tokens=512)
+    slots = [engine.alloc_slot() for _ in seqs]
+    assert torch.equal(step(engine, slots, seqs), want)
+    for back in ([0, 1, 2, 3], [0, 2], [1], [1, 3]):
+        for i in back:
+            engine.free_slot(slots[i])
+        for i in back:
+            slots[i] = engine.alloc_slot()
+        mixer = engine.model.blocks[0].mixer
+        real = mixer.forward
+
+        def failing(ctx, y, x):
+            real(ctx, y, x)
+            raise RuntimeError("after the state has changed")
+        mixer.forward = failing
+        with pytest.raises(RuntimeError, match="has changed"):
+            step(engine, [slots[i] for i in back], [seqs[i] for i in back])
+        mixer.forward = real
+        for g in engine.cache.state_groups.values():
+            assert not g.data[:, [slots[i] for i in back]].any()
+        assert torch.allclose(step(engine, [slots[i] for i in back], [seqs[i] for i in back]), want[back], rtol=1e-5, atol=1e-5)
+
+
 @register("mixer", "toy_decay_on_the_gpu")
 class ToyDecayOnTheGpu(ToyDecayMixer):
     """The same recurrence, but a step in which every sequence brings one token does GPU work only:
