@@ -231,7 +231,8 @@ class Cache:
         return slot
 
     def clear_taken(self):
-        """Clear the state of the slots that were taken since the last call. Whoever is to read or write state calls it."""
+        """Clear the state of the slots that were taken since the last call. Whoever is to read or write state calls it, and
+        so does whoever makes room for a step: views of the state may be held from before."""
         if self._taken:
             taken, self._taken = self._taken, set()
             self.clear_slots(taken)
@@ -265,6 +266,7 @@ class Cache:
     # ---- one step
     def reserve(self, slot, new_tokens):
         """Make room for `new_tokens` more positions of a slot (before the step runs)."""
+        self.clear_taken()
         new_length = self.length(slot) + int(new_tokens)
         if new_length > self.max_positions:
             raise CacheError(f"slot {slot}: {new_length} positions exceed the model's "
@@ -277,6 +279,7 @@ class Cache:
         """`reserve` for every (slot, new tokens) of a step, all or nothing: the pages that each
         group needs are counted first, and a step that does not fit raises CacheError with the
         cache unchanged."""
+        self.clear_taken()
         targets = []
         for slot, new_tokens in wanted:
             new_length = self.length(slot) + int(new_tokens)

@@ -221,7 +221,6 @@ class Engine:
         # fixed-size state is changed in place by the parts: what the step's slots hold is set aside before parts run one after
         # another, so that a step that fails leaves them as they were (a graph's replay begins as a whole or not at all; a sequence's
         # first step found zeros; nothing for a cache without state)
-        self.cache.clear_taken()
         state_before = []
 
         def set_aside():
