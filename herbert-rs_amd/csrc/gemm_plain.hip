@@ -474,14 +474,8 @@ static void launch(const void* A, const void* W, void* C, int M, int N, int K, i
 // It pays up to 8 rows and, where k is long, up to 24; the line at 32 rows (few_rows_takes) is older than the two others.
 #define FEW_ROWS_M 8
 #define FEW_ROWS_K 1024
-__global__ void __launch_bounds__(HB_WAVE)
-gemm_few_rows_kernel(const float* __restrict__ A, const bf16* __restrict__ W, float* __restrict__ C, int M, int N,
-                     int K, int lda, int ldw, int ldc, DecayEpilogue ep, size_t batch_a = 0, size_t batch_w = 0,
-                     size_t batch_c = 0) {
-    // (blockIdx.z: one of a batch of products whose operands lie batch_* elements apart)
-    A += blockIdx.z * batch_a;
-    W += blockIdx.z * batch_w;
-    C += blockIdx.z * batch_c;
+__device__ __forceinline__ void few_rows_product(const float* __restrict__ A, const bf16* __restrict__ W, float* __restrict__ C, int M,
+                                                 int N, int K, int lda, int ldw, int ldc, const DecayEpilogue& ep) {
     __shared__ __attribute__((aligned(16))) float rows_of_a[FEW_ROWS_M * FEW_ROWS_K];
     const int lane = threadIdx.x;
     const int n = blockIdx.x * 16 + lane / 4;
@@ -533,6 +527,28 @@ gemm_few_rows_kernel(const float* __restrict__ A, const bf16* __restrict__ W, fl
         const int i = 4 * j + part;
         if (n < N && i < rows) C[(size_t)(m0 + i) * ldc + n] = ep.rate ? decay_of(ep, s, n) : s;
     }
+}
+
+__global__ void __launch_bounds__(HB_WAVE)
+gemm_few_rows_kernel(const float* __restrict__ A, const bf16* __restrict__ W, float* __restrict__ C, int M, int N,
+                     int K, int lda, int ldw, int ldc, DecayEpilogue ep, size_t batch_a = 0, size_t batch_w = 0,
+                     size_t batch_c = 0) {
+    // (blockIdx.z: one of a batch of products whose operands lie batch_* elements apart)
+    few_rows_product(A + blockIdx.z * batch_a, W + blockIdx.z * batch_w, C + blockIdx.z * batch_c, M, N, K, lda, ldw, ldc, ep);
+}
+
+// Two products of one shape that wait for the same rows and not for each other (a gate's and a decay's through their narrow middles): one
+// launch instead of two of 5 to 7 us each, of which their own work is the smaller part.
+struct FewRowsProduct {
+    const float* A;
+    const bf16* W;
+    float* C;
+    DecayEpilogue ep;
+};
+__global__ void __launch_bounds__(HB_WAVE)
+gemm_few_rows_pair_kernel(FewRowsProduct first, FewRowsProduct second, int M, int N, int K, int lda, int ldw, int ldc) {
+    const FewRowsProduct p = blockIdx.z ? second : first;
+    few_rows_product(p.A, p.W, p.C, M, N, K, lda, ldw, ldc, p.ep);
 }
 
 static bool few_rows_takes(const void* A, int a_dtype, const void* W, int w_dtype, int c_dtype, int M, int K, int lda,
@@ -595,6 +611,24 @@ extern "C" int hb_gemm_plain_short_k(const void* A, int a_dtype, const void* W, 
     }
     HB_CHECK_LAUNCH("gemm_plain");
     return 0;
+}
+
+// Two such products of float32 rows with float32 sums (no decay for the first): C0 = A0 W0^T, C1 = A1 W1^T, shapes and strides alike.
+extern "C" int hb_gemm_plain_short_k_pair(const float* A0, const void* W0, float* C0, const float* A1, const void* W1, float* C1,
+                                          int w_dtype, int M, int N, int K, int lda, int ldw, int ldc, const float* A_log,
+                                          const float* dt_bias, int D, float root, hipStream_t stream) {
+    HB_REQUIRE(M > 0 && N > 0 && K > 0, "gemm: empty problem (M=%d, N=%d, K=%d)", M, N, K);
+    if (few_rows_takes(A0, 0, W0, w_dtype, 0, M, K, lda, ldw, 0) && few_rows_takes(A1, 0, W1, w_dtype, 0, M, K, lda, ldw, 0) &&
+        (A_log == nullptr) == (dt_bias == nullptr) && (!A_log || (D > 0 && N % D == 0)) && lda >= K && ldw >= K && ldc >= N) {
+        const FewRowsProduct first{A0, (const bf16*)W0, C0, DecayEpilogue{nullptr, nullptr, 1, 0.f}};
+        const FewRowsProduct second{A1, (const bf16*)W1, C1, DecayEpilogue{A_log, dt_bias, A_log ? D : 1, root}};
+        gemm_few_rows_pair_kernel<<<dim3((N + 15) / 16, (M + FEW_ROWS_M - 1) / FEW_ROWS_M, 2), HB_WAVE, 0, stream>>>(
+            first, second, M, N, K, lda, ldw, ldc);
+        HB_CHECK_LAUNCH("gemm_few_rows_pair");
+        return 0;
+    }
+    const int rc = hb_gemm_plain_short_k(A0, 0, W0, w_dtype, C0, 0, M, N, K, lda, ldw, ldc, 0, nullptr, nullptr, 1, 0.f, stream);
+    return rc ? rc : hb_gemm_plain_short_k(A1, 0, W1, w_dtype, C1, 0, M, N, K, lda, ldw, ldc, 0, A_log, dt_bias, D, root, stream);
 }
 
 // A batch of such products in one launch: product b reads A + b * batch_a, W + b * batch_w and writes

@@ -574,6 +574,38 @@ def rows_and_base(x, rows, base=None):
     lib.call("elementwise", "hb_rows_and_base", x.data_ptr(), rows.data_ptr(), dtype_code(rows), _ptr(base), x.numel(), _stream())
 
 
+def _decay_args(decay, N):
+    """(rate, bias, D, root) of gemm_plain_columns' `decay` for the C interface, after checks."""
+    if decay is None:
+        return 0, 0, 0, 0.0
+    if decay[0] == "sigmoid_root":
+        _, bias, root = decay
+        _check(bias, "decay bias", torch.float32, (N,))
+        return bias.data_ptr(), bias.data_ptr(), 1, root
+    rate, bias, D = decay
+    if D <= 0 or N % D:
+        raise BackendError("gemm: a decay's columns are whole heads")
+    _check(rate, "A_log", torch.float32, (N // D,))
+    _check(bias, "dt_bias", torch.float32, (N,))
+    return rate.data_ptr(), bias.data_ptr(), D, 0.0
+
+
+def gemm_plain_columns_pair(a, K, col0, w0, c0, col1, w1, c1, decay=None):
+    """Two products of some columns of a's rows (gemm_plain_columns) that share their sizes: c0 = a[:, col0:col0 + K] @ w0^T and
+    c1 = a[:, col1:col1 + K] @ w1^T, the second with `decay`; a and the sums float32. Few rows: one launch."""
+    _check(a, "a", torch.float32, (None, None))
+    M, lda = a.shape
+    N = w0.shape[0]
+    for w, c, col in ((w0, c0, col0), (w1, c1, col1)):
+        _check(w, "w", w0.dtype, (N, K))
+        _check(c, "c", torch.float32, (M, N))
+        if col < 0 or col + K > lda:
+            raise BackendError(f"gemm: columns [{col}, {col + K}) of rows of {lda}")
+    a_log, dt_bias, D, root = _decay_args(decay, N)
+    lib.call("gemm_plain", "hb_gemm_plain_short_k_pair", a.data_ptr() + 4 * col0, w0.data_ptr(), c0.data_ptr(), a.data_ptr() + 4 * col1,
+             w1.data_ptr(), c1.data_ptr(), dtype_code(w0), M, N, K, lda, K, N, a_log, dt_bias, int(D), float(root), _stream())
+
+
 def gemm_plain_columns(a, col0, K, w, c, accumulate=False, decay=None):
     """c[M, N] (+)= a[:, col0:col0 + K] @ w[N, K]^T in float32 arithmetic: the product of some columns of
     wider rows, read where they lie. (Up to 32 float32 rows times bfloat16 rows, k in steps of 32: a kernel of
@@ -591,22 +623,9 @@ def gemm_plain_columns(a, col0, K, w, c, accumulate=False, decay=None):
     _check(c, "c", None, (M, N))
     if accumulate and c.dtype != torch.float32:
         raise BackendError("gemm: accumulation needs a float32 output")
-    a_log = dt_bias = D = 0
-    root = 0.0
-    if decay is not None and decay[0] == "sigmoid_root":
-        _, bias, root = decay
-        if accumulate or c.dtype != torch.float32:
-            raise BackendError("gemm: a decay is float32, stored and not added to")
-        _check(bias, "decay bias", torch.float32, (N,))
-        a_log = dt_bias = bias.data_ptr()
-        D = 1
-    elif decay is not None:
-        rate, bias, D = decay
-        if accumulate or c.dtype != torch.float32 or D <= 0 or N % D:
-            raise BackendError("gemm: a decay is float32, stored and not added to, its columns whole heads")
-        _check(rate, "A_log", torch.float32, (N // D,))
-        _check(bias, "dt_bias", torch.float32, (N,))
-        a_log, dt_bias = rate.data_ptr(), bias.data_ptr()
+    if decay is not None and (accumulate or c.dtype != torch.float32):
+        raise BackendError("gemm: a decay is float32, stored and not added to")
+    a_log, dt_bias, D, root = _decay_args(decay, N)
     lib.call("gemm_plain", "hb_gemm_plain_short_k", a.data_ptr() + col0 * a.element_size(), dtype_code(a), w.data_ptr(),
              dtype_code(w), c.data_ptr(), dtype_code(c), M, N, K, lda, K, N, 1 if accumulate else 0, a_log, dt_bias,
              int(D), float(root), _stream())

@@ -152,11 +152,14 @@ class GatedDelta(Part):
         if self.low_rank is not None:
             # the second products, float32 sums of the float32 middles
             gate_rows, gate_off = rt.buffer("delta_gate", (T, self.heads * self.vdim), torch.float32), 0
-            ops.gemm_plain_columns(proj, self.g_off, self.g_width, self.g2, gate_rows)
             decay_rows, decay_off = rt.buffer("delta_decay", (T, self.decay_width), torch.float32), 0
             # (a decay a channel leaves this product as the decay itself: softplus and exponentials where the sum is stored)
-            ops.gemm_plain_columns(proj, self.a_off, self.a_width, self.a2, decay_rows,
-                                   decay=(self.a_log, self.dt_bias, self.dim) if self.decay == "channel" else None)
+            decay = (self.a_log, self.dt_bias, self.dim) if self.decay == "channel" else None
+            if self.a2.shape == self.g2.shape:
+                ops.gemm_plain_columns_pair(proj, self.a_width, self.g_off, self.g2, gate_rows, self.a_off, self.a2, decay_rows, decay)
+            else:
+                ops.gemm_plain_columns(proj, self.g_off, self.g_width, self.g2, gate_rows)
+                ops.gemm_plain_columns(proj, self.a_off, self.a_width, self.a2, decay_rows, decay=decay)
         if self.decay == "channel":
             factors = decay_rows
             if self.low_rank is None:

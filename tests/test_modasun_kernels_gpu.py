@@ -364,6 +364,22 @@ def test_experts_products_and_the_shared_experts_gated_sum():
         assert torch.allclose(x.cpu(), want, atol=tol, rtol=tol), f"{dtype}"
 
 
+@pytest.mark.parametrize("M,N,K,col0,col1", [(1, 128, 32, 0, 32), (8, 2048, 128, 260, 4), (9, 48, 64, 4, 72), (33, 64, 32, 0, 32), (5, 40, 24, 0, 24),
+                                             (6, 32, 32, 3, 40)])
+@pytest.mark.parametrize("wd", [torch.float32, torch.bfloat16])
+def test_two_products_of_some_columns_at_once(M, N, K, col0, col1, wd):
+    """One launch or two (more rows, another k, columns off 16-byte borders): the bits of each product by itself."""
+    D = 8
+    a, w0, w1 = rand(M, 400, seed=61).to(DEV), rand(N, K, seed=62, scale=0.3).to(wd).to(DEV), rand(N, K, seed=63, scale=0.3).to(wd).to(DEV)
+    rate, bias = rand(N // D, seed=64).to(DEV), rand(N, seed=65).to(DEV)
+    for decay in (None, (rate, bias, D), ("sigmoid_root", bias, 0.25)):
+        want, got = [torch.empty(M, N, device=DEV) for _ in range(2)], [torch.full((M, N), math.nan, device=DEV) for _ in range(2)]
+        ops.gemm_plain_columns(a, col0, K, w0, want[0])
+        ops.gemm_plain_columns(a, col1, K, w1, want[1], decay=decay)
+        ops.gemm_plain_columns_pair(a, K, col0, w0, got[0], col1, w1, got[1], decay)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
 @pytest.mark.parametrize("T,E,top,N,K", [(1, 8, 2, 33, 512), (5, 4, 3, 96, 1536), (17, 1, 1, 70, 2048), (40, 3, 1, 64, 100), (150, 2, 2, 36, 5004), (9, 4, 2, 40, 30)])
 @pytest.mark.parametrize("wd", [torch.float32, torch.bfloat16])
 def test_products_of_experts_in_float32(T, E, top, N, K, wd):
