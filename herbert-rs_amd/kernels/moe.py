@@ -120,16 +120,7 @@ def combine(y, routing, x, shared=None, gate=None, identity=None):
     no matrices (routing.real and beyond); needed where there are such experts."""
     r = routing
     H = x.shape[1]
-    shared_ptr = gate_ptr = None
-    gate_ld = 0
-    if shared is not None:
-        rows, column = gate
-        _check(shared, "shared", torch.float32, (r.T, H))
-        _check(rows, "gate", torch.float32, (r.T, None))
-        gate_ld = rows.shape[1]
-        if not 0 <= column < gate_ld:
-            raise BackendError("moe combine: the gate's column lies outside its rows")
-        shared_ptr, gate_ptr = shared.data_ptr(), rows.data_ptr() + 4 * column
+    shared_ptr, gate_ptr, gate_ld = _shared_args(r, H, shared, gate)
     _check(y, "y", torch.float32, (r.T * r.top, H))
     _check(x, "x", torch.float32, (r.T, H))
     if r.real < r.E and identity is None:
@@ -139,6 +130,41 @@ def combine(y, routing, x, shared=None, gate=None, identity=None):
     lib.call("moe", "hb_moe_combine", y.data_ptr(), r.weight.data_ptr(), r.row_of.data_ptr(), x.data_ptr(), r.T,
              r.top, H, shared_ptr, gate_ptr, gate_ld, _ptr(identity) if r.real < r.E else None,
              0 if identity is None else dtype_code(identity), r.chosen.data_ptr(), r.real, _stream())
+
+
+def _shared_args(r, H, shared, gate):
+    if shared is None:
+        return None, None, 0
+    rows, column = gate
+    _check(shared, "shared", torch.float32, (r.T, H))
+    _check(rows, "gate", torch.float32, (r.T, None))
+    if not 0 <= column < rows.shape[1]:
+        raise BackendError("moe combine: the gate's column lies outside its rows")
+    return shared.data_ptr(), rows.data_ptr() + 4 * column, rows.shape[1]
+
+
+COMBINE_NORM_TOKENS = 64        # (see combine_norm)
+
+
+def combine_norm(y, routing, acc, norm_w, eps, x, rows, alpha_next, shared=None, gate=None):
+    """`combine` into acc (which then holds the sums only if alpha_next is 0: nobody reads them) and ops.postnorm of them, in one
+    kernel: x = sum / rms(sum) * norm_w, rows (or None) = x in its own type, acc = alpha_next x where that is not 0. For up to
+    COMBINE_NORM_TOKENS tokens; False, and nothing done, where the kernel does not take the sizes."""
+    r = routing
+    T, H = acc.shape
+    if T > COMBINE_NORM_TOKENS or H % 4 or H > 8192 or r.real < r.E:
+        return False
+    shared_ptr, gate_ptr, gate_ld = _shared_args(r, H, shared, gate)
+    _check(y, "y", torch.float32, (T * r.top, H))
+    _check(acc, "acc", torch.float32, (r.T, H))
+    _check(norm_w, "norm weight", torch.float32, (H,))
+    _check(x, "x", torch.float32, (T, H))
+    if rows is not None:
+        _check(rows, "rows", None, (T, H))
+    lib.call("moe", "hb_moe_combine_norm", y.data_ptr(), r.weight.data_ptr(), r.row_of.data_ptr(), acc.data_ptr(), T, r.top, H,
+             shared_ptr, gate_ptr, gate_ld, norm_w.data_ptr(), float(eps), x.data_ptr(), _ptr(rows),
+             dtype_code(x if rows is None else rows), float(alpha_next), _stream())
+    return True
 
 
 EPI_F32, EPI_BF16, EPI_GLU = 0, 1, 2

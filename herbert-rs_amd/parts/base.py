@@ -158,6 +158,18 @@ class TanhJoin:
 
 
 @dataclass
+class NormAfter:
+    """What a block that norms after the sum does with the rows `acc` that a part adds to: x = norm(acc), rows (or None) = x in
+    the compute dtype, acc = alpha x (alpha 0: nothing). `done`: the part's last kernel has done it."""
+    acc: Any
+    norm: Any
+    x: Any
+    rows: Any
+    alpha: float
+    done: bool = False
+
+
+@dataclass
 class StepContext:
     """What one step hands down to the parts."""
     rt: Runtime
@@ -189,6 +201,8 @@ class StepContext:
 
     # set by a block that norms after its parts, for the part that runs: a TanhJoin that the part's last product may do
     join: Any = None
+    # set by a block that norms after the sum, for the part that runs: a NormAfter that the part's last kernel may do
+    norm_after: Any = None
     # (x's address, entry, rows): such a block has left, for that entry's block of the same kind, the normed rows that its
     # mixer reads
     ready_rows: Any = None

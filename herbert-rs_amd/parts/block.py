@@ -21,7 +21,7 @@ import torch
 
 from ..kernels import ops
 from ..weights import TensorNeed
-from .base import Part, TanhJoin
+from .base import NormAfter, Part, TanhJoin
 from .registry import build, register
 
 
@@ -261,10 +261,13 @@ class PostNormBlock(Part):
             steps.append((self.feed_forward, self.norms["post_ff"]))
         for i, (part, norm) in enumerate(steps):
             ctx.handed = ctx.norm_ahead = ctx.left = ctx.fresh_rows = None
-            part.forward(ctx, x if y is None else y, acc)
             last = i + 1 == len(steps)
-            ops.postnorm(acc, norm.w, x, None if last and alpha_after == 0.0 else y, norm.eps,
-                         alpha_after if last else self.alpha)
+            after = NormAfter(acc, norm, x, None if last and alpha_after == 0.0 else y, alpha_after if last else self.alpha)
+            ctx.norm_after = after
+            part.forward(ctx, x if y is None else y, acc)
+            ctx.norm_after = None
+            if not after.done:
+                ops.postnorm(acc, norm.w, x, after.rows, norm.eps, after.alpha)
         if alpha_after != 0.0:
             ctx.pending_post = (x.data_ptr(), alpha_after)
 

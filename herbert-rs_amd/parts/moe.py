@@ -180,5 +180,10 @@ class RoutedExperts(Part):
             moe.gemm_plain(act, self.down, out, routing, gather=False)
         if folded:
             shared, out = out[T * top:], out[:T * top]
-        moe.combine(out, routing, x, shared=shared, gate=None if shared is None else (logits, E),
-                    identity=y if self.identity else None)
+        gate = None if shared is None else (logits, E)
+        after = ctx.norm_after
+        if after is not None and after.acc.data_ptr() == x.data_ptr() and moe.combine_norm(
+                out, routing, x, after.norm.w, after.norm.eps, after.x, after.rows, after.alpha, shared=shared, gate=gate):
+            after.done = True
+            return
+        moe.combine(out, routing, x, shared=shared, gate=gate, identity=y if self.identity else None)

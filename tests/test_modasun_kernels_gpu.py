@@ -380,6 +380,33 @@ def test_two_products_of_some_columns_at_once(M, N, K, col0, col1, wd):
         assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
 
 
+@pytest.mark.parametrize("T,H,top", [(1, 64, 1), (8, 2048, 4), (64, 2052, 3), (5, 4100, 9), (3, 8192, 2)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_the_weighted_sum_and_the_norm_behind_it_in_one_kernel(T, H, top, dtype):
+    """Against the two kernels, with and without a shared expert, rows to leave and a next sum: the sums are the same, the norm's
+    sum of squares comes in another order (H roundings of 2^-24 at most)."""
+    E = top + 3
+    routing = moe.Routing(torch.empty(moe.Routing.ints_needed(T, E, top), dtype=torch.int32, device=DEV),
+                          torch.empty(T, top, device=DEV), T, E, top)
+    moe.route(rand(T, E, seed=71).to(DEV), rand(E, seed=72).to(DEV), routing)
+    y, start, w = rand(T * top, H, seed=73).to(DEV), rand(T, H, seed=74).to(DEV), rand(H, seed=75).to(DEV)
+    shared, gate = rand(T, H, seed=76).to(DEV), rand(T, 7, seed=77).to(DEV)
+    for part, alpha in ((None, 2.0), ((shared, (gate, 4)), 0.0)):
+        given = {} if part is None else dict(shared=part[0], gate=part[1])
+        sums, want, got = start.clone(), [torch.empty(T, H, device=DEV), torch.empty(T, H, dtype=dtype, device=DEV)], \
+            [torch.full((T, H), math.nan, device=DEV), torch.empty(T, H, dtype=dtype, device=DEV)]
+        moe.combine(y, routing, sums, **given)
+        ops.postnorm(sums, w, want[0], want[1], 1e-5, alpha)
+        acc = start.clone()
+        assert moe.combine_norm(y, routing, acc, w, 1e-5, got[0], got[1], alpha, **given)
+        bound = H * 2.0 ** -24 + 2.0 ** -22
+        assert bool(((got[0] - want[0]).abs() <= bound * want[0].abs()).all())
+        assert bool(((got[1].float() - want[1].float()).abs() <= (bound + (2.0 ** -7 if dtype == torch.bfloat16 else 0)) * want[0].abs()).all())
+        assert bool(((acc - sums).abs() <= bound * sums.abs()).all()) if alpha else torch.equal(acc, start)
+    refused = torch.zeros(moe.COMBINE_NORM_TOKENS + 1, H, device=DEV)
+    assert not moe.combine_norm(y, routing, refused, w, 1e-5, refused, None, 0.0)
+
+
 @pytest.mark.parametrize("T,E,top,N,K", [(1, 8, 2, 33, 512), (5, 4, 3, 96, 1536), (17, 1, 1, 70, 2048), (40, 3, 1, 64, 100), (150, 2, 2, 36, 5004), (9, 4, 2, 40, 30)])
 @pytest.mark.parametrize("wd", [torch.float32, torch.bfloat16])
 def test_products_of_experts_in_float32(T, E, top, N, K, wd):
