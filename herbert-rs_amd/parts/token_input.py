@@ -15,7 +15,7 @@ import torch
 
 from ..kernels import ops
 from ..weights import TensorNeed
-from .base import Part
+from .base import NormedRows, Part
 from .linear import Linear
 from .registry import register
 
@@ -56,10 +56,17 @@ class GatedTableInput(Part):
         g = ctx.rt.buffer("token_input_gates", (T, self.dim), torch.float32)
         y = ctx.rt.buffer("token_input_rows", (T, self.hidden_size), torch.float32)
         args = (x, ctx.meta.token_ids, self.table, self.layer * self.dim, self.gate, self.proj_t, self.norm_w, self.eps, g, y)
+        # the norm that x meets next, where it is of the kind that is handed on (`NormedRows`, whole)
+        rows = None
+        if ctx.norm_after_block is not None and getattr(ctx.norm_after_block[0], "hands_on", False) \
+                and ops.token_side_norms(self.hidden_size):
+            norm, entry = ctx.norm_after_block
+            ctx.left = NormedRows(norm, entry, x, ctx.rt.buffer("token_input_normed", (T, self.hidden_size)), None)
+            rows = (norm.w, norm.eps, ctx.left.xg)
         if self.proj is not None and T > ops.TOKEN_SIDE_FEW:
             g16 = ctx.rt.buffer("token_input_gates16", (T, self.dim), torch.bfloat16)
             ops.token_side(*args, stage=0, g16=g16)
             self.proj.forward(g16, y)
-            ops.token_side(*args, stage=2)
+            ops.token_side(*args, stage=2, next_norm=rows)
             return
-        ops.token_side(*args)
+        ops.token_side(*args, next_norm=rows)

@@ -307,3 +307,25 @@ def test_token_input(T, H, D, layers, layer):
         ops.token_side(xg, tokens.to(torch.int32).to(DEV), g(tb), layer * D, g(gt), g(pj.t()), g(norm_w), 1e-5,
                        torch.empty(T, D, device=DEV), torch.empty(T, H, device=DEV))
         assert float((xg.cpu() - want).abs().max()) <= tol * float(want.abs().max())
+
+
+@pytest.mark.parametrize("T,H", [(1, 64), (7, 176), (3, 2048), (70, 2052), (2, 4100), (2, 8192)])
+def test_token_input_and_the_norm_behind_it(T, H):
+    """One kernel against two: the same x but for the order of y's squares, and the norm of it (H roundings of 2^-24 a sum)."""
+    D, V = 32, 50
+    x, table, gate, proj = rand(T, H, seed=1, scale=2.0), rand(V, D, seed=2), rand(D, H, seed=3, scale=H ** -0.5), rand(H, D, seed=4)
+    norm_w, next_w = 1 + 0.2 * rand(H, seed=5), 1 + 0.2 * rand(H, seed=7)
+    tokens = torch.randint(0, V, (T,), generator=torch.Generator().manual_seed(6)).to(torch.int32).to(DEV)
+    bound = H * 2.0 ** -24 + 2.0 ** -21
+    for dtype in (torch.float32, torch.bfloat16):
+        one, two, rows = g(x).clone(), g(x).clone(), torch.empty(T, H, dtype=dtype, device=DEV)
+        args = (tokens, g(table), 0, g(gate), g(proj.t().contiguous()), g(norm_w), 1e-5, torch.empty(T, D, device=DEV), torch.empty(T, H, device=DEV))
+        ops.token_side(one, *args)
+        want = torch.empty(T, H, dtype=torch.float32, device=DEV)
+        ops.rmsnorm(one, g(next_w), want, 1e-6)
+        ops.token_side(two, *args, next_norm=(g(next_w), 1e-6, rows))
+        size = one.abs() + (one - g(x)).abs()
+        assert bool(((two - one).abs() <= bound * size).all())
+        slack = bound * (want.abs() + size * (want / one).abs()) + (2.0 ** -8 * want.abs() if dtype == torch.bfloat16 else 0)
+        assert bool(((rows.float() - want).abs() <= slack + 1e-6).all())
+    assert not ops.token_side_norms(H + 1)
