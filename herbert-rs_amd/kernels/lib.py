@@ -1,10 +1,15 @@
-"""Loading the built HIP modules through ctypes.
+"""Loading the built HIP modules through ctypes, and calling them.
 
 A module is loaded when one of its functions is first asked for and is compiled
 then if it is not built. There is no other implementation behind these
 functions: without the extension every call raises BackendError.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
+import threading
+
+import torch  # noqa: F401 (the extension module's symbols are torch's)
 
 from ..errors import BackendError
 from . import build
@@ -129,13 +134,45 @@ def loaded_modules():
     return sorted(_loaded)
 
 
-_functions = {}
+_host = None
+_host_lock = threading.Lock()
+
+
+def host():
+    """The extension module of csrc/hostcall.cpp, built first if need be."""
+    global _host
+    if _host is None:
+        with _host_lock:
+            if _host is None:
+                path = build.build_module(build.HOST_MODULE)
+                loader = importlib.machinery.ExtensionFileLoader(build.HOST_MODULE, path)
+                try:
+                    module = importlib.util.module_from_spec(importlib.util.spec_from_loader(build.HOST_MODULE, loader))
+                    loader.exec_module(module)
+                except ImportError as e:
+                    raise BackendError(f"cannot load {path}: {e}") from None
+                _host = module
+    return _host
+
+
+_entries = {}
+_invoke = None
+
+
+def _entry(module, fname):
+    """What `call` hands to the extension module for an entry point: its address and the kinds of its arguments."""
+    global _invoke
+    fn = getattr(load(module), fname)
+    kinds = "".join("f" if t is _F else "i" for t in fn.argtypes)
+    entry = _entries[(module, fname)] = host().entry(ctypes.cast(fn, _P).value, kinds)
+    _invoke = host().invoke
+    return entry
 
 
 def call(module, fname, *args):
     """Call a C entry point; a non-zero return becomes BackendError with its text."""
-    fn = _functions.get((module, fname))
-    if fn is None:
-        fn = _functions[(module, fname)] = getattr(load(module), fname)
-    if fn(*args) != 0:
+    entry = _entries.get((module, fname))
+    if entry is None:
+        entry = _entry(module, fname)
+    if _invoke(entry, *args) != 0:
         raise BackendError(load(module).hb_last_error().decode(errors="replace"))

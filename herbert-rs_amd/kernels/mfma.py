@@ -290,7 +290,7 @@ def gemm(a, w, out, accumulate=False, packed=False, norm=None, tile=0, leave=Non
     deferred = ctypes.c_int(1) if defer_slices else None
     lib.call("gemm_mfma", "hb_gemm_mfma", a.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K, N,
              EPI_ADD if accumulate else EPI_STORE, 1 if packed else 0, norm_ptr, eps, int(tile), ws_ptr,
-             ws_floats, *hand, ctypes.byref(deferred) if defer_slices else None, 0, _stream())
+             ws_floats, *hand, ctypes.addressof(deferred) if defer_slices else None, 0, _stream())
     if defer_slices:
         return (deferred.value, ws_ptr, M * N) if deferred.value > 1 else (1, out.data_ptr(), 0)
     return None
