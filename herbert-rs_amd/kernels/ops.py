@@ -591,7 +591,7 @@ def _decay_args(decay, N):
 
 def gemm_plain_columns_pair(a, K, col0, w0, c0, col1, w1, c1, decay=None):
     """Two products of some columns of a's rows (gemm_plain_columns) that share their sizes: c0 = a[:, col0:col0 + K] @ w0^T and
-    c1 = a[:, col1:col1 + K] @ w1^T, the second with `decay`; a and the sums float32. Few rows: one launch."""
+    c1 = a[:, col1:col1 + K] @ w1^T, the second with `decay`; a and the sums float32. One launch."""
     _check(a, "a", torch.float32, (None, None))
     M, lda = a.shape
     N = w0.shape[0]
@@ -607,8 +607,7 @@ def gemm_plain_columns_pair(a, K, col0, w0, c0, col1, w1, c1, decay=None):
 
 def gemm_plain_columns(a, col0, K, w, c, accumulate=False, decay=None):
     """c[M, N] (+)= a[:, col0:col0 + K] @ w[N, K]^T in float32 arithmetic: the product of some columns of
-    wider rows, read where they lie. (Up to 32 float32 rows times bfloat16 rows, k in steps of 32: a kernel of
-    more and smaller workgroups than the tiled one, which a short k leaves with few.)
+    wider rows, read where they lie.
     decay (a_log f32 [N / D], dt_bias f32 [N], D): the sums are a decay's pre-activations, and c (float32, not
     added to) takes the decays themselves, exp(-exp(a_log[n // D]) softplus(sum + dt_bias[n])), as
     `recurrent.channel_decay` makes them from rows in memory.
