@@ -18,8 +18,8 @@
 //
 // chunk_prepare_kernel: everything that does not need S_0, one workgroup a (chunk, head), all of them at once. It leaves
 // in scratch, as the operands that the second kernel's lanes load: G q, G_64 / G k, B, and -T beta G K and T beta V.
-// chunk_scan_kernel: the chain of chunks, one workgroup a (head, 16 columns of S): four waves, each 16 tokens of a
-// chunk (U and O) and a quarter of the state's rows (S).
+// chunk_scan_kernel: the chain of chunks, one workgroup a (head, 16 columns of S): four waves for the chain, each 16 tokens of a
+// chunk (U) and a quarter of the state's rows (S), and four for the outputs (O), 16 tokens each.
 //
 // The walk rounds the state and what is subtracted from a value token by token; here a rounding of A, B or T reaches
 // many tokens. So A, B and T are sums in float64 (the decays of the delta rule too), rounded once; sums over tokens run in their order, the
@@ -28,9 +28,9 @@
 // 0.999: the outputs' error is 0.67 to 0.97 of the walk's (0.8e-7 to 1e-6), 0.56 to 0.88 for the linear attention, and that of the
 // state left 0.76 to 1.06. (With A, B and T in float32 the outputs' was up to 1.3 of the walk's, the state's up to 2.)
 //
-// 2,048 tokens of 16 heads of 128 x 128 take 196 us (the walk 781), with a decay a channel 221 (1,084), the linear attention
-// 149 (909); 8 sequences of 300 tokens 192, 228 and 127 (446, 408 and 455). Bound: the second kernel by its chain (112
-// products of 32 cycles a chunk and wave and two exchanges through LDS, 118 us of the 196), the first by its products, in float64 of 64
+// 2,048 tokens of 16 heads of 128 x 128 take 178 us (the walk 781), with a decay a channel 201 (1,084), the linear attention
+// 131 (909); 8 sequences of 300 tokens 184, 217 and 123 (446, 408 and 455). Bound: the second kernel by its chain (64
+// products of 32 cycles a chunk and wave and two exchanges through LDS, 99 us of the 178), the first by its products, in float64 of 64
 // cycles, for which a (chunk, head) has one workgroup a CU.
 #include "common.h"
 #include "mfma_f32.h"
@@ -399,8 +399,12 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
         *(f32x4*)(out + at.w + ((wave * DB + b) * 64 + lane) * 4) = *(const f32x4*)&rows[(16 * wave + r) * KLD + 16 * b + 4 * q];
 }
 
+// Eight waves: four on the chain (a block of 16 tokens of U, then a quarter of the state's rows), four on the outputs (a block of 16 tokens),
+// which nothing waits for: they follow a phase behind the chain, in the gaps that it leaves the matrix cores (a chunk of a head of 128 x 128: chain
+// 64 products of 32 cycles, 0.9 us, with the two exchanges 1.8, outputs 48). One sequence of 2,048 tokens, 16 heads of 128 x 128: 99 us, by four
+// waves that did both, one after the other, 118 (110 with this loop).
 template <int DB, bool DELTA>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(512)
 chunk_scan_kernel(const float* __restrict__ qkv, int C, const float* __restrict__ scratch, float* __restrict__ state,
                   const int4* __restrict__ runs, const int* __restrict__ slots, float* __restrict__ out,
                   int kv_heads, int heads, int V, float out_scale) {
@@ -410,121 +414,189 @@ chunk_scan_kernel(const float* __restrict__ qkv, int C, const float* __restrict_
     const int h = blockIdx.x, vb = blockIdx.y;
     const int4 run = runs[blockIdx.z];
     const int begin = run.z, n_all = run.w, last = (n_all + CHUNK - 1) / CHUNK;
+    if (last <= 0) return;
     const ChunkLayout at = chunk_layout(D, V, DELTA);
     const float* part = scratch + ((size_t)run.y * heads + h) * at.size;
     const size_t chunk_step = (size_t)heads * at.size;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3;
+    const bool chain = __builtin_amdgcn_readfirstlane(tid >> 6) < 4;
     const int r = lane & 15, q = lane >> 4;
     const int col = 16 * vb + r;
-    float* S_mem = state + ((size_t)slots[run.x] * heads + h) * D * V + col;
-    f32x4 S[OWN];
-    auto share = [&](int buf) {
+    // (every load is made, of a place at hand where there is none: with loads that may be left out the compiler waits for all that are in
+    // flight at the first use of any)
+    auto values = [&](int c, float* v) {
+        const int n = n_all - c * CHUNK;
+        const float* from = qkv + (size_t)(begin + c * CHUNK) * C + 2 * kv_heads * D + h * V + col;
+#pragma unroll
+        for (int s = 0; s < 16; ++s) v[s] = from[(size_t)(4 * s + q < n ? 4 * s + q : n - 1) * C];
+    };
+    // u of a chunk's tokens, as the products want them: without a correction the values themselves
+    auto tokens = [&](int c, int buf, const float* v, int from, f32x4* us) {
+        if (DELTA) {
+#pragma unroll
+            for (int b = 0; b < 4; ++b) us[b] = *(const f32x4*)&u_lds[buf][r * ULD + 16 * b + 4 * q];
+            return;
+        }
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int t = 16 * b + 4 * e + q;
+                us[b][e] = t < from && c * CHUNK + t < n_all ? v[4 * b + e] : 0.f;
+            }
+    };
+
+    // Barriers of a chunk: one when u lies in LDS (with a correction), one when the next state does.
+    if (chain) {
+        struct Operands {
+            f32x4 w[DELTA ? DB : 1], k[OWN][4], u, g[OWN];
+            float v[DELTA ? 1 : 16];
+            int from;
+        };
+        auto fetch = [&](int c, Operands& o) {
+            const float* p = part + (size_t)c * chunk_step;
+            if (DELTA) {
+#pragma unroll
+                for (int b = 0; b < DB; ++b) o.w[b] = *(const f32x4*)(p + at.w + ((wave * DB + b) * 64 + lane) * 4);
+                o.u = *(const f32x4*)(p + at.u + ((wave * (V / 16) + vb) * 64 + lane) * 4);
+            } else {
+                values(c, o.v);
+            }
+#pragma unroll
+            for (int i = 0; i < OWN; ++i) {
+                o.g[i] = *(const f32x4*)(p + at.g + 16 * (wave + 4 * i) + 4 * q);
+#pragma unroll
+                for (int s = 0; s < 4; ++s) o.k[i][s] = *(const f32x4*)(p + at.k + (((wave + 4 * i) * 4 + s) * 64 + lane) * 4);
+            }
+            o.from = ((const int*)p)[at.from + col];
+        };
+        float* S_mem = state + ((size_t)slots[run.x] * heads + h) * D * V + col;
+        f32x4 S[OWN];
+        auto share = [&](int buf) {
+#pragma unroll
+            for (int i = 0; i < OWN; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s_lds[buf][r * SLD + 16 * (wave + 4 * i) + 4 * e + q] = S[i][e];
+        };
+        auto step = [&](int c, int buf, const Operands& o, Operands& next) {
+            fetch(c + 1 < last ? c + 1 : c, next);
+            __builtin_amdgcn_sched_barrier(0);
+            if (DELTA) {
+                Chains<8> uc;
+#pragma unroll
+                for (int b = 0; b < DB; ++b) {
+                    const f32x4 s = *(const f32x4*)&s_lds[buf][r * SLD + 16 * b + 4 * q];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) uc.add(o.w[b][e], s[e], 4 * b + e);
+                }
+                const f32x4 u = o.u + uc.sum();
+#pragma unroll
+                for (int e = 0; e < 4; ++e) u_lds[buf][r * ULD + 16 * wave + 4 * e + q] = u[e];
+                hb_workgroup_barrier();
+            }
+            f32x4 us[4];
+            tokens(c, buf, o.v, o.from, us);
+            // The state (and the outputs) token by token in ascending order behind what the state before gives, so that the latest tokens,
+            // mostly the largest, are added last: as the walk rounds, without its decay of every token.
+#pragma unroll
+            for (int i = 0; i < OWN; ++i) S[i] *= o.g[i];
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int i = 0; i < OWN; ++i) S[i] = mfma_k4(o.k[i][b][e], us[b][e], S[i]);
+            if (o.from < CHUNK) {
+#pragma unroll
+                for (int i = 0; i < OWN; ++i) S[i] = f32x4{NAN, NAN, NAN, NAN};
+            }
+            share(buf ^ 1);
+            hb_workgroup_barrier();
+        };
+        __builtin_amdgcn_s_setprio(3);
+        Operands even, odd;
+        fetch(0, even);                                       // (asked for before the state, whose slot is a load away)
 #pragma unroll
         for (int i = 0; i < OWN; ++i)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) s_lds[buf][r * SLD + 16 * (wave + 4 * i) + 4 * e + q] = S[i][e];
-    };
+            for (int e = 0; e < 4; ++e) S[i][e] = S_mem[(size_t)(16 * (wave + 4 * i) + 4 * q + e) * V];
+        share(0);
+        hb_workgroup_barrier();
+        for (int c = 0; c < last; c += 2) {                   // (two by two: the operands' registers take turns, nothing is copied)
+            step(c, 0, even, odd);
+            if (c + 1 < last) step(c + 1, 1, odd, even);
+        }
+#pragma unroll
+        for (int i = 0; i < OWN; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) S_mem[(size_t)(16 * (wave + 4 * i) + 4 * q + e) * V] = S[i][e];
+        return;
+    }
+
     struct Operands {
-        f32x4 w[DELTA ? DB : 1], qg[DB], b[4], k[OWN][4], u;
-        float g[OWN][4], v[DELTA ? 1 : 16];
+        f32x4 qg[DB], b[4];
+        float v[DELTA ? 1 : 16];
         int from, lost;
     };
     auto fetch = [&](int c, Operands& o) {
         const float* p = part + (size_t)c * chunk_step;
 #pragma unroll
-        for (int b = 0; b < DB; ++b) {
-            if (DELTA) o.w[b] = *(const f32x4*)(p + at.w + ((wave * DB + b) * 64 + lane) * 4);
-            o.qg[b] = *(const f32x4*)(p + at.q + ((wave * DB + b) * 64 + lane) * 4);
-        }
-        if (DELTA) o.u = *(const f32x4*)(p + at.u + ((wave * (V / 16) + vb) * 64 + lane) * 4);
+        for (int b = 0; b < DB; ++b) o.qg[b] = *(const f32x4*)(p + at.q + ((wave * DB + b) * 64 + lane) * 4);
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
-            if (b <= wave) o.b[b] = *(const f32x4*)(p + at.b + ((wave * 4 + b) * 64 + lane) * 4);
-#pragma unroll
-        for (int i = 0; i < OWN; ++i)
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                o.k[i][s] = *(const f32x4*)(p + at.k + (((wave + 4 * i) * 4 + s) * 64 + lane) * 4);
-                o.g[i][s] = p[at.g + 16 * (wave + 4 * i) + 4 * q + s];
-            }
+        for (int b = 0; b < 4; ++b) o.b[b] = *(const f32x4*)(p + at.b + ((wave * 4 + (b <= wave ? b : wave)) * 64 + lane) * 4);
+        if (!DELTA) values(c, o.v);
         o.from = ((const int*)p)[at.from + col];
         o.lost = ((const int*)p)[at.lost + wave];
-        if (!DELTA) {
-            const int n = n_all - c * CHUNK;
-            const float* v = qkv + (size_t)(begin + c * CHUNK) * C + 2 * kv_heads * D + h * V + col;
-#pragma unroll
-            for (int s = 0; s < 16; ++s) o.v[s] = 4 * s + q < n ? v[(size_t)(4 * s + q) * C] : 0.f;
-        }
     };
-    Operands next;
-    fetch(0, next);                                           // (asked for before the state, whose slot is a load away)
-#pragma unroll
-    for (int i = 0; i < OWN; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) S[i][e] = S_mem[(size_t)(16 * (wave + 4 * i) + 4 * q + e) * V];
-    share(0);
-    __syncthreads();
-    int buf = 0;
-    for (int c = 0; c < last; ++c, buf ^= 1) {
-        const Operands o = next;
-        if (c + 1 < last) fetch(c + 1, next);
-        Chains<8> uc, oc;
-#pragma unroll
-        for (int b = 0; b < DB; ++b) {
-            const f32x4 s = *(const f32x4*)&s_lds[buf][r * SLD + 16 * b + 4 * q];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                if (DELTA) uc.add(o.w[b][e], s[e], 4 * b + e);
-                oc.add(o.qg[b][e], s[e], 4 * b + e);
-            }
-        }
-        f32x4 us[4];
-        if (DELTA) {
-            const f32x4 u = o.u + uc.sum();
-#pragma unroll
-            for (int e = 0; e < 4; ++e) u_lds[buf][r * ULD + 16 * wave + 4 * e + q] = u[e];
-            __syncthreads();
-#pragma unroll
-            for (int b = 0; b < 4; ++b) us[b] = *(const f32x4*)&u_lds[buf][r * ULD + 16 * b + 4 * q];
-        } else {
-#pragma unroll
-            for (int b = 0; b < 4; ++b)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) us[b][e] = 16 * b + 4 * e + q < o.from ? o.v[4 * b + e] : 0.f;
-        }
-        // The state and the outputs token by token in ascending order behind what the state before gives, so that the latest tokens,
-        // mostly the largest, are added last: as the walk rounds, without its decay of every token.
-        f32x4 sums = oc.sum();
-#pragma unroll
-        for (int i = 0; i < OWN; ++i)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) S[i][e] *= o.g[i][e];
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-#pragma unroll
-                for (int i = 0; i < OWN; ++i) S[i] = mfma_k4(o.k[i][b][e], us[b][e], S[i]);
-                if (b <= wave) sums = mfma_k4(o.b[b][e], us[b][e], sums);
-            }
-        }
-        if (o.from < CHUNK) {
-#pragma unroll
-            for (int i = 0; i < OWN; ++i) S[i] = f32x4{NAN, NAN, NAN, NAN};
-        }
-        share(buf ^ 1);
+    f32x4 held;                                               // a chunk's outputs, on their way before the next but one chunk's loads
+    auto leave = [&](int c) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int t = 16 * wave + 4 * q + e, at_token = c * CHUNK + t;
-            if (at_token < n_all)
-                out[(size_t)(begin + at_token) * heads * V + h * V + col] = t < o.from && !(o.lost >> (4 * q + e) & 1) ? sums[e] * out_scale : NAN;
+            const int at_token = c * CHUNK + 16 * wave + 4 * q + e;
+            if (c >= 0 && at_token < n_all) out[(size_t)(begin + at_token) * heads * V + h * V + col] = held[e];
         }
-        __syncthreads();
+    };
+    // What the chain holds in LDS for chunk c: the state until u of the chunk after it is there, u until the state after that one is. So with a
+    // correction the outputs' products begin once u of their own chunk is there and end in the chunk after it.
+    constexpr int FIRST = DELTA ? 3 * DB / 4 : DB;
+    auto step = [&](int c, int buf, const Operands& o, Operands& next) {
+        if (DELTA) hb_workgroup_barrier();
+        leave(c - 1);
+        fetch(c + 1 < last ? c + 1 : c, next);
+        __builtin_amdgcn_sched_barrier(0);
+        Chains<8> oc;
+        auto of_state = [&](int b) {
+            const f32x4 s = *(const f32x4*)&s_lds[buf][r * SLD + 16 * b + 4 * q];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) oc.add(o.qg[b][e], s[e], 4 * b + e);
+        };
+#pragma unroll
+        for (int b = 0; b < FIRST; ++b) of_state(b);
+        if (DELTA) hb_workgroup_barrier();
+#pragma unroll
+        for (int b = FIRST; b < DB; ++b) of_state(b);
+        f32x4 us[4];
+        tokens(c, buf, o.v, o.from, us);
+        f32x4 sums = oc.sum();
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+            if (b <= wave) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sums = mfma_k4(o.b[b][e], us[b][e], sums);
+            }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            held[e] = 16 * wave + 4 * q + e < o.from && !(o.lost >> (4 * q + e) & 1) ? sums[e] * out_scale : NAN;
+        if (!DELTA) hb_workgroup_barrier();
+    };
+    Operands even, odd;
+    fetch(0, even);
+    hb_workgroup_barrier();
+    for (int c = 0; c < last; c += 2) {
+        step(c, 0, even, odd);
+        if (c + 1 < last) step(c + 1, 1, odd, even);
     }
-#pragma unroll
-    for (int i = 0; i < OWN; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) S_mem[(size_t)(16 * (wave + 4 * i) + 4 * q + e) * V] = S[i][e];
+    leave(last - 1);
 }
 
 // As hb_gated_delta of recurrent.hip, for keys of 64 or 128 and values in steps of 16, rows in whole quads, and for those
@@ -552,7 +624,7 @@ extern "C" int hb_chunked_delta(const float* qkv, int C, const float* proj, int 
         chunk_prepare_kernel<DB, CH, DELTA><<<grid, 256, 0, stream>>>(qkv, C, proj, ld, b_off, a_off, A_log, dt_bias,  \
             decay, (const int2*)chunks, scratch, kv_heads, heads, V);                                                 \
         HB_CHECK_LAUNCH("chunk_prepare");                                                                             \
-        chunk_scan_kernel<DB, DELTA><<<scan, 256, 0, stream>>>(qkv, C, scratch, state, (const int4*)runs, slots, out, \
+        chunk_scan_kernel<DB, DELTA><<<scan, 512, 0, stream>>>(qkv, C, scratch, state, (const int4*)runs, slots, out, \
             kv_heads, heads, V, out_scale);                                                                           \
     } while (0)
     if (D == 128 && !correction) HB_CHUNKS(8, true, false);
