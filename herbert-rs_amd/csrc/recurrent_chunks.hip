@@ -648,12 +648,12 @@ extern "C" int hb_chunked_delta(const float* qkv, int C, const float* proj, int 
 // ssm_pairs_kernel: C_t . B_i of a (chunk, group) once for all its heads, as the second kernel's lanes load them.
 // A factor beyond TOO_LARGE (inputs, B, C, the state) counts as not finite here: below it no product before its decay passes float32's
 // range (sums of 128 products of two are 1.3e38 at most), beyond it one may where the walk, whose state decays first, stays within.
-// ssm_chunks_kernel: the chain of chunks, a workgroup a (head, 32 columns of S, sequence): four waves, each 16 tokens of a chunk for the outputs and a
+// ssm_chunks_kernel: the chain of chunks, a workgroup a (head, 16 or 32 columns of S, sequence): four waves, each 16 tokens of a chunk for the outputs and a
 // quarter of the state's rows. A chunk that holds something not finite is walked token by token instead (ssm_slowly), so that it
 // spoils what it spoils in the walk.
-// 64 heads of 128 x 64 on 8 groups, one sequence of 2,048 tokens 318 us (the walk 802), of 512 91 (209), four of 512 133 (313), 16 of 128 140
-// (310). Bound by a chunk's chain in a workgroup, 9.5 us: 160 products of 40 cycles a wave, and as long again for the decays and for
-// laying out the state and the columns. Errors against 64 bits are 0.2 to 1.02 of the walk's.
+// 64 heads of 128 x 64 on 8 groups, one sequence of 2,048 tokens 226 us (the walk 802), of 512 70 (209), four of 512 130 (313), 16 of 128 140
+// (310). Bound by a chunk's chain in a workgroup, 6.7 us with 16 columns, 9.5 with 32: 80 or 160 products of 40 cycles a wave, and as long again
+// for the decays and for laying out the state and the columns. Errors against 64 bits are 0.2 to 1.02 of the walk's.
 #define TOO_LARGE 1e18f
 __device__ __forceinline__ bool too_large(float v) { return !(fabsf(v) <= TOO_LARGE); }
 
@@ -691,11 +691,12 @@ ssm_pairs_kernel(const float* __restrict__ u, int ldu, int b_at, int c_at, const
     }
 }
 
-// One chunk of 32 columns token by token; the state lies in LDS, a column's entry n at in_quads(n). Eight lanes a column.
-template <int N, int SLD>
+// One chunk of COLS columns token by token; the state lies in LDS, a column's entry n at in_quads(n). Eight lanes a column.
+template <int N, int SLD, int COLS>
 __device__ __forceinline__ void ssm_slowly(float* s_lds, const float* u, int ldu, const float* proj, int ld, int n, int x_at, int b_at, int c_at,
                                            float bias, float rate, float skip, float* y, int ldy, int cols) {
     const int col = threadIdx.x / 8, part = threadIdx.x % 8;
+    if (col >= COLS) return;
     for (int t = 0; t < n; ++t) {
         const float* row = u + (size_t)t * ldu;
         const float z = proj[(size_t)t * ld] + bias, dt = z > 20.f ? z : log1pf(expf(z)), a = expf(-rate * dt);
@@ -712,8 +713,7 @@ __device__ __forceinline__ void ssm_slowly(float* s_lds, const float* u, int ldu
     }
 }
 
-#define SSM_COLS 32
-template <int DB>
+template <int DB, int SSM_COLS>
 __global__ void __launch_bounds__(256, 2)
 ssm_chunks_kernel(const float* __restrict__ u, int ldu, const float* __restrict__ proj, int ld, int dt_off,
                   const float* __restrict__ dt_bias, const float* __restrict__ A_log, const float* __restrict__ Dskip,
@@ -748,15 +748,16 @@ ssm_chunks_kernel(const float* __restrict__ u, int ldu, const float* __restrict_
 #pragma unroll
                 for (int e = 0; e < 4; ++e) s_lds[buf][(16 * cb + r) * SLD + 16 * (wave + 4 * i) + 4 * e + q] = S[i][cb][e];
     };
-    // a chunk's inputs that all waves share: thread tid brings eight columns of token tid / 4 (columns past the head's are zeros)
-    const int my_token = tid / 4, my_col = tid % 4 * 8;
-    f32x4 x_next[2];
+    // a chunk's inputs that all waves share: thread tid brings a quarter of token tid / 4's columns (those past the head's are zeros)
+    constexpr int XQ = SSM_COLS / 16;                          // in quads
+    const int my_token = tid / 4, my_col = tid % 4 * 4 * XQ;
+    f32x4 x_next[XQ];
     float z_next;
     auto fetch = [&](int c) {
         const int n = min(CHUNK, n_all - c * CHUNK);
         const float* row = u + (size_t)(begin + c * CHUNK + my_token) * ldu + x_at + my_col;
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < XQ; ++i)
             x_next[i] = my_token < n && my_col + 4 * i < cols ? *(const f32x4*)(row + 4 * i) : f32x4{0.f, 0.f, 0.f, 0.f};
         z_next = lane < n ? proj[(size_t)(begin + c * CHUNK + lane) * ld + dt_off + h] : 0.f;
     };
@@ -776,7 +777,7 @@ ssm_chunks_kernel(const float* __restrict__ u, int ldu, const float* __restrict_
         const float my_dt = __shfl(dt, my_token & 63, HB_WAVE);
         bool bad = not_finite(dt) || not_finite((float)sum);
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < XQ; ++i)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 bad |= too_large(x_next[i][e]) || too_large(x_next[i][e] * my_dt);
@@ -845,7 +846,7 @@ ssm_chunks_kernel(const float* __restrict__ u, int ldu, const float* __restrict_
         }
         __syncthreads();                                      // (everyone has looked for what is not finite)
         if (spoilt[buf]) {
-            ssm_slowly<N, SLD>(s_lds[buf], u + (size_t)t0 * ldu, ldu, proj + (size_t)t0 * ld + dt_off + h, ld, n, x_at, b_at, c_at, bias, rate, skip,
+            ssm_slowly<N, SLD, SSM_COLS>(s_lds[buf], u + (size_t)t0 * ldu, ldu, proj + (size_t)t0 * ld + dt_off + h, ld, n, x_at, b_at, c_at, bias, rate, skip,
                                y + (size_t)t0 * inner + x_at, inner, cols);
             __syncthreads();
 #pragma unroll
@@ -919,18 +920,24 @@ extern "C" int hb_chunked_ssm(const float* u, int ldu, const float* proj, int ld
                "state-space chunks: rows of %d are not in whole quads", ldu);
     HB_REQUIRE(dt_off >= 0 && dt_off + heads <= ld, "state-space chunks: the columns lie outside their rows");
     HB_REQUIRE((uintptr_t)chunks % 8 == 0 && (uintptr_t)runs % 16 == 0, "state-space chunks: the lists are not aligned");
-    const int tiles = (P + SSM_COLS - 1) / SSM_COLS;
+    // 16 columns of the state a workgroup where that many still fit the chip at once, two a CU: half the products in a chunk's chain, the
+    // decays once more. 64 heads of 128 x 64 in 8 groups, us by 32 | 16 columns: one sequence of 2,048 tokens (128 workgroups of 32 columns)
+    // 313 | 226, of 512 91 | 70, two of 512 and 300 (256) 93 | 78, four of 512 (512) 130 | 167.
+    const bool narrow = (long long)heads * ((P + 31) / 32) * n_runs <= 256;
+    const int tiles = (P + (narrow ? 15 : 31)) / (narrow ? 16 : 32);
     HB_REQUIRE(n_runs <= 65535 && n_chunks <= 65535 && tiles <= 65535, "state-space chunks: too many sequences or columns for the grid");
-#define HB_SSM_CHUNKS(DB)                                                                                                    \
+#define HB_SSM_CHUNKS(DB, COLS)                                                                                              \
     do {                                                                                                                     \
         ssm_pairs_kernel<DB><<<dim3(groups, n_chunks), 256, 0, stream>>>(u, ldu, heads * P, heads * P + groups * N,          \
                                                                          (const int2*)chunks, pairs, groups);                \
         HB_CHECK_LAUNCH("ssm_pairs");                                                                                        \
-        ssm_chunks_kernel<DB><<<dim3(heads, tiles, n_runs), 256, 0, stream>>>(u, ldu, proj, ld, dt_off, dt_bias, A_log, Dskip, \
+        ssm_chunks_kernel<DB, COLS><<<dim3(heads, tiles, n_runs), 256, 0, stream>>>(u, ldu, proj, ld, dt_off, dt_bias, A_log, Dskip, \
             pairs, state, (const int4*)runs, slots, y, heads, groups, P);                                                    \
     } while (0)
-    if (N == 128) HB_SSM_CHUNKS(8);
-    else HB_SSM_CHUNKS(4);
+    if (N == 128 && narrow) HB_SSM_CHUNKS(8, 16);
+    else if (N == 128) HB_SSM_CHUNKS(8, 32);
+    else if (narrow) HB_SSM_CHUNKS(4, 16);
+    else HB_SSM_CHUNKS(4, 32);
 #undef HB_SSM_CHUNKS
     HB_CHECK_LAUNCH("ssm_chunks");
     return 0;

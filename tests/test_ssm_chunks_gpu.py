@@ -124,3 +124,24 @@ def test_large_numbers_pass_no_range_that_they_do_not_pass_in_the_walk(place, wh
         assert torch.equal(a.isfinite(), b.isfinite())
         fine = b.isfinite()
         assert float((a - b)[fine].abs().max()) <= 1e-4 * float(b[fine].abs().max())
+
+
+@pytest.mark.parametrize("bad", [False, True])
+@pytest.mark.parametrize("lengths,heads,groups,N,P", [([64, 130, 65], 96, 3, 64, 16), ([70, 1000], 65, 5, 128, 48), ([129, 64], 129, 1, 64, 32)])
+def test_a_sequence_alone_and_beside_others(lengths, heads, groups, N, P, bad):
+    """Few workgroups take 16 columns of the state each and many 32 (the columns' last ones may be half of that): a sequence has the same bits
+    either way, also where an entry of B has a chunk walked token by token."""
+    u, proj, a_log, dt_bias, d_skip, state, meta = step(lengths, heads, groups, N, P, -2.0)
+    if bad:
+        u[lengths[0] - 3, heads * P + 7] = float("inf")
+    assert heads * ((P + 31) // 32) * len(lengths) > 256 >= heads * ((P + 31) // 32)
+    got, left = run(u, proj, a_log, dt_bias, d_skip, state, meta, heads, groups, N, P)
+    at = 0
+    for b, n in enumerate(lengths):
+        slot = len(lengths) - b
+        one = types.SimpleNamespace(max_new=n, num_seqs=1, seq_starts=torch.tensor([0, n], dtype=torch.int32, device=DEV), derived={},
+                                    host_starts=torch.tensor([0, n], dtype=torch.int32).numpy(), slots=torch.tensor([slot], dtype=torch.int32, device=DEV))
+        alone, alone_left = run(u[at:at + n], proj[at:at + n], a_log, dt_bias, d_skip, state, one, heads, groups, N, P)
+        assert torch.equal(alone.nan_to_num(7.0), got[at:at + n].nan_to_num(7.0))
+        assert torch.equal(alone_left[slot].nan_to_num(7.0), left[slot].nan_to_num(7.0))
+        at += n
