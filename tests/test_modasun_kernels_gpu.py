@@ -368,7 +368,7 @@ def test_experts_products_and_the_shared_experts_gated_sum():
                                              (6, 32, 32, 3, 40)])
 @pytest.mark.parametrize("wd", [torch.float32, torch.bfloat16])
 def test_two_products_of_some_columns_at_once(M, N, K, col0, col1, wd):
-    """One launch or two (more rows, another k, columns off 16-byte borders): the bits of each product by itself."""
+    """For any number of rows, any k and columns off 16-byte borders: the bits of each product by itself."""
     D = 8
     a, w0, w1 = rand(M, 400, seed=61).to(DEV), rand(N, K, seed=62, scale=0.3).to(wd).to(DEV), rand(N, K, seed=63, scale=0.3).to(wd).to(DEV)
     rate, bias = rand(N // D, seed=64).to(DEV), rand(N, seed=65).to(DEV)
@@ -440,8 +440,8 @@ def test_products_of_experts_in_float32(T, E, top, N, K, wd):
 @pytest.mark.parametrize("M,N,K,col0,ld", [(1, 128, 32, 0, 32), (8, 2048, 128, 260, 400), (32, 48, 64, 4, 72), (7, 50, 96, 8, 104),
                                            (33, 64, 32, 0, 32), (5, 40, 24, 0, 24), (6, 32, 32, 3, 40)])
 def test_product_of_some_columns_with_a_short_k(M, N, K, col0, ld):
-    """Few rows of bfloat16 weights take a kernel of their own (k in steps of 32, rows on 16-byte borders);
-    more rows, another k or columns off those borders take the tiled one: both against the plain product."""
+    """Up to 16 rows (rows on 16-byte borders) take the kernel of a wave for every stretch of k; more rows, or columns off those
+    borders, others: all against the plain product."""
     a, w = rand(M, ld, seed=M), rand(N, K, seed=N, scale=0.3)
     for dtype, tol in ((torch.bfloat16, 2e-5), (torch.float32, 2e-5)):
         wd = w.to(dtype)
