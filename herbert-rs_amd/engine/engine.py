@@ -219,7 +219,8 @@ class Engine:
         # all pages of the step or none: a step that does not fit leaves the cache as it was
         self.cache.reserve_all([(e.slot, len(e.tokens)) for e in entries])
         # fixed-size state is changed in place by the parts: what the step's slots hold is set aside before parts run one after
-        # another, so that a step that fails leaves them as they were (a graph's replay begins as a whole or not at all; a sequence's
+        # another, so that a step that fails leaves them as they were (a graph's replay begins as a whole or not at all, and
+        # nothing that can fail follows it: the caller's copy has its memory before; a sequence's
         # first step found zeros; nothing for a cache without state)
         state_before = []
 
@@ -229,9 +230,10 @@ class Engine:
                 state_before.extend(self.cache.save_state(held) or ())
         try:
             if self.static_decode and all(len(e.tokens) == 1 and list(e.want) == [0] for e in entries):
+                own = torch.empty((len(entries), vocab), dtype=torch.float32, device=self.device) if keep_logits else None
                 logits = self._decode_step(entries, starts, tokens_on_device, set_aside)
                 if keep_logits:
-                    logits = logits.clone()
+                    logits = own.copy_(logits)
             else:
                 set_aside()
                 meta = batching.pack(entries, starts, self.device)

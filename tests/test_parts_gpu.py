@@ -7,6 +7,8 @@ import numpy as np
 import pytest
 import torch
 
+from torch.utils._python_dispatch import TorchDispatchMode
+
 from herbert_rs_amd.cache import Cache, KVNeed, StateNeed
 from herbert_rs_amd.engine import Engine, StepEntry
 from herbert_rs_amd.engine import batch as batching
@@ -601,6 +603,56 @@ def test_a_graph_safe_mixer_with_state_through_padded_and_replayed_decode_steps(
         whole = on_host.step([StepEntry(slot, t, list(range(lengths[i] - 1, len(t))))]).cpu()
         on_host.free_slot(slot)
         assert torch.allclose(got[i], whole, atol=1e-4)
+
+
+class NoMemoryFor(TorchDispatchMode):
+    """Whatever makes a tensor of `shape` finds no memory."""
+
+    def __init__(self, shape):
+        super().__init__()
+        self.shape = tuple(shape)
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        out = func(*args, **(kwargs or {}))
+        if isinstance(out, torch.Tensor) and tuple(out.shape) == self.shape and not any(
+                isinstance(a, torch.Tensor) and a.untyped_storage().data_ptr() == out.untyped_storage().data_ptr() for a in args):
+            raise torch.OutOfMemoryError("none left")
+        return out
+
+
+def test_a_replayed_step_without_memory_for_its_logits_leaves_the_state_as_it_was():
+    """Replays have no state set aside, so nothing may fail behind one: where the caller's copy of the logits finds no memory, lengths
+    and state are what they were, and the step run again gives what it gives on an engine that never lacked any."""
+    import dataclasses
+    from herbert_rs_amd.engine.model import Model
+    from herbert_rs_amd.weights import random_tensors
+    spec = toy_spec()
+    spec = dataclasses.replace(spec, layers=[dataclasses.replace(spec.layers[0], mixer=PartSpec("toy_decay_on_the_gpu", spec.layers[0].mixer.params)),
+                                             spec.layers[1]])
+    w = random_tensors(Model(spec).tensor_needs(), 3, "float32", std=0.15, norm_std=0.1)
+
+    def run(fails):
+        engine = Engine(None, spec, w, dtype="float32", max_tokens=64 * 4)
+        slots = [engine.alloc_slot() for _ in range(3)]
+        engine.step([StepEntry(s, [5 + s, 9, 33], [2]) for s in slots])
+        rows = []
+        for step in range(8):
+            entries = [StepEntry(s, [7 + step + s], [0]) for s in slots]
+            if fails and step in (4, 6):
+                assert engine.graphs_captured > 0
+                before = [g.data[:, slots].clone() for g in engine.cache.state_groups.values()]
+                captured = engine.graphs_captured
+                with pytest.raises(torch.OutOfMemoryError, match="none left"), NoMemoryFor((3, spec.vocab_size)):
+                    engine.step(entries)
+                assert engine.graphs_captured == captured
+                for g, b in zip(engine.cache.state_groups.values(), before):
+                    assert torch.equal(g.data[:, slots], b)
+                assert [engine.cache.length(s) for s in slots] == [3 + step] * 3
+                engine.cache.check()
+            rows.append(engine.step(entries).cpu())
+        return torch.stack(rows)
+
+    assert torch.equal(run(True), run(False))
 
 
 @register("mixer", "toy_counting_attention")
