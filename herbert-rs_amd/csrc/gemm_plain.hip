@@ -119,19 +119,20 @@ gemm_plain_tile_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
     if (tile / across >= (unsigned)(M + BM - 1) / BM) return;
     const int m0 = (int)(tile / across) * BM, n0 = (int)(tile % across) * BN;
     const int wm = wave % (BM / WM) * MB, wn = wave / (BM / WM) * NB;    // (in blocks)
-    // rows beyond M or N are the tile's first once more, whose sums go nowhere
+    // rows beyond M or N are the tile's first once more, whose sums go nowhere; rows lie as far apart as they may, but where 32 bits are known to do
+    typedef typename std::conditional<LOADS == WHOLE, unsigned, size_t>::type Offset;
     const TA* const a_tile = A + (size_t)m0 * lda;
     const TW* const w_tile = W + (size_t)n0 * ldw;
-    unsigned a_row[AU], w_row[WU];
+    Offset a_row[AU], w_row[WU];
 #pragma unroll
     for (int i = 0; i < AU; ++i) {
         const int row = 16 * ((EITHER ? wave % AB : wave * AU) + i) + r;
-        a_row[i] = (m0 + row < M ? row : 0) * (unsigned)lda + (LOADS == WHOLE ? 8 * q : 0);
+        a_row[i] = (m0 + row < M ? row : 0) * (Offset)lda + (LOADS == WHOLE ? 8 * q : 0);
     }
 #pragma unroll
     for (int i = 0; i < WU; ++i) {
         const int row = 16 * ((EITHER ? wave % WB : wave * WU) + i) + r;
-        w_row[i] = (n0 + row < N ? row : 0) * (unsigned)ldw + (LOADS == WHOLE ? 8 * q : 0);
+        w_row[i] = (n0 + row < N ? row : 0) * (Offset)ldw + (LOADS == WHOLE ? 8 * q : 0);
     }
     const bool stages_w = EITHER && wave >= AB;
     Oct<TA> a_next[AHEAD][AU];

@@ -170,6 +170,24 @@ def test_gemm_plain_splits_float32_without_loss(M, N, K, ad, wd):
     assert bool(((c.double() - want).abs()[fine] <= (units + 512) * 2.0 ** -24 * size[fine]).all())
 
 
+@pytest.mark.parametrize("K", [40, 37])
+@pytest.mark.parametrize("far", ["a", "w"])
+def test_gemm_plain_rows_that_lie_far_apart(K, far):
+    """The tiles' last row begins beyond 2^32 elements of the first one (8.9 GB of which its few columns are filled): the bits of the same
+    rows side by side."""
+    from herbert_rs_amd.kernels import lib
+    stride = 138547336
+    near = {"a": rand(32, K, seed=51).bfloat16(), "w": rand(32, K, seed=52).bfloat16()}
+    rows = torch.empty(31 * stride + K, dtype=torch.bfloat16, device=dev()).as_strided((32, K), (stride, 1))
+    rows.copy_(near[far])
+    got, want = torch.empty(32, 32, device=dev()), torch.empty(32, 32, device=dev())
+    for operands, c in ((near, want), (dict(near, **{far: rows}), got)):
+        lib.call("gemm_plain", "hb_gemm_plain", operands["a"].data_ptr(), 1, operands["w"].data_ptr(), 1, c.data_ptr(), 0, 32, 32, K,
+                 operands["a"].stride(0), operands["w"].stride(0), 32, 0, torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(got, want)
+    assert bool(((want.double() - near["a"].double() @ near["w"].double().T).abs() <= 1e-5 * K).all())
+
+
 @pytest.mark.parametrize("I", [5, 128, 1000])
 def test_swiglu(I):
     from herbert_rs_amd.kernels import ops
