@@ -63,20 +63,10 @@ __device__ __forceinline__ void store_quad(TC* C, int ldc, int m, int n, int N, 
     }
 }
 
-// A sum that is not finite is summed again in plain float32 (an infinity among the operands, or one that rounds to it): what
-// it then is, a chain of fmaf says. Elements n .. n + 3 of row m.
-template <class TA, class TW>
-__device__ __forceinline__ void mend_quad(const TA* A, const TW* W, int lda, int ldw, int m, int n, int N, int K, f32x4& sums) {
-    bool fine = true;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) fine = fine && fabsf(sums[e]) < INFINITY;
-    if (fine) return;
-#pragma unroll 1
-    for (int e = 0; e < 4 && n + e < N; ++e) {
-        const float sum = hb_sum_in_order(A + (size_t)m * lda, W + (size_t)(n + e) * ldw, K, K_BLOCK);
-        sums[0] = e == 0 ? sum : sums[0], sums[1] = e == 1 ? sum : sums[1];
-        sums[2] = e == 2 ? sum : sums[2], sums[3] = e == 3 ? sum : sums[3];
-    }
+// The rows of A from m0 on for mend_blocks.
+template <class TA>
+__device__ __forceinline__ auto rows_of(const TA* A, int lda, int m0, int M) {
+    return [=](int i) { return m0 + i < M ? A + (size_t)(m0 + i) * lda : nullptr; };
 }
 
 // blockIdx.z: one of a batch of products whose operands lie batch_* elements apart (either way: a pair's lie where they lie).
@@ -230,6 +220,7 @@ gemm_plain_tile_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
             }
     }
 
+    mend_blocks<TA, TW>(rows_of(A, lda, m0 + 16 * wm, M), W, ldw, n0 + 16 * wn, N, K, K_BLOCK, total);
 #pragma unroll
     for (int i = 0; i < MB; ++i) {
         const int m = m0 + 16 * (wm + i) + r;
@@ -237,7 +228,6 @@ gemm_plain_tile_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
 #pragma unroll
         for (int j = 0; j < NB; ++j) {
             const int n = n0 + 16 * (wn + j) + 4 * q;
-            mend_quad(A, W, lda, ldw, m, n, N, K, total[j][i]);
             store_quad<TC, ACCUM, LOADS != SINGLE>(C, ldc, m, n, N, total[j][i], ep);
         }
     }
@@ -295,6 +285,7 @@ gemm_plain_wave_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
                     for (int i = 0; i < MB; ++i) total[j][i] += sums[b][j][i][lane];
     }
     if (wave) return;
+    mend_blocks<TA, TW>(rows_of(A, lda, m0, M), W, ldw, n0, N, K, K_BLOCK, total);
 #pragma unroll
     for (int i = 0; i < MB; ++i) {
         const int m = m0 + 16 * i + r;
@@ -302,7 +293,6 @@ gemm_plain_wave_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
 #pragma unroll
         for (int j = 0; j < NB; ++j) {
             const int n = n0 + 16 * j + 4 * q;
-            mend_quad(A, W, lda, ldw, m, n, N, K, total[j][i]);
             store_quad<TC, ACCUM, true>(C, ldc, m, n, N, total[j][i], ep);
         }
     }
@@ -355,10 +345,9 @@ gemm_plain_stream_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC*
             top = low = f32x4{0.f, 0.f, 0.f, 0.f};
         }
     }
-    if (r < M) {
-        mend_quad(A, W, lda, ldw, r, n0 + 4 * q, N, K, total);
-        store_quad<TC, ACCUM, true>(C, ldc, r, n0 + 4 * q, N, total, ep);
-    }
+    f32x4 sums[1][1] = {{total}};
+    mend_blocks<TA, TW>(rows_of(A, lda, 0, M), W, ldw, n0, N, K, K_BLOCK, sums);
+    if (r < M) store_quad<TC, ACCUM, true>(C, ldc, r, n0 + 4 * q, N, sums[0][0], ep);
 }
 
 // The kernel of a product of more than 16 rows: the one with the least estimated time, in microseconds. A wave of 16 x 16 or 32 x 32

@@ -490,6 +490,7 @@ __device__ __forceinline__ void grouped_plain_rows(const TA* __restrict__ A, con
                     for (int i = 0; i < MB; ++i) total[j][i] += sums[((b * NB + j) * MB + i) * HB_WAVE + lane];
     }
     if (wave) return;
+    mend_blocks<TA, TW>([=](int i) { return from + i < rows ? A + (size_t)src[from + i] * K : nullptr; }, We, K, n0, N, K, SPLIT_STRETCH, total);
 #pragma unroll
     for (int i = 0; i < MB; ++i) {
         const int m = from + 16 * i + r;
@@ -499,10 +500,7 @@ __device__ __forceinline__ void grouped_plain_rows(const TA* __restrict__ A, con
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int n = n0 + 16 * j + 4 * q + e;
-                if (n >= N) continue;
-                float sum = total[j][i][e];
-                if (!(fabsf(sum) < INFINITY)) sum = hb_sum_in_order(A + (size_t)src[m] * K, We + (size_t)n * K, K, SPLIT_STRETCH);
-                C[(size_t)(row0 + m) * N + n] = sum;
+                if (n < N) C[(size_t)(row0 + m) * N + n] = total[j][i][e];
             }
     }
 }

@@ -170,6 +170,37 @@ def test_gemm_plain_splits_float32_without_loss(M, N, K, ad, wd):
     assert bool(((c.double() - want).abs()[fine] <= (units + 512) * 2.0 ** -24 * size[fine]).all())
 
 
+@pytest.mark.parametrize("M,N,K", [(8, 2048, 4096), (64, 2048, 2048), (512, 2048, 2048)])
+@pytest.mark.parametrize("wd", [torch.float32, torch.bfloat16])
+def test_gemm_plain_a_row_that_is_not_finite_holds_up_no_other(M, N, K, wd):
+    """A request of NaN, infinities or numbers that bfloat16 rounds to them leaves the other rows their bits and the step its time, but for
+    a multiple of one product's that is far from the 25 to 90 which an output a lane, an element at a time, took."""
+    from herbert_rs_amd.kernels import ops
+    a, w = rand(M, K, seed=61), rand(N, K, seed=62).to(wd)
+    c, clean = torch.empty(M, N, device=dev()), torch.empty(M, N, device=dev())
+
+    def took(out):
+        best = math.inf
+        for _ in range(5):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(10):
+                ops.gemm_plain(a, w, out)
+            end.record()
+            end.synchronize()
+            best = min(best, start.elapsed_time(end))
+        return best
+    usual = took(clean)
+    others = torch.arange(M, device=dev()) != M // 2
+    for what, where in ((math.nan, slice(None)), (math.inf, 5), (3.4e38, 5)):
+        a[M // 2] = 1.0
+        a[M // 2, where] = what
+        assert took(c) <= 22 * usual, what
+        assert torch.equal(c[others], clean[others])
+        want = (a[M // 2].double() @ w.double().T).float()
+        assert torch.equal(c[M // 2].isnan(), want.isnan()) and torch.equal(c[M // 2].isinf(), want.isinf())
+
+
 @pytest.mark.parametrize("K", [40, 37])
 @pytest.mark.parametrize("far", ["a", "w"])
 def test_gemm_plain_rows_that_lie_far_apart(K, far):

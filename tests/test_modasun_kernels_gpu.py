@@ -436,6 +436,30 @@ def test_products_of_experts_in_float32(T, E, top, N, K, wd):
         assert torch.equal(alone[i], c[order.index(p)])
 
 
+@pytest.mark.parametrize("T,E,N,K", [(5, 3, 70, 512), (60, 2, 36, 1544)])
+@pytest.mark.parametrize("wd", [torch.float32, torch.bfloat16])
+def test_products_of_experts_whose_rows_are_not_finite(T, E, N, K, wd):
+    """Tokens of NaN, of an infinity and of a number that bfloat16 rounds to one: what plain float32 has for them, the others' bits as without."""
+    a, w = rand(T, K, seed=43).to(DEV), rand(E, N, K, seed=44).to(wd).to(DEV)
+    routing = moe.Routing(torch.empty(moe.Routing.ints_needed(T, E, 2), dtype=torch.int32, device=DEV), torch.empty(T, 2, device=DEV), T, E, 2)
+    moe.route(rand(T, E, seed=41).to(DEV), rand(E, seed=42).to(DEV), routing)
+    order, chosen = routing.order.cpu().tolist(), routing.chosen.flatten().cpu().tolist()
+    clean, c = (torch.full((T * 2, N), math.nan, device=DEV) for _ in range(2))
+    moe.gemm_plain(a, w, clean, routing, gather=True)
+    a[0, 7], a[2, K - 1], a[3, 1] = math.nan, -math.inf, 3.4e38
+    moe.gemm_plain(a, w, c, routing, gather=True)
+    for i, p in enumerate(order):
+        if p // 2 not in (0, 2, 3):
+            assert torch.equal(c[i], clean[i])
+            continue
+        m, x = w[chosen[p]].double(), a[p // 2].double()
+        want = (m @ x).float()
+        fine = want.isfinite()
+        bound = (min(K, 512) + (K + 511) // 512) * 2.0 ** -24 * (m.abs() @ x.abs())
+        assert torch.equal(c[i].isnan(), want.isnan()) and torch.equal(c[i].isinf(), want.isinf()) and torch.equal(c[i][want.isinf()], want[want.isinf()])
+        assert bool(((c[i].double() - m @ x).abs()[fine] <= bound[fine]).all())
+
+
 # ---------------------------------------------------------------- the second product of a pair through a narrow middle
 @pytest.mark.parametrize("M,N,K,col0,ld", [(1, 128, 32, 0, 32), (8, 2048, 128, 260, 400), (32, 48, 64, 4, 72), (7, 50, 96, 8, 104),
                                            (33, 64, 32, 0, 32), (5, 40, 24, 0, 24), (6, 32, 32, 3, 40)])
