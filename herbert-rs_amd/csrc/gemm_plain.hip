@@ -80,9 +80,9 @@ __device__ __forceinline__ void to_product(const TA* __restrict__& A, const TW* 
     if (z < ep.from) ep.rate = nullptr;
 }
 
-// How a tile's operands are loaded: element by element; 16 bytes at a time; the same, K being whole stages (then a row is a 32-bit
-// offset from the tile's first and no lane looks where K ends).
-enum { SINGLE, QUADS, WHOLE };
+// How a tile's operands are loaded: element by element; vectors at a time, with bfloat16 8 or 16 bytes; 16 bytes at a time, K being whole stages (then a
+// row is a 32-bit offset from the tile's first and no lane looks where K ends).
+enum { SINGLE = OCT_SINGLE, HALVES = OCT_HALVES, QUADS = OCT_WHOLE, WHOLE };
 
 // More than 16 rows: a workgroup on a tile of BM rows of A by BN rows of W, a wave on WM x WN of it, in stages of 32 k. A stage
 // is asked for two stages ahead (a lane's eight elements, 32 bytes), split into its parts by the wave that asked and
@@ -130,15 +130,15 @@ gemm_plain_tile_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
     auto fetch = [&](int s, Oct<TA>* a, Oct<TW>* w) {
         const int k = s * STAGE, from = LOADS == WHOLE && k > K - STAGE ? K - STAGE : k;      // (a stage beyond K is the last once more)
         if constexpr (EITHER) {
-            a[0] = load_oct((stages_w ? w_tile : a_tile) + from, stages_w ? w_row[0] : a_row[0]);
+            a[0] = load_oct<QUADS>((stages_w ? w_tile : a_tile) + from, stages_w ? w_row[0] : a_row[0]);
             return;
         }
 #pragma unroll
         for (int i = 0; i < AU; ++i)
-            a[i] = LOADS == WHOLE ? load_oct(a_tile + from, a_row[i]) : load_oct<LOADS == QUADS>(a_tile + a_row[i], k + 8 * q, K);
+            a[i] = LOADS == WHOLE ? load_oct<QUADS>(a_tile + from, a_row[i]) : load_oct<LOADS == WHOLE ? QUADS : LOADS>(a_tile + a_row[i], k + 8 * q, K);
 #pragma unroll
         for (int i = 0; i < WU; ++i)
-            w[i] = LOADS == WHOLE ? load_oct(w_tile + from, w_row[i]) : load_oct<LOADS == QUADS>(w_tile + w_row[i], k + 8 * q, K);
+            w[i] = LOADS == WHOLE ? load_oct<QUADS>(w_tile + from, w_row[i]) : load_oct<LOADS == WHOLE ? QUADS : LOADS>(w_tile + w_row[i], k + 8 * q, K);
     };
     auto cut = [&](int s, Oct<TA>* a, Oct<TW>* w) {          // what lies beyond K
         const int left = K - s * STAGE;
@@ -241,7 +241,7 @@ gemm_plain_tile_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
 // and 8 rows, which they had, took at 1 | 8 | 24 rows of bfloat16 weights (2048 x 128) 3.1 | 3.5 | 3.8 us, now 2.6 | 2.6 | 2.6; (4096 x 1024)
 // 14.5 | 16.7 | 19.3, now 5.2 | 5.4 | 7.4; (16 heads of 128 x 512) 7.5 | 8.8 | 9.8, now 3.8 | 4.1 | 4.5.
 #define WAVE_WAVES 8
-template <class TA, class TW, class TC, bool ACCUM, int MB, int NB, int AHEAD>
+template <class TA, class TW, class TC, bool ACCUM, int MB, int NB, int AHEAD, int HOW>
 __global__ void __launch_bounds__(WAVE_WAVES * HB_WAVE, AHEAD == 8 ? 4 : 2)
 gemm_plain_wave_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* __restrict__ C, int M, int N,
                        int K, int lda, int ldw, int ldc, ptrdiff_t batch_a, ptrdiff_t batch_w, ptrdiff_t batch_c,
@@ -270,7 +270,7 @@ gemm_plain_wave_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
         for (int j = 0; j < NB; ++j)
 #pragma unroll
             for (int i = 0; i < MB; ++i) top[j][i] = low[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-        sum_stretch<AHEAD, A_AHEAD>(w_row, a_row, k0, K, q, top, low);
+        sum_stretch<AHEAD, A_AHEAD, HOW>(w_row, a_row, k0, K, q, top, low);
         if (first) __syncthreads();                  // (the round before has been read)
 #pragma unroll
         for (int j = 0; j < NB; ++j)
@@ -320,8 +320,8 @@ gemm_plain_stream_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC*
     auto fetch = [&](int k0) {
 #pragma unroll
         for (int d = 0; d < WAVE_DEPTH; ++d) {
-            w_next[d] = load_oct<true>(w_row, k0 + 32 * d + 8 * q, K);
-            a_next[d] = load_oct<true>(a_row, k0 + 32 * d + 8 * q, K);
+            w_next[d] = load_oct<QUADS>(w_row, k0 + 32 * d + 8 * q, K);
+            a_next[d] = load_oct<QUADS>(a_row, k0 + 32 * d + 8 * q, K);
         }
     };
     fetch(0);
@@ -359,7 +359,7 @@ gemm_plain_stream_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC*
 // 37 / 78 [54], 563 x 4096 x 2048 262 / 139 / 137 / 94 / 80 [114], 563 x 6144 x 2048 388 / 207 / 210 / 126 / 93 [155], 563 x 2048 x 3072 232 / 133 / 113 / 89 / 116 [98];
 // bfloat16 weights: 64 x 2048 x 2048 13 / 16 / 19 / 25 / 49 [39], 563 x 4096 x 2048 191 / 105 / 110 / 69 / 52 [163].
 // whole: K is whole stages, the larger tiles take nothing else; a decay's exponentials and logarithms are a tile's own tail: not 64 of them a lane.
-enum { STREAM, WAVE, WAVE_RING, WAVE_SQUARE, TILE_SINGLE, TILE_QUADS, TILE_32, TILE_64, TILE_128 };
+enum { STREAM, WAVE, WAVE_RING, WAVE_SQUARE, WAVE_HALVES, TILE_SINGLE, TILE_HALVES, TILE_QUADS, TILE_32, TILE_64, TILE_128 };
 static int gemm_plain_choice(int M, int N, int K, int batch, bool both, bool whole, bool decay) {
     auto tiles = [&](int side) { return (double)((N + side - 1ll) / side * ((M + side - 1) / side) * batch); };
     auto most = [&](int side) { return (double)(((long long)tiles(side) + 255) / 256); };
@@ -390,11 +390,14 @@ static int gemm_plain_choice(int M, int N, int K, int batch, bool both, bool who
 template <class TA, class TW, class TC, bool ACCUM>
 static void launch_as(const TA* A, const TW* W, TC* C, int M, int N, int K, int lda, int ldw, int ldc,
                       hipStream_t stream, int batch, ptrdiff_t batch_a, ptrdiff_t batch_w, ptrdiff_t batch_c, DecayEpilogue ep) {
-    // (16-byte loads and stores where rows and strides allow them)
-    constexpr int EA = 16 / sizeof(TA), EW = 16 / sizeof(TW);
-    const bool vec = K % EA == 0 && K % EW == 0 && lda % EA == 0 && ldw % EW == 0 && batch_a % EA == 0 && batch_w % EW == 0 &&
-                     (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0 &&
-                     (sizeof(TC) != 4 || (N % 4 == 0 && ldc % 4 == 0 && batch_c % 4 == 0 && (uintptr_t)C % 16 == 0));
+    // (16-byte loads where rows and strides allow them, or 8-byte ones of bfloat16, 16-byte stores with either: bfloat16 rows 2,052 elements apart, 8 x
+    // 2048 x 2048 7.3 us, 512 rows 39, element by element 42 and 144)
+    auto borders = [&](int ea, int ew) {
+        return K % ea == 0 && K % ew == 0 && lda % ea == 0 && ldw % ew == 0 && batch_a % ea == 0 && batch_w % ew == 0 &&
+               (uintptr_t)A % (ea * sizeof(TA)) == 0 && (uintptr_t)W % (ew * sizeof(TW)) == 0 &&
+               (sizeof(TC) != 4 || (N % 4 == 0 && ldc % 4 == 0 && batch_c % 4 == 0 && (uintptr_t)C % 16 == 0));
+    };
+    const bool vec = borders(16 / sizeof(TA), 16 / sizeof(TW)), half = !vec && borders(4, 4);
     auto tiles = [&](int high, int wide) { return (long long)((N + wide - 1) / wide) * ((M + high - 1) / high) * batch; };
     // (a grid's x holds fewer than 2^32 threads: beyond GRID_X tiles the rest lie along its y)
     auto grid = [&](int high, int wide) {
@@ -406,14 +409,15 @@ static void launch_as(const TA* A, const TW* W, TC* C, int M, int N, int K, int 
     gemm_plain_tile_kernel<TA, TW, TC, ACCUM, BM, BN, WM, WN, LOADS>                                                  \
         <<<grid(BM, BN), 64 * (BM / WM) * (BN / WN), 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, batch_a, batch_w,  \
                                                                  batch_c, ep)
-#define HB_PLAIN_WAVE(MB, NB, AHEAD)                                                                                  \
-    gemm_plain_wave_kernel<TA, TW, TC, ACCUM, MB, NB, AHEAD>                                                          \
+#define HB_PLAIN_WAVE(MB, NB, AHEAD, HOW)                                                                             \
+    gemm_plain_wave_kernel<TA, TW, TC, ACCUM, MB, NB, AHEAD, HOW>                                                     \
         <<<dim3((N + 16 * NB - 1) / (16 * NB), (M + 16 * MB - 1) / (16 * MB), batch), HB_WAVE * at_once, 0, stream>>>( \
             A, W, C, M, N, K, lda, ldw, ldc, batch_a, batch_w, batch_c, ep)
     // (both sides of the first two lines stand at the kernels)
     const long long strips = (N + 15ll) / 16 * batch;
     const int at_once = stretches < WAVE_WAVES ? stretches : WAVE_WAVES;
-    const int which = !vec                                                      ? TILE_SINGLE
+    const int which = half                                                      ? M <= 16 ? WAVE_HALVES : TILE_HALVES
+                      : !vec                                                    ? TILE_SINGLE
                       : M <= 16 && sizeof(TW) == 4 && K < 1024 && K > 64 && K % K_BLOCK ? STREAM
                       : M <= 16                                                 ? strips * at_once > 2048 ? WAVE_RING : WAVE
                                                                                 : gemm_plain_choice(M, N, K, batch, Parts<TA>::COUNT + Parts<TW>::COUNT == 6,
@@ -424,9 +428,16 @@ static void launch_as(const TA* A, const TW* W, TC* C, int M, int N, int K, int 
                 gemm_plain_stream_kernel<TA, TW, TC, ACCUM><<<dim3((N + 15) / 16, 1, batch), HB_WAVE, 0, stream>>>(
                     A, W, C, M, N, K, lda, ldw, ldc, batch_a, batch_w, batch_c, ep);
             break;
-        case WAVE: HB_PLAIN_WAVE(1, 1, 16); break;
-        case WAVE_RING: HB_PLAIN_WAVE(1, 1, 8); break;
-        case WAVE_SQUARE: HB_PLAIN_WAVE(2, 2, 4); break;
+        case WAVE: HB_PLAIN_WAVE(1, 1, 16, QUADS); break;
+        case WAVE_RING: HB_PLAIN_WAVE(1, 1, 8, QUADS); break;
+        case WAVE_SQUARE: HB_PLAIN_WAVE(2, 2, 4, QUADS); break;
+        // (both sides float32: the borders of 8 bytes of bfloat16 are theirs of 16, and none of these two is asked for)
+        case WAVE_HALVES:
+            if constexpr (sizeof(TA) == 2 || sizeof(TW) == 2) HB_PLAIN_WAVE(1, 1, 16, HALVES);
+            break;
+        case TILE_HALVES:
+            if constexpr (sizeof(TA) == 2 || sizeof(TW) == 2) HB_PLAIN_TILE(32, 32, 16, 32, HALVES);
+            break;
         case TILE_SINGLE: HB_PLAIN_TILE(32, 32, 16, 32, SINGLE); break;
         case TILE_QUADS: HB_PLAIN_TILE(32, 32, 16, 32, QUADS); break;
         case TILE_32:            // (a wave stages a block of either operand, where both are of a kind: half the splitting in a stage's chain)

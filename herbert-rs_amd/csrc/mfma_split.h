@@ -28,29 +28,39 @@ template <class T> struct Parts {
     bf16x8 part[COUNT];
 };
 
-// The eight of `row` from k on. VEC: 16-byte loads (the row aligned to 16 bytes, K a multiple of what one holds); what lies at
-// or beyond K is something of the row's: `ends` makes zeros of it. No branch hangs on k, so that no load is waited for where
-// the paths of one would meet. Otherwise: element by element, zeros from K on.
-template <bool VEC>
+// How eight elements are loaded: element by element; float32 16 and bfloat16 8 bytes at a time (rows on such borders, K a multiple of 4); either
+// 16 bytes at a time (K a multiple of 8 where bfloat16 is concerned).
+enum { OCT_SINGLE, OCT_HALVES, OCT_WHOLE };
+// The eight of `row` from k on. Of vector loads, what lies at or beyond K is something of the row's: `ends` makes zeros of it. No branch hangs on
+// k, so that no load is waited for where the paths of one would meet. Element by element: zeros from K on.
+template <int HOW>
 __device__ __forceinline__ Oct<float> load_oct(const float* row, int k, int K) {
-    if (VEC) return Oct<float>{{*(const f32x4*)(row + (k < K ? k : 0)), *(const f32x4*)(row + (k + 4 < K ? k + 4 : 0))}};
+    if (HOW != OCT_SINGLE) return Oct<float>{{*(const f32x4*)(row + (k < K ? k : 0)), *(const f32x4*)(row + (k + 4 < K ? k + 4 : 0))}};
     return Oct<float>{{load_quad<false>(row + k, K - k), load_quad<false>(row + k + 4, K - k - 4)}};
 }
-template <bool VEC>
+__device__ __forceinline__ Oct<bf16> two_halves(const bf16* first, const bf16* second) {
+    const uint2 halves[2] = {*(const uint2*)first, *(const uint2*)second};
+    return __builtin_bit_cast(Oct<bf16>, halves);
+}
+template <int HOW>
 __device__ __forceinline__ Oct<bf16> load_oct(const bf16* row, int k, int K) {
-    if (VEC) return Oct<bf16>{*(const bf16x8*)(row + (k < K ? k : 0))};
+    if (HOW == OCT_WHOLE) return Oct<bf16>{*(const bf16x8*)(row + (k < K ? k : 0))};
+    if (HOW == OCT_HALVES) return two_halves(row + (k < K ? k : 0), row + (k + 4 < K ? k + 4 : 0));
     Oct<bf16> r;
 #pragma unroll
     for (int i = 0; i < 8; ++i) r.all[i] = k + i < K ? __builtin_bit_cast(__bf16, row[k + i].bits) : (__bf16)0.f;
     return r;
 }
 // The eight at `offset` elements from a place that is the same for all lanes.
+template <int HOW>
 __device__ __forceinline__ Oct<float> load_oct(const float* place, unsigned offset) {
     const char* at = (const char*)place + offset * 4u;
     return Oct<float>{{*(const f32x4*)at, *(const f32x4*)(at + 16)}};
 }
+template <int HOW>
 __device__ __forceinline__ Oct<bf16> load_oct(const bf16* place, unsigned offset) {
-    return Oct<bf16>{*(const bf16x8*)((const char*)place + offset * 2u)};
+    const bf16* at = (const bf16*)((const char*)place + offset * 2u);
+    return HOW == OCT_WHOLE ? Oct<bf16>{*(const bf16x8*)at} : two_halves(at, at + 4);
 }
 __device__ __forceinline__ void ends(Oct<float>& o, int left) {
 #pragma unroll
@@ -222,8 +232,8 @@ __device__ __forceinline__ void mend_blocks(Rows row_of, const TW* W, size_t ldw
 #define WAVE_DEPTH 4
 
 // A wave's sums over the stretch of k that starts at k0, for NB blocks of 16 rows of W and MB of A (w_row, a_row: the lane's own rows,
-// 16 bytes at a time; q = lane / 16). AHEAD pieces of 32 k of W and A_AHEAD of A are in flight.
-template <int AHEAD, int A_AHEAD, class TW, class TA, int NB, int MB>
+// vectors at a time, HOW; q = lane / 16). AHEAD pieces of 32 k of W and A_AHEAD of A are in flight.
+template <int AHEAD, int A_AHEAD, int HOW = OCT_WHOLE, class TW, class TA, int NB, int MB>
 __device__ __forceinline__ void sum_stretch(const TW* const (&w_row)[NB], const TA* const (&a_row)[MB], int k0, int K, int q,
                                             f32x4 (&top)[NB][MB], f32x4 (&low)[NB][MB]) {
     constexpr int UNITS = SPLIT_STRETCH / 32;
@@ -232,11 +242,11 @@ __device__ __forceinline__ void sum_stretch(const TW* const (&w_row)[NB], const 
         Oct<TA> a[A_AHEAD][MB];
         auto fetch_w = [&](int u) {
 #pragma unroll
-            for (int j = 0; j < NB; ++j) w[u % AHEAD][j] = load_oct(w_row[j] + k0 + 32 * u, 8u * q);
+            for (int j = 0; j < NB; ++j) w[u % AHEAD][j] = load_oct<HOW>(w_row[j] + k0 + 32 * u, 8u * q);
         };
         auto fetch_a = [&](int u) {
 #pragma unroll
-            for (int i = 0; i < MB; ++i) a[u % A_AHEAD][i] = load_oct(a_row[i] + k0 + 32 * u, 8u * q);
+            for (int i = 0; i < MB; ++i) a[u % A_AHEAD][i] = load_oct<HOW>(a_row[i] + k0 + 32 * u, 8u * q);
         };
 #pragma unroll
         for (int u = 0; u < A_AHEAD; ++u) fetch_a(u);
@@ -265,9 +275,9 @@ __device__ __forceinline__ void sum_stretch(const TW* const (&w_row)[NB], const 
 #pragma unroll
         for (int d = 0; d < WAVE_DEPTH; ++d) {
 #pragma unroll
-            for (int j = 0; j < NB; ++j) w[d][j] = load_oct<true>(w_row[j], k + 32 * d + 8 * q, K);
+            for (int j = 0; j < NB; ++j) w[d][j] = load_oct<HOW>(w_row[j], k + 32 * d + 8 * q, K);
 #pragma unroll
-            for (int i = 0; i < MB; ++i) a[d][i] = load_oct<true>(a_row[i], k + 32 * d + 8 * q, K);
+            for (int i = 0; i < MB; ++i) a[d][i] = load_oct<HOW>(a_row[i], k + 32 * d + 8 * q, K);
         }
 #pragma unroll
         for (int d = 0; d < WAVE_DEPTH; ++d) {

@@ -170,6 +170,33 @@ def test_gemm_plain_splits_float32_without_loss(M, N, K, ad, wd):
     assert bool(((c.double() - want).abs()[fine] <= (units + 512) * 2.0 ** -24 * size[fine]).all())
 
 
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 100])
+@pytest.mark.parametrize("K,step,start", [(4, 4, 0), (12, 16, 4), (44, 48, 4), (512, 516, 0), (1024, 1028, 4), (1500, 1500, 0), (4612, 4616, 4)])
+@pytest.mark.parametrize("ad,wd", [(torch.float32, torch.bfloat16), (torch.bfloat16, torch.float32), (torch.bfloat16, torch.bfloat16)])
+def test_gemm_plain_rows_of_bfloat16_on_8_byte_borders(M, K, step, start, ad, wd):
+    """Rows `step` elements apart from element `start` on, on 8-byte borders and not on 16-byte ones (bfloat16), for few rows and many: the bits of the same
+    rows on 16-byte borders, whole eights of k with zeros behind K."""
+    from herbert_rs_amd.kernels import lib
+    N = 68
+
+    def product(rows, ops):
+        c = torch.full((M, N), math.nan, device=dev())
+        lib.call("gemm_plain", "hb_gemm_plain", ops[0].data_ptr(), int(ad == torch.bfloat16), ops[1].data_ptr(), int(wd == torch.bfloat16), c.data_ptr(), 0,
+                 M, N, rows, ops[0].stride(0), ops[1].stride(0), N, 0, torch.cuda.current_stream().cuda_stream)
+        return c
+    halves, wholes = [], []
+    for count, dtype, seed in ((M, ad, 71), (N, wd, 72)):
+        rows = rand(count, K, seed=seed).to(dtype)
+        at = torch.full((count * step + start,), math.nan, dtype=dtype, device=dev())[start:].view(count, step)[:, :K]
+        whole = torch.zeros(count, (K + 7) // 8 * 8, dtype=dtype, device=dev())
+        at.copy_(rows), whole[:, :K].copy_(rows)
+        halves.append(at), wholes.append(whole)
+    got = product(K, halves)
+    assert torch.equal(got, product(wholes[0].shape[1], wholes))
+    want, size = (halves[0].double() @ halves[1].double().T), (halves[0].double().abs() @ halves[1].double().abs().T)
+    assert bool(((got.double() - want).abs() <= (min(K, 512) + K // 512 + 1) * 2.0 ** -24 * size).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(8, 2048, 4096), (64, 2048, 2048), (512, 2048, 2048)])
 @pytest.mark.parametrize("wd", [torch.float32, torch.bfloat16])
 def test_gemm_plain_a_row_that_is_not_finite_holds_up_no_other(M, N, K, wd):
