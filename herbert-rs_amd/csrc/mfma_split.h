@@ -149,9 +149,10 @@ __device__ __forceinline__ bool hb_wild(f32x4 v) { return hb_wild(v[0]) || hb_wi
 // Sums of a 16 x 16 block that are not finite, as plain float32 has them; all of a wave calls this. row_of(i): the block's i-th row of A, null
 // beyond the last; W: its first row, `columns` of them. A row of A with a NaN is NaN throughout. In others what is not finite
 // among the operands says what the sum is, whatever its order, and only sums of finite numbers (parts or sums beyond the range) are
-// summed again in their order. A wave looks at 64 elements of a row at a time. A product of 8 rows with 2048 x 2048 float32 weights, 11.3 us, takes 12.6
-// where a row is NaN, 42 where one holds an infinity and 90 where one holds 3.4e38 (an output a lane, an element at a time: 504); of
-// 512 rows, 4096 x 4096, 143, 155, 270 and 466 us (2,322).
+// summed again in their order. A wave looks at 64 elements of a row at a time. A product of 8 rows with 2048 x 2048 float32 weights, 10.7 us, takes 12.4
+// where a row is NaN, 52 where one holds an infinity and 93 where one holds 3.4e38 (an output a lane, an element at a time: 504); of
+// 512 rows, 4096 x 4096, 139, 150, 354 and 536 us (2,322). (Sixteen columns at a time: 42 and 270 us with an infinity, but registers that cost
+// the tiles of 64 x 64 one of two workgroups a CU.)
 template <class TA, class TW, class Rows>
 __device__ __forceinline__ void mend_block(Rows row_of, const TW* W, size_t ldw, int columns, int K, int block, f32x4& sums) {
     const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
@@ -171,18 +172,25 @@ __device__ __forceinline__ void mend_block(Rows row_of, const TW* W, size_t ldw,
         float value = NAN;
         if (!__any(none)) {
             unsigned nan_or_up = 0, down = 0;                // a bit a column; +infinity in the upper half
-            for (int k = lane; k < K; k += HB_WAVE) {
-                const float y = hb_to_float(a[k]);
-                float x[16];
+#pragma unroll 1
+            for (int n0 = 0; n0 < 16; n0 += 4) {             // (four columns at a time: the tiles' registers are not to grow for this)
+                const TW* w[4];
 #pragma unroll
-                for (int n = 0; n < 16; ++n) x[n] = hb_to_float(W[(n < columns ? n : 0) * ldw + k]);
+                for (int n = 0; n < 4; ++n) w[n] = W + (n0 + n < columns ? n0 + n : 0) * ldw;
+#pragma unroll 2
+                for (int k = lane; k < K; k += HB_WAVE) {
+                    const float y = hb_to_float(a[k]);
+                    float x[4];
 #pragma unroll
-                for (int n = 0; n < 16; ++n)
-                    if (hb_wild(x[n]) || hb_wild(y)) {
-                        const float p = x[n] * y;
-                        nan_or_up |= p != p ? 1u << n : p > 0.f ? 0x10000u << n : 0u;
-                        down |= p < 0.f ? 1u << n : 0u;
-                    }
+                    for (int n = 0; n < 4; ++n) x[n] = hb_to_float(w[n][k]);
+#pragma unroll
+                    for (int n = 0; n < 4; ++n)
+                        if (hb_wild(x[n]) || hb_wild(y)) {
+                            const float p = x[n] * y;
+                            nan_or_up |= (p != p ? 1u : p > 0.f ? 0x10000u : 0u) << (n0 + n);
+                            down |= (p < 0.f ? 1u : 0u) << (n0 + n);
+                        }
+                }
             }
 #pragma unroll
             for (int off = 1; off < HB_WAVE; off <<= 1) nan_or_up |= __shfl_xor(nan_or_up, off, HB_WAVE), down |= __shfl_xor(down, off, HB_WAVE);
