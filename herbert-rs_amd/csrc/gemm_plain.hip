@@ -228,6 +228,11 @@ gemm_plain_tile_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
 #pragma unroll
         for (int j = 0; j < NB; ++j) {
             const int n = n0 + 16 * (wn + j) + 4 * q;
+            // (one to three products: a chain's roundings are no more than those of the parts' products that are left out)
+            if (LOADS == SINGLE && K < 4)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (n + e < N) total[j][i][e] = hb_sum_in_order(A + (size_t)m * lda, W + (size_t)(n + e) * ldw, K, K_BLOCK);
             store_quad<TC, ACCUM, LOADS != SINGLE>(C, ldc, m, n, N, total[j][i], ep);
         }
     }

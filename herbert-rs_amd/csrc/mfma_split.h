@@ -4,10 +4,10 @@
 // 16 x 16 x 32 costs six instructions of 16 cycles where the float32 matrix instructions need eight of 32, three
 // where one side is stored in bfloat16. The leading parts' products and the five smaller ones have a sum each: the matrix cores round a
 // sum once in 32 k, and the smaller sums' roundings weigh next to nothing. Over normal, positive and very uneven operands and K from
-// 32 to 12288 the error against 64 bits is 0.32 to 0.94 of that of a chain of fmaf in the same stretches (all six in one sum: 0.36 to 0.92, with a drift
+// 32 to 12288 the error against 64 bits is 0.32 to 0.94 of that of a chain of fmaf in the same stretches, normal operands and K = 4 0.68, 16 0.44 (all six in one sum: 0.36 to 0.92, with a drift
 // towards -infinity that the matrix cores' own adding brings and the short sums here do not show).
-// What is not finite spoils its parts (infinity minus infinity), as does what rounds to infinity: callers take a sum that is
-// not finite from `mend_blocks` instead. Numbers below 2^-110 lose the bits that bfloat16 cannot hold (below 2^-133).
+// What is not finite spoils its parts (infinity minus infinity), as does what lies beyond 2^112 or sums beyond 2^96: callers take a sum that is
+// not finite from `mend_blocks` instead.
 #pragma once
 #include "mfma_f32.h"
 
@@ -71,6 +71,10 @@ __device__ __forceinline__ void ends(Oct<bf16>& o, int left) {
     for (int i = 0; i < 8; ++i) o.all[i] = i < left ? o.all[i] : (__bf16)0.f;
 }
 
+// A float32 number's parts are those of 2^16 times it: what it has below 2^-133, where bfloat16 ends, is not lost then, down to float32's own last
+// bit. (Operands of 1e-38 and 10: an error of 2.7e-3 without, 1.3e-7 so. It costs a product of few rows a tenth, float32 weights, 2 x 2048 x 2048 9.2 ->
+// 10.0 us, a tile 0 to 2 %.)
+#define SPLIT_SCALE 65536.f
 // Each rest, v - (float)part, is exact and one instruction: a product of two pairs and a sum, with -1 and 0. (The pair -1, 0 is hidden
 // from the compiler, which would write the float -1, whose halves are 0, -1, in its place.)
 __device__ __forceinline__ void split_pair(float v0, float v1, bf16x2& top, bf16x2& mid, bf16x2& low) {
@@ -88,7 +92,7 @@ __device__ __forceinline__ Parts<float> split(const Oct<float>& o) {
 #pragma unroll
     for (int i = 0; i < 8; i += 2) {
         bf16x2 top, mid, low;
-        split_pair(o.quad[i / 4][i % 4], o.quad[i / 4][i % 4 + 1], top, mid, low);
+        split_pair(o.quad[i / 4][i % 4] * SPLIT_SCALE, o.quad[i / 4][i % 4 + 1] * SPLIT_SCALE, top, mid, low);
         r.part[0][i] = top[0], r.part[0][i + 1] = top[1];
         r.part[1][i] = mid[0], r.part[1][i + 1] = mid[1];
         r.part[2][i] = low[0], r.part[2][i + 1] = low[1];
@@ -96,6 +100,12 @@ __device__ __forceinline__ Parts<float> split(const Oct<float>& o) {
     return r;
 }
 __device__ __forceinline__ Parts<bf16> split(const Oct<bf16>& o) { return Parts<bf16>{{o.all}}; }
+
+// What sums of products of such parts are multiplied by, in the end.
+template <class TW, class TA>
+__device__ __forceinline__ constexpr float split_unit() {
+    return (Parts<TW>::COUNT == 3 ? 1.f / SPLIT_SCALE : 1.f) * (Parts<TA>::COUNT == 3 ? 1.f / SPLIT_SCALE : 1.f);
+}
 
 // Which parts meet, the smallest products first; the last one has the sum `top`, the others `low`.
 #define SPLIT_PRODUCTS 6
@@ -209,14 +219,14 @@ __device__ __forceinline__ void mend_block(Rows row_of, const TW* W, size_t ldw,
     }
 }
 
-// All of a wave's blocks: W's row n0 + 16 j is the first of the blocks [j][..], row_of(16 i) that of the blocks [..][i].
+// The sums of parts' products as the operands' own, all of a wave's blocks: W's row n0 + 16 j is the first of the blocks [j][..], row_of(16 i) that of the blocks [..][i].
 template <class TA, class TW, int NB, int MB, class Rows>
 __device__ __forceinline__ void mend_blocks(Rows row_of, const TW* W, size_t ldw, int n0, int N, int K, int block, f32x4 (&sums)[NB][MB]) {
     bool wild = false;
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll
-        for (int i = 0; i < MB; ++i) wild |= hb_wild(sums[j][i]);
+        for (int i = 0; i < MB; ++i) wild |= hb_wild(sums[j][i]), sums[j][i] *= split_unit<TW, TA>();
     if (!__any(wild)) return;
 #pragma unroll 1
     for (int b = 0; b < NB * MB; ++b) {                      // (one copy of the code: the block is picked out and put back)

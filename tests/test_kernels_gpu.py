@@ -197,6 +197,34 @@ def test_gemm_plain_rows_of_bfloat16_on_8_byte_borders(M, K, step, start, ad, wd
     assert bool(((got.double() - want).abs() <= (min(K, 512) + K // 512 + 1) * 2.0 ** -24 * size).all())
 
 
+@pytest.mark.parametrize("M,N,K", [(4, 100, 512), (16, 96, 992), (33, 100, 544), (64, 2050, 2048), (130, 516, 512), (700, 2052, 1056)])
+@pytest.mark.parametrize("ad,wd,a_size,w_size", [(torch.float32, torch.float32, 1e-36, 1e36), (torch.float32, torch.float32, 1e33, 1e-38),
+                                                 (torch.float32, torch.float32, 1e-41, 1e32), (torch.float32, torch.float32, 1e-38, 10.0),
+                                                 (torch.float32, torch.bfloat16, 1e-38, 1e20), (torch.bfloat16, torch.float32, 1e25, 1e-39)])
+def test_gemm_plain_keeps_the_last_bits_of_small_numbers(M, N, K, ad, wd, a_size, w_size):
+    """As test_gemm_plain_splits_float32_without_loss, for operands down to float32's last bit (2^-149) and whatever makes up for them; a sum is
+    rounded to 2^-149 once more where it is that small."""
+    from herbert_rs_amd.kernels import ops
+    a, w = (rand(M, K, seed=31).double() * a_size).to(ad), (rand(N, K, seed=33).double() * w_size).to(wd)
+    c = torch.empty(M, N, device=dev())
+    ops.gemm_plain(a, w, c)
+    want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    units = 2 * min((K + 31) // 32, 16) + (K + 511) // 512 + 4
+    assert bool(((c.double() - want).abs() <= units * 2.0 ** -24 * size + 2.0 ** -149).all())
+
+
+@pytest.mark.parametrize("K", [1, 2, 3])
+def test_gemm_plain_rounds_a_few_products_as_a_chain_does(K):
+    from herbert_rs_amd.kernels import ops
+    a, w = rand(33, K, seed=81), rand(40, K, seed=82)
+    c = torch.empty(33, 40, device=dev())
+    ops.gemm_plain(a, w, c)
+    want = torch.zeros(33, 40, dtype=torch.float64, device=dev())
+    for k in range(K):                                      # (a product is exact in 64 bits; two roundings of a sum hardly ever differ from one)
+        want = (want + a[:, k:k + 1].double() * w[:, k].double()).float().double()
+    assert torch.equal(c, want.float())
+
+
 @pytest.mark.parametrize("M,N,K", [(8, 2048, 4096), (64, 2048, 2048), (512, 2048, 2048)])
 @pytest.mark.parametrize("wd", [torch.float32, torch.bfloat16])
 def test_gemm_plain_a_row_that_is_not_finite_holds_up_no_other(M, N, K, wd):
