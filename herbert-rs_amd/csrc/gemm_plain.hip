@@ -363,9 +363,9 @@ gemm_plain_stream_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC*
 // 2048 x 2048 11 / 21 / 21 / 32 / 76 [22], 17 x 4096 x 2048 17 / 28 / 21 / 32 / 77 [29], 128 x 2048 x 2048 33 / 21 / 21 / 33 / 78 [23], 200 x 4096 x 2048 97 / 60 / 60 /
 // 37 / 78 [54], 563 x 4096 x 2048 262 / 139 / 137 / 94 / 80 [114], 563 x 6144 x 2048 388 / 207 / 210 / 126 / 93 [155], 563 x 2048 x 3072 232 / 133 / 113 / 89 / 116 [98];
 // bfloat16 weights: 64 x 2048 x 2048 13 / 16 / 19 / 25 / 49 [39], 563 x 4096 x 2048 191 / 105 / 110 / 69 / 52 [163].
-// whole: K is whole stages, the larger tiles take nothing else; a decay's exponentials and logarithms are a tile's own tail: not 64 of them a lane.
+// waves: a grid of them holds the product; whole: K is whole stages, the larger tiles take nothing else; a decay's exponentials and logarithms are a tile's own tail: not 64 of them a lane.
 enum { STREAM, WAVE, WAVE_RING, WAVE_SQUARE, WAVE_HALVES, TILE_SINGLE, TILE_HALVES, TILE_QUADS, TILE_32, TILE_64, TILE_128 };
-static int gemm_plain_choice(int M, int N, int K, int batch, bool both, bool whole, bool decay) {
+static int gemm_plain_choice(int M, int N, int K, int batch, bool both, bool whole, bool decay, bool waves) {
     auto tiles = [&](int side) { return (double)((N + side - 1ll) / side * ((M + side - 1) / side) * batch); };
     auto most = [&](int side) { return (double)(((long long)tiles(side) + 255) / 256); };
     auto larger = [](double a, double b) { return a > b ? a : b; };
@@ -375,8 +375,8 @@ static int gemm_plain_choice(int M, int N, int K, int batch, bool both, bool who
         int kernel;
         double cost;
     } all[5] = {
-        {WAVE, M > 4096 ? never : 2.6 + (both ? 8.0 : 5.3) * larger(per_simd * tiles(16), least)},
-        {WAVE_SQUARE, M > 4096 ? never : both ? 5.0 + larger(16.2 * per_simd * tiles(32), 12.0 * part) : 3.5 + larger(11.5 * per_simd * tiles(32), 10.0 * part)},
+        {WAVE, !waves ? never : 2.6 + (both ? 8.0 : 5.3) * larger(per_simd * tiles(16), least)},
+        {WAVE_SQUARE, !waves ? never : both ? 5.0 + larger(16.2 * per_simd * tiles(32), 12.0 * part) : 3.5 + larger(11.5 * per_simd * tiles(32), 10.0 * part)},
         {whole ? TILE_32 : TILE_QUADS, 2.4 + stages * (both ? larger(0.295, 0.03 + 0.23 * most(32)) : larger(0.27, 0.03 + 0.18 * most(32)))},
         {TILE_64, !whole ? never : 2.4 + stages * (both ? 0.48 : 0.35) * most(64)},
         {TILE_128, !whole || decay ? never : 3.0 + stages * (both ? 1.35 : 0.80) * most(128)}};
@@ -385,8 +385,8 @@ static int gemm_plain_choice(int M, int N, int K, int batch, bool both, bool who
     return all[best].kernel;
 }
 
-#define GRID_X (1 << 23)
-// What the entries take: rows as ever, and tiles of 32 x 32 that GRID_X times 256 hold (2 T sums a product).
+#define GRID_X (1 << 22)
+// What the entries take: rows as ever, and tiles of 32 x 32 that GRID_X times 512 hold (2 T sums a product).
 #define HB_REQUIRE_TILES(M, N)                                                                                        \
     do {                                                                                                              \
         HB_REQUIRE((M) <= 65535 * 64, "gemm: M=%d, at most 4194240 rows are taken", M);                               \
@@ -404,7 +404,7 @@ static void launch_as(const TA* A, const TW* W, TC* C, int M, int N, int K, int 
     };
     const bool vec = borders(16 / sizeof(TA), 16 / sizeof(TW)), half = !vec && borders(4, 4);
     auto tiles = [&](int high, int wide) { return (long long)((N + wide - 1) / wide) * ((M + high - 1) / high) * batch; };
-    // (a grid's x holds fewer than 2^32 threads: beyond GRID_X tiles the rest lie along its y)
+    // (a grid's x holds fewer than 2^32 threads, a tile has up to 512: beyond GRID_X tiles the rest lie along its y)
     auto grid = [&](int high, int wide) {
         const long long n = tiles(high, wide) / batch, x = n < GRID_X ? n : GRID_X;
         return dim3((unsigned)x, (unsigned)((n + x - 1) / x), batch);
@@ -421,12 +421,13 @@ static void launch_as(const TA* A, const TW* W, TC* C, int M, int N, int K, int 
     // (both sides of the first two lines stand at the kernels)
     const long long strips = (N + 15ll) / 16 * batch;
     const int at_once = stretches < WAVE_WAVES ? stretches : WAVE_WAVES;
-    const int which = half                                                      ? M <= 16 ? WAVE_HALVES : TILE_HALVES
+    const bool waves = M <= 4096 && (N + 15ll) / 16 * HB_WAVE * at_once < 1ll << 32;     // (the strips lie along x alone)
+    const int which = half                                                      ? M <= 16 && waves ? WAVE_HALVES : TILE_HALVES
                       : !vec                                                    ? TILE_SINGLE
-                      : M <= 16 && sizeof(TW) == 4 && K < 1024 && K > 64 && K % K_BLOCK ? STREAM
-                      : M <= 16                                                 ? strips * at_once > 2048 ? WAVE_RING : WAVE
+                      : M <= 16 && waves && sizeof(TW) == 4 && K < 1024 && K > 64 && K % K_BLOCK ? STREAM
+                      : M <= 16 && waves                                        ? strips * at_once > 2048 ? WAVE_RING : WAVE
                                                                                 : gemm_plain_choice(M, N, K, batch, Parts<TA>::COUNT + Parts<TW>::COUNT == 6,
-                                                                                                    K % 32 == 0 && lda < 1 << 23 && ldw < 1 << 23, ep.rate != nullptr);
+                                                                                                    K % 32 == 0 && lda < 1 << 23 && ldw < 1 << 23, ep.rate != nullptr, waves);
     switch (which) {
         case STREAM:
             if constexpr (sizeof(TW) == 4)

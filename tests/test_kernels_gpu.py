@@ -256,6 +256,20 @@ def test_gemm_plain_a_row_that_is_not_finite_holds_up_no_other(M, N, K, wd):
         assert torch.equal(c[M // 2].isnan(), want.isnan()) and torch.equal(c[M // 2].isinf(), want.isinf())
 
 
+def test_gemm_plain_more_columns_than_a_grid_has_waves_for():
+    """2^30 columns (17 GB of weights): strips of 16 of them along a grid's x would be 2^32 threads."""
+    from herbert_rs_amd.kernels import ops
+    N, K = 1 << 30, 8
+    part = rand(1 << 16, K, seed=91).bfloat16()
+    w = torch.empty(N, K, dtype=torch.bfloat16, device=dev())
+    w.view(-1, 1 << 16, K).copy_(part[None].expand(N >> 16, -1, -1))
+    a, c = rand(1, K, seed=92).bfloat16(), torch.empty(1, N, dtype=torch.bfloat16, device=dev())
+    ops.gemm_plain(a, w, c)
+    want = torch.empty(1, 1 << 16, dtype=torch.bfloat16, device=dev())
+    ops.gemm_plain(a, part, want)
+    assert bool((c.view(-1, 1 << 16) == want).all())
+
+
 @pytest.mark.parametrize("K", [40, 37])
 @pytest.mark.parametrize("far", ["a", "w"])
 def test_gemm_plain_rows_that_lie_far_apart(K, far):
