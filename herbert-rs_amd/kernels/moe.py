@@ -149,7 +149,7 @@ COMBINE_NORM_TOKENS = 64        # (see combine_norm)
 def combine_norm(y, routing, acc, norm_w, eps, x, rows, alpha_next, shared=None, gate=None):
     """`combine` into acc (which then holds the sums only if alpha_next is 0: nobody reads them) and ops.postnorm of them, in one
     kernel: x = sum / rms(sum) * norm_w, rows (or None) = x in its own type, acc = alpha_next x where that is not 0. For up to
-    COMBINE_NORM_TOKENS tokens; False, and nothing done, where the kernel does not take the sizes."""
+    COMBINE_NORM_TOKENS tokens; False, and nothing done, where the kernel does not take the sizes or rows lie off 16-byte borders."""
     r = routing
     T, H = acc.shape
     if T > COMBINE_NORM_TOKENS or H % 4 or H > 8192 or r.real < r.E:
@@ -161,6 +161,8 @@ def combine_norm(y, routing, acc, norm_w, eps, x, rows, alpha_next, shared=None,
     _check(x, "x", torch.float32, (T, H))
     if rows is not None:
         _check(rows, "rows", None, (T, H))
+    if (y.data_ptr() | acc.data_ptr() | norm_w.data_ptr() | x.data_ptr() | (shared_ptr or 0) | (_ptr(rows) or 0)) % 16:
+        return False
     lib.call("moe", "hb_moe_combine_norm", y.data_ptr(), r.weight.data_ptr(), r.row_of.data_ptr(), acc.data_ptr(), T, r.top, H,
              shared_ptr, gate_ptr, gate_ld, norm_w.data_ptr(), float(eps), x.data_ptr(), _ptr(rows),
              dtype_code(x if rows is None else rows), float(alpha_next), _stream())

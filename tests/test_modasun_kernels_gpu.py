@@ -407,6 +407,32 @@ def test_the_weighted_sum_and_the_norm_behind_it_in_one_kernel(T, H, top, dtype)
     assert not moe.combine_norm(y, routing, refused, w, 1e-5, refused, None, 0.0)
 
 
+@pytest.mark.parametrize("which", ["y", "acc", "w", "x", "rows", "shared"])
+def test_the_weighted_sum_leaves_the_norm_to_others_where_rows_lie_off_16_byte_borders(which):
+    """One operand an element further on: nothing is done, and the two kernels take it."""
+    T, H, top, E = 3, 64, 2, 5
+    routing = moe.Routing(torch.empty(moe.Routing.ints_needed(T, E, top), dtype=torch.int32, device=DEV), torch.empty(T, top, device=DEV), T, E, top)
+    moe.route(rand(T, E, seed=71).to(DEV), rand(E, seed=72).to(DEV), routing)
+
+    def off(t):
+        return torch.cat([t.flatten()[:1], t.flatten()])[1:].view(t.shape)
+    given = dict(y=rand(T * top, H, seed=73), acc=rand(T, H, seed=74), w=rand(H, seed=75), x=torch.full((T, H), 7.0),
+                 rows=torch.full((T, H), 7.0, dtype=torch.bfloat16), shared=rand(T, H, seed=76))
+    given = {k: t.to(DEV) for k, t in given.items()}
+    gate = (rand(T, 7, seed=77).to(DEV), 4)
+    sums, want = given["acc"].clone(), [torch.empty_like(given["x"]), torch.empty_like(given["rows"])]
+    moe.combine(given["y"], routing, sums, shared=given["shared"], gate=gate)
+    ops.postnorm(sums, given["w"], want[0], want[1], 1e-5, 2.0)
+    given[which] = off(given[which])
+    y, acc, w, x, rows, shared = (given[k] for k in ("y", "acc", "w", "x", "rows", "shared"))
+    before = acc.clone()
+    assert not moe.combine_norm(y, routing, acc, w, 1e-5, x, rows, 2.0, shared=shared, gate=gate)
+    assert torch.equal(acc, before) and bool((x == 7).all()) and bool((rows == 7).all())
+    moe.combine(y, routing, acc, shared=shared, gate=gate)
+    ops.postnorm(acc, w, x, rows, 1e-5, 2.0)
+    assert torch.allclose(x, want[0], rtol=1e-5, atol=1e-6) and torch.allclose(rows.float(), want[1].float(), rtol=2.0 ** -7, atol=1e-6)
+
+
 @pytest.mark.parametrize("T,E,top,N,K", [(1, 8, 2, 33, 512), (5, 4, 3, 96, 1536), (17, 1, 1, 70, 2048), (40, 3, 1, 64, 100), (150, 2, 2, 36, 5004), (9, 4, 2, 40, 30)])
 @pytest.mark.parametrize("wd", [torch.float32, torch.bfloat16])
 def test_products_of_experts_in_float32(T, E, top, N, K, wd):
