@@ -714,9 +714,10 @@ def add_bias(x, bias):
     lib.call("elementwise", "hb_add_bias", x.data_ptr(), bias.data_ptr(), T, H, _stream())
 
 
-def token_side_norms(H):
-    """True where `token_side` takes a next_norm."""
-    return H % 4 == 0 and H <= 8192
+def token_side_norms(H, *rows):
+    """True where `token_side` takes a next_norm: a width, and the tensors that its last kernel would read or write by quads (x, y, both
+    norms' weights, the normed rows)."""
+    return H % 4 == 0 and H <= 8192 and all(t.data_ptr() % 16 == 0 for t in rows)
 
 
 TOKEN_SIDE_FEW = 64      # up to so many tokens the gate's rows take a workgroup each
@@ -732,8 +733,8 @@ def token_side(x, token_ids, table, col0, w_gate, w_proj_t, norm_w, eps, g, y, s
     if next_norm is not None:
         _check(next_norm[0], "next norm's weight", torch.float32, (x.shape[1],))
         _check(next_norm[2], "next norm's rows", None, tuple(x.shape))
-        if stage == 0 or not token_side_norms(x.shape[1]):
-            raise BackendError("token input: the norm behind it goes with its last kernel, rows in whole quads up to 8192")
+        if stage == 0 or not token_side_norms(x.shape[1], x, y, norm_w, next_norm[0], next_norm[2]):
+            raise BackendError("token input: the norm behind it goes with its last kernel, rows in whole quads up to 8192 on 16-byte borders")
     if g16 is not None:
         _check(g16, "g16", torch.bfloat16, (x.shape[0], w_gate.shape[0]))
         if stage != 0 or x.shape[0] <= TOKEN_SIDE_FEW:

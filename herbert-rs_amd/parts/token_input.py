@@ -58,11 +58,12 @@ class GatedTableInput(Part):
         args = (x, ctx.meta.token_ids, self.table, self.layer * self.dim, self.gate, self.proj_t, self.norm_w, self.eps, g, y)
         # the norm that x meets next, where it is of the kind that is handed on (`NormedRows`, whole)
         rows = None
-        if ctx.norm_after_block is not None and getattr(ctx.norm_after_block[0], "hands_on", False) \
-                and ops.token_side_norms(self.hidden_size):
+        if ctx.norm_after_block is not None and getattr(ctx.norm_after_block[0], "hands_on", False):
             norm, entry = ctx.norm_after_block
-            ctx.left = NormedRows(norm, entry, x, ctx.rt.buffer("token_input_normed", (T, self.hidden_size)), None)
-            rows = (norm.w, norm.eps, ctx.left.xg)
+            normed = ctx.rt.buffer("token_input_normed", (T, self.hidden_size))
+            if ops.token_side_norms(self.hidden_size, x, y, self.norm_w, norm.w, normed):
+                ctx.left = NormedRows(norm, entry, x, normed, None)
+                rows = (norm.w, norm.eps, normed)
         if self.proj is not None and T > ops.TOKEN_SIDE_FEW:
             g16 = ctx.rt.buffer("token_input_gates16", (T, self.dim), torch.bfloat16)
             ops.token_side(*args, stage=0, g16=g16)

@@ -7,13 +7,16 @@ slots used again, memories long and short, the gated norm in groups), the expert
 groups worth their best member, weights as they are, identity experts in the weighted sum) and the per-layer
 token input."""
 import math
+import types
 
 import pytest
 import torch
 
 from herbert_rs_amd.cache import Cache, KVNeed, StateNeed
 from herbert_rs_amd.kernels import mfma, moe, ops, recurrent
+from herbert_rs_amd.parts import Runtime
 from herbert_rs_amd.parts.position import RotaryPairs
+from herbert_rs_amd.parts.token_input import GatedTableInput
 
 from .plain import bozasun as plain
 from .test_vipalorn_kernels_gpu import step_meta
@@ -329,3 +332,33 @@ def test_token_input_and_the_norm_behind_it(T, H):
         slack = bound * (want.abs() + size * (want / one).abs()) + (2.0 ** -8 * want.abs() if dtype == torch.bfloat16 else 0)
         assert bool(((rows.float() - want).abs() <= slack + 1e-6).all())
     assert not ops.token_side_norms(H + 1)
+
+
+@pytest.mark.parametrize("T", [3, 70])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("which", ["own", "next", "x"])
+def test_token_input_leaves_the_norm_to_others_where_rows_lie_off_16_byte_borders(which, dtype, T):
+    """A norm's weight, or the residual stream, an element further on in a larger tensor on the GPU: the part runs and leaves no normed rows."""
+    H, D, V = 64, 32, 20
+    names = {k: k for k in ("table", "gate", "proj", "norm")}
+    stored = {"table": rand(V, D, seed=2), "gate": rand(D, H, seed=3, scale=H ** -0.5), "proj": rand(H, D, seed=4), "norm": 1 + 0.2 * rand(H, seed=5)}
+
+    def off(t):
+        return torch.cat([t.flatten()[:1], t.flatten()]).to(DEV)[1:].view(t.shape)
+
+    def forward(moved):
+        rt = Runtime(dtype, DEV)
+        part = GatedTableInput(H, V, D, 0, 1, 1e-5, names)
+        part.load({**stored, "norm": off(stored["norm"]) if moved == "own" else g(stored["norm"])}, rt)
+        x, w = rand(T, H, seed=1, scale=2.0), 1 + 0.2 * rand(H, seed=7)
+        x, w = off(x) if moved == "x" else g(x), off(w) if moved == "next" else g(w)
+        tokens = torch.randint(0, V, (T,), generator=torch.Generator().manual_seed(6)).to(torch.int32).to(DEV)
+        ctx = types.SimpleNamespace(rt=rt, meta=types.SimpleNamespace(token_ids=tokens), left=None,
+                                    norm_after_block=(types.SimpleNamespace(hands_on=True, w=w, eps=1e-6), 1))
+        part.forward(ctx, x)
+        return x, ctx.left
+    want, left = forward(None)
+    assert left is not None
+    got, left = forward(which)
+    assert left is None
+    assert torch.allclose(got, want, rtol=1e-5, atol=1e-5)
