@@ -164,8 +164,8 @@ def _entry(module, fname):
     global _invoke
     fn = getattr(load(module), fname)
     kinds = "".join("f" if t is _F else "i" for t in fn.argtypes)
+    _invoke = host().invoke                 # (first: another thread calls what it finds in _entries)
     entry = _entries[(module, fname)] = host().entry(ctypes.cast(fn, _P).value, kinds)
-    _invoke = host().invoke
     return entry
 
 

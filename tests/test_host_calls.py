@@ -57,6 +57,22 @@ def test_what_is_no_argument_is_refused():
         lib.call("gemm_plain", "hb_gemm_plain", None, 0, None, 0, None, 0, 0, 1, 1, 1, 1, 1, 0, None)
 
 
+def test_an_entry_point_is_known_only_once_it_can_be_called(monkeypatch):
+    """Another thread that finds it there calls it at once: also the first one ever."""
+    class Entries(dict):
+        def __setitem__(self, key, entry):
+            super().__setitem__(key, entry)
+            with pytest.raises(BackendError, match="empty problem"):
+                lib.call(*key, None, 0, None, 0, None, 0, 0, 1, 1, 1, 1, 1, 0, None)
+            tried.append(key)
+    tried = []
+    monkeypatch.setattr(lib, "_entries", Entries())
+    monkeypatch.setattr(lib, "_invoke", None)
+    with pytest.raises(BackendError, match="empty problem"):
+        lib.call("gemm_plain", "hb_gemm_plain", None, 0, None, 0, None, 0, 0, 1, 1, 1, 1, 1, 0, None)
+    assert tried == [("gemm_plain", "hb_gemm_plain")]
+
+
 def test_a_tensor_off_the_gpu_is_refused():
     assert not lib.host().fits(torch.zeros(3), None, None) and not lib.host().fits(None, None, None)
     for wrong in (torch.zeros(3), 5, None):
