@@ -183,7 +183,7 @@ attention_plain_kernel(const T* __restrict__ q, const T* __restrict__ k_cache,
         hb_workgroup_barrier();                       // (and the weights of the chunk before have been read)
         const float m_new = fmaxf(m, fmaxf(fmaxf(tops[0][r], tops[1][r]), fmaxf(tops[2][r], tops[3][r])));
         const float corr = expf(sees ? m - m_new : 0.f);
-        m = m_new;
+        m = sees ? m_new : m;                         // (a chunk that is not seen does not hide a sink of NaN)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {                 // (the exponential in any case: no branch an element)
             const bool there = dots[e] != -INFINITY;

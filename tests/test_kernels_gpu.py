@@ -550,6 +550,21 @@ def test_attention_plain_tiles_and_what_no_query_sees(nq, nkv, hd):
     assert torch.equal(out[:60], seen[:60]) and torch.equal(out[70:], seen[70:]) and bool(out[60:70].isnan().all())
 
 
+def test_attention_plain_keeps_a_sink_of_nan():
+    """A head whose sink is NaN is NaN in every row, also where a tile's first chunk of keys lies before a row's window; a huge sink takes all
+    the weight; the other head is as without sinks of either kind."""
+    from herbert_rs_amd.kernels import ops
+    nq, nkv, hd, window, n = 3, 3, 64, 64, 200
+    meta, kv, _ = paged_case([n], [n], nkv, hd, torch.float32, seed=8)
+    q = rand(n, nq * hd, seed=22)
+    out, plain = torch.empty_like(q), torch.empty_like(q)
+    ops.attention_plain(q, meta, kv, plain, nq, nkv, hd, 0.125, window, sinks=torch.zeros(nq, device=dev()))
+    ops.attention_plain(q, meta, kv, out, nq, nkv, hd, 0.125, window, sinks=torch.tensor([float("nan"), 0.0, 1e30], device=dev()))
+    assert bool(out[:, :hd].isnan().all())
+    assert torch.equal(out[:, hd:2 * hd], plain[:, hd:2 * hd])
+    assert bool((out[:, 2 * hd:] == 0).all())
+
+
 @pytest.mark.parametrize("tile_height", [32, 64])
 @pytest.mark.parametrize("nq,nkv,hd,window", [(4, 1, 128, 0), (8, 2, 64, 0), (6, 2, 32, 0), (5, 1, 64, 70),
                                               (3, 3, 128, 100), (16, 2, 128, 0), (2, 2, 32, 0)])
