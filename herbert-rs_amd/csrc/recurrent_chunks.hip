@@ -650,9 +650,9 @@ extern "C" int hb_chunked_delta(const float* qkv, int C, const float* proj, int 
 // range (sums of 128 products of two are 1.3e38 at most), beyond it one may where the walk, whose state decays first, stays within.
 // ssm_chunks_kernel: the chain of chunks, a workgroup a (head, 16 or 32 columns of S, sequence): four waves, each 16 tokens of a chunk for the outputs and a
 // quarter of the state's rows. A chunk that holds something not finite is walked token by token instead (ssm_slowly), so that it
-// spoils what it spoils in the walk.
-// 64 heads of 128 x 64 on 8 groups, one sequence of 2,048 tokens 226 us (the walk 802), of 512 70 (209), four of 512 130 (313), 16 of 128 140
-// (310). Bound by a chunk's chain in a workgroup, 6.7 us with 16 columns, 9.5 with 32: 80 or 160 products of 40 cycles a wave, and as long again
+// spoils what it spoils in the walk: all its columns, or where an input or the state is what is too large, the 16 columns around it.
+// 64 heads of 128 x 64 on 8 groups, one sequence of 2,048 tokens 212 us (the walk 802), of 512 63 (209), four of 512 111 (313), 16 of 128 119
+// (310); with a branch on whether a chunk is walked that the compiler took for one a lane 225, 67, 121 and 128. Bound by a chunk's chain in a workgroup, 6.3 us with 16 columns, 9.5 with 32: 80 or 160 products of 40 cycles a wave, and as long again
 // for the decays and for laying out the state and the columns. Errors against 64 bits are 0.2 to 1.02 of the walk's.
 #define TOO_LARGE 1e18f
 __device__ __forceinline__ bool too_large(float v) { return !(fabsf(v) <= TOO_LARGE); }
@@ -691,12 +691,13 @@ ssm_pairs_kernel(const float* __restrict__ u, int ldu, int b_at, int c_at, const
     }
 }
 
-// One chunk of COLS columns token by token; the state lies in LDS, a column's entry n at in_quads(n). Eight lanes a column.
+// One chunk token by token, of those blocks of 16 of a workgroup's COLS columns whose bit is set; the state lies in LDS, a column's entry n at
+// in_quads(n). Eight lanes a column.
 template <int N, int SLD, int COLS>
-__device__ __forceinline__ void ssm_slowly(float* s_lds, const float* u, int ldu, const float* proj, int ld, int n, int x_at, int b_at, int c_at,
+__device__ __forceinline__ void ssm_slowly(int blocks, float* s_lds, const float* u, int ldu, const float* proj, int ld, int n, int x_at, int b_at, int c_at,
                                            float bias, float rate, float skip, float* y, int ldy, int cols) {
     const int col = threadIdx.x / 8, part = threadIdx.x % 8;
-    if (col >= COLS) return;
+    if (col >= COLS || !(blocks >> col / 16 & 1)) return;
     for (int t = 0; t < n; ++t) {
         const float* row = u + (size_t)t * ldu;
         const float z = proj[(size_t)t * ld] + bias, dt = z > 20.f ? z : log1pf(expf(z)), a = expf(-rate * dt);
@@ -724,7 +725,8 @@ ssm_chunks_kernel(const float* __restrict__ u, int ldu, const float* __restrict_
     __shared__ __attribute__((aligned(16))) float s_lds[2][SSM_COLS * SLD], x_lds[2][SSM_COLS * XLD];
     __shared__ double c_lds[4][CHUNK];
     __shared__ float dt_lds[4][CHUNK];
-    __shared__ int spoilt[2];
+    __shared__ int spoilt[2];                                  // a bit a block of 16 columns that is to be walked
+    constexpr int EVERY = (1 << CB) - 1;
     const int h = blockIdx.x, col0 = blockIdx.y * SSM_COLS, cols = min(SSM_COLS, P - col0);
     const int4 run = runs[blockIdx.z];
     const int begin = run.z, n_all = run.w, last = (n_all + CHUNK - 1) / CHUNK;
@@ -775,7 +777,7 @@ ssm_chunks_kernel(const float* __restrict__ u, int ldu, const float* __restrict_
         c_lds[wave][lane] = sum;
         dt_lds[wave][lane] = dt;
         const float my_dt = __shfl(dt, my_token & 63, HB_WAVE);
-        bool bad = not_finite(dt) || not_finite((float)sum);
+        bool bad = false;
 #pragma unroll
         for (int i = 0; i < XQ; ++i)
 #pragma unroll
@@ -783,7 +785,8 @@ ssm_chunks_kernel(const float* __restrict__ u, int ldu, const float* __restrict_
                 bad |= too_large(x_next[i][e]) || too_large(x_next[i][e] * my_dt);
                 x_lds[buf][(my_col + 4 * i + e) * XLD + in_quads(my_token)] = x_next[i][e];
             }
-        if (bad) spoilt[buf] = 1;
+        const int blocks = (not_finite(dt) || not_finite((float)sum) ? EVERY : 0) | (bad ? 1 << my_col / 16 : 0);
+        if (blocks) atomicOr(&spoilt[buf], blocks);
     };
     // what a wave reads of a chunk for itself: its 16 tokens of C and their pairs, all tokens' B for its rows of the state
     f32x4 cq[DB], pr[4];
@@ -814,7 +817,7 @@ ssm_chunks_kernel(const float* __restrict__ u, int ldu, const float* __restrict_
         const int buf = c & 1, n = min(CHUNK, n_all - c * CHUNK), t0 = begin + c * CHUNK;
         const bool more = c + 1 < last;
         if (more) fetch(c + 1);
-        bool bad = false;
+        bool bad = false, large[CB] = {};
 #pragma unroll
         for (int b = 0; b < DB; ++b)
 #pragma unroll
@@ -828,8 +831,11 @@ ssm_chunks_kernel(const float* __restrict__ u, int ldu, const float* __restrict_
 #pragma unroll
             for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) bad |= too_large(S[i][cb][e]);
-        if (__any(bad) && lane == 0) spoilt[buf] = 1;
+                for (int e = 0; e < 4; ++e) large[cb] |= too_large(S[i][cb][e]);
+        int blocks = __any(bad) ? EVERY : 0;
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) blocks |= __any(large[cb]) ? 1 << cb : 0;
+        if (blocks && lane == 0) atomicOr(&spoilt[buf], blocks);
         // the decays: of a token from the chunk's start, of a pair, and to the chunk's end
         const double own = c_lds[wave][16 * wave + r], end = c_lds[wave][CHUNK - 1];
         float from_start[4], to_end[16], dt[16];
@@ -845,52 +851,59 @@ ssm_chunks_kernel(const float* __restrict__ u, int ldu, const float* __restrict_
             pr[s / 4][s % 4] *= i <= 16 * wave + r ? expf((float)(at - own)) : 0.f;
         }
         __syncthreads();                                      // (everyone has looked for what is not finite)
-        if (spoilt[buf]) {
-            ssm_slowly<N, SLD, SSM_COLS>(s_lds[buf], u + (size_t)t0 * ldu, ldu, proj + (size_t)t0 * ld + dt_off + h, ld, n, x_at, b_at, c_at, bias, rate, skip,
-                               y + (size_t)t0 * inner + x_at, inner, cols);
-            __syncthreads();
+        const int walked = __builtin_amdgcn_readfirstlane(spoilt[buf]);
 #pragma unroll
-            for (int i = 0; i < OWN; ++i)
+        for (int b = 0; b < DB; ++b) transpose_quads(cq[b]);
+        auto products = [&](int cb) {
+            Chains<8> part;
 #pragma unroll
-                for (int cb = 0; cb < CB; ++cb)
+            for (int b = 0; b < DB; ++b) {
+                const f32x4 s = *(const f32x4*)&s_lds[buf][(16 * cb + r) * SLD + 16 * b + 4 * q];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) S[i][cb][e] = s_lds[buf][(16 * cb + r) * SLD + 16 * (wave + 4 * i) + 4 * e + q];
-        } else {
+                for (int e = 0; e < 4; ++e) part.add(cq[b][e], s[e], 4 * b + e);
+            }
+            f32x4 sums = part.sum();
 #pragma unroll
-            for (int b = 0; b < DB; ++b) transpose_quads(cq[b]);
+            for (int e = 0; e < 4; ++e) sums[e] *= from_start[e];
 #pragma unroll
-            for (int cb = 0; cb < CB; ++cb) {
-                Chains<8> part;
+            for (int i = 0; i < OWN; ++i) S[i][cb] *= all;
 #pragma unroll
-                for (int b = 0; b < DB; ++b) {
-                    const f32x4 s = *(const f32x4*)&s_lds[buf][(16 * cb + r) * SLD + 16 * b + 4 * q];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) part.add(cq[b][e], s[e], 4 * b + e);
-                }
-                f32x4 sums = part.sum();
-#pragma unroll
-                for (int e = 0; e < 4; ++e) sums[e] *= from_start[e];
-#pragma unroll
-                for (int i = 0; i < OWN; ++i) S[i][cb] *= all;
-#pragma unroll
-                for (int b = 0; b < 4; ++b) {
-                    f32x4 x = *(const f32x4*)&x_lds[buf][(16 * cb + r) * XLD + 16 * b + 4 * q];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        x[e] *= dt[4 * b + e];
-                        const float late = x[e] * to_end[4 * b + e];
-#pragma unroll
-                        for (int i = 0; i < OWN; ++i) S[i][cb] = mfma_k4(k[i][4 * b + e], late, S[i][cb]);
-                        if (b <= wave) sums = mfma_k4(pr[b][e], x[e], sums);
-                    }
-                }
+            for (int b = 0; b < 4; ++b) {
+                f32x4 x = *(const f32x4*)&x_lds[buf][(16 * cb + r) * XLD + 16 * b + 4 * q];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const int t = 16 * wave + 4 * q + e;
-                    if (t < n && 16 * cb < cols)
-                        y[(size_t)(t0 + t) * inner + x_at + 16 * cb + r] =
-                            fmaf(skip, x_lds[buf][(16 * cb + r) * XLD + in_quads(t)], sums[e]);
+                    x[e] *= dt[4 * b + e];
+                    const float late = x[e] * to_end[4 * b + e];
+#pragma unroll
+                    for (int i = 0; i < OWN; ++i) S[i][cb] = mfma_k4(k[i][4 * b + e], late, S[i][cb]);
+                    if (b <= wave) sums = mfma_k4(pr[b][e], x[e], sums);
                 }
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int t = 16 * wave + 4 * q + e;
+                if (t < n && 16 * cb < cols)
+                    y[(size_t)(t0 + t) * inner + x_at + 16 * cb + r] =
+                        fmaf(skip, x_lds[buf][(16 * cb + r) * XLD + in_quads(t)], sums[e]);
+            }
+        };
+        if (!walked) {
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) products(cb);
+        } else {                                              // (of two blocks perhaps one: a column's bits do not hang on how many share a workgroup)
+            ssm_slowly<N, SLD, SSM_COLS>(walked, s_lds[buf], u + (size_t)t0 * ldu, ldu, proj + (size_t)t0 * ld + dt_off + h, ld, n, x_at, b_at, c_at, bias,
+                                         rate, skip, y + (size_t)t0 * inner + x_at, inner, cols);
+            __syncthreads();
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) {
+                if (!(walked >> cb & 1)) {
+                    products(cb);
+                    continue;
+                }
+#pragma unroll
+                for (int i = 0; i < OWN; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) S[i][cb][e] = s_lds[buf][(16 * cb + r) * SLD + 16 * (wave + 4 * i) + 4 * e + q];
             }
         }
         if (more) {

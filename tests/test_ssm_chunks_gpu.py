@@ -145,3 +145,27 @@ def test_a_sequence_alone_and_beside_others(lengths, heads, groups, N, P, bad):
         assert torch.equal(alone.nan_to_num(7.0), got[at:at + n].nan_to_num(7.0))
         assert torch.equal(alone_left[slot].nan_to_num(7.0), left[slot].nan_to_num(7.0))
         at += n
+
+
+@pytest.mark.parametrize("place", ["x", "state"])
+@pytest.mark.parametrize("what", [float("inf"), 1e20])
+@pytest.mark.parametrize("lengths,heads,groups,N,P", [([64, 130, 65], 96, 3, 64, 64), ([70, 1000], 65, 5, 128, 48), ([129, 64], 129, 1, 64, 32)])
+def test_a_large_column_alone_and_beside_others(lengths, heads, groups, N, P, what, place):
+    """One column's input or state is too large for the products, so that its 16 columns are walked: also in a workgroup of 32, whose other 16 are
+    not. The same bits either way, and in those other 16 the bits that they have without the large one."""
+    u, proj, a_log, dt_bias, d_skip, state, meta = step(lengths, heads, groups, N, P, -2.0)
+    plain, plain_left = run(u, proj, a_log, dt_bias, d_skip, state, meta, heads, groups, N, P)
+    if place == "x":
+        u[lengths[0] - 3, P + 21] = what
+    else:
+        state[len(lengths), 1, 21, 9] = what
+    assert heads * ((P + 31) // 32) * len(lengths) > 256 >= heads * ((P + 31) // 32)
+    got, left = run(u, proj, a_log, dt_bias, d_skip, state, meta, heads, groups, N, P)
+    n, slot = lengths[0], len(lengths)
+    one = types.SimpleNamespace(max_new=n, num_seqs=1, seq_starts=torch.tensor([0, n], dtype=torch.int32, device=DEV), derived={},
+                                host_starts=torch.tensor([0, n], dtype=torch.int32).numpy(), slots=torch.tensor([slot], dtype=torch.int32, device=DEV))
+    alone, alone_left = run(u[:n], proj[:n], a_log, dt_bias, d_skip, state, one, heads, groups, N, P)
+    assert torch.equal(alone.nan_to_num(7.0), got[:n].nan_to_num(7.0))
+    assert torch.equal(alone_left[slot].nan_to_num(7.0), left[slot].nan_to_num(7.0))
+    assert not torch.equal(got[:n, 1, 21], plain[:n, 1, 21])
+    assert torch.equal(got[:, :, :16], plain[:, :, :16]) and torch.equal(left[:, :, :16], plain_left[:, :, :16])
