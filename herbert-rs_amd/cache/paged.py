@@ -150,9 +150,6 @@ class StateGroup:
     def view(self, entry):
         return self.data[self.entries.index(entry)]
 
-    def clear_slot(self, slot):
-        self.data[:, slot].zero_()
-
 
 class Cache:
     """Slots, their lengths, and the groups of storage behind them.
