@@ -239,9 +239,9 @@ gemm_plain_tile_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
 }
 
 // Few rows of A (a decode step, a short prompt): a product bound by the weights' bytes and, narrow ones, by the chain of k. A
-// workgroup on 16 rows of W and MB blocks of 16 rows of A, a wave on every stretch of K_BLOCK (up to MOST of them at a
+// workgroup on 16 rows of W and MB blocks of 16 rows of A, a wave on every stretch of K_BLOCK (up to WAVE_WAVES of them at a
 // time): no load waits for another wave, and a wave asks for all of its stretch of W at once (16 pieces of 8 elements a lane), for A
-// some pieces ahead, and splits both in registers. The stretches' sums meet in LDS, where a thread an output adds them in
+// some pieces ahead, and splits both in registers. The stretches' sums meet in LDS, where the first wave adds them in
 // their order. Short products through a narrow middle are here too, and those of heads with a matrix each: a wave on vector products, 16 columns
 // and 8 rows, which they had, took at 1 | 8 | 24 rows of bfloat16 weights (2048 x 128) 3.1 | 3.5 | 3.8 us, now 2.6 | 2.6 | 2.6; (4096 x 1024)
 // 14.5 | 16.7 | 19.3, now 5.2 | 5.4 | 7.4; (16 heads of 128 x 512) 7.5 | 8.8 | 9.8, now 3.8 | 4.1 | 4.5.
@@ -305,7 +305,11 @@ gemm_plain_wave_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
 
 // Up to 16 rows on float32 weights whose k is so short that there
 // is nothing to share: no LDS and no barrier; a wave goes through the stretches one after another, the next WAVE_DEPTH pieces of 32 k of
-// W and A on their way while the WAVE_DEPTH before are multiplied.
+// W and A on their way while the WAVE_DEPTH before are multiplied. A stretch that is not whole goes by in rounds of four pieces in the kernel above,
+// each waited for; here the next round is on its way. A whole one it asks for at once, and k beyond 1024 gives it more waves than one.
+// Microseconds at 8 rows by this kernel | the one above: 2048 x 128 3.2 | 3.3, 4096 x 256 4.3 | 4.8, 32768 x 640 21.2 | 25.2, 32768 x 768 23.6 | 26.9,
+// but where the strips are few 512 x 640 6.9 | 6.5, 2048 x 768 8.4 | 7.5, 16384 x 128 5.2 | 4.7; whole stretches 32768 x 512 17.5 | 16.6, 16384 x 1024
+// 16.7 | 17.0, 4096 x 2048 18.6 | 12.7, 2048 x 8192 61 | 31.
 template <class TA, class TW, class TC, bool ACCUM>
 __global__ void __launch_bounds__(HB_WAVE)
 gemm_plain_stream_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* __restrict__ C, int M, int N,
@@ -418,7 +422,10 @@ static void launch_as(const TA* A, const TW* W, TC* C, int M, int N, int K, int 
     gemm_plain_wave_kernel<TA, TW, TC, ACCUM, MB, NB, AHEAD, HOW>                                                     \
         <<<dim3((N + 16 * NB - 1) / (16 * NB), (M + 16 * MB - 1) / (16 * MB), batch), HB_WAVE * at_once, 0, stream>>>( \
             A, W, C, M, N, K, lda, ldw, ldc, batch_a, batch_w, batch_c, ep)
-    // (both sides of the first two lines stand at the kernels)
+    // (Both sides of STREAM stand at its kernel. WAVE_RING holds 8 pieces of W instead of 16 and so twice the waves on a CU, for products whose waves fill
+    // the chip at 16 more than once; us at 8 rows by 16 | 8 pieces, the waves in brackets: bfloat16 weights 6144 x 2048 [1536] 11.3 | 13.7, 8192 x 2048 [2048] 11.8 |
+    // 14.4, 11008 x 2048 [2752] 16.1 | 16.1, 32768 x 1024 [4096] 19.8 | 19.6; float32 weights 4096 x 8192 [2048] 37.5 | 37.2, 11008 x 2048 24.8 | 25.0, 32768 x
+    // 1024 32.1 | 28.8, 8192 x 8192 [4096] 68.6 | 57.2.)
     const long long strips = (N + 15ll) / 16 * batch;
     const int at_once = stretches < WAVE_WAVES ? stretches : WAVE_WAVES;
     const bool waves = M <= 4096 && (N + 15ll) / 16 * HB_WAVE * at_once < 1ll << 32;     // (the strips lie along x alone)
@@ -499,10 +506,10 @@ extern "C" int hb_gemm_plain(const void* A, int a_dtype, const void* W, int w_dt
 // A_log [N / D] and dt_bias [N], both or neither: the sums are a decay's pre-activations, and what is stored is
 // the decay a column (float32 in and out, no accumulation). A_log == dt_bias: the decay is
 // sigmoid(sum + dt_bias[n])^root instead.
-extern "C" int hb_gemm_plain_short_k(const void* A, int a_dtype, const void* W, int w_dtype, void* C, int c_dtype,
-                                     int M, int N, int K, int lda, int ldw, int ldc, int accumulate,
-                                     const float* A_log, const float* dt_bias, int D, float root,
-                                     hipStream_t stream) {
+extern "C" int hb_gemm_plain_decay(const void* A, int a_dtype, const void* W, int w_dtype, void* C, int c_dtype,
+                                   int M, int N, int K, int lda, int ldw, int ldc, int accumulate,
+                                   const float* A_log, const float* dt_bias, int D, float root,
+                                   hipStream_t stream) {
     HB_REQUIRE(M > 0 && N > 0 && K > 0, "gemm: empty problem (M=%d, N=%d, K=%d)", M, N, K);
     HB_REQUIRE(lda >= K && ldw >= K && ldc >= N, "gemm: a row stride is smaller than its row");
     HB_REQUIRE((A_log == nullptr) == (dt_bias == nullptr), "gemm: a decay needs its rate and its bias");
@@ -525,9 +532,9 @@ extern "C" int hb_gemm_plain_short_k(const void* A, int a_dtype, const void* W, 
 // Two such products of float32 rows with float32 sums (no decay for the first): C0 = A0 W0^T, C1 = A1 W1^T, shapes and strides alike, in
 // one launch: they wait for the same rows and not for each other, and a launch is the larger part of what one takes (8 x 2048 x 128,
 // bfloat16 weights: 2.6 us, the two together 2.6; 24 rows 2.6 and 2.9).
-extern "C" int hb_gemm_plain_short_k_pair(const float* A0, const void* W0, float* C0, const float* A1, const void* W1, float* C1,
-                                          int w_dtype, int M, int N, int K, int lda, int ldw, int ldc, const float* A_log,
-                                          const float* dt_bias, int D, float root, hipStream_t stream) {
+extern "C" int hb_gemm_plain_decay_pair(const float* A0, const void* W0, float* C0, const float* A1, const void* W1, float* C1,
+                                        int w_dtype, int M, int N, int K, int lda, int ldw, int ldc, const float* A_log,
+                                        const float* dt_bias, int D, float root, hipStream_t stream) {
     HB_REQUIRE(M > 0 && N > 0 && K > 0, "gemm: empty problem (M=%d, N=%d, K=%d)", M, N, K);
     HB_REQUIRE(lda >= K && ldw >= K && ldc >= N, "gemm: a row stride is smaller than its row");
     HB_REQUIRE((A_log == nullptr) == (dt_bias == nullptr), "gemm: a decay needs its rate and its bias");

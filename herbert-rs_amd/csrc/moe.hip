@@ -671,8 +671,8 @@ __global__ void moe_combine_kernel(Combined c, float* __restrict__ x) {
 // The same where a norm of the whole row follows (a block whose norm comes after the sum): acc holds what the sum is added to,
 // x <- sum / rms(sum) * w, y <- x in its own type, acc <- alpha_next x (alpha_next 0: acc stays). A workgroup a token, four
 // columns a thread and PASS, the row in registers between its sum of squares and the stores. For the few tokens of a decode
-// step, where either kernel is a chain of loads and a turn between two launches; with many tokens the two kernels
-// have more loads in flight. 8 tokens of 2,048 columns, four experts and a shared one: 6.1 us in one, 4.6 and 4.7 in two.
+// step, where either kernel is a chain of loads and a turn between two launches. Four experts and a shared one, us in one | in two,
+// 2,048 columns: 1 token 3.2 | 5.9, 8 tokens 3.4 | 5.8, 64 3.5 | 5.9, 128 3.7 | 6.1, 512 6.1 | 9.2; 4,096 columns: 8 tokens 4.5 | 7.1, 64 4.7 | 7.5, 512 12.4 | 17.7.
 template <class TOut, int PASSES>
 __global__ void __launch_bounds__(512)
 moe_combine_norm_kernel(Combined c, float* __restrict__ acc, const float* __restrict__ w, float eps, float* __restrict__ x,

@@ -652,7 +652,8 @@ extern "C" int hb_chunked_delta(const float* qkv, int C, const float* proj, int 
 // quarter of the state's rows. A chunk that holds something not finite is walked token by token instead (ssm_slowly), so that it
 // spoils what it spoils in the walk: all its columns, or where an input or the state is what is too large, the 16 columns around it.
 // 64 heads of 128 x 64 on 8 groups, one sequence of 2,048 tokens 212 us (the walk 802), of 512 63 (209), four of 512 111 (313), 16 of 128 119
-// (310); with a branch on whether a chunk is walked that the compiler took for one a lane 225, 67, 121 and 128. Bound by a chunk's chain in a workgroup, 6.3 us with 16 columns, 9.5 with 32: 80 or 160 products of 40 cycles a wave, and as long again
+// (310); with a branch on whether a chunk is walked that the compiler took for one a lane 225, 67, 121 and 128. Bound by a chunk's chain in a
+// workgroup, 6.3 us with 16 columns, 8.7 with 32: 80 or 160 products of 40 cycles a wave, and as long again
 // for the decays and for laying out the state and the columns. Errors against 64 bits are 0.2 to 1.02 of the walk's.
 #define TOO_LARGE 1e18f
 __device__ __forceinline__ bool too_large(float v) { return !(fabsf(v) <= TOO_LARGE); }
@@ -935,7 +936,7 @@ extern "C" int hb_chunked_ssm(const float* u, int ldu, const float* proj, int ld
     HB_REQUIRE((uintptr_t)chunks % 8 == 0 && (uintptr_t)runs % 16 == 0, "state-space chunks: the lists are not aligned");
     // 16 columns of the state a workgroup where that many still fit the chip at once, two a CU: half the products in a chunk's chain, the
     // decays once more. 64 heads of 128 x 64 in 8 groups, us by 32 | 16 columns: one sequence of 2,048 tokens (128 workgroups of 32 columns)
-    // 313 | 226, of 512 91 | 70, two of 512 and 300 (256) 93 | 78, four of 512 (512) 130 | 167.
+    // 290 | 211, of 512 83 | 63, two of 512 and 300 (256) 84 | 70, three of 512 (384) 109 | 125, four (512) 112 | 148, eight of 128 67 | 85.
     const bool narrow = (long long)heads * ((P + 31) / 32) * n_runs <= 256;
     const int tiles = (P + (narrow ? 15 : 31)) / (narrow ? 16 : 32);
     HB_REQUIRE(n_runs <= 65535 && n_chunks <= 65535 && tiles <= 65535, "state-space chunks: too many sequences or columns for the grid");

@@ -143,7 +143,9 @@ def _shared_args(r, H, shared, gate):
     return shared.data_ptr(), rows.data_ptr() + 4 * column, rows.shape[1]
 
 
-COMBINE_NORM_TOKENS = 64        # (see combine_norm)
+# Up to so many tokens combine_norm runs: a decode step's. (Its kernel in csrc/moe.hip is the faster one as far as it was measured, up to
+# 512 tokens; larger steps keep the two kernels, and with them the order of their sums of squares.)
+COMBINE_NORM_TOKENS = 64
 
 
 def combine_norm(y, routing, acc, norm_w, eps, x, rows, alpha_next, shared=None, gate=None):

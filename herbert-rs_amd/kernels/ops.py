@@ -601,7 +601,7 @@ def gemm_plain_columns_pair(a, K, col0, w0, c0, col1, w1, c1, decay=None):
         if col < 0 or col + K > lda:
             raise BackendError(f"gemm: columns [{col}, {col + K}) of rows of {lda}")
     a_log, dt_bias, D, root = _decay_args(decay, N)
-    lib.call("gemm_plain", "hb_gemm_plain_short_k_pair", a.data_ptr() + 4 * col0, w0.data_ptr(), c0.data_ptr(), a.data_ptr() + 4 * col1,
+    lib.call("gemm_plain", "hb_gemm_plain_decay_pair", a.data_ptr() + 4 * col0, w0.data_ptr(), c0.data_ptr(), a.data_ptr() + 4 * col1,
              w1.data_ptr(), c1.data_ptr(), dtype_code(w0), M, N, K, lda, K, N, a_log, dt_bias, int(D), float(root), _stream())
 
 
@@ -624,7 +624,7 @@ def gemm_plain_columns(a, col0, K, w, c, accumulate=False, decay=None):
     if decay is not None and (accumulate or c.dtype != torch.float32):
         raise BackendError("gemm: a decay is float32, stored and not added to")
     a_log, dt_bias, D, root = _decay_args(decay, N)
-    lib.call("gemm_plain", "hb_gemm_plain_short_k", a.data_ptr() + col0 * a.element_size(), dtype_code(a), w.data_ptr(),
+    lib.call("gemm_plain", "hb_gemm_plain_decay", a.data_ptr() + col0 * a.element_size(), dtype_code(a), w.data_ptr(),
              dtype_code(w), c.data_ptr(), dtype_code(c), M, N, K, lda, K, N, 1 if accumulate else 0, a_log, dt_bias,
              int(D), float(root), _stream())
 
