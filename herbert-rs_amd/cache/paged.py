@@ -231,8 +231,8 @@ class Cache:
         """Clear the state of the slots that were taken since the last call. Whoever is to read or write state calls it, and
         so does whoever makes room for a step: views of the state may be held from before."""
         if self._taken:
-            taken, self._taken = self._taken, set()
-            self.clear_slots(taken)
+            self.clear_slots(self._taken)
+            self._taken = set()     # (a clearing that found no memory is made again)
 
     def clear_slots(self, slots):
         """Fixed-size state of `slots` made zeros, a kernel a group however many they are."""

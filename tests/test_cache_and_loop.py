@@ -125,6 +125,27 @@ def test_state_is_cleared_when_a_slot_is_taken_again():
         c.truncate(s2, 1)
 
 
+def test_state_that_could_not_be_cleared_is_cleared_later(monkeypatch):
+    """Slots apart from each other, whose numbers find no memory on the way to the GPU: the step is refused and nothing is forgotten."""
+    import herbert_rs_amd.cache.paged as paged
+    c = make_cache(state=True)
+    slots = [c.alloc_slot() for _ in range(3)]
+    view = c.state_views(3)[0]
+    view.fill_(5.0)
+    c.free_slot(slots[0]), c.free_slot(slots[2])
+    taken = [c.alloc_slot() for _ in range(2)]
+    assert sorted(taken) == [slots[0], slots[2]]
+
+    def no_memory(*args):
+        raise torch.OutOfMemoryError("none left")
+    with monkeypatch.context() as m:
+        m.setattr(paged, "send", no_memory)
+        with pytest.raises(torch.OutOfMemoryError):
+            c.reserve_all([(s, 1) for s in taken])
+    c.reserve_all([(s, 1) for s in taken])
+    assert bool((view[taken] == 0).all()) and bool((view[slots[1]] == 5).all())
+
+
 def test_random_walk_keeps_the_books():
     rnd = random.Random(3)
     c = make_cache(window=70, max_tokens=64 * 40)
