@@ -243,8 +243,8 @@ gemm_plain_tile_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* _
 // time): no load waits for another wave, and a wave asks for all of its stretch of W at once (16 pieces of 8 elements a lane), for A
 // some pieces ahead, and splits both in registers. The stretches' sums meet in LDS, where the first wave adds them in
 // their order. Short products through a narrow middle are here too, and those of heads with a matrix each: a wave on vector products, 16 columns
-// and 8 rows, which they had, took at 1 | 8 | 24 rows of bfloat16 weights (2048 x 128) 3.1 | 3.5 | 3.8 us, now 2.6 | 2.6 | 2.6; (4096 x 1024)
-// 14.5 | 16.7 | 19.3, now 5.2 | 5.4 | 7.4; (16 heads of 128 x 512) 7.5 | 8.8 | 9.8, now 3.8 | 4.1 | 4.5.
+// and 8 rows, which they had, took at 1 | 8 | 24 rows of bfloat16 weights (2048 x 128) 3.4 | 3.8 | 4.1 us, now 2.9 | 3.0 | 3.0; (4096 x 1024)
+// 13.5 | 15.9 | 19.2, now 5.1 | 5.6 | 7.7; (16 heads of 128 x 512) 7.7 | 9.1 | 10.1, now 4.3 | 4.6 | 5.0.
 #define WAVE_WAVES 8
 template <class TA, class TW, class TC, bool ACCUM, int MB, int NB, int AHEAD, int HOW>
 __global__ void __launch_bounds__(WAVE_WAVES * HB_WAVE, AHEAD == 8 ? 4 : 2)
@@ -364,9 +364,10 @@ gemm_plain_stream_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC*
 // tiles a CU gets, and no less than the chain from its reads of LDS over its products and the next stage's splitting to the barrier. Both sides float32 | one of
 // them bfloat16: 16 x 16 8.0 | 5.3, 32 x 32 by a wave 16.2 | 11.5, tiles of 32 x 32 0.23 | 0.18 a stage (at least 0.295 | 0.27), 64 x 64 0.48 | 0.35,
 // 128 x 128 1.35 | 0.80. Measured, microseconds by 16 x 16 / 32 x 32 / tiles of 32 / 64 / 128 [the float32 matrix instructions before], float32 weights: 17 x
-// 2048 x 2048 11 / 21 / 21 / 32 / 76 [22], 17 x 4096 x 2048 17 / 28 / 21 / 32 / 77 [29], 128 x 2048 x 2048 33 / 21 / 21 / 33 / 78 [23], 200 x 4096 x 2048 97 / 60 / 60 /
-// 37 / 78 [54], 563 x 4096 x 2048 262 / 139 / 137 / 94 / 80 [114], 563 x 6144 x 2048 388 / 207 / 210 / 126 / 93 [155], 563 x 2048 x 3072 232 / 133 / 113 / 89 / 116 [98];
-// bfloat16 weights: 64 x 2048 x 2048 13 / 16 / 19 / 25 / 49 [39], 563 x 4096 x 2048 191 / 105 / 110 / 69 / 52 [163].
+// 2048 x 2048 12 / 17 / 22 / 32 / 78 [22], 17 x 4096 x 2048 17 / 22 / 22 / 32 / 78 [29] (a square is estimated at 17 whatever its weights' bytes, and taken), 128 x 2048 x
+// 2048 35 / 19 / 22 / 32 / 80 [23], 200 x 4096 x 2048 103 / 58 / 60 / 34 / 80 [54], 563 x 4096 x 2048 281 / 138 / 137 / 92 / 81 [114], 563 x 6144 x 2048 417 / 206 /
+// 210 / 121 / 86 [155], 563 x 2048 x 3072 248 / 131 / 113 / 89 / 118 [98]; bfloat16 weights: 64 x 2048 x 2048 13 / 14 / 20 / 26 / 49 [39], 563 x 4096 x 2048 191 / 105 /
+// 109 / 69 / 51 [163].
 // waves: a grid of them holds the product; whole: K is whole stages, the larger tiles take nothing else; a decay's exponentials and logarithms are a tile's own tail: not 64 of them a lane.
 enum { STREAM, WAVE, WAVE_RING, WAVE_SQUARE, WAVE_HALVES, TILE_SINGLE, TILE_HALVES, TILE_QUADS, TILE_32, TILE_64, TILE_128 };
 static int gemm_plain_choice(int M, int N, int K, int batch, bool both, bool whole, bool decay, bool waves) {
@@ -399,8 +400,8 @@ static int gemm_plain_choice(int M, int N, int K, int batch, bool both, bool who
 template <class TA, class TW, class TC, bool ACCUM>
 static void launch_as(const TA* A, const TW* W, TC* C, int M, int N, int K, int lda, int ldw, int ldc,
                       hipStream_t stream, int batch, ptrdiff_t batch_a, ptrdiff_t batch_w, ptrdiff_t batch_c, DecayEpilogue ep) {
-    // (16-byte loads where rows and strides allow them, or 8-byte ones of bfloat16, 16-byte stores with either: bfloat16 rows 2,052 elements apart, 8 x
-    // 2048 x 2048 7.3 us, 512 rows 39, element by element 42 and 144)
+    // (16-byte loads where rows and strides allow them, or 8-byte ones of bfloat16, 16-byte stores with either: float32 rows on bfloat16 ones, 2,052
+    // elements apart, 8 x 2048 x 2048 6.2 us, 512 rows 45, element by element 47 and 158)
     auto borders = [&](int ea, int ew) {
         return K % ea == 0 && K % ew == 0 && lda % ea == 0 && ldw % ew == 0 && batch_a % ea == 0 && batch_w % ew == 0 &&
                (uintptr_t)A % (ea * sizeof(TA)) == 0 && (uintptr_t)W % (ew * sizeof(TW)) == 0 &&
@@ -531,7 +532,7 @@ extern "C" int hb_gemm_plain_decay(const void* A, int a_dtype, const void* W, in
 
 // Two such products of float32 rows with float32 sums (no decay for the first): C0 = A0 W0^T, C1 = A1 W1^T, shapes and strides alike, in
 // one launch: they wait for the same rows and not for each other, and a launch is the larger part of what one takes (8 x 2048 x 128,
-// bfloat16 weights: 2.6 us, the two together 2.6; 24 rows 2.6 and 2.9).
+// bfloat16 weights: 2.9 us, the two together 3.0; 24 rows 3.0 and 3.3).
 extern "C" int hb_gemm_plain_decay_pair(const float* A0, const void* W0, float* C0, const float* A1, const void* W1, float* C1,
                                         int w_dtype, int M, int N, int K, int lda, int ldw, int ldc, const float* A_log,
                                         const float* dt_bias, int D, float root, hipStream_t stream) {

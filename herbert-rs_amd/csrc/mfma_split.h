@@ -72,8 +72,8 @@ __device__ __forceinline__ void ends(Oct<bf16>& o, int left) {
 }
 
 // A float32 number's parts are those of 2^16 times it: what it has below 2^-133, where bfloat16 ends, is not lost then, down to float32's own last
-// bit. (Operands of 1e-38 and 10: an error of 2.7e-3 without, 1.3e-7 so. It costs a product of few rows a tenth, float32 weights, 2 x 2048 x 2048 9.2 ->
-// 10.0 us, a tile 0 to 2 %.)
+// bit. (Operands of 1e-38 and 10: an error of 2.7e-3 without, 1.3e-7 so. It costs a product of few rows a tenth, float32 weights, 2 x 2048 x 2048 9.5 ->
+// 10.5 us, a tile 0 to 3 %.)
 #define SPLIT_SCALE 65536.f
 // Each rest, v - (float)part, is exact and one instruction: a product of two pairs and a sum, with -1 and 0. (The pair -1, 0 is hidden
 // from the compiler, which would write the float -1, whose halves are 0, -1, in its place.)
@@ -159,9 +159,9 @@ __device__ __forceinline__ bool hb_wild(f32x4 v) { return hb_wild(v[0]) || hb_wi
 // Sums of a 16 x 16 block that are not finite, as plain float32 has them; all of a wave calls this. row_of(i): the block's i-th row of A, null
 // beyond the last; W: its first row, `columns` of them. A row of A with a NaN is NaN throughout. In others what is not finite
 // among the operands says what the sum is, whatever its order, and only sums of finite numbers (parts or sums beyond the range) are
-// summed again in their order. A wave looks at 64 elements of a row at a time. A product of 8 rows with 2048 x 2048 float32 weights, 10.7 us, takes 12.4
-// where a row is NaN, 52 where one holds an infinity and 93 where one holds 3.4e38 (an output a lane, an element at a time: 504); of
-// 512 rows, 4096 x 4096, 139, 150, 354 and 536 us (2,322). (Sixteen columns at a time: 42 and 270 us with an infinity, but registers that cost
+// summed again in their order. A wave looks at 64 elements of a row at a time. A product of 8 rows with 2048 x 2048 float32 weights, 11.3 us, takes 13.2
+// where a row is NaN, 53 where one holds an infinity and 92 where one holds 3.4e38 (an output a lane, an element at a time: 504); of
+// 512 rows, 4096 x 4096, 124, 127, 338 and 532 us (2,322). (Sixteen columns at a time: 42 and 270 us with an infinity, but registers that cost
 // the tiles of 64 x 64 one of two workgroups a CU.)
 template <class TA, class TW, class Rows>
 __device__ __forceinline__ void mend_block(Rows row_of, const TW* W, size_t ldw, int columns, int K, int block, f32x4& sums) {

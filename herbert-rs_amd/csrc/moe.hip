@@ -449,8 +449,8 @@ moe_gemm_plain_kernel(const TA* __restrict__ A, const TW* __restrict__ W, TC* __
 // The same where rows lie on 16-byte borders: the split products of mfma_split.h, a workgroup on 32 rows of an expert's matrix and all of a
 // tile's rows, a wave on every stretch of k (up to GROUPED_WAVES at a time), the stretches' sums added in their order. Up to 16
 // rows are one pass over the matrix' rows and bound by their bytes, more rows two blocks of 16 at a time, which read them again from
-// the caches. Gate and up of two tokens, 8 experts of 1536 x 2048, 25 us, their down product (768) 17; of 200 tokens,
-// 32 experts, 147 and 89; the kernel above, one chain of vector multiply-adds: 303, 116, 445 and 187.
+// the caches. Gate and up of two tokens, four of 8 experts each (1536 x 2048), 24 us, their down product (2048 x 768) 15; of 200 tokens, four of
+// 32 experts each, 155 and 85; the kernel above, one chain of vector multiply-adds: 268, 101, 462 and 155.
 #define GROUPED_WAVES 8
 template <class TA, class TW, int MB, int AHEAD, int A_AHEAD>
 __device__ __forceinline__ void grouped_plain_rows(const TA* __restrict__ A, const TW* __restrict__ We, float* __restrict__ C, const int* src, int from,
