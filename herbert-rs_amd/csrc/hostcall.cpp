@@ -8,6 +8,8 @@
 
 #include <stdint.h>
 
+#include <exception>
+
 #if !defined(__x86_64__) || !defined(__linux__)
 #error "entry points are called as the x86-64 System V calling convention passes their arguments"
 #endif
@@ -80,31 +82,35 @@ PyObject* invoke(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return PyLong_FromLong(rc);
 }
 
+bool has_form(const at::Tensor& t, PyObject* dtype, PyObject* shape) {
+    if (!t.is_cuda() || !t.is_contiguous()) return false;
+    if (dtype != Py_None && (!THPDtype_Check(dtype) || ((THPDtype*)dtype)->scalar_type != t.scalar_type())) return false;
+    if (shape == Py_None) return true;
+    if (!PyTuple_Check(shape) || PyTuple_GET_SIZE(shape) != t.dim()) return false;
+    for (int64_t i = 0; i < t.dim(); ++i) {
+        PyObject* want = PyTuple_GET_ITEM(shape, i);
+        if (want == Py_None) continue;
+        const long long size = PyLong_AsLongLong(want);
+        if ((size == -1 && PyErr_Occurred()) || size != t.size(i)) return false;
+    }
+    return true;
+}
+
 // fits(tensor, dtype or None, shape or None): True for a contiguous tensor on the GPU of that type and shape (None within the
-// shape: any size). Anything else is False, and the caller says what is wrong.
+// shape: any size). Anything else is False, and the caller says what is wrong; also a tensor that throws where it is asked (a sparse one
+// or a subclass has no strides to look at): an exception of C++ must not leave a function that the interpreter called.
 PyObject* fits(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (n != 3) {
         PyErr_SetString(PyExc_TypeError, "a tensor, a type and a shape are needed");
         return nullptr;
     }
-    if (!THPVariable_Check(args[0])) Py_RETURN_FALSE;
-    const at::Tensor& t = THPVariable_Unpack(args[0]);
-    if (!t.is_cuda() || !t.is_contiguous()) Py_RETURN_FALSE;
-    if (args[1] != Py_None && (!THPDtype_Check(args[1]) || ((THPDtype*)args[1])->scalar_type != t.scalar_type())) Py_RETURN_FALSE;
-    if (args[2] == Py_None) Py_RETURN_TRUE;
-    PyObject* shape = args[2];
-    if (!PyTuple_Check(shape) || PyTuple_GET_SIZE(shape) != t.dim()) Py_RETURN_FALSE;
-    for (int64_t i = 0; i < t.dim(); ++i) {
-        PyObject* want = PyTuple_GET_ITEM(shape, i);
-        if (want == Py_None) continue;
-        const long long size = PyLong_AsLongLong(want);
-        if (size == -1 && PyErr_Occurred()) {
-            PyErr_Clear();
-            Py_RETURN_FALSE;
-        }
-        if (size != t.size(i)) Py_RETURN_FALSE;
+    bool is = false;
+    try {
+        is = THPVariable_Check(args[0]) && has_form(THPVariable_Unpack(args[0]), args[1], args[2]);
+    } catch (const std::exception&) {
     }
-    Py_RETURN_TRUE;
+    PyErr_Clear();
+    return PyBool_FromLong(is);
 }
 
 PyMethodDef methods[] = {{"entry", make_entry, METH_VARARGS, nullptr},

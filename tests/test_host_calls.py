@@ -80,6 +80,25 @@ def test_a_tensor_off_the_gpu_is_refused():
             ops._check(wrong, "rows")
 
 
+class Stubborn(torch.Tensor):
+    """Says that it lies on the GPU and raises whatever else it is asked."""
+    @staticmethod
+    def __new__(cls, policy):
+        return torch.Tensor._make_wrapper_subclass(cls, (2, 3), dtype=torch.float32, device="cuda", dispatch_sizes_strides_policy=policy)
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        raise RuntimeError("not to be asked")
+
+
+@pytest.mark.parametrize("policy", ["strides", "sizes"])
+def test_a_tensor_that_raises_is_refused_with_its_own_error(policy):
+    t = Stubborn(policy)
+    assert lib.host().fits(t, torch.float32, (2, 3)) is False
+    with pytest.raises(RuntimeError, match="not to be asked"):
+        ops._check(t, "rows", torch.float32, (2, 3))
+
+
 @pytest.mark.gpu
 def test_what_an_operand_must_be():
     t = torch.zeros(3, 4, 5, device="cuda")
