@@ -234,6 +234,12 @@ class Cache:
             self.clear_slots(self._taken)
             self._taken = set()     # (a clearing that found no memory is made again)
 
+    def clear_again(self, slots):
+        """The state of `slots` is zeros, as when they were taken: now, or where no memory is found for that, at the next call."""
+        if self.state_groups:
+            self._taken.update(int(s) for s in slots)
+            self.clear_taken()
+
     def clear_slots(self, slots):
         """Fixed-size state of `slots` made zeros, a kernel a group however many they are."""
         if not self.state_groups or not slots:

@@ -244,7 +244,7 @@ class Engine:
             for e in entries:       # nothing was committed: give back what was taken for the step
                 self.cache.unreserve(e.slot)
             self.cache.restore_state(state_before)
-            self.cache.clear_slots([e.slot for e, start in zip(entries, starts) if start == 0])
+            self.cache.clear_again([e.slot for e, start in zip(entries, starts) if start == 0])
             raise
         for e in entries:
             self.cache.commit(e.slot, len(e.tokens))

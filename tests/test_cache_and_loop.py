@@ -146,6 +146,27 @@ def test_state_that_could_not_be_cleared_is_cleared_later(monkeypatch):
     assert bool((view[taken] == 0).all()) and bool((view[slots[1]] == 5).all())
 
 
+def test_state_that_could_not_be_cleared_again_is_cleared_later(monkeypatch):
+    """The same after a step that failed: `clear_again` itself may find no memory."""
+    import herbert_rs_amd.cache.paged as paged
+    c = make_cache(state=True)
+    slots = [c.alloc_slot() for _ in range(3)]
+    view = c.state_views(3)[0]
+    view.fill_(5.0)
+
+    def no_memory(*args):
+        raise torch.OutOfMemoryError("none left")
+    with monkeypatch.context() as m:
+        m.setattr(paged, "send", no_memory)
+        with pytest.raises(torch.OutOfMemoryError):
+            c.clear_again([slots[0], slots[2]])
+    assert bool((view[slots] == 5).all())
+    c.reserve(slots[0], 1)
+    assert bool((view[[slots[0], slots[2]]] == 0).all()) and bool((view[slots[1]] == 5).all())
+    c.clear_again([slots[1]])
+    assert bool((view[slots] == 0).all())
+
+
 def test_random_walk_keeps_the_books():
     rnd = random.Random(3)
     c = make_cache(window=70, max_tokens=64 * 40)

@@ -539,6 +539,43 @@ def test_slots_that_come_back_start_from_zeros_whichever_they_are():
         assert torch.allclose(step(engine, [slots[i] for i in back], [seqs[i] for i in back]), want[back], rtol=1e-5, atol=1e-5)
 
 
+def test_a_first_step_that_fails_for_want_of_memory_starts_from_zeros_again(monkeypatch):
+    """First steps of slots that are no neighbours fail after the state has changed, and so does clearing it, whose list of slots finds no
+    memory: the same step, run again, gives what it gives on a fresh cache."""
+    import herbert_rs_amd.cache.paged as paged
+    from herbert_rs_amd.weights import random_tensors
+    from herbert_rs_amd.engine.model import Model
+    spec = toy_spec()
+    w = random_tensors(Model(spec).tensor_needs(), 3, "float32", std=0.15, norm_std=0.1)
+    seqs = [[5, 9, 33, 2, 41], [7, 3, 50, 1]]
+
+    def run(fail_once):
+        engine = Engine(None, spec, w, dtype="float32", max_tokens=512)
+        slots = [engine.alloc_slot() for _ in range(3)]
+        entries = [StepEntry(s, t, list(range(len(t)))) for s, t in zip((slots[0], slots[2]), seqs)]
+        if fail_once:
+            mixer = engine.model.blocks[0].mixer
+            real = mixer.forward
+
+            def no_memory(*args):
+                raise torch.OutOfMemoryError("none left")
+
+            def failing(ctx, y, x):
+                real(ctx, y, x)
+                m.setattr(paged, "send", no_memory)
+                raise torch.OutOfMemoryError("none left")
+            with monkeypatch.context() as m:
+                engine.cache.reserve(slots[0], 1), engine.cache.unreserve(slots[0])     # (all three slots were cleared as neighbours)
+                mixer.forward = failing
+                with pytest.raises(torch.OutOfMemoryError):
+                    engine.step(entries)
+                mixer.forward = real
+            assert any(bool(g.data[:, slots[0]].any()) for g in engine.cache.state_groups.values())
+        return engine.step(entries).cpu()
+
+    assert torch.equal(run(True), run(False))
+
+
 @register("mixer", "toy_decay_on_the_gpu")
 class ToyDecayOnTheGpu(ToyDecayMixer):
     """The same recurrence, but a step in which every sequence brings one token does GPU work only:
