@@ -231,8 +231,9 @@ class Cache:
         """Clear the state of the slots that were taken since the last call. Whoever is to read or write state calls it, and
         so does whoever makes room for a step: views of the state may be held from before."""
         if self._taken:
-            self.clear_slots(self._taken)
-            self._taken = set()     # (a clearing that found no memory is made again)
+            taken = set(self._taken)
+            self.clear_slots(taken)
+            self._taken -= taken    # (a clearing that found no memory is made again, a slot that was taken meanwhile is still to be cleared)
 
     def clear_again(self, slots):
         """The state of `slots` is zeros, as when they were taken: now, or where no memory is found for that, at the next call."""

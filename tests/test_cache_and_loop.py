@@ -167,6 +167,24 @@ def test_state_that_could_not_be_cleared_again_is_cleared_later(monkeypatch):
     assert bool((view[slots] == 0).all())
 
 
+def test_a_slot_taken_while_others_are_cleared_is_cleared_too(monkeypatch):
+    """As by another thread that takes one between the kernel and the books."""
+    c = make_cache(state=True)
+    view = c.state_views(3)[0]
+    view.fill_(5.0)
+    slots, clear = [c.alloc_slot()], c.clear_slots
+
+    def clear_and_take(which):
+        clear(which)
+        if len(slots) == 1:
+            slots.append(c.alloc_slot())
+    monkeypatch.setattr(c, "clear_slots", clear_and_take)
+    c.reserve(slots[0], 1)
+    assert len(slots) == 2
+    c.reserve(slots[1], 1)
+    assert bool((view[slots] == 0).all())
+
+
 def test_random_walk_keeps_the_books():
     rnd = random.Random(3)
     c = make_cache(window=70, max_tokens=64 * 40)
