@@ -32,7 +32,6 @@ HB_MODULE_ERROR_SLOT()
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 #define EPI_STORE 0
 #define EPI_ADD 1
@@ -667,14 +666,16 @@ static void pick_skinny(const void* X, const void* W, void* C, int M, int N, int
 // The product for many rows (prompts). Tiles go from global memory straight into LDS
 // (hb_load_to_lds) through rings of stages that are loaded ahead of the MFMAs; what has landed
 // is waited for by count (hb_wait_vmcnt) before a bare barrier (hb_workgroup_barrier).
-// 32x32x16 MFMA (of the two bf16 shapes the one with the higher rate), weight rows first: an
-// operand is 32 rows x 16 k, lane l = row l % 32, k 8 (l / 32) .. + 8; a lane ends with 16 sums
-// of one m: n = 8 q + 4 (l / 32) + j for register 4 q + j.
+// 16x16x32 MFMA, weight rows first: an operand is 16 rows x 32 k, lane l = row l % 16, k 8 (l / 16) .. + 8;
+// a lane ends with 4 sums of one m: n = 4 (l / 16) + j for register j. Of the two bf16 shapes this is the
+// one that takes less power: the card lowers its clock when the matrix units work on numbers that are
+// not all alike (from 2.4 GHz to 1.75 with 32x32x16 and to 2.0 with 16x16x32, both issued back to back
+// from registers on normal random numbers), and the rates are then 1.74 to 1.83 and 2.04 to 2.11 PFLOP/s.
+// (On zeros both reach 2.4: measurements on zeros say nothing about prompts.)
 // Weights lie in LDS as in memory when packed: 1 KB blocks of 16 rows x 32 k, chunk
-// 16 (k / 8 % 4) + row % 16. For the k-half h of a k-step of 32 an operand is then: block
-// (l % 32) / 16 of a pair of blocks, chunk 16 (2 h + l / 32) + l % 16: 16 lanes read 256
-// contiguous bytes, free of bank conflicts.
-// Workgroup: WNW x WMW waves, each TNB x TMB blocks of 16: BN = 16 TNB WNW, BM = 16 TMB WMW.
+// 16 (k / 8 % 4) + row % 16, which is the operand of lane (chunk): a wave reads 1 KB in a row, free
+// of bank conflicts.
+// Workgroup: WNW x WMW waves, each TN x TM blocks of 16: BN = 16 TN WNW, BM = 16 TM WMW.
 // Workgroups go round the 8 XCDs, each with an L2 of its own: an XCD takes a run of tiles, and
 // within it bands of 8 tiles in m are walked n first, so that the workgroups that are resident
 // together share both their weight and their activation panels in that L2.
@@ -691,113 +692,99 @@ __device__ __forceinline__ bool tile_of_workgroup(int m_tiles, int n_tiles, int&
     return true;
 }
 
-// A wave's sums to memory. m_base, n_base: first row and column of the wave's tile.
-template <int EPI, int TN32, int TM32, int GLU = GLU_SILU>
-__device__ __forceinline__ void store_wave_tile(const f32x16 (&acc)[TN32][TM32], void* Cv, int M, int N, int ldc,
-                                                int m_base, int n_base, int c32, int g2) {
+// A wave's sums to memory. m_base, n_base: first row and column of the wave's tile of TM x TN blocks of 16.
+template <int EPI, int TN, int TM, int GLU = GLU_SILU>
+__device__ __forceinline__ void store_wave_tile(const f32x4 (&acc)[TN][TM], void* Cv, int M, int N, int ldc,
+                                                int m_base, int n_base, int r16, int g4) {
 #pragma unroll
-    for (int b = 0; b < TM32; ++b) {
-        const int m = m_base + 32 * b + c32;
+    for (int b = 0; b < TM; ++b) {
+        const int m = m_base + 16 * b + r16;
         if (m >= M) continue;
-        if (EPI == EPI_ACT) {
+        if (EPI == EPI_ACT || EPI == EPI_SWIGLU) {
+            // (gated units: a block of gate rows and the block of the same outputs' up rows after it)
+            constexpr int STEP = EPI == EPI_SWIGLU ? 2 : 1;
+            const int outs = EPI == EPI_SWIGLU ? N / 2 : N;
             bf16* C = (bf16*)Cv;
 #pragma unroll
-            for (int a = 0; a < TN32; ++a)
+            for (int a = 0; a < TN; a += STEP) {
+                const int n = (n_base + 16 * a) / STEP + 4 * g4;
+                bf16x4 v;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int n = n_base + 32 * a + 8 * q + 4 * g2;
-                    bf16x4 v;
+                for (int j = 0; j < 4; ++j)
+                    v[j] = (__bf16)(EPI == EPI_SWIGLU ? glu_mul<GLU>(acc[a][b][j], acc[a + STEP - 1][b][j])
+                                                      : unary(acc[a][b][j], GLU));
+                if (n + 3 < outs && (ldc & 3) == 0) {
+                    *(bf16x4*)((__bf16*)C + (size_t)m * ldc + n) = v;
+                } else {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) v[j] = (__bf16)unary(acc[a][b][4 * q + j], GLU);
-                    if (n + 3 < N && (ldc & 3) == 0) {
-                        *(bf16x4*)((__bf16*)C + (size_t)m * ldc + n) = v;
-                    } else {
-#pragma unroll
-                        for (int j = 0; j < 4; ++j)
-                            if (n + j < N) ((__bf16*)C)[(size_t)m * ldc + n + j] = v[j];
-                    }
+                    for (int j = 0; j < 4; ++j)
+                        if (n + j < outs) ((__bf16*)C)[(size_t)m * ldc + n + j] = v[j];
                 }
-        } else if (EPI == EPI_SWIGLU) {
-            bf16* C = (bf16*)Cv;
-#pragma unroll
-            for (int a = 0; a < TN32; ++a)
-#pragma unroll
-                for (int q = 0; q < 2; ++q) {
-                    // rows 0..15 of a piece are gate rows, 16..31 the up rows of the same outputs
-                    const int n = (n_base + 32 * a) / 2 + 8 * q + 4 * g2;
-                    if (n + 3 < N / 2 && (ldc & 3) == 0) {
-                        bf16x4 v;
-#pragma unroll
-                        for (int j = 0; j < 4; ++j)
-                            v[j] = (__bf16)glu_mul<GLU>(acc[a][b][4 * q + j], acc[a][b][4 * q + 8 + j]);
-                        *(bf16x4*)((__bf16*)C + (size_t)m * ldc + n) = v;
-                    } else {
-#pragma unroll
-                        for (int j = 0; j < 4; ++j)
-                            if (n + j < N / 2)
-                                C[(size_t)m * ldc + n + j] = hb_from_float<bf16>(
-                                    glu_mul<GLU>(acc[a][b][4 * q + j], acc[a][b][4 * q + 8 + j]));
-                    }
-                }
+            }
         } else {
             float* C = (float*)Cv;
 #pragma unroll
-            for (int a = 0; a < TN32; ++a)
+            for (int a = 0; a < TN; ++a) {
+                const int n = n_base + 16 * a + 4 * g4;
+                float* dst = C + (size_t)m * ldc + n;
+                if (n + 3 < N && (ldc & 3) == 0) {
+                    f32x4 v = acc[a][b];
+                    if (EPI == EPI_ADD) v += *(const f32x4*)dst;
+                    *(f32x4*)dst = v;
+                } else {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int n = n_base + 32 * a + 8 * q + 4 * g2;
-                    float* dst = C + (size_t)m * ldc + n;
-                    if (n + 3 < N && (ldc & 3) == 0) {
-                        f32x4 v = {acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2],
-                                   acc[a][b][4 * q + 3]};
-                        if (EPI == EPI_ADD) v += *(const f32x4*)dst;
-                        *(f32x4*)dst = v;
-                    } else {
-#pragma unroll
-                        for (int j = 0; j < 4; ++j)
-                            if (n + j < N) {
-                                if (EPI == EPI_ADD)
-                                    dst[j] += acc[a][b][4 * q + j];
-                                else
-                                    dst[j] = acc[a][b][4 * q + j];
-                            }
-                    }
+                    for (int j = 0; j < 4; ++j)
+                        if (n + j < N) {
+                            if (EPI == EPI_ADD)
+                                dst[j] += acc[a][b][j];
+                            else
+                                dst[j] = acc[a][b][j];
+                        }
                 }
+            }
         }
     }
 }
 
 // The same through LDS, for float32 outputs of the large tiles: a lane's sums are runs of four
-// columns of 32 different rows, so a store instruction of the direct way touches 32 lines in
-// pieces of 32 bytes, and reading C back for the add does the same (a round of 256 x 256 tiles
-// spent 45 us beside its products with the store and 68 us with the add, against 19 us with the
-// bfloat16 SwiGLU output). Here a wave first lays PB x 32 rows of its tile into LDS of its own
-// (`stage`, rows of TN32 x 32 floats, the 16-byte chunk c of row r at chunk c ^ (r mod chunks)),
-// then reads them back along the rows: an instruction then moves whole rows, 512 contiguous
-// bytes for a tile 128 wide. Needs ldc and N in steps of 4 and C aligned to 16 bytes.
-template <int EPI, int TN32, int TM32, int PB>
-__device__ __forceinline__ void store_wave_tile_lds(const f32x16 (&acc)[TN32][TM32], float* C, int M, int N, int ldc,
-                                                    int m_base, int n_base, int lane, float* stage) {
-    static_assert(TM32 % PB == 0, "the passes divide the wave's tile");
-    constexpr int CH = TN32 * 8;            // 16-byte chunks of a row
+// columns of 16 different rows, so a store instruction of the direct way touches 16 lines in
+// pieces of 64 bytes, and reading C back for the add does the same. Here a wave first lays PB x 16
+// rows of its tile into LDS of its own (`stage`, rows of TN x 16 floats, the 16-byte chunk c of row r
+// at chunk c ^ (r mod chunks)), then reads them back along the rows: an instruction then moves whole
+// rows, 512 contiguous bytes for a tile 128 wide. Where ldc or N is no multiple of 4 or C lies off a
+// 16-byte border (`whole` is false) they go to memory element by element.
+template <int EPI, int TN, int TM, int PB>
+__device__ __forceinline__ void store_wave_tile_lds(const f32x4 (&acc)[TN][TM], float* C, int M, int N, int ldc,
+                                                    int m_base, int n_base, int lane, float* stage, bool whole) {
+    static_assert(TM % PB == 0, "the passes divide the wave's tile");
+    constexpr int CH = TN * 4;              // 16-byte chunks of a row
+    static_assert((CH & (CH - 1)) == 0, "chunks change places by their bits");
     constexpr int RPI = 64 / CH;            // rows an instruction moves
-    constexpr int ITER = PB * 32 / RPI;
+    constexpr int ITER = PB * 16 / RPI;
     constexpr int GROUP = ITER < 8 ? ITER : 8;
-    const int c32 = lane & 31, g2 = lane >> 5;
+    const int r16 = lane & 15, g4 = lane >> 4;
     const int rrow = lane / CH, rchunk = lane % CH;
 #pragma unroll
-    for (int b0 = 0; b0 < TM32; b0 += PB) {
+    for (int b0 = 0; b0 < TM; b0 += PB) {
+        __builtin_amdgcn_sched_barrier(0);      // (a pass after the other: all at once take more registers than there are)
 #pragma unroll
         for (int bb = 0; bb < PB; ++bb)
 #pragma unroll
-            for (int a = 0; a < TN32; ++a)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int row = 32 * bb + c32, chunk = 8 * a + 2 * q + g2;
-                    const f32x4 v = {acc[a][b0 + bb][4 * q], acc[a][b0 + bb][4 * q + 1], acc[a][b0 + bb][4 * q + 2],
-                                     acc[a][b0 + bb][4 * q + 3]};
-                    *(f32x4*)(stage + row * (CH * 4) + ((chunk ^ (row & (CH - 1))) * 4)) = v;
+            for (int a = 0; a < TN; ++a) {
+                const int row = 16 * bb + r16, chunk = 4 * a + g4;
+                *(f32x4*)(stage + row * (CH * 4) + ((chunk ^ (row & (CH - 1))) * 4)) = acc[a][b0 + bb];
+            }
+        if (!whole) {
+            for (int i = 0; i < PB * 16; ++i) {
+                const int m = m_base + 16 * b0 + i;
+                for (int c = lane; c < CH * 4 && m < M && n_base + c < N; c += 64) {
+                    float* const dst = C + (size_t)m * ldc + n_base + c;
+                    const float v = stage[i * (CH * 4) + (((c >> 2) ^ (i & (CH - 1))) * 4) + (c & 3)];
+                    *dst = EPI == EPI_ADD ? *dst + v : v;
                 }
+            }
+            continue;
+        }
 #pragma unroll
         for (int i0 = 0; i0 < ITER; i0 += GROUP) {
             f32x4 before[GROUP];
@@ -805,14 +792,14 @@ __device__ __forceinline__ void store_wave_tile_lds(const f32x16 (&acc)[TN32][TM
 #pragma unroll
                 for (int u = 0; u < GROUP; ++u) {
                     const int row = (i0 + u) * RPI + rrow;
-                    const int m = m_base + 32 * b0 + row, n = n_base + 4 * rchunk;
+                    const int m = m_base + 16 * b0 + row, n = n_base + 4 * rchunk;
                     before[u] = (m < M && n < N) ? *(const f32x4*)(C + (size_t)m * ldc + n) : f32x4{0.f, 0.f, 0.f, 0.f};
                 }
             }
 #pragma unroll
             for (int u = 0; u < GROUP; ++u) {
                 const int row = (i0 + u) * RPI + rrow;
-                const int m = m_base + 32 * b0 + row, n = n_base + 4 * rchunk;
+                const int m = m_base + 16 * b0 + row, n = n_base + 4 * rchunk;
                 f32x4 v = *(const f32x4*)(stage + row * (CH * 4) + ((rchunk ^ (row & (CH - 1))) * 4));
                 if (EPI == EPI_ADD) v += before[u];
                 if (m < M && n < N) *(f32x4*)(C + (size_t)m * ldc + n) = v;
@@ -821,89 +808,69 @@ __device__ __forceinline__ void store_wave_tile_lds(const f32x16 (&acc)[TN32][TM
     }
 }
 
-// The SwiGLU outputs of the large tiles through LDS as well. A lane holds runs of four outputs of
-// 32 different rows, 8 bytes each: a store instruction of the direct way touches 32 lines in pieces
-// of 16 bytes (a round of 256 x 256 tiles spent 15 us beside its products that way, for a quarter
-// of the bytes that the float32 store moves in 8). Here a wave lays its whole tile's outputs into
-// LDS of its own (rows of TN32 x 16 bfloat16, the 16-byte chunk c of row r at chunk c ^ (r mod
-// chunks), or (c + r) mod chunks where the chunks are no power of two), then reads them back
-// along the rows: an instruction stores whole rows, 128 contiguous bytes for a tile 128 wide.
-// n_base: the wave's first column among the interleaved gate/up columns. Needs ldc in steps of
-// 8 and C aligned to 16 bytes.
-template <int TN32, int TM32, int GLU>
-__device__ __forceinline__ void store_wave_tile_swiglu_lds(const f32x16 (&acc)[TN32][TM32], bf16* C, int M, int N,
-                                                           int ldc, int m_base, int n_base, int lane, bf16* stage) {
-    constexpr int CH = 2 * TN32;            // 16-byte chunks of a row: 16 outputs a piece of 32 columns
+// The bfloat16 outputs of the large tiles (gated units, activations) through LDS as well. A lane holds
+// runs of four outputs of 16 different rows, 8 bytes each: a store instruction of the direct way touches
+// 16 lines in pieces of 32 bytes. Here a wave lays its whole tile's outputs into LDS of its own (the
+// 16-byte chunk c of row r at chunk c ^ (r mod chunks), or (c + r) mod chunks where the chunks are no
+// power of two), then reads them back along the rows: an instruction stores whole rows, 128 contiguous
+// bytes for a gated tile 128 wide. n_base: the wave's first column (of the gate/up columns). Where ldc is
+// no multiple of 8 or C lies off a 16-byte border (`whole` is false) they go to memory element by element.
+// `second`: the second gated unit or activation of its kind (GLU_RELU, UNARY_GELU) in place of the first; taken by a
+// choice at every output, since two copies of this code have the compiler move sums to memory.
+template <int EPI, int TN, int TM>
+__device__ __forceinline__ void store_wave_tile_bf16_lds(const f32x4 (&acc)[TN][TM], bf16* C, int M, int N, int ldc, int m_base,
+                                                         int n_base, int lane, bf16* stage, bool whole, bool second) {
+    constexpr int STEP = EPI == EPI_ACT ? 1 : 2;
+    constexpr int CH = 2 * TN / STEP;       // 16-byte chunks of a row: 16 outputs a block, or a gate block and its up block
     constexpr int RPI = 64 / CH;            // rows an instruction moves
-    constexpr int ROWS = 32 * TM32;
+    constexpr int ROWS = 16 * TM;
     constexpr bool POW2 = (CH & (CH - 1)) == 0;
     auto place = [&](int row, int chunk) { return POW2 ? (chunk ^ (row & (CH - 1))) : (chunk + row) % CH; };
-    const int c32 = lane & 31, g2 = lane >> 5;
+    const int r16 = lane & 15, g4 = lane >> 4;
+    const int outs = N / STEP;
+    auto output = [&](float g, float u) {
+        if (EPI == EPI_GEGLU) return gelu_tanh_mul(g, u);
+        const float z = fmaxf(g, 0.f);
+        float f = EPI == EPI_ACT ? gelu_erf(g) : silu_mul(g, u);
+        asm volatile("" : "+v"(f));                 // (both, then a select: no branch an output)
+        if (EPI == EPI_ACT) return second ? f : z * z;
+        return second ? z * u : f;
+    };
 #pragma unroll
-    for (int b = 0; b < TM32; ++b)
+    for (int b = 0; b < TM; ++b) {
+        __builtin_amdgcn_sched_barrier(0);      // (a block of rows after the other: all at once take more registers than there are)
 #pragma unroll
-        for (int a = 0; a < TN32; ++a)
+        for (int a = 0; a < TN; a += STEP) {
+            const int row = 16 * b + r16;
+            bf16x4 v;
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                // rows 0..15 of a piece are gate rows, 16..31 the up rows of the same outputs
-                const int row = 32 * b + c32;
-                bf16x4 v;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) v[j] = (__bf16)glu_mul<GLU>(acc[a][b][4 * q + j], acc[a][b][4 * q + 8 + j]);
-                *(bf16x4*)((__bf16*)stage + row * (CH * 8) + place(row, 2 * a + q) * 8 + 4 * g2) = v;
-            }
+            for (int j = 0; j < 4; ++j) v[j] = (__bf16)output(acc[a][b][j], acc[a + STEP - 1][b][j]);
+            *(bf16x4*)((__bf16*)stage + row * (CH * 8) + place(row, 2 * a / STEP + (g4 >> 1)) * 8 + 4 * (g4 & 1)) = v;
+        }
+    }
+    if (!whole) {
+        for (int row = 0; row < ROWS; ++row) {
+            const int m = m_base + row;
+            for (int c = lane; c < CH * 8 && m < M && n_base / STEP + c < outs; c += 64)
+                C[(size_t)m * ldc + n_base / STEP + c] = stage[row * (CH * 8) + place(row, c >> 3) * 8 + (c & 7)];
+        }
+        return;
+    }
     const int rrow = lane / CH, rchunk = lane % CH;
     if (lane >= RPI * CH) return;
 #pragma unroll
     for (int i = 0; i < (ROWS + RPI - 1) / RPI; ++i) {
         const int row = i * RPI + rrow;
         if (row >= ROWS) break;
-        const int m = m_base + row, n = n_base / 2 + 8 * rchunk;
+        const int m = m_base + row, n = n_base / STEP + 8 * rchunk;
         const bf16x8 v = *(const bf16x8*)((const __bf16*)stage + row * (CH * 8) + place(row, rchunk) * 8);
         if (m >= M) continue;
-        if (n + 7 < N / 2) {
+        if (n + 7 < outs) {
             *(bf16x8*)((__bf16*)C + (size_t)m * ldc + n) = v;
         } else {
 #pragma unroll
             for (int j = 0; j < 8; ++j)
-                if (n + j < N / 2) ((__bf16*)C)[(size_t)m * ldc + n + j] = v[j];
-        }
-    }
-}
-
-// The outputs of epilogue 5 through LDS in the same way: rows of TN32 x 32 bfloat16.
-template <int TN32, int TM32, int ACT>
-__device__ __forceinline__ void store_wave_tile_act_lds(const f32x16 (&acc)[TN32][TM32], bf16* C, int M, int N, int ldc,
-                                                        int m_base, int n_base, int lane, bf16* stage) {
-    constexpr int CH = 4 * TN32;            // 16-byte chunks of a row (a power of two)
-    constexpr int RPI = 64 / CH;
-    constexpr int ROWS = 32 * TM32;
-    const int c32 = lane & 31, g2 = lane >> 5;
-#pragma unroll
-    for (int b = 0; b < TM32; ++b)
-#pragma unroll
-        for (int a = 0; a < TN32; ++a)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int row = 32 * b + c32;
-                bf16x4 v;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) v[j] = (__bf16)unary(acc[a][b][4 * q + j], ACT);
-                *(bf16x4*)((__bf16*)stage + row * (CH * 8) + (((4 * a + q) ^ (row & (CH - 1))) * 8) + 4 * g2) = v;
-            }
-    const int rrow = lane / CH, rchunk = lane % CH;
-#pragma unroll
-    for (int i = 0; i < ROWS / RPI; ++i) {
-        const int row = i * RPI + rrow;
-        const int m = m_base + row, n = n_base + 8 * rchunk;
-        const bf16x8 v = *(const bf16x8*)((const __bf16*)stage + row * (CH * 8) + ((rchunk ^ (row & (CH - 1))) * 8));
-        if (m >= M) continue;
-        if (n + 7 < N) {
-            *(bf16x8*)((__bf16*)C + (size_t)m * ldc + n) = v;
-        } else {
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (n + j < N) ((__bf16*)C)[(size_t)m * ldc + n + j] = v[j];
+                if (n + j < outs) ((__bf16*)C)[(size_t)m * ldc + n + j] = v[j];
         }
     }
 }
@@ -929,90 +896,75 @@ struct QkvEpilogue {
     int nq, nkv;
 };
 
-// lane: row m = m_base + 32 b + c32; register 4 q + j of piece a: element 32 a + 8 q + 4 g2 + j of the head
-template <int TN32, int TM32>
-__device__ __forceinline__ void store_wave_tile_qkv(f32x16 (&acc)[TN32][TM32], const QkvEpilogue& e, int M, int N,
-                                                    int m_base, int n_base, int c32, int g2) {
-    static_assert(TN32 == 4, "a wave's tile must be one head of 128 wide");
+// lane: row m = m_base + 16 b + r16; register j of block a: element 16 a + 4 g4 + j of the head
+template <int TN, int TM>
+__device__ __forceinline__ void store_wave_tile_qkv(f32x4 (&acc)[TN][TM], const QkvEpilogue& e, int M, int N,
+                                                    int m_base, int n_base, int r16, int g4) {
+    static_assert(TN == 8, "a wave's tile must be one head of 128 wide");
     if (n_base >= N) return;
     const int head = n_base / 128;
     const bool is_q = head < e.nq, is_v = head >= e.nq + e.nkv;
     const float* norm_w = is_q ? e.q_norm_w : e.k_norm_w;
 #pragma unroll
-    for (int b = 0; b < TM32; ++b) {
-        const int m = m_base + 32 * b + c32;
+    for (int b = 0; b < TM; ++b) {
+        __builtin_amdgcn_sched_barrier(0);
+        const int m = m_base + 16 * b + r16;
         const int mc = m < M ? m : M - 1;
         const int pos = e.positions[mc];
         if (!is_v) {
             if (norm_w) {
                 float ss = 0.f;
 #pragma unroll
-                for (int a = 0; a < 4; ++a)
+                for (int a = 0; a < 8; ++a)
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) ss = fmaf(acc[a][b][i], acc[a][b][i], ss);
+                    for (int j = 0; j < 4; ++j) ss = fmaf(acc[a][b][j], acc[a][b][j], ss);
+                ss += __shfl_xor(ss, 16, 64);
                 ss += __shfl_xor(ss, 32, 64);
                 const float inv = 1.0f / sqrtf(ss / 128.0f + e.eps);
 #pragma unroll
-                for (int a = 0; a < 4; ++a)
+                for (int a = 0; a < 8; ++a) {
+                    const f32x4 w = *(const f32x4*)(norm_w + 16 * a + 4 * g4);
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const f32x4 w = *(const f32x4*)(norm_w + 32 * a + 8 * q + 4 * g2);
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) acc[a][b][4 * q + j] = acc[a][b][4 * q + j] * inv * w[j];
-                    }
+                    for (int j = 0; j < 4; ++j) acc[a][b][j] = acc[a][b][j] * inv * w[j];
+                }
             }
             if (e.cos_t) {
-                // element d < 64 pairs with d + 64: pieces a and a + 2, the same register
+                // element d < 64 pairs with d + 64: blocks a and a + 4, the same register
 #pragma unroll
-                for (int a = 0; a < 2; ++a)
+                for (int a = 0; a < 4; ++a) {
+                    const size_t at = (size_t)pos * 64 + 16 * a + 4 * g4;
+                    const f32x4 c = *(const f32x4*)(e.cos_t + at), s = *(const f32x4*)(e.sin_t + at);
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const size_t at = (size_t)pos * 64 + 32 * a + 8 * q + 4 * g2;
-                        const f32x4 c = *(const f32x4*)(e.cos_t + at), s = *(const f32x4*)(e.sin_t + at);
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            const float x0 = acc[a][b][4 * q + j], x1 = acc[a + 2][b][4 * q + j];
-                            acc[a][b][4 * q + j] = x0 * c[j] - x1 * s[j];
-                            acc[a + 2][b][4 * q + j] = x0 * s[j] + x1 * c[j];
-                        }
+                    for (int j = 0; j < 4; ++j) {
+                        const float x0 = acc[a][b][j], x1 = acc[a + 4][b][j];
+                        acc[a][b][j] = x0 * c[j] - x1 * s[j];
+                        acc[a + 4][b][j] = x0 * s[j] + x1 * c[j];
                     }
+                }
             }
         }
         if (m >= M) continue;
-        if (is_q) {
-            bf16* dst = e.q_out + ((size_t)m * e.nq + head) * 128;
+        bf16* dst = e.q_out + ((size_t)m * e.nq + head) * 128;
+        if (!is_q) {
+            const int page = e.page_table[(size_t)e.slots[e.seq_of[m]] * e.max_pages + pos / 64];
+            const int in_page = pos % 64;
+            if (is_v) {
+                // transposed pages: for one element 16 lanes write 16 neighbouring tokens
+                bf16* vt = e.v_cache + ((size_t)page * e.nkv + (head - e.nq - e.nkv)) * 128 * 64 + in_page;
 #pragma unroll
-            for (int a = 0; a < 4; ++a)
+                for (int a = 0; a < 8; ++a)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    bf16x4 v;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) v[j] = (__bf16)acc[a][b][4 * q + j];
-                    *(bf16x4*)((__bf16*)dst + 32 * a + 8 * q + 4 * g2) = v;
-                }
-            continue;
+                    for (int j = 0; j < 4; ++j) vt[(size_t)(16 * a + 4 * g4 + j) * 64] = hb_from_float<bf16>(acc[a][b][j]);
+                continue;
+            }
+            dst = e.k_cache + (((size_t)page * e.nkv + (head - e.nq)) * 64 + in_page) * 128;
         }
-        const int page = e.page_table[(size_t)e.slots[e.seq_of[m]] * e.max_pages + pos / 64];
-        const int in_page = pos % 64;
-        if (!is_v) {
-            bf16* dst = e.k_cache + (((size_t)page * e.nkv + (head - e.nq)) * 64 + in_page) * 128;
 #pragma unroll
-            for (int a = 0; a < 4; ++a)
+        for (int a = 0; a < 8; ++a) {
+            bf16x4 v;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    bf16x4 v;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) v[j] = (__bf16)acc[a][b][4 * q + j];
-                    *(bf16x4*)((__bf16*)dst + 32 * a + 8 * q + 4 * g2) = v;
-                }
-        } else {
-            // transposed pages: for one element the 32 lanes of a half wave write 32 neighbouring tokens
-            bf16* dst = e.v_cache + ((size_t)page * e.nkv + (head - e.nq - e.nkv)) * 128 * 64 + in_page;
-#pragma unroll
-            for (int a = 0; a < 4; ++a)
-#pragma unroll
-                for (int i = 0; i < 16; ++i)
-                    dst[(size_t)(32 * a + 8 * (i >> 2) + 4 * g2 + (i & 3)) * 64] = hb_from_float<bf16>(acc[a][b][i]);
+            for (int j = 0; j < 4; ++j) v[j] = (__bf16)acc[a][b][j];
+            *(bf16x4*)((__bf16*)dst + 16 * a + 4 * g4) = v;
         }
     }
 }
@@ -1030,29 +982,47 @@ struct RowScale {
 // instruction, 8 lanes a row) and not half lines twice; the 16-byte chunk c of row r sits at
 // chunk c ^ ((r >> 1) & 7) of its row, so that the operand reads of 16 rows at one k fall into
 // 16 different bank groups. The weights have a ring of WST stages, the activations one of XST.
-// There is no branch in the main loop (the last step is peeled off), and what is no MFMA is
+// There is no branch in the main loop, and what is no MFMA is
 // dealt out between the MFMAs by hand: a wave has an MFMA in the pipe while it issues its reads
 // and loads, also right after the barrier, where no other wave could fill in. Operands are in
 // two sets of registers: the reads of a k-step go out during the MFMAs of the one before.
-template <int EPI, bool PACKED, int TNB, int TMB, int WNW, int WMW, int WST, int XST>
+// Where the loads go: a step has one barrier, after its first k-step, and behind it the stage of its own
+// step is free. SPREAD (the tall tiles, bound by their MFMAs): the operand that has a third stage (of
+// two such the activations) is loaded during the first k-step, two steps ahead, the other one during the
+// second, so that the CU's loads are dealt out over the whole step (8192 x 8192 x 8192 with eight waves:
+// 838 us, all in the second k-step 896). Otherwise (tiles that wait for memory) all loads go out
+// during the second k-step, WST and XST steps ahead.
+// Against the same loop on 32x32x16 MFMAs with two stages and all loads in the second k-step, on one card, random
+// numbers, us: 256 x 256 tiles 8192 x 8192 x 8192 (store) 822 -> 743, 2048 x 24576 x 4096 (gated) 331 -> 303,
+// 9004 x 12288 x 2048 (gated) 385 -> 354; 256 x 192 9004 x 2048 x 6144 (add) 230 -> 210; 256 x 128 2048 x 4096 x 12288
+// (add) 194 -> 177; 192 x 256 1000 x 24576 x 4096 (gated) 183 -> 166. Eight waves of 128 x 64 instead of four of 128 x 128
+// read half as many operands again from LDS: 864 us where these take 793.
+template <int EPI, bool PACKED, int TN, int TM, int WNW, int WMW, int WST, int XST>
 __global__ void __launch_bounds__(64 * WNW * WMW)
 gemm_tile_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, void* __restrict__ Cv, int M, int N,
                  int K, int ldc, int m_tiles, int n_tiles, float* __restrict__ partial, QkvEpilogue qkv,
                  RowScale scale) {
     constexpr int NW = WNW * WMW;
-    constexpr int BN = 16 * TNB * WNW, BM = 16 * TMB * WMW;
+    constexpr int BN = 16 * TN * WNW, BM = 16 * TM * WMW;
     constexpr int WBLK = BN / 16;                       // weight blocks of a k-step of 32
     constexpr int WL = WBLK / NW;                       // of which a wave loads
     constexpr int XR = BM / 8 / NW;                     // loads of 8 activation rows of a wave per step
     constexpr int W_STAGE = 2 * WBLK * 512, X_STAGE = BM * 64;      // elements
     constexpr int NLW = 2 * WL, NLX = XR;               // a wave's loads per step
     static_assert(WBLK % NW == 0 && BM % (8 * NW) == 0, "the loads must divide over the waves");
-    static_assert(TNB % 2 == 0 && TMB % 2 == 0, "a wave's tile is made of 32 x 32 pieces");
     static_assert((WST == 2 || WST == 3) && (XST == 2 || XST == 3),
                   "the wait before the barrier counts on the loads of at most one later step");
-    constexpr bool X_FIRST = XST <= WST;                // in a step's loads: the operand with the shorter ring first
-    constexpr int LATER = (WST == 3 ? NLW : 0) + (XST == 3 ? NLX : 0);   // loads that may be in flight at the barrier
-    constexpr int TN32 = TNB / 2, TM32 = TMB / 2;
+    constexpr bool SCALES = BM <= 32;                   // a handed-on norm comes with at most 16 rows
+    constexpr bool SPREAD = BM >= 128 && (WST == 3 || XST == 3);
+    constexpr bool X_EARLY = SPREAD && XST == 3, W_EARLY = SPREAD && XST == 2;     // loaded during the first k-step
+    constexpr int EARLY = (X_EARLY ? NLX : 0) + (W_EARLY ? NLW : 0), LATE = NLX + NLW - EARLY;
+    constexpr int X_AHEAD = X_EARLY ? 2 : XST, W_AHEAD = W_EARLY ? 2 : WST;        // steps
+    constexpr bool X_FIRST = XST <= WST;                // of loads in one k-step: the operand with the shorter ring first
+    // The last step is peeled off, with nothing to load; but where that makes the compiler move sums by way of memory
+    // (the largest tiles with bfloat16 outputs) it is a step like any other, which loads and reads what nobody uses.
+    constexpr bool PEELED = TN * TM <= 32 || !(EPI == EPI_SWIGLU || EPI == EPI_GEGLU || EPI == EPI_ACT);
+    // a wave's loads that may be in flight at the barrier of a step: those of steps later than the next one
+    constexpr int LATER = EARLY + (!W_EARLY && WST == 3 ? NLW : 0) + (!X_EARLY && XST == 3 ? NLX : 0);
     extern __shared__ __attribute__((aligned(1024))) bf16 lds[];    // [WST][W_STAGE], then [XST][X_STAGE]
     bf16* const xlds = lds + WST * W_STAGE;
 
@@ -1061,7 +1031,7 @@ gemm_tile_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, void* _
     const int m0 = m_tile * BM, n0 = n_tile * BN;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // uniform: LDS addresses stay scalar
-    const int r16 = lane & 15, g4 = lane >> 4, c32 = lane & 31, g2 = lane >> 5;
+    const int r16 = lane & 15, g4 = lane >> 4;
     const int wn = wave / WMW, wm = wave % WMW;
     // gridDim.y > 1: K is cut into slices over workgroups (few tiles, long K); a workgroup leaves the
     // sums of its slice in `partial` [slice][M][N] and gemm_slices_kernel adds the slices in order
@@ -1093,48 +1063,45 @@ gemm_tile_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, void* _
         if (m >= M) m = M - 1;
         xsrc[i] = X + (size_t)m * K + (((lane & 7) ^ ((r >> 1) & 7)) * 8) + (size_t)step0 * 64;
     }
-    // The idx-th load of a step: activations of step xstep into stage xstage, weights of step
-    // wstep into stage wstage. The operand with the shorter ring comes first: it is the one
-    // that is needed a step earlier.
-    auto load_one = [&](int xstep, int xstage, int wstep, int wstage, int idx) {
-        const bool is_x = X_FIRST ? idx < NLX : idx >= NLW;
-        const int i = X_FIRST ? (is_x ? idx : idx - NLX) : (is_x ? idx - NLW : idx);
-        if (is_x) {
-            hb_load_to_lds(xsrc[i] + (size_t)xstep * 64, xlds + xstage * X_STAGE + (wave * XR + i) * 512);
-        } else {
-            const int ks = i / WL, w = i % WL;
-            hb_load_to_lds(wsrc[w] + ((size_t)wstep * 2 + ks) * WSTEP,
-                           lds + wstage * W_STAGE + ks * WBLK * 512 + (wave * WL + w) * 512);
-        }
+    auto load_x = [&](int step, int stage, int i) {
+        hb_load_to_lds(xsrc[i] + (size_t)step * 64, xlds + stage * X_STAGE + (wave * XR + i) * 512);
     };
-    auto load_is_x = [&](int idx) { return X_FIRST ? idx < NLX : idx >= NLW; };
+    auto load_w = [&](int step, int stage, int i) {
+        const int ks = i / WL, w = i % WL;
+        hb_load_to_lds(wsrc[w] + ((size_t)step * 2 + ks) * WSTEP, lds + stage * W_STAGE + ks * WBLK * 512 + (wave * WL + w) * 512);
+    };
 
-    f32x16 acc[TN32][TM32];
+    f32x4 acc[TN][TM];
 #pragma unroll
-    for (int a = 0; a < TN32; ++a)
+    for (int a = 0; a < TN; ++a)
 #pragma unroll
-        for (int b = 0; b < TM32; ++b)
+        for (int b = 0; b < TM; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // The sums are held in accumulation registers where the loop begins and ends: without that the compiler moves
+    // them from one kind of register to the other between the MFMAs (a fifth of the issue slots for 256 of them).
+    auto hold = [&]() {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.f;
+        for (int a = 0; a < TN; ++a)
+#pragma unroll
+            for (int b = 0; b < TM; ++b) asm volatile("" : "+a"(acc[a][b]));
+    };
 
-    constexpr int NM = 2 * TN32 * TM32;              // MFMAs of a k-step of 32
-    constexpr int NR = 2 * (TN32 + TM32);            // operand reads of a k-step
-    constexpr int SLOTS = NM > 6 ? NM - 4 : NM;      // the last MFMAs cover the latency of the last reads
-    const int w_lane = (c32 >> 4) * 512 + (16 * g2 + (lane & 15)) * 8 + wn * TNB * 512;
-    const int x_lane = (wm * TMB * 16 + c32) * 64;
-    const int x_swizzle = (c32 >> 1) & 7;            // of this lane's rows: they are c32 + a multiple of 16
-    bf16x8 wv[2][2][TN32], xv[2][2][TM32];           // [set][k-half][piece]
+    constexpr int NM = TN * TM;                      // MFMAs of a k-step of 32
+    constexpr int NR = TN + TM;                      // operand reads of a k-step
+    constexpr int SLOTS = NM > 12 ? NM - 8 : NM;     // the last MFMAs cover the latency of the last reads
+    const int w_lane = lane * 8 + wn * TN * 512;
+    const int x_lane = (wm * TM * 16 + r16) * 64;
+    const int x_swizzle = (r16 >> 1) & 7;            // of this lane's rows: they are r16 + a multiple of 16
+    bf16x8 wv[2][TN], xv[2][TM];                     // [set][block]
     auto mfma_one = [&](int set, int j) {
-        const int h = j / (TN32 * TM32), a = j / TM32 % TN32, b = j % TM32;
-        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv[set][h][a], xv[set][h][b], acc[a][b], 0, 0, 0);
+        const int a = j / TM, b = j % TM;
+        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[set][a], xv[set][b], acc[a][b], 0, 0, 0);
     };
-    auto read_one = [&](int set, int step, int ks, int idx) {
-        const int h = idx / (TN32 + TM32), r = idx % (TN32 + TM32);
-        if (r < TN32)
-            wv[set][h][r] = *(const bf16x8*)(lds + (step % WST) * W_STAGE + ks * WBLK * 512 + w_lane + r * 1024 + h * 256);
+    auto read_one = [&](int set, int wstage, int xstage, int ks, int idx) {
+        // (all activations and the first weights are needed first)
+        if (idx < TM)
+            xv[set][idx] = *(const bf16x8*)(xlds + xstage * X_STAGE + x_lane + idx * 16 * 64 + (((4 * ks + g4) ^ x_swizzle) * 8));
         else
-            xv[set][h][r - TN32] = *(const bf16x8*)(xlds + (step % XST) * X_STAGE + x_lane + (r - TN32) * 32 * 64 +
-                                                    (((4 * ks + 2 * h + g2) ^ x_swizzle) * 8));
+            wv[set][idx - TM] = *(const bf16x8*)(lds + wstage * W_STAGE + ks * WBLK * 512 + w_lane + (idx - TM) * 512);
     };
     // between the MFMAs j and j + 1 of a k-step: nl loads and NR reads, dealt out evenly over the
     // first SLOTS MFMAs, the loads spread among the reads (a burst of loads from all waves at
@@ -1151,20 +1118,29 @@ gemm_tile_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, void* _
     };
     auto clamp = [&](int step) { return step < nsteps ? step : nsteps - 1; };   // past the end: the last step again
 
-    // in flight before the loop: steps 0 and 1, and step 2 of what has a ring of three stages
+    // in flight before the loop: steps 0 and 1, and step 2 of what is loaded three steps ahead
 #pragma unroll
-    for (int i = 0; i < NLX + NLW; ++i) load_one(0, 0, 0, 0, i);
+    for (int i = 0; i < NLX; ++i) load_x(0, 0, i);
 #pragma unroll
-    for (int i = 0; i < NLX + NLW; ++i) load_one(clamp(1), 1, clamp(1), 1, i);
+    for (int i = 0; i < NLW; ++i) load_w(0, 0, i);
 #pragma unroll
-    for (int i = 0; i < NLX + NLW; ++i)
-        if (load_is_x(i) ? XST == 3 : WST == 3) load_one(clamp(2), 2, clamp(2), 2, i);
+    for (int i = 0; i < NLX; ++i) load_x(clamp(1), 1, i);
+#pragma unroll
+    for (int i = 0; i < NLW; ++i) load_w(clamp(1), 1, i);
+    if constexpr (X_AHEAD == 3) {
+#pragma unroll
+        for (int i = 0; i < NLX; ++i) load_x(clamp(2), 2, i);
+    }
+    if constexpr (W_AHEAD == 3) {
+#pragma unroll
+        for (int i = 0; i < NLW; ++i) load_w(clamp(2), 2, i);
+    }
     // A handed-on norm: every row's sum of squares is added up here, behind the first loads, by
     // all threads (thread t: row t % MP, parts t / MP, t / MP + threads / MP, ...), then over the
     // lanes of a row and, after the barrier, over the waves in their order.
     float* const row_sums = (float*)(xlds + XST * X_STAGE);       // [NW][16]
     const int MP = M <= 1 ? 1 : (M <= 2 ? 2 : (M <= 4 ? 4 : (M <= 8 ? 8 : 16)));
-    if (scale.partial) {
+    if (SCALES && scale.partial) {
         // (asked for HP at a time: one after another, as a plain loop over the parts does it, every
         // part costs a trip to the L2; with 16 rows and 256 parts that were eight trips, 8 us)
         constexpr int HP = 16;
@@ -1183,117 +1159,109 @@ gemm_tile_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, void* _
         for (int d = 32; d >= MP; d >>= 1) sum += __shfl_xor(sum, d, 64);
         if (lane < MP) row_sums[wave * 16 + lane] = sum;
     }
-    hb_wait_vmcnt<NLX + NLW + LATER>();
+    hb_wait_vmcnt<NLX + NLW + (X_AHEAD == 3 ? NLX : 0) + (W_AHEAD == 3 ? NLW : 0)>();
     hb_workgroup_barrier();
-    float inv_rms = 1.f;          // of row c32 (the scaled product has at most 16 rows, all in the first piece)
-    if (scale.partial) {
+    float inv_rms = 1.f;          // of row r16 (the scaled product has at most 16 rows, all in the first block)
+    if (SCALES && scale.partial) {
         float sum = 0.f;
-        for (int w = 0; w < NW; ++w) sum += row_sums[w * 16 + (c32 & (MP - 1))];
+        for (int w = 0; w < NW; ++w) sum += row_sums[w * 16 + (r16 & (MP - 1))];
         inv_rms = 1.0f / sqrtf(sum / (float)K + scale.eps);
     }
 #pragma unroll
-    for (int i = 0; i < NR; ++i) read_one(0, 0, 0, i);
+    for (int i = 0; i < NR; ++i) read_one(0, 0, 0, 0, i);
+    hold();
 
-    for (int t = 0; t + 1 < nsteps; ++t) {
-        // first k-step of step t; between its MFMAs the reads of the second one
+    for (int t = 0; t + (PEELED ? 1 : 0) < nsteps; ++t) {
+        const int ws = t % WST, xs = t % XST, ws1 = (t + 1) % WST, xs1 = (t + 1) % XST;
+        const int xstep = clamp(t + X_AHEAD), wstep = clamp(t + W_AHEAD);
+        // First k-step of step t; between its MFMAs the reads of the second one and the early loads, into
+        // the stage that step t - 1 left at its barrier.
 #pragma unroll
         for (int j = 0; j < NM; ++j) {
             mfma_one(0, j);
-            between(j, 0, [&](int) {}, [&](int i) { read_one(1, t, 1, i); });
+            between(j, EARLY, [&](int i) {
+                if constexpr (X_EARLY) load_x(xstep, (t + 2) % XST, i);
+                else load_w(wstep, (t + 2) % WST, i);
+            }, [&](int i) { read_one(1, ws, xs, 1, i); });
             __builtin_amdgcn_sched_barrier(0);
         }
-        // Step t + 1 has landed (of what this wave has in flight only the weights of the later
-        // steps may be missing), after the barrier for every wave, and nobody reads step t any
-        // more: between the MFMAs of its second k-step go the loads into its stages, the
-        // activations of step t + XST and the weights of step t + WST, and the reads of step t + 1.
+        // Step t + 1 has landed (of what this wave has in flight only loads of later steps may be
+        // missing), after the barrier for every wave, and nobody reads step t any more: between the MFMAs
+        // of its second k-step go the other loads, into its stages, and the reads of step t + 1.
         hb_wait_vmcnt<LATER>();
         hb_workgroup_barrier();
-        const int xstep = clamp(t + XST), wstep = clamp(t + WST);
 #pragma unroll
         for (int j = 0; j < NM; ++j) {
             mfma_one(1, j);
-            // (a clamped step goes where step t + XST or t + WST would: into the stage just freed)
-            between(j, NLX + NLW, [&](int i) { load_one(xstep, t % XST, wstep, t % WST, i); },
-                    [&](int i) { read_one(0, t + 1, 0, i); });
+            // (a clamped step goes where step t + X_AHEAD or t + W_AHEAD would: into the stage just freed)
+            between(j, LATE, [&](int i) {
+                if constexpr (X_EARLY) load_w(wstep, ws, i);
+                else if constexpr (W_EARLY) load_x(xstep, xs, i);
+                else if (X_FIRST ? i < NLX : i >= NLW) load_x(xstep, xs, X_FIRST ? i : i - NLW);
+                else load_w(wstep, ws, X_FIRST ? i - NLX : i);
+            }, [&](int i) { read_one(0, ws1, xs1, 0, i); });
             __builtin_amdgcn_sched_barrier(0);
         }
+        hold();
     }
-    {
-        const int t = nsteps - 1;
+    if constexpr (PEELED) {
+        const int t = nsteps - 1, ws = t % WST, xs = t % XST;
 #pragma unroll
         for (int j = 0; j < NM; ++j) {
             mfma_one(0, j);
-            between(j, 0, [&](int) {}, [&](int i) { read_one(1, t, 1, i); });
+            between(j, 0, [&](int) {}, [&](int i) { read_one(1, ws, xs, 1, i); });
             __builtin_amdgcn_sched_barrier(0);
         }
+        hold();
 #pragma unroll
         for (int j = 0; j < NM; ++j) mfma_one(1, j);
+        hold();
     }
     hb_wait_vmcnt<0>();      // the loads past the end (repeats of the last step) have landed too
-    if (scale.partial) {
+    if (SCALES && scale.partial) {
 #pragma unroll
-        for (int a = 0; a < TN32; ++a)
+        for (int a = 0; a < TN; ++a)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) acc[a][0][i] *= inv_rms;
+            for (int j = 0; j < 4; ++j) acc[a][0][j] *= inv_rms;
     }
+    const int m_base = m0 + wm * TM * 16, n_base = n0 + wn * TN * 16;
     if constexpr (EPI == EPI_QKV)
-        store_wave_tile_qkv<TN32, TM32>(acc, qkv, M, N, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
+        store_wave_tile_qkv<TN, TM>(acc, qkv, M, N, m_base, n_base, r16, g4);
     else {
-        // float32 outputs of the large tiles go through LDS (see store_wave_tile_lds): each wave has a
-        // quarter of what the rings held, once every wave's loads have landed and its reads are done
-        constexpr int REGION = (WST * W_STAGE + XST * X_STAGE) * (int)sizeof(bf16) / NW;       // bytes
-        constexpr int PB_FIT = REGION / (32 * TN32 * 128);
-        constexpr int PB = PB_FIT >= TM32 ? TM32 : (PB_FIT >= 2 && TM32 % 2 == 0 ? 2 : 1);
-        constexpr bool VIA_LDS = (EPI == EPI_STORE || EPI == EPI_ADD) && BM >= 128 && PB_FIT >= 1;
         const bool sliced = gridDim.y > 1;
         float* const dst = sliced ? partial + (size_t)blockIdx.y * M * N : (float*)Cv;
         const int ld = sliced ? N : ldc;
-        constexpr bool SWIGLU_VIA_LDS = (EPI == EPI_SWIGLU || EPI == EPI_GEGLU) && BM >= 128 && REGION >= 32 * TM32 * TN32 * 32;
-        if (SWIGLU_VIA_LDS && !sliced && (ldc & 7) == 0 && ((size_t)Cv & 15) == 0) {
-            hb_workgroup_barrier();
-            bf16* const stage = (bf16*)((char*)lds + wave * REGION);
-            if constexpr (EPI == EPI_GEGLU)
-                store_wave_tile_swiglu_lds<TN32, TM32, GLU_GELU_TANH>(acc, (bf16*)Cv, M, N, ldc, m0 + wm * TMB * 16,
-                                                                      n0 + wn * TNB * 16, lane, stage);
-            else if (scale.glu == GLU_RELU)
-                store_wave_tile_swiglu_lds<TN32, TM32, GLU_RELU>(acc, (bf16*)Cv, M, N, ldc, m0 + wm * TMB * 16,
-                                                                 n0 + wn * TNB * 16, lane, stage);
-            else
-                store_wave_tile_swiglu_lds<TN32, TM32, GLU_SILU>(acc, (bf16*)Cv, M, N, ldc, m0 + wm * TMB * 16,
-                                                                 n0 + wn * TNB * 16, lane, stage);
-        } else if (VIA_LDS && (ld & 3) == 0 && (N & 3) == 0 && ((size_t)dst & 15) == 0) {
+        constexpr bool GATED = EPI == EPI_SWIGLU || EPI == EPI_GEGLU, BF16_OUT = GATED || EPI == EPI_ACT;
+        if constexpr (BM >= 128) {
+            // outputs of the large tiles go through LDS (see store_wave_tile_lds): each wave has its share
+            // of what the rings held, once every wave's loads have landed and its reads are done
+            constexpr int REGION = (WST * W_STAGE + XST * X_STAGE) * (int)sizeof(bf16) / NW;       // bytes
+            constexpr int PB_FIT = REGION / (16 * TN * 64);
+            constexpr int PB = PB_FIT >= TM ? TM : (PB_FIT >= 4 && TM % 4 == 0 ? 4 : (PB_FIT >= 3 && TM % 3 == 0 ? 3 : (PB_FIT >= 2 && TM % 2 == 0 ? 2 : 1)));
+            static_assert(PB_FIT >= 1 && (!BF16_OUT || REGION >= 16 * TM * TN * (GATED ? 16 : 32)), "a wave's outputs must fit its share of LDS");
             hb_workgroup_barrier();
             float* const stage = (float*)((char*)lds + wave * REGION);
-            if (sliced || EPI == EPI_STORE)
-                store_wave_tile_lds<EPI_STORE, TN32, TM32, PB>(acc, dst, M, N, ld, m0 + wm * TMB * 16,
-                                                               n0 + wn * TNB * 16, lane, stage);
-            else
-                store_wave_tile_lds<EPI_ADD, TN32, TM32, PB>(acc, dst, M, N, ld, m0 + wm * TMB * 16,
-                                                             n0 + wn * TNB * 16, lane, stage);
-        } else if (EPI == EPI_ACT && sliced && BM >= 128 && PB_FIT >= 1 && (N & 3) == 0 && ((size_t)dst & 15) == 0) {
-            hb_workgroup_barrier();
-            store_wave_tile_lds<EPI_STORE, TN32, TM32, PB>(acc, dst, M, N, N, m0 + wm * TMB * 16, n0 + wn * TNB * 16, lane,
-                                                           (float*)((char*)lds + wave * REGION));
-        } else if (EPI == EPI_ACT && !sliced && BM >= 128 && REGION >= 32 * TM32 * TN32 * 64 && (TN32 & (TN32 - 1)) == 0 &&
-                   (ldc & 7) == 0 && ((size_t)Cv & 15) == 0) {
-            hb_workgroup_barrier();
-            bf16* const stage = (bf16*)((char*)lds + wave * REGION);
-            if (scale.glu == UNARY_GELU)
-                store_wave_tile_act_lds<TN32, TM32, UNARY_GELU>(acc, (bf16*)Cv, M, N, ldc, m0 + wm * TMB * 16,
-                                                                n0 + wn * TNB * 16, lane, stage);
-            else
-                store_wave_tile_act_lds<TN32, TM32, UNARY_RELU_SQUARED>(acc, (bf16*)Cv, M, N, ldc, m0 + wm * TMB * 16,
-                                                                        n0 + wn * TNB * 16, lane, stage);
-        } else if (EPI == EPI_ACT && !sliced && scale.glu == UNARY_GELU) {
-            store_wave_tile<EPI, TN32, TM32, UNARY_GELU>(acc, Cv, M, N, ldc, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
+            if constexpr (BF16_OUT)
+                if (!sliced) {
+                    const bool whole = (ldc & 7) == 0 && ((size_t)Cv & 15) == 0;
+                    store_wave_tile_bf16_lds<EPI, TN, TM>(acc, (bf16*)Cv, M, N, ldc, m_base, n_base, lane, (bf16*)stage, whole, scale.glu == 1);
+                    return;
+                }
+            if constexpr ((TN & (TN - 1)) == 0) {           // (tiles of another width are launched for gated units alone, whole)
+                const bool whole = (ld & 3) == 0 && (N & 3) == 0 && ((size_t)dst & 15) == 0;
+                if (EPI == EPI_ADD && !sliced)
+                    store_wave_tile_lds<EPI_ADD, TN, TM, PB>(acc, dst, M, N, ld, m_base, n_base, lane, stage, whole);
+                else
+                    store_wave_tile_lds<EPI_STORE, TN, TM, PB>(acc, dst, M, N, ld, m_base, n_base, lane, stage, whole);
+            }
         } else if (sliced) {
-            store_wave_tile<EPI_STORE, TN32, TM32>(acc, dst, M, N, N, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
-        } else if (EPI == EPI_SWIGLU && scale.glu == GLU_RELU) {
-            store_wave_tile<EPI, TN32, TM32, GLU_RELU>(acc, Cv, M, N, ldc, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
+            store_wave_tile<EPI_STORE, TN, TM>(acc, dst, M, N, N, m_base, n_base, r16, g4);
         } else if constexpr (EPI == EPI_GEGLU) {
-            store_wave_tile<EPI_SWIGLU, TN32, TM32, GLU_GELU_TANH>(acc, Cv, M, N, ldc, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
+            store_wave_tile<EPI_SWIGLU, TN, TM, GLU_GELU_TANH>(acc, Cv, M, N, ldc, m_base, n_base, r16, g4);
+        } else if (BF16_OUT && scale.glu == 1) {
+            store_wave_tile<EPI, TN, TM, 1>(acc, Cv, M, N, ldc, m_base, n_base, r16, g4);
         } else {
-            store_wave_tile<EPI, TN32, TM32>(acc, Cv, M, N, ldc, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
+            store_wave_tile<EPI, TN, TM>(acc, Cv, M, N, ldc, m_base, n_base, r16, g4);
         }
     }
 }
@@ -1301,17 +1269,15 @@ gemm_tile_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, void* _
 // K in steps of 32 only: one k-step a stage, everything in 1 KB blocks (the activations too: a
 // block of 16 rows x 32 k is loaded as 16 half lines), a ring of STAGES stages loaded STAGES - 1
 // steps ahead, the plain order read / multiply with the operands in two sets of registers.
-template <int EPI, bool PACKED, int TNB, int TMB, int WNW, int WMW, int STAGES>
+template <int EPI, bool PACKED, int TN, int TM, int WNW, int WMW, int STAGES>
 __global__ void __launch_bounds__(64 * WNW * WMW)
 gemm_tile32_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, void* __restrict__ Cv, int M, int N,
                    int K, int ldc, int m_tiles, int n_tiles, int glu) {
     constexpr int NW = WNW * WMW;
-    constexpr int BN = 16 * TNB * WNW, BM = 16 * TMB * WMW;
+    constexpr int BN = 16 * TN * WNW, BM = 16 * TM * WMW;
     constexpr int WBLK = BN / 16, XBLK = BM / 16, BLKS = WBLK + XBLK;   // 1 KB blocks of a stage
     constexpr int WL = WBLK / NW, XL = XBLK / NW;                      // loads of a wave per stage
     static_assert(WBLK % NW == 0 && XBLK % NW == 0, "blocks must divide over the waves");
-    static_assert(TNB % 2 == 0 && TMB % 2 == 0, "a wave's tile is made of 32 x 32 pieces");
-    constexpr int TN32 = TNB / 2, TM32 = TMB / 2;
     extern __shared__ __attribute__((aligned(1024))) bf16 lds[];        // [STAGES][BLKS][512]
 
     int m_tile, n_tile;
@@ -1319,7 +1285,7 @@ gemm_tile32_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, void*
     const int m0 = m_tile * BM, n0 = n_tile * BN;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r16 = lane & 15, g4 = lane >> 4, c32 = lane & 31, g2 = lane >> 5;
+    const int r16 = lane & 15, g4 = lane >> 4;
     const int wn = wave / WMW, wm = wave % WMW;
     const int nsteps = K / 32;
 
@@ -1355,37 +1321,26 @@ gemm_tile32_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, void*
             hb_load_to_lds(xsrc[i] + (size_t)step * 32, base + (WBLK + wave * XL + i) * 512);
     };
 
-    f32x16 acc[TN32][TM32];
+    f32x4 acc[TN][TM];
 #pragma unroll
-    for (int a = 0; a < TN32; ++a)
+    for (int a = 0; a < TN; ++a)
 #pragma unroll
-        for (int b = 0; b < TM32; ++b)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.f;
+        for (int b = 0; b < TM; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    const int lane_off = (c32 >> 4) * 512 + (16 * g2 + (lane & 15)) * 8;   // + 32 * 8 for the second k-half
-    bf16x8 wv[2][2][TN32], xv[2][2][TM32];       // [set][k-half][piece]
+    bf16x8 wv[2][TN], xv[2][TM];                 // [set][block]
     auto read_operands = [&](int set, int stage) {
-        const bf16* base = lds + (size_t)stage * BLKS * 512 + lane_off;
+        const bf16* base = lds + (size_t)stage * BLKS * 512 + lane * 8;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        for (int a = 0; a < TN; ++a) wv[set][a] = *(const bf16x8*)(base + (wn * TN + a) * 512);
 #pragma unroll
-            for (int a = 0; a < TN32; ++a)
-                wv[set][h][a] = *(const bf16x8*)(base + (wn * TNB + 2 * a) * 512 + h * 256);
-#pragma unroll
-            for (int b = 0; b < TM32; ++b)
-                xv[set][h][b] = *(const bf16x8*)(base + (WBLK + wm * TMB + 2 * b) * 512 + h * 256);
-        }
+        for (int b = 0; b < TM; ++b) xv[set][b] = *(const bf16x8*)(base + (WBLK + wm * TM + b) * 512);
     };
     auto multiply = [&](int set) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+        for (int a = 0; a < TN; ++a)
 #pragma unroll
-            for (int a = 0; a < TN32; ++a)
-#pragma unroll
-                for (int b = 0; b < TM32; ++b)
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv[set][h][a], xv[set][h][b], acc[a][b],
-                                                                        0, 0, 0);
+            for (int b = 0; b < TM; ++b)
+                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[set][a], xv[set][b], acc[a][b], 0, 0, 0);
     };
     // Before step t + 1 is read: this wave's loads of it have landed (those of the STAGES - 2 later
     // steps may be in flight) and its reads of step t are in registers; after the barrier that
@@ -1413,12 +1368,13 @@ gemm_tile32_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, void*
     }
     hb_wait_vmcnt<0>();      // the loads past the end (repeats of the last step) have landed too
     static_assert((int)GLU_RELU == (int)UNARY_GELU, "the second of either kind");
+    const int m_base = m0 + wm * TM * 16, n_base = n0 + wn * TN * 16;
     if ((EPI == EPI_SWIGLU || EPI == EPI_ACT) && glu == GLU_RELU)
-        store_wave_tile<EPI, TN32, TM32, GLU_RELU>(acc, Cv, M, N, ldc, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
+        store_wave_tile<EPI, TN, TM, GLU_RELU>(acc, Cv, M, N, ldc, m_base, n_base, r16, g4);
     else if constexpr (EPI == EPI_GEGLU)
-        store_wave_tile<EPI_SWIGLU, TN32, TM32, GLU_GELU_TANH>(acc, Cv, M, N, ldc, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
+        store_wave_tile<EPI_SWIGLU, TN, TM, GLU_GELU_TANH>(acc, Cv, M, N, ldc, m_base, n_base, r16, g4);
     else
-        store_wave_tile<EPI, TN32, TM32>(acc, Cv, M, N, ldc, m0 + wm * TMB * 16, n0 + wn * TNB * 16, c32, g2);
+        store_wave_tile<EPI, TN, TM>(acc, Cv, M, N, ldc, m_base, n_base, r16, g4);
 }
 
 // More than 64 KB of dynamic LDS has to be allowed per kernel, once.
@@ -1463,14 +1419,14 @@ static int launch_tiles(Kernel kern, size_t lds, int threads, long total, int sl
     } while (0)
 
 // slices > 1: the sums of the slices go to `partial`; the caller adds them up afterwards
-template <int TNB, int TMB, int WNW, int WMW, int WST, int XST>
+template <int TN, int TM, int WNW, int WMW, int WST, int XST>
 static int launch_tile64(const void* X, const void* W, void* C, int M, int N, int K, int ldc, int epi, int packed,
                          hipStream_t stream, int slices = 1, float* partial = nullptr, RowScale scale = RowScale{}) {
-    constexpr int BN = 16 * TNB * WNW, BM = 16 * TMB * WMW;
+    constexpr int BN = 16 * TN * WNW, BM = 16 * TM * WMW;
     HB_REQUIRE(K % 64 == 0, "gemm_mfma: K=%d is no multiple of 64", K);
     const int m_tiles = (M + BM - 1) / BM, n_tiles = (N + BN - 1) / BN;
     const long total = (long)m_tiles * n_tiles;
-    const size_t lds = (size_t)(WST * BN + XST * BM) * 64 * sizeof(bf16) + WNW * WMW * 16 * sizeof(float);
+    const size_t lds = (size_t)(WST * BN + XST * BM) * 64 * sizeof(bf16) + (BM <= 32 ? WNW * WMW * 16 * sizeof(float) : 0);
     const int threads = 64 * WNW * WMW;
     const bf16* x = (const bf16*)X;
     const bf16* w = (const bf16*)W;
@@ -1480,26 +1436,26 @@ static int launch_tile64(const void* X, const void* W, void* C, int M, int N, in
     HB_REQUIRE((K / 64 + slices - 1) / slices * (slices - 1) < K / 64, "gemm_mfma: a slice of K would be empty");
     const int glu = scale.glu;
 #define EXTRA , partial, QkvEpilogue{}, scale
-    TILE_DISPATCH(gemm_tile_kernel, TNB, TMB, WNW, WMW, WST, XST);
+    TILE_DISPATCH(gemm_tile_kernel, TN, TM, WNW, WMW, WST, XST);
 #undef EXTRA
 }
 
 // Tiles whose width is no power of two (192 = three pieces of 32 a wave): for the SwiGLU epilogue
 // only, whose bfloat16 output goes to memory lane by lane (the float32 epilogues' way through LDS
 // counts on rows of a power of two of 16-byte chunks).
-template <int TNB, int TMB, int WNW, int WMW, int WST, int XST>
+template <int TN, int TM, int WNW, int WMW, int WST, int XST>
 static int launch_tile64_swiglu(const void* X, const void* W, void* C, int M, int N, int K, int ldc, int epi,
                                 int packed, hipStream_t stream, int slices, RowScale scale) {
-    constexpr int BN = 16 * TNB * WNW, BM = 16 * TMB * WMW;
+    constexpr int BN = 16 * TN * WNW, BM = 16 * TM * WMW;
     HB_REQUIRE(epi == EPI_SWIGLU && slices == 1, "gemm_mfma: this tile takes the SwiGLU product whole only");
     HB_REQUIRE(K % 64 == 0, "gemm_mfma: K=%d is no multiple of 64", K);
     const int m_tiles = (M + BM - 1) / BM, n_tiles = (N + BN - 1) / BN;
     const long total = (long)m_tiles * n_tiles;
-    const size_t lds = (size_t)(WST * BN + XST * BM) * 64 * sizeof(bf16) + WNW * WMW * 16 * sizeof(float);
+    const size_t lds = (size_t)(WST * BN + XST * BM) * 64 * sizeof(bf16) + (BM <= 32 ? WNW * WMW * 16 * sizeof(float) : 0);
     const bf16* x = (const bf16*)X;
     const bf16* w = (const bf16*)W;
 #define SWIGLU_GO(EPIV, PK)                                                                                                    \
-    return launch_tiles(gemm_tile_kernel<EPIV, PK, TNB, TMB, WNW, WMW, WST, XST>, lds, 64 * WNW * WMW, total, 1, x, w, C, M, N, K, \
+    return launch_tiles(gemm_tile_kernel<EPIV, PK, TN, TM, WNW, WMW, WST, XST>, lds, 64 * WNW * WMW, total, 1, x, w, C, M, N, K, \
                         ldc, m_tiles, n_tiles, stream, (float*)nullptr, QkvEpilogue{}, scale)
     if (scale.glu == GLU_GELU_TANH) {
         if (packed) SWIGLU_GO(EPI_GEGLU, true);
@@ -1510,10 +1466,10 @@ static int launch_tile64_swiglu(const void* X, const void* W, void* C, int M, in
 #undef SWIGLU_GO
 }
 
-template <int TNB, int TMB, int WNW, int WMW, int STAGES>
+template <int TN, int TM, int WNW, int WMW, int STAGES>
 static int launch_tile32(const void* X, const void* W, void* C, int M, int N, int K, int ldc, int epi, int packed,
                          hipStream_t stream, int glu) {
-    constexpr int BN = 16 * TNB * WNW, BM = 16 * TMB * WMW;
+    constexpr int BN = 16 * TN * WNW, BM = 16 * TM * WMW;
     const int m_tiles = (M + BM - 1) / BM, n_tiles = (N + BN - 1) / BN;
     const long total = (long)m_tiles * n_tiles;
     const size_t lds = (size_t)STAGES * (BN + BM) * 32 * sizeof(bf16);
@@ -1522,7 +1478,7 @@ static int launch_tile32(const void* X, const void* W, void* C, int M, int N, in
     const bf16* w = (const bf16*)W;
     const int slices = 1;
 #define EXTRA , glu
-    TILE_DISPATCH(gemm_tile32_kernel, TNB, TMB, WNW, WMW, STAGES);
+    TILE_DISPATCH(gemm_tile32_kernel, TN, TM, WNW, WMW, STAGES);
 #undef EXTRA
 }
 #undef TILE_DISPATCH
@@ -1532,17 +1488,17 @@ static int launch_tile32(const void* X, const void* W, void* C, int M, int N, in
 // one head wide; shape: 0 = tiles of 256 x 256 (waves 2 x 2, for long prompts), 1 = a head wide and 256
 // rows high (four waves one above the other, 64 rows each), 2 = a head wide and 128 rows high (32
 // rows a wave): more and smaller tiles for prompts whose 256 x 256 tiles would not fill the CUs.
-template <int TNB, int TMB, int WNW, int WMW, int WST, int XST>
+template <int TN, int TM, int WNW, int WMW, int WST, int XST>
 static int launch_qkv(const bf16* x, const bf16* w, int M, int N, int K, int packed, const QkvEpilogue& e,
                       hipStream_t stream) {
-    constexpr int BN = 16 * TNB * WNW, BM = 16 * TMB * WMW;
+    constexpr int BN = 16 * TN * WNW, BM = 16 * TM * WMW;
     const int m_tiles = (M + BM - 1) / BM, n_tiles = (N + BN - 1) / BN;
     const long total = (long)m_tiles * n_tiles;
-    const size_t lds = (size_t)(WST * BN + XST * BM) * 64 * sizeof(bf16) + WNW * WMW * 16 * sizeof(float);
+    const size_t lds = (size_t)(WST * BN + XST * BM) * 64 * sizeof(bf16) + (BM <= 32 ? WNW * WMW * 16 * sizeof(float) : 0);
     if (packed)
-        return launch_tiles(gemm_tile_kernel<EPI_QKV, true, TNB, TMB, WNW, WMW, WST, XST>, lds, 64 * WNW * WMW, total, 1, x,
+        return launch_tiles(gemm_tile_kernel<EPI_QKV, true, TN, TM, WNW, WMW, WST, XST>, lds, 64 * WNW * WMW, total, 1, x,
                             w, nullptr, M, N, K, N, m_tiles, n_tiles, stream, (float*)nullptr, e, RowScale{});
-    return launch_tiles(gemm_tile_kernel<EPI_QKV, false, TNB, TMB, WNW, WMW, WST, XST>, lds, 64 * WNW * WMW, total, 1, x, w,
+    return launch_tiles(gemm_tile_kernel<EPI_QKV, false, TN, TM, WNW, WMW, WST, XST>, lds, 64 * WNW * WMW, total, 1, x, w,
                         nullptr, M, N, K, N, m_tiles, n_tiles, stream, (float*)nullptr, e, RowScale{});
 }
 
@@ -1560,7 +1516,7 @@ extern "C" int hb_gemm_qkv_mfma(const void* X, const void* W, int M, int K, int 
                            max_pages, q_norm_w, k_norm_w, cos_t, sin_t, eps, nq, nkv};
     const bf16* x = (const bf16*)X;
     const bf16* w = (const bf16*)W;
-    if (shape == 0) return launch_qkv<8, 8, 2, 2, 2, 2>(x, w, M, N, K, packed, e, stream);
+    if (shape == 0) return launch_qkv<8, 8, 2, 2, 3, 2>(x, w, M, N, K, packed, e, stream);
     if (shape == 1) return launch_qkv<8, 4, 1, 4, 3, 2>(x, w, M, N, K, packed, e, stream);
     return launch_qkv<8, 2, 1, 4, 3, 2>(x, w, M, N, K, packed, e, stream);
 }
@@ -1822,16 +1778,16 @@ extern "C" int hb_gemm_mfma(const void* X, const void* W, void* C, int M, int N,
     HB_REQUIRE(!scale_partial || tile == 112, "gemm_mfma: only the few-row kernels take a handed-on norm");
     int rc;
     switch (tile) {
-        // (ring depths, measured with weights that come from HBM: a third weight stage gains a
-        // tenth for 256 x 128 and nothing for the other two; a third activation stage nothing)
-        case 188: rc = launch_tile64<8, 8, 2, 2, 2, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 256 x 256
-        case 142: rc = launch_tile64<8, 4, 2, 2, 3, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 256 (n) x 128 (m)
-        case 186: rc = launch_tile64<8, 6, 2, 2, 2, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 256 (n) x 192 (m)
+        // (ring depths: as much as LDS holds; the weights, which come from HBM, have the third stage where there is
+        // room for one: 8192 x 8192 x 8192 on 256 x 256 tiles 792 us, with the activations' third stage instead 838)
+        case 188: rc = launch_tile64<8, 8, 2, 2, 3, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 256 x 256
+        case 142: rc = launch_tile64<8, 4, 2, 2, 3, 3>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 256 (n) x 128 (m)
+        case 186: rc = launch_tile64<8, 6, 2, 2, 3, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 256 (n) x 192 (m)
         case 122: rc = launch_tile64<4, 4, 2, 2, 2, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 128 x 128, two to a CU
         case 124: rc = launch_tile64<2, 4, 4, 1, 3, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 128 (n) x 64 (m)
         case 112: rc = launch_tile64<2, 2, 4, 1, 3, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 128 (n) x 32 (m)
         case 184: rc = launch_tile64<4, 4, 4, 1, 3, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 256 (n) x 64 (m)
-        case 168: rc = launch_tile64_swiglu<6, 8, 2, 2, 2, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, row_scale); break;   // 192 (n) x 256 (m)
+        case 168: rc = launch_tile64_swiglu<6, 8, 2, 2, 3, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, row_scale); break;   // 192 (n) x 256 (m)
         case 164: rc = launch_tile64_swiglu<6, 2, 1, 2, 3, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, row_scale); break;   // 96 (n) x 64 (m), two waves one above the other
         case 123:                                                                                                           // 128 x 128, K in steps of 32
             HB_REQUIRE(slices == 1, "gemm_mfma: this tile does not cut K");

@@ -347,6 +347,42 @@ def test_gemm_mfma_large_tiles_with_ragged_edges(M, N, K, tile):
         assert float((c2 - (base + want)).abs().max()) <= tol
 
 
+@pytest.mark.parametrize("tile", [188, 142, 186, 122])
+@pytest.mark.parametrize("M,N,K,packed", [(300, 330, 128, False), (257, 272, 64, True), (129, 1027, 320, False)])
+def test_gemm_mfma_tall_tiles_off_16_byte_borders(M, N, K, packed, tile):
+    """Tall tiles whose outputs cannot leave LDS 16 bytes at a time: widths that are no multiple of 8 and outputs that
+    begin off a 16-byte border, for the store, the add, the activations and the gated unit; nothing around them is written."""
+    from herbert_rs_amd.kernels import mfma
+    a = rand(M, K, seed=23, dtype=torch.bfloat16)
+    w = rand(N, K, seed=24, dtype=torch.bfloat16, scale=0.1)
+    wt = mfma.pack_weight(w) if packed else w
+    want = (a.double() @ w.double().T).float()
+
+    def view(width, dtype):
+        whole = torch.full((M * width + 2,), 3.0, dtype=dtype, device=dev())
+        return whole, whole[1:-1].view(M, width)
+
+    tol = 2e-6 * K ** 0.5 * float(want.abs().max()) + 1e-4          # float32 sums of K products in another order
+    whole, c = view(N, torch.float32)
+    mfma.gemm(a, wt, c, packed=packed, tile=tile)
+    assert float((c - want).abs().max()) <= tol
+    mfma.gemm(a, wt, c, accumulate=True, packed=packed, tile=tile)
+    assert float((c - 2 * want).abs().max()) <= 2 * tol and whole[0] == 3.0 and whole[-1] == 3.0
+    whole, c = view(N, torch.bfloat16)
+    for name, exact in (("relu_squared", torch.relu(want) ** 2), ("gelu", torch.nn.functional.gelu(want))):
+        mfma.gemm_activated(a, wt, c, name, packed=packed, tile=tile)
+        bound = 2 ** -8 * exact.abs() + 2 * tol * (1 + want.abs())   # one rounding to bfloat16 behind the float32 sums
+        assert bool(((c.float() - exact).abs() <= bound).all()) and whole[0] == 3.0 and whole[-1] == 3.0
+    if N % 32 == 0:
+        whole, c = view(N // 2, torch.bfloat16)
+        wi = mfma.interleave_gate_up(w[:N // 2].contiguous(), w[N // 2:].contiguous())
+        g, u = want[:, :N // 2], want[:, N // 2:]
+        for name, unit in (("silu", torch.nn.functional.silu(g)), ("relu", torch.relu(g))):
+            mfma.gemm_swiglu(a, mfma.pack_weight(wi) if packed else wi, c, packed, tile=tile, activation=name)
+            bound = 2 ** -8 * (unit * u).abs() + 2 * tol * (1 + u.abs() + g.abs())
+            assert bool(((c.float() - unit * u).abs() <= bound).all()) and whole[0] == 3.0 and whole[-1] == 3.0
+
+
 @pytest.mark.parametrize("M,I,K", [(1, 16, 32), (8, 12288, 4096), (40, 48, 96), (64, 1024, 64),
                                    (100, 176, 128), (300, 256, 64)])
 def test_gemm_mfma_swiglu(M, I, K):
