@@ -1483,11 +1483,41 @@ static int launch_tile32(const void* X, const void* W, void* C, int M, int N, in
 }
 #undef TILE_DISPATCH
 
+// The tiles of products of more than 64 rows: number, columns, rows, workgroups on a CU, a step's time and what a round of
+// tiles costs beside its steps (us).
+// (168: three quarters of the 256 x 256 tile's arithmetic a step, for the SwiGLU product whole: where that
+// one's tiles fill the last round of 256 badly, 192 columns often fill it)
+// (186: 224, 192 or 160 rows high, whichever is done sooner, for row counts whose tiles of 256 rows leave CUs empty and whose
+// tiles of 128 rows need another round; the heights beside 192: 9,404 rows x 2,048 columns (K 6144, add) 212 us on
+// 192, 197 on 160; 2,600 x 24576 x 4096 (gated) 441 on tile 168, 398 on 224)
+// (cut_us: a step's time as split_rows has it, 0 for tiles that it leaves out)
+struct Mid { int id, bn, bm, per_cu; double step_us, round_us, cut_us; };
+static const Mid mid_tiles[] = {{188, 256, 256, 1, 1.21, 4.8, 1.26}, {186, 256, 224, 1, 1.09, 7.7, 0}, {186, 256, 192, 1, 1.01, 5.3, 1.08},
+                                {186, 256, 160, 1, 0.91, 5.9, 0}, {142, 256, 128, 1, 0.77, 4.8, 0.77}, {122, 128, 128, 2, 0.73, 3.1, 0.95},
+                                {124, 128, 64, 2, 0.40, 4.4, 0.48}, {184, 256, 64, 1, 0.72, 3.1, 0.67}, {168, 192, 256, 1, 0.93, 5.3, 1.0}};
+// the rounds of a product's tiles, one after the other
+static double mid_stepping(const Mid& v, int M, int N, int K, int slices, bool cutting = false) {
+    const long wgs = (long)((M + v.bm - 1) / v.bm) * ((N + v.bn - 1) / v.bn) * slices, slots = 256 * v.per_cu;
+    const long rounds = (wgs + slots - 1) / slots, on_a_cu = ((wgs < slots ? wgs : slots) + 255) / 256;
+    const int per = (K / 64 + slices - 1) / slices;
+    if (cutting) return (double)rounds * per * v.cut_us * (1 + 1.06 * (on_a_cu - 1));
+    return (double)rounds * (per * v.step_us * (1 + 0.54 * (on_a_cu - 1)) + v.round_us);
+}
+// The rows of the tiles of 256 columns, from 160 to `tallest`, with which a product's rounds are done soonest.
+static int tall_rows(int M, int N, int K, int slices, int tallest) {
+    const Mid* best = nullptr;
+    for (const Mid& v : mid_tiles)
+        if ((v.id == 186 || v.id == 188) && v.bm <= tallest &&
+            (!best || mid_stepping(v, M, N, K, slices) < mid_stepping(*best, M, N, K, slices)))
+            best = &v;
+    return best->bm;
+}
+
 // The q/k/v projection of a step with many rows, fused with norm, rotation and cache write
 // (see QkvEpilogue). X [M, K] bf16; W [(nq + 2 nkv) 128, K] bf16, rows q | k | v. A wave's tile is
-// one head wide; shape: 0 = tiles of 256 x 256 (waves 2 x 2, for long prompts), 1 = a head wide and 256
-// rows high (four waves one above the other, 64 rows each), 2 = a head wide and 128 rows high (32
-// rows a wave): more and smaller tiles for prompts whose 256 x 256 tiles would not fill the CUs.
+// one head wide; shape: 0 = tiles of 256 columns (waves 2 x 2, for long prompts), 160 to 256 rows high, whichever are done
+// soonest, 1 = a head wide and 256 rows high (four waves one above the other, 64 rows each), 2 = a head
+// wide and 128 rows high (32 rows a wave): more and smaller tiles for prompts whose 256 x 256 tiles would not fill the CUs.
 template <int TN, int TM, int WNW, int WMW, int WST, int XST>
 static int launch_qkv(const bf16* x, const bf16* w, int M, int N, int K, int packed, const QkvEpilogue& e,
                       hipStream_t stream) {
@@ -1516,7 +1546,13 @@ extern "C" int hb_gemm_qkv_mfma(const void* X, const void* W, int M, int K, int 
                            max_pages, q_norm_w, k_norm_w, cos_t, sin_t, eps, nq, nkv};
     const bf16* x = (const bf16*)X;
     const bf16* w = (const bf16*)W;
-    if (shape == 0) return launch_qkv<8, 8, 2, 2, 3, 2>(x, w, M, N, K, packed, e, stream);
+    if (shape == 0) {
+        const int rows = tall_rows(M, N, K, 1, 256);
+        if (rows == 256) return launch_qkv<8, 8, 2, 2, 3, 2>(x, w, M, N, K, packed, e, stream);
+        if (rows == 224) return launch_qkv<8, 7, 2, 2, 3, 2>(x, w, M, N, K, packed, e, stream);
+        if (rows == 192) return launch_qkv<8, 6, 2, 2, 3, 2>(x, w, M, N, K, packed, e, stream);
+        return launch_qkv<8, 5, 2, 2, 3, 3>(x, w, M, N, K, packed, e, stream);
+    }
     if (shape == 1) return launch_qkv<8, 4, 1, 4, 3, 2>(x, w, M, N, K, packed, e, stream);
     return launch_qkv<8, 2, 1, 4, 3, 2>(x, w, M, N, K, packed, e, stream);
 }
@@ -1539,7 +1575,7 @@ static double few_rows_cost(int M, int N, int K, int epi) {
 
 struct GemmPlan { int tile, slices; double cost = -1; };      // cost: the estimated time in us where the plan was chosen by one
 static GemmPlan plan_gemm(int M, int N, int K, int ldc, int epi, bool norm_w, bool emit_g, bool scale_partial,
-                          int tile_hint, size_t workspace_floats, bool deferred = false) {
+                          int tile_hint, size_t workspace_floats, bool deferred = false, bool cutting = false) {
     int tile = tile_hint % 1000, slices = tile_hint >= 1000 ? tile_hint / 1000 : 1;
     double low_cost = -1, mid_cost = -1;
     if (tile_hint == 1) return M <= 16 ? GemmPlan{0, 1} : GemmPlan{-1, 0};      // the few-row kernel, asked for by name
@@ -1613,41 +1649,28 @@ static GemmPlan plan_gemm(int M, int N, int K, int ldc, int epi, bool norm_w, bo
     if (tile == 0 && K % 64 == 0) {
         // More than 64 rows: neither the arithmetic nor the weights alone decide. All tiles from 128 x 64
         // to 256 x 256 with 1 to 16 K slices are candidates; a candidate takes as long as the slowest
-        // of: its workgroups' steps one after another (a step's time alone on a CU, about twice that
-        // with two on a CU), what all workgroups move out of the L2s (16 TB/s), what comes from
-        // HBM once (7 TB/s); plus a start and, for slices, the second kernel. Fitted to the four
-        // products of a layer for three model sizes and 96 to 1024 rows (the choice is then 1 % from
-        // the best candidate on average, 12 % at worst), checked on three other sizes (2 %, 13 %) and
-        // on 1280 to 4096 rows (under 1 %, 7 %).
-        struct Mid { int id, bn, bm, per_cu; double step_us; };
-        // (168: three quarters of the 256 x 256 tile's arithmetic a step, for the SwiGLU product whole:
-        // where that one's tiles fill the last round of 256 badly, 192 columns often fill it)
-        // (186: 192 rows high, for row counts whose tiles of 256 rows leave CUs empty and whose tiles of
-        // 128 rows need a second round: 2,400 to 3,072 rows of 4096 columns, 6 to 14 % off)
-        static const Mid mid[] = {{188, 256, 256, 1, 1.26}, {142, 256, 128, 1, 0.77}, {122, 128, 128, 2, 0.95},
-                                  {124, 128, 64, 2, 0.48}, {184, 256, 64, 1, 0.67}, {168, 192, 256, 1, 1.0},
-                                  {186, 256, 192, 1, 1.08}};
+        // of: its rounds' steps one after another (a step's time alone on a CU, half as much again with two
+        // on a CU) and what a round costs beside them, what all workgroups move out of the L2s (16 TB/s),
+        // what comes from HBM once (6.5 TB/s); plus, for slices, the second kernel. Fitted to every tile's time
+        // at eleven products of four model sizes and 96 to 9,404 rows: the choice is then 0.8 % from the
+        // best candidate on average (2.0 % without a round's own cost and the two heights between), 25 % at worst.
         const int steps = K / 64;
         double best = -1;
-        for (const Mid& v : mid) {
-            if (v.id == 168 && epi != EPI_SWIGLU) continue;
+        for (const Mid& v : mid_tiles) {
+            if ((v.id == 168 && epi != EPI_SWIGLU) || (cutting && v.cut_us == 0)) continue;
             const long tiles = (long)((M + v.bm - 1) / v.bm) * ((N + v.bn - 1) / v.bn);
             for (int sl = 1; sl <= 16; sl *= 2) {
                 if (v.id == 168 && sl > 1) break;
                 if (sl > 1 && !slices_fit(steps, sl)) break;
                 if (emit_g && (sl == 1 || !reducer_norms)) continue;      // the kernel that adds the slices up norms
                 if (deferred && sl > 8) break;                            // whoever adds the slices up takes 2, 4 or 8
-                const long wgs = tiles * sl, slots = 256 * v.per_cu;
-                const long rounds = (wgs + slots - 1) / slots;
-                const long on_a_cu = ((wgs < slots ? wgs : slots) + 255) / 256;
-                const int per = (steps + sl - 1) / sl;
-                const double stepping = (double)rounds * per * v.step_us * (1 + 1.06 * (on_a_cu - 1));
-                const double moving = (double)wgs * per * (v.bn + v.bm) * 128 / 16.3e6;
-                const double fetching = ((double)N + M) * K * 2 / 7.1e6;
+                const double stepping = mid_stepping(v, M, N, K, sl, cutting);
+                const double moving = (double)(tiles * sl) * ((steps + sl - 1) / sl) * (v.bn + v.bm) * 128 / 16.3e6;
+                const double fetching = ((double)N + M) * K * 2 / (cutting ? 7.1e6 : 6.5e6);
                 double cost = stepping > moving ? stepping : moving;
                 if (fetching > cost) cost = fetching;
-                cost += 2.3;
-                if (sl > 1) cost += deferred ? (double)sl * M * N * 4 / 2.3e6 : 1.5 + (double)(sl + 1) * M * N * 4 / 2.3e6;
+                if (cutting) cost += 2.3;
+                if (sl > 1) cost += deferred ? (double)sl * M * N * 4 / 2.5e6 : 1.3 + (double)(sl + 1) * M * N * 4 / 2.5e6;
                 if (best < 0 || cost < best) {
                     best = cost;
                     tile = v.id;
@@ -1663,22 +1686,24 @@ static GemmPlan plan_gemm(int M, int N, int K, int ldc, int epi, bool norm_w, bo
     return GemmPlan{tile, slices, mid_cost >= 0 ? mid_cost : low_cost};
 }
 
-// The rows of the first of two products that M rows are better cut into (see hb_gemm_mfma), or 0.
+// The rows of the first of two products that M rows are better cut into (see hb_gemm_mfma), or 0. Its estimates leave out the
+// heights of 224 and 160 rows and a round's own cost, with which its margin of a tenth was found; a cut that the
+// product's own estimates, which have them, put a tenth behind the whole product is not made.
 static int split_rows(int M, int N, int K, int ldc, int epi, bool special, int tile_hint, size_t workspace_floats,
                       const GemmPlan& whole) {
     if (special || M <= 128 || (tile_hint != 0 && tile_hint != -128 && tile_hint != -256)) return 0;
     int best_main = 0;
-    double best = whole.cost;
+    auto estimate = [&](int rows, bool cutting) { return plan_gemm(rows, N, K, ldc, epi, false, false, false, 0, workspace_floats, false, cutting); };
+    double best = whole.cost < 0 ? -1 : estimate(M, true).cost;
     for (int bm = 128; bm <= 256; bm *= 2) {
         const int main_rows = M / bm * bm, rest = M - main_rows;
         if (rest == 0 || main_rows == 0) continue;
-        const GemmPlan a = plan_gemm(main_rows, N, K, ldc, epi, false, false, false, 0, workspace_floats);
-        const GemmPlan b = plan_gemm(rest, N, K, ldc, epi, false, false, false, 0, workspace_floats);
+        const GemmPlan a = estimate(main_rows, true), b = estimate(rest, true);
         if (a.tile < 0 || b.tile < 0) continue;
         if (tile_hint == -bm) return main_rows;
         if (tile_hint != 0 || whole.cost < 0 || a.cost < 0 || b.cost < 0) continue;
         // (a second launch and its start are in the estimates; a tenth is kept as a margin for their error)
-        if (a.cost + b.cost < 0.9 * best) {
+        if (a.cost + b.cost < 0.9 * best && estimate(main_rows, false).cost + estimate(rest, false).cost < 1.1 * whole.cost) {
             best = (a.cost + b.cost) / 0.9;
             best_main = main_rows;
         }
@@ -1782,7 +1807,13 @@ extern "C" int hb_gemm_mfma(const void* X, const void* W, void* C, int M, int N,
         // room for one: 8192 x 8192 x 8192 on 256 x 256 tiles 792 us, with the activations' third stage instead 838)
         case 188: rc = launch_tile64<8, 8, 2, 2, 3, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 256 x 256
         case 142: rc = launch_tile64<8, 4, 2, 2, 3, 3>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 256 (n) x 128 (m)
-        case 186: rc = launch_tile64<8, 6, 2, 2, 3, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 256 (n) x 192 (m)
+        case 186: {                                                                                                          // 256 (n) x 160, 192 or 224 (m)
+            const int rows = tall_rows(M, N, K, slices, 224);
+            if (rows == 224) rc = launch_tile64<8, 7, 2, 2, 3, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale);
+            else if (rows == 192) rc = launch_tile64<8, 6, 2, 2, 3, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale);
+            else rc = launch_tile64<8, 5, 2, 2, 3, 3>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale);
+            break;
+        }
         case 122: rc = launch_tile64<4, 4, 2, 2, 2, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 128 x 128, two to a CU
         case 124: rc = launch_tile64<2, 4, 4, 1, 3, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 128 (n) x 64 (m)
         case 112: rc = launch_tile64<2, 2, 4, 1, 3, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 128 (n) x 32 (m)
