@@ -28,10 +28,12 @@
 // 0.999: the outputs' error is 0.67 to 0.97 of the walk's (0.8e-7 to 1e-6), 0.56 to 0.88 for the linear attention, and that of the
 // state left 0.76 to 1.06. (With A, B and T in float32 the outputs' was up to 1.3 of the walk's, the state's up to 2.)
 //
-// 2,048 tokens of 16 heads of 128 x 128 take 178 us (the walk 781), with a decay a channel 201 (1,084), the linear attention
-// 131 (909); 8 sequences of 300 tokens 184, 217 and 123 (446, 408 and 455). Bound: the second kernel by its chain (64
-// products of 32 cycles a chunk and wave and two exchanges through LDS, 99 us of the 178), the first by its products, in float64 of 64
-// cycles, for which a (chunk, head) has one workgroup a CU.
+// 2,048 tokens of 16 heads of 128 x 128 take 152 us (the walk 781), with a decay a channel 201 (1,084), the linear attention
+// 131 (909); 8 sequences of 300 tokens with a decay a channel 217 (408), the linear attention 123 (455). Bound: the second kernel by its
+// chain (64 products of 32 cycles a chunk and wave and two exchanges through LDS, 100 us of the 152), the first by its products in
+// float64 of 64 cycles and what lies between them. With one decay a head its pairs within a block are summed once instead of once a
+// level (256 of 448 products of its longest wave), and its pieces lie in LDS twice over, so that two workgroups fit a CU: 86 us -> 52. With a
+// decay a channel and keys of 128 a lane's decays take more than half of the registers: one workgroup a CU (two spill 270 of them).
 #include "common.h"
 #include "mfma_f32.h"
 #include <math.h>
@@ -89,7 +91,7 @@ __device__ __forceinline__ f64x4 mfma64_k4(double w, double a, f64x4 sums) {
 __device__ __forceinline__ bool not_finite(float v) { return !(fabsf(v) <= 3.4028235e38f); }
 
 template <int DB, bool CH, bool DELTA>
-__global__ void __launch_bounds__(256, DELTA ? 1 : 2)         // (without the correction two workgroups a CU fit the LDS)
+__global__ void __launch_bounds__(256, DELTA && CH && DB == 8 ? 1 : 2)    // (two workgroups a CU: up to 75 KB of LDS and half of the registers each)
 chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restrict__ proj, int ld, int b_off, int a_off,
                      const float* __restrict__ A_log, const float* __restrict__ dt_bias,
                      const float* __restrict__ decay, const int2* __restrict__ chunks, float* __restrict__ scratch,
@@ -98,12 +100,16 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
     constexpr int NG = CH ? 4 * DB : 1;                       // decays a lane holds of its token
     // (the linear attention's decays multiply single entries of a sum, whose roundings average out)
     using Decay = typename std::conditional<DELTA, double, float>::type;
-    // columns' keys in the order their lanes read them, later G_64 / G k with a row a key entry
-    __shared__ __attribute__((aligned(16))) float cols[D * TLD];
-    __shared__ __attribute__((aligned(16))) float rows[CHUNK * (DELTA ? KLD : TLD)];     // B, later G k and -T beta G k
+    // The same LDS twice: first the keys of columns in the order their lanes read them, and B; then G k and -T beta G k, and T beta.
+    constexpr int FIRST_USE = CHUNK * (D + TLD), SECOND_USE = DELTA ? CHUNK * (KLD + TLD) : 0;
+    __shared__ __attribute__((aligned(16))) float region[FIRST_USE > SECOND_USE ? FIRST_USE : SECOND_USE];
+    float* const cols = region;
+    float* const b_rows = region + CHUNK * D;
+    float* const rows = region;                               // DELTA alone, as are the next three
+    float* const solve = region + CHUNK * KLD;                // T beta
     __shared__ __attribute__((aligned(16))) float lower[DELTA ? CHUNK * TLD : 4];        // beta A below the diagonal
     __shared__ __attribute__((aligned(16))) float inverse[DELTA ? 4 * 16 * 20 : 4];      // of I + its diagonal blocks
-    __shared__ __attribute__((aligned(16))) float solve[DELTA ? CHUNK * TLD : 4];        // T beta
+    __shared__ Decay behind[CH ? 1 : CHUNK];                  // a token's product of decays to its block's end
     __shared__ Decay total[4][CH ? D : 1];                    // a block's product of decays
     __shared__ float betas[CHUNK];
     __shared__ int wild_from, wild_values;
@@ -202,26 +208,42 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
 #pragma unroll
     for (int e = 0; e < 4; ++e)
         if (4 * e + q == r) b_sum[e] = own;
+    // With one decay a head the pairs' sums over the key's entries are made once, without decays, and each takes the product of the
+    // decays between behind it; with a decay a channel a level's decays are in its operands.
+    f64x4 al = {0.0, 0.0, 0.0, 0.0}, bl = al;
+    auto pairs = [&]() {
+        al = bl = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int i = 0; i < 4 * DB; ++i) {
+            const double k = kq[i / 4][i % 4];
+            if (DELTA) al = mfma64_k4(k, k, al);
+            bl = mfma64_k4(qq[i / 4][i % 4], k, bl);
+        }
+    };
+    if (!CH) pairs();
 #pragma unroll
     for (int level = 0; level < 4; ++level) {
         const int s = 1 << level;
         const bool late = (r / s) & 1;
-        // (the keys and queries are made float64 anew in every level: kept so they would take twice their registers)
+        if (CH) {
+            // (the keys and queries are made float64 anew in every level: kept so they would take twice their registers)
 #pragma unroll
-        for (int b = 0; b < DB; ++b) asm volatile("" : "+v"(kq[b]), "+v"(qq[b]));
-        f64x4 al = {0.0, 0.0, 0.0, 0.0}, bl = al;
+            for (int b = 0; b < DB; ++b) asm volatile("" : "+v"(kq[b]), "+v"(qq[b]));
+            al = bl = f64x4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for (int i = 0; i < 4 * DB; ++i) {
-            const Decay f = late ? pre[CH ? i : 0] : suf[CH ? i : 0];
-            const double k = kq[i / 4][i % 4] * f;
-            if (DELTA) al = mfma64_k4(k, k, al);
-            bl = mfma64_k4(qq[i / 4][i % 4] * f, k, bl);
+            for (int i = 0; i < 4 * DB; ++i) {
+                const Decay f = late ? pre[CH ? i : 0] : suf[CH ? i : 0];
+                const double k = kq[i / 4][i % 4] * f;
+                if (DELTA) al = mfma64_k4(k, k, al);
+                bl = mfma64_k4(qq[i / 4][i % 4] * f, k, bl);
+            }
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int t = 4 * e + q;
             const bool pair = t / (2 * s) == r / (2 * s) && ((t / s) & 1) && !((r / s) & 1);
-            if (pair) a_sum[e] = al[e], b_sum[e] = bl[e];
+            const double f = CH ? 1.0 : __shfl(pre[0], (lane & 48) + t, HB_WAVE) * suf[0];
+            if (pair) a_sum[e] = CH ? al[e] : al[e] * f, b_sum[e] = CH ? bl[e] : bl[e] * f;
         }
         // the products over runs of 2 s: up to a token from its run's start, and behind a token to its run's end
         const int before = (lane & 48) + (r & ~(2 * s - 1)) + s - 1, after = before + s;
@@ -243,17 +265,20 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
     }
 #pragma unroll
     for (int b = 0; b < DB; ++b) {
-        f32x4 k;
+        f32x4 k = kq[b];
+        if (CH) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) k[e] = (float)(kq[b][e] * suf[CH ? 4 * b + e : 0]);
+            for (int e = 0; e < 4; ++e) k[e] = (float)(kq[b][e] * suf[CH ? 4 * b + e : 0]);
+        }
         *(f32x4*)&cols[((wave * DB + b) * 64 + lane) * 4] = k;
     }
+    if (!CH && q == 0) behind[CH ? 0 : token] = suf[0];
     auto put = [&](f64x4 a, f64x4 b, int block) {             // sums of (16 wave + 4 e + q, 16 block + r)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int t = 16 * wave + 4 * e + q;
             if (DELTA) lower[t * TLD + in_quads(16 * block + r)] = (float)(betas[t] * a[e]);
-            rows[t * TLD + in_quads(16 * block + r)] = (float)b[e];
+            b_rows[t * TLD + in_quads(16 * block + r)] = (float)b[e];
         }
     };
     put(a_sum, b_sum, wave);
@@ -280,13 +305,26 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
             const f32x4 k = *(const f32x4*)&cols[((block * DB + b) * 64 + lane) * 4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const Decay p = pre[CH ? 4 * b + e : 0];
-                if (DELTA) al = mfma64_k4(kq[b][e] * p, k[e], al);
-                bl = mfma64_k4(qq[b][e] * p, k[e], bl);
-                if (CH) pre[4 * b + e] *= total[block][16 * b + 4 * e + q];
+                if (CH) {
+                    const Decay p = pre[CH ? 4 * b + e : 0];
+                    if (DELTA) al = mfma64_k4(kq[b][e] * p, k[e], al);
+                    bl = mfma64_k4(qq[b][e] * p, k[e], bl);
+                    pre[CH ? 4 * b + e : 0] *= total[block][CH ? 16 * b + 4 * e + q : 0];
+                } else {
+                    if (DELTA) al = mfma64_k4(kq[b][e], k[e], al);
+                    bl = mfma64_k4(qq[b][e], k[e], bl);
+                }
             }
         }
-        if (!CH) pre[0] *= total[block][0];
+        if (!CH) {
+            const double f = behind[CH ? 0 : 16 * block + r];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const double g = __shfl(pre[0], (lane & 48) + 4 * e + q, HB_WAVE) * f;
+                al[e] *= g, bl[e] *= g;
+            }
+            pre[0] *= total[block][0];
+        }
         put(al, bl, block);
     }
     f32x4 gk[DELTA ? DB : 1];                                 // G k
@@ -310,28 +348,28 @@ chunk_prepare_kernel(const float* __restrict__ qkv, int C, const float* __restri
 #pragma unroll
     for (int b = 0; b < 4; ++b)
         if (b <= wave)
-            *(f32x4*)(out + at.b + ((wave * 4 + b) * 64 + lane) * 4) = *(const f32x4*)&rows[(16 * wave + r) * TLD + 16 * b + 4 * q];
+            *(f32x4*)(out + at.b + ((wave * 4 + b) * 64 + lane) * 4) = *(const f32x4*)&b_rows[(16 * wave + r) * TLD + 16 * b + 4 * q];
     if (CH) {
         for (int d = tid; d < D; d += 256) out[at.g + d] = total[0][d] * total[1][d] * total[2][d] * total[3][d];
     } else {
         for (int d = tid; d < D; d += 256) out[at.g + d] = (float)(total[0][0] * total[1][0] * total[2][0] * total[3][0]);
     }
-    __syncthreads();                                          // cols and rows have been read
+    __syncthreads();                                          // cols and B have been read
+    // G_64 / G k with a row a key entry: a block of 16 tokens and 16 entries at a time, turned in LDS of the wave's own
+    float* const turn = (DELTA ? solve : region) + wave * 16 * 20;
 #pragma unroll
-    for (int b = 0; b < DB; ++b)
+    for (int b = 0; b < DB; ++b) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int d = 16 * b + 4 * e + q;
-            cols[d * TLD + in_quads(token)] = (float)(kq[b][e] * suf[CH ? 4 * b + e : 0]);
-            if (DELTA) rows[token * KLD + in_quads(d)] = gk[b][e];
+            turn[(4 * e + q) * 20 + in_quads(r)] = (float)(kq[b][e] * suf[CH ? 4 * b + e : 0]);
+            if (DELTA) rows[token * KLD + in_quads(16 * b + 4 * e + q)] = gk[b][e];
         }
-    __syncthreads();
-#pragma unroll
-    for (int b = wave; b < DB; b += 4)
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-            *(f32x4*)(out + at.k + ((b * 4 + s) * 64 + lane) * 4) = *(const f32x4*)&cols[(16 * b + r) * TLD + 16 * s + 4 * q];
+        asm volatile("" ::: "memory");                        // (a wave's LDS accesses keep their order)
+        *(f32x4*)(out + at.k + ((b * 4 + wave) * 64 + lane) * 4) = *(const f32x4*)&turn[r * 20 + 4 * q];
+        asm volatile("" ::: "memory");
+    }
     if (!DELTA) return;
+    __syncthreads();                                          // turn has been read
 
     // ---- T beta, a block of 16 columns a wave: its blocks of rows one after another, as the next product wants them
     {
