@@ -938,31 +938,33 @@ grouped_mfma_kernel(const bf16* __restrict__ A, int lda, size_t a_group_off, con
     }
 }
 
-// The same for groups of many rows: a workgroup on 64 TM rows (128, 192 or 256) and 256 weight rows (EPI 2: 128 gate rows and the
-// 128 up rows that go with them, in turns of 16), each of four waves on 128 weight rows x 32 TM rows by 32x32x16 products. What bounds
-// it are the bytes that a CU takes out of the caches, about 45 a nanosecond whatever the kernel: 48 to 64 KB a step of 64 k here, which last
+// The same for groups of many rows: a workgroup on 32 TM rows (128, 192 or 256) and 256 weight rows (EPI 2: 128 gate rows and the
+// 128 up rows that go with them, in turns of 16), each of four waves on 128 weight rows x 16 TM rows. What bounds
+// it are the bytes that a CU takes out of the caches, 48 to 64 KB a step of 64 k here, which last
 // longer than the step's products, so the tile is as high as a group's rows fill it (rows beyond a tile's own read its last row
 // again, which costs no such bytes). The kernel above reads the weights for every 64 rows. Weights and activations go straight into rings in LDS (hb_load_to_lds),
-// waited for by count before a bare barrier. There is no branch in the main loop (the last step is peeled off); reads and loads are dealt
-// out between the products, the reads of a k-step during the products of the one before. An activation row is 128 bytes, its 16-byte
+// waited for by count before a bare barrier. There is no branch in the main loop; reads and loads are dealt
+// out between the products, the reads of a k-step during the products of the one before. The weights' third stage lets their loads, two
+// steps ahead, go out during a step's first 32 k and the activations' during its second, so that a CU's loads last the whole step. An
+// activation row is 128 bytes, its 16-byte
 // chunk c at chunk c ^ ((row >> 1) & 7); a block of 16 weight rows and 32 k is 1 KB as packed. K in steps of 64.
 // Gate/up of 32 experts of 768 on 2,048, weights from memory (40 us at the rate of a large copy), by tiles of 64 and by the tile that
-// tall_rows of moe.py takes: 2,048 tokens, four experts each, 127 us, 90 (128 rows); 1,712 (without a shared expert) 103, 76 (256); 1,282 101, 60 (192); 512 63, 49
-// (128). 64 experts of 1,536 on 4,096, 2,500 tokens: 522, 353 (192).
-typedef float hb_f32x16 __attribute__((ext_vector_type(16)));
+// tall_rows of moe.py takes, in brackets that one by 32x32x16 products with all loads of a step in its second half: 2,048 tokens, four experts
+// each, 117 us, 84 (128 rows; 88); 1,712 101, 67 (256; 73); 1,282 98, 56 (192; 59); 512 57, 47 (128; 48). 64 experts of 1,536 on 4,096, 2,500
+// tokens: 505, 398 (192; 435); 1,500 340, 303 (128; 307).
 #define TALL_BN 256
 #define TALL_W_STAGE (TALL_BN * 64)          // elements
-// (a third stage of the weights for tiles of 128 and 192; with one 256 takes as long or 3 % longer)
-constexpr int tall_wst(int TM) { return TM <= 3 ? 3 : 2; }
-constexpr int tall_lds_of(int TM) { return (tall_wst(TM) * TALL_W_STAGE + 2 * 64 * TM * 64) * 2; }
+#define TALL_WST 3
+#define TALL_XST 2
+constexpr int tall_lds_of(int TM) { return (TALL_WST * TALL_W_STAGE + TALL_XST * 32 * TM * 64) * 2; }
 template <int EPI, int TM>
 __global__ void __launch_bounds__(256)
 grouped_tile_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W, int N, int K, void* __restrict__ Cv, int ldc,
                     const int* __restrict__ order, int top, const int* __restrict__ tile_group,
                     const int* __restrict__ tile_row0, const int* __restrict__ tile_rows, float limit, float alpha, float shift,
                     int tiles, int columns) {
-    extern __shared__ __attribute__((aligned(1024))) bf16 tall_lds[];       // [WST][W_STAGE], then [XST][X_STAGE]
-    constexpr int WST = tall_wst(TM), XST = 2, X_STAGE = 64 * TM * 64;
+    extern __shared__ __attribute__((aligned(1024))) bf16 tall_lds[];       // [TALL_WST][W_STAGE], then [TALL_XST][X_STAGE]
+    constexpr int WST = TALL_WST, XST = TALL_XST, X_STAGE = 32 * TM * 64;
     bf16* const xlds = tall_lds + WST * TALL_W_STAGE;
     // (which tile and block of columns: as in the kernel above)
     const int turn = blockIdx.x / XCDS, run = turn / TILE_RUN * XCDS + blockIdx.x % XCDS;
@@ -972,13 +974,12 @@ grouped_tile_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict_
     if (group < 0) return;
     const int row0 = tile_row0[tile], rows = tile_rows[tile];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int c32 = lane & 31, g2 = lane >> 5;
+    const int r16 = lane & 15, g4 = lane >> 4;
     const int wn = wave >> 1, wm = wave & 1;
     const int F = N / 2, out_cols = EPI == 2 ? F : N;
     const int nsteps = K / 64;
     const size_t wstep = (size_t)(N / 16) * 512;
-    constexpr int WL = 4, XR = 2 * TM, NLW = 2 * WL, NLX = XR, TN = 4;
-    constexpr int LATER = WST == 3 ? NLW : 0;              // loads that may be in flight at the barrier: a later step's weights
+    constexpr int WL = 4, NLX = TM, NLW = 2 * WL, TN = 8;  // a wave's loads of a step
     const bf16* wsrc[WL];
 #pragma unroll
     for (int i = 0; i < WL; ++i) {
@@ -989,46 +990,46 @@ grouped_tile_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict_
         if (EPI == 2 && (blk & 1)) nb += F / 16;
         wsrc[i] = W + (size_t)group * N * K + ((size_t)nb * 64 + lane) * 8;
     }
-    const bf16* xsrc[XR];
+    const bf16* xsrc[NLX];
 #pragma unroll
-    for (int i = 0; i < XR; ++i) {
-        const int r = (wave * XR + i) * 8 + (lane >> 3), m = r < rows ? r : rows - 1;
+    for (int i = 0; i < NLX; ++i) {
+        const int r = (wave * NLX + i) * 8 + (lane >> 3), m = r < rows ? r : rows - 1;
         const int src = top > 0 ? order[row0 + m] / top : row0 + m;
         xsrc[i] = A + (size_t)src * lda + ((lane & 7) ^ ((r >> 1) & 7)) * 8;
     }
-    // the idx-th load of a step: first the activations of step xstep, then the weights of step w_step
-    auto load_one = [&](int xstep, int xstage, int w_step, int wstage, int idx) {
-        if (idx < NLX) {
-            hb_load_to_lds(xsrc[idx] + (size_t)xstep * 64, xlds + xstage * X_STAGE + (wave * XR + idx) * 512);
-        } else {
-            const int ks = (idx - NLX) / WL, w = (idx - NLX) % WL;
-            hb_load_to_lds(wsrc[w] + ((size_t)w_step * 2 + ks) * wstep,
-                           tall_lds + wstage * TALL_W_STAGE + ks * (TALL_BN / 16) * 512 + (wave * WL + w) * 512);
-        }
+    auto load_x = [&](int step, int stage, int i) {
+        hb_load_to_lds(xsrc[i] + (size_t)step * 64, xlds + stage * X_STAGE + (wave * NLX + i) * 512);
     };
-    hb_f32x16 acc[TN][TM];
+    auto load_w = [&](int step, int stage, int i) {
+        const int ks = i / WL, w = i % WL;
+        hb_load_to_lds(wsrc[w] + ((size_t)step * 2 + ks) * wstep,
+                       tall_lds + stage * TALL_W_STAGE + ks * (TALL_BN / 16) * 512 + (wave * WL + w) * 512);
+    };
+    hb_f32x4 acc[TN][TM];
 #pragma unroll
     for (int a = 0; a < TN; ++a)
 #pragma unroll
-        for (int b = 0; b < TM; ++b)
+        for (int b = 0; b < TM; ++b) acc[a][b] = hb_f32x4{0.f, 0.f, 0.f, 0.f};
+    // (the sums stay in accumulation registers: without this the compiler moves them between the products)
+    auto hold = [&]() {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.f;
-    constexpr int NM = 2 * TN * TM, NR = 2 * (TN + TM), SLOTS = NM - 4;
-    const int w_lane = (c32 >> 4) * 512 + (16 * g2 + (lane & 15)) * 8 + wn * 8 * 512;
-    const int x_lane = (wm * TM * 32 + c32) * 64, x_swizzle = (c32 >> 1) & 7;
-    hb_bf16x8 wv[2][2][TN], xv[2][2][TM];                  // [set][k-half][piece]
-    auto mfma_one = [&](int set, int j) {
-        const int h = j / (TN * TM), a = j / TM % TN, b = j % TM;
-        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv[set][h][a], xv[set][h][b], acc[a][b], 0, 0, 0);
+        for (int a = 0; a < TN; ++a)
+#pragma unroll
+            for (int b = 0; b < TM; ++b) asm volatile("" : "+a"(acc[a][b]));
     };
-    auto read_one = [&](int set, int step, int ks, int idx) {
-        const int h = idx / (TN + TM), r = idx % (TN + TM);
-        if (r < TN)
-            wv[set][h][r] = *(const hb_bf16x8*)(tall_lds + (step % WST) * TALL_W_STAGE + ks * (TALL_BN / 16) * 512 + w_lane +
-                                                r * 1024 + h * 256);
+    constexpr int NM = TN * TM, NR = TN + TM, SLOTS = NM - 8;
+    const int w_lane = lane * 8 + wn * TN * 512;
+    const int x_lane = (wm * TM * 16 + r16) * 64, x_swizzle = (r16 >> 1) & 7;
+    hb_bf16x8 wv[2][TN], xv[2][TM];                        // [set][block]
+    auto mfma_one = [&](int set, int j) {
+        const int a = j / TM, b = j % TM;
+        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[set][a], xv[set][b], acc[a][b], 0, 0, 0);
+    };
+    auto read_one = [&](int set, int step, int ks, int idx) {      // (all activations and the first weights are needed first)
+        if (idx < TM)
+            xv[set][idx] = *(const hb_bf16x8*)(xlds + (step % XST) * X_STAGE + x_lane + idx * 16 * 64 + (((4 * ks + g4) ^ x_swizzle) * 8));
         else
-            xv[set][h][r - TN] = *(const hb_bf16x8*)(xlds + (step % XST) * X_STAGE + x_lane + (r - TN) * 32 * 64 +
-                                                     (((4 * ks + 2 * h + g2) ^ x_swizzle) * 8));
+            wv[set][idx - TM] = *(const hb_bf16x8*)(tall_lds + (step % WST) * TALL_W_STAGE + ks * (TALL_BN / 16) * 512 + w_lane + (idx - TM) * 512);
     };
     // between the products j and j + 1 of a k-step: nl loads and NR reads, dealt out over the first SLOTS products
     auto between = [&](int j, int nl, auto&& load, auto&& read) {
@@ -1042,52 +1043,43 @@ grouped_tile_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict_
         }
     };
     auto clamp = [&](int step) { return step < nsteps ? step : nsteps - 1; };   // past the end: the last step again
-    // in flight before the loop: steps 0 and 1, and with a third stage step 2 of the weights
+    // in flight before the loop: steps 0 and 1
 #pragma unroll
-    for (int i = 0; i < NLX + NLW; ++i) load_one(0, 0, 0, 0, i);
+    for (int s = 0; s < 2; ++s) {
 #pragma unroll
-    for (int i = 0; i < NLX + NLW; ++i) load_one(clamp(1), 1, clamp(1), 1, i);
-    if (WST == 3) {
+        for (int i = 0; i < NLX; ++i) load_x(clamp(s), s, i);
 #pragma unroll
-        for (int i = NLX; i < NLX + NLW; ++i) load_one(0, 0, clamp(2), 2, i);
+        for (int i = 0; i < NLW; ++i) load_w(clamp(s), s, i);
     }
-    hb_wait_vmcnt<NLX + NLW + LATER>();
+    hb_wait_vmcnt<NLX + NLW>();
     hb_workgroup_barrier();
 #pragma unroll
     for (int i = 0; i < NR; ++i) read_one(0, 0, 0, i);
-    for (int t = 0; t + 1 < nsteps; ++t) {
+    hold();
+    // (the last step is one like any other: what it loads and reads ahead nobody uses)
+    for (int t = 0; t < nsteps; ++t) {
+        const int ahead = clamp(t + 2);
+        // the first half of a step; its weights of two steps on go into the stage that step t - 1 left at its barrier
 #pragma unroll
         for (int j = 0; j < NM; ++j) {
             mfma_one(0, j);
-            between(j, 0, [&](int) {}, [&](int i) { read_one(1, t, 1, i); });
+            between(j, NLW, [&](int i) { load_w(ahead, (t + 2) % WST, i); }, [&](int i) { read_one(1, t, 1, i); });
             __builtin_amdgcn_sched_barrier(0);
         }
-        // step t + 1 has landed (in flight at most the weights of a later step) and, after the barrier, nobody reads step t any more
-        hb_wait_vmcnt<LATER>();
+        // step t + 1 has landed (in flight at most those weights) and, after the barrier, nobody reads step t any more
+        hb_wait_vmcnt<NLW>();
         hb_workgroup_barrier();
-        const int xstep = clamp(t + XST), w_step = clamp(t + WST);
 #pragma unroll
         for (int j = 0; j < NM; ++j) {
             mfma_one(1, j);
-            between(j, NLX + NLW, [&](int i) { load_one(xstep, t % XST, w_step, t % WST, i); },
-                    [&](int i) { read_one(0, t + 1, 0, i); });
+            between(j, NLX, [&](int i) { load_x(ahead, t % XST, i); }, [&](int i) { read_one(0, t + 1, 0, i); });
             __builtin_amdgcn_sched_barrier(0);
         }
-    }
-    {
-        const int t = nsteps - 1;
-#pragma unroll
-        for (int j = 0; j < NM; ++j) {
-            mfma_one(0, j);
-            between(j, 0, [&](int) {}, [&](int i) { read_one(1, t, 1, i); });
-            __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int j = 0; j < NM; ++j) mfma_one(1, j);
+        hold();
     }
     hb_wait_vmcnt<0>();      // the loads past the end (repeats of the last step) have landed too
     hb_workgroup_barrier();
-    // A lane holds runs of four columns of rows 32 b + c32: through LDS of the wave's own, so that whole rows leave. Rows of CH
+    // A lane holds runs of four columns of rows 16 b + r16: through LDS of the wave's own, so that whole rows leave. Rows of CH
     // 16-byte chunks, chunk c of row r at c ^ (r mod CH).
     constexpr int COLS = EPI == 2 ? 64 : 128;              // the wave's output columns
     constexpr int PER = EPI == 0 ? 4 : 8;                  // columns a chunk
@@ -1097,22 +1089,22 @@ grouped_tile_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict_
     const int rrow = lane / CH, rchunk = lane % CH;
     const int n = column * (EPI == 2 ? TALL_BN / 2 : TALL_BN) + wn * COLS + rchunk * PER;
 #pragma unroll
-    for (int b = 0; b < TM; ++b) {
+    for (int b0 = 0; b0 < TM; b0 += 2) {
 #pragma unroll
-        for (int a = 0; a < TN; ++a)
+        for (int b = b0; b < b0 + 2; ++b) {
+            __builtin_amdgcn_sched_barrier(0);             // (a block of rows after the other: all at once take more registers than there are)
 #pragma unroll
-            for (int q = 0; q < (EPI == 2 ? 2 : 4); ++q) {
-                hb_f32x4 v;
+            for (int a = 0; a < TN; a += EPI == 2 ? 2 : 1) {
+                hb_f32x4 v = acc[a][b];
+                if (EPI == 2) {                            // a block of gate rows, then one of their up rows
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    v[i] = acc[a][b][4 * q + i];
-                    if (EPI == 2) {                        // rows 0 .. 15 of a piece are gate rows, 16 .. 31 their up rows
-                        const float g = fminf(v[i], limit), u = fminf(fmaxf(acc[a][b][4 * q + 8 + i], -limit), limit);
+                    for (int i = 0; i < 4; ++i) {
+                        const float g = fminf(v[i], limit), u = fminf(fmaxf(acc[a + 1][b][i], -limit), limit);
                         v[i] = g / (1.0f + expf(-alpha * g)) * (u + shift);
                     }
                 }
-                const int col = (EPI == 2 ? 16 : 32) * a + 8 * q + 4 * g2;
-                char* const at = stage + (c32 * CH + ((col / PER) ^ (c32 & (CH - 1)))) * 16;
+                const int row = 16 * (b - b0) + r16, col = (EPI == 2 ? 8 : 16) * a + 4 * g4;
+                char* const at = stage + (row * CH + ((col / PER) ^ (row & (CH - 1)))) * 16;
                 if (EPI == 0) {
                     *(hb_f32x4*)at = v;
                 } else {
@@ -1122,9 +1114,10 @@ grouped_tile_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict_
                     *(uint2*)(at + (col % PER) * 2) = uint2{o[0].bits | ((unsigned)o[1].bits << 16), o[2].bits | ((unsigned)o[3].bits << 16)};
                 }
             }
+        }
 #pragma unroll
         for (int i = 0; i < 32 / RPI; ++i) {
-            const int row = i * RPI + rrow, m = (wm * TM + b) * 32 + row;
+            const int row = i * RPI + rrow, m = (wm * TM + b0) * 16 + row;
             const uint4 v = *(const uint4*)(stage + (row * CH + (rchunk ^ (row & (CH - 1)))) * 16);
             if (m < rows && n < out_cols)                  // (columns come in whole blocks of 16)
                 *(uint4*)((char*)Cv + ((size_t)(row0 + m) * ldc + n) * (EPI == 0 ? 4 : 2)) = v;
@@ -1157,9 +1150,9 @@ extern "C" int hb_grouped_tall(const void* A, int lda, const void* W, int N, int
     } while (0)
 #define HB_TALL_OF(E)                       \
     do {                                    \
-        if (tile_m == 128) HB_TALL(E, 2);   \
-        else if (tile_m == 192) HB_TALL(E, 3); \
-        else HB_TALL(E, 4);                 \
+        if (tile_m == 128) HB_TALL(E, 4);   \
+        else if (tile_m == 192) HB_TALL(E, 6); \
+        else HB_TALL(E, 8);                 \
     } while (0)
     if (epi == 0) HB_TALL_OF(0);
     else if (epi == 1) HB_TALL_OF(1);
