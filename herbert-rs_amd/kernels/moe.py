@@ -178,12 +178,10 @@ EPI_F32, EPI_BF16, EPI_GLU = 0, 1, 2
 # 19 / 32, 64 rows 32 / 37. A head's product of rows that all heads share, 16 of 512 x 128: 16 rows 4.4 / 5.4, 64 rows 5.4 / 8.0.
 FEW_ROWS = 16
 # From so many rows an expert on the kernel of tall tiles takes gate/up. Microseconds by tiles of 64 / of 128 (weights from memory): 32
-# experts of 768 on 2,048: 32 rows an expert 58 / 48, 50 rows 59 / 48, 64 rows 63 / 49, 96 rows 63 / 50; 64 of 1,536 on 4,096: 62 rows
-# 363 / 310; where fewer than half the CUs get a tile (16 of 512 on 1,024: 64 rows 24 / 23) nothing is gained. A tile's start and
-# end weigh as much as eight of its steps of 64 k, so down, whose k is short, takes tall tiles from DOWN_STEPS steps and DOWN_ROWS rows on:
-# 12 steps 52 / 67 in a model whose experts are unequally busy (214 rows on average), 68 / 67 (256 rows); 24 steps, 156 rows 259 / 218, 62
-# rows 169 / 182.
-DOWN_STEPS, DOWN_ROWS = 16, 128
+# experts of 768 on 2,048: 32 rows an expert 58 / 48, 50 rows 59 / 48, 64 rows 57 / 47, 96 rows 63 / 50; 64 of 1,536 on 4,096: 62 rows
+# 363 / 310; where fewer than half the CUs get a tile (16 of 512 on 1,024: 64 rows 24 / 23) nothing is gained.
+# Down, whose k is short, takes tall tiles from DOWN_STEPS steps of 64 k and DOWN_ROWS rows on where down_tall expects them to be done sooner.
+DOWN_STEPS, DOWN_ROWS = 12, 128
 TALL_ROWS = 48
 
 
@@ -191,6 +189,15 @@ def mfma_takes(K, lda, a_group_off=0, N=16):
     """True if the matrix-core kernel takes products of this inner size, layout and N weight rows
     (bfloat16 operands)."""
     return K % 32 == 0 and lda % 8 == 0 and a_group_off % 8 == 0 and N % 16 == 0
+
+
+def tiles_expected(height, T, rows, experts, shared):
+    """The tiles of `height` rows of a step of T tokens whose experts have `rows` rows on average, spread as a random choice spreads them."""
+    tiles, k = 1.0, 1
+    while k * height < rows + 4.0 * rows ** 0.5:           # more than k tiles: the chance that an expert has more than k height rows
+        tiles += 0.5 * math.erfc((k * height - rows) / (2.0 * rows) ** 0.5)
+        k += 1
+    return experts * tiles + (-(-T // height) if shared else 0)
 
 
 @functools.lru_cache(maxsize=1024)
@@ -213,14 +220,27 @@ def tall_rows(T, top, routed, experts, hidden, inter, shared=False):
     columns = -(-2 * inter // 256)
 
     def workgroups(height):
-        tiles, k = 1.0, 1
-        while k * height < rows + 4.0 * rows ** 0.5:       # more than k tiles: the chance that an expert has more than k height rows
-            tiles += 0.5 * math.erfc((k * height - rows) / (2.0 * rows) ** 0.5)
-            k += 1
-        return (experts * tiles + (-(-T // height) if shared else 0)) * columns
+        return tiles_expected(height, T, rows, experts, shared) * columns
     cost = {h: math.ceil(workgroups(h) / 256 + 0.1) * (256 + h) for h in TALL_TILES if workgroups(h) >= 128}
     cost[0] = math.ceil(workgroups(TILE_M) / 512 + 0.1) * 540 if cost else 0
     return min(cost, key=cost.get)
+
+
+@functools.lru_cache(maxsize=1024)
+def down_tall(T, top, routed, experts, hidden, inter, shared, height):
+    """True if the down product of a layer whose gate/up takes tall tiles of `height` rows takes them too: where its rounds of tiles over the
+    CUs are expected to be done before the low tiles', two to a CU. A round of `steps` steps of 64 k takes height / 122 us a step and 8
+    beside them, one of low tiles 1.75 and 3. Microseconds by low / tall tiles, 32 experts of 768 on 2,048, four each: 2,048 tokens 69 / 62
+    (128 rows), with a shared expert 70 / 81 (192, the low ones here), 1,712 tokens 51 / 44 (256), 4,000 tokens 108 / 98 (256); 64 of 1,536 on
+    4,096: 2,500 tokens 271 / 237 (192)."""
+    steps, rows = inter // 64, T * top / routed
+    if not height or steps < DOWN_STEPS or rows < DOWN_ROWS:
+        return False
+    columns = -(-hidden // 256)
+
+    def rounds(tile, at_once):
+        return math.ceil(tiles_expected(tile, T, rows, experts, shared) * columns / at_once + 0.1)
+    return rounds(height, 256) * (height / 122 * steps + 8) < rounds(TILE_M, 512) * (1.75 * steps + 3)
 
 
 def fold_pays(T, top, experts, hidden, inter):

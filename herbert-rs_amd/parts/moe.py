@@ -172,7 +172,7 @@ class RoutedExperts(Part):
             moe.grouped_mfma(y, self.hidden_size, 0, gate_up, act, F, 0, moe.EPI_GLU, routing, gather=True,
                              limit=self.limit, alpha=self.alpha, shift=self.shift, tall=tall > 0)
             moe.grouped_mfma(act, F, 0, down, out, self.hidden_size, 0, moe.EPI_F32, routing,
-                             tall=tall > 0 and F >= 64 * moe.DOWN_STEPS and T * top >= moe.DOWN_ROWS * E)
+                             tall=moe.down_tall(T, top, E, self.experts, self.hidden_size, F, folded, tall))
         else:
             gu = rt.buffer("moe_gate_up", (T * top, 2 * F), torch.float32)
             moe.gemm_plain(y, self.gate_up, gu, routing, gather=True)

@@ -119,6 +119,15 @@ def test_tile_heights_by_the_rows_an_expert_has():
     assert moe.tall_rows(512, 6, 64, 64, 2048, 1408, True) == 0 and moe.tall_rows(1600, 8, 256, 256, 2048, 512) == 0
 
 
+def test_tiles_of_the_down_product():
+    """Tall tiles where their rounds are done sooner than the low tiles': both sides of the lines in steps of k, rows and rounds."""
+    assert not moe.down_tall(2048, 4, 32, 32, 2048, 768, False, 0)
+    assert moe.down_tall(2048, 4, 32, 32, 2048, 768, False, 128) and not moe.down_tall(2048, 4, 32, 32, 2048, 704, False, 128)
+    assert not moe.down_tall(2048, 4, 32, 32, 2048, 768, True, 192)
+    assert moe.down_tall(1712, 4, 32, 32, 2048, 768, False, 256) and not moe.down_tall(1000, 4, 32, 32, 2048, 768, False, 128)
+    assert moe.down_tall(2500, 4, 64, 64, 4096, 1536, False, 192) and not moe.down_tall(1500, 4, 64, 64, 4096, 1536, False, 128)
+
+
 def test_a_shared_expert_is_folded_only_where_that_pays():
     """Both sides of the lines: always beyond the steps of few rows an expert, in them while its rows are few tiles of matrices
     that are small enough to be read again."""
