@@ -224,65 +224,60 @@ extern "C" int hb_latent_attention_plain(const float* q_full, const void* pages,
 }
 
 // ------------------------------------------------ the same attention on the matrix cores (bfloat16 rows)
-// A wave takes 16 heads of one token (the rows of its matrix products) and a range of the keys, in
-// chunks of 32. Scores: S^T = K Q^T, the chunk's rows straight from memory as operands (a lane: one
+// A workgroup of four waves takes 16 heads of one token (the rows of its matrix products) and a range of the keys, in
+// chunks of 32; a wave takes a quarter of a row's numbers. Scores: S^T = K Q^T, the chunk's rows straight from memory as operands (a lane: one
 // key's 8 consecutive numbers), the query (times the scale) in registers as two bfloat16 halves, high
 // and low, so that it keeps 16 bits of mantissa (with the high half alone a test with large queries
-// lost a digit). The sums are float32, and so are the softmax and its state, which are a lane's own
-// (a lane holds scores of one head only). Weighted sums: O^T = V^T P^T
+// lost a digit). The sums are float32; the waves' parts of them meet in LDS, where every wave adds them in the waves' order. The softmax and
+// its state are a lane's own (a lane holds scores of one head only) and the same in every wave. Weighted sums: O^T = V^T P^T
 // with the weights again as high and low halves (they are never rounded to 8 bits), and V^T, the
-// chunk's first `rank` numbers a key with the keys along a row, written to LDS from the registers
-// that hold them as the scores' operands. The 32 keys
-// of a product stand in the order in which the scores' lanes hold them (4 g + i of the first block of
-// 16, then of the second), so the weights go from the scores' registers into the next product as they
-// are. With more than one range a token the unnormalised sums, maxima and denominators go to scratch
-// and a second kernel joins them in the ranges' order.
-// Sizes: rank and rot multiples of 32; RB >= rank / 16, KSM >= (rank + rot) / 32.
+// wave's part of the chunk's first `rank` numbers a key with the keys along a row, written to LDS from the registers
+// that hold them as the scores' operands: it is the wave's own. A chunk's 32 keys stand there in pairs, n and 16 + n, so that a pair is one
+// write and a lane's eight keys of a product one read; the weights go from the scores' registers into the product in the same order.
+// The next chunk's rows are asked for as soon as a chunk's are in LDS. With more than one range a token the unnormalised sums,
+// maxima and denominators go to scratch and a second kernel joins them in the ranges' order.
+// Bound by its own chain: positions, slot, page, rows, scores, exchange, softmax, sums, and by code that a CU reads for the first time, which
+// was four times as long by one wave that held a whole row. With the kernel that joins the ranges, by one wave | now, 16 heads of 512 + 64, us:
+// 1 token at 100 keys 20.9 | 10.9, at 4,000 37 | 21; 4 at 509 22.5 | 12.5; 8 at 2,000 39 | 25; 32 at 1,000 40 | 31; 64 at 2,000 78 | 47; 200 at 300 74 | 36;
+// 32 heads, 32 at 4,000 130 | 67; 8 heads of 256 + 64, 4 at 300 13.3 | 8.7.
+// Sizes: rank and rot multiples of 32; VW >= rank / 128 steps of 32 numbers a wave, KX >= rot / 128 of the rotated part.
 typedef __bf16 la_bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 la_bf16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 la_bf16x2 __attribute__((ext_vector_type(2)));
 typedef float la_f32x4 __attribute__((ext_vector_type(4)));
 #define LA_CHUNK 32
-#define LA_VT_STRIDE 36          // bfloat16 a row of V^T in LDS: 32 keys and 8 bytes, so rows start at other banks
+#define LA_WAVES 4
+#define LA_VT_STRIDE 40          // bfloat16 a row of V^T in LDS: 32 keys and 16 bytes, so rows start at other banks
 
 __device__ __forceinline__ void la_split(float v, __bf16& hi, __bf16& lo) {
     hi = (__bf16)v;
     lo = (__bf16)(v - (float)hi);
 }
 
-template <int RB, int KSM>
-__global__ void __launch_bounds__(HB_WAVE)
+template <int VW, int KX>
+__global__ void __launch_bounds__(LA_WAVES * HB_WAVE)
 latent_attention_mfma_kernel(const float* __restrict__ q_full, const bf16* __restrict__ pages,
                              bf16* __restrict__ out, float* __restrict__ part_acc, float* __restrict__ part_ml,
                              const float* __restrict__ gate, int gate_ld, const int* __restrict__ positions,
                              const int* __restrict__ seq_of, const int* __restrict__ slots,
                              const int* __restrict__ page_table, int max_pages, int page_size, int H, int rank,
                              int rot, float scale, int splits, int chunks_per_split, const float* __restrict__ sinks) {
-    __shared__ __attribute__((aligned(16))) __bf16 Vt[RB * 16 * LA_VT_STRIDE];
+    constexpr int RB = 2 * VW, KSM = VW + KX;                // a wave's blocks of 16 sums, its steps of the scores
+    __shared__ __attribute__((aligned(16))) __bf16 Vt_all[LA_WAVES][RB * 16 * LA_VT_STRIDE];
+    __shared__ __attribute__((aligned(16))) la_f32x4 parts[2][LA_WAVES][2][HB_WAVE];
     const int HB = (H + 15) / 16;
     const int t = blockIdx.x / HB, hb = blockIdx.x % HB, split = blockIdx.y;
-    const int lane = threadIdx.x, n = lane & 15, g = lane >> 4;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 15, g = lane >> 4;
     const int h = hb * 16 + n;
     const bool head = h < H;
     const int pos = positions[t];
-    const int* pt = page_table + (size_t)slots[seq_of[t]] * max_pages;
-    const int kd = rank + rot, KS = kd / 32, rblocks = rank / 16, vsteps = rank / 32;
-    __bf16* vt_w = Vt + (8 * g) * LA_VT_STRIDE + n;          // where this lane's numbers of a key go
-
-    la_bf16x8 qh[KSM], ql[KSM];
-    {
-        const float* qrow = q_full + ((size_t)t * H + (head ? h : H - 1)) * kd + 8 * g;
-#pragma unroll
-        for (int ks = 0; ks < KSM; ++ks)
-            if (ks < KS) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    __bf16 hi, lo;
-                    la_split(qrow[32 * ks + e] * scale, hi, lo);
-                    qh[ks][e] = hi;
-                    ql[ks][e] = lo;
-                }
-            }
-    }
+    const int kd = rank + rot, KS = kd / 32, vsteps = rank / 32;
+    const int v_each = (vsteps + LA_WAVES - 1) / LA_WAVES, v_first = wave * v_each;         // v_each <= VW
+    const int v_mine = vsteps - v_first < v_each ? vsteps - v_first : v_each;               // (0 or less: none)
+    // the wave's i-th step: of its own quarter of the latent, then every fourth of the rotated part
+    auto step_at = [&](int i) { return i < VW ? v_first + i : vsteps + wave + LA_WAVES * (i - VW); };
+    auto has = [&](int i) { return i < VW ? i < v_mine : step_at(i) < KS; };
+    __bf16* const Vt = Vt_all[wave];
     const int n_chunks = (pos + LA_CHUNK) / LA_CHUNK;            // chunks that hold a key <= pos
     const int c_begin = split * chunks_per_split;
     const int c_end = n_chunks < c_begin + chunks_per_split ? n_chunks : c_begin + chunks_per_split;
@@ -291,99 +286,124 @@ latent_attention_mfma_kernel(const float* __restrict__ q_full, const bf16* __res
 #pragma unroll
     for (int db = 0; db < RB; ++db) acc[db] = la_f32x4{0.f, 0.f, 0.f, 0.f};
 
-    for (int c = c_begin; c < c_end; ++c) {
-        const int j0 = c * LA_CHUNK;
-        // the chunk's 32 keys lie in one page (pages hold a multiple of 32 positions)
-        const bf16* chunk = pages + ((size_t)pt[j0 / page_size] * page_size + j0 % page_size) * kd;
-        la_f32x4 s[2];
+    if (c_begin < c_end) {
+        const int* pt = page_table + (size_t)slots[seq_of[t]] * max_pages;
+        la_bf16x8 qh[KSM], ql[KSM], kv[2][KSM];
+        // a chunk's 32 keys lie in one page (pages hold a multiple of 32 positions)
+        auto page_of = [&](int c) { return pt[(c < c_end ? c : c_end - 1) * LA_CHUNK / page_size]; };
+        auto fetch = [&](int c, int page) {
+            const bf16* chunk = pages + ((size_t)page * page_size + c * LA_CHUNK % page_size + n) * kd + 8 * g;
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-            s[kb] = la_f32x4{0.f, 0.f, 0.f, 0.f};
-            const bf16* krow = chunk + (size_t)(kb * 16 + n) * kd + 8 * g;
+            for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-            for (int ks = 0; ks < KSM; ++ks)
-                if (ks < KS) {
-                    const la_bf16x8 kv = *(const la_bf16x8*)(krow + 32 * ks);
-                    s[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kv, qh[ks], s[kb], 0, 0, 0);
-                    s[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kv, ql[ks], s[kb], 0, 0, 0);
-                    // the same numbers are the key's part of V^T: key 16 kb + n, numbers 32 ks + 8 g + e
-                    if (ks < vsteps) {
+                for (int i = 0; i < KSM; ++i)
+                    if (has(i)) kv[kb][i] = *(const la_bf16x8*)(chunk + (size_t)(16 * kb) * kd + 32 * step_at(i));
+        };
+        const int page = page_of(c_begin);
+        int page_next = page_of(c_begin + 1);
+        const float* qrow = q_full + ((size_t)t * H + (head ? h : H - 1)) * kd + 8 * g;
 #pragma unroll
-                        for (int e = 0; e < 8; ++e) vt_w[(32 * ks + e) * LA_VT_STRIDE + 16 * kb] = kv[e];
+        for (int i = 0; i < KSM; ++i)
+            if (has(i)) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    __bf16 hi, lo;
+                    la_split(qrow[32 * step_at(i) + e] * scale, hi, lo);
+                    qh[i][e] = hi;
+                    ql[i][e] = lo;
+                }
+            }
+        fetch(c_begin, page);
+        for (int c = c_begin; c < c_end; ++c) {
+            const int j0 = c * LA_CHUNK;
+            la_f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+            for (int i = 0; i < KSM; ++i)
+                if (has(i)) {
+#pragma unroll
+                    for (int kb = 0; kb < 2; ++kb) s[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kv[kb][i], qh[i], s[kb], 0, 0, 0);
+#pragma unroll
+                    for (int kb = 0; kb < 2; ++kb) s[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kv[kb][i], ql[i], s[kb], 0, 0, 0);
+                    // the same numbers are the keys' part of V^T: keys n and 16 + n, numbers 32 i + 8 g + e of the wave's
+                    if (i < VW) {
+#pragma unroll
+                        for (int e = 0; e < 8; ++e)
+                            *(la_bf16x2*)(Vt + (32 * i + 8 * g + e) * LA_VT_STRIDE + 2 * n) = la_bf16x2{kv[0][i][e], kv[1][i][e]};
                     }
                 }
-            // (the second block's loads stay behind the first block's products: all of a chunk's rows in
-            //  flight at once would not fit the registers beside the sums)
-            __builtin_amdgcn_sched_barrier(0);
+            if (c + 1 < c_end) {
+                fetch(c + 1, page_next);
+                page_next = page_of(c + 2);
+            }
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb) parts[c & 1][wave][kb][lane] = s[kb];
+            hb_workgroup_barrier();                              // (one a chunk: the parts lie in two places by turns)
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb) {
+                s[kb] = parts[c & 1][0][kb][lane];
+#pragma unroll
+                for (int w = 1; w < LA_WAVES; ++w) s[kb] += parts[c & 1][w][kb][lane];
+            }
+            // s[kb][i]: key j0 + 16 kb + 4 g + i against head n
+            float cmax = -INFINITY;
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (j0 + 16 * kb + 4 * g + i > pos) s[kb][i] = -INFINITY;
+                    cmax = fmaxf(cmax, s[kb][i]);
+                }
+            cmax = fmaxf(cmax, __shfl_xor(cmax, 16, HB_WAVE));
+            cmax = fmaxf(cmax, __shfl_xor(cmax, 32, HB_WAVE));
+            const float m_new = fmaxf(m, cmax);                  // finite: the chunk holds a key <= pos
+            const float corr = expf(m - m_new);
+            la_bf16x8 ph, pl;
+            float psum = 0.f;
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float p = expf(s[kb][i] - m_new);
+                    psum += p;
+                    __bf16 hi, lo;
+                    la_split(p, hi, lo);
+                    ph[2 * i + kb] = hi;
+                    pl[2 * i + kb] = lo;
+                }
+            l = l * corr + psum;
+            m = m_new;
+#pragma unroll
+            for (int db = 0; db < RB; ++db)
+                if (db < 2 * v_mine) {
+                    acc[db] *= corr;
+                    const la_bf16x8 vv = *(const la_bf16x8*)(Vt + (db * 16 + n) * LA_VT_STRIDE + 8 * g);
+                    acc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv, ph, acc[db], 0, 0, 0);
+                    acc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv, pl, acc[db], 0, 0, 0);
+                }
         }
-        // s[kb][i]: key j0 + 16 kb + 4 g + i against head n
-        float cmax = -INFINITY;
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if (j0 + 16 * kb + 4 * g + i > pos) s[kb][i] = -INFINITY;
-                cmax = fmaxf(cmax, s[kb][i]);
-            }
-        cmax = fmaxf(cmax, __shfl_xor(cmax, 16, HB_WAVE));
-        cmax = fmaxf(cmax, __shfl_xor(cmax, 32, HB_WAVE));
-        const float m_new = fmaxf(m, cmax);                     // finite: the chunk holds a key <= pos
-        const float corr = expf(m - m_new);
-        la_bf16x8 ph, pl;
-        float psum = 0.f;
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float p = expf(s[kb][i] - m_new);
-                psum += p;
-                __bf16 hi, lo;
-                la_split(p, hi, lo);
-                ph[4 * kb + i] = hi;
-                pl[4 * kb + i] = lo;
-            }
-        l = l * corr + psum;
-        m = m_new;
-        // (rescaled every time: a branch around this, for chunks that leave the maximum as it is, made the
-        //  compiler spill the sums)
-#pragma unroll
-        for (int db = 0; db < RB; ++db)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc[db][i] *= corr;
-        __syncthreads();
-#pragma unroll
-        for (int db = 0; db < RB; ++db)
-            if (db < rblocks) {
-                const __bf16* vr = Vt + (db * 16 + n) * LA_VT_STRIDE + 4 * g;
-                const uint2 v0 = *(const uint2*)vr, v1 = *(const uint2*)(vr + 16);
-                const la_bf16x8 vv = __builtin_bit_cast(la_bf16x8, uint4{v0.x, v0.y, v1.x, v1.y});
-                acc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv, ph, acc[db], 0, 0, 0);
-                acc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv, pl, acc[db], 0, 0, 0);
-                if (db % 8 == 7) __builtin_amdgcn_sched_barrier(0);      // (no more than eight blocks' reads in flight)
-            }
-        __syncthreads();
+        l += __shfl_xor(l, 16, HB_WAVE);
+        l += __shfl_xor(l, 32, HB_WAVE);
     }
-    l += __shfl_xor(l, 16, HB_WAVE);
-    l += __shfl_xor(l, 32, HB_WAVE);
     if (!head) return;
-    // acc[db][i]: number 16 db + 4 g + i of head n's sum
+    // acc[db][i]: number 32 v_first + 16 db + 4 g + i of head n's sum
     const size_t row = (size_t)t * H + h;
+    const int first = 32 * v_first + 4 * g;
     if (splits == 1) {
         if (sinks) l += expf(sinks[h] - m);                 // (an infinite share, a sink far above every score, leaves 0)
         float w = l > 0.f ? 1.0f / l : 0.f;
         if (gate) w *= 1.0f / (1.0f + expf(-gate[(size_t)t * gate_ld + h]));
 #pragma unroll
         for (int db = 0; db < RB; ++db)
-            if (db < rblocks) {
+            if (db < 2 * v_mine) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) out[row * rank + db * 16 + 4 * g + i] = hb_from_float<bf16>(acc[db][i] * w);
+                for (int i = 0; i < 4; ++i) out[row * rank + first + db * 16 + i] = hb_from_float<bf16>(acc[db][i] * w);
             }
     } else {
-        float* pa = part_acc + (row * splits + split) * rank;
+        float* pa = part_acc + (row * splits + split) * rank + first;
 #pragma unroll
         for (int db = 0; db < RB; ++db)
-            if (db < rblocks) *(la_f32x4*)(pa + db * 16 + 4 * g) = acc[db];
-        if (g == 0) {
+            if (db < 2 * v_mine) *(la_f32x4*)(pa + db * 16) = acc[db];
+        if (wave == 0 && g == 0) {
             part_ml[(row * splits + split) * 2] = m;
             part_ml[(row * splits + split) * 2 + 1] = l;
         }
@@ -1120,13 +1140,14 @@ extern "C" int hb_latent_attention_mfma(const float* q_full, const void* pages, 
         return 0;
     }
     const dim3 grid((unsigned)blocks, splits);
-#define LA_LAUNCH(RBV, KSV)                                                                                      \
-    latent_attention_mfma_kernel<RBV, KSV><<<grid, HB_WAVE, 0, stream>>>(                                          \
+#define LA_LAUNCH(VWV, KXV)                                                                                      \
+    latent_attention_mfma_kernel<VWV, KXV><<<grid, LA_WAVES * HB_WAVE, 0, stream>>>(                               \
         q_full, (const bf16*)pages, (bf16*)out, part_acc, part_ml, gate, gate_ld, positions, seq_of, slots,      \
         page_table, max_pages, page_size, H, rank, rot, scale, splits, chunks_per_split, sinks)
-    if (rank <= 128 && rank + rot <= 256) LA_LAUNCH(8, 8);
-    else if (rank <= 256 && rank + rot <= 384) LA_LAUNCH(16, 12);
-    else LA_LAUNCH(32, 20);
+    if (rot > 128) LA_LAUNCH(4, 5);
+    else if (rank <= 128) LA_LAUNCH(1, 1);
+    else if (rank <= 256) LA_LAUNCH(2, 1);
+    else LA_LAUNCH(4, 1);
 #undef LA_LAUNCH
     HB_CHECK_LAUNCH("latent_attention_mfma");
     if (splits > 1) {

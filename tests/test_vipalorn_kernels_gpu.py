@@ -302,6 +302,40 @@ def test_prompt_tokens_share_their_keys(H, rank, rot):
             assert not again[late:150].view(10, H, rank)[:, :, 7:9].isfinite().any()
 
 
+@pytest.mark.parametrize("ranges", [1, 1024])
+@pytest.mark.parametrize("H,rank,rot", [(16, 512, 64), (5, 512, 128), (3, 480, 0), (17, 160, 96), (8, 32, 0), (20, 288, 32), (16, 128, 128)])
+def test_a_token_a_sequence_by_waves_that_share_a_row(H, rank, rot, ranges, monkeypatch):
+    """The latent attention of one token a sequence, whose four waves take a quarter of a row's numbers each: latents and rotated parts
+    that no four waves share evenly, one chunk of keys and several at their edges, one range and as many as there are chunks, a sink and a
+    gate, against float64; the tolerance of the prompts' kernel."""
+    row, held = rank + rot, [1, 31, 32, 33, 64, 150, 330]
+    monkeypatch.setattr(latent, "TARGET_WAVES", ranges)
+    cache = Cache({0: KVNeed(1, row, None, values=False)}, 64 * 24, 4096, torch.bfloat16, DEV, max_slots=len(held))
+    kv = cache.kv_view(0)
+    slots = [cache.alloc_slot() for _ in held]
+    for s, n in zip(slots, held):
+        if n > 1:
+            step_meta(cache, [s], [n - 1])
+    meta = step_meta(cache, slots, [1] * len(held))
+    kv.k.zero_()
+    rows = [rand(n, row, seed=i).to(torch.bfloat16) for i, n in enumerate(held)]
+    for s, r in zip(slots, rows):
+        table = kv.page_table[s].cpu().tolist()
+        for p in range(0, r.shape[0], 64):
+            kv.k[table[p // 64], 0, :min(64, r.shape[0] - p)] = r[p:p + 64].to(DEV)
+    q, gate, sinks = rand(len(held), H * row, seed=9), rand(len(held), H, seed=10), rand(H, seed=11)
+    out = torch.empty(len(held), H * rank, dtype=torch.bfloat16, device=DEV)
+    latent.latent_attention_mfma(q.to(DEV), meta, kv, out, gate.to(DEV), 0, H, rank, rot, row ** -0.5,
+                                 lambda name, shape, dt: torch.empty(shape, dtype=dt, device=DEV), sinks=sinks.to(DEV))
+    for t, r in enumerate(rows):
+        keys = r.double()
+        score = q[t].view(H, row).double() @ keys.T * row ** -0.5
+        w = torch.softmax(torch.cat([score, sinks.double()[:, None]], 1), -1)[:, :-1]
+        want = (w @ keys[:, :rank]) * torch.sigmoid(gate[t].double())[:, None]
+        err = (out[t].cpu().double().view(H, rank) - want).abs().max()
+        assert float(err) <= 2.0 ** -8 * float(want.abs().max()) + 1e-3, held[t]
+
+
 @pytest.mark.parametrize("M", [1, 16, 17, 64, 65, 200, 700])
 @pytest.mark.parametrize("G,N,K,pad", [(1, 16, 32, 0), (5, 48, 160, 0), (3, 272, 64, 4), (4, 512, 96, 3)])
 def test_grouped_products_of_any_rows(M, G, N, K, pad):
