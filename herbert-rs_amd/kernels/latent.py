@@ -98,12 +98,18 @@ def latent_attention_plain(q_full, meta, cache, out, gate, gate_off, H, rank, ro
 
 
 CHUNK = 32
-TARGET_WAVES = 1024        # a decode step's keys are cut into ranges until about this many waves run
+# A decode step's keys are cut into ranges until about so many workgroups of four waves run, one a CU, and into twice as many where a
+# range would have more than RANGE_CHUNKS chunks: every range leaves sums that another kernel reads. With 256 / 512 / 1,024 of them, 16 heads of
+# 512 + 64, us: 8 tokens at 2,000 keys (2 chunks a range) 19 / 25 / 25, 16 at 1,000 (2) 17 / 23 / 23, 32 at 1,000 (4) 20.5 / 21.7 / 31, 64 at 2,000 (16)
+# 44 / 36 / 47, 48 at 300 (2) 19.6 / 18.2 / 21.9; 32 heads, 32 at 4,000 (32) 78 / 55 / 66.
+TARGET_WAVES = 256
+RANGE_CHUNKS = 4
 
 
 # Steps of several tokens a sequence take the kernel whose workgroups share their keys from contexts beyond this on: two
-# chunks of 32 keys leave it nothing to share (8 prompts of 64 tokens: 24 us, a wave a token's heads 23; of 20 tokens 32 and
-# 26), at 100 tokens it takes 40 us against 51.
+# chunks of 32 keys leave it nothing to share (8 prompts of 64 tokens 34 us, four waves a token 19; of 100 tokens 42 and 37, of 200 87 and 79, of 300
+# 128 and 128). The line lies below where the times meet because only that kernel keeps a later token's number that is not finite out of the
+# tokens before it.
 PROMPT_FROM = 64
 
 
@@ -298,6 +304,8 @@ def latent_attention_mfma(q_full, meta, cache, out, gate, gate_off, H, rank, rot
         chunks = -(-max(meta.context_bucket if part is None else 0, context) // CHUNK)
         blocks = rows * ((H + 15) // 16)
         splits = max(1, min(TARGET_WAVES // blocks, chunks, 64))
+        if -(-chunks // splits) > RANGE_CHUNKS:
+            splits = max(1, min(2 * TARGET_WAVES // blocks, chunks, 64))
         per = -(-chunks // splits)
     part_acc = part_ml = None
     if splits > 1:
