@@ -180,8 +180,9 @@ FEW_ROWS = 16
 # From so many rows an expert on the kernel of tall tiles takes gate/up. Microseconds by tiles of 64 / of 128 (weights from memory): 32
 # experts of 768 on 2,048: 32 rows an expert 58 / 48, 50 rows 59 / 48, 64 rows 57 / 47, 96 rows 63 / 50; 64 of 1,536 on 4,096: 62 rows
 # 363 / 310; where fewer than half the CUs get a tile (16 of 512 on 1,024: 64 rows 24 / 23) nothing is gained.
-# Down, whose k is short, takes tall tiles from DOWN_STEPS steps of 64 k and DOWN_ROWS rows on where down_tall expects them to be done sooner.
-DOWN_STEPS, DOWN_ROWS = 12, 128
+# Down, whose k is short, takes tall tiles from DOWN_ROWS rows and DOWN_STEPS steps of 64 k on, below DOWN_ALWAYS steps only where down_tall
+# expects them to be done sooner.
+DOWN_STEPS, DOWN_ALWAYS, DOWN_ROWS = 12, 16, 128
 TALL_ROWS = 48
 
 
@@ -228,14 +229,18 @@ def tall_rows(T, top, routed, experts, hidden, inter, shared=False):
 
 @functools.lru_cache(maxsize=1024)
 def down_tall(T, top, routed, experts, hidden, inter, shared, height):
-    """True if the down product of a layer whose gate/up takes tall tiles of `height` rows takes them too: where its rounds of tiles over the
-    CUs are expected to be done before the low tiles', two to a CU. A round of `steps` steps of 64 k takes height / 122 us a step and 8
-    beside them, one of low tiles 1.75 and 3. Microseconds by low / tall tiles, 32 experts of 768 on 2,048, four each: 2,048 tokens 69 / 62
-    (128 rows), with a shared expert 70 / 81 (192, the low ones here), 1,712 tokens 51 / 44 (256), 4,000 tokens 108 / 98 (256); 64 of 1,536 on
-    4,096: 2,500 tokens 271 / 237 (192)."""
+    """True if the down product of a layer whose gate/up takes tall tiles of `height` rows takes them too: from DOWN_ALWAYS steps of 64 k on,
+    and from DOWN_STEPS on where its rounds of tiles over the CUs are expected to be done before the low tiles', two to a CU. A round of
+    `steps` steps takes height / 122 us a step and 8 beside them, one of low tiles 1.75 and 3. Microseconds by low / tall tiles, 32 experts
+    of 768 on 2,048, four each: 2,048 tokens 70 / 63 (128 rows), with a shared expert 71 / 80 (192, the low ones here), 1,712 tokens 51 / 44
+    (256); from 16 steps on: 64 of 1,536 on 4,096, 2,500 tokens 267 / 235 (192), 16 of 2,048 on 2,048, two each, 3,000 tokens 98 / 91 (192). There the
+    estimate, which adds a round for experts busier than the mean, would be wrong where that round does not come: 64 of 1,408 on 2,048, six
+    each, 1,400 tokens 123 / 107 (192), 8 of 3,584 on 4,096, two each, 700 tokens 86 / 81 (256)."""
     steps, rows = inter // 64, T * top / routed
     if not height or steps < DOWN_STEPS or rows < DOWN_ROWS:
         return False
+    if steps >= DOWN_ALWAYS:
+        return True
     columns = -(-hidden // 256)
 
     def rounds(tile, at_once):

@@ -128,6 +128,13 @@ def test_tiles_of_the_down_product():
     assert moe.down_tall(2500, 4, 64, 64, 4096, 1536, False, 192) and not moe.down_tall(1500, 4, 64, 64, 4096, 1536, False, 128)
 
 
+def test_down_products_of_16_steps_and_more_take_the_tall_tiles():
+    """From 128 rows an expert on whatever the rounds, which the estimate counts too high where experts are about as busy as the mean."""
+    assert moe.down_tall(1400, 6, 64, 64, 2048, 1408, False, 192) and moe.down_tall(700, 2, 8, 8, 4096, 3584, False, 256)
+    assert moe.down_tall(1400, 6, 64, 64, 2048, 1024, False, 192) and not moe.down_tall(1400, 6, 64, 64, 2048, 960, False, 192)
+    assert not moe.down_tall(1300, 6, 64, 64, 2048, 1408, False, 192) and not moe.down_tall(1400, 6, 64, 64, 2048, 1408, False, 0)
+
+
 def test_a_shared_expert_is_folded_only_where_that_pays():
     """Both sides of the lines: always beyond the steps of few rows an expert, in them while its rows are few tiles of matrices
     that are small enough to be read again."""
