@@ -1487,13 +1487,13 @@ static int launch_tile32(const void* X, const void* W, void* C, int M, int N, in
 // tiles costs beside its steps (us).
 // (168: three quarters of the 256 x 256 tile's arithmetic a step, for the SwiGLU product whole: where that
 // one's tiles fill the last round of 256 badly, 192 columns often fill it)
-// (186: 224, 192 or 160 rows high, whichever is done sooner, for row counts whose tiles of 256 rows leave CUs empty and whose
+// (187, 186, 185: 224, 192 and 160 rows high, for row counts whose tiles of 256 rows leave CUs empty and whose
 // tiles of 128 rows need another round; the heights beside 192: 9,404 rows x 2,048 columns (K 6144, add) 212 us on
 // 192, 197 on 160; 2,600 x 24576 x 4096 (gated) 441 on tile 168, 398 on 224)
 // (cut_us: a step's time as split_rows has it, 0 for tiles that it leaves out)
 struct Mid { int id, bn, bm, per_cu; double step_us, round_us, cut_us; };
-static const Mid mid_tiles[] = {{188, 256, 256, 1, 1.21, 4.8, 1.26}, {186, 256, 224, 1, 1.09, 7.7, 0}, {186, 256, 192, 1, 1.01, 5.3, 1.08},
-                                {186, 256, 160, 1, 0.91, 5.9, 0}, {142, 256, 128, 1, 0.77, 4.8, 0.77}, {122, 128, 128, 2, 0.73, 3.1, 0.95},
+static const Mid mid_tiles[] = {{188, 256, 256, 1, 1.21, 4.8, 1.26}, {187, 256, 224, 1, 1.09, 7.7, 0}, {186, 256, 192, 1, 1.01, 5.3, 1.08},
+                                {185, 256, 160, 1, 0.91, 5.9, 0}, {142, 256, 128, 1, 0.77, 4.8, 0.77}, {122, 128, 128, 2, 0.73, 3.1, 0.95},
                                 {124, 128, 64, 2, 0.40, 4.4, 0.48}, {184, 256, 64, 1, 0.72, 3.1, 0.67}, {168, 192, 256, 1, 0.93, 5.3, 1.0}};
 // the rounds of a product's tiles, one after the other
 static double mid_stepping(const Mid& v, int M, int N, int K, int slices, bool cutting = false) {
@@ -1503,20 +1503,29 @@ static double mid_stepping(const Mid& v, int M, int N, int K, int slices, bool c
     if (cutting) return (double)rounds * per * v.cut_us * (1 + 1.06 * (on_a_cu - 1));
     return (double)rounds * (per * v.step_us * (1 + 0.54 * (on_a_cu - 1)) + v.round_us);
 }
-// The rows of the tiles of 256 columns, from 160 to `tallest`, with which a product's rounds are done soonest.
-static int tall_rows(int M, int N, int K, int slices, int tallest) {
+// What a product's tiles take, without what adds its slices up: the slowest of its rounds, of what all workgroups move out of the
+// L2s (16 TB/s) and of what comes from HBM once (6.5 TB/s).
+static double mid_time(const Mid& v, int M, int N, int K, int slices, bool cutting = false) {
+    const long wgs = (long)((M + v.bm - 1) / v.bm) * ((N + v.bn - 1) / v.bn) * slices;
+    const double stepping = mid_stepping(v, M, N, K, slices, cutting);
+    const double moving = (double)wgs * ((K / 64 + slices - 1) / slices) * (v.bn + v.bm) * 128 / 16.3e6;
+    const double fetching = ((double)N + M) * K * 2 / (cutting ? 7.1e6 : 6.5e6);
+    const double slower = stepping > moving ? stepping : moving;
+    return fetching > slower ? fetching : slower;
+}
+
+// The tile of the fused q/k/v product of shape 0: 256 columns and the height with which it is expected to be done soonest.
+extern "C" int hb_gemm_qkv_tile(int M, int N, int K) {
     const Mid* best = nullptr;
     for (const Mid& v : mid_tiles)
-        if ((v.id == 186 || v.id == 188) && v.bm <= tallest &&
-            (!best || mid_stepping(v, M, N, K, slices) < mid_stepping(*best, M, N, K, slices)))
-            best = &v;
-    return best->bm;
+        if (v.id >= 185 && v.id <= 188 && (!best || mid_time(v, M, N, K, 1) < mid_time(*best, M, N, K, 1))) best = &v;
+    return best->id;
 }
 
 // The q/k/v projection of a step with many rows, fused with norm, rotation and cache write
 // (see QkvEpilogue). X [M, K] bf16; W [(nq + 2 nkv) 128, K] bf16, rows q | k | v. A wave's tile is
 // one head wide; shape: 0 = tiles of 256 columns (waves 2 x 2, for long prompts), 160 to 256 rows high, whichever are done
-// soonest, 1 = a head wide and 256 rows high (four waves one above the other, 64 rows each), 2 = a head
+// soonest (hb_gemm_qkv_tile; 185 to 188: the tile of that number), 1 = a head wide and 256 rows high (four waves one above the other, 64 rows each), 2 = a head
 // wide and 128 rows high (32 rows a wave): more and smaller tiles for prompts whose 256 x 256 tiles would not fill the CUs.
 template <int TN, int TM, int WNW, int WMW, int WST, int XST>
 static int launch_qkv(const bf16* x, const bf16* w, int M, int N, int K, int packed, const QkvEpilogue& e,
@@ -1540,21 +1549,20 @@ extern "C" int hb_gemm_qkv_mfma(const void* X, const void* W, int M, int K, int 
     HB_REQUIRE(hd == 128 && page_size == 64, "gemm_qkv: heads of 128 and pages of 64 tokens only");
     HB_REQUIRE(M > 0 && nq > 0 && nkv > 0 && K > 0 && K % 64 == 0, "gemm_qkv: bad sizes (M=%d, K=%d)", M, K);
     HB_REQUIRE((cos_t == nullptr) == (sin_t == nullptr), "gemm_qkv: cos and sin tables come together");
-    HB_REQUIRE(shape >= 0 && shape <= 2, "gemm_qkv: unknown tile shape %d", shape);
+    HB_REQUIRE((shape >= 0 && shape <= 2) || (shape >= 185 && shape <= 188), "gemm_qkv: unknown tile shape %d", shape);
     const int N = (nq + 2 * nkv) * 128;
     const QkvEpilogue e = {(bf16*)q_out, (bf16*)k_cache, (bf16*)v_cache, positions, seq_of, slots, page_table,
                            max_pages, q_norm_w, k_norm_w, cos_t, sin_t, eps, nq, nkv};
     const bf16* x = (const bf16*)X;
     const bf16* w = (const bf16*)W;
-    if (shape == 0) {
-        const int rows = tall_rows(M, N, K, 1, 256);
-        if (rows == 256) return launch_qkv<8, 8, 2, 2, 3, 2>(x, w, M, N, K, packed, e, stream);
-        if (rows == 224) return launch_qkv<8, 7, 2, 2, 3, 2>(x, w, M, N, K, packed, e, stream);
-        if (rows == 192) return launch_qkv<8, 6, 2, 2, 3, 2>(x, w, M, N, K, packed, e, stream);
-        return launch_qkv<8, 5, 2, 2, 3, 3>(x, w, M, N, K, packed, e, stream);
+    switch (shape == 0 ? hb_gemm_qkv_tile(M, N, K) : shape) {
+        case 188: return launch_qkv<8, 8, 2, 2, 3, 2>(x, w, M, N, K, packed, e, stream);
+        case 187: return launch_qkv<8, 7, 2, 2, 3, 2>(x, w, M, N, K, packed, e, stream);
+        case 186: return launch_qkv<8, 6, 2, 2, 3, 2>(x, w, M, N, K, packed, e, stream);
+        case 185: return launch_qkv<8, 5, 2, 2, 3, 3>(x, w, M, N, K, packed, e, stream);
+        case 1: return launch_qkv<8, 4, 1, 4, 3, 2>(x, w, M, N, K, packed, e, stream);
+        default: return launch_qkv<8, 2, 1, 4, 3, 2>(x, w, M, N, K, packed, e, stream);
     }
-    if (shape == 1) return launch_qkv<8, 4, 1, 4, 3, 2>(x, w, M, N, K, packed, e, stream);
-    return launch_qkv<8, 2, 1, 4, 3, 2>(x, w, M, N, K, packed, e, stream);
 }
 
 // Which kernel a product runs on: tile 0 = the few-row kernel, otherwise a tile variant by number and
@@ -1658,17 +1666,12 @@ static GemmPlan plan_gemm(int M, int N, int K, int ldc, int epi, bool norm_w, bo
         double best = -1;
         for (const Mid& v : mid_tiles) {
             if ((v.id == 168 && epi != EPI_SWIGLU) || (cutting && v.cut_us == 0)) continue;
-            const long tiles = (long)((M + v.bm - 1) / v.bm) * ((N + v.bn - 1) / v.bn);
             for (int sl = 1; sl <= 16; sl *= 2) {
                 if (v.id == 168 && sl > 1) break;
                 if (sl > 1 && !slices_fit(steps, sl)) break;
                 if (emit_g && (sl == 1 || !reducer_norms)) continue;      // the kernel that adds the slices up norms
                 if (deferred && sl > 8) break;                            // whoever adds the slices up takes 2, 4 or 8
-                const double stepping = mid_stepping(v, M, N, K, sl, cutting);
-                const double moving = (double)(tiles * sl) * ((steps + sl - 1) / sl) * (v.bn + v.bm) * 128 / 16.3e6;
-                const double fetching = ((double)N + M) * K * 2 / (cutting ? 7.1e6 : 6.5e6);
-                double cost = stepping > moving ? stepping : moving;
-                if (fetching > cost) cost = fetching;
+                double cost = mid_time(v, M, N, K, sl, cutting);
                 if (cutting) cost += 2.3;
                 if (sl > 1) cost += deferred ? (double)sl * M * N * 4 / 2.5e6 : 1.3 + (double)(sl + 1) * M * N * 4 / 2.5e6;
                 if (best < 0 || cost < best) {
@@ -1720,12 +1723,22 @@ extern "C" int hb_gemm_mfma_split(int M, int N, int K, int epi, size_t workspace
 
 // The plan as a number for tests and measurements: tile + 1000 x slices (slices > 1), 0 for the
 // few-row kernel, -1 if the product is refused. emit: 0 none, 1 a norm is left behind. deferred:
-// the slices are left for the next kernel to add up.
+// the slices are left for the next kernel to add up. 186 stands for all three heights between 128 and 256 rows, which
+// hb_gemm_mfma_plan_rows tells apart.
 extern "C" int hb_gemm_mfma_plan(int M, int N, int K, int epi, int normed_input, int emit, int scaled,
                                  size_t workspace_floats, int deferred) {
     const GemmPlan p = plan_gemm(M, N, K, epi == EPI_SWIGLU ? N / 2 : N, epi, normed_input != 0, emit != 0, scaled != 0, 0,
                                  workspace_floats, deferred != 0);
-    return p.tile <= 0 ? p.tile : p.tile + (p.slices > 1 ? 1000 * p.slices : 0);
+    if (p.tile <= 0) return p.tile;
+    return (p.tile == 185 || p.tile == 187 ? 186 : p.tile) + (p.slices > 1 ? 1000 * p.slices : 0);
+}
+
+// The rows of the tiles that a plain product of more than 64 rows is planned on, or 0 where it runs on no such tile.
+extern "C" int hb_gemm_mfma_plan_rows(int M, int N, int K, int epi, size_t workspace_floats) {
+    const GemmPlan p = plan_gemm(M, N, K, epi == EPI_SWIGLU ? N / 2 : N, epi, false, false, false, 0, workspace_floats);
+    for (const Mid& v : mid_tiles)
+        if (M > 64 && v.id == p.tile) return v.bm;
+    return 0;
 }
 
 // The estimated time in us of the plan that hb_gemm_mfma_plan gives, or a negative number where the
@@ -1807,13 +1820,9 @@ extern "C" int hb_gemm_mfma(const void* X, const void* W, void* C, int M, int N,
         // room for one: 8192 x 8192 x 8192 on 256 x 256 tiles 792 us, with the activations' third stage instead 838)
         case 188: rc = launch_tile64<8, 8, 2, 2, 3, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 256 x 256
         case 142: rc = launch_tile64<8, 4, 2, 2, 3, 3>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 256 (n) x 128 (m)
-        case 186: {                                                                                                          // 256 (n) x 160, 192 or 224 (m)
-            const int rows = tall_rows(M, N, K, slices, 224);
-            if (rows == 224) rc = launch_tile64<8, 7, 2, 2, 3, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale);
-            else if (rows == 192) rc = launch_tile64<8, 6, 2, 2, 3, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale);
-            else rc = launch_tile64<8, 5, 2, 2, 3, 3>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale);
-            break;
-        }
+        case 187: rc = launch_tile64<8, 7, 2, 2, 3, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 256 (n) x 224 (m)
+        case 186: rc = launch_tile64<8, 6, 2, 2, 3, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 256 (n) x 192 (m)
+        case 185: rc = launch_tile64<8, 5, 2, 2, 3, 3>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 256 (n) x 160 (m)
         case 122: rc = launch_tile64<4, 4, 2, 2, 2, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 128 x 128, two to a CU
         case 124: rc = launch_tile64<2, 4, 4, 1, 3, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 128 (n) x 64 (m)
         case 112: rc = launch_tile64<2, 2, 4, 1, 3, 2>(X, W, C, M, N, K, ldc, epi, packed, stream, slices, workspace, row_scale); break;   // 128 (n) x 32 (m)

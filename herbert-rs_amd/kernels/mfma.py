@@ -27,7 +27,9 @@ lib.register_signatures("gemm_mfma", {
     "hb_gemm_mfma_join": [_P, _P, _P, _I, _I, _I, _I, _F, _P, _P, _P, _P, _F, _P, _P, _P, _P],
     "hb_gemm_mfma_plan": [_I, _I, _I, _I, _I, _I, _I, ctypes.c_size_t, _I],
     "hb_gemm_mfma_plan_cost": [_I, _I, _I, _I, _I, _I, _I, ctypes.c_size_t, _I],
+    "hb_gemm_mfma_plan_rows": [_I, _I, _I, _I, ctypes.c_size_t],
     "hb_gemm_mfma_split": [_I, _I, _I, _I, ctypes.c_size_t],
+    "hb_gemm_qkv_tile": [_I, _I, _I],
     "hb_gemm_qkv_mfma": [_P, _P, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _P, _P, _P, _P, _F, _I, _I, _I, _I, _P],
 })
 

@@ -195,3 +195,25 @@ def test_decode_attention_takes_a_list_of_ranges_only_where_it_fits():
     assert mfma._decode_ranges(meta_of(half[8:72]), 8, 0)[0] == 128
     prompt = pack([StepEntry(0, [1, 2, 3], [2]), StepEntry(1, [4], [0])], [9000, 10], torch.device("cpu"))
     assert prompt.unequal and mfma._decode_ranges(prompt, 8, 0) is None     # not one token a sequence
+
+
+def test_a_plan_names_the_height_of_its_tiles(plan):
+    """What is launched is the plan's own tile, heights between 128 and 256 rows among them: every plan of more than 64 rows has the
+    height of its number, 186 one of three, each of which some product takes; and the q/k/v product that writes the cache."""
+    rows_of = lib.load("gemm_mfma").hb_gemm_mfma_plan_rows
+    taken = set()
+    for M, N, K in itertools.product([64, 65, 200, 700, 1500, 2048, 2600, 3072, 5000, 9404], WIDTHS, [512, 2048, 4096, 12288]):
+        for epi in (EPI_STORE, EPI_ADD, EPI_SWIGLU):
+            rows, tile = rows_of(M, N, K, epi, 1 << 24), plan(M, N, K, epi) % 1000
+            if M <= 64:
+                assert rows == 0
+            elif tile == 186:
+                assert rows in (160, 192, 224), (M, N, K, epi)
+                taken.add(rows)
+            else:
+                assert rows == TILES[tile][1], (M, N, K, epi)
+    assert taken == {160, 192, 224}
+    assert rows_of(300, 4096, 4096 + 32, EPI_STORE, 1 << 24) == 0          # K in steps of 32: a kernel of its own
+    qkv = lib.load("gemm_mfma").hb_gemm_qkv_tile
+    assert qkv(2048, 6144, 4096) == 187 and qkv(8192, 6144, 4096) == 188
+    assert {qkv(m, n, 2048) for m in range(1500, 9500, 100) for n in (4096, 6144)} == {185, 186, 187, 188}

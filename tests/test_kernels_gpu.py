@@ -779,30 +779,31 @@ def test_qk_norm_rope_write(nq, nkv, hd, rot, norm, dtype):
         assert float((kv.v.double().cpu() - exp_v).abs().max()) <= tol * float(exp_v.abs().max())
 
 
-@pytest.mark.parametrize("M", [10001, 12001, 14001, 16001])
-def test_tiles_of_256_columns_are_160_to_256_rows_high(M):
-    """1,024 columns and so many rows that one round of tiles 160, 192, 224 or 256 rows high takes them and the next lower one
-    does not: the tiles between 128 and 256 rows by name (up to 224), and the q/k/v product that norms, rotates and writes
-    the cache, against the product and the kernel of its own. The last tile of either ends inside."""
+@pytest.mark.parametrize("tile", [185, 186, 187, 188])
+@pytest.mark.parametrize("M,K", [(481, 64), (700, 320), (1025, 128)])
+def test_tiles_of_256_columns_are_160_to_256_rows_high(tile, M, K):
+    """The tiles of 256 columns by name, 160 (185), 192, 224 and 256 rows high: the product and the q/k/v product that norms, rotates
+    and writes the cache, against float64 and the kernel of its own. The last tile of each ends inside, and a step, two and
+    five of K go through rings of two and three stages."""
     from herbert_rs_amd.cache.paged import LayerKV
     from herbert_rs_amd.kernels import mfma, ops
-    nq, nkv, hd, K, N = 4, 2, 128, 128, 1024
+    nq, nkv, hd, N = 4, 2, 128, 1024
     a = rand(M, K, seed=81, dtype=torch.bfloat16)
     w = rand(N, K, seed=82, dtype=torch.bfloat16, scale=0.1)
     wp = mfma.pack_weight(w)
     want = (a.double() @ w.double().T).float()
     tol = 2e-6 * K ** 0.5 * float(want.abs().max()) + 1e-4          # float32 sums of K products in another order
     c = torch.full((M + 1, N), 7.0, device=dev())
-    mfma.gemm(a, wp, c[:M], packed=True, tile=186)
+    mfma.gemm(a, wp, c[:M], packed=True, tile=tile)
     assert float((c[:M] - want).abs().max()) <= tol and bool((c[M] == 7.0).all())
-    mfma.gemm(a, wp, c[:M], accumulate=True, packed=True, tile=186)
+    mfma.gemm(a, wp, c[:M], accumulate=True, packed=True, tile=tile)
     assert float((c[:M] - 2 * want).abs().max()) <= 2 * tol and bool((c[M] == 7.0).all())
     half = torch.full((M + 1, N // 2), 3.0, dtype=torch.bfloat16, device=dev())
-    mfma.gemm_swiglu(a, mfma.pack_weight(mfma.interleave_gate_up(w[:N // 2].contiguous(), w[N // 2:].contiguous())), half[:M], True, tile=186)
+    mfma.gemm_swiglu(a, mfma.pack_weight(mfma.interleave_gate_up(w[:N // 2].contiguous(), w[N // 2:].contiguous())), half[:M], True, tile=tile)
     unit = torch.nn.functional.silu(want[:, :N // 2]) * want[:, N // 2:]
     assert bool(((half[:M].float() - unit).abs() <= 2 ** -8 * unit.abs() + 2 * tol * (1 + want[:, :N // 2].abs() + want[:, N // 2:].abs())).all())
     assert bool((half[M] == 3.0).all())
-    meta, kv, _ = paged_case([M], [M], nkv, hd, torch.bfloat16, seed=3, n_pages=256)
+    meta, kv, _ = paged_case([M], [M], nkv, hd, torch.bfloat16, seed=3)
     kv2 = LayerKV(kv.k.clone(), kv.v.clone(), kv.page_table, 64, 0)
     ang = torch.arange(M + 1, dtype=torch.float32)[:, None] * (10000.0 ** (-torch.arange(hd // 2) / (hd // 2)))[None]
     cos, sin = ang.cos().to(dev()).contiguous(), ang.sin().to(dev()).contiguous()
@@ -811,7 +812,7 @@ def test_tiles_of_256_columns_are_160_to_256_rows_high(M):
     want_q = torch.empty(M, nq * hd, dtype=torch.bfloat16, device=dev())
     ops.qk_norm_rope_write(qkv, qw, kw, cos, sin, hd, meta, kv, want_q, nq, nkv, hd, 1e-5)
     got_q = torch.empty_like(want_q)
-    mfma.gemm_qkv(a, wp, True, qw, kw, cos, sin, meta, kv2, got_q, nq, nkv, hd, 1e-5, shape=0)
+    mfma.gemm_qkv(a, wp, True, qw, kw, cos, sin, meta, kv2, got_q, nq, nkv, hd, 1e-5, shape=tile)
     # the two paths add the squares and the products in other orders: an element may round the other way
     for got, wanted in ((got_q, want_q), (kv2.k, kv.k), (kv2.v, kv.v)):
         d = (got.float() - wanted.float()).abs()
