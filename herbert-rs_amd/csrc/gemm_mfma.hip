@@ -1483,33 +1483,26 @@ static int launch_tile32(const void* X, const void* W, void* C, int M, int N, in
 }
 #undef TILE_DISPATCH
 
-// The tiles of products of more than 64 rows: number, columns, rows, workgroups on a CU, a step's time and what a round of
-// tiles costs beside its steps (us).
+// The tiles of products of more than 64 rows: number, columns, rows, workgroups on a CU, a step's time, what a second
+// workgroup on the CU adds to it (a share) and what a round of tiles costs beside its steps (us).
 // (168: three quarters of the 256 x 256 tile's arithmetic a step, for the SwiGLU product whole: where that
 // one's tiles fill the last round of 256 badly, 192 columns often fill it)
 // (187, 186, 185: 224, 192 and 160 rows high, for row counts whose tiles of 256 rows leave CUs empty and whose
 // tiles of 128 rows need another round; the heights beside 192: 9,404 rows x 2,048 columns (K 6144, add) 212 us on
 // 192, 197 on 160; 2,600 x 24576 x 4096 (gated) 441 on tile 168, 398 on 224)
-// (cut_us: a step's time as split_rows has it, 0 for tiles that it leaves out)
-struct Mid { int id, bn, bm, per_cu; double step_us, round_us, cut_us; };
-static const Mid mid_tiles[] = {{188, 256, 256, 1, 1.21, 4.8, 1.26}, {187, 256, 224, 1, 1.09, 7.7, 0}, {186, 256, 192, 1, 1.01, 5.3, 1.08},
-                                {185, 256, 160, 1, 0.91, 5.9, 0}, {142, 256, 128, 1, 0.77, 4.8, 0.77}, {122, 128, 128, 2, 0.73, 3.1, 0.95},
-                                {124, 128, 64, 2, 0.40, 4.4, 0.48}, {184, 256, 64, 1, 0.72, 3.1, 0.67}, {168, 192, 256, 1, 0.93, 5.3, 1.0}};
-// the rounds of a product's tiles, one after the other
-static double mid_stepping(const Mid& v, int M, int N, int K, int slices, bool cutting = false) {
+struct Mid { int id, bn, bm, per_cu; double step_us, second, round_us; };
+static const Mid mid_tiles[] = {{188, 256, 256, 1, 1.155, 0, 7.283}, {187, 256, 224, 1, 1.063, 0, 6.462}, {186, 256, 192, 1, 0.927, 0, 7.139},
+                                {185, 256, 160, 1, 0.881, 0, 6.813}, {142, 256, 128, 1, 0.714, 0, 5.56}, {122, 128, 128, 2, 0.861, 0.086, 3.357},
+                                {124, 128, 64, 2, 0.428, 0.584, 3.116}, {184, 256, 64, 1, 0.629, 0, 3.623}, {168, 192, 256, 1, 0.917, 0, 5.569}};
+// What a product's tiles take, without what adds its slices up: the slowest of its rounds one after the other, of what all
+// workgroups move out of the L2s (27 TB/s) and of what comes from HBM once (6.5 TB/s).
+static double mid_time(const Mid& v, int M, int N, int K, int slices) {
     const long wgs = (long)((M + v.bm - 1) / v.bm) * ((N + v.bn - 1) / v.bn) * slices, slots = 256 * v.per_cu;
     const long rounds = (wgs + slots - 1) / slots, on_a_cu = ((wgs < slots ? wgs : slots) + 255) / 256;
     const int per = (K / 64 + slices - 1) / slices;
-    if (cutting) return (double)rounds * per * v.cut_us * (1 + 1.06 * (on_a_cu - 1));
-    return (double)rounds * (per * v.step_us * (1 + 0.54 * (on_a_cu - 1)) + v.round_us);
-}
-// What a product's tiles take, without what adds its slices up: the slowest of its rounds, of what all workgroups move out of the
-// L2s (16 TB/s) and of what comes from HBM once (6.5 TB/s).
-static double mid_time(const Mid& v, int M, int N, int K, int slices, bool cutting = false) {
-    const long wgs = (long)((M + v.bm - 1) / v.bm) * ((N + v.bn - 1) / v.bn) * slices;
-    const double stepping = mid_stepping(v, M, N, K, slices, cutting);
-    const double moving = (double)wgs * ((K / 64 + slices - 1) / slices) * (v.bn + v.bm) * 128 / 16.3e6;
-    const double fetching = ((double)N + M) * K * 2 / (cutting ? 7.1e6 : 6.5e6);
+    const double stepping = (double)rounds * (per * v.step_us * (1 + v.second * (on_a_cu - 1)) + v.round_us);
+    const double moving = (double)wgs * per * (v.bn + v.bm) * 128 / 27.576e6;
+    const double fetching = ((double)N + M) * K * 2 / 6.507e6;
     const double slower = stepping > moving ? stepping : moving;
     return fetching > slower ? fetching : slower;
 }
@@ -1583,7 +1576,7 @@ static double few_rows_cost(int M, int N, int K, int epi) {
 
 struct GemmPlan { int tile, slices; double cost = -1; };      // cost: the estimated time in us where the plan was chosen by one
 static GemmPlan plan_gemm(int M, int N, int K, int ldc, int epi, bool norm_w, bool emit_g, bool scale_partial,
-                          int tile_hint, size_t workspace_floats, bool deferred = false, bool cutting = false) {
+                          int tile_hint, size_t workspace_floats, bool deferred = false) {
     int tile = tile_hint % 1000, slices = tile_hint >= 1000 ? tile_hint / 1000 : 1;
     double low_cost = -1, mid_cost = -1;
     if (tile_hint == 1) return M <= 16 ? GemmPlan{0, 1} : GemmPlan{-1, 0};      // the few-row kernel, asked for by name
@@ -1656,24 +1649,22 @@ static GemmPlan plan_gemm(int M, int N, int K, int ldc, int epi, bool norm_w, bo
     if (tile == 0 && K % 64) tile = 123;
     if (tile == 0 && K % 64 == 0) {
         // More than 64 rows: neither the arithmetic nor the weights alone decide. All tiles from 128 x 64
-        // to 256 x 256 with 1 to 16 K slices are candidates; a candidate takes as long as the slowest
-        // of: its rounds' steps one after another (a step's time alone on a CU, half as much again with two
-        // on a CU) and what a round costs beside them, what all workgroups move out of the L2s (16 TB/s),
-        // what comes from HBM once (6.5 TB/s); plus, for slices, the second kernel. Fitted to every tile's time
-        // at eleven products of four model sizes and 96 to 9,404 rows: the choice is then 0.8 % from the
-        // best candidate on average (2.0 % without a round's own cost and the two heights between), 25 % at worst.
+        // to 256 x 256 with 1 to 16 K slices are candidates, by mid_time and, for slices, the second kernel. Fitted to every
+        // candidate's time, weights from memory, at 16 products of four model sizes and 72 to 9,404 rows (520 sizes): the choice is
+        // 1.0 % from the best candidate on average and 21 % at worst; without a quarter of the sizes the fit is 1.3 % off on those.
+        // (One share for both tiles of two workgroups a CU had tile 124 displace 184: 128 rows of 24576 x 4096 51.4 us where 184 takes
+        // 47.0, of 4096 x 12288 35.3 and 34.0.)
         const int steps = K / 64;
         double best = -1;
         for (const Mid& v : mid_tiles) {
-            if ((v.id == 168 && epi != EPI_SWIGLU) || (cutting && v.cut_us == 0)) continue;
+            if (v.id == 168 && epi != EPI_SWIGLU) continue;
             for (int sl = 1; sl <= 16; sl *= 2) {
                 if (v.id == 168 && sl > 1) break;
                 if (sl > 1 && !slices_fit(steps, sl)) break;
                 if (emit_g && (sl == 1 || !reducer_norms)) continue;      // the kernel that adds the slices up norms
                 if (deferred && sl > 8) break;                            // whoever adds the slices up takes 2, 4 or 8
-                double cost = mid_time(v, M, N, K, sl, cutting);
-                if (cutting) cost += 2.3;
-                if (sl > 1) cost += deferred ? (double)sl * M * N * 4 / 2.5e6 : 1.3 + (double)(sl + 1) * M * N * 4 / 2.5e6;
+                double cost = mid_time(v, M, N, K, sl);
+                if (sl > 1) cost += deferred ? (double)sl * M * N * 4 / 3.312e6 : 3.993 + (double)(sl + 1) * M * N * 4 / 3.312e6;
                 if (best < 0 || cost < best) {
                     best = cost;
                     tile = v.id;
@@ -1689,25 +1680,25 @@ static GemmPlan plan_gemm(int M, int N, int K, int ldc, int epi, bool norm_w, bo
     return GemmPlan{tile, slices, mid_cost >= 0 ? mid_cost : low_cost};
 }
 
-// The rows of the first of two products that M rows are better cut into (see hb_gemm_mfma), or 0. Its estimates leave out the
-// heights of 224 and 160 rows and a round's own cost, with which its margin of a tenth was found; a cut that the
-// product's own estimates, which have them, put a tenth behind the whole product is not made.
+// The rows of the first of two products that M rows are better cut into (see hb_gemm_mfma), or 0: where both are expected to be done
+// sooner than the whole. Of 634 sizes (12 products, 130 to 6,200 rows, most a little past whole tiles) 68 are cut; the choice is
+// 0.35 % from the better one on average and 17 % at worst (never cut: 0.6 and 23).
 static int split_rows(int M, int N, int K, int ldc, int epi, bool special, int tile_hint, size_t workspace_floats,
                       const GemmPlan& whole) {
     if (special || M <= 128 || (tile_hint != 0 && tile_hint != -128 && tile_hint != -256)) return 0;
     int best_main = 0;
-    auto estimate = [&](int rows, bool cutting) { return plan_gemm(rows, N, K, ldc, epi, false, false, false, 0, workspace_floats, false, cutting); };
-    double best = whole.cost < 0 ? -1 : estimate(M, true).cost;
+    double best = 0.99 * whole.cost;
     for (int bm = 128; bm <= 256; bm *= 2) {
         const int main_rows = M / bm * bm, rest = M - main_rows;
         if (rest == 0 || main_rows == 0) continue;
-        const GemmPlan a = estimate(main_rows, true), b = estimate(rest, true);
+        const GemmPlan a = plan_gemm(main_rows, N, K, ldc, epi, false, false, false, 0, workspace_floats);
+        const GemmPlan b = plan_gemm(rest, N, K, ldc, epi, false, false, false, 0, workspace_floats);
         if (a.tile < 0 || b.tile < 0) continue;
         if (tile_hint == -bm) return main_rows;
         if (tile_hint != 0 || whole.cost < 0 || a.cost < 0 || b.cost < 0) continue;
-        // (a second launch and its start are in the estimates; a tenth is kept as a margin for their error)
-        if (a.cost + b.cost < 0.9 * best && estimate(main_rows, false).cost + estimate(rest, false).cost < 1.1 * whole.cost) {
-            best = (a.cost + b.cost) / 0.9;
+        // (a second launch and its start are in the estimates)
+        if (a.cost + b.cost < best) {
+            best = a.cost + b.cost;
             best_main = main_rows;
         }
     }

@@ -217,3 +217,31 @@ def test_a_plan_names_the_height_of_its_tiles(plan):
     qkv = lib.load("gemm_mfma").hb_gemm_qkv_tile
     assert qkv(2048, 6144, 4096) == 187 and qkv(8192, 6144, 4096) == 188
     assert {qkv(m, n, 2048) for m in range(1500, 9500, 100) for n in (4096, 6144)} == {185, 186, 187, 188}
+
+
+def test_products_of_65_to_256_rows_keep_the_tiles_of_256_columns(plan):
+    """One workgroup a CU on tiles of 256 x 64 does the 8B shape's products of around 100 rows sooner than two on tiles of 128 x 64
+    (128 rows: gate/up 47 against 51 us, down 34 against 35); with other shares of K they are even, and o's few columns go the other way."""
+    for M in (100, 128):
+        assert plan(M, 24576, 4096, EPI_SWIGLU) == 184 and plan(M, 4096, 12288, EPI_ADD) == 8184, M
+        assert plan(M, 6144, 4096) == 4184 and plan(M, 4096, 4096, EPI_ADD) == 4124, M
+    assert plan(200, 12288, 2048, EPI_SWIGLU) == 184 and plan(256, 12288, 2048, EPI_SWIGLU) == 184      # 25 and 26 us; on 124 26 and 30
+    assert plan(128, 6144, 4096, deferred=True) % 1000 == 184
+
+
+def test_a_cut_along_the_rows_is_done_sooner_by_the_estimates():
+    """Products whose rows end a little past whole tiles are cut exactly where the two parts' estimates come to less than the whole's."""
+    import ctypes
+    from herbert_rs_amd.kernels import mfma  # noqa: F401
+    native = lib.load("gemm_mfma")
+    cost = native.hb_gemm_mfma_plan_cost
+    cost.restype = ctypes.c_double
+    W, cuts = 1 << 24, 0
+    for M, (N, K, epi) in itertools.product([130, 257, 520, 1025, 1300, 2060, 2600, 3075, 4100],
+                                            [(24576, 4096, EPI_SWIGLU), (4096, 12288, EPI_ADD), (2048, 2048, EPI_ADD), (6144, 4096, EPI_STORE)]):
+        of = lambda m: cost(m, N, K, epi, 0, 0, 0, W, 0)
+        parts = {a: of(a) + of(M - a) for a in (M // 128 * 128, M // 256 * 256) if 0 < a < M}
+        rows, best = native.hb_gemm_mfma_split(M, N, K, epi, W), min(parts.values())
+        assert parts[rows] == best < of(M) if rows else best >= 0.99 * of(M) * (1 - 1e-9), (M, N, K, epi)
+        cuts += rows > 0
+    assert 3 < cuts < 30
