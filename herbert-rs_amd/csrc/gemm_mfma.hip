@@ -32,6 +32,9 @@ HB_MODULE_ERROR_SLOT()
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+// the same on an element's own border, as memory accesses may lie (LDS accesses may not)
+typedef __bf16 bf16x8_any __attribute__((ext_vector_type(8), aligned(2)));
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
 #define EPI_STORE 0
 #define EPI_ADD 1
@@ -751,8 +754,8 @@ __device__ __forceinline__ void store_wave_tile(const f32x4 (&acc)[TN][TM], void
 // pieces of 64 bytes, and reading C back for the add does the same. Here a wave first lays PB x 16
 // rows of its tile into LDS of its own (`stage`, rows of TN x 16 floats, the 16-byte chunk c of row r
 // at chunk c ^ (r mod chunks)), then reads them back along the rows: an instruction then moves whole
-// rows, 512 contiguous bytes for a tile 128 wide. Where ldc or N is no multiple of 4 or C lies off a
-// 16-byte border (`whole` is false) they go to memory element by element.
+// rows, 512 contiguous bytes for a tile 128 wide, on any border of 4 bytes (element by element, 2048 x 12288 x 2048 added
+// off a 16-byte border took 212 us, and 111 so). Where N is no multiple of 4 (`whole` is false) they go to memory element by element.
 template <int EPI, int TN, int TM, int PB>
 __device__ __forceinline__ void store_wave_tile_lds(const f32x4 (&acc)[TN][TM], float* C, int M, int N, int ldc,
                                                     int m_base, int n_base, int lane, float* stage, bool whole) {
@@ -793,7 +796,7 @@ __device__ __forceinline__ void store_wave_tile_lds(const f32x4 (&acc)[TN][TM], 
                 for (int u = 0; u < GROUP; ++u) {
                     const int row = (i0 + u) * RPI + rrow;
                     const int m = m_base + 16 * b0 + row, n = n_base + 4 * rchunk;
-                    before[u] = (m < M && n < N) ? *(const f32x4*)(C + (size_t)m * ldc + n) : f32x4{0.f, 0.f, 0.f, 0.f};
+                    before[u] = (m < M && n < N) ? *(const f32x4_any*)(C + (size_t)m * ldc + n) : f32x4{0.f, 0.f, 0.f, 0.f};
                 }
             }
 #pragma unroll
@@ -802,7 +805,7 @@ __device__ __forceinline__ void store_wave_tile_lds(const f32x4 (&acc)[TN][TM], 
                 const int m = m_base + 16 * b0 + row, n = n_base + 4 * rchunk;
                 f32x4 v = *(const f32x4*)(stage + row * (CH * 4) + ((rchunk ^ (row & (CH - 1))) * 4));
                 if (EPI == EPI_ADD) v += before[u];
-                if (m < M && n < N) *(f32x4*)(C + (size_t)m * ldc + n) = v;
+                if (m < M && n < N) *(f32x4_any*)(C + (size_t)m * ldc + n) = v;
             }
         }
     }
@@ -813,13 +816,12 @@ __device__ __forceinline__ void store_wave_tile_lds(const f32x4 (&acc)[TN][TM], 
 // 16 lines in pieces of 32 bytes. Here a wave lays its whole tile's outputs into LDS of its own (the
 // 16-byte chunk c of row r at chunk c ^ (r mod chunks), or (c + r) mod chunks where the chunks are no
 // power of two), then reads them back along the rows: an instruction stores whole rows, 128 contiguous
-// bytes for a gated tile 128 wide. n_base: the wave's first column (of the gate/up columns). Where ldc is
-// no multiple of 8 or C lies off a 16-byte border (`whole` is false) they go to memory element by element.
+// bytes for a gated tile 128 wide. on whatever border C and ldc put them. n_base: the wave's first column (of the gate/up columns).
 // `second`: the second gated unit or activation of its kind (GLU_RELU, UNARY_GELU) in place of the first; taken by a
 // choice at every output, since two copies of this code have the compiler move sums to memory.
 template <int EPI, int TN, int TM>
 __device__ __forceinline__ void store_wave_tile_bf16_lds(const f32x4 (&acc)[TN][TM], bf16* C, int M, int N, int ldc, int m_base,
-                                                         int n_base, int lane, bf16* stage, bool whole, bool second) {
+                                                         int n_base, int lane, bf16* stage, bool second) {
     constexpr int STEP = EPI == EPI_ACT ? 1 : 2;
     constexpr int CH = 2 * TN / STEP;       // 16-byte chunks of a row: 16 outputs a block, or a gate block and its up block
     constexpr int RPI = 64 / CH;            // rows an instruction moves
@@ -848,14 +850,6 @@ __device__ __forceinline__ void store_wave_tile_bf16_lds(const f32x4 (&acc)[TN][
             *(bf16x4*)((__bf16*)stage + row * (CH * 8) + place(row, 2 * a / STEP + (g4 >> 1)) * 8 + 4 * (g4 & 1)) = v;
         }
     }
-    if (!whole) {
-        for (int row = 0; row < ROWS; ++row) {
-            const int m = m_base + row;
-            for (int c = lane; c < CH * 8 && m < M && n_base / STEP + c < outs; c += 64)
-                C[(size_t)m * ldc + n_base / STEP + c] = stage[row * (CH * 8) + place(row, c >> 3) * 8 + (c & 7)];
-        }
-        return;
-    }
     const int rrow = lane / CH, rchunk = lane % CH;
     if (lane >= RPI * CH) return;
 #pragma unroll
@@ -866,7 +860,7 @@ __device__ __forceinline__ void store_wave_tile_bf16_lds(const f32x4 (&acc)[TN][
         const bf16x8 v = *(const bf16x8*)((const __bf16*)stage + row * (CH * 8) + place(row, rchunk) * 8);
         if (m >= M) continue;
         if (n + 7 < outs) {
-            *(bf16x8*)((__bf16*)C + (size_t)m * ldc + n) = v;
+            *(bf16x8_any*)((__bf16*)C + (size_t)m * ldc + n) = v;
         } else {
 #pragma unroll
             for (int j = 0; j < 8; ++j)
@@ -1243,12 +1237,11 @@ gemm_tile_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, void* _
             float* const stage = (float*)((char*)lds + wave * REGION);
             if constexpr (BF16_OUT)
                 if (!sliced) {
-                    const bool whole = (ldc & 7) == 0 && ((size_t)Cv & 15) == 0;
-                    store_wave_tile_bf16_lds<EPI, TN, TM>(acc, (bf16*)Cv, M, N, ldc, m_base, n_base, lane, (bf16*)stage, whole, scale.glu == 1);
+                    store_wave_tile_bf16_lds<EPI, TN, TM>(acc, (bf16*)Cv, M, N, ldc, m_base, n_base, lane, (bf16*)stage, scale.glu == 1);
                     return;
                 }
             if constexpr ((TN & (TN - 1)) == 0) {           // (tiles of another width are launched for gated units alone, whole)
-                const bool whole = (ld & 3) == 0 && (N & 3) == 0 && ((size_t)dst & 15) == 0;
+                const bool whole = (N & 3) == 0;
                 if (EPI == EPI_ADD && !sliced)
                     store_wave_tile_lds<EPI_ADD, TN, TM, PB>(acc, dst, M, N, ld, m_base, n_base, lane, stage, whole);
                 else
