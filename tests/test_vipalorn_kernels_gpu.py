@@ -302,13 +302,15 @@ def test_prompt_tokens_share_their_keys(H, rank, rot):
             assert not again[late:150].view(10, H, rank)[:, :, 7:9].isfinite().any()
 
 
-@pytest.mark.parametrize("ranges", [1, 1024])
+@pytest.mark.parametrize("ranges", [1, 14, 21, 1024])
 @pytest.mark.parametrize("H,rank,rot", [(16, 512, 64), (5, 512, 128), (3, 480, 0), (17, 160, 96), (8, 32, 0), (20, 288, 32), (16, 128, 128)])
 def test_a_token_a_sequence_by_waves_that_share_a_row(H, rank, rot, ranges, monkeypatch):
     """The latent attention of one token a sequence, whose four waves take a quarter of a row's numbers each: latents and rotated parts
-    that no four waves share evenly, one chunk of keys and several at their edges, one range and as many as there are chunks, a sink and a
-    gate, against float64; the tolerance of the prompts' kernel."""
+    that no four waves share evenly, one chunk of keys and several at their edges, one range, two to six of several chunks (the later ones empty or
+    shorter; twice as many as workgroups were asked for, because their chunks would be too many) and as many as there are chunks,
+    a sink and a gate, against float64; the tolerance of the prompts' kernel."""
     row, held = rank + rot, [1, 31, 32, 33, 64, 150, 330]
+    given = []
     monkeypatch.setattr(latent, "TARGET_WAVES", ranges)
     cache = Cache({0: KVNeed(1, row, None, values=False)}, 64 * 24, 4096, torch.bfloat16, DEV, max_slots=len(held))
     kv = cache.kv_view(0)
@@ -325,8 +327,12 @@ def test_a_token_a_sequence_by_waves_that_share_a_row(H, rank, rot, ranges, monk
             kv.k[table[p // 64], 0, :min(64, r.shape[0] - p)] = r[p:p + 64].to(DEV)
     q, gate, sinks = rand(len(held), H * row, seed=9), rand(len(held), H, seed=10), rand(H, seed=11)
     out = torch.empty(len(held), H * rank, dtype=torch.bfloat16, device=DEV)
-    latent.latent_attention_mfma(q.to(DEV), meta, kv, out, gate.to(DEV), 0, H, rank, rot, row ** -0.5,
-                                 lambda name, shape, dt: torch.empty(shape, dtype=dt, device=DEV), sinks=sinks.to(DEV))
+
+    def buffer(name, shape, dt):
+        given.append(shape[0] // (len(held) * H))
+        return torch.empty(shape, dtype=dt, device=DEV)
+    latent.latent_attention_mfma(q.to(DEV), meta, kv, out, gate.to(DEV), 0, H, rank, rot, row ** -0.5, buffer, sinks=sinks.to(DEV))
+    assert set(given) == ({1: set(), 14: {4}, 21: {6}, 1024: {16}} if H <= 16 else {1: set(), 14: {2}, 21: {3}, 1024: {16}})[ranges]
     for t, r in enumerate(rows):
         keys = r.double()
         score = q[t].view(H, row).double() @ keys.T * row ** -0.5
