@@ -1115,7 +1115,7 @@ extern "C" int hb_latent_attention_mfma(const float* q_full, const void* pages, 
                                         int chunks_per_split, const float* sinks, const int* seq_starts, int n_seqs,
                                         int longest, const int* which, hipStream_t stream) {
     HB_REQUIRE(T > 0 && H > 0, "latent attention: empty input");
-    HB_REQUIRE(rank > 0 && rank % 32 == 0 && rank <= 512 && rot % 32 == 0 && rank + rot <= 640,
+    HB_REQUIRE(rank > 0 && rank % 32 == 0 && rank <= 512 && rot >= 0 && rot % 32 == 0 && rot <= 128,
                "latent attention: the matrix-core kernel takes a latent and a rotated part in steps of 32, up to 512 + 128, not %d + %d", rank, rot);
     HB_REQUIRE(page_size % LA_CHUNK == 0, "latent attention: pages of %d positions", page_size);
     HB_REQUIRE(splits >= 1 && splits <= HB_WAVE && chunks_per_split >= 1, "latent attention: %d ranges, the kernels take 1 to 64", splits);
@@ -1144,8 +1144,7 @@ extern "C" int hb_latent_attention_mfma(const float* q_full, const void* pages, 
     latent_attention_mfma_kernel<VWV, KXV><<<grid, LA_WAVES * HB_WAVE, 0, stream>>>(                               \
         q_full, (const bf16*)pages, (bf16*)out, part_acc, part_ml, gate, gate_ld, positions, seq_of, slots,      \
         page_table, max_pages, page_size, H, rank, rot, scale, splits, chunks_per_split, sinks)
-    if (rot > 128) LA_LAUNCH(4, 5);
-    else if (rank <= 128) LA_LAUNCH(1, 1);
+    if (rank <= 128) LA_LAUNCH(1, 1);
     else if (rank <= 256) LA_LAUNCH(2, 1);
     else LA_LAUNCH(4, 1);
 #undef LA_LAUNCH
