@@ -1477,27 +1477,30 @@ static int launch_tile32(const void* X, const void* W, void* C, int M, int N, in
 #undef TILE_DISPATCH
 
 // The tiles of products of more than 64 rows: number, columns, rows, workgroups on a CU, a step's time, what a second
-// workgroup on the CU adds to it (a share) and what a round of tiles costs beside its steps (us).
+// workgroup on the CU adds to it (a share), what a round of tiles costs beside its steps (us) and what they wait for bytes that come
+// from memory (us a MB).
 // (168: three quarters of the 256 x 256 tile's arithmetic a step, for the SwiGLU product whole: where that
 // one's tiles fill the last round of 256 badly, 192 columns often fill it)
 // (187, 186, 185: 224, 192 and 160 rows high, for row counts whose tiles of 256 rows leave CUs empty and whose
 // tiles of 128 rows need another round; the heights beside 192: 9,404 rows x 2,048 columns (K 6144, add) 212 us on
 // 192, 197 on 160; 2,600 x 24576 x 4096 (gated) 441 on tile 168, 398 on 224)
-struct Mid { int id, bn, bm, per_cu; double step_us, second, round_us; };
-static const Mid mid_tiles[] = {{188, 256, 256, 1, 1.155, 0, 7.283}, {187, 256, 224, 1, 1.063, 0, 6.462}, {186, 256, 192, 1, 0.927, 0, 7.139},
-                                {185, 256, 160, 1, 0.881, 0, 6.813}, {142, 256, 128, 1, 0.714, 0, 5.56}, {122, 128, 128, 2, 0.861, 0.086, 3.357},
-                                {124, 128, 64, 2, 0.428, 0.584, 3.116}, {184, 256, 64, 1, 0.629, 0, 3.623}, {168, 192, 256, 1, 0.917, 0, 5.569}};
-// What a product's tiles take, without what adds its slices up: the slowest of its rounds one after the other, of what all
-// workgroups move out of the L2s (27 TB/s) and of what comes from HBM once (6.5 TB/s).
+struct Mid { int id, bn, bm, per_cu; double step_us, second, round_us, wait_us; };
+static const Mid mid_tiles[] = {{188, 256, 256, 1, 1.237, 0, 3.493, 0.046}, {187, 256, 224, 1, 1.124, 0, 4.621, 0.057},
+                                {186, 256, 192, 1, 0.915, 0, 5.571, 0.052}, {185, 256, 160, 1, 0.83, 0, 5.598, 0.061},
+                                {142, 256, 128, 1, 0.636, 0, 4.584, 0.059}, {122, 128, 128, 2, 0.682, 0, 3.098, 0.06},
+                                {124, 128, 64, 2, 0.304, 0.47, 3.372, 0.058}, {184, 256, 64, 1, 0.48, 0, 4.225, 0.032},
+                                {168, 192, 256, 1, 0.954, 0, 3.077, 0.048}};
+// What a product's tiles take, without what adds its slices up: their rounds one after the other, what all workgroups move out of
+// the L2s (46.4 TB/s beside the steps) and what of the bytes from memory they wait for; no less than these take at 7 TB/s.
 static double mid_time(const Mid& v, int M, int N, int K, int slices) {
-    const long wgs = (long)((M + v.bm - 1) / v.bm) * ((N + v.bn - 1) / v.bn) * slices, slots = 256 * v.per_cu;
+    const long m_tiles = (M + v.bm - 1) / v.bm, n_tiles = (N + v.bn - 1) / v.bn, wgs = m_tiles * n_tiles * slices, slots = 256 * v.per_cu;
     const long rounds = (wgs + slots - 1) / slots, on_a_cu = ((wgs < slots ? wgs : slots) + 255) / 256;
     const int per = (K / 64 + slices - 1) / slices;
     const double stepping = (double)rounds * (per * v.step_us * (1 + v.second * (on_a_cu - 1)) + v.round_us);
-    const double moving = (double)wgs * per * (v.bn + v.bm) * 128 / 27.576e6;
-    const double fetching = ((double)N + M) * K * 2 / 6.507e6;
-    const double slower = stepping > moving ? stepping : moving;
-    return fetching > slower ? fetching : slower;
+    const double moving = ((double)n_tiles * M + (double)m_tiles * N) * K * 2 / 46.414e6;
+    const double memory = ((double)N + M) * K * 2 / 1e6;
+    const double time = stepping + moving + v.wait_us * memory;
+    return time > memory / 7.0 ? time : memory / 7.0;
 }
 
 // The tile of the fused q/k/v product of shape 0: 256 columns and the height with which it is expected to be done soonest.
@@ -1644,7 +1647,7 @@ static GemmPlan plan_gemm(int M, int N, int K, int ldc, int epi, bool norm_w, bo
         // More than 64 rows: neither the arithmetic nor the weights alone decide. All tiles from 128 x 64
         // to 256 x 256 with 1 to 16 K slices are candidates, by mid_time and, for slices, the second kernel. Fitted to every
         // candidate's time, weights from memory, at 16 products of four model sizes and 72 to 9,404 rows (520 sizes): the choice is
-        // 1.0 % from the best candidate on average and 21 % at worst; without a quarter of the sizes the fit is 1.3 % off on those.
+        // 0.7 % from the best candidate on average and 21 % at worst, at 287 sizes of seven other products 1.5 %.
         // (One share for both tiles of two workgroups a CU had tile 124 displace 184: 128 rows of 24576 x 4096 51.4 us where 184 takes
         // 47.0, of 4096 x 12288 35.3 and 34.0.)
         const int steps = K / 64;
@@ -1657,7 +1660,7 @@ static GemmPlan plan_gemm(int M, int N, int K, int ldc, int epi, bool norm_w, bo
                 if (emit_g && (sl == 1 || !reducer_norms)) continue;      // the kernel that adds the slices up norms
                 if (deferred && sl > 8) break;                            // whoever adds the slices up takes 2, 4 or 8
                 double cost = mid_time(v, M, N, K, sl);
-                if (sl > 1) cost += deferred ? (double)sl * M * N * 4 / 3.312e6 : 3.993 + (double)(sl + 1) * M * N * 4 / 3.312e6;
+                if (sl > 1) cost += deferred ? (double)sl * M * N * 4 / 3.384e6 : 1.639 + (double)(sl + 1) * M * N * 4 / 3.384e6;
                 if (best < 0 || cost < best) {
                     best = cost;
                     tile = v.id;
@@ -1674,8 +1677,9 @@ static GemmPlan plan_gemm(int M, int N, int K, int ldc, int epi, bool norm_w, bo
 }
 
 // The rows of the first of two products that M rows are better cut into (see hb_gemm_mfma), or 0: where both are expected to be done
-// sooner than the whole. Of 634 sizes (12 products, 130 to 6,200 rows, most a little past whole tiles) 68 are cut; the choice is
-// 0.35 % from the better one on average and 17 % at worst (never cut: 0.6 and 23).
+// sooner than the whole. Of 634 sizes (12 products, 130 to 6,200 rows, most a little past whole tiles) 63 are cut; the choice is
+// 0.3 % from the better one on average and 12 % at worst (never cut: 0.5 and 19). Some cuts lose: 2,049 rows of 4096 x 4096 take 72 us so and
+// 66 on tiles of 160 rows, of 4096 x 12288 182 and 177.
 static int split_rows(int M, int N, int K, int ldc, int epi, bool special, int tile_hint, size_t workspace_floats,
                       const GemmPlan& whole) {
     if (special || M <= 128 || (tile_hint != 0 && tile_hint != -128 && tile_hint != -256)) return 0;
