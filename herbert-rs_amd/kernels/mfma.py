@@ -338,21 +338,21 @@ def gemm_join(a, w, x, after, extra=None, step=None, before=None, y=None, packed
              ptr(y), _stream())
 
 
-QKV_FUSE_MIN_TILES = 136   # of 256 x 256; with fewer (measured: 120 lose, 144 win) the plain product's smaller tiles or K slices fill the CUs better
+# Of 256 x 256, or of a head's width: with fewer the plain product's smaller tiles or K slices fill the CUs as well. Microseconds fused / by a
+# plain product and the kernel behind it: shape 0 72 tiles (768 x 6144, K 4096) 67 / 56, 120 (768 x 10240, K 5120) 94 / 92, 130 (3,100 x 2560,
+# K 2048) 43 / 52, 144 (1,300 x 6144) 76 / 80, 1,480 (9,404 x 10240) 760 / 895; shape 1 144 (768 x 6144) 58 / 56, 192 (1,000 x 6144) 59 / 70;
+# shape 2 120 (768 x 2560) 25 / 30, 160 (1,000 x 2560) 25 / 39.
+QKV_FUSE_MIN_TILES = 136
 
 
 def qkv_tile_shape(M, N):
     """The tiles on which a q/k/v projection of M rows and N = heads x 128 columns norms, rotates and
     writes the cache itself, or None where it should not (too few tiles to fill the CUs: the plain
     product's smaller tiles and K slices then do better, and a kernel of its own does the rest).
-    0: 256 x 256; 1: a head wide, 256 rows high; 2: a head wide, 128 rows high."""
-    tiles = -(-M // 256) * -(-N // 256)
-    if tiles >= QKV_FUSE_MIN_TILES:
-        # (rows that end a little past whole tiles, with a last round of tiles that is nearly empty:
-        # the plain product cuts such rows off as a product of their own and is then ahead, 3 % of a
-        # prompt of 2,600 tokens)
-        if tiles > 256 and tiles % 256 < 64 and 0 < M % 256 <= 64:
-            return None
+    0: 256 columns, 160 to 256 rows high, whichever are done soonest (so rows a little past whole tiles of 256 are no exception:
+    8,200 x 6144, K 4096, 359 us and 425 by the plain product, 2,600 138 and 148); 1: a head wide, 256 rows high; 2: a head
+    wide, 128 rows high."""
+    if -(-M // 256) * -(-N // 256) >= QKV_FUSE_MIN_TILES:
         return 0
     heads = N // 128
     for shape, rows in ((1, 256), (2, 128)):

@@ -245,3 +245,12 @@ def test_a_cut_along_the_rows_is_done_sooner_by_the_estimates():
         assert parts[rows] == best < of(M) if rows else best >= 0.99 * of(M) * (1 - 1e-9), (M, N, K, epi)
         cuts += rows > 0
     assert 3 < cuts < 30
+
+
+def test_long_projections_past_whole_tiles_write_the_cache_themselves():
+    """Rows a little past whole tiles of 256, with a last round of those that is nearly empty: the fused q/k/v product has tiles of
+    other heights too and is done sooner than a plain product cut along the rows (8,200 rows of 4096 columns 143 against 179 us)."""
+    from herbert_rs_amd.kernels import mfma
+    for M, N in ((2600, 6144), (3100, 6144), (8200, 6144), (4120, 4096), (8200, 4096), (3100, 10240), (2048, 6144), (2300, 6144)):
+        assert mfma.qkv_tile_shape(M, N) == 0, (M, N)
+    assert mfma.qkv_tile_shape(128, 6144) is None and mfma.qkv_tile_shape(2048, 4096) == 1
