@@ -238,8 +238,8 @@ extern "C" int hb_latent_attention_plain(const float* q_full, const void* pages,
 // maxima and denominators go to scratch and a second kernel joins them in the ranges' order.
 // Bound by its own chain: positions, slot, page, rows, scores, exchange, softmax, sums, and by code that a CU reads for the first time, which
 // was four times as long by one wave that held a whole row. With the kernel that joins the ranges, by one wave | now, 16 heads of 512 + 64, us:
-// 1 token at 100 keys 20.9 | 10.9, at 4,000 37 | 21; 4 at 509 22.5 | 12.5; 8 at 2,000 39 | 25; 32 at 1,000 40 | 31; 64 at 2,000 78 | 47; 200 at 300 74 | 36;
-// 32 heads, 32 at 4,000 130 | 67; 8 heads of 256 + 64, 4 at 300 13.3 | 8.7.
+// 1 token at 100 keys 20.3 | 10.5, at 4,000 37 | 20; 4 at 300 22 | 12; 8 at 2,000 39 | 20; 32 at 1,000 40 | 20; 64 at 2,000 78 | 38; 200 at 300 74 | 34,
+// at 1,500 209 | 88; 400 at 500 166 | 55; 128 heads, 64 at 1,000 242 | 99; 8 heads of 256 + 64, 4 at 300 13.0 | 8.3, 256 at 1,000 68 | 42.
 // Sizes: rank and rot multiples of 32; VW >= rank / 128 steps of 32 numbers a wave, KX >= rot / 128 of the rotated part.
 typedef __bf16 la_bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 la_bf16x4 __attribute__((ext_vector_type(4)));

@@ -3,11 +3,12 @@
 //   few rows (M <= 16, decoding): HBM-bound. The weights stream from memory straight into
 //     16x16x32 MFMA operands (each is used once), the waves of a workgroup split K between
 //     them and add their parts through LDS in a fixed order.
-//   tiled: 32x32x16 MFMA; tiles loaded from global memory straight into rings of LDS stages, a
+//   tiled: 16x16x32 MFMA; tiles loaded from global memory straight into rings of LDS stages, a
 //     step of 64 k ahead of the MFMAs that consume them; with few tiles K is cut into slices
 //     over further workgroups, whose sums a second kernel (or the caller's next kernel) adds up.
-//     256 x 256, 256 x 128 or 128 x 128 for prompts; one block of rows high (128 x 32, 128 x 64,
-//     256 x 64) for at most 64 rows, where it competes with the few-row kernel (see plan_gemm).
+//     256 columns and 256, 224, 192, 160, 128 or 64 rows, 192 x 256, 128 x 128 and 128 x 64 for more than
+//     64 rows (see mid_tiles); 128 x 32, 128 x 64, 256 x 64 and 96 x 64 for at most 64 rows, where they compete
+//     with the few-row kernel (see plan_gemm).
 // Between a product that adds to the residual stream and the next one an RMSNorm can be handed
 // on instead of run (see NormHandoff).
 // In both the weight rows are the MFMA's first operand, so a lane ends up with runs of four
@@ -816,9 +817,10 @@ __device__ __forceinline__ void store_wave_tile_lds(const f32x4 (&acc)[TN][TM], 
 // 16 lines in pieces of 32 bytes. Here a wave lays its whole tile's outputs into LDS of its own (the
 // 16-byte chunk c of row r at chunk c ^ (r mod chunks), or (c + r) mod chunks where the chunks are no
 // power of two), then reads them back along the rows: an instruction stores whole rows, 128 contiguous
-// bytes for a gated tile 128 wide. on whatever border C and ldc put them. n_base: the wave's first column (of the gate/up columns).
+// bytes for a gated tile 128 wide, on whatever border C and ldc put them. n_base: the wave's first column (of the gate/up columns).
 // `second`: the second gated unit or activation of its kind (GLU_RELU, UNARY_GELU) in place of the first; taken by a
-// choice at every output, since two copies of this code have the compiler move sums to memory.
+// choice at every output, since two copies of this code have the compiler move sums to memory. (It still does with 12 to 16 registers of the
+// 256 x 256 tiles, 52 to 68 bytes a lane: behind the main loop, stored and read back once a tile.)
 template <int EPI, int TN, int TM>
 __device__ __forceinline__ void store_wave_tile_bf16_lds(const f32x4 (&acc)[TN][TM], bf16* C, int M, int N, int ldc, int m_base,
                                                          int n_base, int lane, bf16* stage, bool second) {
@@ -1433,9 +1435,8 @@ static int launch_tile64(const void* X, const void* W, void* C, int M, int N, in
 #undef EXTRA
 }
 
-// Tiles whose width is no power of two (192 = three pieces of 32 a wave): for the SwiGLU epilogue
-// only, whose bfloat16 output goes to memory lane by lane (the float32 epilogues' way through LDS
-// counts on rows of a power of two of 16-byte chunks).
+// Tiles whose width is no power of two (192 and 96, six blocks of 16 a wave): for the SwiGLU epilogue only. The float32 epilogues'
+// way through LDS counts on rows of a power of two of 16-byte chunks; the bfloat16 outputs' does not.
 template <int TN, int TM, int WNW, int WMW, int WST, int XST>
 static int launch_tile64_swiglu(const void* X, const void* W, void* C, int M, int N, int K, int ldc, int epi,
                                 int packed, hipStream_t stream, int slices, RowScale scale) {

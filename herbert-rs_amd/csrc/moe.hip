@@ -950,8 +950,8 @@ grouped_mfma_kernel(const bf16* __restrict__ A, int lda, size_t a_group_off, con
 // chunk c at chunk c ^ ((row >> 1) & 7); a block of 16 weight rows and 32 k is 1 KB as packed. K in steps of 64.
 // Gate/up of 32 experts of 768 on 2,048, weights from memory (40 us at the rate of a large copy), by tiles of 64 and by the tile that
 // tall_rows of moe.py takes, in brackets that one by 32x32x16 products with all loads of a step in its second half: 2,048 tokens, four experts
-// each, 117 us, 84 (128 rows; 88); 1,712 101, 67 (256; 73); 1,282 98, 56 (192; 59); 512 57, 47 (128; 48). 64 experts of 1,536 on 4,096, 2,500
-// tokens: 505, 398 (192; 435); 1,500 340, 303 (128; 307).
+// each, 104 us, 80 (128 rows; 83); 1,712 99, 64 (256; 71); 1,282 98, 56 (192; 58); 512 58, 47 (128; 48). 64 experts of 1,536 on 4,096, 2,500
+// tokens: 496, 391 (192; 403); 1,500 348, 308 (128; 312). (All three in one run, experts chosen at random; how unequally busy they are moves these by a tenth.)
 #define TALL_BN 256
 #define TALL_W_STAGE (TALL_BN * 64)          // elements
 #define TALL_WST 3

@@ -28,12 +28,14 @@
 // 0.999: the outputs' error is 0.67 to 0.97 of the walk's (0.8e-7 to 1e-6), 0.56 to 0.88 for the linear attention, and that of the
 // state left 0.76 to 1.06. (With A, B and T in float32 the outputs' was up to 1.3 of the walk's, the state's up to 2.)
 //
-// 2,048 tokens of 16 heads of 128 x 128 take 152 us (the walk 781), with a decay a channel 201 (1,084), the linear attention
+// 2,048 tokens of 16 heads of 128 x 128 take 141 us (the walk 781), with a decay a channel 199 (1,084), the linear attention
 // 131 (909); 8 sequences of 300 tokens with a decay a channel 217 (408), the linear attention 123 (455). Bound: the second kernel by its
-// chain (64 products of 32 cycles a chunk and wave and two exchanges through LDS, 100 us of the 152), the first by its products in
+// chain (64 products of 32 cycles a chunk and wave and two exchanges through LDS, 100 us of the 141), the first by its products in
 // float64 of 64 cycles and what lies between them. With one decay a head its pairs within a block are summed once instead of once a
-// level (256 of 448 products of its longest wave), and its pieces lie in LDS twice over, so that two workgroups fit a CU: 86 us -> 52. With a
-// decay a channel and keys of 128 a lane's decays take more than half of the registers: one workgroup a CU (two spill 270 of them).
+// level (256 of 448 products of its longest wave), and its pieces lie in LDS twice over, so that two workgroups fit a CU: 86 us -> 52, though
+// half of the registers are 27 too few for keys of 128 (112 bytes a lane in memory). With a decay a channel and keys of 64 two are 25 too few
+// and still ahead, both kernels: 2,048 tokens of 16 heads 116 us -> 105, four times that of 32 heads 596 -> 477, 128 tokens 32.4 -> 33.4. With
+// keys of 128 a lane's decays take more than half of the registers: one workgroup a CU (two spill 270 of them).
 #include "common.h"
 #include "mfma_f32.h"
 #include <math.h>

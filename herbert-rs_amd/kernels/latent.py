@@ -101,15 +101,17 @@ CHUNK = 32
 # A decode step's keys are cut into ranges until about so many workgroups of four waves run, one a CU, and into twice as many where a
 # range would have more than RANGE_CHUNKS chunks: every range leaves sums that another kernel reads. With 256 / 512 / 1,024 of them, 16 heads of
 # 512 + 64, us: 8 tokens at 2,000 keys (2 chunks a range) 19 / 25 / 25, 16 at 1,000 (2) 17 / 23 / 23, 32 at 1,000 (4) 20.5 / 21.7 / 31, 64 at 2,000 (16)
-# 44 / 36 / 47, 48 at 300 (2) 19.6 / 18.2 / 21.9; 32 heads, 32 at 4,000 (32) 78 / 55 / 66.
-TARGET_WAVES = 256
+# 44 / 36 / 47, 48 at 300 (2) 19.6 / 18.2 / 21.9; 32 heads, 32 at 4,000 (32) 78 / 55 / 66. Steps of more than 64 workgroups, by this rule with 256 / with
+# 512: 128 tokens at 2,000 72 / 78, 200 at 1,500 88 / 92 (at 150 to 1,500 71 / 65), 300 at 700 66 / 69, 400 at 500 55 / 73; 128 heads, 64 at 1,000 99 / 118.
+TARGET_WORKGROUPS = 256
 RANGE_CHUNKS = 4
 
 
 # Steps of several tokens a sequence take the kernel whose workgroups share their keys from contexts beyond this on: two
-# chunks of 32 keys leave it nothing to share (8 prompts of 64 tokens 34 us, four waves a token 19; of 100 tokens 42 and 37, of 200 87 and 79, of 300
-# 128 and 128). The line lies below where the times meet because only that kernel keeps a later token's number that is not finite out of the
-# tokens before it.
+# chunks of 32 keys leave it nothing to share. Microseconds by it / by four waves a token, 16 heads of 512 + 64: one prompt of 64 tokens 32 / 12, of
+# 128 38 / 16, of 300 55 / 34; 8 of 64 34 / 19, of 100 42 / 37, of 300 128 / 127; 8 heads of 256 + 64: one of 128 24 / 10, 8 of 64 20 / 9, of 100 22 / 18,
+# of 200 31 / 36, 4 of 400 42 / 54. The line lies below where the times meet because only that kernel keeps a later token's number that is not
+# finite out of the tokens before it; prompts whose heads' keys are built come by neither.
 PROMPT_FROM = 64
 
 
@@ -144,10 +146,10 @@ def _sequence_form(new, context, H, dim, rank, rot, most_bytes):
     the other's, so that a step of many sequences with a few tokens each behind long contexts does not pay for every one's contexts.
     The estimates: products of the heads' matrices with latents (keys here, tokens there) at 400 TFLOP/s, the attentions' own at 600 and
     500, and alone no less than the context's chain of tiles, 1.7 us for 64 keys here and 3.2 us for 32 there. Microseconds of a layer's
-    kernels on the latents / built, 16 heads of 128 + 64 and 128 on 512: prompts of 2 tokens 31 / 22, of 64 53 / 23, 8 of 8 45 / 24, 32 of
-    64 137 / 38; 16 tokens behind 1,000 124 / 48 (4.7 times the work: on the latents), 30 behind 1,000 134 / 47, 20 behind 8,192 818 / 239,
-    50 behind 4,096: one 433 / 131, 4 435 / 200, 10 438 / 442, 32 867 / 1,292; 8 heads of 128 + 64 on 256: 2 tokens 20 / 19, 32 of 64 66 / 27,
-    50 behind 4,096: one 275 / 118, 32 317 / 590."""
+    kernels on the latents / built, 16 heads of 128 + 64 and 128 on 512: prompts of 2 tokens 25 / 27, of 64 41 / 29, 8 of 8 39 / 32, 32 of
+    64 124 / 52; 16 tokens behind 1,000 133 / 56 (4.7 times the work: on the latents), 30 behind 1,000 142 / 55, 20 behind 8,192 826 / 253,
+    50 behind 4,096: one 444 / 143, 4 450 / 217, 10 452 / 492, 32 944 / 1,423; 8 heads of 128 + 64 on 256: 2 tokens 18 / 24, 32 of 64 61 / 38,
+    50 behind 4,096: one 281 / 125, 32 337 / 633. (Of these the prompts of a few tokens alone are built where the latents are ahead, by 2 to 6 us.)"""
     pairs = new * (context - new) + new * (new + 1) // 2
     matrices = 4 * H * rank * dim / 400e6                   # (microseconds a row)
     here, there = 4 * pairs * H * (2 * dim + rot) / 600e6, 4 * pairs * H * (2 * rank + rot) / 500e6
@@ -303,9 +305,9 @@ def latent_attention_mfma(q_full, meta, cache, out, gate, gate_off, H, rank, rot
         # the grid must not depend on the contexts themselves (a recorded step is replayed at others of its bucket)
         chunks = -(-max(meta.context_bucket if part is None else 0, context) // CHUNK)
         blocks = rows * ((H + 15) // 16)
-        splits = max(1, min(TARGET_WAVES // blocks, chunks, 64))
+        splits = max(1, min(TARGET_WORKGROUPS // blocks, chunks, 64))
         if -(-chunks // splits) > RANGE_CHUNKS:
-            splits = max(1, min(2 * TARGET_WAVES // blocks, chunks, 64))
+            splits = max(1, min(2 * TARGET_WORKGROUPS // blocks, chunks, 64))
         per = -(-chunks // splits)
     part_acc = part_ml = None
     if splits > 1:

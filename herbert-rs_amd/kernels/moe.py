@@ -209,11 +209,12 @@ def tall_rows(T, top, routed, experts, hidden, inter, shared=False):
     tiles of 64, two to a CU, are expected to be done sooner (a round of theirs as long as one of 284 rows: 64 experts of 1,536 on 4,096,
     four each and a shared one, 800 tokens: 307 us, 353 by tiles of 128; 64 of 1,408 on 2,048, six each and a shared one, 512 tokens 160 and
     157 to 174). An expert's rows are taken to be spread around their mean as a random choice spreads them, and a round to be full at
-    nine tenths, since some experts of a model are busier than that. Over 132 layers (16 to 256 experts, 400 to 4,096 tokens) the height
-    that this gives is 2.0 % slower than the best one where experts are chosen at random (without the low tiles 2.3; 2.1 with rounds full
-    to the last tile, 7.8 full at eight tenths) and 9.7 % where they are very unequally busy, deviations of 0.5 to 1.2 of the mean (10.3;
-    11.2, 9.3): there one height for all experts costs a round that is nearly empty more often than not. An estimate that averaged the
-    rounds over both kinds of routing was better by a tenth of a layer's time at some token counts and worse by as much at others.
+    nine tenths, since some experts of a model are busier than that. Over 49 layers (8 to 256 experts, 250 to 4,000 tokens) the height
+    that this gives is 3.8 % slower than the best one where experts are chosen at random (1.6 with rounds full to the last tile, 6.2 full at
+    eight tenths; at worst 16 experts of 2,048, 1,500 tokens: 35) and at 98 layers of unequally busy ones, deviations of 0.4 to 2.6 of the
+    mean, 8.9 % (9.7, 7.1; without the low tiles 10.1): there one height for all experts costs a round that is nearly empty more often than
+    not. An estimate that averaged the rounds over both kinds of routing was better by a tenth of a layer's time at some token counts and
+    worse by as much at others.
     shared: every token takes one more expert."""
     rows = T * top / routed
     if rows < TALL_ROWS or hidden % 64 or inter % 64:

@@ -311,7 +311,7 @@ def test_a_token_a_sequence_by_waves_that_share_a_row(H, rank, rot, ranges, monk
     a sink and a gate, against float64; the tolerance of the prompts' kernel."""
     row, held = rank + rot, [1, 31, 32, 33, 64, 150, 330]
     given = []
-    monkeypatch.setattr(latent, "TARGET_WAVES", ranges)
+    monkeypatch.setattr(latent, "TARGET_WORKGROUPS", ranges)
     cache = Cache({0: KVNeed(1, row, None, values=False)}, 64 * 24, 4096, torch.bfloat16, DEV, max_slots=len(held))
     kv = cache.kv_view(0)
     slots = [cache.alloc_slot() for _ in held]
