@@ -1500,8 +1500,12 @@ static double mid_time(const Mid& v, int M, int N, int K, int slices) {
     const double stepping = (double)rounds * (per * v.step_us * (1 + v.second * (on_a_cu - 1)) + v.round_us);
     const double moving = ((double)n_tiles * M + (double)m_tiles * N) * K * 2 / 46.414e6;
     const double memory = ((double)N + M) * K * 2 / 1e6;
+    // (Tiles alone on a CU that fill the chip leave their slices' sums behind all at once. 300 rows of 2560 x 9728 in eight slices: 240 tiles of
+    // 256 x 128 34 to 42 us from run to run, 480 of 128 x 128 34; prompts of the 8B shape without / with this: 257 tokens 7.5 / 7.35 ms, 350 8.05 /
+    // 7.94, 400 8.6 / 8.45, 200 6.66 / 6.66. Tiles of 64 rows, 128 rows of 4096 x 12288, are not slower for it.)
+    const double leaving = slices > 1 && v.per_cu == 1 && v.bm >= 128 && wgs > 230 ? 0.7 * slices * v.bm / 128 : 0;
     const double time = stepping + moving + v.wait_us * memory;
-    return time > memory / 7.0 ? time : memory / 7.0;
+    return leaving + (time > memory / 7.0 ? time : memory / 7.0);
 }
 
 // The tile of the fused q/k/v product of shape 0: 256 columns and the height with which it is expected to be done soonest.
@@ -1647,8 +1651,9 @@ static GemmPlan plan_gemm(int M, int N, int K, int ldc, int epi, bool norm_w, bo
     if (tile == 0 && K % 64 == 0) {
         // More than 64 rows: neither the arithmetic nor the weights alone decide. All tiles from 128 x 64
         // to 256 x 256 with 1 to 16 K slices are candidates, by mid_time and, for slices, the second kernel. Fitted to every
-        // candidate's time, weights from memory, at 16 products of four model sizes and 72 to 9,404 rows (520 sizes): the choice is
-        // 0.7 % from the best candidate on average and 21 % at worst, at 287 sizes of seven other products 1.5 %.
+        // candidate's time, weights from memory, at 16 products of four model sizes and 72 to 9,404 rows (520 sizes; 0.7 % from the best
+        // candidate on average); at 13 products of 72 to 2,048 rows (325 sizes) the choice is 1.0 % from the best on average and
+        // 23 % at worst (72 rows of 1024 x 3072), at nine others (180 sizes) 1.9 and 16.
         // (One share for both tiles of two workgroups a CU had tile 124 displace 184: 128 rows of 24576 x 4096 51.4 us where 184 takes
         // 47.0, of 4096 x 12288 35.3 and 34.0.)
         const int steps = K / 64;

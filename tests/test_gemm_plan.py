@@ -254,3 +254,11 @@ def test_long_projections_past_whole_tiles_write_the_cache_themselves():
     for M, N in ((2600, 6144), (3100, 6144), (8200, 6144), (4120, 4096), (8200, 4096), (3100, 10240), (2048, 6144), (2300, 6144)):
         assert mfma.qkv_tile_shape(M, N) == 0, (M, N)
     assert mfma.qkv_tile_shape(128, 6144) is None and mfma.qkv_tile_shape(2048, 4096) == 1
+
+
+def test_slices_that_fill_the_chip_with_tiles_alone_on_a_cu_cost_more(plan):
+    """Where tiles of 256 columns in eight slices would take nearly every CU, fewer slices or tiles of two a CU are ahead (450 rows of
+    2048 x 6144 28.5 to 33 us in eight slices, 26 to 29 in four); with CUs left over the tiles of 256 columns stay."""
+    for M, N, K in ((450, 2048, 6144), (500, 2048, 6144), (300, 2560, 9728), (350, 2560, 9728), (384, 4096, 12288)):
+        assert not 8140 < plan(M, N, K, EPI_ADD) < 8190, (M, N, K)
+    assert plan(200, 2560, 9728, EPI_ADD) == 8142
